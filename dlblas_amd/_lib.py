@@ -190,8 +190,9 @@ def plan_full(mode: int, rows: int, N: int, K: int, workspace_bytes: int = None,
 
 def plan_grouped(mode: int, rows: int, N: int, K: int, G: int, expected_m: int = -1, workspace_bytes: int = None,
                  compute_units: int = 256):
-    """(variant name, tile lists used) of a grouped launch (mode 1 contiguous, 2 masked) with G experts and the masked
-    layout's hint; touches no GPU."""
+    """(variant name, flag) of a grouped launch (mode 1 contiguous, 2 masked) with G experts and the masked layout's hint;
+    the flag says whether a contiguous launch uses the tile lists / whether a masked one takes the weight-streaming kernel
+    in place of the named ring kernel.  Touches no GPU."""
     lib = load()
     v, t = ctypes.c_int(), ctypes.c_int()
     ws = WORKSPACE_BYTES if workspace_bytes is None else workspace_bytes
@@ -210,7 +211,7 @@ def force_variant(name_or_id) -> None:
 
 
 KNOBS = {'splitk': 0, 'skinny_waves': 1, 'skinny_unroll': 2, 'skinny_nfrags': 3, 'group_m': 4, 'skinny_dma': 5, 'epilogue': 6, 'skinny_bn': 7,
-         'splitk_mode': 8, 'spin_limit': 9, 'scale_table': 10, 'lds_oversize': 11, 'masked_grid': 12, 'tile_list': 13}
+         'splitk_mode': 8, 'spin_limit': 9, 'scale_table': 10, 'lds_oversize': 11, 'masked_grid': 12, 'tile_list': 13, 'stream': 14}
 
 
 def tune(knob: str, value) -> None:

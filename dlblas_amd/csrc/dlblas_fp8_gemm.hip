@@ -3,7 +3,9 @@
 #include "../../include/dlblas_fp8_gemm.h"
 #include "../../include/dlblas_fp8_moe.h"
 
+#include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -12,6 +14,7 @@
 #include "host_common.h"
 #include "fp8_gemm_pipelined.h"
 #include "fp8_gemm_skinny.h"
+#include "fp8_gemm_stream.h"
 #include "fp8_gemm_tiled.h"
 #include "fp8_quant.h"
 
@@ -99,9 +102,10 @@ enum Knob : int {
   kKnobLdsOversize,  // test hook: 1 = ask for more LDS than the GPU has, so that the launch is refused before anything is enqueued
   kKnobMaskedGrid,   // workgroups per CU of the masked layout's persistent grid (0 = default)
   kKnobTileList,     // expert-contiguous rows: 1 = device-built tile lists whenever possible, 2 = never (0 = by batch size)
+  kKnobStream,       // masked layout: 1 = never the weight-streaming kernel, 2 + i = its tile shape i wherever it applies (0 = by size)
   kKnobCount
 };
-thread_local int g_knob[kKnobCount] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+thread_local int g_knob[kKnobCount] = {};
 // set while run() asks every kernel of the call for its launch attributes, before the first pre-pass is enqueued
 thread_local bool g_prepare_only = false;
 constexpr int kDefaultSpinLimit = 400;  // x about 0.5 us: far beyond the spread of the slices of one round of workgroups
@@ -157,6 +161,16 @@ typedef PipeCfg<2, 4, 2, 2, 3, 2, false, true, 16> Pipe128x256w8T;  // the maske
 static_assert(Pipe128x256w8T::LDS_BYTES <= 160 * 1024 && Pipe128x128T::LDS_BYTES <= 160 * 1024 && Pipe128x64T::LDS_BYTES <= 160 * 1024, "ring + table fit the LDS");
 constexpr int kFusedMaxTiles = DLB_WS_COUNTER_BYTES / 16;  // four counter words per tile in the workspace head
 
+// Tile shapes of the weight-streaming grouped kernel: rows x weight rows per tile, and the ring each leaves room for.
+typedef StreamCfg<1, 4, 1, 2, 4, 16> Stream32x256;
+typedef StreamCfg<1, 4, 2, 2, 3, 16> Stream64x256;
+typedef StreamCfg<1, 4, 2, 1, 6, 16> Stream64x128;
+typedef StreamCfg<2, 4, 2, 2, 3, 11> Stream128x256;
+typedef StreamCfg<2, 2, 1, 1, 9, 16> Stream64x64;
+enum StreamShape : int { kStreamNone = -1, kStream32x256 = 0, kStream64x256, kStream64x128, kStream128x256, kStream64x64, kStreamCount };
+struct StreamDims { int bm, bn, stages, ch; };
+constexpr StreamDims kStreamDims[kStreamCount] = {{32, 256, 4, 16}, {64, 256, 3, 16}, {64, 128, 6, 16}, {128, 256, 3, 11}, {64, 64, 9, 16}};
+
 // Raise a kernel's dynamic LDS limit once per (kernel, device).
 template <class Kernel>
 hipError_t ensure_lds(Kernel kernel, int bytes, int dev, std::atomic<unsigned long long>* done_mask) {
@@ -208,6 +222,34 @@ hipError_t launch_pipelined(const Args& args, int grid, int dev, hipStream_t str
   if (e != hipSuccess || g_prepare_only) return e;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, args);
   return hipGetLastError();
+}
+
+template <class Cfg, int EPI, bool GATHER>
+hipError_t launch_stream(const Args& args, int grid, int dev, hipStream_t stream) {
+  static std::atomic<unsigned long long> lds_done{0};
+  auto kernel = fp8_gemm_stream_kernel<Cfg, EPI, GATHER>;
+  hipError_t e = ensure_lds(kernel, Cfg::LDS_BYTES, dev, &lds_done);
+  if (e != hipSuccess || g_prepare_only) return e;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, args);
+  return hipGetLastError();
+}
+
+template <int EPI, bool GATHER>
+hipError_t launch_stream_shape(int shape, const Args& args, int grid, int dev, hipStream_t stream) {
+  switch (shape) {
+    case kStream32x256: return launch_stream<Stream32x256, EPI, GATHER>(args, grid, dev, stream);
+    case kStream64x256: return launch_stream<Stream64x256, EPI, GATHER>(args, grid, dev, stream);
+    case kStream128x256: return launch_stream<Stream128x256, EPI, GATHER>(args, grid, dev, stream);
+    default: break;
+  }
+  if constexpr (EPI == kStoreProduct) {
+    switch (shape) {
+      case kStream64x128: return launch_stream<Stream64x128, EPI, GATHER>(args, grid, dev, stream);
+      case kStream64x64: return launch_stream<Stream64x64, EPI, GATHER>(args, grid, dev, stream);
+      default: break;
+    }
+  }
+  return hipErrorInvalidValue;
 }
 
 template <class Cfg>
@@ -611,7 +653,48 @@ struct Resolved {
   bool sctab;                // small ring kernels: row-major activation scales through the per-tile table in LDS
   int sct_pitch;             //   floats per table row (odd)
   bool fused;                // K slices added inside the launch (counters in the workspace head), no second pass
+  int stream;                // masked layout: tile shape of the weight-streaming kernel (kStreamNone: a ring kernel)
+  int chunk_len;             //   K blocks per chunk of its scale table
 };
+
+// K blocks per chunk of the streaming kernel's scale table: equal chunks of at most `ch` blocks, none shorter than the
+// stages - 1 steps the issue side runs ahead (the table has two buffers).  0: no such cut.
+int stream_chunk_len(int kblocks, int ch, int stages) {
+  for (int len = static_cast<int>(ceil_div(kblocks, ceil_div(kblocks, ch))); len >= stages - 1 && len > 0; --len) {
+    const int last = kblocks % len == 0 ? len : kblocks % len;
+    if (last >= stages - 1) return len;
+  }
+  return 0;
+}
+
+// Which tile shape of the weight-streaming kernel runs a masked launch (kStreamNone: none), from the typical rows of an
+// expert (twice the caller's hint covers nearly all of them).  A tile's step lasts what is longer of the trip its loads
+// take with the chip to themselves, 0.25 us + 1.9 ns per row of the two operands (a lone CU fetches 40 - 50 GB/s), and its
+// share of the HBM stream (6.9 TB/s over the busy CUs); tiles of 64 or 128 weight rows win while those of 256 leave CUs idle.
+int pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, int cus, int* chunk_len) {
+  const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
+  const int knob = g_knob[kKnobStream];
+  if (knob == 1 || g_forced_variant >= 0) return kStreamNone;
+  const double span = static_cast<double>(hint_rows > 0 && 2 * hint_rows < M ? 2 * hint_rows : M);
+  if (knob == 0 && span > 192) return kStreamNone;
+  int best = kStreamNone;
+  double best_us = 0.0;
+  for (int i = 0; i < kStreamCount; ++i) {
+    const StreamDims& d = kStreamDims[i];
+    if (knob >= 2 && i != knob - 2) continue;
+    if ((act && d.bn != 256) || kblocks < d.stages - 1) continue;
+    const int len = stream_chunk_len(kblocks, d.ch, d.stages);
+    if (len <= 0) continue;
+    const double mtiles = span <= d.bm ? 1.0 : 0.5 * (span / d.bm + 1.0);
+    const double tiles = static_cast<double>(G) * mtiles * static_cast<double>(act ? N / 256 : ceil_div(N, d.bn));
+    const double rows = std::min(0.5 * span, static_cast<double>(d.bm));
+    auto step = [&](double busy) { return std::max(0.25 + 0.0019 * (d.bn + rows), d.bn * 128.0 * busy / 6.9e6); };
+    const double full = std::floor(tiles / cus), rest = tiles - full * cus;
+    const double us = full * (1.0 + kblocks * step(cus)) + (rest > 0.5 ? 1.0 + kblocks * step(rest) : 0.0);
+    if (best == kStreamNone || us < best_us) best = i, best_us = us, *chunk_len = len;
+  }
+  return best;
+}
 
 // fused_act: the launch is one of the gate/up GEMMs with the activation in its epilogue (their kernels take no scale table)
 Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as_sm, int64_t as_sk, bool have_ws,
@@ -623,6 +706,9 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
   const bool usable_ws = have_ws && ws_bytes > DLB_WS_COUNTER_BYTES;
   r.pl = make_plan(mode, rows, N, K, cus, usable_ws ? ws_bytes : 0, dma_ok, G, hint_rows, fused_act || gather_scales);
   const Plan& pl = r.pl;
+  r.stream = kStreamNone;
+  if (mode == kMasked && dma_ok && K % kScaleBlock == 0 && K > 0 && static_cast<int64_t>(G) * rows < (1ll << 31))
+    r.stream = pick_stream(rows, N, K, G, hint_rows, fused_act, cus, &r.chunk_len);
   const int want = usable_ws ? pl.splitk : 1;
   r.kb_per_split = static_cast<int>(ceil_div(kblocks > 0 ? kblocks : 1, want));
   r.splitk = static_cast<int>(ceil_div(kblocks > 0 ? kblocks : 1, r.kb_per_split));  // no empty slice
@@ -661,9 +747,9 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
                                   : (pl.variant == kVarPipe128x64 ? Pipe128x64T::SCTAB_KB : Pipe128x128T::SCTAB_KB)) &&
            as_sk < (1ll << 20) && dma_ok;
   };
-  r.sctab = table_fits(r.kb_per_split);
+  r.sctab = r.stream == kStreamNone && table_fits(r.kb_per_split);
   // gather_scales: the re-layout pass also brings the rows into the GEMM's order, so it runs whatever the strides
-  if (is_pipelined(pl.variant) && usable_ws && !r.sctab &&
+  if (is_pipelined(pl.variant) && usable_ws && !r.sctab && r.stream == kStreamNone &&
       (gather_scales ? kblocks > 0 : as_sk == 1 && as_sm > 1 && kblocks > 1 && rows > kRelayoutMinRows)) {
     // row-major activation scales: re-lay them rows-contiguous in the workspace first (a few microseconds) so the
     // GEMM fetches 8 cache lines of scales per K step and tile instead of 256.  Up to 128 rows the extra launch costs
@@ -807,7 +893,7 @@ int run(const Problem& pr) {
     // the fused epilogue exists for the tile-list kernel (contiguous) and the 128 x 256 ring kernel (masked) only:
     // whole 128-blocks of K and of the output, a workspace for the list, no forced variant; anything else is the
     // caller's cue to run the GEMM and the activation apart
-    const bool kernel_ok = pr.mode == kContiguous ? rs.tile_list : pr.mode == kMasked && pl.variant == kVarPipe128x256w8;
+    const bool kernel_ok = pr.mode == kContiguous ? rs.tile_list : pr.mode == kMasked && (rs.stream != kStreamNone || pl.variant == kVarPipe128x256w8);
     if (!kernel_ok || pr.K % kScaleBlock != 0 || pr.N % (2 * kScaleBlock) != 0 || pr.N * pr.K >= (1ll << 32))
       return fail(DLB_ERR_BAD_SHAPE,
                   "fused activation needs K %% 128 == 0, N %% 256 == 0, N K < 2^32%s (N=%lld K=%lld)",
@@ -872,6 +958,7 @@ int run(const Problem& pr) {
   ar.fused_reduce = rs.fused ? 1 : 0;
   ar.spin_limit = g_knob[kKnobSpinLimit] > 0 ? g_knob[kKnobSpinLimit] - 1 : kDefaultSpinLimit;
   ar.sct_pitch = rs.sct_pitch;
+  ar.chunk_len = rs.chunk_len;
   const bool tile_list = rs.tile_list;
   const size_t esz = ar.out_f32 ? 4 : 2;
 
@@ -897,6 +984,13 @@ int run(const Problem& pr) {
         return launch_skinny(8, pl.sk_nfrags, pl.sk_waves, pl.sk_unroll, pl.sk_dma, ar, dev, pr.stream);
       default:
         break;
+    }
+    if (rs.stream != kStreamNone) {
+      ar.tiles_n = static_cast<int>(pr.act ? pr.N / 256 : ceil_div(pr.N, kStreamDims[rs.stream].bn));
+      const int64_t worst = static_cast<int64_t>(ar.tiles_n) * pr.G * ceil_div(pr.rows, kStreamDims[rs.stream].bm);
+      const int grid = static_cast<int>(ceil_div(worst < cus ? worst : cus, 32) * 32);  // tiles are dealt to the XCDs four at a time
+      return pr.act ? launch_stream_shape<kSiluQuantMasked, false>(rs.stream, ar, grid, dev, pr.stream)
+                    : launch_stream_shape<kStoreProduct, false>(rs.stream, ar, grid, dev, pr.stream);
     }
     const int g = static_cast<int>(rs.grid);
     const int g_dense = rs.resident ? cus : g;
@@ -1169,7 +1263,6 @@ int dlb_fp8_gemm_grouped_masked_silu_quant(const void* a, const void* b, const f
                                            int64_t N, int64_t K, int32_t G, int64_t as_stride_g, int64_t as_stride_m,
                                            int64_t as_stride_k, int64_t os_stride_g, int64_t os_stride_m, int64_t os_stride_k,
                                            float eps, void* workspace, size_t workspace_bytes, void* stream) {
-  (void)expected_m;
   dlb::Problem pr{dlb::kMasked, a, b, a_s, b_s, out_q, masked_m, M_max, N, K, G, as_stride_g, as_stride_m, as_stride_k,
                   DLB_OUT_BF16, workspace, workspace_bytes, static_cast<hipStream_t>(stream)};
   pr.act = true;
@@ -1178,6 +1271,7 @@ int dlb_fp8_gemm_grouped_masked_silu_quant(const void* a, const void* b, const f
   pr.act_s_sm = os_stride_m;
   pr.act_s_sk = os_stride_k;
   pr.act_eps = eps;
+  pr.hint_rows = expected_m;
   if (M_max > 0 && N > 0 && G > 0 && !out_s) return dlb::fail(DLB_ERR_NULL_POINTER, "out_s is NULL");
   return dlb::run(pr);
 }
@@ -1300,7 +1394,7 @@ int dlb_fp8_gemm_plan_grouped(int mode, int64_t rows, int64_t N, int64_t K, int3
   const dlb::Resolved rs = dlb::resolve(mode, rows, N, K, G, dlb::ceil_div(K, dlb::kScaleBlock), 1, workspace_bytes > 0, workspace_bytes,
                                         compute_units, false, false, mode == dlb::kMasked ? expected_m : -1);
   if (variant) *variant = rs.pl.variant;
-  if (tile_lists) *tile_lists = rs.tile_list ? 1 : 0;
+  if (tile_lists) *tile_lists = rs.tile_list || rs.stream != dlb::kStreamNone ? 1 : 0;
   return DLB_OK;
 }
 

@@ -74,6 +74,10 @@ struct Args {
   int64_t act_q_stride;
   int act_cols;
   float act_eps;
+  // weight-streaming grouped kernel (fp8_gemm_stream.h)
+  const int32_t* row_start;  // or NULL (masked layout): expert e owns rows [row_start[e], gidx[e])
+  int64_t a_src_rows;        // gathered activations: rows of a
+  int chunk_len;             // K blocks per chunk of its scale table
 };
 
 // Arithmetic shared by the activation kernels, the quantisers and the GEMM epilogue that fuses both, so that the

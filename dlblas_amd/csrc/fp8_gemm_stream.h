@@ -1,0 +1,418 @@
+// Weight-streaming grouped FP8 block-scaled GEMM for gfx950: experts with at most a few dozen rows each (decode steps,
+// short prefill chunks), where reading every expert's weights once from HBM is the whole cost.
+//
+// One persistent workgroup per CU walks its tiles with ONE LDS ring that runs on across tile boundaries: the DMA of the
+// next tile's first K blocks is issued STAGES - 1 steps ahead like any other, so a CU never drains its loads between two
+// tiles.  What the ring needs for that:
+//   - sources are addressed through buffer descriptors: a lane's byte offset (row x K + chunk) is the same for every tile,
+//     only scalar registers change with the tile, and rows past an expert's last one are out of the descriptor's range
+//     (the load returns zero and asks memory for nothing), so no per-tile address arithmetic sits in the issue path;
+//   - the epilogue leaves from the accumulator registers and never touches the ring;
+//   - activation scales go into a small double-buffered table in LDS, a chunk of K blocks at a time, by the same DMA
+//     queue: no re-layout launch, one line request per row and chunk; weight scales come through scalar loads.
+//
+// Measured (MI355X, 32 experts, against the 128 x 256 ring kernel it replaces there): gate/up + activation 4096 x 7168,
+// ~16 / ~32 rows per expert 186 -> 143 / 161 -> 148 us, down 7168 x 2048 97 -> 83 / 101 -> 91 us; 940 MB of weights at 4 rows
+// 138 us = 6.8 TB/s, i.e. 12 us + bytes at 7.5 TB/s.  Over 90 problems of 8 .. 32 experts, 512 .. 7168 weight rows and K, up
+// to 192 rows per expert: 1.26 x (geometric mean; the largest gains where 256-column tiles left CUs idle).  Above 192 rows
+// the ring kernels stay: row tiles of one expert drift apart there and fetch its weights twice (0 .. 256 rows, 7168 x 2048:
+// 127 against 134 us).
+//
+// Arithmetic: fp8_gemm_kernel of the reference (dlblas/kernels/fp8_gemm.py:49-60), same order of additions as the ring
+// kernels of fp8_gemm_pipelined.h, so results have the same bits.  Requires K % 128 == 0 and K / 128 >= STAGES - 1.
+#pragma once
+
+#include "fp8_gemm_common.h"
+#include "fp8_gemm_pipelined.h"
+
+namespace dlb {
+
+// What the epilogue does: store the product; silu(gate) * up + quantise with one rounding (expert-contiguous rows) or
+// with the masked activation's two (dlblas/kernels/moe.py:256-257).
+enum StreamEpilogue : int { kStoreProduct = 0, kSiluQuant = 1, kSiluQuantMasked = 2 };
+
+template <int WGM_, int WGN_, int MF_, int NF_, int STAGES_, int CH_>
+struct StreamCfg {
+  static constexpr int WGM = WGM_, WGN = WGN_, MF = MF_, NF = NF_, STAGES = STAGES_;
+  static constexpr int WAVES = WGM * WGN;
+  static constexpr int NT = WAVES * 64;
+  static constexpr int BM = WGM * MF * 32;
+  static constexpr int BN = WGN * NF * 32;
+  static constexpr int A_INST = BM / 8 / WAVES;
+  static constexpr int B_INST = BN / 8 / WAVES;
+  static constexpr int A_BYTES = BM * kScaleBlock;
+  static constexpr int B_BYTES = BN * kScaleBlock;
+  static constexpr int STAGE_BYTES = A_BYTES + B_BYTES;
+  static constexpr int L = A_INST + B_INST;  // vmcnt units per wave and step, scale chunks aside
+  static constexpr int CH = CH_;             // K blocks per chunk of the scale table, at most
+  static constexpr int PITCH = CH | 1;       // floats per table row (odd: 32 rows lie in 32 banks)
+  static constexpr int TAB_INST = (BM * PITCH + 64 * WAVES - 1) / (64 * WAVES);  // DMA instructions per wave and chunk
+  static constexpr int TAB_BYTES = TAB_INST * WAVES * 256;
+  static constexpr int TAB_OFF = STAGES * STAGE_BYTES;
+  static constexpr int ROW_OFF = TAB_OFF + 2 * TAB_BYTES;  // source rows of the issue tile (gathered activations)
+  static constexpr int MAX_OFF = ROW_OFF + BM * 4;         // row maxima of the waves (quantising epilogue)
+  static constexpr int LDS_BYTES = MAX_OFF + WGN * BM * 4;
+  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "tile rows must divide over the DMA instructions");
+  static_assert(WAVES % 2 == 0, "chunk swizzle must not depend on the DMA instruction index");
+  static_assert(L * (STAGES - 1) < 64, "vmcnt is a 6-bit counter");
+  static_assert(LDS_BYTES <= 160 * 1024, "ring, table and row maxima fit the LDS");
+};
+
+typedef const __attribute__((address_space(4))) float* const_float_ptr_t;
+
+template <int POLICY>
+__device__ __forceinline__ void buf_dma_16(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff, uint8_t* lds_dst) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)lds_dst, 16, voff, soff, 0, POLICY);
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const uint8_t* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, bytes, 0x00020000);
+}
+
+// Row ranges of the experts, 64 at a time: lane i of every wave holds expert first + i.
+struct ExpertWalk {
+  int first, base, total;  // first expert of the window, tiles before it, tiles in it
+  int row0, rows, mtiles, incl;
+};
+
+// GATHER: row r of the GEMM is row a_rows[r] of a and a_s.
+template <class Cfg, int EPI, bool GATHER>
+__global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) {
+  constexpr int BM = Cfg::BM, BN = Cfg::BN, MF = Cfg::MF, NF = Cfg::NF, WAVES = Cfg::WAVES, STAGES = Cfg::STAGES;
+  constexpr bool kAct = EPI != kStoreProduct;
+  static_assert(!kAct || BN == 256, "a quantisation group is the 128 output columns of 256 weight rows");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int l32 = lane & 31, h = lane >> 5;
+  const int wm0 = (wave / Cfg::WGN) * (MF * 32);
+  const int wn0 = (wave % Cfg::WGN) * (NF * 32);
+  const LaneChunks lc = make_lane_chunks(l32, h);
+  const int nk = p.kblocks;
+  const int grid = static_cast<int>(gridDim.x);
+  const int bid = static_cast<int>(blockIdx.x);
+  // the row tiles of an expert are adjacent in the order; of every 32 consecutive tiles an XCD takes 4 consecutive ones
+  const int slot0 = (bid / 32) * 32 + (bid % 8) * 4 + (bid / 8) % 4;
+
+  ExpertWalk ew;
+  auto load_window = [&](int first, int base) {
+    ew.first = first;
+    ew.base = base;
+    const int e = first + lane;
+    int row0 = 0, rows = 0;
+    if (e < p.G) {
+      if (p.row_start != nullptr) {
+        row0 = p.row_start[e];
+        rows = max(p.gidx[e] - row0, 0);
+      } else {
+        row0 = e * p.M;
+        rows = min(max(p.gidx[e], 0), p.M);
+      }
+    }
+    ew.row0 = row0;
+    ew.rows = rows;
+    ew.mtiles = (rows + BM - 1) / BM;
+    int incl = ew.mtiles * p.tiles_n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int up = __shfl_up(incl, off);
+      if (lane >= off) incl += up;
+    }
+    ew.incl = incl;
+    ew.total = __builtin_amdgcn_readlane(incl, 63);
+  };
+
+  // one tile: wave-uniform
+  struct Tile {
+    int g, row, rows, n0;  // expert, first row (of a / of the output), valid rows, first weight row / output column
+    bool ok;
+  };
+  auto locate = [&](int id) {
+    Tile t{};
+    while (id >= ew.base + ew.total) {
+      if (ew.first + 64 >= p.G) return t;
+      load_window(ew.first + 64, ew.base + ew.total);
+    }
+    const int rel = id - ew.base;
+    const int i = __builtin_ctzll(__ballot(ew.incl > rel));
+    const int mtiles = __builtin_amdgcn_readlane(ew.mtiles, i);
+    const int local = rel - (__builtin_amdgcn_readlane(ew.incl, i) - mtiles * p.tiles_n);
+    const int nt = local / mtiles, mt = local - nt * mtiles;
+    t.g = ew.first + i;
+    t.row = __builtin_amdgcn_readlane(ew.row0, i) + mt * BM;
+    t.rows = min(BM, __builtin_amdgcn_readlane(ew.rows, i) - mt * BM);
+    t.n0 = nt * (kAct ? BN / 2 : BN);
+    t.ok = true;
+    return t;
+  };
+
+  // ---- issue side --------------------------------------------------------------------------------------------------
+  const int dma_row = 8 * wave + (lane >> 3);
+  const uint32_t dma_chunk = static_cast<uint32_t>(((lane & 7) ^ chunk_swizzle(dma_row)) * 16);
+  const uint32_t uK = static_cast<uint32_t>(p.K);
+  uint32_t a_off[Cfg::A_INST], b_off[Cfg::B_INST];
+#pragma unroll
+  for (int j = 0; j < Cfg::A_INST; ++j) a_off[j] = static_cast<uint32_t>(dma_row + 8 * j * WAVES) * uK + dma_chunk;
+#pragma unroll
+  for (int j = 0; j < Cfg::B_INST; ++j) {
+    const int c = dma_row + 8 * j * WAVES;
+    // quantising epilogue: tile rows 0 .. 127 are gate rows, 128 .. 255 the up rows of the same output columns
+    b_off[j] = static_cast<uint32_t>(kAct && c >= BN / 2 ? p.act_cols + c - BN / 2 : c) * uK + dma_chunk;
+  }
+  int* rows_lds = reinterpret_cast<int*>(smem + Cfg::ROW_OFF);
+  // scale table: entry (row, j) of a chunk at row * tab_rs + j * tab_js; the side that is contiguous in a_s is the
+  // contiguous one here too, so that a DMA instruction moves whole runs
+  const bool tab_by_row = p.as_sk == 1;
+  const int tab_rs = tab_by_row ? Cfg::PITCH : 1, tab_js = tab_by_row ? 1 : BM;
+
+  Tile it;                      // the tile the issue side works on
+  int it_seq = 0, it_kb = 0;    // its number in this workgroup's sequence; its next K block
+  int it_stage = 0, it_tab = 0, it_chunk_kb = 0;
+  __amdgpu_buffer_rsrc_t a_src, b_src;
+  const float* as_src = nullptr;
+
+  auto enter_tile = [&]() {
+    it = locate(it_seq * grid + slot0);
+    ++it_seq;
+    it_kb = 0;
+    it_chunk_kb = 0;
+    if (!it.ok) return;
+    const uint8_t* bg = p.b + static_cast<int64_t>(it.g) * p.b_gs + static_cast<int64_t>(it.n0) * p.K;
+    b_src = make_rsrc(bg, static_cast<uint32_t>(kAct ? p.N - it.n0 : min(BN, p.N - it.n0)) * uK);
+    if (GATHER) {
+      a_src = make_rsrc(p.a, static_cast<uint32_t>(p.a_src_rows) * uK);
+      as_src = p.a_s;
+      // every wave fetches and writes the whole list itself (same values): no barrier
+      for (int r = lane; r < BM; r += 64) rows_lds[r] = r < it.rows ? max(p.a_rows[it.row + r], 0) : -1;
+#pragma unroll
+      for (int j = 0; j < Cfg::A_INST; ++j) {
+        const int src = rows_lds[dma_row + 8 * j * WAVES];
+        a_off[j] = src < 0 ? 0x80000000u : static_cast<uint32_t>(src) * uK + dma_chunk;  // 2^31: beyond the descriptor
+      }
+    } else {
+      a_src = make_rsrc(p.a + static_cast<int64_t>(it.row) * p.K, static_cast<uint32_t>(it.rows) * uK);
+      // masked layout: a_s has a group stride of its own; t.row counts rows of all experts
+      as_src = p.row_start != nullptr ? p.a_s + static_cast<int64_t>(it.row) * p.as_sm
+                                      : p.a_s + static_cast<int64_t>(it.g) * p.as_gs + static_cast<int64_t>(it.row - it.g * p.M) * p.as_sm;
+    }
+  };
+
+  auto issue_step = [&]() {
+    if (it.ok && it_kb == nk) enter_tile();
+    if (!it.ok) return;
+    uint8_t* sbase = smem + it_stage * Cfg::STAGE_BYTES;
+    if (it_kb == it_chunk_kb) {
+      // this step opens a chunk of the scale table
+      const int len = min(p.chunk_len, nk - it_kb);
+      uint8_t* tab = smem + Cfg::TAB_OFF + it_tab * Cfg::TAB_BYTES;
+#pragma unroll
+      for (int i = 0; i < Cfg::TAB_INST; ++i) {
+        const int e = (i * WAVES + wave) * 64 + lane;
+        int row = tab_by_row ? static_cast<int>((static_cast<float>(e) + 0.5f) * (1.0f / Cfg::PITCH)) : e % BM;
+        int j = tab_by_row ? e - row * Cfg::PITCH : e / BM;
+        row = min(row, it.rows - 1);
+        j = min(j, len - 1);
+        if (GATHER) row = rows_lds[row];
+        dma_4(reinterpret_cast<const uint8_t*>(as_src + static_cast<int64_t>(row) * p.as_sm + static_cast<int64_t>(it_kb + j) * p.as_sk), 0,
+              tab + (i * WAVES + wave) * 256);
+      }
+      it_tab ^= 1;
+      it_chunk_kb += p.chunk_len;
+    }
+    const uint32_t koff = static_cast<uint32_t>(it_kb) * kScaleBlock;
+#pragma unroll
+    for (int j = 0; j < Cfg::B_INST; ++j) buf_dma_16<kDmaStream>(b_src, b_off[j], koff, sbase + Cfg::A_BYTES + (j * WAVES + wave) * 1024);
+#pragma unroll
+    for (int j = 0; j < Cfg::A_INST; ++j) buf_dma_16<kDmaKeep>(a_src, a_off[j], koff, sbase + (j * WAVES + wave) * 1024);
+    ++it_kb;
+    it_stage = it_stage + 1 == STAGES ? 0 : it_stage + 1;
+  };
+
+  load_window(0, 0);
+  enter_tile();
+  if (!it.ok) return;
+  Tile ct = it;  // the tile the compute side works on
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s) issue_step();
+
+  // ---- compute side ------------------------------------------------------------------------------------------------
+  // A step reads its fragments when it needs them: the stream from HBM, not the matrix pipe, sets the pace here, and a
+  // wave whose rows are all past the expert's last one skips its reads.  (The software-pipelined loop of
+  // fp8_gemm_pipelined.h on the same ring, which reads and multiplies all 128 rows: 182 against 146 us at ~16 rows.)
+  int frag_off[NF];  // lane-dependent for the quantising epilogue
+#pragma unroll
+  for (int ni = 0; ni < NF; ++ni) {
+    // kAct: fragment rows 0 .. 15 are the gate rows of 16 output columns, 16 .. 31 their up rows.  l32 >= 16 then reads LDS
+    // row 128 + 16 f + (l32 - 16); row & 15 is the same, so the lane's swizzled chunk offsets hold
+    frag_off[ni] = Cfg::A_BYTES + (kAct ? ((wave % Cfg::WGN) * NF + ni) * 16 + (l32 >= 16 ? BN / 2 - 16 : 0) : wn0 + ni * 32) * kScaleBlock;
+  }
+  int stage = 0, tab = 0;
+  while (true) {
+    v16f acc[MF][NF];
+#pragma unroll
+    for (int mi = 0; mi < MF; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < NF; ++ni)
+#pragma unroll
+        for (int t = 0; t < 16; ++t) acc[mi][ni][t] = 0.f;
+    // weight scales of the wave's columns: one 128-block per wave (kAct: one for the gate, one for the up half)
+    const float* bs_g = p.b_s + static_cast<int64_t>(ct.g) * p.bs_gs;
+    const int nb0 = kAct ? ct.n0 / kScaleBlock : min((ct.n0 + wn0) / kScaleBlock, p.nblocks - 1);
+    const const_float_ptr_t bs0 = (const_float_ptr_t)(bs_g + static_cast<int64_t>(nb0) * nk);
+    const const_float_ptr_t bs1 = (const_float_ptr_t)(bs_g + static_cast<int64_t>(kAct ? nb0 + p.act_cols / kScaleBlock : nb0) * nk);
+    float sb0 = bs0[0], sb1 = bs1[0];
+    int chunk_end = 0, chunk_kb = 0;
+    const float* tab_ptr = nullptr;
+
+    for (int kb = 0; kb < nk; ++kb) {
+      // the loads of this step have landed: behind them at most the groups of the next STAGES - 2 steps are out
+      if (it.ok)
+        wait_vmcnt<(STAGES - 2) * Cfg::L>();
+      else
+        wait_vmcnt<0>();
+      lds_barrier();  // ... those of every wave, and nobody reads the stage before this one any more
+      issue_step();
+      if (kb == chunk_end) {
+        tab_ptr = reinterpret_cast<const float*>(smem + Cfg::TAB_OFF + tab * Cfg::TAB_BYTES);
+        tab ^= 1;
+        chunk_kb = kb;
+        chunk_end += p.chunk_len;
+      }
+      const int base = stage * Cfg::STAGE_BYTES;
+      if (BM == 32 || wm0 < ct.rows) {
+        v8i w[NF][2];
+#pragma unroll
+        for (int ni = 0; ni < NF; ++ni) {
+          w[ni][0] = lds_read_frag32(smem, base + frag_off[ni], lc, 0);
+          w[ni][1] = lds_read_frag32(smem, base + frag_off[ni], lc, 1);
+        }
+#pragma unroll
+        for (int mi = 0; mi < MF; ++mi) {
+          if (mi > 0 && wm0 + mi * 32 >= ct.rows) continue;  // no valid row in this fragment
+          const v8i x0 = lds_read_frag32(smem, base + (wm0 + mi * 32) * kScaleBlock, lc, 0);
+          const v8i x1 = lds_read_frag32(smem, base + (wm0 + mi * 32) * kScaleBlock, lc, 1);
+          const float sa = tab_ptr[(wm0 + mi * 32 + l32) * tab_rs + (kb - chunk_kb) * tab_js];
+          const float s0 = sa * sb0, s1 = sa * sb1;
+#pragma unroll
+          for (int ni = 0; ni < NF; ++ni) {
+            v16f z;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) z[u] = 0.f;
+            z = mfma_32x32x64_e4m3(w[ni][0], x0, z);
+            z = mfma_32x32x64_e4m3(w[ni][1], x1, z);
+#pragma unroll
+            for (int u = 0; u < 16; ++u) acc[mi][ni][u] = fmaf(z[u], kAct && u >= 8 ? s1 : s0, acc[mi][ni][u]);
+          }
+        }
+      }
+      const int kn = min(kb + 1, nk - 1);
+      sb0 = bs0[kn];
+      sb1 = bs1[kn];
+      stage = stage + 1 == STAGES ? 0 : stage + 1;
+    }
+
+    // ---- epilogue: lane holds rows wm0 + 32 mi + l32, weight rows 8 u + 4 h + 0..3 of every fragment, u = 0..3 -------
+    if constexpr (kAct) {
+      // u = 0, 1: gate, u = 2, 3: up of output columns c0 + 8 u + 4 h + 0..3.  The values pass through bf16 as the plain
+      // GEMM would have stored them, so codes and scales have the bits of the three separate steps.
+      float* maxima = reinterpret_cast<float*>(smem + Cfg::MAX_OFF);
+      float amax[MF];
+#pragma unroll
+      for (int mi = 0; mi < MF; ++mi) {
+        amax[mi] = 0.f;
+#pragma unroll
+        for (int ni = 0; ni < NF; ++ni)
+#pragma unroll
+          for (int t = 0; t < 8; ++t) {
+            const float gate = static_cast<float>(static_cast<__bf16>(acc[mi][ni][t]));
+            const float up = static_cast<float>(static_cast<__bf16>(acc[mi][ni][t + 8]));
+            float v;
+            if (EPI == kSiluQuantMasked)
+              v = static_cast<float>(static_cast<__bf16>(up * static_cast<float>(static_cast<__bf16>(act_silu_f32(gate)))));
+            else
+              v = static_cast<float>(static_cast<__bf16>(act_silu_f32(gate) * up));
+            acc[mi][ni][t] = v;
+            amax[mi] = fmaxf(amax[mi], fabsf(v));
+          }
+        amax[mi] = fmaxf(amax[mi], __shfl_xor(amax[mi], 32));
+        if (h == 0) maxima[(wave % Cfg::WGN) * BM + wm0 + mi * 32 + l32] = amax[mi];
+      }
+      lds_barrier();
+#pragma unroll
+      for (int mi = 0; mi < MF; ++mi) {
+        const int row = wm0 + mi * 32 + l32;
+#pragma unroll
+        for (int w2 = 0; w2 < Cfg::WGN; ++w2) amax[mi] = fmaxf(amax[mi], maxima[w2 * BM + row]);
+        const float scale = fmaxf(amax[mi], p.act_eps) / 448.0f;
+        const float inv_scale = 1.0f / scale;
+        // p.c / p.act_s are indexed by the row of all experts; the masked layout's scales have a group stride of their own
+        uint8_t* q_row = static_cast<uint8_t*>(p.c) + static_cast<int64_t>(ct.row + row) * p.act_q_stride + ct.n0;
+        const int64_t s_at = p.row_start != nullptr ? static_cast<int64_t>(ct.row + row) * p.act_s_sm
+                                                    : static_cast<int64_t>(ct.g) * p.act_s_gs + static_cast<int64_t>(ct.row + row - ct.g * p.M) * p.act_s_sm;
+        const bool live = row < ct.rows;
+        if (live && h == 0 && wave % Cfg::WGN == 0) p.act_s[s_at + static_cast<int64_t>(ct.n0 / kScaleBlock) * p.act_s_sk] = scale;
+#pragma unroll
+        for (int ni = 0; ni < NF; ++ni) {
+          int packed[2];
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            float c4[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              c4[j] = fminf(fmaxf(act_div_by_scale(acc[mi][ni][4 * u + j], scale, inv_scale), -448.0f), 448.0f);
+            int wd = __builtin_amdgcn_cvt_pk_fp8_f32(c4[0], c4[1], 0, false);
+            packed[u] = __builtin_amdgcn_cvt_pk_fp8_f32(c4[2], c4[3], wd, true);
+          }
+          // lanes l and l + 32 hold columns 0-3 and 4-7 (u = 0), 8-11 and 12-15 (u = 1): after the swap the lower one has
+          // columns 0-7, the upper one 8-15
+          const auto sw = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(packed[0]), static_cast<unsigned>(packed[1]), false, false);
+          if (live) *reinterpret_cast<v2i*>(q_row + ((wave % Cfg::WGN) * NF + ni) * 16 + 8 * h) = v2i{static_cast<int>(sw[0]), static_cast<int>(sw[1])};
+        }
+      }
+    } else {
+#pragma unroll
+      for (int mi = 0; mi < MF; ++mi) {
+        const int row = wm0 + mi * 32 + l32;
+        const bool live = row < ct.rows;
+        char* c_row = static_cast<char*>(p.c) + static_cast<int64_t>(ct.row + row) * p.N * (p.out_f32 ? 4 : 2);
+#pragma unroll
+        for (int ni = 0; ni < NF; ++ni) {
+          const int nf = ct.n0 + wn0 + ni * 32;
+          if (p.c_vec16) {
+            // bf16 rows that are 16-byte aligned: lanes l and l + 32 swap halves so that each stores 8 consecutive columns
+#pragma unroll
+            for (int u = 0; u < 4; u += 2) {
+              v2i lo, hi;
+              {
+                const v4f a4 = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
+                const v4f b4 = {acc[mi][ni][4 * u + 4], acc[mi][ni][4 * u + 5], acc[mi][ni][4 * u + 6], acc[mi][ni][4 * u + 7]};
+                lo = __builtin_bit_cast(v2i, __builtin_convertvector(a4, v4bf));
+                hi = __builtin_bit_cast(v2i, __builtin_convertvector(b4, v4bf));
+              }
+              const auto s0 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.x), static_cast<unsigned>(hi.x), false, false);
+              const auto s1 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.y), static_cast<unsigned>(hi.y), false, false);
+              const int n = nf + 8 * u + 8 * h;
+              if (live && n < p.N)
+                *reinterpret_cast<v4i*>(c_row + static_cast<int64_t>(n) * 2) =
+                    v4i{static_cast<int>(s0[0]), static_cast<int>(s1[0]), static_cast<int>(s0[1]), static_cast<int>(s1[1])};
+            }
+          } else if (live) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int n = nf + u * 8 + h * 4;
+              const v4f v = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
+              if (p.out_f32)
+                store_row4<true>(c_row, n, v, p.N - n, p.vec_store);
+              else
+                store_row4<false>(c_row, n, v, p.N - n, p.vec_store);
+            }
+          }
+        }
+      }
+    }
+    if (!it.ok) break;  // the issue side is one tile ahead: it has found no further one
+    ct = it;
+  }
+}
+
+}  // namespace dlb

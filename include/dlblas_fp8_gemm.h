@@ -213,9 +213,9 @@ int dlb_fp8_gemm_grouped_contiguous_gather_silu_quant(const void* a, const void*
  *                                             into a valid result nor written.  Values are clamped
  *                                             to [0, M_max].
  *   expected_m                                scheduling hint only (typical masked_m); <= 0 = unknown.
- *                                             It picks the tile shape (128 x 128 for a few short experts,
- *                                             256-row tiles from several hundred rows per expert on) and
- *                                             never changes a result bit.
+ *                                             It picks kernel and tile shape (the weight-streaming kernel while
+ *                                             twice the hint, or M_max, is at most 192 rows; 256-row tiles from
+ *                                             several hundred rows per expert on) and never changes a result bit.
  *
  * The tile schedule is built on the device from masked_m: no host synchronisation and no tiles
  * for empty row ranges.  K % 16 == 0 is required.
@@ -314,7 +314,8 @@ int dlb_fp8_gemm_plan(int mode, int64_t rows, int64_t N, int64_t K, size_t works
  * The same query for the grouped layouts with what their choice depends on besides the shape: the expert count and, for
  * the masked layout (mode 2), the caller's expected_m (<= 0: unknown).  mode 1 = contiguous (rows = M_sum), 2 = masked
  * (rows = M_max).  Outputs (each may be NULL): the kernel variant id; whether a contiguous launch of this size pairs
- * blocks into taller tiles from lists built on the device (1) or runs uniform 128-row tiles (0).  The fused gate/up
+ * blocks into taller tiles from lists built on the device (1) or runs uniform 128-row tiles (0); for the masked layout,
+ * whether the weight-streaming kernel for short experts runs in place of the named variant (1).  The fused gate/up
  * entry points always take the lists, so a caller that can also run GEMM and activation apart does that where this
  * says 0 (a batch of at most a round or two of tiles, where the uniform tiles are faster).  No counterpart in the
  * reference.
@@ -353,6 +354,8 @@ int dlb_fp8_gemm_force_variant(int variant);
  *   DLB_KNOB_TILE_LIST      expert-contiguous rows: 1 = 256- / 192- / 128-row tiles from lists built on the device
  *                           whenever a workspace allows it, 2 = uniform 128-row tiles (default: lists from more than two
  *                           rounds of 128 x 256 tiles on)
+ *   DLB_KNOB_STREAM         masked layout: 1 = never the weight-streaming kernel, 2 .. 6 = its tile shape 0 .. 4 (32 x 256,
+ *                           64 x 256, 64 x 128, 128 x 256, 64 x 64) wherever it applies (default: by size)
  *   DLB_KNOB_LDS_OVERSIZE   test hook: 1 = every kernel asks for more LDS than the GPU has, so the call is refused
  *                           (DLB_ERR_LAUNCH) before anything is enqueued
  */
@@ -370,6 +373,7 @@ int dlb_fp8_gemm_force_variant(int variant);
 #define DLB_KNOB_LDS_OVERSIZE 11
 #define DLB_KNOB_MASKED_GRID 12
 #define DLB_KNOB_TILE_LIST 13
+#define DLB_KNOB_STREAM 14
 int dlb_fp8_gemm_tune(int knob, int value);
 
 /* Name of kernel variant `variant`, or NULL beyond the last one. */
