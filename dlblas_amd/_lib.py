@@ -12,7 +12,7 @@ import torch
 
 from ._build import LIB_PATH
 
-ABI_VERSION = 7
+ABI_VERSION = 8
 OUT_BF16, OUT_F32 = 0, 1
 WS_COUNTER_BYTES = 65536
 WORKSPACE_BYTES = WS_COUNTER_BYTES + (32 << 20)
@@ -42,6 +42,10 @@ SYMBOLS = {
     (ctypes.c_int, [_c_vp] * 7 + [_c_i32] + [_c_i64] * 3 + [_c_i32] + [_c_i64] * 6 + [ctypes.c_float, _c_vp, _c_sz, _c_vp]),
     'dlb_fp8_gemm_grouped_masked':
     (ctypes.c_int, [_c_vp] * 6 + [_c_i32] + [_c_i64] * 3 + [_c_i32] + [_c_i64] * 3 + [ctypes.c_int, _c_vp, _c_sz, _c_vp]),
+    'dlb_fp8_gemm_grouped_ragged':
+    (ctypes.c_int, [_c_vp] * 7 + [_c_i32] + [_c_i64] * 3 + [_c_i32] + [_c_i64] * 2 + [ctypes.c_int, _c_vp]),
+    'dlb_fp8_gemm_grouped_ragged_silu_quant':
+    (ctypes.c_int, [_c_vp] * 9 + [_c_i64, _c_i32] + [_c_i64] * 3 + [_c_i32] + [_c_i64] * 4 + [ctypes.c_float, _c_vp]),
     'dlb_fp8_quant_1x128': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp, _c_vp] + [_c_i64] * 5 + [ctypes.c_float, _c_vp]),
     'dlb_fp8_quant_group': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp, _c_vp] + [_c_i64] * 6 + [ctypes.c_float, _c_vp]),
     'dlb_fp8_quant_128x128': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp, _c_vp] + [_c_i64] * 4 + [ctypes.c_float, _c_vp]),
@@ -63,6 +67,9 @@ SYMBOLS = {
     'dlb_ep_scatter_rows':
     (ctypes.c_int, [_c_vp, ctypes.c_int, _c_i64, _c_i64, _c_vp, _c_vp, ctypes.c_int, _c_vp, _c_vp, _c_i64, _c_vp, ctypes.c_int,
                     _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp, _c_sz, _c_vp]),
+    'dlb_ep_scatter_rows_host':
+    (ctypes.c_int, [_c_vp, ctypes.c_int, _c_i64, _c_i64] + [_c_vp] * 6 + [_c_i64, _c_vp, ctypes.c_int] + [_c_i64] * 5 +
+     [_c_vp, _c_sz, _c_vp]),
     'dlb_ep_gather':
     (ctypes.c_int, [_c_vp, ctypes.c_int, _c_i64, _c_vp, ctypes.c_int, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64, _c_vp, ctypes.c_int,
                     _c_i64, _c_i64, _c_vp, ctypes.c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp]),
@@ -421,6 +428,57 @@ def ep_scatter_rows(recv_topk, counts, expert_start_loc, m_indices, src_row, out
                                       _ptr(expert_start_loc), _idx_code(expert_start_loc), _ptr(m_indices), _ptr(src_row),
                                       m_indices.numel(), _ptr(output_index), _idx_code(output_index), output_index.stride(0),
                                       output_index.stride(1), T, topk, E, _ptr(ws), ws.numel(), ctypes.c_void_p(stream)))
+
+
+def ep_scatter_rows_host(recv_topk, counts, row_start, row_end, expert_start_loc, m_indices, src_row, output_index) -> bool:
+    """ep_scatter_rows with the reserved rows per expert as a Python list (they travel in the launch) and the row range of
+    every expert as further outputs.  False when the library wants the counts in device memory (nothing enqueued)."""
+    lib = load()
+    _require_gpu(recv_topk, row_start, row_end, expert_start_loc, m_indices, src_row, output_index)
+    T, topk = recv_topk.shape
+    E = len(counts)
+    host = (ctypes.c_int32 * E)(*counts)
+    with torch.cuda.device(recv_topk.device):
+        stream, ws = _stream_and_ws(recv_topk)
+        if lib.dlb_ep_scatter_workspace_bytes(T, topk, E) > ws.numel():
+            return False
+        rc = lib.dlb_ep_scatter_rows_host(_ptr(recv_topk), _idx_code(recv_topk), recv_topk.stride(0), recv_topk.stride(1), host,
+                                          _ptr(row_start), _ptr(row_end), _ptr(expert_start_loc), _ptr(m_indices), _ptr(src_row),
+                                          m_indices.numel(), _ptr(output_index), _idx_code(output_index), output_index.stride(0),
+                                          output_index.stride(1), T, topk, E, _ptr(ws), ws.numel(), ctypes.c_void_p(stream))
+    if rc == ERR_BAD_SHAPE:
+        return False
+    check(rc)
+    return True
+
+
+def gemm_ragged(a, b, a_s, b_s, c, row_start, row_end, expected_m) -> bool:
+    """dlb_fp8_gemm_grouped_ragged; False when the library declines the shape (nothing enqueued)."""
+    _require_gpu(a, b, a_s, b_s, c, row_start, row_end)
+    lib = load()
+    G, N, K = b.shape
+    with torch.cuda.device(a.device):
+        rc = lib.dlb_fp8_gemm_grouped_ragged(_ptr(a), _ptr(b), _ptr(a_s), _ptr(b_s), _ptr(c), _ptr(row_start), _ptr(row_end), expected_m,
+                                             a.size(0), N, K, G, a_s.stride(0), a_s.stride(1), out_code(c.dtype), _stream(a))
+    if rc == ERR_BAD_SHAPE:
+        return False
+    check(rc)
+    return True
+
+
+def gemm_ragged_silu_quant(a, b, a_s, b_s, out_q, out_s, row_start, row_end, a_row_index, expected_m, eps) -> bool:
+    """dlb_fp8_gemm_grouped_ragged_silu_quant (a_row_index: None or the source row of every GEMM row); False when declined."""
+    _require_gpu(a, b, a_s, b_s, out_q, out_s, row_start, row_end)
+    lib = load()
+    G, N, K = b.shape
+    with torch.cuda.device(a.device):
+        rc = lib.dlb_fp8_gemm_grouped_ragged_silu_quant(_ptr(a), _ptr(b), _ptr(a_s), _ptr(b_s), _ptr(out_q), _ptr(out_s), _ptr(row_start),
+                                                        _ptr(row_end), _ptr(a_row_index), a.size(0), expected_m, out_q.size(0), N, K, G,
+                                                        a_s.stride(0), a_s.stride(1), out_s.stride(0), out_s.stride(1), float(eps), _stream(a))
+    if rc == ERR_BAD_SHAPE:
+        return False
+    check(rc)
+    return True
 
 
 def ep_gather_args(inp, topk_ids, topk_weight, index, out):

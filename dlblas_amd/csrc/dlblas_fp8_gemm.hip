@@ -829,6 +829,94 @@ struct Problem {
 };
 
 
+// Expert-contiguous rows given as one range per expert (rows the ranges leave out are not touched), on the weight-streaming
+// kernel.  DLB_ERR_BAD_SHAPE, with nothing enqueued, where that kernel does not apply.
+struct RaggedProblem {
+  const void *a, *b;
+  const float *a_s, *b_s;
+  void* c;
+  const int32_t *row_start, *row_end;
+  const int32_t* a_rows;  // or NULL: row r is row a_rows[r] of a and a_s, which have a_src_rows rows
+  int64_t a_src_rows, M_sum, N, K;
+  int G;
+  int64_t hint_rows, as_sm, as_sk;
+  int out_dtype;
+  bool act;
+  float* act_s;
+  int64_t act_s_sm, act_s_sk;
+  float eps;
+  hipStream_t stream;
+};
+
+int run_ragged(const RaggedProblem& pr) {
+  clear_error();
+  if (pr.out_dtype != DLB_OUT_BF16 && pr.out_dtype != DLB_OUT_F32)
+    return fail(DLB_ERR_BAD_DTYPE, "out_dtype %d is neither DLB_OUT_BF16 nor DLB_OUT_F32", pr.out_dtype);
+  if (pr.M_sum < 0 || pr.N < 0 || pr.K < 0 || pr.G < 0 || pr.a_src_rows < 0)
+    return fail(DLB_ERR_BAD_SHAPE, "negative dimension (rows=%lld N=%lld K=%lld G=%d)", (long long)pr.M_sum, (long long)pr.N, (long long)pr.K, pr.G);
+  if (pr.M_sum == 0 || pr.N == 0 || pr.G == 0) return DLB_OK;
+  if (!pr.a || !pr.b || !pr.a_s || !pr.b_s || !pr.c || !pr.row_start || !pr.row_end || (pr.act && !pr.act_s))
+    return fail(DLB_ERR_NULL_POINTER, "a tensor pointer is NULL");
+  if (pr.as_sm < 0 || pr.as_sk < 0 || (pr.act && (pr.act_s_sm < 0 || pr.act_s_sk < 0))) return fail(DLB_ERR_BAD_STRIDE, "negative scale stride");
+  if (misaligned(pr.a, 16) || misaligned(pr.b, 16) || misaligned(pr.c, pr.act ? 8 : 2) || misaligned(pr.a_s, 4) || misaligned(pr.b_s, 4) ||
+      (pr.act && misaligned(pr.act_s, 4)))
+    return fail(DLB_ERR_ALIGNMENT, "a and b must be 16-byte aligned, c / out_q 2- / 8-byte, scales 4-byte");
+  int dev = 0;
+  const int cus = device_cu_count(&dev);
+  if (cus < 0) return fail(DLB_ERR_LAUNCH, "hipGetDevice failed");
+  const int64_t kblocks = ceil_div(pr.K, kScaleBlock);
+  int chunk_len = 0;
+  int shape = kStreamNone;
+  const bool fits = pr.K > 0 && pr.K % kScaleBlock == 0 && pr.K < (1ll << 24) && pr.as_sm < (1ll << 21) && pr.M_sum < (1ll << 31) &&
+                    pr.N < (1ll << 31) && (!pr.act || (pr.N % (2 * kScaleBlock) == 0 && pr.N * pr.K < (1ll << 32))) &&
+                    (!pr.a_rows || (pr.act && pr.a_src_rows > 0 && pr.a_src_rows * pr.K < (1ll << 31)));
+  if (fits) shape = pick_stream(pr.M_sum, pr.N, pr.K, pr.G, pr.hint_rows, pr.act, cus, &chunk_len);
+  if (shape == kStreamNone)
+    return fail(DLB_ERR_BAD_SHAPE, "the weight-streaming kernel does not take this problem (N=%lld K=%lld, about %lld rows per expert)",
+                (long long)pr.N, (long long)pr.K, (long long)pr.hint_rows);
+  Args ar;
+  memset(&ar, 0, sizeof(ar));
+  ar.a = static_cast<const uint8_t*>(pr.a);
+  ar.b = static_cast<const uint8_t*>(pr.b);
+  ar.a_s = pr.a_s;
+  ar.b_s = pr.b_s;
+  ar.c = pr.c;
+  ar.row_start = pr.row_start;
+  ar.gidx = pr.row_end;
+  ar.a_rows = pr.a_rows;
+  ar.a_src_rows = pr.a_src_rows;
+  ar.M = static_cast<int>(pr.M_sum);
+  ar.N = static_cast<int>(pr.N);
+  ar.K = static_cast<int>(pr.K);
+  ar.G = pr.G;
+  ar.kblocks = static_cast<int>(kblocks);
+  ar.nblocks = static_cast<int>(ceil_div(pr.N, kScaleBlock));
+  ar.as_sm = pr.as_sm;
+  ar.as_sk = pr.as_sk;
+  ar.b_gs = pr.N * pr.K;
+  ar.bs_gs = static_cast<int64_t>(ar.nblocks) * kblocks;
+  ar.chunk_len = chunk_len;
+  ar.tiles_n = static_cast<int>(pr.act ? pr.N / 256 : ceil_div(pr.N, kStreamDims[shape].bn));
+  ar.out_f32 = pr.out_dtype == DLB_OUT_F32;
+  ar.act_s = pr.act_s;
+  ar.act_s_sm = pr.act_s_sm;
+  ar.act_s_sk = pr.act_s_sk;
+  ar.act_eps = pr.eps;
+  ar.act_cols = static_cast<int>(pr.N / 2);
+  ar.act_q_stride = pr.N / 2;
+  ar.vec_store = (pr.N % 4 == 0) && !misaligned(pr.c, 4 * (ar.out_f32 ? 4 : 2));
+  ar.c_vec16 = !ar.out_f32 && pr.N % 8 == 0 && !misaligned(pr.c, 16);
+  const int64_t worst = static_cast<int64_t>(ar.tiles_n) * (pr.G + pr.M_sum / kStreamDims[shape].bm);
+  const int grid = static_cast<int>(ceil_div(worst < cus ? worst : cus, 32) * 32);
+  hipError_t e;
+  if (pr.act)
+    e = pr.a_rows ? launch_stream_shape<kSiluQuant, true>(shape, ar, grid, dev, pr.stream) : launch_stream_shape<kSiluQuant, false>(shape, ar, grid, dev, pr.stream);
+  else
+    e = launch_stream_shape<kStoreProduct, false>(shape, ar, grid, dev, pr.stream);
+  if (e != hipSuccess) return fail(DLB_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
+  return DLB_OK;
+}
+
 // Argument checks that need no device.  Returns DLB_OK with *empty set when there is nothing to compute.
 int check_problem(const Problem& pr, bool* empty) {
   g_err[0] = '\0';
@@ -1284,6 +1372,24 @@ int dlb_fp8_gemm_grouped_masked(const void* a, const void* b, const float* a_s, 
                   out_dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream)};
   pr.hint_rows = expected_m;
   return dlb::run(pr);
+}
+
+int dlb_fp8_gemm_grouped_ragged(const void* a, const void* b, const float* a_s, const float* b_s, void* c, const int32_t* row_start,
+                                const int32_t* row_end, int32_t expected_m, int64_t M_sum, int64_t N, int64_t K, int32_t G,
+                                int64_t as_stride_m, int64_t as_stride_k, int out_dtype, void* stream) {
+  dlb::RaggedProblem pr{a, b, a_s, b_s, c, row_start, row_end, nullptr, 0, M_sum, N, K, G, expected_m, as_stride_m, as_stride_k, out_dtype,
+                        false, nullptr, 0, 0, 0.f, static_cast<hipStream_t>(stream)};
+  return dlb::run_ragged(pr);
+}
+
+int dlb_fp8_gemm_grouped_ragged_silu_quant(const void* a, const void* b, const float* a_s, const float* b_s, void* out_q, float* out_s,
+                                           const int32_t* row_start, const int32_t* row_end, const int32_t* a_row_index,
+                                           int64_t a_rows, int32_t expected_m, int64_t M_sum, int64_t N, int64_t K, int32_t G,
+                                           int64_t as_stride_m, int64_t as_stride_k, int64_t os_stride_m, int64_t os_stride_k,
+                                           float eps, void* stream) {
+  dlb::RaggedProblem pr{a, b, a_s, b_s, out_q, row_start, row_end, a_row_index, a_rows, M_sum, N, K, G, expected_m, as_stride_m, as_stride_k,
+                        DLB_OUT_BF16, true, out_s, os_stride_m, os_stride_k, eps, static_cast<hipStream_t>(stream)};
+  return dlb::run_ragged(pr);
 }
 
 int dlb_fp8_quant_group(const void* x, int x_dtype, void* q, float* s, int64_t rows, int64_t K, int64_t group_size,

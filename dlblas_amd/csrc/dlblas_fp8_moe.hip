@@ -159,7 +159,16 @@ size_t dlb_ep_scatter_workspace_bytes(int64_t tokens, int64_t topk, int64_t expe
 
 namespace {
 
-// ep_scatter with its tables only (index_only: no row is moved, src_row names every destination row's token) or in full
+// What the tables-only form has besides the arguments of ep_scatter: src_row names every destination row's token; the
+// reserved rows may come from host memory.
+struct RowTables {
+  int32_t* src_row = nullptr;
+  int32_t* row_start = nullptr;
+  int32_t* row_end = nullptr;
+  bool host_counts = false;
+};
+
+// ep_scatter in full, or (tables) its tables only: no row is moved
 int scatter_impl(const void* recv_x, int64_t x_row_stride, const float* recv_x_scale, int64_t xs_stride_m,
                  int64_t xs_stride_k, const void* recv_topk, int topk_dtype, int64_t topk_stride_m,
                  int64_t topk_stride_k, const int32_t* num_recv_tokens_per_expert, void* expert_start_loc,
@@ -167,7 +176,8 @@ int scatter_impl(const void* recv_x, int64_t x_row_stride, const float* recv_x_s
                  int64_t os_stride_m, int64_t os_stride_k, int32_t* m_indices, int64_t m_indices_len,
                  void* output_index, int index_dtype, int64_t oi_stride_m, int64_t oi_stride_k, int64_t tokens,
                  int64_t hidden, int64_t topk, int64_t experts, void* workspace, size_t workspace_bytes,
-                 void* stream, int32_t* src_row, bool index_only) {
+                 void* stream, const RowTables* tables) {
+  const bool index_only = tables != nullptr;
   using namespace dlb;
   clear_error();
   if (bad_index_dtype(topk_dtype) || bad_index_dtype(start_dtype) || bad_index_dtype(index_dtype))
@@ -186,7 +196,9 @@ int scatter_impl(const void* recv_x, int64_t x_row_stride, const float* recv_x_s
   const bool has_entries = tokens > 0 && topk > 0;
   if (has_entries && (!recv_topk || !output_index)) return fail(DLB_ERR_NULL_POINTER, "recv_topk or output_index is NULL");
   if (index_only) {
-    if (m_indices_len > 0 && !src_row) return fail(DLB_ERR_NULL_POINTER, "src_row is NULL");
+    if (m_indices_len > 0 && !tables->src_row) return fail(DLB_ERR_NULL_POINTER, "src_row is NULL");
+    if (tables->host_counts && experts > kRowsInlineCounts)
+      return fail(DLB_ERR_BAD_SHAPE, "host counts are passed in the launch: at most %d experts, got %lld", kRowsInlineCounts, (long long)experts);
     if (tokens > (1ll << 31) - 1) return fail(DLB_ERR_BAD_SHAPE, "tokens=%lld does not fit the int32 row table", (long long)tokens);
   } else {
     if (has_entries && hidden > 0 && (!recv_x || !recv_x_scale || !output_tensor || !output_tensor_scale))
@@ -225,11 +237,23 @@ int scatter_impl(const void* recv_x, int64_t x_row_stride, const float* recv_x_s
   a.H = static_cast<int>(hidden), a.E = static_cast<int>(experts), a.topk_n = static_cast<int>(topk > 0 ? topk : 1);
   a.nblocks = scatter_blocks(a.T, a.topk_n, &a.tokens_per_block);
   a.topk_is64 = topk_dtype == DLB_IDX_I64, a.start_is64 = start_dtype == DLB_IDX_I64, a.oi_is64 = index_dtype == DLB_IDX_I64;
-  a.src_row = src_row;
-  a.index_only = index_only;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid(static_cast<unsigned>(a.nblocks)), block(kPermuteThreads);
   a.fused_scan = static_cast<int64_t>(a.nblocks) * a.E <= kFusedScanMaxInts;
+  RowsArgs ra;
+  const size_t rows_lds = (static_cast<size_t>(7) * a.E + 1) * sizeof(int);
+  if (tables) {
+    a.src_row = tables->src_row, a.row_start = tables->row_start, a.row_end = tables->row_end;
+    ra.inline_counts = tables->host_counts;
+    if (tables->host_counts) memcpy(ra.counts, num_recv_tokens_per_expert, experts * sizeof(int32_t));
+    ra.s = a;
+    if (a.T * a.topk_n <= kRowsOneLaunch) {
+      hipLaunchKernelGGL(ep_rows_kernel<kRowsAlone>, grid, dim3(kRowsThreads), rows_lds, st, ra);
+      return finish("ep_scatter_rows");
+    }
+    if (tables->host_counts && !a.fused_scan)
+      return fail(DLB_ERR_BAD_SHAPE, "%lld tokens x %lld experts need the reserved rows in device memory", (long long)tokens, (long long)experts);
+  }
   hipLaunchKernelGGL(ep_scatter_count_kernel, grid, block, static_cast<size_t>(a.E) * sizeof(int), st, a);
   if (int rc = finish("ep_scatter (count)")) return rc;
   if (!a.fused_scan) {
@@ -246,7 +270,14 @@ int scatter_impl(const void* recv_x, int64_t x_row_stride, const float* recv_x_s
     hipLaunchKernelGGL(ep_scatter_scan_kernel, dim3(1), dim3(kScanThreads), kScanTileInts * 4, st, a);
     if (int rc = finish("ep_scatter (scan)")) return rc;
   }
-  hipLaunchKernelGGL(ep_scatter_copy_kernel, grid, dim3(index_only ? kPermuteThreads : kCopyThreads), 0, st, a);
+  if (tables) {
+    if (a.fused_scan)
+      hipLaunchKernelGGL(ep_rows_kernel<kRowsSum>, grid, dim3(kRowsThreads), rows_lds, st, ra);
+    else
+      hipLaunchKernelGGL(ep_rows_kernel<kRowsScanned>, grid, dim3(kRowsThreads), rows_lds, st, ra);
+    return finish("ep_scatter_rows");
+  }
+  hipLaunchKernelGGL(ep_scatter_copy_kernel, grid, dim3(kCopyThreads), 0, st, a);
   return finish("ep_scatter (copy)");
 }
 
@@ -263,7 +294,7 @@ int dlb_ep_scatter(const void* recv_x, int64_t x_row_stride, const float* recv_x
   return scatter_impl(recv_x, x_row_stride, recv_x_scale, xs_stride_m, xs_stride_k, recv_topk, topk_dtype, topk_stride_m,
                       topk_stride_k, num_recv_tokens_per_expert, expert_start_loc, start_dtype, output_tensor, out_row_stride,
                       output_tensor_scale, os_stride_m, os_stride_k, m_indices, m_indices_len, output_index, index_dtype,
-                      oi_stride_m, oi_stride_k, tokens, hidden, topk, experts, workspace, workspace_bytes, stream, nullptr, false);
+                      oi_stride_m, oi_stride_k, tokens, hidden, topk, experts, workspace, workspace_bytes, stream, nullptr);
 }
 
 int dlb_ep_scatter_rows(const void* recv_topk, int topk_dtype, int64_t topk_stride_m, int64_t topk_stride_k,
@@ -271,9 +302,24 @@ int dlb_ep_scatter_rows(const void* recv_topk, int topk_dtype, int64_t topk_stri
                         int32_t* m_indices, int32_t* src_row, int64_t m_indices_len, void* output_index, int index_dtype,
                         int64_t oi_stride_m, int64_t oi_stride_k, int64_t tokens, int64_t topk, int64_t experts,
                         void* workspace, size_t workspace_bytes, void* stream) {
+  RowTables tables;
+  tables.src_row = src_row;
   return scatter_impl(nullptr, 0, nullptr, 0, 0, recv_topk, topk_dtype, topk_stride_m, topk_stride_k, num_recv_tokens_per_expert,
                       expert_start_loc, start_dtype, nullptr, 0, nullptr, 0, 0, m_indices, m_indices_len, output_index, index_dtype,
-                      oi_stride_m, oi_stride_k, tokens, 0, topk, experts, workspace, workspace_bytes, stream, src_row, true);
+                      oi_stride_m, oi_stride_k, tokens, 0, topk, experts, workspace, workspace_bytes, stream, &tables);
+}
+
+int dlb_ep_scatter_rows_host(const void* recv_topk, int topk_dtype, int64_t topk_stride_m, int64_t topk_stride_k,
+                             const int32_t* num_recv_tokens_per_expert_host, int32_t* row_start, int32_t* row_end,
+                             int32_t* expert_start_loc, int32_t* m_indices, int32_t* src_row, int64_t m_indices_len,
+                             void* output_index, int index_dtype, int64_t oi_stride_m, int64_t oi_stride_k, int64_t tokens,
+                             int64_t topk, int64_t experts, void* workspace, size_t workspace_bytes, void* stream) {
+  RowTables tables;
+  tables.src_row = src_row, tables.row_start = row_start, tables.row_end = row_end;
+  tables.host_counts = true;
+  return scatter_impl(nullptr, 0, nullptr, 0, 0, recv_topk, topk_dtype, topk_stride_m, topk_stride_k, num_recv_tokens_per_expert_host,
+                      expert_start_loc, DLB_IDX_I32, nullptr, 0, nullptr, 0, 0, m_indices, m_indices_len, output_index, index_dtype,
+                      oi_stride_m, oi_stride_k, tokens, 0, topk, experts, workspace, workspace_bytes, stream, &tables);
 }
 
 int dlb_ep_gather(const void* input, int in_dtype, int64_t in_row_stride, const void* recv_topk_ids, int topk_dtype,

@@ -45,8 +45,10 @@ struct ScatterArgs {
   int H, E, topk_n, tokens_per_block, nblocks;
   int topk_is64, start_is64, oi_is64;
   int fused_scan;  // the copy kernel derives the block's first rows from the raw histograms itself (no scan launch)
-  int32_t* src_row;  // [m_len] or NULL: source token of every destination row (0 for rows nobody is copied to)
-  int index_only;    // fill the tables only: no row of x or xs is moved
+  // tables only (ep_rows_kernel): no row of x or xs is moved
+  int32_t* src_row;    // [m_len]: source token of every destination row (0 for rows nobody is copied to)
+  int32_t* row_start;  // [E] or NULL: first row of every expert's span
+  int32_t* row_end;    // [E] or NULL: one past its last row that holds a slot, never beyond the span
 };
 
 // Expert id of entry `i` (token-major) of block `b`, or -1.
@@ -67,12 +69,6 @@ __global__ void __launch_bounds__(kPermuteThreads) ep_scatter_count_kernel(const
   if (id >= 0) atomicAdd(&hist[id], 1);
   __syncthreads();
   for (int e = threadIdx.x; e < p.E; e += kPermuteThreads) p.block_hist[static_cast<int64_t>(blockIdx.x) * p.E + e] = hist[e];
-  // rows that no slot is copied to (the padding of every expert's span) name token 0: any valid row will do for them,
-  // and this launch is ordered before the one that writes the real entries
-  if (p.src_row != nullptr)
-    for (int64_t r = static_cast<int64_t>(blockIdx.x) * kPermuteThreads + threadIdx.x; r < p.m_len;
-         r += static_cast<int64_t>(gridDim.x) * kPermuteThreads)
-      p.src_row[r] = 0;
 }
 
 // Pass 2 (one block of 1024): start_excl = exclusive prefix sum of counts; block_hist[b][e] becomes the first row
@@ -163,7 +159,7 @@ __global__ void __launch_bounds__(kCopyThreads) ep_scatter_copy_kernel(const Sca
   __shared__ int64_t base_l[kScanMaxExperts];      //             first row this block writes for every expert
   __shared__ int psum[kCopyThreads];
   const int tid = threadIdx.x;
-  const int nthreads = static_cast<int>(blockDim.x);  // kCopyThreads when rows are copied, kPermuteThreads for the tables only
+  constexpr int nthreads = kCopyThreads;
   const int b = blockIdx.x;
   int id = -1;
   if (tid < kPermuteThreads) {
@@ -218,7 +214,6 @@ __global__ void __launch_bounds__(kCopyThreads) ep_scatter_copy_kernel(const Sca
       d = (p.fused_scan ? base_l[id] : static_cast<int64_t>(p.block_hist[static_cast<int64_t>(b) * p.E + id])) + rank;
       const int64_t t = static_cast<int64_t>(b) * p.tokens_per_block + tid / p.topk_n;
       store_index(p.out_index, p.oi_is64, t * p.oi_s0 + (tid % p.topk_n) * p.oi_s1, d);
-      if (p.src_row != nullptr && d < p.m_len) p.src_row[d] = static_cast<int32_t>(t);
     }
     dest[tid] = d;
   }
@@ -243,7 +238,6 @@ __global__ void __launch_bounds__(kCopyThreads) ep_scatter_copy_kernel(const Sca
     }
   }
 
-  if (p.index_only) return;
   // copies: one wave per token; a lane loads up to 8 chunks of 16 bytes (8 KB per wave and trip) before it stores
   // them to the row of every routed slot
   const int lane = tid & 63, wave = tid >> 6;
@@ -279,6 +273,150 @@ __global__ void __launch_bounds__(kCopyThreads) ep_scatter_copy_kernel(const Sca
       }
     }
   }
+}
+
+// The tables of the scatter without its copy.  A block ranks its 256 entries by matching the expert ids inside a wave (one
+// ballot per id bit) on top of the counts of the waves before it.  What it has to know of the other blocks' entries:
+//   kRowsAlone: it reads the ids of every entry itself and counts them in LDS (up to kRowsOneLaunch entries: 4096 entries take
+//     6.2 us where the count launch and the summing launch took 4.2 + 18.6);
+//   kRowsSum: ep_scatter_count_kernel has left the blocks' histograms, and the rows of the blocks before (for the padding
+//     also behind) are added up 8 loads at a time (65536 entries: 15.3 -> 5.3 us against one dependent load after the other);
+//   kRowsScanned: many blocks; ep_scatter_scan_kernel has turned the histograms into first rows.
+// Reserved rows per expert come from p.counts or, when the host has them at hand, inside the launch (no upload).
+constexpr int kRowsThreads = 1024;
+enum RowsMode : int { kRowsAlone = 0, kRowsSum = 1, kRowsScanned = 2 };
+constexpr int kRowsOneLaunch = 16384;
+constexpr int kRowsInlineCounts = 256;
+
+struct RowsArgs {
+  ScatterArgs s;
+  int inline_counts;
+  int32_t counts[kRowsInlineCounts];
+};
+
+template <int MODE>
+__global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a) {
+  const ScatterArgs& p = a.s;
+  extern __shared__ int lds[];
+  const int E = p.E;
+  int* before = lds;              // [E] entries of earlier blocks
+  int* routed = before + E;       // [E] entries of all blocks
+  int* excl = routed + E;         // [E + 1] exclusive prefix sum of the reserved rows
+  int* wave_cnt = excl + E + 1;   // [4][E] entries of this block's first four waves
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int b = blockIdx.x;
+  for (int i = tid; i < 2 * E; i += kRowsThreads) lds[i] = 0;
+  for (int i = tid; i < 4 * E; i += kRowsThreads) wave_cnt[i] = 0;
+  __syncthreads();
+  auto reserved = [&](int e) { return max(a.inline_counts ? a.counts[e] : p.counts[e], 0); };
+  if (MODE == kRowsAlone) {
+    const int n = static_cast<int>(p.T) * p.topk_n;
+    const int mine = b * p.tokens_per_block * p.topk_n;
+    for (int i0 = tid; i0 < n; i0 += 4 * kRowsThreads) {
+      int id[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int i = i0 + u * kRowsThreads;
+        id[u] = -1;
+        if (i < n) {
+          const int64_t v = load_index(p.topk, p.topk_is64, static_cast<int64_t>(i / p.topk_n) * p.topk_s0 + (i % p.topk_n) * p.topk_s1);
+          if (v >= 0 && v < E) id[u] = static_cast<int>(v);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (id[u] >= 0) {
+          atomicAdd(&routed[id[u]], 1);
+          if (i0 + u * kRowsThreads < mine) atomicAdd(&before[id[u]], 1);
+        }
+    }
+  } else if (MODE == kRowsScanned) {
+    for (int e = tid; e < E; e += kRowsThreads) {
+      const int first = static_cast<int>(p.start_excl[e]);
+      before[e] = p.block_hist[static_cast<int64_t>(b) * E + e] - first;
+      routed[e] = static_cast<int>(load_index(p.start_loc, p.start_is64, e)) - first;
+    }
+  } else {
+    // thread (part, expert column): rows part, part + P, ... of the histogram matrix
+    const int cols = min(E, kRowsThreads), P = kRowsThreads / cols;
+    const int part = tid / cols;
+    for (int e = tid % cols; e < E && part < P; e += cols) {
+      int sum_before = 0, sum_all = 0;
+      for (int r0 = part; r0 < p.nblocks; r0 += 8 * P) {
+        int v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int r = r0 + u * P;
+          v[u] = r < p.nblocks ? p.block_hist[static_cast<int64_t>(r) * E + e] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          sum_all += v[u];
+          if (r0 + u * P < b) sum_before += v[u];
+        }
+      }
+      atomicAdd(&routed[e], sum_all);
+      atomicAdd(&before[e], sum_before);
+    }
+  }
+  if (wave == 4) {  // a wave with no entries of its own scans the reserved rows
+    int carry = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane;
+      const int c = e < E ? reserved(e) : 0;
+      int incl = c;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int up = __shfl_up(incl, off);
+        if (lane >= off) incl += up;
+      }
+      if (e < E) excl[e] = carry + incl - c;
+      carry += __shfl(incl, 63);
+    }
+    if (lane == 0) excl[E] = carry;
+  }
+  int id = -1, rank = 0;
+  if (wave < kPermuteThreads / 64) {
+    id = scatter_entry_id(p, b, tid);
+    uint64_t peers = __ballot(id >= 0);
+    for (int bit = 0; (1 << bit) < E; ++bit) {
+      const bool on = (id >> bit) & 1;
+      const uint64_t m = __ballot(on);
+      peers &= on ? m : ~m;
+    }
+    rank = __popcll(peers & ((1ull << lane) - 1));
+    if (id >= 0 && rank == 0) wave_cnt[wave * E + id] = __popcll(peers);
+  }
+  __syncthreads();
+  if (id >= 0) {
+    for (int w = 0; w < wave; ++w) rank += wave_cnt[w * E + id];
+    const int d = excl[id] + before[id] + rank;
+    const int64_t t = static_cast<int64_t>(b) * p.tokens_per_block + tid / p.topk_n;
+    store_index(p.out_index, p.oi_is64, t * p.oi_s0 + (tid % p.topk_n) * p.oi_s1, d);
+    if (d < p.m_len) p.src_row[d] = static_cast<int32_t>(t);
+  }
+  // rows [0, excl[E]) in slices over the blocks: their expert, and token 0 for the rows that no slot is given
+  const int total = static_cast<int>(min(static_cast<int64_t>(excl[E]), p.m_len));
+  const int per = (total + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x);
+  const int r1 = min(total, (b + 1) * per);
+  for (int r = b * per + tid; r < r1; r += kRowsThreads) {
+    int lo = 0, hi = E;  // largest e with excl[e] <= r
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (excl[mid] <= r)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    p.m_indices[r] = lo;
+    if (r >= excl[lo] + routed[lo]) p.src_row[r] = 0;
+  }
+  if (b == 0)
+    for (int e = tid; e < E; e += kRowsThreads) {
+      if (MODE != kRowsScanned) store_index(p.start_loc, p.start_is64, e, static_cast<int64_t>(excl[e]) + routed[e]);
+      if (p.row_start != nullptr) p.row_start[e] = excl[e];
+      if (p.row_end != nullptr) p.row_end[e] = min(excl[e] + routed[e], excl[e + 1]);
+    }
 }
 
 struct GatherArgs {

@@ -104,6 +104,11 @@ def ep_gather(
     return
 
 
+def _down(act, w2_weight_fp8, row_expert, out):
+    m_grouped_fp8_gemm_nt_contiguous(act, w2_weight_fp8, out, row_expert)
+    return out
+
+
 def fused_moe_v3(
     hidden_states_fp8: Tuple[torch.Tensor, torch.Tensor],
     topk_idx,
@@ -130,44 +135,58 @@ def fused_moe_v3(
 
     row_expert = buf((rows_total, ), torch.int32)
     slot_row = torch.empty_like(topk_idx)
-    per_expert = torch.tensor(num_recv_tokens_per_expert, dtype=torch.int32, pin_memory=True).to(dev, non_blocking=True)
-    first_row = torch.empty_like(per_expert)
+    n_experts = len(num_recv_tokens_per_expert)
+    down = None
 
     # gate/up projection, silu(gate) * up and the 1 x 128 quantiser as one kernel that reads the tokens where they lie:
-    # ep_scatter_rows only fills the tables (which expert and which token each sorted row stands for), the kernel
-    # follows them, and neither the expert-sorted copy of the activations nor the bf16 [rows, 2 I] intermediate reaches
-    # memory.  Same bits as the steps of the reference (:288-334).
-    # (A batch of at most a round or two of tiles runs faster on uniform 128-row tiles, which have no fused epilogue:
-    # the library's planner says which, and such a batch takes the three steps below.)
-    fused = None
-    want_fused = _lib.plan_grouped(1, rows_total, inter2, hidden, w13_weight_fp8[0].size(0))[1]
-    if want_fused and tokens_q.is_contiguous() and hidden % 128 == 0 and inter2 % 256 == 0 and n_tokens * hidden < (1 << 32):
-        row_token = buf((rows_total, ), torch.int32)
-        ep_scatter_rows(topk_idx, per_expert, first_row, row_expert, row_token, slot_row)
-        fused = fp8_gemm_grouped_contiguous_silu_quant(tokens_q, tokens_scale, w13_weight_fp8[0], w13_weight_fp8[1], row_expert,
-                                                       column_major_scales=True,  # the layout the down GEMM reads in place
-                                                       a_row_index=row_token)
-    if fused is not None:
-        act_q, act_scale = fused
-    else:
+    # the row tables say which expert and which token each sorted row stands for, the kernel follows them, and neither
+    # the expert-sorted copy of the activations nor the bf16 [rows, 2 I] intermediate reaches memory.  Same bits as the
+    # steps of the reference (:288-334).
+    direct = tokens_q.is_contiguous() and hidden % 128 == 0 and inter2 % 256 == 0 and n_tokens * hidden < (1 << 31)
+    if direct and n_experts <= 256:
+        # A short batch - a block or so of rows per expert, most of them padding - is a matter of reading the experts'
+        # weights once: the weight-streaming kernels, on the rows that hold a token (500 tokens, 32 experts of 7168 x 2048:
+        # 333 -> 245 us).  A long one pairs the blocks of an expert into taller tiles.  In between, where the library's
+        # planner prefers uniform 128-row tiles, which have no fused epilogue, the three steps below are the faster way.
+        used = sum(1 for c in num_recv_tokens_per_expert if c > 0)
+        rows_each = max(1, min(rows_total // used - 64, -(-n_tokens * topk_idx.size(1) // used)))  # half a block of padding on average
+        streams = (_lib.plan_grouped(2, rows_total, inter2, hidden, n_experts, rows_each)[1]
+                   and _lib.plan_grouped(2, rows_total, hidden, inter2 // 2, n_experts, rows_each)[1])
+        if streams or _lib.plan_grouped(1, rows_total, inter2, hidden, n_experts)[1]:
+            row_token = buf((rows_total, ), torch.int32)
+            ranges = buf((3, n_experts), torch.int32)
+            if _lib.ep_scatter_rows_host(topk_idx, num_recv_tokens_per_expert, ranges[0], ranges[1], ranges[2], row_expert, row_token,
+                                         slot_row):
+                down = buf((rows_total, hidden), torch.bfloat16)
+                act_q = buf((rows_total, inter2 // 2), torch.float8_e4m3fn)
+                act_scale = buf((rows_total, inter2 // 256), torch.float32)
+                if not (streams
+                        and _lib.gemm_ragged_silu_quant(tokens_q, w13_weight_fp8[0], tokens_scale, w13_weight_fp8[1], act_q, act_scale,
+                                                        ranges[0], ranges[1], row_token, rows_each, 1e-10)
+                        and _lib.gemm_ragged(act_q, w2_weight_fp8[0], act_scale, w2_weight_fp8[1], down, ranges[0], ranges[1], rows_each)):
+                    fused = fp8_gemm_grouped_contiguous_silu_quant(tokens_q, tokens_scale, w13_weight_fp8[0], w13_weight_fp8[1],
+                                                                   row_expert, column_major_scales=True,  # what the down GEMM reads in place
+                                                                   a_row_index=row_token)
+                    down = _down(fused, w2_weight_fp8, row_expert, down) if fused is not None else None
+    if down is None:
         # Expert-sorted activations.  The spans are padded to 128 rows per expert; the padding rows keep whatever the
         # allocator hands out, as in the reference driver (:269-278).  The GEMMs and the quantiser treat every row on its
         # own, so what those rows turn into (NaN included) stays in rows that ep_gather never reads.
+        per_expert = torch.tensor(num_recv_tokens_per_expert, dtype=torch.int32, pin_memory=True).to(dev, non_blocking=True)
+        first_row = torch.empty_like(per_expert)
         sorted_q = buf((rows_total, hidden), torch.uint8).view(tokens_q.dtype)
         sorted_scale = buf((rows_total, hidden // 128), torch.float32)
         ep_scatter(tokens_q, tokens_scale, topk_idx, per_expert, first_row, sorted_q, sorted_scale, row_expert, slot_row)
-        if want_fused:
+        fused = None
+        if _lib.plan_grouped(1, rows_total, inter2, hidden, w13_weight_fp8[0].size(0))[1]:
             fused = fp8_gemm_grouped_contiguous_silu_quant(sorted_q, sorted_scale, w13_weight_fp8[0], w13_weight_fp8[1], row_expert,
                                                            column_major_scales=True)
-        if fused is not None:
-            act_q, act_scale = fused
-        else:  # the three steps of the reference (:307-334)
+        if fused is None:  # the three steps of the reference (:307-334)
             gate_up = buf((rows_total, inter2), torch.bfloat16)
             m_grouped_fp8_gemm_nt_contiguous((sorted_q, sorted_scale), w13_weight_fp8, gate_up, row_expert)
-            act_q, act_scale = silu_and_mul_post_quant(gate_up, 128)
+            fused = silu_and_mul_post_quant(gate_up, 128)
             del gate_up
-    down = buf((rows_total, hidden), torch.bfloat16)
-    m_grouped_fp8_gemm_nt_contiguous((act_q, act_scale), w2_weight_fp8, down, row_expert)
+        down = _down(fused, w2_weight_fp8, row_expert, buf((rows_total, hidden), torch.bfloat16))
 
     combined = buf((n_tokens, hidden), torch.bfloat16)
     ep_gather(down, topk_idx, topk_weights, slot_row, combined)

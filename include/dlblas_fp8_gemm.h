@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define DLB_ABI_VERSION 7
+#define DLB_ABI_VERSION 8
 
 /* output element type of C */
 #define DLB_OUT_BF16 0
@@ -249,6 +249,33 @@ int dlb_fp8_gemm_grouped_masked_silu_quant(const void* a, const void* b, const f
                                            int64_t as_stride_g, int64_t as_stride_m, int64_t as_stride_k,
                                            int64_t os_stride_g, int64_t os_stride_m, int64_t os_stride_k, float eps,
                                            void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * Grouped GEMM over expert-contiguous rows given as one row range per expert: rows [row_start[e], row_end[e]) (int32 on the
+ * device, as dlb_ep_scatter_rows_host leaves them) of a, a_s and c belong to expert e.  Unlike m_indices the ranges say
+ * which rows of an expert's padded span hold a token, so the padding is neither read nor multiplied nor written.  For short
+ * experts (expected_m = typical rows per expert, <= 96 or so): the work is reading every expert's weights once.
+ *
+ *   a [M_sum, K], b [G, N, K], a_s, b_s, c [M_sum, N], out_dtype   as dlb_fp8_gemm_grouped_contiguous
+ *
+ * DLB_ERR_BAD_SHAPE, nothing enqueued: K is no multiple of 128, or the experts are too long for this path; the caller then
+ * uses dlb_fp8_gemm_grouped_contiguous.  Same bits as that call.
+ */
+int dlb_fp8_gemm_grouped_ragged(const void* a, const void* b, const float* a_s, const float* b_s, void* c, const int32_t* row_start,
+                                const int32_t* row_end, int32_t expected_m, int64_t M_sum, int64_t N, int64_t K, int32_t G,
+                                int64_t as_stride_m, int64_t as_stride_k, int out_dtype, void* stream);
+
+/*
+ * The gate/up projection on such ranges with silu(gate) * up and the 1 x 128 quantiser in its epilogue: the outputs of
+ * dlb_fp8_gemm_grouped_contiguous_silu_quant (a_row_index NULL) or of its gathering form (a_row_index [M_sum]: row r is row
+ * a_row_index[r] of a and a_s, which have a_rows rows; a_rows * K < 2^31) on the rows of the ranges, same bits.  Declined
+ * like dlb_fp8_gemm_grouped_ragged.
+ */
+int dlb_fp8_gemm_grouped_ragged_silu_quant(const void* a, const void* b, const float* a_s, const float* b_s, void* out_q, float* out_s,
+                                           const int32_t* row_start, const int32_t* row_end, const int32_t* a_row_index,
+                                           int64_t a_rows, int32_t expected_m, int64_t M_sum, int64_t N, int64_t K, int32_t G,
+                                           int64_t as_stride_m, int64_t as_stride_k, int64_t os_stride_m, int64_t os_stride_k,
+                                           float eps, void* stream);
 
 /* element type of the quantiser input */
 #define DLB_IN_BF16 0

@@ -110,6 +110,19 @@ int dlb_ep_scatter_rows(const void* recv_topk, int topk_dtype, int64_t topk_stri
                         void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * dlb_ep_scatter_rows for callers that have the reserved rows per expert in HOST memory (fused_moe_v3 is given a list):
+ * they travel in the launch itself, so nothing is uploaded; at most 256 experts.  Also leaves the row range of every
+ * expert, [row_start[e], row_end[e]) int32 = the rows that hold a slot, clipped to the expert's reserved span (either may be
+ * NULL): the form dlb_fp8_gemm_grouped_ragged takes.  DLB_ERR_BAD_SHAPE (nothing enqueued): more experts, or so many tokens
+ * that the tables need the scan launch; the caller then uploads the counts and uses dlb_ep_scatter_rows.
+ */
+int dlb_ep_scatter_rows_host(const void* recv_topk, int topk_dtype, int64_t topk_stride_m, int64_t topk_stride_k,
+                             const int32_t* num_recv_tokens_per_expert_host, int32_t* row_start, int32_t* row_end,
+                             int32_t* expert_start_loc, int32_t* m_indices, int32_t* src_row, int64_t m_indices_len,
+                             void* output_index, int index_dtype, int64_t oi_stride_m, int64_t oi_stride_k, int64_t tokens,
+                             int64_t topk, int64_t experts, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * out[t, :] = sum over the slots j with recv_topk_ids[t, j] >= 0, in slot order, of
  * input[input_index[t, j], :] * recv_topk_weight[t, j]; fp32 fused multiply-add chain, one cast at the end; a token
  * without a routed slot gets zeros.  Replaces ep_gather (dlblas/kernels/fused_moe_v3.py:199-233; kernel :161-196).

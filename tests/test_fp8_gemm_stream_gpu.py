@@ -88,3 +88,84 @@ def test_masked_activation_equals_the_ring_kernel(dev, masked, M_max, inter, K):
         outs.append((q, s))
     for q, s in outs[1:]:
         assert torch.equal(q, outs[0][0]) and torch.equal(s, outs[0][1])
+
+
+@pytest.mark.parametrize('T,K,inter,E,topk,shape', [
+    (96, 512, 256, 4, 2, '32x256'),
+    (250, 1024, 384, 8, 4, '128x256'),    # up to two row tiles per expert
+    (40, 2176, 128, 70, 3, '64x256'),     # experts without a token; a second window of experts
+])
+def test_ragged_rows_equal_the_contiguous_kernels(dev, T, K, inter, E, topk, shape):
+    """Row ranges instead of m_indices, rows gathered through the token table: the bytes, scales and products of the
+    expert-contiguous kernels on every row that holds a token; rows no range names keep their content."""
+    from dlblas_amd import _lib
+    from dlblas_amd.kernels.fp8_gemm_grouped import fp8_gemm_grouped_contiguous_silu_quant, m_grouped_fp8_gemm_nt_contiguous
+    print(f'case ragged T={T} K={K} I={inter} E={E} topk={topk} {shape}', flush=True)
+    g = helpers.gen(300 + T)
+    x_q, x_s = orc.quant_act_1x128((torch.randn(T, K, generator=g) * 1.5).to(torch.bfloat16))
+    quant = lambda n, k: [orc.quant_weight_128x128((torch.randn(n, k, generator=g) * 0.05).to(torch.bfloat16)) for _ in range(4)]
+    stack = lambda ws: tuple(torch.stack([ws[e % 4][i] for e in range(E)]).to(dev) for i in (0, 1))
+    (w13_q, w13_s), (w2_q, w2_s) = stack(quant(2 * inter, K)), stack(quant(256, inter))
+    ids = torch.randint(-1, E, (T, topk), generator=g)
+    routed = torch.bincount(ids[ids >= 0], minlength=E)
+    counts = ((routed + 127) // 128 * 128).tolist()
+    rows = sum(counts)
+    i32 = lambda *s: torch.full(s, -9, dtype=torch.int32, device=dev)
+    start, end, first, m_indices, row_token, slot = i32(E), i32(E), i32(E), i32(rows), i32(rows), torch.full_like(ids, -9, device=dev)
+    assert _lib.ep_scatter_rows_host(ids.to(dev), counts, start, end, first, m_indices, row_token, slot)
+    excl = torch.cumsum(torch.tensor([0] + counts[:-1]), 0)
+    assert torch.equal(start.cpu().long(), excl) and torch.equal(end.cpu().long(), excl + routed) and torch.equal(first, end)
+    x_q, x_s = x_q.to(dev), x_s.to(dev)
+    ref_q, ref_s = fp8_gemm_grouped_contiguous_silu_quant(x_q, x_s, w13_q, w13_s, m_indices, a_row_index=row_token)
+    _lib.tune('stream', 2 + SHAPES.index(shape))
+    q = torch.full((rows, inter), 0x5a, dtype=torch.uint8, device=dev).view(torch.float8_e4m3fn)
+    s = torch.full((rows, inter // 128), -7.0, device=dev)
+    assert _lib.gemm_ragged_silu_quant(x_q, w13_q, x_s, w13_s, q, s, start, end, row_token, 64, 1e-10)
+    sorted_q, sorted_s = x_q.view(torch.uint8)[row_token.long()].view(torch.float8_e4m3fn), x_s[row_token.long()]
+    q2, s2 = torch.zeros_like(q), torch.zeros_like(s)
+    assert _lib.gemm_ragged_silu_quant(sorted_q, w13_q, sorted_s, w13_s, q2, s2, start, end, None, 64, 1e-10)
+    row = torch.arange(rows, device=dev)
+    held = ((row[None] >= start[:, None]) & (row[None] < end[:, None])).any(0)
+    torch.cuda.synchronize()
+    for got_q, got_s in ((q, s), (q2, s2)):
+        assert torch.equal(got_q.view(torch.uint8)[held], ref_q.view(torch.uint8)[held]) and torch.equal(got_s[held], ref_s[held])
+    assert (s[~held] == -7.0).all() and (q.view(torch.uint8)[~held] == 0x5a).all()
+    if inter % 256 == 0 or inter == 128 and shape != '128x256':
+        out = torch.full((rows, 256), -555.0, dtype=torch.bfloat16, device=dev)
+        if _lib.gemm_ragged(q, w2_q, s, w2_s, out, start, end, 64):
+            ref = torch.zeros(rows, 256, dtype=torch.bfloat16, device=dev)
+            m_grouped_fp8_gemm_nt_contiguous((ref_q, ref_s), (w2_q, w2_s), ref, m_indices)
+            torch.cuda.synchronize()
+            assert torch.equal(out[held], ref[held]) and (out[~held] == -555.0).all()
+
+
+@pytest.mark.parametrize('T,topk,E', [(1, 1, 1), (33, 8, 32), (2048, 8, 32), (2049, 8, 300), (5000, 64, 7)])
+def test_row_tables_around_the_one_launch_limit(dev, T, topk, E):
+    """16384 entries are the most that one launch ranks by itself; expert counts that are no power of two; token counts
+    that leave the last block short."""
+    from dlblas_amd.kernels.fused_moe_v3 import ep_scatter_rows
+    print(f'case row tables T={T} topk={topk} E={E}', flush=True)
+    g = helpers.gen(T + E)
+    ids = torch.randint(-2, E, (T, topk), generator=g)
+    flat = ids.flatten()
+    routed = torch.bincount(flat[flat >= 0], minlength=E)
+    counts = (routed + 127) // 128 * 128
+    rows = int(counts.sum())
+    i32 = lambda n: torch.full((n, ), -9, dtype=torch.int32, device=dev)
+    first, m_indices, src, slot = i32(E), i32(rows), i32(rows), torch.full_like(ids, -9, device=dev)
+    ep_scatter_rows(ids.to(dev), counts.to(torch.int32).to(dev), first, m_indices, src, slot)
+    torch.cuda.synchronize()
+    excl = torch.cumsum(counts, 0) - counts
+    order = torch.sort(flat, stable=True)
+    rank = torch.empty_like(flat)
+    n_none = int((flat < 0).sum())
+    cum = torch.cumsum(routed, 0) - routed
+    pos = torch.arange(flat.numel()) - n_none
+    dest = torch.where(order.values >= 0, excl[order.values.clamp(min=0)] + pos - cum[order.values.clamp(min=0)], torch.full_like(pos, -9))
+    rank[order.indices] = dest
+    assert torch.equal(slot.cpu().flatten(), rank)
+    assert torch.equal(first.cpu().long(), excl + routed)
+    assert torch.equal(m_indices.cpu().long(), torch.repeat_interleave(torch.arange(E), counts))
+    src_ref = torch.zeros(rows, dtype=torch.long)
+    src_ref[rank[flat >= 0]] = (torch.arange(flat.numel()) // topk)[flat >= 0]
+    assert torch.equal(src.cpu().long(), src_ref)
