@@ -1,0 +1,35 @@
+"""The entry points as native calls (csrc/host_calls.cpp): ``_fast.fp8_gemm(a, b, a_s, b_s)`` and so on return the result of
+the Python function of that name, or None without having done anything when the call is not a plain one; the Python function
+then takes its own path.  The module is loaded at the first use; ImportError when it has not been built."""
+import importlib.util
+import os
+
+from . import _lib
+from ._build import HOST_PATH
+
+# the library's entry points in the order of the Abi struct in csrc/host_calls.cpp
+_ABI = ('dlb_last_error', 'dlb_fp8_gemm', 'dlb_fp8_gemm_grouped_contiguous', 'dlb_fp8_gemm_grouped_contiguous_gather_silu_quant',
+        'dlb_fp8_gemm_grouped_masked', 'dlb_fp8_gemm_grouped_masked_silu_quant', 'dlb_fp8_gemm_grouped_ragged',
+        'dlb_fp8_gemm_grouped_ragged_silu_quant', 'dlb_fp8_gemm_plan_grouped', 'dlb_fp8_gemm_variant_name', 'dlb_fp8_quant_group',
+        'dlb_silu_mul_quant_masked', 'dlb_ep_scatter_workspace_bytes', 'dlb_ep_scatter_rows_host', 'dlb_ep_gather')
+
+
+def _load():
+    import ctypes
+    lib = _lib.load()
+    if not os.path.exists(HOST_PATH):
+        raise ImportError(f'{HOST_PATH} has not been built; run `python -m dlblas_amd._build` (needs hipcc)')
+    spec = importlib.util.spec_from_file_location('dlblas_amd._host', HOST_PATH)
+    host = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(host)
+    host.init([ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _ABI], _lib.workspace)
+    return host
+
+
+def __getattr__(name):
+    if name.startswith('_'):
+        raise AttributeError(name)
+    host = _load()
+    for fn in ('fp8_gemm', 'quant', 'grouped_contiguous', 'grouped_masked', 'low_latency_experts', 'ep_gather', 'fused_moe_v3'):
+        globals()[fn] = getattr(host, fn)
+    return globals()[name]

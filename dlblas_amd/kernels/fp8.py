@@ -9,7 +9,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from .. import _lib
+from .. import _fast, _lib
 from ..utils import SymVar, Tensor, register_dlblas_op
 
 
@@ -34,6 +34,10 @@ def per_token_group_quant_fp8(
     Returns ``(x_q, x_s)``: ``x_q`` like ``x`` in fp8, ``x_s`` fp32 ``[..., K / group_size]`` (a column-major view
     when ``column_major_scales``), with ``x_s = max(amax, eps) / 448`` per group.
     """
+    if dtype is torch.float8_e4m3fn and not torch.compiler.is_compiling():
+        qs = _fast.quant(x, group_size, eps, column_major_scales)
+        if qs is not None:
+            return qs
     assert (x.shape[-1] % group_size == 0), (
         f"the last dimension of 'x' {x.shape[-1]} must be divisible by 'group_size' {group_size}")
     assert x.stride(-1) == 1, f'{x} groups must be contiguous'

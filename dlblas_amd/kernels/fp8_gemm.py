@@ -8,7 +8,7 @@ never registers, dlblas/kernels/fp8_gemm.py:10).
 """
 import torch
 
-from .. import _lib
+from .. import _fast, _lib
 from ..utils import SymVar, Tensor, register_dlblas_op
 
 BLOCK = 128  # K extent of one activation scale, K and N extent of one weight scale
@@ -69,6 +69,10 @@ def fp8_gemm(a: torch.Tensor, b: torch.Tensor, a_s: torch.Tensor, b_s: torch.Ten
     Returns:
         ``[..., N]`` in ``torch.get_default_dtype()``, newly allocated, enqueued on the current stream.
     """
+    if not torch.compiler.is_compiling():
+        c = _fast.fp8_gemm(a, b, a_s, b_s)
+        if c is not None:
+            return c
     _check_dense(a, b, a_s, b_s)
     return fp8_gemm_op(a, b, a_s, b_s, torch.get_default_dtype())
 

@@ -9,7 +9,7 @@ from typing import Sequence
 
 import torch
 
-from .. import _lib
+from .. import _fast, _lib
 from ..utils import SymVar, Tensor, register_dlblas_op
 
 BLOCK = 128
@@ -60,6 +60,8 @@ def fp8_gemm_grouped_contiguous(a, a_s, w, w_s, out, m_indices):
     contiguous, every expert's span is a multiple of 128 rows, a 128-row block whose first index is negative
     is skipped.  ``a_s`` may be any strided 2-D view (the reference passes a column-major one,
     dlblas/kernels/quant_dequant.py:65-83)."""
+    if not torch.compiler.is_compiling() and _fast.grouped_contiguous(a, a_s, w, w_s, out, m_indices):
+        return
     G, N, K = _check_common(a, a_s, w, w_s, out)
     if a.dim() != 2 or a.size(1) != K:
         raise ValueError(f'a must be [M_sum, {K}], got {tuple(a.shape)}')
@@ -150,6 +152,8 @@ def fp8_gemm_grouped_contiguous_silu_quant(a, a_s, w13, w13_s, m_indices, eps: f
 def fp8_gemm_grouped_masked(a, a_s, w, w_s, out, masked_m, expected_m=0):
     """For every expert g, rows ``[0, masked_m[g])`` of ``out[g]`` get ``(a[g] * a_s[g]) @ (w[g] * w_s[g]).T``;
     the other rows of ``out`` are left untouched and the matching rows of ``a`` are never used."""
+    if not torch.compiler.is_compiling() and _fast.grouped_masked(a, a_s, w, w_s, out, masked_m, expected_m):
+        return
     G, N, K = _check_common(a, a_s, w, w_s, out)
     if a.dim() != 3 or a.size(0) != G or a.size(2) != K:
         raise ValueError(f'a must be [{G}, M_max, {K}], got {tuple(a.shape)}')

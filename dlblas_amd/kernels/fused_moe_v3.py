@@ -10,7 +10,7 @@ from typing import List, Optional, Tuple
 
 import torch
 
-from .. import _lib
+from .. import _fast, _lib
 from .activation import silu_and_mul_post_quant
 from .fp8_gemm_grouped import fp8_gemm_grouped_contiguous_silu_quant, m_grouped_fp8_gemm_nt_contiguous
 
@@ -95,6 +95,8 @@ def ep_gather(
     output_tensor: torch.Tensor,
 ):
     """output_tensor[t] = sum_j input_tensor[input_index[t, j]] * recv_topk_weight[t, j] over slots with an expert."""
+    if not torch.compiler.is_compiling() and _fast.ep_gather(input_tensor, recv_topk_ids, recv_topk_weight, input_index, output_tensor):
+        return
     hidden_size = input_tensor.shape[1]
     assert hidden_size % 8 == 0
     assert input_tensor.stride(1) == 1 and output_tensor.stride(1) == 1, 'rows must be contiguous'
@@ -123,6 +125,10 @@ def fused_moe_v3(
     returns of the reference driver (dlblas/kernels/fused_moe_v3.py:246-343); every intermediate is allocated here,
     per call, as there."""
     tokens_q, tokens_scale = hidden_states_fp8
+    if num_recv_tokens_per_expert is not None and not torch.compiler.is_compiling():
+        combined = _fast.fused_moe_v3(tokens_q, tokens_scale, topk_idx, topk_weights, *w13_weight_fp8, *w2_weight_fp8, num_recv_tokens_per_expert)
+        if combined is not None:
+            return combined
     rows_total = 0 if num_recv_tokens_per_expert is None else sum(num_recv_tokens_per_expert)
     if rows_total <= 0:
         return tokens_q.to(torch.bfloat16)  # nothing routed to a local expert: the caller gets its input back in bf16

@@ -7,7 +7,7 @@ the caller's ``output`` / ``output_scale``.  It runs between the two masked grou
 """
 import torch
 
-from .. import _lib
+from .. import _fast, _lib
 
 
 @torch.library.custom_op('dlblas::silu_and_mul_masked_post_quant', mutates_args=('output', 'output_scale'), device_types='cuda')
@@ -68,6 +68,10 @@ def low_latency_experts(
     """
     from .fp8_gemm_grouped import fp8_gemm_grouped_masked_silu_quant, m_grouped_fp8_gemm_nt_masked
     a, a_s = hidden_states_fp8
+    if out_dtype is torch.bfloat16 and block_size == 128 and not torch.compiler.is_compiling():
+        down = _fast.low_latency_experts(a, a_s, gate_up_weight, gate_up_scale, gate_down_weight, gate_down_scale, masked_m, expected_m)
+        if down is not None:
+            return down
     num_groups, m, k = a.shape
     n = gate_up_weight.size(1)
     expected_m = min(expected_m, m)

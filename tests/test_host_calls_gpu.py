@@ -1,0 +1,119 @@
+"""The native form of the entry points (csrc/host_calls.cpp) does what their Python form does - same bits, same shapes and
+strides - for the calls it takes, and leaves every other call to it."""
+import threading
+
+import pytest
+import torch
+
+import helpers
+from oracle import fp8_block_gemm as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope='module')
+def dev():
+    if not torch.cuda.is_available():
+        pytest.skip('no GPU')
+    return torch.device('cuda:0')
+
+
+def _operands(lead, N, K, dev, seed=5):
+    g = helpers.gen(seed)
+    rows = 1
+    for d in lead:
+        rows *= d
+    whole = -(-K // 128) * 128  # a ragged last block keeps the scale of the whole one
+    a, a_s = orc.quant_act_1x128(torch.randn(rows, whole, generator=g).to(torch.bfloat16))
+    b, b_s = orc.quant_weight_128x128((torch.randn(N, whole, generator=g) * 0.05).to(torch.bfloat16))
+    a, b = a[:, :K].contiguous(), b[:, :K].contiguous()
+    return a.view(*lead, K).to(dev), b.to(dev), a_s.view(*lead, -1).to(dev), b_s.to(dev)
+
+
+@pytest.mark.parametrize('lead,N,K', [((1, ), 128, 256), ((3, 5), 136, 400), ((130, ), 512, 1024)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32, torch.float16])
+def test_fp8_gemm_equals_the_custom_op(dev, lead, N, K, dtype):
+    from dlblas_amd import _fast
+    from dlblas_amd.kernels.fp8_gemm import fp8_gemm
+    args = _operands(lead, N, K, dev)
+    prev = torch.get_default_dtype()
+    torch.set_default_dtype(dtype)
+    try:
+        native, out = _fast.fp8_gemm(*args), fp8_gemm(*args)
+    finally:
+        torch.set_default_dtype(prev)
+    ref = torch.ops.dlblas.fp8_gemm(*args, dtype)
+    torch.cuda.synchronize()
+    assert (native is None) == (dtype == torch.float16)  # a type the kernels do not write is converted on the Python path
+    assert out.dtype == ref.dtype and out.shape == ref.shape and torch.equal(out, ref)
+
+
+@pytest.mark.parametrize('shape', [(7, 256), (2, 3, 384), (2, 1, 4, 128)])
+@pytest.mark.parametrize('col_major', [False, True])
+def test_quantiser_equals_the_custom_op(dev, shape, col_major):
+    from dlblas_amd import _fast, _lib
+    from dlblas_amd.kernels.fp8 import per_token_group_quant_fp8, quant_op
+    x = torch.randn(*shape, generator=helpers.gen(6)).to(torch.bfloat16).to(dev)
+    assert _fast.quant(x, 128, 1e-10, col_major) is not None
+    q, s = per_token_group_quant_fp8(x, 128, column_major_scales=col_major)
+    K = shape[-1]
+    rows = x.numel() // K
+    ref_q = torch.empty(rows, K, dtype=torch.float8_e4m3fn, device=dev)
+    ref_s = torch.empty(rows, K // 128, device=dev)
+    quant_op(x.view(-1, K), ref_q, ref_s, 1e-10, 128)
+    torch.cuda.synchronize()
+    assert q.shape == x.shape and torch.equal(q.view(-1, K).view(torch.uint8), ref_q.view(torch.uint8))
+    assert s.shape == x.shape[:-1] + (K // 128, ) and torch.equal(s.reshape(rows, -1), ref_s)
+    if col_major:
+        buf = torch.empty((K // 128, ) + x.shape[:-1]).movedim(0, -1)
+        assert s.stride() == buf.stride()
+    wide = torch.randn(5, 512, device=dev)[:, :256]  # rows further apart than they are long
+    assert torch.equal(per_token_group_quant_fp8(wide, 128)[1], per_token_group_quant_fp8(wide.contiguous(), 128)[1])
+
+
+def test_other_calls_are_left_to_the_python_path(dev):
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from dlblas_amd import _fast
+    from dlblas_amd.kernels.fp8_gemm import fp8_gemm
+    a, b, a_s, b_s = _operands((16, ), 128, 256, dev)
+    assert _fast.fp8_gemm(a, b, a_s, b_s) is not None
+    assert _fast.fp8_gemm(a, b.t(), a_s, b_s) is None and _fast.fp8_gemm(a, b, a_s[:, :1], b_s) is None
+    assert _fast.fp8_gemm(a, b, a_s, b_s.half()) is None and _fast.fp8_gemm(a, b, a_s.cpu(), b_s) is None
+    assert _fast.fp8_gemm(a, b, a_s.clone().requires_grad_(), b_s) is None
+    assert _fast.fp8_gemm(a, b, None, b_s) is None and _fast.fp8_gemm(a, b, torch.nn.Parameter(a_s), b_s) is None
+    with FakeTensorMode() as mode:
+        fake = [mode.from_tensor(t) for t in (a, b, a_s, b_s)]
+        assert _fast.fp8_gemm(*fake) is None and tuple(fp8_gemm(*fake).shape) == (16, 128)
+    with pytest.raises(AssertionError, match='contiguous'):
+        fp8_gemm(a[:, ::2], b, a_s, b_s)
+    with pytest.raises(ValueError):
+        fp8_gemm(a, b, a_s, b_s[:, :1].contiguous())
+
+
+def test_streams_and_threads_share_the_workspaces_of_the_python_path(dev):
+    from dlblas_amd import _lib
+    from dlblas_amd.kernels.fp8_gemm import fp8_gemm
+    args = _operands((200, ), 392, 2048, dev)  # K slices in the workspace
+    ref = fp8_gemm(*args)
+    torch.cuda.synchronize()
+    results, failed = {}, []
+
+    def work(i):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                outs = [fp8_gemm(*args) for _ in range(20)]
+            stream.synchronize()
+            results[i] = all(torch.equal(o, ref) for o in outs)
+            assert (dev.index or 0, stream.cuda_stream) in _lib._workspaces
+        except Exception as exc:  # reported by the test's own thread
+            failed.append(exc)
+
+    threads = [threading.Thread(target=work, args=(i, )) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
+    assert len(results) == 3 and all(results.values())
