@@ -54,6 +54,7 @@ SYMBOLS = {
     'dlb_fp8_gemm_variant_name': (ctypes.c_char_p, [ctypes.c_int]),
     'dlb_fp8_gemm_plan': (ctypes.c_int, [ctypes.c_int, _c_i64, _c_i64, _c_i64, _c_sz, ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 3 +
                           [ctypes.POINTER(_c_i64)]),
+    'dlb_fp8_gemm_plan_wave_k': (ctypes.c_int, [_c_i64] * 3 + [_c_sz, ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 3),
     'dlb_fp8_gemm_plan_grouped': (ctypes.c_int, [ctypes.c_int, _c_i64, _c_i64, _c_i64, ctypes.c_int32, ctypes.c_int32, _c_sz, ctypes.c_int,
                                                 ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]),
     'dlb_silu_mul': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp] + [_c_i64] * 4 + [_c_vp]),
@@ -195,6 +196,15 @@ def plan_full(mode: int, rows: int, N: int, K: int, workspace_bytes: int = None,
     return variant_names()[v.value], s.value, c.value, n.value
 
 
+def plan_wave_k(M: int, N: int, K: int, workspace_bytes: int = None, compute_units: int = 256):
+    """(tile rows, tile columns, waves) when the kernel whose waves split K takes a dense launch over from the variant that
+    plan() names, None otherwise; touches no GPU."""
+    out = [ctypes.c_int() for _ in range(3)]
+    ws = WORKSPACE_BYTES if workspace_bytes is None else workspace_bytes
+    check(load().dlb_fp8_gemm_plan_wave_k(M, N, K, ws, compute_units, *(ctypes.byref(v) for v in out)))
+    return tuple(v.value for v in out) if out[0].value else None
+
+
 def plan_grouped(mode: int, rows: int, N: int, K: int, G: int, expected_m: int = -1, workspace_bytes: int = None,
                  compute_units: int = 256):
     """(variant name, flag) of a grouped launch (mode 1 contiguous, 2 masked) with G experts and the masked layout's hint;
@@ -218,7 +228,7 @@ def force_variant(name_or_id) -> None:
 
 
 KNOBS = {'splitk': 0, 'skinny_waves': 1, 'skinny_unroll': 2, 'skinny_nfrags': 3, 'group_m': 4, 'skinny_dma': 5, 'epilogue': 6, 'skinny_bn': 7,
-         'splitk_mode': 8, 'spin_limit': 9, 'scale_table': 10, 'lds_oversize': 11, 'masked_grid': 12, 'tile_list': 13, 'stream': 14}
+         'splitk_mode': 8, 'spin_limit': 9, 'scale_table': 10, 'lds_oversize': 11, 'masked_grid': 12, 'tile_list': 13, 'stream': 14, 'wave_k': 15}
 
 
 def tune(knob: str, value) -> None:

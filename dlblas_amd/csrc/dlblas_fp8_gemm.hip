@@ -16,6 +16,7 @@
 #include "fp8_gemm_skinny.h"
 #include "fp8_gemm_stream.h"
 #include "fp8_gemm_tiled.h"
+#include "fp8_gemm_wavek.h"
 #include "fp8_quant.h"
 
 // Scratch for dlb_fp8_gemm_noalloc: device memory that is part of the loaded code object, so a caller that cannot
@@ -103,6 +104,7 @@ enum Knob : int {
   kKnobMaskedGrid,   // workgroups per CU of the masked layout's persistent grid (0 = default)
   kKnobTileList,     // expert-contiguous rows: 1 = device-built tile lists whenever possible, 2 = never (0 = by batch size)
   kKnobStream,       // masked layout: 1 = never the weight-streaming kernel, 2 + i = its tile shape i wherever it applies (0 = by size)
+  kKnobWaveK,        // dense: 1 = never the kernel whose waves split K, 2 + i = its tile shape i wherever it applies (0 = by size)
   kKnobCount
 };
 thread_local int g_knob[kKnobCount] = {};
@@ -171,6 +173,12 @@ enum StreamShape : int { kStreamNone = -1, kStream32x256 = 0, kStream64x256, kSt
 struct StreamDims { int bm, bn, stages, ch; };
 constexpr StreamDims kStreamDims[kStreamCount] = {{32, 256, 4, 16}, {64, 256, 3, 16}, {64, 128, 6, 16}, {128, 256, 3, 11}, {64, 64, 9, 16}};
 
+// Tile shapes of the dense kernel whose waves split K
+struct WaveKDims { int mf, nf, waves; };
+constexpr WaveKDims kWaveKDims[] = {{1, 1, 8}, {1, 1, 4}, {2, 1, 8}, {1, 2, 4}, {2, 1, 4}, {2, 2, 4}, {2, 2, 2}};
+constexpr int kWaveKCount = sizeof(kWaveKDims) / sizeof(kWaveKDims[0]);
+constexpr int kWaveKNone = -1;
+
 // Raise a kernel's dynamic LDS limit once per (kernel, device).
 template <class Kernel>
 hipError_t ensure_lds(Kernel kernel, int bytes, int dev, std::atomic<unsigned long long>* done_mask) {
@@ -222,6 +230,30 @@ hipError_t launch_pipelined(const Args& args, int grid, int dev, hipStream_t str
   if (e != hipSuccess || g_prepare_only) return e;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, args);
   return hipGetLastError();
+}
+
+template <class Cfg, bool KTAIL>
+hipError_t launch_wavek_cfg(const Args& args, int grid, int dev, hipStream_t stream) {
+  static std::atomic<unsigned long long> lds_done{0};
+  auto kernel = fp8_gemm_wavek_kernel<Cfg, KTAIL>;
+  hipError_t e = ensure_lds(kernel, 160 * 1024, dev, &lds_done);
+  if (e != hipSuccess || g_prepare_only) return e;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NT), Cfg::lds_bytes(args.sct_pitch), stream, args);
+  return hipGetLastError();
+}
+
+template <bool KTAIL>
+hipError_t launch_wavek(int shape, const Args& args, int grid, int dev, hipStream_t stream) {
+  switch (shape) {
+    case 0: return launch_wavek_cfg<WaveKCfg<1, 1, 8>, KTAIL>(args, grid, dev, stream);
+    case 1: return launch_wavek_cfg<WaveKCfg<1, 1, 4>, KTAIL>(args, grid, dev, stream);
+    case 2: return launch_wavek_cfg<WaveKCfg<2, 1, 8>, KTAIL>(args, grid, dev, stream);
+    case 3: return launch_wavek_cfg<WaveKCfg<1, 2, 4>, KTAIL>(args, grid, dev, stream);
+    case 4: return launch_wavek_cfg<WaveKCfg<2, 1, 4>, KTAIL>(args, grid, dev, stream);
+    case 5: return launch_wavek_cfg<WaveKCfg<2, 2, 4>, KTAIL>(args, grid, dev, stream);
+    case 6: return launch_wavek_cfg<WaveKCfg<2, 2, 2>, KTAIL>(args, grid, dev, stream);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 template <class Cfg, int EPI, bool GATHER>
@@ -379,12 +411,13 @@ int64_t pick_mixed_split(int64_t M, int64_t N, int cus, double* makespan = nullp
 // leave much of a round empty (2048 x 4096: 128 tiles of 256 x 256 on 256 CUs, but 256 tiles of 128 x 256), or K is so
 // short that the fixed part decides: 384 x 18432 x 7168 82 -> 67 us, 2048 x 4096 x 7168 79 -> 67 us,
 // 4096 x 32768 x 512 166 -> 155 us.
-bool prefers_128_row_tiles(int64_t M, int64_t N, int kblocks, int cus) {
+bool prefers_128_row_tiles(int64_t M, int64_t N, int kblocks, int cus, double* us = nullptr) {
   double span = 0.0;
   pick_mixed_split(M, N, cus, &span);
   const double wide_us = span * (11.5 + 1.62 * kblocks);
   const int64_t rounds = ceil_div(ceil_div(M, 128) * ceil_div(N, 256), cus);
   const double half_us = static_cast<double>(rounds) * ((rounds >= 4 ? 4.3 : 5.5) + 1.0 * kblocks);
+  if (us) *us = std::min(wide_us, half_us);
   return half_us < 0.95 * wide_us;
 }
 
@@ -505,6 +538,20 @@ MidChoice pick_mid_plan(int64_t M, int64_t N, int kblocks, int cus, size_t ws_av
   return best;
 }
 
+// Estimate for the decode kernels at 33 .. 128 rows: what is larger of their workgroups each reading all activation rows from
+// the L2 (about 8.5 TB/s over the chip) and of their waves' K blocks, fetched one after the other: a round of 8 blocks lasts
+// 0.8 x (0.14 us + 24 ns per activation row + 40 ns per weight row of the workgroup) (measured at 33 .. 128 rows, 4 .. 28
+// weight rows, K = 2048 .. 16384).
+double decode_us(int64_t M, int64_t N, int64_t K, int kblocks, int cus) {
+  const int bn = pick_skinny_bn(N, M <= 64 ? 64 : 128, cus);
+  const int64_t wgs = ceil_div(N, bn);
+  const double m_eff = M <= 64 ? static_cast<double>(M) : 0.5 * (M + 128.0);  // the 128-row kernel computes all 8 row fragments
+  const double round_us = 0.14 + 0.0239 * m_eff + 0.04 * bn;
+  const double chain_us = 0.8 * round_us * static_cast<double>(ceil_div(kblocks, 8)) * static_cast<double>(ceil_div(wgs, cus));
+  const double l2_us = static_cast<double>(wgs) * M * K / 8.5e6;
+  return 2.6 + (l2_us > chain_us ? l2_us : chain_us);
+}
+
 // dma_ok: the DMA kernels address their sources with 32-bit byte offsets from the tile's first row (up to 256 rows x K
 // bytes, 512 scale rows x stride); false sends such problems to the kernels with 64-bit addressing.
 // G, hint_rows (grouped layouts): experts, and the masked layout's typical rows per expert (<= 0: unknown).
@@ -528,20 +575,9 @@ Plan make_plan(int mode, int64_t M, int64_t N, int64_t K, int cus, size_t ws_byt
       // (measured at M = 128: 2112 x 7168 44 -> 22 us, 4096 x 7168 45 -> 23 us; 7168 x 2048 stays: 16 vs 19 us)
       if (M > 64 && kblocks >= 32 && ceil_div(N, 128) * 2 <= cus) v = kVarTile128x128;
       if (M > 32 && whole_blocks) {
-        // 33 .. 128 rows: the streaming kernel costs what is larger of its workgroups each reading all activation rows
-        // from the L2 (about 8.5 TB/s over the chip) and of its waves' K blocks, fetched one after the other: a round
-        // of 8 blocks lasts 0.8 x (0.14 us + 24 ns per activation row + 40 ns per weight row of the workgroup) (measured at
-        // 33 .. 128 rows, 4 .. 28 weight rows, K = 2048 .. 16384).  A K-split tile kernel wins when the weight matrix
-        // is narrow and K long (2112 x 7168: 18.3 -> 14.1 us at 64 rows, 29 -> 17.4 us at 128; at 33 rows the streaming
-        // kernel stays ahead, 11.9 against 13.2 us)
-        const int rows = M <= 64 ? 64 : 128;
-        const int bn = pick_skinny_bn(N, rows, cus);
-        const int64_t wgs = ceil_div(N, bn);
-        const double m_eff = M <= 64 ? static_cast<double>(M) : 0.5 * (M + 128.0);  // the 128-row kernel computes all 8 row fragments
-        const double round_us = 0.14 + 0.0239 * m_eff + 0.04 * bn;
-        const double chain_us = 0.8 * round_us * static_cast<double>(ceil_div(kblocks, 8)) * static_cast<double>(ceil_div(wgs, cus));
-        const double l2_us = static_cast<double>(wgs) * M * K / 8.5e6;
-        const double stream_us = 2.6 + (l2_us > chain_us ? l2_us : chain_us);
+        // A K-split tile kernel wins when the weight matrix is narrow and K long (2112 x 7168: 18.3 -> 14.1 us at 64 rows,
+        // 29 -> 17.4 us at 128; at 33 rows the streaming kernel stays ahead, 11.9 against 13.2 us)
+        const double stream_us = decode_us(M, N, K, kblocks, cus);
         const MidChoice mid = pick_mid_plan(M, N, kblocks, cus, ws_avail);
         if (mid.us < stream_us) v = mid.variant, mid_splitk = mid.splitk;
         else v = M <= 64 ? kVarSkinny64 : kVarSkinny128;
@@ -655,7 +691,63 @@ struct Resolved {
   bool fused;                // K slices added inside the launch (counters in the workspace head), no second pass
   int stream;                // masked layout: tile shape of the weight-streaming kernel (kStreamNone: a ring kernel)
   int chunk_len;             //   K blocks per chunk of its scale table
+  int wavek;                 // dense: tile shape of the kernel whose waves split K (kWaveKNone: another kernel)
 };
+
+int wavek_lds(const WaveKDims& d, int pitch) {
+  const int bm = 32 * d.mf, bn = 32 * d.nf;
+  return d.waves * (bm + bn) * kScaleBlock + (bm * pitch * 4 + 255) / 256 * 256;
+}
+
+// Which tile shape of the kernel whose waves split K runs a dense launch (kWaveKNone: none).
+// Estimate of a launch: 1.8 us + what is longest of
+//   - the busiest CU's workgroups: 1.5 us per round of resident ones (start, final sum) + K blocks x the time per block, which is
+//     the larger of its bytes at 86 GB/s (the DMA path of a CU) and the trip of one block (0.21 us + 3.8 ns per operand row)
+//     shared by the waves that are resident at once;
+//   - every tile's operands from the L2s at 17 TB/s;  - the matrices from HBM at 6 TB/s.
+// (rms error 13 % over 110 problems of 1 .. 1300 rows, 512 .. 36864 weight rows, K = 512 .. 18432; its choice of shape is
+// within 3 % of the best, geometric mean.)  Against the kernels it would replace: up to 16 rows the decode kernels' 16-row
+// fragments waste less (16 x 7168 x 2048 5.2 against 5.4 us), unless K is ragged or N so large that they take many rounds
+// (1 x 28480 x 1152 9.0 -> 7.6 us); from 17 to 64 rows this kernel is ahead wherever measured (23 x 12632 x 16768 45 -> 32 us);
+// above, the smaller estimate wins (100 x 2112 x 7168 13.4 -> 10.2 us, 500 x 4096 x 7168 33 -> 26 us, 64 x 2112 x 7168 12.7 ->
+// 7.9 us; 473 x 7088 x 6528 stays with 128 x 128 tiles, 40 against 45 us).  The register-staged kernels, the only others for
+// a ragged K, lose everywhere measured (300 x 1000 x 1040 11.4 -> 4.7 us, 225 x 17536 x 5280 126 -> 62 us).
+int pick_wavek(int64_t M, int64_t N, int64_t K, int cus, size_t ws_bytes) {
+  const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
+  const int knob = g_knob[kKnobWaveK];
+  if (knob == 1 || g_forced_variant >= 0 || g_knob[kKnobSplitK] > 0) return kWaveKNone;
+  if (kblocks >= 1024) return kWaveKNone;  // no table of that many scales fits
+  const bool ragged = K % kScaleBlock != 0;
+  if (knob == 0 && M <= 16 && !ragged && N < 24576) return kWaveKNone;
+  int best = kWaveKNone;
+  double best_us = 0.0;
+  for (int i = 0; i < kWaveKCount; ++i) {
+    const WaveKDims& d = kWaveKDims[i];
+    if (knob >= 2 && i != knob - 2) continue;
+    const int lds = wavek_lds(d, kblocks | 1);
+    if (lds > 160 * 1024) continue;
+    const double rows = 32.0 * (d.mf + d.nf);
+    const double tiles = static_cast<double>(ceil_div(M, 32 * d.mf)) * static_cast<double>(ceil_div(N, 32 * d.nf));
+    const double resident = std::max(1, std::min(160 * 1024 / lds, 16 / d.waves));
+    const double per_cu = std::ceil(tiles / cus);
+    const double slots = static_cast<double>(ceil_div(kblocks, d.waves)) * d.waves;
+    const double block_us = std::max(rows * 128.0 / 88e3, (0.21 + 0.0038 * rows) / (d.waves * std::min(per_cu, resident)));
+    const double cu_us = std::ceil(per_cu / resident) * 1.5 + per_cu * slots * block_us;
+    const double l2_us = tiles * kblocks * rows * 128.0 / 17e6;
+    const double hbm_us = (static_cast<double>(N) + static_cast<double>(M)) * static_cast<double>(K) / 6e6;
+    const double us = 1.8 + std::max(cu_us, std::max(l2_us, hbm_us));
+    if (best == kWaveKNone || us < best_us) best = i, best_us = us;
+  }
+  if (best == kWaveKNone || knob >= 2 || M <= 64 || ragged) return best;
+  const size_t ws_avail = ws_bytes > DLB_WS_COUNTER_BYTES ? ws_bytes - DLB_WS_COUNTER_BYTES : 0;
+  double other;
+  if (M > 128 && ceil_div(M, 256) * ceil_div(N, 256) * 2 >= cus)
+    prefers_128_row_tiles(M, N, kblocks, cus, &other);
+  else
+    other = pick_mid_plan(M, N, kblocks, cus, ws_avail).us;
+  if (M <= 128) other = std::min(other, 1.3 * decode_us(M, N, K, kblocks, cus));  // (the 128-row decode kernel runs above its estimate at short K)
+  return best_us < 0.95 * other ? best : kWaveKNone;
+}
 
 // K blocks per chunk of the streaming kernel's scale table: equal chunks of at most `ch` blocks, none shorter than the
 // stages - 1 steps the issue side runs ahead (the table has two buffers).  0: no such cut.
@@ -696,9 +788,10 @@ int pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool 
   return best;
 }
 
+// overlay: the kernel whose waves split K may take the launch over from the planned variant.
 // fused_act: the launch is one of the gate/up GEMMs with the activation in its epilogue (their kernels take no scale table)
 Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as_sm, int64_t as_sk, bool have_ws,
-                 size_t ws_bytes, int cus, bool gather_scales = false, bool fused_act = false, int64_t hint_rows = -1) {
+                 size_t ws_bytes, int cus, bool gather_scales = false, bool fused_act = false, int64_t hint_rows = -1, bool overlay = true) {
   Resolved r{};
   const int64_t kblocks = ceil_div(K, kScaleBlock);
   const int64_t groups = mode == kMasked ? G : 1;  // a_s is per expert only in the masked layout; contiguous rows are one matrix
@@ -707,6 +800,17 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
   r.pl = make_plan(mode, rows, N, K, cus, usable_ws ? ws_bytes : 0, dma_ok, G, hint_rows, fused_act || gather_scales);
   const Plan& pl = r.pl;
   r.stream = kStreamNone;
+  r.wavek = kWaveKNone;
+  if (overlay && mode == kDense && dma_ok && as_sk < (1ll << 20) && K > 0 && K % 16 == 0) r.wavek = pick_wavek(rows, N, K, cus, usable_ws ? ws_bytes : 0);
+  if (r.wavek != kWaveKNone) {
+    r.pl.splitk = 1;
+    r.kb_per_split = static_cast<int>(kblocks);
+    r.splitk = 1;
+    r.n_split = N;
+    r.sct_pitch = static_cast<int>(kblocks) | 1;
+    r.grid = ceil_div(rows, 32 * kWaveKDims[r.wavek].mf) * ceil_div(N, 32 * kWaveKDims[r.wavek].nf);
+    return r;
+  }
   if (mode == kMasked && dma_ok && K % kScaleBlock == 0 && K > 0 && static_cast<int64_t>(G) * rows < (1ll << 31))
     r.stream = pick_stream(rows, N, K, G, hint_rows, fused_act, cus, &r.chunk_len);
   const int want = usable_ws ? pl.splitk : 1;
@@ -1053,7 +1157,7 @@ int run(const Problem& pr) {
   // The main kernel of the call.  With g_prepare_only set it only raises the kernel's dynamic-LDS limit (the one
   // step of a launch that can still fail), so that run() can do that before it enqueues the first pre-pass.
   auto main_kernel = [&]() -> hipError_t {
-    switch (pl.variant) {
+    if (rs.wavek == kWaveKNone) switch (pl.variant) {
       case kVarExact: {
         if (g_prepare_only) return hipSuccess;
         // rows in a grid-stride loop: the second grid dimension is limited to 65535
@@ -1072,6 +1176,12 @@ int run(const Problem& pr) {
         return launch_skinny(8, pl.sk_nfrags, pl.sk_waves, pl.sk_unroll, pl.sk_dma, ar, dev, pr.stream);
       default:
         break;
+    }
+    if (rs.wavek != kWaveKNone) {
+      ar.tiles_m = static_cast<int>(ceil_div(pr.rows, 32 * kWaveKDims[rs.wavek].mf));
+      ar.tiles_n = static_cast<int>(ceil_div(pr.N, 32 * kWaveKDims[rs.wavek].nf));
+      return pr.K % kScaleBlock != 0 ? launch_wavek<true>(rs.wavek, ar, static_cast<int>(rs.grid), dev, pr.stream)
+                                     : launch_wavek<false>(rs.wavek, ar, static_cast<int>(rs.grid), dev, pr.stream);
     }
     if (rs.stream != kStreamNone) {
       ar.tiles_n = static_cast<int>(pr.act ? pr.N / 256 : ceil_div(pr.N, kStreamDims[rs.stream].bn));
@@ -1481,11 +1591,26 @@ int dlb_fp8_gemm_plan(int mode, int64_t rows, int64_t N, int64_t K, size_t works
   if (compute_units <= 0) return dlb::fail(DLB_ERR_BAD_SHAPE, "compute_units must be positive");
   // row-major activation scales, as the dense Python entry point hands them over
   const dlb::Resolved rs = dlb::resolve(mode, rows, N, K, mode == dlb::kDense ? 1 : 32, dlb::ceil_div(K, dlb::kScaleBlock), 1,
-                                        workspace_bytes > 0, workspace_bytes, compute_units);
+                                        workspace_bytes > 0, workspace_bytes, compute_units, false, false, -1, false);
   if (variant) *variant = rs.pl.variant;
   if (k_slices) *k_slices = rs.splitk;
   if (decode_columns) *decode_columns = dlb::is_skinny(rs.pl.variant) ? rs.pl.sk_bn : 0;
   if (narrow_from) *narrow_from = rs.n_split;
+  return DLB_OK;
+}
+
+int dlb_fp8_gemm_plan_wave_k(int64_t M, int64_t N, int64_t K, size_t workspace_bytes, int compute_units, int* tile_rows, int* tile_columns,
+                             int* waves) {
+  dlb::clear_error();
+  const int64_t lim = (1ll << 31) - 1024;
+  if (M < 0 || N < 0 || K < 0 || M > lim || N > lim || K > lim || compute_units <= 0)
+    return dlb::fail(DLB_ERR_BAD_SHAPE, "bad dimension (M=%lld, N=%lld, K=%lld)", (long long)M, (long long)N, (long long)K);
+  const dlb::Resolved rs = dlb::resolve(dlb::kDense, M, N, K, 1, dlb::ceil_div(K, dlb::kScaleBlock), 1, workspace_bytes > 0, workspace_bytes,
+                                        compute_units);
+  const bool on = rs.wavek != dlb::kWaveKNone;
+  if (tile_rows) *tile_rows = on ? 32 * dlb::kWaveKDims[rs.wavek].mf : 0;
+  if (tile_columns) *tile_columns = on ? 32 * dlb::kWaveKDims[rs.wavek].nf : 0;
+  if (waves) *waves = on ? dlb::kWaveKDims[rs.wavek].waves : 0;
   return DLB_OK;
 }
 

@@ -328,7 +328,7 @@ int dlb_fp8_quant_128x128(const void* w, int w_dtype, void* q, float* s, int64_t
  * mode 0 = dlb_fp8_gemm, 1 = grouped contiguous (rows = M_sum), 2 = grouped masked (rows = M_max); `compute_units`
  * is the CU count to plan for (256 on MI355X); activation scales are taken to be row-major.  Outputs (each may be
  * NULL): the kernel variant id (dlb_fp8_gemm_variant_name); the number of K slices summed in a second pass (1 = none),
- * exactly as a launch with this workspace size would use it; the output columns per workgroup of the decode kernels
+ * exactly as a launch with this workspace size would use it (unless the kernel of dlb_fp8_gemm_plan_wave_k takes it over); the output columns per workgroup of the decode kernels
  * (0 for other variants); the first column of the 192-wide tiles of the mixed-width prefill launch (N when all tiles
  * are equal).  Honours the calling thread's forced variant and knobs, as a launch does (both run the same code).
  * Costs a few microseconds at most and keeps no state.  No counterpart in the reference, whose single Triton
@@ -336,6 +336,14 @@ int dlb_fp8_quant_128x128(const void* w, int w_dtype, void* q, float* s, int64_t
  */
 int dlb_fp8_gemm_plan(int mode, int64_t rows, int64_t N, int64_t K, size_t workspace_bytes, int compute_units, int* variant,
                       int* k_slices, int* decode_columns, int64_t* narrow_from);
+
+/*
+ * Whether the kernel whose waves split K (a few dozen to a few hundred rows, or a ragged K) takes a dense launch over from
+ * the variant dlb_fp8_gemm_plan names, and with which tile: rows, columns and waves of its workgroups, all 0 when it does
+ * not.  No counterpart in the reference.
+ */
+int dlb_fp8_gemm_plan_wave_k(int64_t M, int64_t N, int64_t K, size_t workspace_bytes, int compute_units, int* tile_rows, int* tile_columns,
+                             int* waves);
 
 /*
  * The same query for the grouped layouts with what their choice depends on besides the shape: the expert count and, for
@@ -383,6 +391,8 @@ int dlb_fp8_gemm_force_variant(int variant);
  *                           rounds of 128 x 256 tiles on)
  *   DLB_KNOB_STREAM         masked layout: 1 = never the weight-streaming kernel, 2 .. 6 = its tile shape 0 .. 4 (32 x 256,
  *                           64 x 256, 64 x 128, 128 x 256, 64 x 64) wherever it applies (default: by size)
+ *   DLB_KNOB_WAVE_K         dense: 1 = never the kernel whose waves split K, 2 .. 8 = its tile shape 0 .. 6 (32 x 32 with 8 / 4
+ *                           waves, 64 x 32 with 8, 32 x 64 with 4, 64 x 32 with 4, 64 x 64 with 4 / 2) wherever it applies
  *   DLB_KNOB_LDS_OVERSIZE   test hook: 1 = every kernel asks for more LDS than the GPU has, so the call is refused
  *                           (DLB_ERR_LAUNCH) before anything is enqueued
  */
@@ -401,6 +411,7 @@ int dlb_fp8_gemm_force_variant(int variant);
 #define DLB_KNOB_MASKED_GRID 12
 #define DLB_KNOB_TILE_LIST 13
 #define DLB_KNOB_STREAM 14
+#define DLB_KNOB_WAVE_K 15
 int dlb_fp8_gemm_tune(int knob, int value);
 
 /* Name of kernel variant `variant`, or NULL beyond the last one. */
