@@ -103,7 +103,7 @@ enum Knob : int {
   kKnobLdsOversize,  // test hook: 1 = ask for more LDS than the GPU has, so that the launch is refused before anything is enqueued
   kKnobMaskedGrid,   // workgroups per CU of the masked layout's persistent grid (0 = default)
   kKnobTileList,     // expert-contiguous rows: 1 = device-built tile lists whenever possible, 2 = never (0 = by batch size)
-  kKnobStream,       // masked layout: 1 = never the weight-streaming kernel, 2 + i = its tile shape i wherever it applies (0 = by size)
+  kKnobStream,       // masked layout: 1 = never the weight-streaming kernel, 2 + i = its tile shape i wherever it applies (0 = by size), 7 + i = the same, fragments read ahead
   kKnobWaveK,        // dense: 1 = never the kernel whose waves split K, 2 + i = its tile shape i wherever it applies (0 = by size)
   kKnobCount
 };
@@ -256,32 +256,39 @@ hipError_t launch_wavek(int shape, const Args& args, int grid, int dev, hipStrea
   }
 }
 
-template <class Cfg, int EPI, bool GATHER>
+template <class Cfg, int EPI, bool GATHER, bool AHEAD>
 hipError_t launch_stream(const Args& args, int grid, int dev, hipStream_t stream) {
   static std::atomic<unsigned long long> lds_done{0};
-  auto kernel = fp8_gemm_stream_kernel<Cfg, EPI, GATHER>;
+  auto kernel = fp8_gemm_stream_kernel<Cfg, EPI, GATHER, AHEAD>;
   hipError_t e = ensure_lds(kernel, Cfg::LDS_BYTES, dev, &lds_done);
   if (e != hipSuccess || g_prepare_only) return e;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, args);
   return hipGetLastError();
 }
 
+// ahead: fragments read one step ahead of their use (plain product, tiles of 64 rows or more)
 template <int EPI, bool GATHER>
-hipError_t launch_stream_shape(int shape, const Args& args, int grid, int dev, hipStream_t stream) {
-  switch (shape) {
-    case kStream32x256: return launch_stream<Stream32x256, EPI, GATHER>(args, grid, dev, stream);
-    case kStream64x256: return launch_stream<Stream64x256, EPI, GATHER>(args, grid, dev, stream);
-    case kStream128x256: return launch_stream<Stream128x256, EPI, GATHER>(args, grid, dev, stream);
-    default: break;
-  }
+hipError_t launch_stream_shape(int shape, bool ahead, const Args& args, int grid, int dev, hipStream_t stream) {
   if constexpr (EPI == kStoreProduct) {
+    if (ahead) switch (shape) {
+      case kStream64x256: return launch_stream<Stream64x256, EPI, GATHER, true>(args, grid, dev, stream);
+      case kStream64x128: return launch_stream<Stream64x128, EPI, GATHER, true>(args, grid, dev, stream);
+      case kStream128x256: return launch_stream<Stream128x256, EPI, GATHER, true>(args, grid, dev, stream);
+      case kStream64x64: return launch_stream<Stream64x64, EPI, GATHER, true>(args, grid, dev, stream);
+      default: break;
+    }
     switch (shape) {
-      case kStream64x128: return launch_stream<Stream64x128, EPI, GATHER>(args, grid, dev, stream);
-      case kStream64x64: return launch_stream<Stream64x64, EPI, GATHER>(args, grid, dev, stream);
+      case kStream64x128: return launch_stream<Stream64x128, EPI, GATHER, false>(args, grid, dev, stream);
+      case kStream64x64: return launch_stream<Stream64x64, EPI, GATHER, false>(args, grid, dev, stream);
       default: break;
     }
   }
-  return hipErrorInvalidValue;
+  switch (shape) {
+    case kStream32x256: return launch_stream<Stream32x256, EPI, GATHER, false>(args, grid, dev, stream);
+    case kStream64x256: return launch_stream<Stream64x256, EPI, GATHER, false>(args, grid, dev, stream);
+    case kStream128x256: return launch_stream<Stream128x256, EPI, GATHER, false>(args, grid, dev, stream);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 template <class Cfg>
@@ -691,6 +698,7 @@ struct Resolved {
   bool fused;                // K slices added inside the launch (counters in the workspace head), no second pass
   int stream;                // masked layout: tile shape of the weight-streaming kernel (kStreamNone: a ring kernel)
   int chunk_len;             //   K blocks per chunk of its scale table
+  bool ahead;                //   and whether it reads its fragments one step ahead
   int wavek;                 // dense: tile shape of the kernel whose waves split K (kWaveKNone: another kernel)
 };
 
@@ -759,31 +767,41 @@ int stream_chunk_len(int kblocks, int ch, int stages) {
   return 0;
 }
 
+// Rows that cover nearly all experts: twice the caller's hint, at most the buffers' height.
+int64_t stream_span(int64_t M, int64_t hint_rows) { return hint_rows > 0 && 2 * hint_rows < M ? 2 * hint_rows : M; }
+constexpr int kStreamActSpan = 192;  // the longest experts the weight-streaming kernel takes with the quantising epilogue
+
 // Which tile shape of the weight-streaming kernel runs a masked launch (kStreamNone: none), from the typical rows of an
 // expert (twice the caller's hint covers nearly all of them).  A tile's step lasts what is longer of the trip its loads
 // take with the chip to themselves, 0.25 us + 1.9 ns per row of the two operands (a lone CU fetches 40 - 50 GB/s), and its
 // share of the HBM stream (6.9 TB/s over the busy CUs); tiles of 64 or 128 weight rows win while those of 256 leave CUs idle.
-int pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, int cus, int* chunk_len) {
+int pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, int cus, int* chunk_len, bool* ahead) {
   const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
   const int knob = g_knob[kKnobStream];
   if (knob == 1 || g_forced_variant >= 0) return kStreamNone;
-  const double span = static_cast<double>(hint_rows > 0 && 2 * hint_rows < M ? 2 * hint_rows : M);
-  if (knob == 0 && span > 192) return kStreamNone;
+  const double span = static_cast<double>(stream_span(M, hint_rows));
+  // Longer experts go to the ring kernels.  Plain product, us here / there, 0 .. cap rows: 32 x 7168 x 2048 cap 256 116 / 141,
+  // cap 384 161 / 166, cap 512 210 / 205; 32 x 7168 x 1024 cap 448 116 / 123; 32 x 4096 x 7168 cap 256 217 / 226, cap 384 305 /
+  // 298; 32 x 2048 x 7168 cap 448 208 / 202.  The quantising epilogue (its row tiles drift apart and fetch weights twice): kStreamActSpan.
+  if (knob == 0 && span > (act ? kStreamActSpan : kblocks <= 24 ? 448 : 256)) return kStreamNone;
   int best = kStreamNone;
   double best_us = 0.0;
   for (int i = 0; i < kStreamCount; ++i) {
     const StreamDims& d = kStreamDims[i];
-    if (knob >= 2 && i != knob - 2) continue;
-    if ((act && d.bn != 256) || kblocks < d.stages - 1) continue;
+    if (knob >= 2 && i != (knob - 2) % kStreamCount) continue;
+    if ((act && d.bn != 256) || kblocks < d.stages) continue;
     const int len = stream_chunk_len(kblocks, d.ch, d.stages);
     if (len <= 0) continue;
     const double mtiles = span <= d.bm ? 1.0 : 0.5 * (span / d.bm + 1.0);
     const double tiles = static_cast<double>(G) * mtiles * static_cast<double>(act ? N / 256 : ceil_div(N, d.bn));
     const double rows = std::min(0.5 * span, static_cast<double>(d.bm));
-    auto step = [&](double busy) { return std::max(0.25 + 0.0019 * (d.bn + rows), d.bn * 128.0 * busy / 6.9e6); };
+    // the row tiles of long experts run in step and share the weights in the L2 (30 problems of 8 .. 32 experts, 200 .. 448
+    // rows: this choice against the ring kernels 1.19 x, geometric mean; 0.96 the worst)
+    const double sharing = span > 192 ? mtiles : 1.0;
+    auto step = [&](double busy) { return std::max(0.25 + 0.0019 * (d.bn + rows), d.bn * 128.0 * busy / sharing / 6.9e6); };
     const double full = std::floor(tiles / cus), rest = tiles - full * cus;
     const double us = full * (1.0 + kblocks * step(cus)) + (rest > 0.5 ? 1.0 + kblocks * step(rest) : 0.0);
-    if (best == kStreamNone || us < best_us) best = i, best_us = us, *chunk_len = len;
+    if (best == kStreamNone || us < best_us) best = i, best_us = us, *chunk_len = len, *ahead = !act && (knob >= 2 ? knob >= 2 + kStreamCount : span > d.bm);
   }
   return best;
 }
@@ -812,7 +830,7 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
     return r;
   }
   if (mode == kMasked && dma_ok && K % kScaleBlock == 0 && K > 0 && static_cast<int64_t>(G) * rows < (1ll << 31))
-    r.stream = pick_stream(rows, N, K, G, hint_rows, fused_act, cus, &r.chunk_len);
+    r.stream = pick_stream(rows, N, K, G, hint_rows, fused_act, cus, &r.chunk_len, &r.ahead);
   const int want = usable_ws ? pl.splitk : 1;
   r.kb_per_split = static_cast<int>(ceil_div(kblocks > 0 ? kblocks : 1, want));
   r.splitk = static_cast<int>(ceil_div(kblocks > 0 ? kblocks : 1, r.kb_per_split));  // no empty slice
@@ -970,11 +988,12 @@ int run_ragged(const RaggedProblem& pr) {
   if (cus < 0) return fail(DLB_ERR_LAUNCH, "hipGetDevice failed");
   const int64_t kblocks = ceil_div(pr.K, kScaleBlock);
   int chunk_len = 0;
+  bool ahead = false;
   int shape = kStreamNone;
   const bool fits = pr.K > 0 && pr.K % kScaleBlock == 0 && pr.K < (1ll << 24) && pr.as_sm < (1ll << 21) && pr.M_sum < (1ll << 31) &&
                     pr.N < (1ll << 31) && (!pr.act || (pr.N % (2 * kScaleBlock) == 0 && pr.N * pr.K < (1ll << 32))) &&
                     (!pr.a_rows || (pr.act && pr.a_src_rows > 0 && pr.a_src_rows * pr.K < (1ll << 31)));
-  if (fits) shape = pick_stream(pr.M_sum, pr.N, pr.K, pr.G, pr.hint_rows, pr.act, cus, &chunk_len);
+  if (fits) shape = pick_stream(pr.M_sum, pr.N, pr.K, pr.G, pr.hint_rows, pr.act, cus, &chunk_len, &ahead);
   if (shape == kStreamNone)
     return fail(DLB_ERR_BAD_SHAPE, "the weight-streaming kernel does not take this problem (N=%lld K=%lld, about %lld rows per expert)",
                 (long long)pr.N, (long long)pr.K, (long long)pr.hint_rows);
@@ -1014,9 +1033,9 @@ int run_ragged(const RaggedProblem& pr) {
   const int grid = static_cast<int>(ceil_div(worst < cus ? worst : cus, 32) * 32);
   hipError_t e;
   if (pr.act)
-    e = pr.a_rows ? launch_stream_shape<kSiluQuant, true>(shape, ar, grid, dev, pr.stream) : launch_stream_shape<kSiluQuant, false>(shape, ar, grid, dev, pr.stream);
+    e = pr.a_rows ? launch_stream_shape<kSiluQuant, true>(shape, false, ar, grid, dev, pr.stream) : launch_stream_shape<kSiluQuant, false>(shape, false, ar, grid, dev, pr.stream);
   else
-    e = launch_stream_shape<kStoreProduct, false>(shape, ar, grid, dev, pr.stream);
+    e = launch_stream_shape<kStoreProduct, false>(shape, ahead, ar, grid, dev, pr.stream);
   if (e != hipSuccess) return fail(DLB_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
   return DLB_OK;
 }
@@ -1187,8 +1206,8 @@ int run(const Problem& pr) {
       ar.tiles_n = static_cast<int>(pr.act ? pr.N / 256 : ceil_div(pr.N, kStreamDims[rs.stream].bn));
       const int64_t worst = static_cast<int64_t>(ar.tiles_n) * pr.G * ceil_div(pr.rows, kStreamDims[rs.stream].bm);
       const int grid = static_cast<int>(ceil_div(worst < cus ? worst : cus, 32) * 32);  // tiles are dealt to the XCDs four at a time
-      return pr.act ? launch_stream_shape<kSiluQuantMasked, false>(rs.stream, ar, grid, dev, pr.stream)
-                    : launch_stream_shape<kStoreProduct, false>(rs.stream, ar, grid, dev, pr.stream);
+      return pr.act ? launch_stream_shape<kSiluQuantMasked, false>(rs.stream, false, ar, grid, dev, pr.stream)
+                    : launch_stream_shape<kStoreProduct, false>(rs.stream, rs.ahead, ar, grid, dev, pr.stream);
     }
     const int g = static_cast<int>(rs.grid);
     const int g_dense = rs.resident ? cus : g;
@@ -1625,7 +1644,9 @@ int dlb_fp8_gemm_plan_grouped(int mode, int64_t rows, int64_t N, int64_t K, int3
   const dlb::Resolved rs = dlb::resolve(mode, rows, N, K, G, dlb::ceil_div(K, dlb::kScaleBlock), 1, workspace_bytes > 0, workspace_bytes,
                                         compute_units, false, false, mode == dlb::kMasked ? expected_m : -1);
   if (variant) *variant = rs.pl.variant;
-  if (tile_lists) *tile_lists = rs.tile_list || rs.stream != dlb::kStreamNone ? 1 : 0;
+  // (callers ask whether the form with the quantising epilogue applies)
+  const bool streams = rs.stream != dlb::kStreamNone && (dlb::g_knob[dlb::kKnobStream] >= 2 || dlb::stream_span(rows, expected_m) <= dlb::kStreamActSpan);
+  if (tile_lists) *tile_lists = rs.tile_list || streams ? 1 : 0;
   return DLB_OK;
 }
 

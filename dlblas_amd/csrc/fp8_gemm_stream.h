@@ -2,7 +2,7 @@
 // short prefill chunks), where reading every expert's weights once from HBM is the whole cost.
 //
 // One persistent workgroup per CU walks its tiles with ONE LDS ring that runs on across tile boundaries: the DMA of the
-// next tile's first K blocks is issued STAGES - 1 steps ahead like any other, so a CU never drains its loads between two
+// next tile's first K blocks is issued STAGES steps ahead like any other, so a CU never drains its loads between two
 // tiles.  What the ring needs for that:
 //   - sources are addressed through buffer descriptors: a lane's byte offset (row x K + chunk) is the same for every tile,
 //     only scalar registers change with the tile, and rows past an expert's last one are out of the descriptor's range
@@ -14,12 +14,13 @@
 // Measured (MI355X, 32 experts, against the 128 x 256 ring kernel it replaces there): gate/up + activation 4096 x 7168,
 // ~16 / ~32 rows per expert 186 -> 143 / 161 -> 148 us, down 7168 x 2048 97 -> 83 / 101 -> 91 us; 940 MB of weights at 4 rows
 // 138 us = 6.8 TB/s, i.e. 12 us + bytes at 7.5 TB/s.  Over 90 problems of 8 .. 32 experts, 512 .. 7168 weight rows and K, up
-// to 192 rows per expert: 1.26 x (geometric mean; the largest gains where 256-column tiles left CUs idle).  Above 192 rows
-// the ring kernels stay: row tiles of one expert drift apart there and fetch its weights twice (0 .. 256 rows, 7168 x 2048:
-// 127 against 134 us).
+// to 192 rows per expert: 1.26 x (geometric mean; the largest gains where 256-column tiles left CUs idle).  With AHEAD (below)
+// 0 .. 256 rows: 7168 x 2048 141 -> 128 us with cold operands, 8 experts x 4096 x 7168 88 -> 68, 16 x 1024 x 2048 (0 .. 448
+// rows) 37 -> 25.  Its 128 x 256 step without any load takes 0.85 us, half of that the 128 KB of fragment reads.  The longest
+// experts stay with the ring kernels, whose 256-row tiles read less LDS per product.
 //
 // Arithmetic: fp8_gemm_kernel of the reference (dlblas/kernels/fp8_gemm.py:49-60), same order of additions as the ring
-// kernels of fp8_gemm_pipelined.h, so results have the same bits.  Requires K % 128 == 0 and K / 128 >= STAGES - 1.
+// kernels of fp8_gemm_pipelined.h, so results have the same bits.  Requires K % 128 == 0 and K / 128 >= STAGES.
 #pragma once
 
 #include "fp8_gemm_common.h"
@@ -69,6 +70,19 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const uint8_t* base,
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, bytes, 0x00020000);
 }
 
+// Wait until at most `younger` (0 .. MAX) groups of L vector-memory instructions are on their way.
+template <int L, int MAX>
+__device__ __forceinline__ void wait_groups(int younger) {
+  if constexpr (MAX > 0) {
+    if (younger >= MAX)
+      wait_vmcnt<MAX * L>();
+    else
+      wait_groups<L, MAX - 1>(younger);
+  } else {
+    wait_vmcnt<0>();
+  }
+}
+
 // Row ranges of the experts, 64 at a time: lane i of every wave holds expert first + i.
 struct ExpertWalk {
   int first, base, total;  // first expert of the window, tiles before it, tiles in it
@@ -76,17 +90,21 @@ struct ExpertWalk {
 };
 
 // GATHER: row r of the GEMM is row a_rows[r] of a and a_s.
-template <class Cfg, int EPI, bool GATHER>
+// AHEAD: fragments are read one step ahead of their use, in a loop without branches while an expert's tiles are full; else
+// when they are needed, by the waves that need them.  Ahead is for experts of more rows than a tile has: masked layout, 32
+// experts x 0 .. 256 rows, 7168 x 2048 130 -> 116 us (128 x 256 tiles; the ring kernel 141), 16 x 0 .. 128 rows, 1024 x 3072
+// 20.3 -> 19.1 us.  Short experts lose by it (8 experts, 12 rows, 3200 x 1280: 9.7 -> 10.9 us): most of their steps take the
+// path with the branches.
+template <class Cfg, int EPI, bool GATHER, bool AHEAD>
 __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) {
-  constexpr int BM = Cfg::BM, BN = Cfg::BN, MF = Cfg::MF, NF = Cfg::NF, WAVES = Cfg::WAVES, STAGES = Cfg::STAGES;
+  constexpr int BM = Cfg::BM, BN = Cfg::BN, MF = Cfg::MF, NF = Cfg::NF, WAVES = Cfg::WAVES, WGM = Cfg::WGM, STAGES = Cfg::STAGES;
   constexpr bool kAct = EPI != kStoreProduct;
   static_assert(!kAct || BN == 256, "a quantisation group is the 128 output columns of 256 weight rows");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int l32 = lane & 31, h = lane >> 5;
-  const int wm0 = (wave / Cfg::WGN) * (MF * 32);
-  const int wn0 = (wave % Cfg::WGN) * (NF * 32);
+  const int wrow = wave / Cfg::WGN;  // the wave's fragment mi is the tile's fragment mi WGM + wrow: wave rows share short tiles evenly
   const LaneChunks lc = make_lane_chunks(l32, h);
   const int nk = p.kblocks;
   const int grid = static_cast<int>(gridDim.x);
@@ -139,8 +157,11 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     const int local = rel - (__builtin_amdgcn_readlane(ew.incl, i) - mtiles * p.tiles_n);
     const int nt = local / mtiles, mt = local - nt * mtiles;
     t.g = ew.first + i;
-    t.row = __builtin_amdgcn_readlane(ew.row0, i) + mt * BM;
-    t.rows = min(BM, __builtin_amdgcn_readlane(ew.rows, i) - mt * BM);
+    // the row tiles of an expert are equally high (in fragments): they run side by side and share its weights in the L2
+    const int rows = __builtin_amdgcn_readlane(ew.rows, i);
+    const int height = ((rows + 31) / 32 + mtiles - 1) / mtiles * 32;
+    t.row = __builtin_amdgcn_readlane(ew.row0, i) + mt * height;
+    t.rows = min(height, rows - mt * height);
     t.n0 = nt * (kAct ? BN / 2 : BN);
     t.ok = true;
     return t;
@@ -197,10 +218,19 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     }
   };
 
+  auto issue_loads = [&]() __attribute__((always_inline)) {
+    uint8_t* sbase = smem + it_stage * Cfg::STAGE_BYTES;
+    const uint32_t koff = static_cast<uint32_t>(it_kb) * kScaleBlock;
+#pragma unroll
+    for (int j = 0; j < Cfg::B_INST; ++j) buf_dma_16<kDmaStream>(b_src, b_off[j], koff, sbase + Cfg::A_BYTES + (j * WAVES + wave) * 1024);
+#pragma unroll
+    for (int j = 0; j < Cfg::A_INST; ++j) buf_dma_16<kDmaKeep>(a_src, a_off[j], koff, sbase + (j * WAVES + wave) * 1024);
+    ++it_kb;
+    it_stage = it_stage + 1 == STAGES ? 0 : it_stage + 1;
+  };
   auto issue_step = [&]() {
     if (it.ok && it_kb == nk) enter_tile();
     if (!it.ok) return;
-    uint8_t* sbase = smem + it_stage * Cfg::STAGE_BYTES;
     if (it_kb == it_chunk_kb) {
       // this step opens a chunk of the scale table
       const int len = min(p.chunk_len, nk - it_kb);
@@ -219,13 +249,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
       it_tab ^= 1;
       it_chunk_kb += p.chunk_len;
     }
-    const uint32_t koff = static_cast<uint32_t>(it_kb) * kScaleBlock;
-#pragma unroll
-    for (int j = 0; j < Cfg::B_INST; ++j) buf_dma_16<kDmaStream>(b_src, b_off[j], koff, sbase + Cfg::A_BYTES + (j * WAVES + wave) * 1024);
-#pragma unroll
-    for (int j = 0; j < Cfg::A_INST; ++j) buf_dma_16<kDmaKeep>(a_src, a_off[j], koff, sbase + (j * WAVES + wave) * 1024);
-    ++it_kb;
-    it_stage = it_stage + 1 == STAGES ? 0 : it_stage + 1;
+    issue_loads();
   };
 
   load_window(0, 0);
@@ -233,12 +257,16 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
   if (!it.ok) return;
   Tile ct = it;  // the tile the compute side works on
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s) issue_step();
+  for (int s = 0; s < (AHEAD ? STAGES : STAGES - 1); ++s) issue_step();
 
   // ---- compute side ------------------------------------------------------------------------------------------------
-  // A step reads its fragments when it needs them: the stream from HBM, not the matrix pipe, sets the pace here, and a
-  // wave whose rows are all past the expert's last one skips its reads.  (The software-pipelined loop of
-  // fp8_gemm_pipelined.h on the same ring, which reads and multiplies all 128 rows: 182 against 146 us at ~16 rows.)
+  // AHEAD: the fragments of a K block are in registers when its step begins; each is replaced by the next block's as soon as
+  // the last matrix instruction that reads it has been issued.  Most steps open no tile and no chunk of the scale table and
+  // have valid rows in every fragment: those run in a loop of their own (run_fast) without a branch; the others skip
+  // fragments whose rows are all past the expert's last one, reads included.  (With the checks in every step their 150 scalar
+  // instructions were the bound: 1.1 us a 128 x 256 step without any load, now 0.85.  A loop for every number of live
+  // fragments made the compiler spill: 2.8 x slower.)
+  const int wn0 = (wave % Cfg::WGN) * (NF * 32);
   int frag_off[NF];  // lane-dependent for the quantising epilogue
 #pragma unroll
   for (int ni = 0; ni < NF; ++ni) {
@@ -246,72 +274,219 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     // row 128 + 16 f + (l32 - 16); row & 15 is the same, so the lane's swizzled chunk offsets hold
     frag_off[ni] = Cfg::A_BYTES + (kAct ? ((wave % Cfg::WGN) * NF + ni) * 16 + (l32 >= 16 ? BN / 2 - 16 : 0) : wn0 + ni * 32) * kScaleBlock;
   }
-  int stage = 0, tab = 0;
+  v8i x[MF][2], w[NF][2];
+  float sa[MF];
+  int base = 0;                     // ring stage (in bytes) of the block whose fragments are read next
+  int tab = 0;                      // its buffer of the scale table
+  int tab_kb = 0, chunk_end = 0;    // its number in its chunk; the first block of the chunk after it
+  const float* tab_ptr = nullptr;
+  auto frag_row = [&](int mi) { return (mi * WGM + wrow) * 32; };
+  auto read_x = [&](int mi) __attribute__((always_inline)) {
+    x[mi][0] = lds_read_frag32(smem, base + frag_row(mi) * kScaleBlock, lc, 0);
+    x[mi][1] = lds_read_frag32(smem, base + frag_row(mi) * kScaleBlock, lc, 1);
+    sa[mi] = tab_ptr[(frag_row(mi) + l32) * tab_rs + tab_kb * tab_js];
+  };
+  auto read_w = [&](int ni) __attribute__((always_inline)) {
+    w[ni][0] = lds_read_frag32(smem, base + frag_off[ni], lc, 0);
+    w[ni][1] = lds_read_frag32(smem, base + frag_off[ni], lc, 1);
+  };
+  auto next_stage = [&]() __attribute__((always_inline)) { base = base + Cfg::STAGE_BYTES == STAGES * Cfg::STAGE_BYTES ? 0 : base + Cfg::STAGE_BYTES; };
+  auto enter_block = [&](int kb) {  // block kb of a tile is the one whose fragments are read next
+    ++tab_kb;
+    if (kb == 0) chunk_end = 0;
+    if (kb == chunk_end) {
+      tab_ptr = reinterpret_cast<const float*>(smem + Cfg::TAB_OFF + tab * Cfg::TAB_BYTES);
+      tab ^= 1;
+      tab_kb = 0;
+      chunk_end += p.chunk_len;
+    }
+  };
+  // weight scales of the wave's columns: one 128-block per wave (kAct: one for the gate, one for the up half)
+  const_float_ptr_t bs0, bs1;
+  auto enter_scales = [&](const Tile& t) {
+    const float* bs_g = p.b_s + static_cast<int64_t>(t.g) * p.bs_gs;
+    const int nb0 = kAct ? t.n0 / kScaleBlock : min((t.n0 + wn0) / kScaleBlock, p.nblocks - 1);
+    bs0 = (const_float_ptr_t)(bs_g + static_cast<int64_t>(nb0) * nk);
+    bs1 = (const_float_ptr_t)(bs_g + static_cast<int64_t>(kAct ? nb0 + p.act_cols / kScaleBlock : nb0) * nk);
+  };
+  auto multiply = [&](int ni, int mi) __attribute__((always_inline)) {
+    v16f z;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) z[u] = 0.f;
+    z = mfma_32x32x64_e4m3(w[ni][0], x[mi][0], z);
+    return mfma_32x32x64_e4m3(w[ni][1], x[mi][1], z);
+  };
+  v16f acc[MF][NF];
+  float sb0, sb1;
+  auto accumulate = [&](int mi, int ni, const v16f& z, float s0, float s1) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) acc[mi][ni][u] = fmaf(z[u], kAct && u >= 8 ? s1 : s0, acc[mi][ni][u]);
+  };
+
+  if constexpr (AHEAD) {
+    enter_scales(ct);
+    sb0 = bs0[0], sb1 = bs1[0];
+    wait_vmcnt<(STAGES - 1) * Cfg::L>();
+    lds_barrier();
+    enter_block(0);
+#pragma unroll
+    for (int mi = 0; mi < MF; ++mi)
+      if (frag_row(mi) < ct.rows) read_x(mi);
+#pragma unroll
+    for (int ni = 0; ni < NF; ++ni) read_w(ni);
+  }
+
+  // n steps from block kb on: the block after each is in the same tile and chunk, and so is what each issues
+  auto run_fast = [&](int kb, int n) __attribute__((always_inline)) {
+    const_float_ptr_t q0 = bs0 + kb + 1, q1 = bs1 + kb + 1;
+#pragma unroll 1
+    for (; n > 0; --n, ++q0, ++q1) {
+      v16f z[NF];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ni = 0; ni < NF; ++ni) z[ni] = multiply(ni, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      // the next block's loads have landed, and every wave holds this block in registers: its stage can be refilled
+      wait_vmcnt<(STAGES - 2) * Cfg::L>();
+      lds_barrier();
+      float s0[MF], s1[MF];
+#pragma unroll
+      for (int mi = 0; mi < MF; ++mi) s0[mi] = sa[mi] * sb0, s1[mi] = sa[mi] * sb1;
+      sb0 = *q0;
+      if (kAct) sb1 = *q1;
+      else sb1 = sb0;
+      issue_loads();
+      next_stage();
+      ++tab_kb;
+      if (MF == 1) {
+#pragma unroll
+        for (int ni = 0; ni < NF; ++ni) read_w(ni);
+      }
+      read_x(0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ni = 0; ni < NF; ++ni) accumulate(0, ni, z[ni], s0[0], s1[0]);
+#pragma unroll
+      for (int mi = 1; mi < MF; ++mi) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ni = 0; ni < NF; ++ni) {
+          z[ni] = multiply(ni, mi);
+          if (mi == MF - 1) {
+            __builtin_amdgcn_sched_barrier(0);
+            read_w(ni);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        read_x(mi);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ni = 0; ni < NF; ++ni) accumulate(mi, ni, z[ni], s0[mi], s1[mi]);
+      }
+    }
+  };
+
   while (true) {
-    v16f acc[MF][NF];
+    if (!AHEAD) {
+      enter_scales(ct);
+      sb0 = bs0[0], sb1 = bs1[0];
+    }
 #pragma unroll
     for (int mi = 0; mi < MF; ++mi)
 #pragma unroll
       for (int ni = 0; ni < NF; ++ni)
 #pragma unroll
         for (int t = 0; t < 16; ++t) acc[mi][ni][t] = 0.f;
-    // weight scales of the wave's columns: one 128-block per wave (kAct: one for the gate, one for the up half)
-    const float* bs_g = p.b_s + static_cast<int64_t>(ct.g) * p.bs_gs;
-    const int nb0 = kAct ? ct.n0 / kScaleBlock : min((ct.n0 + wn0) / kScaleBlock, p.nblocks - 1);
-    const const_float_ptr_t bs0 = (const_float_ptr_t)(bs_g + static_cast<int64_t>(nb0) * nk);
-    const const_float_ptr_t bs1 = (const_float_ptr_t)(bs_g + static_cast<int64_t>(kAct ? nb0 + p.act_cols / kScaleBlock : nb0) * nk);
-    float sb0 = bs0[0], sb1 = bs1[0];
-    int chunk_end = 0, chunk_kb = 0;
-    const float* tab_ptr = nullptr;
+    const bool full = AHEAD && frag_row(MF - 1) < ct.rows;
 
-    for (int kb = 0; kb < nk; ++kb) {
-      // the loads of this step have landed: behind them at most the groups of the next STAGES - 2 steps are out
-      if (it.ok)
-        wait_vmcnt<(STAGES - 2) * Cfg::L>();
-      else
-        wait_vmcnt<0>();
-      lds_barrier();  // ... those of every wave, and nobody reads the stage before this one any more
-      issue_step();
-      if (kb == chunk_end) {
-        tab_ptr = reinterpret_cast<const float*>(smem + Cfg::TAB_OFF + tab * Cfg::TAB_BYTES);
-        tab ^= 1;
-        chunk_kb = kb;
-        chunk_end += p.chunk_len;
-      }
-      const int base = stage * Cfg::STAGE_BYTES;
-      if (BM == 32 || wm0 < ct.rows) {
-        v8i w[NF][2];
-#pragma unroll
-        for (int ni = 0; ni < NF; ++ni) {
-          w[ni][0] = lds_read_frag32(smem, base + frag_off[ni], lc, 0);
-          w[ni][1] = lds_read_frag32(smem, base + frag_off[ni], lc, 1);
+    for (int kb = 0; AHEAD && kb < nk; ++kb) {
+      if (full && it.ok) {
+        const int n = min(min(nk, it_chunk_kb) - it_kb, min(nk, chunk_end) - 1 - kb);
+        if (n > 0) {
+          run_fast(kb, n);
+          kb += n;
         }
+      }
+      float s0[MF], s1[MF];
 #pragma unroll
-        for (int mi = 0; mi < MF; ++mi) {
-          if (mi > 0 && wm0 + mi * 32 >= ct.rows) continue;  // no valid row in this fragment
-          const v8i x0 = lds_read_frag32(smem, base + (wm0 + mi * 32) * kScaleBlock, lc, 0);
-          const v8i x1 = lds_read_frag32(smem, base + (wm0 + mi * 32) * kScaleBlock, lc, 1);
-          const float sa = tab_ptr[(wm0 + mi * 32 + l32) * tab_rs + (kb - chunk_kb) * tab_js];
-          const float s0 = sa * sb0, s1 = sa * sb1;
+      for (int mi = 0; mi < MF; ++mi) s0[mi] = sa[mi] * sb0, s1[mi] = sa[mi] * sb1;
+      int rows_n = 0, kb_n = 0;
 #pragma unroll
-          for (int ni = 0; ni < NF; ++ni) {
-            v16f z;
+      for (int mi = 0; mi < MF; ++mi) {
+        if (frag_row(mi) < ct.rows) {
+          v16f z[NF];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) z[u] = 0.f;
-            z = mfma_32x32x64_e4m3(w[ni][0], x0, z);
-            z = mfma_32x32x64_e4m3(w[ni][1], x1, z);
+          for (int ni = 0; ni < NF; ++ni) z[ni] = multiply(ni, mi);
 #pragma unroll
-            for (int u = 0; u < 16; ++u) acc[mi][ni][u] = fmaf(z[u], kAct && u >= 8 ? s1 : s0, acc[mi][ni][u]);
+          for (int ni = 0; ni < NF; ++ni) accumulate(mi, ni, z[ni], s0[mi], s1[mi]);
+        }
+        if (mi == 0) {
+          // younger than the next block's loads: those of STAGES - 2 steps, fewer at the end of the last tile
+          wait_groups<Cfg::L, STAGES - 2>(it.ok ? STAGES - 2 : nk - 2 - kb);
+          lds_barrier();
+          issue_step();
+          next_stage();
+          if (kb + 1 < nk) {
+            kb_n = kb + 1;
+            rows_n = ct.rows;
+          } else {
+            // the issue side is in the next tile: nk >= STAGES
+            rows_n = it.ok ? it.rows : 0;
+            if (it.ok) enter_scales(it);
           }
+          enter_block(kb_n);
+          sb0 = bs0[kb_n];
+          sb1 = bs1[kb_n];
         }
+        if (frag_row(mi) < rows_n) read_x(mi);
       }
-      const int kn = min(kb + 1, nk - 1);
-      sb0 = bs0[kn];
-      sb1 = bs1[kn];
-      stage = stage + 1 == STAGES ? 0 : stage + 1;
+      if (frag_row(0) < rows_n) {
+#pragma unroll
+        for (int ni = 0; ni < NF; ++ni) read_w(ni);
+      }
     }
 
-    // ---- epilogue: lane holds rows wm0 + 32 mi + l32, weight rows 8 u + 4 h + 0..3 of every fragment, u = 0..3 -------
+    if constexpr (!AHEAD) {
+      for (int kb = 0; kb < nk; ++kb) {
+        // the loads of this step have landed: behind them at most the groups of the next STAGES - 2 steps are out
+        wait_groups<Cfg::L, STAGES - 2>(it.ok ? STAGES - 2 : nk - 1 - kb);
+        lds_barrier();  // ... those of every wave, and nobody reads the stage before this one any more
+        issue_step();
+        enter_block(kb);
+        if (WGM == 1 || frag_row(0) < ct.rows) {
+          v8i wf[NF][2];
+#pragma unroll
+          for (int ni = 0; ni < NF; ++ni) {
+            wf[ni][0] = lds_read_frag32(smem, base + frag_off[ni], lc, 0);
+            wf[ni][1] = lds_read_frag32(smem, base + frag_off[ni], lc, 1);
+          }
+#pragma unroll
+          for (int mi = 0; mi < MF; ++mi) {
+            if (mi > 0 && frag_row(mi) >= ct.rows) continue;  // no valid row in this fragment
+            const v8i x0 = lds_read_frag32(smem, base + frag_row(mi) * kScaleBlock, lc, 0);
+            const v8i x1 = lds_read_frag32(smem, base + frag_row(mi) * kScaleBlock, lc, 1);
+            const float sk = tab_ptr[(frag_row(mi) + l32) * tab_rs + tab_kb * tab_js];
+            const float s0 = sk * sb0, s1 = sk * sb1;
+#pragma unroll
+            for (int ni = 0; ni < NF; ++ni) {
+              v16f z;
+#pragma unroll
+              for (int u = 0; u < 16; ++u) z[u] = 0.f;
+              z = mfma_32x32x64_e4m3(wf[ni][0], x0, z);
+              z = mfma_32x32x64_e4m3(wf[ni][1], x1, z);
+              accumulate(mi, ni, z, s0, s1);
+            }
+          }
+        }
+        const int kn = min(kb + 1, nk - 1);
+        sb0 = bs0[kn];
+        sb1 = bs1[kn];
+        next_stage();
+      }
+    }
+
+    // ---- epilogue: lane holds rows frag_row(mi) + l32, weight rows 8 u + 4 h + 0..3 of every fragment, u = 0..3 -------
     if constexpr (kAct) {
       // u = 0, 1: gate, u = 2, 3: up of output columns c0 + 8 u + 4 h + 0..3.  The values pass through bf16 as the plain
       // GEMM would have stored them, so codes and scales have the bits of the three separate steps.
@@ -335,12 +510,12 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
             amax[mi] = fmaxf(amax[mi], fabsf(v));
           }
         amax[mi] = fmaxf(amax[mi], __shfl_xor(amax[mi], 32));
-        if (h == 0) maxima[(wave % Cfg::WGN) * BM + wm0 + mi * 32 + l32] = amax[mi];
+        if (h == 0) maxima[(wave % Cfg::WGN) * BM + frag_row(mi) + l32] = amax[mi];
       }
       lds_barrier();
 #pragma unroll
       for (int mi = 0; mi < MF; ++mi) {
-        const int row = wm0 + mi * 32 + l32;
+        const int row = frag_row(mi) + l32;
 #pragma unroll
         for (int w2 = 0; w2 < Cfg::WGN; ++w2) amax[mi] = fmaxf(amax[mi], maxima[w2 * BM + row]);
         const float scale = fmaxf(amax[mi], p.act_eps) / 448.0f;
@@ -372,7 +547,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     } else {
 #pragma unroll
       for (int mi = 0; mi < MF; ++mi) {
-        const int row = wm0 + mi * 32 + l32;
+        const int row = frag_row(mi) + l32;
         const bool live = row < ct.rows;
         char* c_row = static_cast<char*>(p.c) + static_cast<int64_t>(ct.row + row) * p.N * (p.out_f32 ? 4 : 2);
 #pragma unroll

@@ -350,7 +350,8 @@ int dlb_fp8_gemm_plan_wave_k(int64_t M, int64_t N, int64_t K, size_t workspace_b
  * the masked layout (mode 2), the caller's expected_m (<= 0: unknown).  mode 1 = contiguous (rows = M_sum), 2 = masked
  * (rows = M_max).  Outputs (each may be NULL): the kernel variant id; whether a contiguous launch of this size pairs
  * blocks into taller tiles from lists built on the device (1) or runs uniform 128-row tiles (0); for the masked layout,
- * whether the weight-streaming kernel for short experts runs in place of the named variant (1).  The fused gate/up
+ * whether the weight-streaming kernel runs in place of the named variant, at row counts where its form with the
+ * quantising epilogue does too (1).  The fused gate/up
  * entry points always take the lists, so a caller that can also run GEMM and activation apart does that where this
  * says 0 (a batch of at most a round or two of tiles, where the uniform tiles are faster).  No counterpart in the
  * reference.

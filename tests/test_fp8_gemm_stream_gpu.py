@@ -11,6 +11,7 @@ from oracle import fp8_block_gemm as orc
 pytestmark = pytest.mark.gpu
 
 SHAPES = ['32x256', '64x256', '64x128', '128x256', '64x64']
+AHEAD = ['64x256 ahead', '64x128 ahead', '128x256 ahead', '64x64 ahead']  # knob values 8 .. 11
 
 
 @pytest.fixture(scope='module')
@@ -40,7 +41,10 @@ def _inputs(masked, M_max, N, K, seed, dev):
     ([5, 200, 0, 17], 200, 130, 1152, torch.float32, False),            # N no multiple of 8: element stores
     ([i % 4 for i in range(70)], 8, 128, 1024, torch.float32, True),    # a second window of 64 experts
     ([0, 0, 0], 32, 256, 1024, torch.bfloat16, False),                  # nothing to do
-    ([40, 100], 100, 384, 256, torch.bfloat16, False),                  # 2 K blocks: only the three-stage rings
+    ([40, 100], 100, 384, 256, torch.bfloat16, False),                  # 2 K blocks: shorter than every ring
+    ([128, 64, 97], 128, 256, 384, torch.bfloat16, True),               # 3 K blocks: as short as the three-stage rings
+    ([150, 256, 300, 129] * 5, 304, 2048, 1152, torch.bfloat16, False), # several tiles per workgroup, most of them full
+    ([190, 70, 0, 33] * 6, 192, 1160, 2304, torch.float32, True),       # 18 blocks in two chunks; full and short tiles in turn
 ])
 def test_masked_equals_the_ring_kernels(dev, masked, M_max, N, K, out_dtype, col_major):
     from dlblas_amd import _lib
@@ -49,15 +53,15 @@ def test_masked_equals_the_ring_kernels(dev, masked, M_max, N, K, out_dtype, col
     if col_major:
         a_s = a_s.transpose(1, 2).contiguous().transpose(1, 2)
     outs = []
-    for knob in [1] + [2 + i for i in range(len(SHAPES))]:
-        print(f'case stream masked={masked[:6]} M_max={M_max} N={N} K={K} {out_dtype} shape={"ring" if knob == 1 else SHAPES[knob - 2]}', flush=True)
+    for knob, shape in zip([1, 2, 3, 4, 5, 6, 8, 9, 10, 11], ['ring'] + SHAPES + AHEAD):
+        print(f'case stream masked={masked[:6]} M_max={M_max} N={N} K={K} {out_dtype} shape={shape}', flush=True)
         out = torch.full((len(masked), M_max, N), -555.0, dtype=out_dtype, device=dev)
         _lib.tune('stream', knob)
         m_grouped_fp8_gemm_nt_masked((a_q, a_s), (w_q, w_s), out, mm, 0)
         torch.cuda.synchronize()
         _lib.tune('stream', 0)
         outs.append(out)
-    for shape, out in zip(SHAPES, outs[1:]):
+    for shape, out in zip(SHAPES + AHEAD, outs[1:]):
         assert torch.equal(out, outs[0]), shape
     ref = orc.grouped_masked_ref(a_q.cpu(), a_s.cpu(), w_q.cpu(), w_s.cpu(), torch.full((len(masked), M_max, N), -555.0), mm.cpu())
     valid = torch.arange(M_max)[None, :] < mm.cpu()[:, None]
