@@ -4,11 +4,12 @@
 // waited for the host (1 x 2112 x 7168: 19.6 us per call, 6.0 us of it the kernel).
 //
 // Every function takes the arguments of the Python function of its name and either does the call or returns None without
-// having enqueued anything.  None means "not a plain call": tensor subclasses, dispatch modes, tracing, inputs that require
-// grad, arguments the checks refuse, layouts only the Python path handles.  The Python function then goes on as it would
-// without this module, through its custom op and its own checks and messages.
+// having enqueued anything.  None means "not a plain call": tensor subclasses, dispatch and function modes, tracing, inputs
+// that require grad, arguments the checks refuse, layouts only the Python path handles.  The Python function then goes on as
+// it would without this module, through its custom op and its own checks and messages.
 #include <Python.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DefaultDtype.h>
@@ -61,7 +62,7 @@ const c10::DispatchKeySet kPlainIncluded({c10::DispatchKey::BackendSelect, c10::
 // (raw bits: set difference on DispatchKeySet leaves the backend bits alone)
 bool within(c10::DispatchKeySet keys, c10::DispatchKeySet allowed) { return (keys.raw_repr() & ~allowed.raw_repr()) == 0; }
 
-bool no_modes() { return within(c10::impl::tls_local_dispatch_key_set().included_, kPlainIncluded); }
+bool no_modes() { return within(c10::impl::tls_local_dispatch_key_set().included_, kPlainIncluded) && !at::impl::torch_function_mode_enabled(); }
 
 // A dense GPU tensor that nothing but its own storage stands behind; nullptr otherwise.
 const at::Tensor* plain(PyObject* o) {

@@ -85,6 +85,17 @@ def test_other_calls_are_left_to_the_python_path(dev):
     with FakeTensorMode() as mode:
         fake = [mode.from_tensor(t) for t in (a, b, a_s, b_s)]
         assert _fast.fp8_gemm(*fake) is None and tuple(fp8_gemm(*fake).shape) == (16, 128)
+
+    class Calls(torch.overrides.TorchFunctionMode):
+        seen = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Calls():
+        fp8_gemm(a, b, a_s, b_s)
+    assert any('dlblas.fp8_gemm' in f for f in Calls.seen)
     with pytest.raises(AssertionError, match='contiguous'):
         fp8_gemm(a[:, ::2], b, a_s, b_s)
     with pytest.raises(ValueError):
