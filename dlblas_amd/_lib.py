@@ -34,6 +34,8 @@ SYMBOLS = {
     'dlb_fp8_gemm_noalloc': (ctypes.c_int, [_c_vp] * 5 + [_c_i64] * 5 + [ctypes.c_int, _c_vp]),
     'dlb_fp8_gemm_grouped_contiguous':
     (ctypes.c_int, [_c_vp] * 6 + [_c_i64] * 3 + [_c_i32] + [_c_i64] * 2 + [ctypes.c_int, _c_vp, _c_sz, _c_vp]),
+    'dlb_fp8_gemm_grouped_contiguous_same_rows':
+    (ctypes.c_int, [_c_vp] * 6 + [_c_i64] * 3 + [_c_i32] + [_c_i64] * 2 + [ctypes.c_int, _c_vp, _c_sz, _c_vp]),
     'dlb_fp8_gemm_grouped_contiguous_silu_quant':
     (ctypes.c_int, [_c_vp] * 7 + [_c_i64] * 3 + [_c_i32] + [_c_i64] * 4 + [ctypes.c_float, _c_vp, _c_sz, _c_vp]),
     'dlb_fp8_gemm_grouped_contiguous_gather_silu_quant':

@@ -948,6 +948,7 @@ struct Problem {
   float act_eps = 0.f;
   bool act = false;
   int64_t hint_rows = -1;  // masked layout: the caller's expected_m
+  bool list_there = false;  // contiguous: the workspace still holds the tile lists of these rows
 };
 
 
@@ -1287,11 +1288,14 @@ int run(const Problem& pr) {
     ar.as_gs = kblocks * rs.rows_pad;
   }
   if (tile_list && !one_prepass) {
-    // expert-contiguous rows: device-built lists of 256-, 192- and 128-row tiles (see contiguous_tile_list_block)
+    // expert-contiguous rows: device-built lists of 256-, 192- and 128-row tiles (see contiguous_tile_list_block); they depend
+    // on the rows and the experts only and lie at the same place for every N and K
     int32_t* tl = reinterpret_cast<int32_t*>(ar.ws);
-    hipLaunchKernelGGL(contiguous_tile_list_kernel, dim3(1), dim3(256), 0, pr.stream, pr.gidx, static_cast<int>(pr.rows), pr.G, tl,
-                       static_cast<int>(rs.nblk));
-    e = hipGetLastError();
+    if (!pr.list_there) {
+      hipLaunchKernelGGL(contiguous_tile_list_kernel, dim3(1), dim3(256), 0, pr.stream, pr.gidx, static_cast<int>(pr.rows), pr.G, tl,
+                         static_cast<int>(rs.nblk));
+      e = hipGetLastError();
+    }
     if (e != hipSuccess) return fail(DLB_ERR_LAUNCH, "tile list launch failed: %s", hipGetErrorString(e));
     ar.tlist = tl;
     ar.tlist_cap = static_cast<int>(rs.nblk);
@@ -1436,6 +1440,16 @@ int dlb_fp8_gemm_grouped_contiguous(const void* a, const void* b, const float* a
                                     size_t workspace_bytes, void* stream) {
   dlb::Problem pr{dlb::kContiguous, a, b, a_s, b_s, c, m_indices, M_sum, N, K, G, 0, as_stride_m, as_stride_k,
                   out_dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream)};
+  return dlb::run(pr);
+}
+
+int dlb_fp8_gemm_grouped_contiguous_same_rows(const void* a, const void* b, const float* a_s, const float* b_s, void* c,
+                                              const int32_t* m_indices, int64_t M_sum, int64_t N, int64_t K, int32_t G,
+                                              int64_t as_stride_m, int64_t as_stride_k, int out_dtype, void* workspace,
+                                              size_t workspace_bytes, void* stream) {
+  dlb::Problem pr{dlb::kContiguous, a, b, a_s, b_s, c, m_indices, M_sum, N, K, G, 0, as_stride_m, as_stride_k,
+                  out_dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream)};
+  pr.list_there = true;
   return dlb::run(pr);
 }
 

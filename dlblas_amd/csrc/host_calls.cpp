@@ -39,6 +39,7 @@ struct Abi {
   decltype(&dlb_last_error) last_error;
   decltype(&dlb_fp8_gemm) gemm;
   decltype(&dlb_fp8_gemm_grouped_contiguous) contiguous;
+  decltype(&dlb_fp8_gemm_grouped_contiguous_same_rows) contiguous_same_rows;
   decltype(&dlb_fp8_gemm_grouped_contiguous_gather_silu_quant) contiguous_gather_act;
   decltype(&dlb_fp8_gemm_grouped_masked) masked;
   decltype(&dlb_fp8_gemm_grouped_masked_silu_quant) masked_act;
@@ -465,7 +466,8 @@ PyObject* fused_moe_v3(PyObject*, PyObject* const* args, Py_ssize_t n) {
                                    x_s.stride(1), s_m, s_k, 1e-10f, ws.ptr, ws.bytes, stream);
     if (rc == DLB_ERR_BAD_SHAPE) NOT_PLAIN;  // the Python path starts over with the three steps
     if (rc == DLB_OK)
-      rc = abi.contiguous(ptr(q), ptr(w2), fptr(s), fptr(w2_s), ptr(down), row_expert, rows, H, inter, g, s_m, s_k, DLB_OUT_BF16, ws.ptr, ws.bytes, stream);
+      rc = abi.contiguous_same_rows(ptr(q), ptr(w2), fptr(s), fptr(w2_s), ptr(down), row_expert, rows, H, inter, g, s_m, s_k, DLB_OUT_BF16, ws.ptr,
+                                    ws.bytes, stream);
   }
   if (rc == DLB_OK) rc = gather(down, ids, weights, slot_row, out, stream);
   if (rc != DLB_OK) return launch_failed(rc);

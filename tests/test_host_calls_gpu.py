@@ -128,3 +128,37 @@ def test_streams_and_threads_share_the_workspaces_of_the_python_path(dev):
         t.join()
     assert not failed, failed
     assert len(results) == 3 and all(results.values())
+
+
+@pytest.mark.parametrize('tokens,E', [(40, 3), (300, 2), (3000, 6)])
+def test_fused_moe_v3_with_the_tile_lists_kept_equals_the_steps(dev, tokens, E):
+    """The native expert MLP leaves the tile lists of the first GEMM to the second; under a function mode the Python path
+    builds them for each.  Runs of 1, 2, 3 and more blocks per expert, an expert without rows, twice on one workspace."""
+    from dlblas_amd import _fast, _lib
+    from dlblas_amd.kernels.fp8 import per_block_quant_fp8, per_token_group_quant_fp8
+    from dlblas_amd.kernels.fused_moe_v3 import fused_moe_v3
+    H, inter = 512, 256
+    g = helpers.gen(9)
+
+    def weights(n, k):
+        q, s = zip(*(per_block_quant_fp8((torch.randn(n, k, generator=g) * 0.05).to(torch.bfloat16).to(dev)) for _ in range(E)))
+        return torch.stack(q), torch.stack(s)
+
+    w13, w2 = weights(2 * inter, H), weights(H, inter)
+    x = per_token_group_quant_fp8(torch.randn(tokens, H, generator=g).to(torch.bfloat16).to(dev), 128)
+    share = torch.arange(1, E + 1).float()
+    share[0] = 0
+    try:
+        for knob, value in (('tile_list', 1), ('stream', 1)):
+            _lib.tune(knob, value)
+        for _ in range(2):
+            ids = torch.multinomial(share, 2 * tokens, replacement=True, generator=g).view(tokens, 2)
+            counts = ((torch.bincount(ids.flatten(), minlength=E) + 127) // 128 * 128).tolist()
+            args = ids.to(dev), torch.rand(tokens, 2, generator=g).to(dev), w13, w2, counts
+            out = _fast.fused_moe_v3(*x, *args[:2], *w13, *w2, counts)
+            with torch.overrides.BaseTorchFunctionMode():
+                ref = fused_moe_v3(x, *args)
+            torch.cuda.synchronize()
+            assert out is not None and torch.equal(out, ref)
+    finally:
+        _lib.tune('tile_list', 0), _lib.tune('stream', 0)
