@@ -395,11 +395,16 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
     store_index(p.out_index, p.oi_is64, t * p.oi_s0 + (tid % p.topk_n) * p.oi_s1, d);
     if (d < p.m_len) p.src_row[d] = static_cast<int32_t>(t);
   }
-  // rows [0, excl[E]) in slices over the blocks: their expert, and token 0 for the rows that no slot is given
+  // the rows in slices over the blocks: their expert below excl[E], and token 0 for every row that no slot is given.  That
+  // includes the rows of a longer table past the spans: readers of src_row follow every entry, whatever m_indices says
   const int total = static_cast<int>(min(static_cast<int64_t>(excl[E]), p.m_len));
-  const int per = (total + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x);
-  const int r1 = min(total, (b + 1) * per);
-  for (int r = b * per + tid; r < r1; r += kRowsThreads) {
+  const int64_t per = (p.m_len + gridDim.x - 1) / gridDim.x;
+  const int64_t r1 = min(p.m_len, (b + 1) * per);
+  for (int64_t r = b * per + tid; r < r1; r += kRowsThreads) {
+    if (r >= total) {
+      p.src_row[r] = 0;
+      continue;
+    }
     int lo = 0, hi = E;  // largest e with excl[e] <= r
     while (hi - lo > 1) {
       const int mid = (lo + hi) >> 1;

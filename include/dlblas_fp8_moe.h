@@ -99,7 +99,7 @@ int dlb_ep_scatter(const void* recv_x, int64_t x_row_stride, const float* recv_x
 /*
  * The tables of dlb_ep_scatter without the copy: m_indices, expert_start_loc and output_index exactly as that call
  * leaves them, plus src_row [m_indices_len] int32 = the token whose row dlb_ep_scatter would have copied to each
- * destination row (0 for the rows of an expert's span that no slot is copied to).  No row of recv_x is read or written:
+ * destination row (0 for every row that no slot is copied to, a longer table's rows past the last span among them).  No row of recv_x is read or written:
  * dlb_fp8_gemm_grouped_contiguous_gather_silu_quant reads the tokens through src_row.  No counterpart in the
  * reference, whose ep_scatter always copies (dlblas/kernels/fused_moe_v3.py:95-158).  Workspace as dlb_ep_scatter.
  */

@@ -173,3 +173,63 @@ def test_row_tables_around_the_one_launch_limit(dev, T, topk, E):
     src_ref = torch.zeros(rows, dtype=torch.long)
     src_ref[rank[flat >= 0]] = (torch.arange(flat.numel()) // topk)[flat >= 0]
     assert torch.equal(src.cpu().long(), src_ref)
+
+
+def _row_tables_ref(ids, counts):
+    """Tables of the stable counting sort: first row of every expert, destination row of every slot (-9: none), token of
+    every destination row (0 where no slot lies)."""
+    flat = ids.flatten()
+    excl = torch.cumsum(counts, 0) - counts
+    routed = torch.bincount(flat[flat >= 0], minlength=len(counts))
+    dest = torch.full_like(flat, -9)
+    order = torch.sort(flat, stable=True).indices[int((flat < 0).sum()):]
+    dest[order] = torch.cat([torch.arange(int(a), int(a) + int(n)) for a, n in zip(excl, routed)])
+    return excl, routed, dest
+
+
+@pytest.mark.parametrize('T,topk,E', [(33, 4, 5), (2100, 8, 40), (5000, 8, 300)])
+def test_row_tables_longer_than_the_spans(dev, T, topk, E):
+    """A table of fixed capacity: its rows past the experts' spans name token 0, whichever of the three forms of the kernel
+    fills it (the ids ranked in one launch, summed histograms, scanned histograms), and keep the -1 that the caller put
+    into m_indices."""
+    from dlblas_amd.kernels.fused_moe_v3 import ep_scatter_rows
+    print(f'case long row tables T={T} topk={topk} E={E}', flush=True)
+    g = helpers.gen(T + E + 1)
+    ids = torch.randint(-2, E, (T, topk), generator=g).clamp(min=-1)
+    counts = (torch.bincount(ids[ids >= 0], minlength=E) + 127) // 128 * 128
+    rows, longer = int(counts.sum()), int(counts.sum()) + 384
+    i32 = lambda n, v: torch.full((n, ), v, dtype=torch.int32, device=dev)
+    first, m_indices, src, slot = i32(E, -9), i32(longer, -1), i32(longer, 0x7fffffff), torch.full_like(ids, -9, device=dev)
+    ep_scatter_rows(ids.to(dev), counts.to(torch.int32).to(dev), first, m_indices, src, slot)
+    torch.cuda.synchronize()
+    excl, routed, dest = _row_tables_ref(ids, counts)
+    src_ref = torch.zeros(longer, dtype=torch.long)
+    src_ref[dest[dest >= 0]] = (torch.arange(T * topk) // topk)[dest >= 0]
+    assert torch.equal(src.cpu().long(), src_ref)
+    assert torch.equal(slot.cpu().flatten(), dest) and torch.equal(first.cpu().long(), excl + routed)
+    assert torch.equal(m_indices[:rows].cpu().long(), torch.repeat_interleave(torch.arange(E), counts)) and (m_indices[rows:] == -1).all()
+
+
+def test_gathering_gemm_on_a_table_longer_than_the_spans(dev):
+    from dlblas_amd.kernels.fp8_gemm_grouped import fp8_gemm_grouped_contiguous_silu_quant
+    from dlblas_amd.kernels.fused_moe_v3 import ep_scatter_rows
+    print('case gathering GEMM, long row table', flush=True)
+    T, topk, E, K, inter = 50, 2, 3, 512, 128
+    g = helpers.gen(11)
+    x_q, x_s = (t.to(dev) for t in orc.quant_act_1x128(torch.randn(T, K, generator=g).to(torch.bfloat16)))
+    ws = [orc.quant_weight_128x128((torch.randn(2 * inter, K, generator=g) * 0.05).to(torch.bfloat16)) for _ in range(E)]
+    w_q, w_s = (torch.stack([w[i] for w in ws]).to(dev) for i in (0, 1))
+    ids = torch.randint(0, E, (T, topk), generator=g)
+    counts = (torch.bincount(ids.flatten(), minlength=E) + 127) // 128 * 128
+    rows = int(counts.sum())
+    outs = []
+    for length in (rows, rows + 256):
+        first, slot = torch.empty(E, dtype=torch.int32, device=dev), torch.empty_like(ids, device=dev)
+        m_indices = torch.full((length, ), -1, dtype=torch.int32, device=dev)
+        src = torch.full((length, ), 0x7fffffff, dtype=torch.int32, device=dev)
+        ep_scatter_rows(ids.to(dev), counts.to(torch.int32).to(dev), first, m_indices, src, slot)
+        assert int(src.max()) < T  # before the GEMM follows them
+        outs.append(fp8_gemm_grouped_contiguous_silu_quant(x_q, x_s, w_q, w_s, m_indices, a_row_index=src))
+    torch.cuda.synchronize()
+    (q, s), (q2, s2) = outs
+    assert torch.equal(q2.view(torch.uint8)[:rows], q.view(torch.uint8)) and torch.equal(s2[:rows], s)
