@@ -48,7 +48,7 @@ struct ScatterArgs {
   // tables only (ep_rows_kernel): no row of x or xs is moved
   int32_t* src_row;    // [m_len]: source token of every destination row (0 for rows nobody is copied to)
   int32_t* row_start;  // [E] or NULL: first row of every expert's span
-  int32_t* row_end;    // [E] or NULL: one past its last row that holds a slot, never beyond the span
+  int32_t* row_end;    // [E] or NULL: one past the last row of the span that holds a slot
 };
 
 // Expert id of entry `i` (token-major) of block `b`, or -1.
@@ -395,6 +395,17 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
     store_index(p.out_index, p.oi_is64, t * p.oi_s0 + (tid % p.topk_n) * p.oi_s1, d);
     if (d < p.m_len) p.src_row[d] = static_cast<int32_t>(t);
   }
+  // One past the last row that holds a slot of the experts up to e.  Where more slots are routed to an expert than it has
+  // rows, they run on into the spans behind its own, as in ep_scatter, and those rows are not empty.
+  int over = 0;
+  for (int e = tid; e < E; e += kRowsThreads) over |= routed[e] > excl[e + 1] - excl[e];
+  over = __syncthreads_or(over);
+  auto end_of = [&](int e) {
+    int end = excl[e] + routed[e];
+    if (over)
+      for (int i = 0; i < e; ++i) end = max(end, excl[i] + routed[i]);
+    return end;
+  };
   // the rows in slices over the blocks: their expert below excl[E], and token 0 for every row that no slot is given.  That
   // includes the rows of a longer table past the spans: readers of src_row follow every entry, whatever m_indices says
   const int total = static_cast<int>(min(static_cast<int64_t>(excl[E]), p.m_len));
@@ -402,7 +413,7 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
   const int64_t r1 = min(p.m_len, (b + 1) * per);
   for (int64_t r = b * per + tid; r < r1; r += kRowsThreads) {
     if (r >= total) {
-      p.src_row[r] = 0;
+      if (r >= end_of(E - 1)) p.src_row[r] = 0;
       continue;
     }
     int lo = 0, hi = E;  // largest e with excl[e] <= r
@@ -414,13 +425,13 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
         hi = mid;
     }
     p.m_indices[r] = lo;
-    if (r >= excl[lo] + routed[lo]) p.src_row[r] = 0;
+    if (r >= end_of(lo)) p.src_row[r] = 0;
   }
   if (b == 0)
     for (int e = tid; e < E; e += kRowsThreads) {
       if (MODE != kRowsScanned) store_index(p.start_loc, p.start_is64, e, static_cast<int64_t>(excl[e]) + routed[e]);
       if (p.row_start != nullptr) p.row_start[e] = excl[e];
-      if (p.row_end != nullptr) p.row_end[e] = min(excl[e] + routed[e], excl[e + 1]);
+      if (p.row_end != nullptr) p.row_end[e] = min(end_of(e), excl[e + 1]);
     }
 }
 

@@ -73,8 +73,8 @@ def ep_scatter_rows(recv_topk: torch.Tensor, num_recv_tokens_per_expert: torch.T
                     m_indices: torch.Tensor, src_row: torch.Tensor, output_index: torch.Tensor):
     """The tables of ``ep_scatter`` without its copy: ``m_indices``, ``expert_start_loc`` and ``output_index`` as that call
     leaves them, and ``src_row`` [rows] int32 = the token ``ep_scatter`` would have copied to every destination row (0 for
-    rows that stay empty, those past the last span of a longer table among them).  ``fp8_gemm_grouped_contiguous_silu_quant(..., a_row_index=src_row)`` then
-    reads the tokens where they lie."""
+    rows that stay empty, those past the last span of a longer table among them).
+    ``fp8_gemm_grouped_contiguous_silu_quant(..., a_row_index=src_row)`` then reads the tokens where they lie."""
     assert m_indices.shape[0] % 128 == 0, 'every expert span is a whole number of 128-row GEMM blocks'
     if num_recv_tokens_per_expert.dtype != torch.int32 or m_indices.dtype != torch.int32 or src_row.dtype != torch.int32:
         raise TypeError('num_recv_tokens_per_expert, m_indices and src_row must be int32')

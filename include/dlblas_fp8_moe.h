@@ -99,9 +99,10 @@ int dlb_ep_scatter(const void* recv_x, int64_t x_row_stride, const float* recv_x
 /*
  * The tables of dlb_ep_scatter without the copy: m_indices, expert_start_loc and output_index exactly as that call
  * leaves them, plus src_row [m_indices_len] int32 = the token whose row dlb_ep_scatter would have copied to each
- * destination row (0 for every row that no slot is copied to, a longer table's rows past the last span among them).  No row of recv_x is read or written:
- * dlb_fp8_gemm_grouped_contiguous_gather_silu_quant reads the tokens through src_row.  No counterpart in the
- * reference, whose ep_scatter always copies (dlblas/kernels/fused_moe_v3.py:95-158).  Workspace as dlb_ep_scatter.
+ * destination row (0 for every row that no slot is copied to, a longer table's rows past the last span among them).  No
+ * row of recv_x is read or written: dlb_fp8_gemm_grouped_contiguous_gather_silu_quant reads the tokens through src_row.
+ * No counterpart in the reference, whose ep_scatter always copies (dlblas/kernels/fused_moe_v3.py:95-158).  Workspace as
+ * dlb_ep_scatter.
  */
 int dlb_ep_scatter_rows(const void* recv_topk, int topk_dtype, int64_t topk_stride_m, int64_t topk_stride_k,
                         const int32_t* num_recv_tokens_per_expert, void* expert_start_loc, int start_dtype,
@@ -112,8 +113,8 @@ int dlb_ep_scatter_rows(const void* recv_topk, int topk_dtype, int64_t topk_stri
 /*
  * dlb_ep_scatter_rows for callers that have the reserved rows per expert in HOST memory (fused_moe_v3 is given a list):
  * they travel in the launch itself, so nothing is uploaded; at most 256 experts.  Also leaves the row range of every
- * expert, [row_start[e], row_end[e]) int32 = the rows that hold a slot, clipped to the expert's reserved span (either may be
- * NULL): the form dlb_fp8_gemm_grouped_ragged takes.  DLB_ERR_BAD_SHAPE (nothing enqueued): more experts, or so many tokens
+ * expert, [row_start[e], row_end[e]) int32 = the rows of the expert's reserved span up to the last one that holds a slot (either
+ * may be NULL): the form dlb_fp8_gemm_grouped_ragged takes.  DLB_ERR_BAD_SHAPE (nothing enqueued): more experts, or so many tokens
  * that the tables need the scan launch; the caller then uploads the counts and uses dlb_ep_scatter_rows.
  */
 int dlb_ep_scatter_rows_host(const void* recv_topk, int topk_dtype, int64_t topk_stride_m, int64_t topk_stride_k,

@@ -233,3 +233,38 @@ def test_gathering_gemm_on_a_table_longer_than_the_spans(dev):
     torch.cuda.synchronize()
     (q, s), (q2, s2) = outs
     assert torch.equal(q2.view(torch.uint8)[:rows], q.view(torch.uint8)) and torch.equal(s2[:rows], s)
+
+
+@pytest.mark.parametrize('T,topk,E', [(250, 1, 3), (2300, 8, 40), (5100, 8, 300)])
+def test_row_tables_where_more_slots_are_routed_than_reserved(dev, T, topk, E):
+    """The slots an expert has no rows for go on into the span behind its own, as ep_scatter lays them: an expert without
+    slots of its own follows every one that is too short, so each row has one owner."""
+    from dlblas_amd import _lib
+    from dlblas_amd.kernels.fused_moe_v3 import ep_scatter_rows
+    print(f'case row tables, short reserve T={T} topk={topk} E={E}', flush=True)
+    g = helpers.gen(T + E + 2)
+    ids = torch.randint(0, (E + 1) // 2, (T, topk), generator=g) * 2  # even experts only
+    ids[ids >= E - 1] = 0  # ... and the last one has none: the rows of all slots are in the table
+    routed = torch.bincount(ids.flatten(), minlength=E)
+    counts = torch.where(torch.arange(E) % 2 == 0, routed - routed.clamp(max=5), torch.tensor(8))
+    counts[-1] += -int(counts.sum()) % 128
+    rows = int(counts.sum())
+    excl, _, dest = _row_tables_ref(ids, counts)
+    src_ref = torch.zeros(rows, dtype=torch.long)
+    src_ref[dest] = torch.arange(T * topk) // topk
+    i32 = lambda n: torch.full((n, ), -9, dtype=torch.int32, device=dev)
+    first, m_indices, src, slot = i32(E), i32(rows), i32(rows), torch.full_like(ids, -9, device=dev)
+    ep_scatter_rows(ids.to(dev), counts.to(torch.int32).to(dev), first, m_indices, src, slot)
+    torch.cuda.synchronize()
+    assert torch.equal(slot.cpu().flatten(), dest) and torch.equal(src.cpu().long(), src_ref)
+    start, end = i32(E), i32(E)
+    src.fill_(-9)
+    if _lib.ep_scatter_rows_host(ids.to(dev), counts.tolist(), start, end, first, m_indices, src, slot):
+        held = torch.zeros(rows, dtype=torch.bool)
+        held[dest] = True
+        got = torch.zeros(rows, dtype=torch.bool)
+        for a, b in zip(start.tolist(), end.tolist()):
+            got[a:b] = True
+        assert torch.equal(got, held) and torch.equal(src.cpu().long(), src_ref)
+    else:
+        assert E > 256
