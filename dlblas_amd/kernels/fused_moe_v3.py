@@ -139,6 +139,9 @@ def fused_moe_v3(
     def buf(shape, dtype):
         return torch.empty(shape, device=dev, dtype=dtype)
 
+    def upload_counts():
+        return torch.tensor(num_recv_tokens_per_expert, dtype=torch.int32, pin_memory=True).to(dev, non_blocking=True)
+
     row_expert = buf((rows_total, ), torch.int32)
     slot_row = torch.empty_like(topk_idx)
     n_experts = len(num_recv_tokens_per_expert)
@@ -148,28 +151,41 @@ def fused_moe_v3(
     # the row tables say which expert and which token each sorted row stands for, the kernel follows them, and neither
     # the expert-sorted copy of the activations nor the bf16 [rows, 2 I] intermediate reaches memory.  Same bits as the
     # steps of the reference (:288-334).
-    direct = tokens_q.is_contiguous() and hidden % 128 == 0 and inter2 % 256 == 0 and n_tokens * hidden < (1 << 31)
-    if direct and n_experts <= 256:
+    if tokens_q.is_contiguous() and hidden % 128 == 0 and inter2 % 256 == 0 and n_tokens * hidden < (1 << 32):
         # A short batch - a block or so of rows per expert, most of them padding - is a matter of reading the experts'
         # weights once: the weight-streaming kernels, on the rows that hold a token (500 tokens, 32 experts of 7168 x 2048:
-        # 333 -> 245 us).  A long one pairs the blocks of an expert into taller tiles.  In between, where the library's
-        # planner prefers uniform 128-row tiles, which have no fused epilogue, the three steps below are the faster way.
-        used = sum(1 for c in num_recv_tokens_per_expert if c > 0)
-        rows_each = max(1, min(rows_total // used - 64, -(-n_tokens * topk_idx.size(1) // used)))  # half a block of padding on average
-        streams = (_lib.plan_grouped(2, rows_total, inter2, hidden, n_experts, rows_each)[1]
-                   and _lib.plan_grouped(2, rows_total, hidden, inter2 // 2, n_experts, rows_each)[1])
-        if streams or _lib.plan_grouped(1, rows_total, inter2, hidden, n_experts)[1]:
+        # 333 -> 245 us; their token offsets are 31 bits).  A long one pairs the blocks of an expert into taller tiles.  In
+        # between, where the library's planner prefers uniform 128-row tiles, which have no fused epilogue, the three steps
+        # below are the faster way.
+        streams = False
+        if n_experts <= 256 and n_tokens * hidden < (1 << 31):
+            used = sum(1 for c in num_recv_tokens_per_expert if c > 0)
+            rows_each = max(1, min(rows_total // used - 64, -(-n_tokens * topk_idx.size(1) // used)))  # half a block of padding on average
+            streams = (_lib.plan_grouped(2, rows_total, inter2, hidden, n_experts, rows_each)[1]
+                       and _lib.plan_grouped(2, rows_total, hidden, inter2 // 2, n_experts, rows_each)[1])
+        lists = _lib.plan_grouped(1, rows_total, inter2, hidden, n_experts)[1]
+        if streams or lists:
             row_token = buf((rows_total, ), torch.int32)
             ranges = buf((3, n_experts), torch.int32)
-            if _lib.ep_scatter_rows_host(topk_idx, num_recv_tokens_per_expert, ranges[0], ranges[1], ranges[2], row_expert, row_token,
-                                         slot_row):
+            have_tables = _lib.ep_scatter_rows_host(topk_idx, num_recv_tokens_per_expert, ranges[0], ranges[1], ranges[2], row_expert,
+                                                    row_token, slot_row)
+            if not have_tables:
+                streams = False  # the row ranges come with the tables of the host form only
+                if lists:
+                    # more experts, or more tokens times experts, than travel in the launch: the same tables from counts
+                    # in device memory
+                    ep_scatter_rows(topk_idx, upload_counts(), ranges[2], row_expert, row_token, slot_row)
+                    have_tables = True
+            if have_tables:
                 down = buf((rows_total, hidden), torch.bfloat16)
-                act_q = buf((rows_total, inter2 // 2), torch.float8_e4m3fn)
-                act_scale = buf((rows_total, inter2 // 256), torch.float32)
-                if not (streams
-                        and _lib.gemm_ragged_silu_quant(tokens_q, w13_weight_fp8[0], tokens_scale, w13_weight_fp8[1], act_q, act_scale,
-                                                        ranges[0], ranges[1], row_token, rows_each, 1e-10)
-                        and _lib.gemm_ragged(act_q, w2_weight_fp8[0], act_scale, w2_weight_fp8[1], down, ranges[0], ranges[1], rows_each)):
+                if streams:
+                    act_q = buf((rows_total, inter2 // 2), torch.float8_e4m3fn)
+                    act_scale = buf((rows_total, inter2 // 256), torch.float32)
+                    streams = (_lib.gemm_ragged_silu_quant(tokens_q, w13_weight_fp8[0], tokens_scale, w13_weight_fp8[1], act_q,
+                                                           act_scale, ranges[0], ranges[1], row_token, rows_each, 1e-10)
+                               and _lib.gemm_ragged(act_q, w2_weight_fp8[0], act_scale, w2_weight_fp8[1], down, ranges[0], ranges[1],
+                                                    rows_each))
+                if not streams:
                     fused = fp8_gemm_grouped_contiguous_silu_quant(tokens_q, tokens_scale, w13_weight_fp8[0], w13_weight_fp8[1],
                                                                    row_expert, column_major_scales=True,  # what the down GEMM reads in place
                                                                    a_row_index=row_token)
@@ -178,7 +194,7 @@ def fused_moe_v3(
         # Expert-sorted activations.  The spans are padded to 128 rows per expert; the padding rows keep whatever the
         # allocator hands out, as in the reference driver (:269-278).  The GEMMs and the quantiser treat every row on its
         # own, so what those rows turn into (NaN included) stays in rows that ep_gather never reads.
-        per_expert = torch.tensor(num_recv_tokens_per_expert, dtype=torch.int32, pin_memory=True).to(dev, non_blocking=True)
+        per_expert = upload_counts()
         first_row = torch.empty_like(per_expert)
         sorted_q = buf((rows_total, hidden), torch.uint8).view(tokens_q.dtype)
         sorted_scale = buf((rows_total, hidden // 128), torch.float32)

@@ -162,3 +162,52 @@ def test_fused_moe_v3_with_the_tile_lists_kept_equals_the_steps(dev, tokens, E):
             assert out is not None and torch.equal(out, ref)
     finally:
         _lib.tune('tile_list', 0), _lib.tune('stream', 0)
+
+
+@pytest.mark.parametrize('tokens,topk,E,H', [
+    (4097, 8, 256, 256),     # one token more than 256 experts' histograms may have for counts in the launch
+    (300, 4, 300, 256),      # more experts than counts travel in the launch
+    (131073, 1, 2, 16384),   # token offsets of 32 bits: no row ranges (every fourth token is routed here)
+])
+def test_fused_moe_v3_reads_the_tokens_in_place_beyond_the_native_call(dev, monkeypatch, tokens, topk, E, H):
+    """Batches that the native call leaves to the Python path still go through row tables and the gathering GEMM, with no
+    expert-sorted copy of the activations, and give the bits of the three steps."""
+    import importlib
+
+    from dlblas_amd import _fast, _lib
+    moe = importlib.import_module('dlblas_amd.kernels.fused_moe_v3')
+    print(f'case fused_moe_v3 in place tokens={tokens} topk={topk} E={E} H={H}', flush=True)
+    inter = 128
+    g = torch.Generator(device=dev).manual_seed(12)
+
+    def codes(*shape):  # finite e4m3 codes of either sign
+        return (torch.randint(0, 0x60, shape, device=dev, generator=g, dtype=torch.uint8) |
+                (torch.randint(0, 2, shape, device=dev, generator=g, dtype=torch.uint8) << 7)).view(torch.float8_e4m3fn)
+
+    def scales(*shape):
+        return torch.rand(*shape, device=dev, generator=g) * 2e-3 + 1e-3
+
+    x = codes(tokens, H), scales(tokens, H // 128)
+    w13, w2 = (codes(E, 2 * inter, H), scales(E, 2, H // 128)), (codes(E, H, inter), scales(E, H // 128, 1))
+    ids = torch.randint(0, E, (tokens, topk), device=dev, generator=g)
+    if tokens > 100000:
+        ids[torch.arange(tokens, device=dev) % 4 > 0] = -1
+    wts = torch.rand(tokens, topk, device=dev, generator=g)
+    counts = ((torch.bincount(ids[ids >= 0], minlength=E) + 127) // 128 * 128).tolist()
+    ran = []
+    copy, tables, gemm = moe.ep_scatter, moe.ep_scatter_rows, moe.fp8_gemm_grouped_contiguous_silu_quant
+    monkeypatch.setattr(moe, 'ep_scatter', lambda *a: (ran.append('copy'), copy(*a)))
+    monkeypatch.setattr(moe, 'ep_scatter_rows', lambda *a: (ran.append('tables'), tables(*a)))
+    monkeypatch.setattr(moe, 'fp8_gemm_grouped_contiguous_silu_quant',
+                        lambda *a, **kw: (ran.append('gathering GEMM' if 'a_row_index' in kw else 'GEMM'), gemm(*a, **kw))[1])
+    _lib.tune('stream', 1), _lib.tune('tile_list', 1)
+    assert _fast.fused_moe_v3(*x, ids, wts, *w13, *w2, counts) is None
+    out = moe.fused_moe_v3(x, ids, wts, w13, w2, counts)
+    assert 'gathering GEMM' in ran and 'copy' not in ran
+    assert ('tables' in ran) == (H == 256)  # the last one's counts do travel in the launch
+    del ran[:]
+    _lib.tune('tile_list', 2)
+    ref = moe.fused_moe_v3(x, ids, wts, w13, w2, counts)
+    torch.cuda.synchronize()
+    assert ran == ['copy']  # ... and three steps
+    assert torch.equal(out, ref) and bool(out.isfinite().all()) and float(out.abs().max()) > 0
