@@ -819,7 +819,9 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
   const Plan& pl = r.pl;
   r.stream = kStreamNone;
   r.wavek = kWaveKNone;
-  if (overlay && mode == kDense && dma_ok && as_sk < (1ll << 20) && K > 0 && K % 16 == 0) r.wavek = pick_wavek(rows, N, K, cus, usable_ws ? ws_bytes : 0);
+  // (its scale table is fetched through 32-bit byte offsets from the tile's first row; tiles have up to 64 rows)
+  const bool table_near = dma_ok && as_sk < (1ll << 20) && 63 * as_sm + (kblocks - 1) * as_sk < (1ll << 30);
+  if (overlay && mode == kDense && table_near && K > 0 && K % 16 == 0) r.wavek = pick_wavek(rows, N, K, cus, usable_ws ? ws_bytes : 0);
   if (r.wavek != kWaveKNone) {
     r.pl.splitk = 1;
     r.kb_per_split = static_cast<int>(kblocks);

@@ -83,3 +83,24 @@ def test_library_choice_full_size(dev, M, N, K):
     assert torch.equal(out, again)
     rows = [0, 31, 32, M // 2, M - 1]
     helpers.tolerance_check(out[rows], orc.dequant_ref(a[rows], a_s[rows], b, b_s), f'wave_k {M}x{N}x{K}')
+
+
+def test_scales_further_apart_than_32_bit_offsets(dev):
+    """1023 K blocks whose scales lie up to 4.5 GB behind a tile's first one: beyond what the scale table's fetch can address,
+    so the launch goes to a kernel with 64-bit addressing."""
+    from dlblas_amd import _lib
+    lib = _lib.load()
+    M, N, K, sm, sk = 33, 32, 1023 * 128, (1 << 21) - 1, (1 << 20) - 1
+    print(f'case wave_k far scales {M}x{N}x{K}', flush=True)
+    a, b, a_s, b_s = _operands(M, N, K, 8)
+    ref = orc.dequant_ref(a, a_s, b, b_s)
+    far = torch.zeros((M - 1) * sm + (K // 128 - 1) * sk + 1, device=dev).as_strided((M, K // 128), (sm, sk))
+    far.copy_(a_s)
+    a, b, b_s = a.to(dev), b.to(dev), b_s.to(dev)
+    ws = _lib.workspace(dev, torch.cuda.current_stream().cuda_stream)
+    vp = ctypes.c_void_p
+    out = torch.empty(M, N, device=dev)
+    _lib.check(lib.dlb_fp8_gemm(vp(a.data_ptr()), vp(b.data_ptr()), vp(far.data_ptr()), vp(b_s.data_ptr()), vp(out.data_ptr()), M, N, K, sm, sk,
+                                _lib.OUT_F32, vp(ws.data_ptr()), ws.numel(), vp(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    helpers.tolerance_check(out, ref, f'wave_k far scales {M}x{N}x{K}')
