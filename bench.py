@@ -465,7 +465,8 @@ def grouped_workloads(dev):
     """One GPU's expert share of the two MoE layouts; FLOPs count real tokens only, bytes count every operand once."""
     import torch
 
-    from dlblas_amd.kernels.fp8_gemm_grouped import fp8_gemm_grouped_contiguous, fp8_gemm_grouped_masked
+    from dlblas_amd.kernels.fp8_gemm_grouped import (fp8_gemm_grouped_contiguous, fp8_gemm_grouped_masked,
+                                                     fp8_gemm_grouped_masked_silu_quant)
     rows = []
     # expert-contiguous (prefill): per-expert counts from a seeded multinomial, padded to multiples of 128
     c = GROUPED_CONTIGUOUS
@@ -739,22 +740,33 @@ def planner_sweep(dev, which):
     'dense': kernel variants (no K split forced) over 13 weight shapes x 15 row counts; 'mid': the three small ring
     kernels x 1 ... 16 K slices where the planner picks one of them; 'decode': columns per workgroup x waves x blocks in
     flight of the streaming kernels at 1, 16 and 32 rows; 'grouped': ring variants for both grouped layouts, 8 and 32
-    experts.  A row's 'regret' is default / best - 1."""
+    experts; 'wave_k': the launch without the kernel whose waves split K and with each of its tile shapes, at the row counts
+    and the ragged K it is meant for and around them; 'stream': the same for the weight-streaming kernel of the masked layout,
+    plain and with the quantising epilogue.  A row's 'regret' is default / best - 1."""
     import torch
 
     from dlblas_amd import _lib
-    from dlblas_amd.kernels.fp8_gemm_grouped import fp8_gemm_grouped_contiguous, fp8_gemm_grouped_masked
+    from dlblas_amd.kernels.fp8_gemm_grouped import (fp8_gemm_grouped_contiguous, fp8_gemm_grouped_masked,
+                                                     fp8_gemm_grouped_masked_silu_quant)
     rows = []
 
-    def report(name, plan, t_default, best_t, best_what):
+    def report(name, plan, t_default, best_t, best_what, every=None):
         row = {'problem': name, 'plan': plan, 'default_us': t_default, 'best_us': best_t, 'best': best_what,
                'regret': t_default / best_t - 1.0}
         rows.append(row)
-        print(f"{name}: default {plan} {t_default:.1f} us; best {best_what} {best_t:.1f} us; regret {100 * row['regret']:.0f} %", flush=True)
+        print(f"{name}: default {plan} {t_default:.1f} us; best {best_what} {best_t:.1f} us; regret {100 * row['regret']:.0f} %"
+              + (' (' + ', '.join(f'{n} {t:.1f}' for n, t in every.items() if t is not None) + ')' if every else ''), flush=True)
+
+    def wave_k_or(plan, M, N, K):
+        tile = _lib.plan_wave_k(M, N, K)
+        return 'wave_k {}x{} tiles, {} waves'.format(*tile) if tile else plan
 
     def dense_problem(M, N, K):
         copies = max(2, min(24, int(400e6 // (N * K))))
-        a_q, a_s, ws = make_inputs(M, N, K, dev, weight_copies=copies)
+        whole = -(-K // 128) * 128
+        a_q, a_s, ws = make_inputs(M, N, whole, dev, weight_copies=copies)
+        if K < whole:  # a ragged last block keeps the scale of the whole one
+            a_q, ws = a_q[:, :K].contiguous(), [(q[:, :K].contiguous(), s) for q, s in ws]
         out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
         launch = DenseLauncher(a_q, a_s, ws, out)
         reps = int(max(10, min(200, 3e-2 / max(2.0 * M * N * K / 2e15, 5e-6))))
@@ -788,7 +800,7 @@ def planner_sweep(dev, which):
                                 best = (t, v)
                         _lib.force_variant(None)
                         t0 = min(t0, timed(launch, reps))
-                    report(f'{M}x{N}x{K}', plan[:2], t0, min(best[0], t0), best[1])
+                    report(f'{M}x{N}x{K}', wave_k_or(plan[:2], M, N, K), t0, min(best[0], t0), best[1])
         elif which == 'mid':
             for (N, K) in PLANNER_SWEEP_WEIGHTS + [(4096, 4096), (1024, 16384), (7168, 4096)]:
                 for M in (48, 64, 96, 128, 192, 256, 384, 512, 1024):
@@ -810,7 +822,7 @@ def planner_sweep(dev, which):
                         _lib.tune('splitk', 0)
                     _lib.force_variant(None)
                     t0 = min(t0, timed(launch, reps))
-                    report(f'{M}x{N}x{K}', plan[:2], t0, min(best[0], t0), best[1])
+                    report(f'{M}x{N}x{K}', wave_k_or(plan[:2], M, N, K), t0, min(best[0], t0), best[1])
         elif which == 'decode':
             for (N, K) in PLANNER_SWEEP_WEIGHTS + [(4096, 4096), (8192, 1024), (16384, 2048)]:
                 for M in (1, 16, 32):
@@ -828,7 +840,7 @@ def planner_sweep(dev, which):
                     for knob in ('skinny_bn', 'skinny_waves', 'skinny_unroll'):
                         _lib.tune(knob, 0)
                     t0 = min(t0, timed(launch, reps))
-                    report(f'{M}x{N}x{K}', plan, t0, min(best[0], t0), best[1])
+                    report(f'{M}x{N}x{K}', wave_k_or(plan, M, N, K), t0, min(best[0], t0), best[1])
         elif which == 'grouped':
             gd = torch.Generator(device=dev).manual_seed(21)
             ring = ('pipe128x256w8', 'pipe256x256', 'pipe128x128')
@@ -881,6 +893,54 @@ def planner_sweep(dev, which):
                                _lib.plan_grouped(2, M_max, N, K, G, hint), t0, min(best[0], t0), best[1])
                         del a_q, a_s, out
                 del w_q, w_s
+        elif which == 'wave_k':
+            shapes = ('32x32/8', '32x32/4', '64x32/8', '32x64/4', '64x32/4', '64x64/4', '64x64/2')  # knob values 2 .. 8
+            problems = [(M, N, K) for (N, K) in PLANNER_SWEEP_WEIGHTS + [(4096, 4096), (1024, 16384), (12544, 512)]
+                        for M in (17, 32, 48, 64, 100, 128, 200, 300, 500, 1000)]
+            problems += [(M, N, K) for (N, K) in ((24576, 512), (24576, 1536), (28480, 1152), (28672, 4096), (32768, 2048), (36864, 3072),
+                                                  (36864, 7168), (65536, 1024)) for M in (1, 8, 16)]
+            problems += [(M, N, K) for K in (528, 1040, 2064, 5136) for N in (1000, 4096, 24576)
+                         for M in (1, 16, 100, 300, 1000, 2048, 4096)]
+            for M, N, K in problems:
+                launch, reps = dense_problem(M, N, K)
+                times = {}
+                for knob, name in enumerate(('default', 'other kernels') + shapes):
+                    _lib.tune('wave_k', knob)
+                    times[name] = timed(launch, reps)
+                _lib.tune('wave_k', 0)
+                times['default'] = min(times['default'], timed(launch, reps))
+                best = min((n for n in times if times[n] is not None), key=lambda n: times[n])
+                report(f'{M}x{N}x{K}', wave_k_or(_lib.plan(0, M, N, K)[:2], M, N, K), times['default'], times[best], best,
+                       {n: t for n, t in times.items() if n != 'default'})
+        elif which == 'stream':
+            shapes = ('32x256', '64x256', '64x128', '128x256', '64x64', None, '64x256 ahead', '64x128 ahead', '128x256 ahead', '64x64 ahead')
+            for (G, N, K) in ((32, 4096, 7168), (32, 7168, 2048), (8, 4096, 7168), (8, 7168, 2048), (16, 1024, 3072), (32, 2048, 1024)):
+                w_q, w_s = expert_weights(G, N, K, dev, 22)
+                gd = torch.Generator(device=dev).manual_seed(21)
+                for M_max in (16, 32, 64, 128, 192, 256, 384, 512):
+                    mm = torch.randint(0, M_max + 1, (G, ), generator=torch.Generator().manual_seed(20), dtype=torch.int32).to(dev)
+                    hint = int(mm.float().mean())
+                    a_q, a_s = quantise_act(torch.randn(G * M_max, K, device=dev, generator=gd).to(torch.bfloat16))
+                    a_q, a_s = a_q.reshape(G, M_max, K), a_s.reshape(G, M_max, K // 128)
+                    out = torch.empty(G, M_max, N, dtype=torch.bfloat16, device=dev)
+                    q, sc = torch.empty(G, M_max, N // 2, dtype=torch.float8_e4m3fn, device=dev), torch.empty(G, M_max, N // 256, device=dev)
+                    plain = lambda: fp8_gemm_grouped_masked(a_q, a_s, w_q, w_s, out, mm, hint)  # noqa: E731
+                    act = lambda: fp8_gemm_grouped_masked_silu_quant(a_q, a_s, w_q, w_s, q, sc, mm, hint)  # noqa: E731
+                    for what, call in (('plain', plain), ('silu_quant', act)):
+                        times = {}
+                        for knob, name in enumerate(('default', 'ring kernels') + shapes):
+                            if name is None or what == 'silu_quant' and name not in ('default', 'ring kernels', '32x256', '64x256', '128x256'):
+                                continue
+                            _lib.tune('stream', knob)
+                            times[name] = timed(call, 30)
+                        _lib.tune('stream', 0)
+                        times['default'] = min(times['default'], timed(call, 30))
+                        best = min((n for n in times if times[n] is not None), key=lambda n: times[n])
+                        report(f'masked {what}, {G} experts x {M_max} slots, {int(mm.sum())} valid rows, {N}x{K}',
+                               _lib.plan_grouped(2, M_max, N, K, G, hint), times['default'], times[best], best,
+                               {n: t for n, t in times.items() if n != 'default'})
+                    del a_q, a_s, out, q, sc
+                del w_q, w_s
         else:
             raise ValueError(which)
     finally:
@@ -918,7 +978,7 @@ def main():
     ap.add_argument('--grouped-only', action='store_true',
                     help='run only the two grouped MoE workloads and print their rows (the command the rocprofv3 summaries of '
                     'the grouped kernels are made with)')
-    ap.add_argument('--planner-sweep', choices=['dense', 'mid', 'decode', 'grouped'], default=None,
+    ap.add_argument('--planner-sweep', choices=['dense', 'mid', 'decode', 'grouped', 'wave_k', 'stream'], default=None,
                     help="time the planner's launch against every alternative forced in turn over a grid of problems and "
                     'print where it is not the fastest (a minute or two)')
     args = ap.parse_args()
