@@ -713,20 +713,28 @@ int wavek_lds(const WaveKDims& d, int pitch) {
 //     the larger of its bytes at 86 GB/s (the DMA path of a CU) and the trip of one block (0.21 us + 3.8 ns per operand row)
 //     shared by the waves that are resident at once;
 //   - every tile's operands from the L2s at 17 TB/s;  - the matrices from HBM at 6 TB/s.
-// (rms error 13 % over 110 problems of 1 .. 1300 rows, 512 .. 36864 weight rows, K = 512 .. 18432; its choice of shape is
-// within 3 % of the best, geometric mean.)  Against the kernels it would replace: up to 16 rows the decode kernels' 16-row
-// fragments waste less (16 x 7168 x 2048 5.2 against 5.4 us), unless K is ragged or N so large that they take many rounds
-// (1 x 28480 x 1152 9.0 -> 7.6 us); from 17 to 64 rows this kernel is ahead wherever measured (23 x 12632 x 16768 45 -> 32 us);
-// above, the smaller estimate wins (100 x 2112 x 7168 13.4 -> 10.2 us, 500 x 4096 x 7168 33 -> 26 us, 64 x 2112 x 7168 12.7 ->
-// 7.9 us; 473 x 7088 x 6528 stays with 128 x 128 tiles, 40 against 45 us).  The register-staged kernels, the only others for
-// a ragged K, lose everywhere measured (300 x 1000 x 1040 11.4 -> 4.7 us, 225 x 17536 x 5280 126 -> 62 us).
+// The estimate chooses the shape (2 - 3 % behind the best one, geometric mean over 1500 problems; its rms error is 15 - 29 %,
+// mostly too low where the weights come from HBM).  Whether the kernel runs at all depends on where the operands come from:
+// from the caches (three weight matrices of up to 80 MB in turn stay in the 256 MB Infinity cache) it is ahead of the others,
+// from HBM it may be behind.  Its time over theirs, cache / HBM, geometric means over random problems of 512 .. 36864 weight
+// rows and K = 512 .. 18432 (bench.py --planner-sweep wave_k has the fixed ones):
+//   - up to 16 rows the decode kernels' 16-row fragments waste less (16 x 7168 x 2048 5.2 against 5.4 us), but very many columns
+//     take them several rounds, whose waves idle while K is short.  From 24576 columns on 0.95 / 1.04 at up to 7 K blocks, 0.87 /
+//     1.05 at 8 .. 11, 0.97 / 1.15 at 12 .. 16, 1.08 / 1.19 and 1.17 / 1.15 above (16 x 36864 x 7168 50.3 against 46.9 us): up to 11;
+//   - 17 .. 64 rows: always.  17 .. 32 rows 0.84 / 1.08 at up to 80 MB (K < 2048 0.90 / 1.00, < 4096 0.86 / 1.07, longer 0.77 / 1.15:
+//     32 x 2112 x 7168 11.5 against 9.6 us from HBM), 1.00 / 1.03 above; 33 .. 64 rows 0.75 / 0.91 and 1.04 / 1.00;
+//   - more rows: where the estimates say so, at up to 80 MB (0.69 / 0.84 there; 100 x 2112 x 7168 14.5 -> 12.8 us, 300 x 4096 x 4096
+//     20 -> 18 us); larger matrices come from HBM, 1.11 where the estimates would choose it (128 x 7168 x 18432 49.8 against 40.3 us);
+//   - a ragged K, for which only the register-staged kernels remain: always.  Up to 16 rows 0.80 / 1.01 at up to 80 MB and 0.68 /
+//     0.71 above, 17 .. 64 rows 0.70 from HBM, more rows 0.67 (300 x 1000 x 1040 11.2 -> 4.6 us, 4096 x 24576 x 1040 372 -> 237 us).
 int pick_wavek(int64_t M, int64_t N, int64_t K, int cus, size_t ws_bytes) {
   const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
   const int knob = g_knob[kKnobWaveK];
   if (knob == 1 || g_forced_variant >= 0 || g_knob[kKnobSplitK] > 0) return kWaveKNone;
   if (kblocks >= 1024) return kWaveKNone;  // no table of that many scales fits
   const bool ragged = K % kScaleBlock != 0;
-  if (knob == 0 && M <= 16 && !ragged && N < 24576) return kWaveKNone;
+  if (knob == 0 && !ragged && M <= 16 && (N < 24576 || kblocks > 11)) return kWaveKNone;
+  if (knob == 0 && !ragged && M > 64 && static_cast<double>(N) * static_cast<double>(K) > 80e6) return kWaveKNone;
   int best = kWaveKNone;
   double best_us = 0.0;
   for (int i = 0; i < kWaveKCount; ++i) {

@@ -195,3 +195,14 @@ def test_decode_wave_count_is_clamped_to_the_lds():
         assert _lib.plan(DENSE, 128, 7168, 2048)[0] == 'skinny128'
     finally:
         _lib.tune('skinny_waves', 0)
+
+
+def test_where_the_wave_split_kernel_takes_over():
+    """Few rows of whole K blocks stay with the decode kernels unless the columns are very many and K is short; many rows with
+    the ring kernels where the weights are too large for the caches; a ragged K always goes to the wave-split kernel."""
+    for M, N, K in ((1, 2112, 7168), (16, 7168, 2048), (1, 24576, 1536), (16, 36864, 7168), (8, 28672, 4096), (100, 18432, 7168),
+                    (128, 7168, 18432), (300, 7168, 16384), (4096, 7168, 18432), (1000, 24576, 1536)):
+        assert _lib.plan_wave_k(M, N, K) is None, (M, N, K)
+    for M, N, K in ((1, 28480, 1152), (16, 36864, 512), (17, 2112, 7168), (64, 7168, 18432), (100, 2112, 7168), (500, 4096, 7168),
+                    (1, 4096, 1040), (300, 1000, 1040), (4096, 24576, 1040), (300, 24576, 5136)):
+        assert _lib.plan_wave_k(M, N, K) is not None, (M, N, K)
