@@ -761,6 +761,10 @@ def planner_sweep(dev, which):
         tile = _lib.plan_wave_k(M, N, K)
         return 'wave_k {}x{} tiles, {} waves'.format(*tile) if tile else plan
 
+    def stream_or(variant, M_max, N, K, G, hint, quantising=False):
+        tile = _lib.plan_stream(M_max, N, K, G, hint, quantising)
+        return 'stream {}x{}{}'.format(tile[0], tile[1], ' ahead' if tile[2] else '') if tile else variant
+
     def dense_problem(M, N, K):
         copies = max(2, min(24, int(400e6 // (N * K))))
         whole = -(-K // 128) * 128
@@ -890,7 +894,7 @@ def planner_sweep(dev, which):
                         _lib.force_variant(None)
                         t0 = min(t0, timed(call, 30))
                         report(f'masked, {G} experts x {M_max} slots, {int(masked_m.sum())} valid rows, {N}x{K}',
-                               _lib.plan_grouped(2, M_max, N, K, G, hint), t0, min(best[0], t0), best[1])
+                               stream_or(_lib.plan_grouped(2, M_max, N, K, G, hint)[0], M_max, N, K, G, hint), t0, min(best[0], t0), best[1])
                         del a_q, a_s, out
                 del w_q, w_s
         elif which == 'wave_k':
@@ -937,7 +941,8 @@ def planner_sweep(dev, which):
                         times['default'] = min(times['default'], timed(call, 30))
                         best = min((n for n in times if times[n] is not None), key=lambda n: times[n])
                         report(f'masked {what}, {G} experts x {M_max} slots, {int(mm.sum())} valid rows, {N}x{K}',
-                               _lib.plan_grouped(2, M_max, N, K, G, hint), times['default'], times[best], best,
+                               stream_or(_lib.plan_grouped(2, M_max, N, K, G, hint)[0], M_max, N, K, G, hint, what == 'silu_quant'),
+                               times['default'], times[best], best,
                                {n: t for n, t in times.items() if n != 'default'})
                     del a_q, a_s, out, q, sc
                 del w_q, w_s

@@ -12,7 +12,7 @@ import torch
 
 from ._build import LIB_PATH
 
-ABI_VERSION = 8
+ABI_VERSION = 9
 OUT_BF16, OUT_F32 = 0, 1
 WS_COUNTER_BYTES = 65536
 WORKSPACE_BYTES = WS_COUNTER_BYTES + (32 << 20)
@@ -59,6 +59,7 @@ SYMBOLS = {
     'dlb_fp8_gemm_plan_wave_k': (ctypes.c_int, [_c_i64] * 3 + [_c_sz, ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 3),
     'dlb_fp8_gemm_plan_grouped': (ctypes.c_int, [ctypes.c_int, _c_i64, _c_i64, _c_i64, ctypes.c_int32, ctypes.c_int32, _c_sz, ctypes.c_int,
                                                 ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]),
+    'dlb_fp8_gemm_plan_stream': (ctypes.c_int, [_c_i64] * 3 + [_c_i32] * 2 + [ctypes.c_int] * 2 + [ctypes.POINTER(ctypes.c_int)] * 3),
     'dlb_silu_mul': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp] + [_c_i64] * 4 + [_c_vp]),
     'dlb_silu_mul_quant': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp, _c_vp] + [_c_i64] * 5 + [ctypes.c_float, _c_vp]),
     'dlb_silu_mul_quant_masked': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp, _c_vp, _c_vp] + [_c_i64] * 6 + [_c_vp]),
@@ -184,7 +185,8 @@ def variant_names():
 
 
 def plan(mode: int, rows: int, N: int, K: int, workspace_bytes: int = None, compute_units: int = 256):
-    """(variant name, K slices, decode columns per workgroup) the library would use; touches no GPU."""
+    """(variant name, K slices, decode columns per workgroup) the library would use where plan_wave_k() / plan_stream() name no
+    other kernel; touches no GPU."""
     return plan_full(mode, rows, N, K, workspace_bytes, compute_units)[:3]
 
 
@@ -209,14 +211,22 @@ def plan_wave_k(M: int, N: int, K: int, workspace_bytes: int = None, compute_uni
 
 def plan_grouped(mode: int, rows: int, N: int, K: int, G: int, expected_m: int = -1, workspace_bytes: int = None,
                  compute_units: int = 256):
-    """(variant name, flag) of a grouped launch (mode 1 contiguous, 2 masked) with G experts and the masked layout's hint;
-    the flag says whether a contiguous launch uses the tile lists / whether a masked one takes the weight-streaming kernel
-    in place of the named ring kernel.  Touches no GPU."""
+    """(variant name, tile lists used) of a grouped launch (mode 1 contiguous, 2 masked) with G experts and the masked
+    layout's hint; plan_stream() says whether a masked launch takes another kernel than the named one.  Touches no GPU."""
     lib = load()
     v, t = ctypes.c_int(), ctypes.c_int()
     ws = WORKSPACE_BYTES if workspace_bytes is None else workspace_bytes
     check(lib.dlb_fp8_gemm_plan_grouped(mode, rows, N, K, G, expected_m, ws, compute_units, ctypes.byref(v), ctypes.byref(t)))
     return variant_names()[v.value], bool(t.value)
+
+
+def plan_stream(M_max: int, N: int, K: int, G: int, expected_m: int = -1, quantising: bool = False, compute_units: int = 256):
+    """(tile rows, weight rows per tile, fragments read ahead) when the weight-streaming kernel takes a masked launch over from
+    the variant that plan_grouped() names, None otherwise; quantising: the gate/up GEMM with the activation in its epilogue,
+    N = its weight rows.  Touches no GPU."""
+    out = [ctypes.c_int() for _ in range(3)]
+    check(load().dlb_fp8_gemm_plan_stream(M_max, N, K, G, expected_m, int(quantising), compute_units, *(ctypes.byref(v) for v in out)))
+    return (out[0].value, out[1].value, bool(out[2].value)) if out[0].value else None
 
 
 def force_variant(name_or_id) -> None:

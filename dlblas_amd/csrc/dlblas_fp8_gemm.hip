@@ -1668,9 +1668,22 @@ int dlb_fp8_gemm_plan_grouped(int mode, int64_t rows, int64_t N, int64_t K, int3
   const dlb::Resolved rs = dlb::resolve(mode, rows, N, K, G, dlb::ceil_div(K, dlb::kScaleBlock), 1, workspace_bytes > 0, workspace_bytes,
                                         compute_units, false, false, mode == dlb::kMasked ? expected_m : -1);
   if (variant) *variant = rs.pl.variant;
-  // (callers ask whether the form with the quantising epilogue applies)
-  const bool streams = rs.stream != dlb::kStreamNone && (dlb::g_knob[dlb::kKnobStream] >= 2 || dlb::stream_span(rows, expected_m) <= dlb::kStreamActSpan);
-  if (tile_lists) *tile_lists = rs.tile_list || streams ? 1 : 0;
+  if (tile_lists) *tile_lists = rs.tile_list ? 1 : 0;
+  return DLB_OK;
+}
+
+int dlb_fp8_gemm_plan_stream(int64_t rows, int64_t N, int64_t K, int32_t G, int32_t expected_m, int quantising, int compute_units,
+                             int* tile_rows, int* tile_columns, int* ahead) {
+  dlb::clear_error();
+  const int64_t lim = (1ll << 31) - 1024;
+  if (rows < 0 || N < 0 || K < 0 || G < 0 || rows > lim || N > lim || K > lim || compute_units <= 0)
+    return dlb::fail(DLB_ERR_BAD_SHAPE, "bad dimension (rows=%lld, N=%lld, K=%lld, G=%d)", (long long)rows, (long long)N, (long long)K, G);
+  const bool act = quantising != 0;
+  const dlb::Resolved rs = dlb::resolve(dlb::kMasked, rows, N, K, G, dlb::ceil_div(K, dlb::kScaleBlock), 1, false, 0, compute_units, false, act, expected_m);
+  const bool on = rs.stream != dlb::kStreamNone && (!act || (N % (2 * dlb::kScaleBlock) == 0 && N * K < (1ll << 32)));
+  if (tile_rows) *tile_rows = on ? dlb::kStreamDims[rs.stream].bm : 0;
+  if (tile_columns) *tile_columns = on ? dlb::kStreamDims[rs.stream].bn : 0;
+  if (ahead) *ahead = on && rs.ahead ? 1 : 0;
   return DLB_OK;
 }
 

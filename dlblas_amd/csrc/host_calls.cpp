@@ -46,6 +46,7 @@ struct Abi {
   decltype(&dlb_fp8_gemm_grouped_ragged) ragged;
   decltype(&dlb_fp8_gemm_grouped_ragged_silu_quant) ragged_act;
   decltype(&dlb_fp8_gemm_plan_grouped) plan_grouped;
+  decltype(&dlb_fp8_gemm_plan_stream) plan_stream;
   decltype(&dlb_fp8_gemm_variant_name) variant_name;
   decltype(&dlb_fp8_quant_group) quant_group;
   decltype(&dlb_silu_mul_quant_masked) silu_masked;
@@ -310,8 +311,11 @@ PyObject* grouped_masked(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // ---- expert MLPs ------------------------------------------------------------------------------------------------------
 
-bool plan_grouped(int mode, int64_t rows, int64_t N, int64_t K, int64_t G, int64_t hint, const Workspace& ws, int* variant, int* flag) {
-  return abi.plan_grouped(mode, rows, N, K, static_cast<int32_t>(G), static_cast<int32_t>(hint), ws.bytes, 256, variant, flag) == DLB_OK;
+// whether the weight-streaming kernel runs experts of about `hint` rows
+bool streams(int64_t rows, int64_t N, int64_t K, int64_t G, int64_t hint, bool quantising) {
+  int tile_rows = 0;
+  return abi.plan_stream(rows, N, K, static_cast<int32_t>(G), static_cast<int32_t>(hint), quantising, 256, &tile_rows, nullptr, nullptr) == DLB_OK &&
+         tile_rows > 0;
 }
 
 // low_latency_experts(a, a_s, w13, w13_s, w2, w2_s, masked_m, expected_m) -> down_output (bf16)
@@ -335,8 +339,8 @@ PyObject* low_latency_experts(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const hipStream_t stream = stream_of(a);
   Workspace ws;
   if (!workspace_of(scope.dev, stream, a, &ws)) return nullptr;
-  int variant = 0, streams = 0;
-  if (!plan_grouped(2, M, N, K, G, hint, ws, &variant, &streams)) NOT_PLAIN;
+  int variant = 0;
+  if (abi.plan_grouped(2, M, N, K, static_cast<int32_t>(G), static_cast<int32_t>(hint), ws.bytes, 256, &variant, nullptr) != DLB_OK) NOT_PLAIN;
   static const int kRing128 = [] {
     for (int i = 0;; ++i) {
       const char* name = abi.variant_name(i);
@@ -347,7 +351,7 @@ PyObject* low_latency_experts(PyObject*, PyObject* const* args, Py_ssize_t n) {
   at::Tensor q = empty({G, M, inter}, at::kFloat8_e4m3fn, a);
   at::Tensor s;
   bool fused = false;
-  if (streams || variant == kRing128) {
+  if (variant == kRing128 || streams(M, N, K, G, hint, true)) {
     // rows of a K block contiguous: what the second GEMM reads without a re-layout pass
     s = empty_strided({G, M, inter / kBlock}, {inter / kBlock * M, 1, M}, at::kFloat, a);
     fused = abi.masked_act(ptr(a), ptr(w13), fptr(a_s), fptr(w13_s), ptr(q), fptr(s), iptr(mm), static_cast<int32_t>(hint), M, N, K, g,
@@ -435,11 +439,10 @@ PyObject* fused_moe_v3(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (abi.scatter_ws(T, topk, E) > ws.bytes) NOT_PLAIN;
   // typical rows of an expert: half a block of its span is padding on average
   const int64_t rows_each = std::max<int64_t>(1, std::min(rows / used - 64, ceil_div(T * topk, used)));
-  int variant = 0, streams = 0, streams2 = 0, lists = 0;
-  if (!plan_grouped(2, rows, N, H, E, rows_each, ws, &variant, &streams) || !plan_grouped(2, rows, H, inter, E, rows_each, ws, &variant, &streams2))
-    NOT_PLAIN;
-  const bool short_experts = streams && streams2;
-  if (!short_experts && (!plan_grouped(1, rows, N, H, E, -1, ws, &variant, &lists) || !lists)) NOT_PLAIN;  // three steps on uniform tiles
+  int lists = 0;
+  const bool short_experts = streams(rows, N, H, E, rows_each, true) && streams(rows, H, inter, E, rows_each, false);
+  if (!short_experts && (abi.plan_grouped(1, rows, N, H, static_cast<int32_t>(E), -1, ws.bytes, 256, nullptr, &lists) != DLB_OK || !lists))
+    NOT_PLAIN;  // three steps on uniform tiles
 
   // one allocation for the int32 tables: expert and token of every row, row ranges and first free rows of the experts
   at::Tensor tables = empty({2 * rows + 3 * E}, at::kInt, x);

@@ -161,8 +161,8 @@ def fused_moe_v3(
         if n_experts <= 256 and n_tokens * hidden < (1 << 31):
             used = sum(1 for c in num_recv_tokens_per_expert if c > 0)
             rows_each = max(1, min(rows_total // used - 64, -(-n_tokens * topk_idx.size(1) // used)))  # half a block of padding on average
-            streams = (_lib.plan_grouped(2, rows_total, inter2, hidden, n_experts, rows_each)[1]
-                       and _lib.plan_grouped(2, rows_total, hidden, inter2 // 2, n_experts, rows_each)[1])
+            streams = (_lib.plan_stream(rows_total, inter2, hidden, n_experts, rows_each, quantising=True) is not None
+                       and _lib.plan_stream(rows_total, hidden, inter2 // 2, n_experts, rows_each) is not None)
         lists = _lib.plan_grouped(1, rows_total, inter2, hidden, n_experts)[1]
         if streams or lists:
             row_token = buf((rows_total, ), torch.int32)

@@ -80,8 +80,8 @@ def low_latency_experts(
     # The fused epilogue exists for the weight-streaming kernel (short experts) and for the 128 x 256 tiles; where the
     # library picks other tiles for the plain GEMM (several hundred rows per expert) the steps apart are faster (32
     # experts x ~520 rows: 619 against 678 us).
-    variant, streams = _lib.plan_grouped(2, m, n, k, num_groups, expected_m)
-    want_fused = streams or variant == 'pipe128x256w8'
+    want_fused = (_lib.plan_grouped(2, m, n, k, num_groups, expected_m)[0] == 'pipe128x256w8'
+                  or _lib.plan_stream(m, n, k, num_groups, expected_m, quantising=True) is not None)
     if want_fused and out_dtype == torch.bfloat16 and block_size == 128 and n % 256 == 0 and masked_m.dtype == torch.int32:
         # one kernel for GEMM + activation + quantiser, same bits; its scales go out with the rows of a K block
         # contiguous, the layout the second GEMM reads without a re-layout pass

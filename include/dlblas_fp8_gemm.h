@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define DLB_ABI_VERSION 8
+#define DLB_ABI_VERSION 9
 
 /* output element type of C */
 #define DLB_OUT_BF16 0
@@ -340,8 +340,8 @@ int dlb_fp8_quant_128x128(const void* w, int w_dtype, void* q, float* s, int64_t
  * mode 0 = dlb_fp8_gemm, 1 = grouped contiguous (rows = M_sum), 2 = grouped masked (rows = M_max); `compute_units`
  * is the CU count to plan for (256 on MI355X); activation scales are taken to be row-major.  Outputs (each may be
  * NULL): the kernel variant id (dlb_fp8_gemm_variant_name); the number of K slices summed in a second pass (1 = none),
- * exactly as a launch with this workspace size would use it (unless the kernel of dlb_fp8_gemm_plan_wave_k takes it over); the output columns per workgroup of the decode kernels
- * (0 for other variants); the first column of the 192-wide tiles of the mixed-width prefill launch (N when all tiles
+ * exactly as a launch with this workspace size would use it, unless the kernel of dlb_fp8_gemm_plan_wave_k takes it over
+ * (mode 2: that of dlb_fp8_gemm_plan_stream); the output columns per workgroup of the decode kernels (0 for other variants); the first column of the 192-wide tiles of the mixed-width prefill launch (N when all tiles
  * are equal).  Honours the calling thread's forced variant and knobs, as a launch does (both run the same code).
  * Costs a few microseconds at most and keeps no state.  No counterpart in the reference, whose single Triton
  * configuration needs no plan.
@@ -361,15 +361,24 @@ int dlb_fp8_gemm_plan_wave_k(int64_t M, int64_t N, int64_t K, size_t workspace_b
  * The same query for the grouped layouts with what their choice depends on besides the shape: the expert count and, for
  * the masked layout (mode 2), the caller's expected_m (<= 0: unknown).  mode 1 = contiguous (rows = M_sum), 2 = masked
  * (rows = M_max).  Outputs (each may be NULL): the kernel variant id; whether a contiguous launch of this size pairs
- * blocks into taller tiles from lists built on the device (1) or runs uniform 128-row tiles (0); for the masked layout,
- * whether the weight-streaming kernel runs in place of the named variant, at row counts where its form with the
- * quantising epilogue does too (1).  The fused gate/up
- * entry points always take the lists, so a caller that can also run GEMM and activation apart does that where this
- * says 0 (a batch of at most a round or two of tiles, where the uniform tiles are faster).  No counterpart in the
+ * blocks into taller tiles from lists built on the device (1) or runs uniform 128-row tiles (0; always 0 for the masked
+ * layout, where dlb_fp8_gemm_plan_stream may take the launch over from the named variant).  The fused gate/up entry points
+ * of the contiguous layout always take the lists, so a caller that can also run GEMM and activation apart does that where
+ * this says 0 (a batch of at most a round or two of tiles, where the uniform tiles are faster).  No counterpart in the
  * reference.
  */
 int dlb_fp8_gemm_plan_grouped(int mode, int64_t rows, int64_t N, int64_t K, int32_t G, int32_t expected_m, size_t workspace_bytes,
                               int compute_units, int* variant, int* tile_lists);
+
+/*
+ * Whether the weight-streaming kernel takes a masked launch over from the variant dlb_fp8_gemm_plan_grouped names, and with
+ * which tile: rows, weight rows and whether it reads its fragments one step ahead, all 0 when it does not.  `quantising` != 0
+ * asks for dlb_fp8_gemm_grouped_masked_silu_quant (N = its weight rows), 0 for dlb_fp8_gemm_grouped_masked.  The ragged entry
+ * points run the same choice with rows = M_sum and have no other kernel: they decline where this says 0.  No counterpart in
+ * the reference.
+ */
+int dlb_fp8_gemm_plan_stream(int64_t rows, int64_t N, int64_t K, int32_t G, int32_t expected_m, int quantising, int compute_units,
+                             int* tile_rows, int* tile_columns, int* ahead);
 
 /*
  * Tuning / test hook: force the kernel variant the next calls FROM THIS THREAD use.

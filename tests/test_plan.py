@@ -206,3 +206,26 @@ def test_where_the_wave_split_kernel_takes_over():
     for M, N, K in ((1, 28480, 1152), (16, 36864, 512), (17, 2112, 7168), (64, 7168, 18432), (100, 2112, 7168), (500, 4096, 7168),
                     (1, 4096, 1040), (300, 1000, 1040), (4096, 24576, 1040), (300, 24576, 5136)):
         assert _lib.plan_wave_k(M, N, K) is not None, (M, N, K)
+
+
+def test_plan_stream_answers_for_either_form():
+    """Experts of 193 to 448 rows stream in the plain form only; K shorter than the ring, a ragged K and a forced variant leave
+    the launch to the named ring kernel.  The tile-list output of the grouped query is about the contiguous layout alone."""
+    assert _lib.plan_stream(256, 7168, 2048, 32, 128) == (128, 256, True)
+    assert _lib.plan_stream(256, 7168, 2048, 32, 128, quantising=True) is None
+    assert _lib.plan_stream(448, 7168, 3072, 32) is not None and _lib.plan_stream(449, 7168, 3072, 32) is None
+    assert _lib.plan_stream(256, 4096, 7168, 32) is not None and _lib.plan_stream(257, 4096, 7168, 32) is None
+    assert _lib.plan_stream(192, 4096, 7168, 32, quantising=True) is not None and _lib.plan_stream(193, 4096, 7168, 32, quantising=True) is None
+    assert _lib.plan_stream(1024, 4096, 7168, 32, 32, quantising=True) == (64, 256, False)  # twice the hint covers the experts
+    assert _lib.plan_stream(64, 4096, 256, 32) is None and _lib.plan_stream(64, 4096, 400, 32) is None
+    assert _lib.plan_stream(64, 384, 1024, 8) is not None and _lib.plan_stream(64, 384, 1024, 8, quantising=True) is None
+    _lib.force_variant('pipe128x256w8')
+    assert _lib.plan_stream(256, 7168, 2048, 32, 128) is None
+    _lib.force_variant(None)
+    _lib.tune('stream', 4)
+    assert _lib.plan_stream(256, 7168, 2048, 32, 128)[:2] == (64, 128)
+    _lib.tune('stream', 0)
+    for rows, hint in ((16, 8), (128, 32), (256, 128), (512, 256)):
+        assert _lib.plan_grouped(MASKED, rows, 4096, 7168, 32, hint)[1] is False
+    assert _lib.plan_grouped(CONTIGUOUS, 9728, 4096, 7168, 32)[1] is True
+    assert _lib.load().dlb_fp8_gemm_plan_stream(-1, 1, 1, 1, 0, 0, 256, None, None, None) == _lib.ERR_BAD_SHAPE
