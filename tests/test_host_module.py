@@ -1,0 +1,50 @@
+"""Loading of the native entry points (dlblas_amd/_fast.py): what happens without the module or without the library.  No GPU."""
+import warnings
+
+import pytest
+
+from dlblas_amd import _fast, _lib
+
+
+@pytest.fixture
+def fresh(monkeypatch):
+    """_fast as before its first use; restored afterwards."""
+    for name in _fast._FUNCTIONS:
+        monkeypatch.delitem(_fast.__dict__, name, raising=False)
+    yield monkeypatch
+    for name in _fast._FUNCTIONS:
+        _fast.__dict__.pop(name, None)
+
+
+@pytest.mark.parametrize('content', [None, b'not a library'])
+def test_without_the_module_every_call_is_declined(fresh, tmp_path, content):
+    path = tmp_path / '_host.so'
+    if content is not None:
+        path.write_bytes(content)
+    fresh.setattr(_fast, 'HOST_PATH', str(path))
+    with pytest.warns(RuntimeWarning, match='_host.so'):
+        assert _fast.fp8_gemm(1, 2, 3, 4) is None
+    with warnings.catch_warnings():
+        warnings.simplefilter('error')  # one warning, not one a call
+        for name in _fast._FUNCTIONS:
+            assert getattr(_fast, name)() is None
+
+
+def test_without_the_library_the_python_path_reports_it(fresh, tmp_path):
+    import torch
+
+    from dlblas_amd.kernels.fp8 import per_token_group_quant_fp8
+    fresh.setattr(_lib, '_lib', None)
+    fresh.setenv('DLBLAS_AMD_LIB', str(tmp_path / 'missing.so'))
+    assert _fast.quant(torch.zeros(2, 128), 128, 1e-10, False) is None
+    with pytest.raises(NotImplementedError):  # the op itself: no kernel for CPU tensors
+        per_token_group_quant_fp8(torch.zeros(2, 128, dtype=torch.bfloat16), 128)
+    with pytest.raises(ImportError, match='has not been built'):
+        _lib.load()
+
+
+def test_the_module_is_used_when_it_is_there(fresh):
+    with warnings.catch_warnings():
+        warnings.simplefilter('error')
+        assert _fast.fp8_gemm is not _fast._declined
+        assert _fast.fp8_gemm(1, 2, 3, 4) is None  # not tensors: left to the Python path
