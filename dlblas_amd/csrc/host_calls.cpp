@@ -12,6 +12,7 @@
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/record_function.h>
 #include <c10/core/DefaultDtype.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -26,6 +27,7 @@
 #include <string>
 #include <unordered_map>
 #include <utility>
+#include <vector>
 
 #include "../../include/dlblas_fp8_gemm.h"
 #include "../../include/dlblas_fp8_moe.h"
@@ -151,6 +153,19 @@ int out_code(at::ScalarType t) { return t == at::kBFloat16 ? DLB_OUT_BF16 : t ==
 int in_code(at::ScalarType t) { return t == at::kBFloat16 ? DLB_IN_BF16 : t == at::kHalf ? DLB_IN_F16 : t == at::kFloat ? DLB_IN_F32 : -1; }
 int idx_code(at::ScalarType t) { return t == at::kInt ? DLB_IDX_I32 : t == at::kLong ? DLB_IDX_I64 : -1; }
 
+// An op event of torch's profiler, as the custom ops of the Python path leave one; nothing when nobody records.
+struct OpRecord {
+  at::RecordFunction guard{at::RecordScope::FUNCTION};
+  std::vector<c10::IValue> inputs;
+  template <size_t N>
+  OpRecord(const char* name, const at::Tensor* const (&t)[N]) {
+    if (!guard.isActive()) return;
+    if (guard.needsInputs())
+      for (const at::Tensor* x : t) inputs.emplace_back(*x);
+    guard.before(name, c10::ArrayRef<const c10::IValue>(inputs.data(), inputs.size()));
+  }
+};
+
 // After the first launch of a chain there is no way back to the Python path.
 PyObject* launch_failed(int rc) {
   return PyErr_Format(PyExc_RuntimeError, "dlblas fp8_gemm error %d: %s", rc, abi.last_error());
@@ -184,6 +199,7 @@ PyObject* fp8_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (K == 0 || N == 0 || a.size(-1) != K) NOT_PLAIN;
   const int64_t M = a.numel() / K;
   if (M == 0 || a_s.numel() != M * kb || a_s.size(-1) != kb || b_s.size(0) != ceil_div(N, kBlock) || b_s.size(1) != kb) NOT_PLAIN;
+  const OpRecord record("dlblas::fp8_gemm", t);
   DeviceScope scope(a);
   const hipStream_t stream = stream_of(a);
   Workspace ws;
@@ -214,6 +230,7 @@ PyObject* quant(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (in_code(x.scalar_type()) < 0 || x.dim() < 2 || group <= 0 || x.stride(-1) != 1 || x.numel() == 0) NOT_PLAIN;
   const int64_t K = x.size(-1), rows = x.numel() / K;
   if (K % group != 0 || (x.dim() > 2 && !x.is_contiguous())) NOT_PLAIN;
+  const OpRecord record("dlblas::per_token_group_quant_fp8", t);
   const int64_t groups = K / group;
   const int64_t row_stride = x.dim() == 2 ? x.stride(0) : K;
   DeviceScope scope(x);
@@ -263,6 +280,7 @@ PyObject* grouped_contiguous(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (M == 0 || !a.is_contiguous() || !out.is_contiguous() || a_s.size(0) != M || a_s.size(1) != kb || out.size(0) != M || out.size(1) != N ||
       !index_vector(idx, M))
     NOT_PLAIN;
+  const OpRecord record("dlblas::fp8_gemm_grouped_contiguous", t);
   DeviceScope scope(a);
   const hipStream_t stream = stream_of(a);
   Workspace ws;
@@ -296,6 +314,7 @@ PyObject* grouped_masked(PyObject*, PyObject* const* args, Py_ssize_t n) {
     PyErr_Clear();
     NOT_PLAIN;
   }
+  const OpRecord record("dlblas::fp8_gemm_grouped_masked", t);
   DeviceScope scope(a);
   const hipStream_t stream = stream_of(a);
   Workspace ws;
@@ -335,6 +354,7 @@ PyObject* low_latency_experts(PyObject*, PyObject* const* args, Py_ssize_t n) {
   }
   hint = std::min<long>(hint, M);
   if (hint != static_cast<int32_t>(hint)) NOT_PLAIN;
+  const OpRecord record("dlblas::low_latency_experts", t);
   DeviceScope scope(a);
   const hipStream_t stream = stream_of(a);
   Workspace ws;
@@ -395,6 +415,7 @@ PyObject* ep_gather(PyObject*, PyObject* const* args, Py_ssize_t n) {
       out.stride(1) != 1 || in_code(in.scalar_type()) < 0 || in_code(out.scalar_type()) < 0 || !routing_ok(ids, weights, out.size(0)) ||
       idx_code(index.scalar_type()) < 0 || index.sizes() != ids.sizes())
     NOT_PLAIN;
+  const OpRecord record("dlblas::ep_gather", t);
   DeviceScope scope(in);
   if (gather(in, ids, weights, index, out, stream_of(in)) != DLB_OK) NOT_PLAIN;
   written(out);
@@ -443,6 +464,7 @@ PyObject* fused_moe_v3(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const bool short_experts = streams(rows, N, H, E, rows_each, true) && streams(rows, H, inter, E, rows_each, false);
   if (!short_experts && (abi.plan_grouped(1, rows, N, H, static_cast<int32_t>(E), -1, ws.bytes, 256, nullptr, &lists) != DLB_OK || !lists))
     NOT_PLAIN;  // three steps on uniform tiles
+  const OpRecord record("dlblas::fused_moe_v3", t);
 
   // one allocation for the int32 tables: expert and token of every row, row ranges and first free rows of the experts
   at::Tensor tables = empty({2 * rows + 3 * E}, at::kInt, x);

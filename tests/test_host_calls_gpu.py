@@ -211,3 +211,37 @@ def test_fused_moe_v3_reads_the_tokens_in_place_beyond_the_native_call(dev, monk
     torch.cuda.synchronize()
     assert ran == ['copy']  # ... and three steps
     assert torch.equal(out, ref) and bool(out.isfinite().all()) and float(out.abs().max()) > 0
+
+
+def _small_experts(dev, E=2, H=512, inter=512):
+    g = torch.Generator(device=dev).manual_seed(5)
+    codes = lambda *s: torch.randint(0, 0x60, s, device=dev, generator=g, dtype=torch.uint8).view(torch.float8_e4m3fn)
+    return (codes(E, 2 * inter, H), torch.ones(E, 2 * inter // 128, H // 128, device=dev)), (codes(E, H, inter), torch.ones(E, H // 128, inter // 128, device=dev)), codes
+
+
+def test_native_calls_are_ops_to_the_profiler(dev):
+    """Every native call leaves an op event, with its inputs' shapes where they are asked for."""
+    from dlblas_amd.kernels.fp8 import per_token_group_quant_fp8
+    from dlblas_amd.kernels.fp8_gemm import fp8_gemm
+    from dlblas_amd.kernels.fp8_gemm_grouped import m_grouped_fp8_gemm_nt_contiguous, m_grouped_fp8_gemm_nt_masked
+    from dlblas_amd.kernels.fused_moe_v3 import ep_gather, fused_moe_v3
+    from dlblas_amd.kernels.moe import low_latency_experts
+    w13, w2, codes = _small_experts(dev)
+    args = _operands((16, ), 128, 256, dev)
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=dev)
+    a3, s3 = codes(2, 64, 512), torch.ones(2, 64, 4, device=dev)
+    ids, wts = torch.tensor([[0], [1], [0]], device=dev), torch.ones(3, 1, device=dev)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], record_shapes=True) as prof:
+        per_token_group_quant_fp8(torch.ones(4, 256, dtype=torch.bfloat16, device=dev), 128)
+        fp8_gemm(*args)
+        m_grouped_fp8_gemm_nt_contiguous((codes(128, 512), torch.ones(128, 4, device=dev)), w13, torch.empty(128, 1024, dtype=torch.bfloat16, device=dev),
+                                         torch.zeros(128, dtype=torch.int32, device=dev))
+        m_grouped_fp8_gemm_nt_masked((a3, s3), w13, torch.empty(2, 64, 1024, dtype=torch.bfloat16, device=dev), i32(3, 0), 2)
+        down = low_latency_experts((a3, s3), *w13, *w2, i32(3, 1), 2)
+        ep_gather(down.view(-1, 512), ids, wts, i32(0, 64, 1).view(3, 1), torch.empty(3, 512, dtype=torch.bfloat16, device=dev))
+        fused_moe_v3((codes(3, 512), torch.ones(3, 4, device=dev)), ids, wts, w13, w2, [128, 128])
+        torch.cuda.synchronize()
+    shapes = {e.name: e.input_shapes for e in prof.events() if e.name.startswith('dlblas::')}
+    assert shapes.keys() >= {'dlblas::' + n for n in ('per_token_group_quant_fp8', 'fp8_gemm', 'fp8_gemm_grouped_contiguous', 'fp8_gemm_grouped_masked',
+                                                      'low_latency_experts', 'ep_gather', 'fused_moe_v3')}
+    assert shapes['dlblas::fp8_gemm'][:2] == [[16, 256], [128, 256]]
