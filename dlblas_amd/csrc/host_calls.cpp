@@ -5,7 +5,7 @@
 //
 // Every function takes the arguments of the Python function of its name and either does the call or returns None without
 // having enqueued anything.  None means "not a plain call": tensor subclasses, dispatch and function modes, tracing, inputs
-// that require grad, arguments the checks refuse, layouts only the Python path handles.  The Python function then goes on as
+// that require grad or carry a tangent, arguments the checks refuse, layouts only the Python path handles.  The Python function then goes on as
 // it would without this module, through its custom op and its own checks and messages.
 #include <Python.h>
 
@@ -73,7 +73,7 @@ const at::Tensor* plain(PyObject* o) {
   if (!THPVariable_CheckExact(o)) return nullptr;
   const at::Tensor& t = THPVariable_Unpack(o);
   if (!t.defined() || !t.is_cuda() || !within(t.key_set(), kPlainKeys)) return nullptr;
-  if (t.is_conj() || t.is_neg() || (c10::GradMode::is_enabled() && t.requires_grad())) return nullptr;
+  if (t.is_conj() || t.is_neg() || (c10::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(0).defined()) return nullptr;
   return &t;
 }
 

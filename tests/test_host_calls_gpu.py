@@ -245,3 +245,15 @@ def test_native_calls_are_ops_to_the_profiler(dev):
     assert shapes.keys() >= {'dlblas::' + n for n in ('per_token_group_quant_fp8', 'fp8_gemm', 'fp8_gemm_grouped_contiguous', 'fp8_gemm_grouped_masked',
                                                       'low_latency_experts', 'ep_gather', 'fused_moe_v3')}
     assert shapes['dlblas::fp8_gemm'][:2] == [[16, 256], [128, 256]]
+
+
+def test_tensors_with_a_tangent_are_left_to_the_python_path(dev):
+    """Forward-mode derivatives are the dispatcher's to refuse or to drop, not the native call's to overlook."""
+    from torch.autograd import forward_ad
+
+    from dlblas_amd import _fast
+    x = torch.randn(4, 256, device=dev)
+    assert _fast.quant(x, 128, 1e-10, False) is not None
+    with forward_ad.dual_level():
+        assert _fast.quant(forward_ad.make_dual(x, torch.ones_like(x)), 128, 1e-10, False) is None
+    assert _fast.quant(x, 128, 1e-10, False) is not None
