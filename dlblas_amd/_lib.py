@@ -59,6 +59,8 @@ SYMBOLS = {
     'dlb_fp8_gemm_plan_wave_k': (ctypes.c_int, [_c_i64] * 3 + [_c_sz, ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 3),
     'dlb_fp8_gemm_plan_grouped': (ctypes.c_int, [ctypes.c_int, _c_i64, _c_i64, _c_i64, ctypes.c_int32, ctypes.c_int32, _c_sz, ctypes.c_int,
                                                 ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]),
+    'dlb_workspace_lock': (ctypes.c_int, [_c_vp]),
+    'dlb_workspace_unlock': (ctypes.c_int, [_c_vp]),
     'dlb_fp8_gemm_plan_stream': (ctypes.c_int, [_c_i64] * 3 + [_c_i32] * 2 + [ctypes.c_int] * 2 + [ctypes.POINTER(ctypes.c_int)] * 3),
     'dlb_silu_mul': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp] + [_c_i64] * 4 + [_c_vp]),
     'dlb_silu_mul_quant': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp, _c_vp] + [_c_i64] * 5 + [ctypes.c_float, _c_vp]),
@@ -137,7 +139,8 @@ def check(rc: int) -> None:
 
 
 def workspace(device: torch.device, stream_handle: int) -> torch.Tensor:
-    """Zero-initialised scratch buffer, one per (device, stream): calls on one stream never overlap."""
+    """Zero-initialised scratch buffer, one per (device, stream): calls on one stream never overlap, and the library lets the
+    launches of one call go out together when several threads use the stream."""
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream_handle)
     buf = _workspaces.get(key)
     if buf is None:

@@ -1097,6 +1097,7 @@ int run(const Problem& pr) {
   bool empty = false;
   const int bad = check_problem(pr, &empty);
   if (bad != DLB_OK || empty) return bad;
+  const WorkspaceLock lock(pr.ws);
   const int64_t groups = pr.mode == kDense ? 1 : pr.G;
   const int64_t kblocks = ceil_div(pr.K, kScaleBlock);
 
@@ -1407,6 +1408,20 @@ size_t dlb_fp8_gemm_workspace_bytes(int64_t rows, int64_t N, int64_t K) {
   const int64_t padded = dlb::ceil_div(rows, 128) * dlb::ceil_div(N, 128);
   const size_t want = padded > 1024 ? cap : static_cast<size_t>(padded) * 128 * 128 * sizeof(float) * 16;
   return DLB_WS_COUNTER_BYTES + (want < cap ? want : cap);
+}
+
+int dlb_workspace_lock(const void* workspace) {
+  dlb::clear_error();
+  if (!workspace) return dlb::fail(DLB_ERR_NULL_POINTER, "workspace is NULL");
+  dlb::workspace_mutex(workspace).lock();
+  return DLB_OK;
+}
+
+int dlb_workspace_unlock(const void* workspace) {
+  dlb::clear_error();
+  if (!workspace) return dlb::fail(DLB_ERR_NULL_POINTER, "workspace is NULL");
+  dlb::workspace_mutex(workspace).unlock();
+  return DLB_OK;
 }
 
 int dlb_fp8_gemm(const void* a, const void* b, const float* a_s, const float* b_s, void* c, int64_t M, int64_t N,

@@ -214,6 +214,7 @@ int scatter_impl(const void* recv_x, int64_t x_row_stride, const float* recv_x_s
   if (!workspace || workspace_bytes < need)
     return fail(DLB_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace ? workspace_bytes : (size_t)0);
   if (misaligned(workspace, 8)) return fail(DLB_ERR_ALIGNMENT, "workspace must be 8-byte aligned");
+  const WorkspaceLock lock(workspace);
 
   ScatterArgs a;
   memset(&a, 0, sizeof(a));

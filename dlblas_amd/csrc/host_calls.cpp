@@ -39,6 +39,8 @@ constexpr int64_t kBlock = 128;
 // The entry points of the library that ctypes has loaded, by address (init() below): one library, whichever was chosen.
 struct Abi {
   decltype(&dlb_last_error) last_error;
+  decltype(&dlb_workspace_lock) lock;
+  decltype(&dlb_workspace_unlock) unlock;
   decltype(&dlb_fp8_gemm) gemm;
   decltype(&dlb_fp8_gemm_grouped_contiguous) contiguous;
   decltype(&dlb_fp8_gemm_grouped_contiguous_same_rows) contiguous_same_rows;
@@ -166,6 +168,32 @@ struct OpRecord {
   }
 };
 
+// Allocations and launches run without the GIL: a launch waits while the hardware queue is full.  No Python object is touched
+// in such a scope.
+class NoGil {
+ public:
+  NoGil() : state_(PyEval_SaveThread()) {}
+  ~NoGil() { PyEval_RestoreThread(state_); }
+  NoGil(const NoGil&) = delete;
+  NoGil& operator=(const NoGil&) = delete;
+
+ private:
+  PyThreadState* state_;
+};
+
+// Keeps the launches of several library calls on one workspace together.  Inside a NoGil scope only: a thread that waits for
+// the lock must not keep its holder from finishing.
+class Together {
+ public:
+  explicit Together(const Workspace& ws) : ws_(ws.ptr) { abi.lock(ws_); }
+  ~Together() { abi.unlock(ws_); }
+  Together(const Together&) = delete;
+  Together& operator=(const Together&) = delete;
+
+ private:
+  const void* ws_;
+};
+
 // After the first launch of a chain there is no way back to the Python path.
 PyObject* launch_failed(int rc) {
   return PyErr_Format(PyExc_RuntimeError, "dlblas fp8_gemm error %d: %s", rc, abi.last_error());
@@ -206,8 +234,13 @@ PyObject* fp8_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!workspace_of(scope.dev, stream, a, &ws)) return nullptr;
   at::DimVector size(a.sizes());
   size.back() = N;
-  at::Tensor c = empty(size, out, a);
-  const int rc = abi.gemm(ptr(a), ptr(b), fptr(a_s), fptr(b_s), ptr(c), M, N, K, kb, 1, out_code(out), ws.ptr, ws.bytes, stream);
+  at::Tensor c;
+  int rc;
+  {
+    const NoGil nogil;
+    c = empty(size, out, a);
+    rc = abi.gemm(ptr(a), ptr(b), fptr(a_s), fptr(b_s), ptr(c), M, N, K, kb, 1, out_code(out), ws.ptr, ws.bytes, stream);
+  }
   if (rc != DLB_OK) NOT_PLAIN;
   return THPVariable_Wrap(std::move(c));
   HANDLE_EXCEPTIONS_END
@@ -234,21 +267,25 @@ PyObject* quant(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int64_t groups = K / group;
   const int64_t row_stride = x.dim() == 2 ? x.stride(0) : K;
   DeviceScope scope(x);
-  at::Tensor q = empty(x.sizes(), at::kFloat8_e4m3fn, x);
-  at::Tensor s;
+  at::Tensor q, s;
   at::DimVector size(x.sizes());
   size.back() = groups;
-  if (col_major) {
-    // a [groups, rows...] buffer viewed with the group axis last
-    at::DimVector stride(x.dim(), 1);
-    for (int64_t d = x.dim() - 3; d >= 0; --d) stride[d] = stride[d + 1] * size[d + 1];
-    stride.back() = rows;
-    s = empty_strided(size, stride, at::kFloat, x);
-  } else {
-    s = empty(size, at::kFloat, x);
+  int rc;
+  {
+    const NoGil nogil;
+    q = empty(x.sizes(), at::kFloat8_e4m3fn, x);
+    if (col_major) {
+      // a [groups, rows...] buffer viewed with the group axis last
+      at::DimVector stride(x.dim(), 1);
+      for (int64_t d = x.dim() - 3; d >= 0; --d) stride[d] = stride[d + 1] * size[d + 1];
+      stride.back() = rows;
+      s = empty_strided(size, stride, at::kFloat, x);
+    } else {
+      s = empty(size, at::kFloat, x);
+    }
+    rc = abi.quant_group(ptr(x), in_code(x.scalar_type()), ptr(q), fptr(s), rows, K, group, row_stride, col_major ? 1 : groups, col_major ? rows : 1,
+                         eps, stream_of(x));
   }
-  const int rc = abi.quant_group(ptr(x), in_code(x.scalar_type()), ptr(q), fptr(s), rows, K, group, row_stride, col_major ? 1 : groups,
-                                 col_major ? rows : 1, eps, stream_of(x));
   if (rc != DLB_OK) NOT_PLAIN;
   PyObject* out = PyTuple_New(2);
   if (!out) return nullptr;
@@ -285,8 +322,12 @@ PyObject* grouped_contiguous(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const hipStream_t stream = stream_of(a);
   Workspace ws;
   if (!workspace_of(scope.dev, stream, a, &ws)) return nullptr;
-  const int rc = abi.contiguous(ptr(a), ptr(w), fptr(a_s), fptr(w_s), ptr(out), iptr(idx), M, N, K, static_cast<int32_t>(G), a_s.stride(0),
-                                a_s.stride(1), out_code(out.scalar_type()), ws.ptr, ws.bytes, stream);
+  int rc;
+  {
+    const NoGil nogil;
+    rc = abi.contiguous(ptr(a), ptr(w), fptr(a_s), fptr(w_s), ptr(out), iptr(idx), M, N, K, static_cast<int32_t>(G), a_s.stride(0), a_s.stride(1),
+                        out_code(out.scalar_type()), ws.ptr, ws.bytes, stream);
+  }
   if (rc != DLB_OK) NOT_PLAIN;
   written(out);
   Py_RETURN_TRUE;
@@ -319,9 +360,12 @@ PyObject* grouped_masked(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const hipStream_t stream = stream_of(a);
   Workspace ws;
   if (!workspace_of(scope.dev, stream, a, &ws)) return nullptr;
-  const int rc = abi.masked(ptr(a), ptr(w), fptr(a_s), fptr(w_s), ptr(out), iptr(mm), static_cast<int32_t>(hint), a.size(1), N, K,
-                            static_cast<int32_t>(G), a_s.stride(0), a_s.stride(1), a_s.stride(2), out_code(out.scalar_type()), ws.ptr, ws.bytes,
-                            stream);
+  int rc;
+  {
+    const NoGil nogil;
+    rc = abi.masked(ptr(a), ptr(w), fptr(a_s), fptr(w_s), ptr(out), iptr(mm), static_cast<int32_t>(hint), a.size(1), N, K, static_cast<int32_t>(G),
+                    a_s.stride(0), a_s.stride(1), a_s.stride(2), out_code(out.scalar_type()), ws.ptr, ws.bytes, stream);
+  }
   if (rc != DLB_OK) NOT_PLAIN;
   written(out);
   Py_RETURN_TRUE;
@@ -367,30 +411,42 @@ PyObject* low_latency_experts(PyObject*, PyObject* const* args, Py_ssize_t n) {
       if (!name || std::string(name) == "pipe128x256w8") return i;
     }
   }();
-  const int32_t g = static_cast<int32_t>(G);
-  at::Tensor q = empty({G, M, inter}, at::kFloat8_e4m3fn, a);
-  at::Tensor s;
-  bool fused = false;
-  if (variant == kRing128 || streams(M, N, K, G, hint, true)) {
-    // rows of a K block contiguous: what the second GEMM reads without a re-layout pass
-    s = empty_strided({G, M, inter / kBlock}, {inter / kBlock * M, 1, M}, at::kFloat, a);
-    fused = abi.masked_act(ptr(a), ptr(w13), fptr(a_s), fptr(w13_s), ptr(q), fptr(s), iptr(mm), static_cast<int32_t>(hint), M, N, K, g,
-                           a_s.stride(0), a_s.stride(1), a_s.stride(2), s.stride(0), s.stride(1), s.stride(2), 1e-10f, ws.ptr, ws.bytes,
-                           stream) == DLB_OK;
+  const int32_t g = static_cast<int32_t>(G), m_hint = static_cast<int32_t>(hint);
+  at::Tensor q, s, gate_up, out;
+  int rc = DLB_OK;
+  bool begun = false;  // something is enqueued: no way back to the Python path
+  {
+    const NoGil nogil;
+    q = empty({G, M, inter}, at::kFloat8_e4m3fn, a);
+    bool fused = false;
+    if (variant == kRing128 || streams(M, N, K, G, hint, true)) {
+      // rows of a K block contiguous: what the second GEMM reads without a re-layout pass
+      s = empty_strided({G, M, inter / kBlock}, {inter / kBlock * M, 1, M}, at::kFloat, a);
+      fused = abi.masked_act(ptr(a), ptr(w13), fptr(a_s), fptr(w13_s), ptr(q), fptr(s), iptr(mm), m_hint, M, N, K, g, a_s.stride(0), a_s.stride(1),
+                             a_s.stride(2), s.stride(0), s.stride(1), s.stride(2), 1e-10f, ws.ptr, ws.bytes, stream) == DLB_OK;
+    }
+    if (!fused) {
+      gate_up = empty({G, M, N}, at::kBFloat16, a);
+      rc = abi.masked(ptr(a), ptr(w13), fptr(a_s), fptr(w13_s), ptr(gate_up), iptr(mm), m_hint, M, N, K, g, a_s.stride(0), a_s.stride(1), a_s.stride(2),
+                      DLB_OUT_BF16, ws.ptr, ws.bytes, stream);
+      if (rc == DLB_OK) {
+        begun = true;
+        s = empty({G, M, inter / kBlock}, at::kFloat, a);
+        rc = abi.silu_masked(ptr(gate_up), DLB_IN_BF16, ptr(q), fptr(s), iptr(mm), G, M, inter, s.stride(0), s.stride(1), s.stride(2), stream);
+        gate_up.reset();
+      }
+    }
+    if (rc == DLB_OK) {
+      begun = true;
+      out = empty({G, M, H}, at::kBFloat16, a);
+      rc = abi.masked(ptr(q), ptr(w2), fptr(s), fptr(w2_s), ptr(out), iptr(mm), m_hint, M, H, inter, g, s.stride(0), s.stride(1), s.stride(2),
+                      DLB_OUT_BF16, ws.ptr, ws.bytes, stream);
+    }
   }
-  if (!fused) {
-    at::Tensor gate_up = empty({G, M, N}, at::kBFloat16, a);
-    int rc = abi.masked(ptr(a), ptr(w13), fptr(a_s), fptr(w13_s), ptr(gate_up), iptr(mm), static_cast<int32_t>(hint), M, N, K, g, a_s.stride(0),
-                        a_s.stride(1), a_s.stride(2), DLB_OUT_BF16, ws.ptr, ws.bytes, stream);
-    if (rc != DLB_OK) NOT_PLAIN;
-    s = empty({G, M, inter / kBlock}, at::kFloat, a);
-    rc = abi.silu_masked(ptr(gate_up), DLB_IN_BF16, ptr(q), fptr(s), iptr(mm), G, M, inter, s.stride(0), s.stride(1), s.stride(2), stream);
-    if (rc != DLB_OK) return launch_failed(rc);
+  if (rc != DLB_OK) {
+    if (begun) return launch_failed(rc);
+    NOT_PLAIN;
   }
-  at::Tensor out = empty({G, M, H}, at::kBFloat16, a);
-  const int rc = abi.masked(ptr(q), ptr(w2), fptr(s), fptr(w2_s), ptr(out), iptr(mm), static_cast<int32_t>(hint), M, H, inter, g, s.stride(0),
-                            s.stride(1), s.stride(2), DLB_OUT_BF16, ws.ptr, ws.bytes, stream);
-  if (rc != DLB_OK) return launch_failed(rc);
   return THPVariable_Wrap(std::move(out));
   HANDLE_EXCEPTIONS_END
 }
@@ -417,7 +473,12 @@ PyObject* ep_gather(PyObject*, PyObject* const* args, Py_ssize_t n) {
     NOT_PLAIN;
   const OpRecord record("dlblas::ep_gather", t);
   DeviceScope scope(in);
-  if (gather(in, ids, weights, index, out, stream_of(in)) != DLB_OK) NOT_PLAIN;
+  int rc;
+  {
+    const NoGil nogil;
+    rc = gather(in, ids, weights, index, out, stream_of(in));
+  }
+  if (rc != DLB_OK) NOT_PLAIN;
   written(out);
   Py_RETURN_TRUE;
   HANDLE_EXCEPTIONS_END
@@ -466,36 +527,48 @@ PyObject* fused_moe_v3(PyObject*, PyObject* const* args, Py_ssize_t n) {
     NOT_PLAIN;  // three steps on uniform tiles
   const OpRecord record("dlblas::fused_moe_v3", t);
 
-  // one allocation for the int32 tables: expert and token of every row, row ranges and first free rows of the experts
-  at::Tensor tables = empty({2 * rows + 3 * E}, at::kInt, x);
-  int32_t* row_expert = iptr(tables);
-  int32_t *row_token = row_expert + rows, *row_start = row_token + rows, *row_end = row_start + E, *first_free = row_end + E;
-  at::Tensor slot_row = empty(ids.sizes(), ids.scalar_type(), x);
-  at::Tensor q = empty({rows, inter}, at::kFloat8_e4m3fn, x);
-  at::Tensor s = empty({rows, inter / kBlock}, at::kFloat, x);
-  at::Tensor down = empty({rows, H}, at::kBFloat16, x);
-  at::Tensor out = empty({T, H}, at::kBFloat16, x);
-  const int32_t g = static_cast<int32_t>(E), hint = static_cast<int32_t>(rows_each);
-  int rc = abi.scatter_rows(ptr(ids), idx_code(ids.scalar_type()), ids.stride(0), ids.stride(1), counts, row_start, row_end, first_free, row_expert, row_token,
-                            rows, ptr(slot_row), idx_code(slot_row.scalar_type()), topk, 1, T, topk, E, ws.ptr, ws.bytes, stream);
-  if (rc != DLB_OK) NOT_PLAIN;
-  int64_t s_m = inter / kBlock, s_k = 1;
-  if (short_experts) {
-    rc = abi.ragged_act(ptr(x), ptr(w13), fptr(x_s), fptr(w13_s), ptr(q), fptr(s), row_start, row_end, row_token, T, hint, rows, N, H, g, x_s.stride(0),
-                        x_s.stride(1), s_m, s_k, 1e-10f, stream);
-    if (rc == DLB_OK) rc = abi.ragged(ptr(q), ptr(w2), fptr(s), fptr(w2_s), ptr(down), row_start, row_end, hint, rows, H, inter, g, s_m, s_k, DLB_OUT_BF16, stream);
+  at::Tensor out;
+  int rc;
+  bool begun = false;
+  {
+    const NoGil nogil;
+    // one allocation for the int32 tables: expert and token of every row, row ranges and first free rows of the experts
+    at::Tensor tables = empty({2 * rows + 3 * E}, at::kInt, x);
+    int32_t* row_expert = iptr(tables);
+    int32_t *row_token = row_expert + rows, *row_start = row_token + rows, *row_end = row_start + E, *first_free = row_end + E;
+    at::Tensor slot_row = empty(ids.sizes(), ids.scalar_type(), x);
+    at::Tensor q = empty({rows, inter}, at::kFloat8_e4m3fn, x);
+    at::Tensor s = empty({rows, inter / kBlock}, at::kFloat, x);
+    at::Tensor down = empty({rows, H}, at::kBFloat16, x);
+    out = empty({T, H}, at::kBFloat16, x);
+    const int32_t g = static_cast<int32_t>(E), hint = static_cast<int32_t>(rows_each);
+    const Together together(ws);  // the down GEMM reads what the gate/up GEMM leaves in the workspace
+    rc = abi.scatter_rows(ptr(ids), idx_code(ids.scalar_type()), ids.stride(0), ids.stride(1), counts, row_start, row_end, first_free, row_expert, row_token,
+                          rows, ptr(slot_row), idx_code(slot_row.scalar_type()), topk, 1, T, topk, E, ws.ptr, ws.bytes, stream);
+    int64_t s_m = inter / kBlock, s_k = 1;
+    bool lists_now = rc == DLB_OK;
+    if (rc == DLB_OK && short_experts) {
+      rc = abi.ragged_act(ptr(x), ptr(w13), fptr(x_s), fptr(w13_s), ptr(q), fptr(s), row_start, row_end, row_token, T, hint, rows, N, H, g, x_s.stride(0),
+                          x_s.stride(1), s_m, s_k, 1e-10f, stream);
+      if (rc == DLB_OK) rc = abi.ragged(ptr(q), ptr(w2), fptr(s), fptr(w2_s), ptr(down), row_start, row_end, hint, rows, H, inter, g, s_m, s_k, DLB_OUT_BF16, stream);
+      lists_now = rc == DLB_ERR_BAD_SHAPE;
+      begun = !lists_now;
+    }
+    if (lists_now) {
+      s_m = 1, s_k = rows;  // rows of a K block contiguous: what the down GEMM reads in place
+      rc = abi.contiguous_gather_act(ptr(x), ptr(w13), fptr(x_s), fptr(w13_s), ptr(q), fptr(s), row_expert, row_token, T, rows, N, H, g, x_s.stride(0),
+                                     x_s.stride(1), s_m, s_k, 1e-10f, ws.ptr, ws.bytes, stream);
+      begun = rc != DLB_ERR_BAD_SHAPE;  // declined: the Python path starts over with the three steps
+      if (rc == DLB_OK)
+        rc = abi.contiguous_same_rows(ptr(q), ptr(w2), fptr(s), fptr(w2_s), ptr(down), row_expert, rows, H, inter, g, s_m, s_k, DLB_OUT_BF16, ws.ptr,
+                                      ws.bytes, stream);
+    }
+    if (rc == DLB_OK) rc = gather(down, ids, weights, slot_row, out, stream);
   }
-  if (!short_experts || rc == DLB_ERR_BAD_SHAPE) {
-    s_m = 1, s_k = rows;  // rows of a K block contiguous: what the down GEMM reads in place
-    rc = abi.contiguous_gather_act(ptr(x), ptr(w13), fptr(x_s), fptr(w13_s), ptr(q), fptr(s), row_expert, row_token, T, rows, N, H, g, x_s.stride(0),
-                                   x_s.stride(1), s_m, s_k, 1e-10f, ws.ptr, ws.bytes, stream);
-    if (rc == DLB_ERR_BAD_SHAPE) NOT_PLAIN;  // the Python path starts over with the three steps
-    if (rc == DLB_OK)
-      rc = abi.contiguous_same_rows(ptr(q), ptr(w2), fptr(s), fptr(w2_s), ptr(down), row_expert, rows, H, inter, g, s_m, s_k, DLB_OUT_BF16, ws.ptr,
-                                    ws.bytes, stream);
+  if (rc != DLB_OK) {
+    if (begun) return launch_failed(rc);
+    NOT_PLAIN;
   }
-  if (rc == DLB_OK) rc = gather(down, ids, weights, slot_row, out, stream);
-  if (rc != DLB_OK) return launch_failed(rc);
   return THPVariable_Wrap(std::move(out));
   HANDLE_EXCEPTIONS_END
 }

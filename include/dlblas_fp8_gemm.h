@@ -24,7 +24,8 @@
  *     overwrites: re-laid activation scales, fp32 partial sums of the split-K path, the tile
  *     list of the expert-contiguous path; nothing there has to be initialised or to survive
  *     between calls, so one buffer serves any number of calls that do not overlap in time.
- *     Two calls that may run concurrently (different streams) need separate workspaces.
+ *     Two calls that may run concurrently (different streams) need separate workspaces.  Threads may call on one
+ *     stream and workspace at a time: a call holds a lock of its workspace while it enqueues (dlb_workspace_lock).
  *
  * Reference interfaces these replace (paths relative to the DLBlas source tree):
  *   - dlb_fp8_gemm                     : dlblas/kernels/fp8_gemm.py:15-65 (kernel) and :68-89 (host wrapper)
@@ -77,6 +78,14 @@ const char* dlb_last_error(void);
  * length K.  Never fails; returns at least DLB_WS_COUNTER_BYTES.
  */
 size_t dlb_fp8_gemm_workspace_bytes(int64_t rows, int64_t N, int64_t K);
+
+/*
+ * The lock every call that is given `workspace` holds while it enqueues its launches, for callers that need several calls
+ * to stay together (dlb_fp8_gemm_grouped_contiguous_same_rows) while other threads use the workspace.  Recursive; the thread
+ * that locks unlocks.  Workspaces may share a lock, so hold one at a time.  No counterpart in the reference.
+ */
+int dlb_workspace_lock(const void* workspace);
+int dlb_workspace_unlock(const void* workspace);
 
 /*
  * Dense block-scaled GEMM.   Replaces fp8_gemm_kernel / fp8_gemm (dlblas/kernels/fp8_gemm.py:15-89).
@@ -151,8 +160,8 @@ int dlb_fp8_gemm_grouped_contiguous(const void* a, const void* b, const float* a
 
 /*
  * dlb_fp8_gemm_grouped_contiguous right behind a dlb_fp8_gemm_grouped_contiguous_silu_quant or _gather_silu_quant that
- * succeeded, on the same stream and workspace (nothing else used the workspace in between) and with the same m_indices,
- * M_sum and G: the down GEMM of an expert MLP.  It reads the tile lists that call left in the workspace instead of building
+ * succeeded, on the same stream and workspace (nothing else used the workspace in between: where another thread may, hold
+ * dlb_workspace_lock over both calls) and with the same m_indices, M_sum and G: the down GEMM of an expert MLP.  It reads the tile lists that call left in the workspace instead of building
  * them again, one launch of 5 us less.  No counterpart in the reference.
  */
 int dlb_fp8_gemm_grouped_contiguous_same_rows(const void* a, const void* b, const float* a_s, const float* b_s,

@@ -257,3 +257,89 @@ def test_tensors_with_a_tangent_are_left_to_the_python_path(dev):
     with forward_ad.dual_level():
         assert _fast.quant(forward_ad.make_dual(x, torch.ones_like(x)), 128, 1e-10, False) is None
     assert _fast.quant(x, 128, 1e-10, False) is not None
+
+
+def _calls_through_the_workspace(dev):
+    """name -> a call whose launches hand data on in the workspace: K slices, tile lists with re-laid scales, histograms."""
+    from dlblas_amd.kernels.fp8_gemm import fp8_gemm
+    from dlblas_amd.kernels.fp8_gemm_grouped import m_grouped_fp8_gemm_nt_contiguous
+    from dlblas_amd.kernels.fused_moe_v3 import ep_scatter_rows
+    w13, _, codes = _small_experts(dev)
+    args = _operands((200, ), 392, 2048, dev)
+    a, a_s, idx = codes(512, 512), torch.ones(512, 4, device=dev), torch.zeros(512, dtype=torch.int32, device=dev)
+    i32 = lambda n: torch.empty(n, dtype=torch.int32, device=dev)
+    ids = torch.zeros(4000, 8, dtype=torch.int64, device=dev)
+    return {
+        'native dense': lambda: fp8_gemm(*args),
+        'custom op dense': lambda: torch.ops.dlblas.fp8_gemm(*args, torch.bfloat16),
+        'native contiguous': lambda: m_grouped_fp8_gemm_nt_contiguous((a, a_s), w13, torch.empty(512, 1024, dtype=torch.bfloat16, device=dev), idx),
+        'row tables': lambda: ep_scatter_rows(ids, torch.tensor([32000, 0], dtype=torch.int32, device=dev), i32(2), i32(32000), i32(32000),
+                                              torch.empty_like(ids)),
+    }
+
+
+@pytest.mark.parametrize('name', ['native dense', 'custom op dense', 'native contiguous', 'row tables'])
+def test_launches_of_a_call_go_out_under_the_lock_of_its_workspace(dev, name):
+    """Two threads on one stream share its workspace: a call waits while another one's launches are being enqueued."""
+    import ctypes
+
+    from dlblas_amd import _lib
+    lib = _lib.load()
+    call = _calls_through_the_workspace(dev)[name]
+    call()
+    torch.cuda.synchronize()
+    ws = ctypes.c_void_p(_lib.workspace(dev, torch.cuda.current_stream().cuda_stream).data_ptr())
+    done = threading.Event()
+
+    def work():
+        call()
+        done.set()
+
+    assert lib.dlb_workspace_lock(ws) == 0 and lib.dlb_workspace_lock(ws) == 0
+    worker = threading.Thread(target=work)
+    try:
+        call()  # the holder's own calls go on
+        worker.start()
+        assert not done.wait(0.3)
+    finally:
+        lib.dlb_workspace_unlock(ws), lib.dlb_workspace_unlock(ws)
+    assert done.wait(20)
+    worker.join()
+    torch.cuda.synchronize()
+
+
+def test_native_calls_run_without_the_interpreter_lock(dev):
+    """A launch waits while the hardware queue is full; other Python threads go on meanwhile.  PyGILState_Check stands in for
+    the library's launching entry points: it returns 0, which is success to the caller, when the lock is not held."""
+    import ctypes
+
+    from dlblas_amd import _fast, _lib
+    lib = _lib.load()
+    w13, w2, codes = _small_experts(dev)
+    args = _operands((16, ), 128, 256, dev)
+    a3, s3, mm = codes(2, 64, 512), torch.ones(2, 64, 4, device=dev), torch.tensor([3, 0], dtype=torch.int32, device=dev)
+    ids, wts = torch.tensor([[0], [1], [0]], device=dev), torch.ones(3, 1, device=dev)
+    calls = {
+        'fp8_gemm': args, 'quant': (torch.ones(4, 256, device=dev), 128, 1e-10, False),
+        'grouped_contiguous': (codes(128, 512), torch.ones(128, 4, device=dev), *w13, torch.empty(128, 1024, device=dev), torch.zeros(128, dtype=torch.int32, device=dev)),
+        'grouped_masked': (a3, s3, *w13, torch.empty(2, 64, 1024, device=dev), mm, 2),
+        'low_latency_experts': (a3, s3, *w13, *w2, mm, 2),
+        'ep_gather': (torch.ones(4, 512, device=dev), ids, wts, ids, torch.empty(3, 512, device=dev)),
+        'fused_moe_v3': (codes(3, 512), torch.ones(3, 4, device=dev), ids, wts, *w13, *w2, [128, 128]),
+    }
+    assert calls.keys() == set(_fast._FUNCTIONS)
+    for name, a in calls.items():  # with the library itself: nothing declines these
+        assert getattr(_fast, name)(*a) is not None, name
+    torch.cuda.synchronize()
+    init = _fast.fp8_gemm.__self__.init
+    address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+    real = [address(getattr(lib, n)) for n in _fast._ABI]
+    asks = ('dlb_last_error', 'dlb_workspace_lock', 'dlb_workspace_unlock', 'dlb_fp8_gemm_plan_grouped', 'dlb_fp8_gemm_plan_stream',
+            'dlb_fp8_gemm_variant_name', 'dlb_ep_scatter_workspace_bytes')
+    probe = address(ctypes.pythonapi.PyGILState_Check)
+    try:
+        init([r if n in asks else probe for n, r in zip(_fast._ABI, real)], _lib.workspace)
+        without = {name: getattr(_fast, name)(*a) is not None for name, a in calls.items()}
+    finally:
+        init(real, _lib.workspace)
+    assert all(without.values()), without
