@@ -58,11 +58,13 @@ def test_prefill_full_size(dev, M, N, K):
     (16, 36864, 7168, 'skinny16', 1),          # six rounds of decode workgroups
 ])
 def test_planner_choices_full_size(dev, M, N, K, variant, slices):
-    """Shapes whose launch the planner's later rules decide, at their real size: sampled rows against the oracle,
-    exact power-of-two linearity, row permutation."""
+    """Shapes whose variant the planner's later rules decide, at their real size (without the kernel whose waves split K,
+    which takes two of them over): sampled rows against the oracle, exact power-of-two linearity, row permutation."""
     from dlblas_amd import _lib
     print(f'case planner choice full size M={M} N={N} K={K}', flush=True)
     assert _lib.plan(0, M, N, K)[:2] == (variant, slices)
+    _lib.tune('wave_k', 1)
+    assert _lib.plan_wave_k(M, N, K) is None
     a_q, a_s, b_q, b_s = helpers.make_dense_device(M, N, K, dev, seed=M + K)
     out = _gemm(a_q, b_q, a_s, b_s)
     torch.cuda.synchronize()

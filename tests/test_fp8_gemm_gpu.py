@@ -71,17 +71,21 @@ def test_every_variant(dev, variant, M, N, K):
 @pytest.mark.parametrize('M,N,K', [(128, 2112, 7168), (200, 392, 2048), (129, 130, 1040), (70, 131, 4096)])
 def test_split_k_two_pass(dev, M, N, K, variant, splitk, out_dtype):
     """K split over workgroups: fp32 partial matrices in the workspace, a second kernel adds them in index order.
-    (None, 0) is the library's own choice, which splits (128, 2112, 7168).  Two calls must agree bit for bit."""
+    (None, 0) is the library's own choice among the kernels that split K over workgroups.  Two
+    calls must agree bit for bit."""
     from dlblas_amd import _lib
     print(f'case split-K variant={variant} splitk={splitk} M={M} N={N} K={K} {out_dtype}', flush=True)
     a_q, a_s, b_q, b_s = helpers.make_dense(M, N, K, seed=11)
     ref = orc.dequant_ref(a_q, a_s, b_q, b_s)
     try:
         _lib.force_splitk(splitk)
+        _lib.tune('wave_k', 1 if variant is None else 0)
+        assert variant is not None or _lib.plan(0, M, N, K)[1] > 1
         out = _run_dense(dev, a_q, a_s, b_q, b_s, dtype=out_dtype, variant=variant)
         again = _run_dense(dev, a_q, a_s, b_q, b_s, dtype=out_dtype, variant=variant)
     finally:
         _lib.force_splitk(0)
+        _lib.tune('wave_k', 0)
     assert out.dtype == out_dtype
     helpers.tolerance_check(out, ref, f'split-K {variant}/{splitk} {M}x{N}x{K}')
     assert torch.equal(out, again)
@@ -196,10 +200,12 @@ def test_decode_column_split(dev, M, N, K, bn, out_dtype):
     a_q, a_s, b_q, b_s = helpers.make_dense(M, N, K, seed=31)
     ref = orc.dequant_ref(a_q, a_s, b_q, b_s)
     _lib.tune('skinny_bn', bn)
+    _lib.tune('wave_k', 1)  # 40 and 100 rows
     try:
         out = _run_dense(dev, a_q, a_s, b_q, b_s, dtype=out_dtype)
     finally:
         _lib.tune('skinny_bn', 0)
+        _lib.tune('wave_k', 0)
     assert out.dtype == out_dtype and tuple(out.shape) == (M, N)
     helpers.tolerance_check(out, ref, f'decode bn={bn} {M}x{N}x{K}')
 
@@ -534,6 +540,7 @@ def test_grouped_masked_scale_table(dev, K):
     a_q = a_bits.view(torch.float8_e4m3fn)
     sentinel = -555.0
     ref = orc.grouped_masked_ref(a_q, a_s, w_q, w_s, torch.full((G, M_max, N), sentinel), masked_m)
+    _lib.tune('stream', 1)  # the ring kernels
     outs = []
     for knob in (0, 2):
         out = torch.full((G, M_max, N), sentinel, dtype=torch.bfloat16, device=dev)
@@ -544,6 +551,7 @@ def test_grouped_masked_scale_table(dev, K):
         finally:
             _lib.tune('scale_table', 0)
         outs.append(out)
+    _lib.tune('stream', 0)
     for e in range(G):
         assert torch.all(outs[0][e, int(masked_m[e]):] == sentinel)
     helpers.tolerance_check(outs[0], ref, f'masked scale table K={K}')

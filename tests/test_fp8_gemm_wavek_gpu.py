@@ -65,7 +65,7 @@ def test_every_shape_matches_the_oracle(dev, M, N, K, out_dtype):
 
 @pytest.mark.parametrize('M,N,K', [(100, 2112, 7168), (300, 1000, 1040), (500, 4096, 7168)])
 def test_library_choice_full_size(dev, M, N, K):
-    """Sizes the library gives to this kernel, sampled rows against the oracle; a row's result does not depend on M."""
+    """Sizes the library gives to this kernel: sampled rows against the oracle; two calls agree bit for bit."""
     from dlblas_amd import _lib
     from dlblas_amd.kernels.fp8_gemm import fp8_gemm
     print(f'case wave_k choice {M}x{N}x{K}', flush=True)

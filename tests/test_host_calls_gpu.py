@@ -103,20 +103,28 @@ def test_other_calls_are_left_to_the_python_path(dev):
 
 
 def test_streams_and_threads_share_the_workspaces_of_the_python_path(dev):
-    from dlblas_amd import _lib
+    """Partial sums of K slices lie in the workspace of (device, stream): threads on streams of their own, with operands of
+    their own, would see each other's if two streams shared one."""
+    from dlblas_amd import _fast, _lib
     from dlblas_amd.kernels.fp8_gemm import fp8_gemm
-    args = _operands((200, ), 392, 2048, dev)  # K slices in the workspace
-    ref = fp8_gemm(*args)
+    M, N, K = 200, 392, 2048
+    operands = [_operands((M, ), N, K, dev, seed=5 + i) for i in range(3)]
+    _lib.tune('wave_k', 1)
+    assert _lib.plan_wave_k(M, N, K) is None and _lib.plan(0, M, N, K)[1] > 1
+    refs = [fp8_gemm(*args) for args in operands]
     torch.cuda.synchronize()
+    assert not torch.equal(refs[0], refs[1])
     results, failed = {}, []
 
     def work(i):
         try:
+            _lib.tune('wave_k', 1)  # knobs are the thread's own
             stream = torch.cuda.Stream()
             with torch.cuda.stream(stream):
-                outs = [fp8_gemm(*args) for _ in range(20)]
+                assert _fast.fp8_gemm(*operands[i]) is not None
+                outs = [fp8_gemm(*operands[i]) for _ in range(40)]
             stream.synchronize()
-            results[i] = all(torch.equal(o, ref) for o in outs)
+            results[i] = all(torch.equal(o, refs[i]) for o in outs)
             assert (dev.index or 0, stream.cuda_stream) in _lib._workspaces
         except Exception as exc:  # reported by the test's own thread
             failed.append(exc)
@@ -343,3 +351,29 @@ def test_native_calls_run_without_the_interpreter_lock(dev):
     finally:
         init(real, _lib.workspace)
     assert all(without.values()), without
+
+
+def test_threads_on_one_stream_keep_their_launches_together(dev):
+    """Threads that share a stream share its workspace: every call's partial sums are still its own."""
+    from dlblas_amd import _lib
+    from dlblas_amd.kernels.fp8_gemm import fp8_gemm
+    M, N, K = 200, 392, 2048
+    operands = [_operands((M, ), N, K, dev, seed=5 + i) for i in range(3)]
+    _lib.tune('wave_k', 1)
+    refs = [fp8_gemm(*args) for args in operands]
+    torch.cuda.synchronize()
+    results = {}
+
+    def work(i):
+        _lib.tune('wave_k', 1)
+        call = (lambda: fp8_gemm(*operands[i])) if i else (lambda: torch.ops.dlblas.fp8_gemm(*operands[i], torch.get_default_dtype()))
+        outs = [call() for _ in range(100)]
+        torch.cuda.synchronize()
+        results[i] = all(torch.equal(o, refs[i]) for o in outs)
+
+    threads = [threading.Thread(target=work, args=(i, )) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(results) == 3 and all(results.values())
