@@ -396,26 +396,22 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
     if (d < p.m_len) p.src_row[d] = static_cast<int32_t>(t);
   }
   // One past the last row that holds a slot of the experts up to e.  Where more slots are routed to an expert than it has
-  // rows, they run on into the spans behind its own, as in ep_scatter, and those rows are not empty.
+  // rows, they run on into the spans behind its own, as in ep_scatter, and those rows are not empty.  Every wave looks for
+  // such an expert itself: with a vote of the block and 64-bit row numbers in the main loop the kernel took 0.4 .. 1.0 us longer.
   int over = 0;
-  for (int e = tid; e < E; e += kRowsThreads) over |= routed[e] > excl[e + 1] - excl[e];
-  over = __syncthreads_or(over);
+  for (int e = lane; e < E; e += 64) over |= routed[e] > excl[e + 1] - excl[e];
+  over = __any(over);
   auto end_of = [&](int e) {
     int end = excl[e] + routed[e];
     if (over)
       for (int i = 0; i < e; ++i) end = max(end, excl[i] + routed[i]);
     return end;
   };
-  // the rows in slices over the blocks: their expert below excl[E], and token 0 for every row that no slot is given.  That
-  // includes the rows of a longer table past the spans: readers of src_row follow every entry, whatever m_indices says
+  // rows [0, excl[E]) in slices over the blocks: their expert, and token 0 for the rows that no slot is given
   const int total = static_cast<int>(min(static_cast<int64_t>(excl[E]), p.m_len));
-  const int64_t per = (p.m_len + gridDim.x - 1) / gridDim.x;
-  const int64_t r1 = min(p.m_len, (b + 1) * per);
-  for (int64_t r = b * per + tid; r < r1; r += kRowsThreads) {
-    if (r >= total) {
-      if (r >= end_of(E - 1)) p.src_row[r] = 0;
-      continue;
-    }
+  const int per = (total + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x);
+  const int r1 = min(total, (b + 1) * per);
+  for (int r = b * per + tid; r < r1; r += kRowsThreads) {
     int lo = 0, hi = E;  // largest e with excl[e] <= r
     while (hi - lo > 1) {
       const int mid = (lo + hi) >> 1;
@@ -426,6 +422,12 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
     }
     p.m_indices[r] = lo;
     if (r >= end_of(lo)) p.src_row[r] = 0;
+  }
+  // rows of a longer table past the spans: readers of src_row follow every entry, whatever m_indices says
+  if (p.m_len > total) {
+    const int last = end_of(E - 1);
+    for (int64_t r = total + static_cast<int64_t>(b) * kRowsThreads + tid; r < p.m_len; r += static_cast<int64_t>(gridDim.x) * kRowsThreads)
+      if (r >= last) p.src_row[r] = 0;
   }
   if (b == 0)
     for (int e = tid; e < E; e += kRowsThreads) {
