@@ -735,6 +735,73 @@ PLANNER_SWEEP_WEIGHTS = [(2112, 7168), (24576, 1536), (32768, 512), (7168, 16384
                          (7168, 18432), (36864, 7168), (576, 7168), (4608, 7168), (7168, 2304), (18432, 7168)]
 
 
+def wave_k_random(dev, count=1500, seconds=240):
+    """Random dense problems (512 .. 36864 weight rows, K = 512 .. 18432, a quarter of them ragged) on the kernel whose waves split K
+    and on the others: its time over theirs by class, with three weight matrices in turn (up to 80 MB each the Infinity cache
+    holds them) and with 700 MB of weights in turn (from HBM).  The tile shape is the one the estimate picks."""
+    import math
+    import random
+
+    import torch
+
+    from dlblas_amd import _lib
+    rng, t_end = random.Random(20), time.perf_counter() + seconds
+    pick = lambda lo, hi, step=1: max(lo, min(hi, int(round(math.exp(rng.uniform(math.log(lo), math.log(hi))) / step)) * step))
+    pool = torch.randint(0, 0x60, (700_000_000, ), dtype=torch.uint8, device=dev)  # finite e4m3 codes
+    scales = torch.rand(1 << 17, device=dev)
+    classes = [(f'up to 16 rows, from 24576 columns, {a} .. {b} K blocks', lambda M, N, kb, ragged, mb, a=a, b=b: M <= 16 and not ragged and N >= 24576 and a <= kb <= b)
+               for a, b in ((4, 7), (8, 11), (12, 16), (17, 32), (33, 144))]
+    for lo, hi in ((17, 32), (33, 64)):
+        classes += [(f'{lo} .. {hi} rows, up to 80 MB, K = {a} .. {b}',
+                     lambda M, N, kb, ragged, mb, lo=lo, hi=hi, a=a, b=b: lo <= M <= hi and not ragged and mb <= 80 and a <= kb * 128 <= b)
+                    for a, b in ((512, 2047), (2048, 4095), (4096, 18432), (512, 18432))]
+        classes += [(f'{lo} .. {hi} rows, above 80 MB', lambda M, N, kb, ragged, mb, lo=lo, hi=hi: lo <= M <= hi and not ragged and mb > 80)]
+    classes += [('more rows, up to 80 MB, where the library chooses it', lambda M, N, kb, ragged, mb: M > 64 and not ragged and mb <= 80),
+                ('more rows, above 80 MB', lambda M, N, kb, ragged, mb: M > 64 and not ragged and mb > 80)]
+    classes += [(f'ragged K, {name}', f) for name, f in (('up to 16 rows, up to 80 MB', lambda M, N, kb, ragged, mb: M <= 16 and ragged and mb <= 80),
+                                                         ('up to 16 rows, above 80 MB', lambda M, N, kb, ragged, mb: M <= 16 and ragged and mb > 80),
+                                                         ('17 .. 64 rows', lambda M, N, kb, ragged, mb: 17 <= M <= 64 and ragged),
+                                                         ('more rows', lambda M, N, kb, ragged, mb: M > 64 and ragged))]
+    ratios = {name: ([], []) for name, _ in classes}
+    shapes = ((32, 32, 8), (32, 32, 4), (64, 32, 8), (32, 64, 4), (64, 32, 4), (64, 64, 4), (64, 64, 2))
+    done = 0
+    while done < count and time.perf_counter() < t_end:
+        ragged, wide = rng.random() < 0.25, rng.random() < 0.15
+        M, N, K = pick(1, 16) if wide or ragged and rng.random() < 0.5 else pick(17, 1500), pick(24576 if wide else 512, 36864, rng.choice([8, 64, 128, 512])), \
+            pick(512, 18432, 16 if ragged and not wide else 128)
+        kb, nb, ragged = -(-K // 128), -(-N // 128), K % 128 != 0
+        if N * K > 36864 * 7168 or M * N * K > 1500 * 7168 * 7168:
+            continue
+        hit = [name for name, f in classes if f(M, N, kb, ragged, N * K / 1e6)]
+        _lib.tune('wave_k', 0)
+        tile = _lib.plan_wave_k(M, N, K)
+        if not hit or 'where the library chooses it' in hit[0] and tile is None:
+            continue
+        done += 1
+        step = -(-N * K // 256) * 256
+        a_q, a_s = pool[:M * K].clone().view(M, K).view(torch.float8_e4m3fn), torch.rand(M, kb, device=dev)
+        ws = [(pool[i * step:i * step + N * K].view(N, K).view(torch.float8_e4m3fn), scales[:nb * kb].view(nb, kb)) for i in range(min(3000, 700_000_000 // step))]
+        out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+        reps = int(max(10, min(120, 2e-2 / max(2.0 * M * N * K / 2e15, 5e-6))))
+        for where, copies in enumerate((ws[:3], ws)):
+            launch = DenseLauncher(a_q, a_s, copies, out)
+            # the library's tile, or (where it leaves the problem to the other kernels) the best of the two it would take there
+            knobs = [2 + shapes.index(tile)] if tile else [2, 3, 5] if M <= 16 else [7, 8]
+            t = []
+            for knob in [1] + knobs:
+                _lib.tune('wave_k', knob)
+                time_call(launch, reps, reps)
+                t.append(min(time_call(launch, reps, 3) for _ in range(2)))
+            for name in hit:
+                ratios[name][where].append(min(t[1:]) / t[0])
+        _lib.tune('wave_k', 0)
+        del a_q, a_s, ws, out, launch
+    gm = lambda v: math.exp(sum(map(math.log, v)) / len(v)) if v else float('nan')
+    print(f'{done} problems; time of the wave-split kernel over the other kernels\': problems, three matrices in turn, from HBM')
+    for name, (cache, hbm) in ratios.items():
+        print(f'{name}: {len(hbm)}, {gm(cache):.2f}, {gm(hbm):.2f}', flush=True)
+
+
 def planner_sweep(dev, which):
     """The planner's launch against every alternative forced in turn; prints one line per problem and returns the rows.
     'dense': kernel variants (no K split forced) over 13 weight shapes x 15 row counts; 'mid': the three small ring
@@ -983,7 +1050,7 @@ def main():
     ap.add_argument('--grouped-only', action='store_true',
                     help='run only the two grouped MoE workloads and print their rows (the command the rocprofv3 summaries of '
                     'the grouped kernels are made with)')
-    ap.add_argument('--planner-sweep', choices=['dense', 'mid', 'decode', 'grouped', 'wave_k', 'stream'], default=None,
+    ap.add_argument('--planner-sweep', choices=['dense', 'mid', 'decode', 'grouped', 'wave_k', 'stream', 'wave_k_random'], default=None,
                     help="time the planner's launch against every alternative forced in turn over a grid of problems and "
                     'print where it is not the fastest (a minute or two)')
     args = ap.parse_args()
@@ -1003,6 +1070,10 @@ def main():
 
     if args.decode_floor:
         print(json.dumps({'decode_floor': decode_floor(dev)}), flush=True)
+        return
+
+    if args.planner_sweep == 'wave_k_random':
+        wave_k_random(dev)
         return
 
     if args.planner_sweep:

@@ -713,20 +713,20 @@ int wavek_lds(const WaveKDims& d, int pitch) {
 //     the larger of its bytes at 86 GB/s (the DMA path of a CU) and the trip of one block (0.21 us + 3.8 ns per operand row)
 //     shared by the waves that are resident at once;
 //   - every tile's operands from the L2s at 17 TB/s;  - the matrices from HBM at 6 TB/s.
-// The estimate chooses the shape (2 - 3 % behind the best one, geometric mean over 1500 problems; its rms error is 15 - 29 %,
-// mostly too low where the weights come from HBM).  Whether the kernel runs at all depends on where the operands come from:
-// from the caches (three weight matrices of up to 80 MB in turn stay in the 256 MB Infinity cache) it is ahead of the others,
-// from HBM it may be behind.  Its time over theirs, cache / HBM, geometric means over random problems of 512 .. 36864 weight
-// rows and K = 512 .. 18432 (bench.py --planner-sweep wave_k has the fixed ones):
+// The estimate chooses the shape (2 - 3 % behind the best one, geometric mean; its rms error is 15 - 29 %, mostly too low where
+// the weights come from HBM).  Whether the kernel runs at all depends on where the operands come from: from the caches (three
+// weight matrices of up to 80 MB in turn stay in the 256 MB Infinity cache) it is ahead of the others, from HBM it may be
+// behind.  Its time over theirs, caches / HBM, geometric means (bench.py --planner-sweep wave_k_random, 1500 problems of 512 ..
+// 36864 weight rows and K = 512 .. 18432; the examples are from --planner-sweep wave_k, from HBM):
 //   - up to 16 rows the decode kernels' 16-row fragments waste less (16 x 7168 x 2048 5.2 against 5.4 us), but very many columns
-//     take them several rounds, whose waves idle while K is short.  From 24576 columns on 0.95 / 1.04 at up to 7 K blocks, 0.87 /
-//     1.05 at 8 .. 11, 0.97 / 1.15 at 12 .. 16, 1.08 / 1.19 and 1.17 / 1.15 above (16 x 36864 x 7168 50.3 against 46.9 us): up to 11;
-//   - 17 .. 64 rows: always.  17 .. 32 rows 0.84 / 1.08 at up to 80 MB (K < 2048 0.90 / 1.00, < 4096 0.86 / 1.07, longer 0.77 / 1.15:
-//     32 x 2112 x 7168 11.5 against 9.6 us from HBM), 1.00 / 1.03 above; 33 .. 64 rows 0.75 / 0.91 and 1.04 / 1.00;
-//   - more rows: where the estimates say so, at up to 80 MB (0.69 / 0.84 there; 100 x 2112 x 7168 14.5 -> 12.8 us, 300 x 4096 x 4096
-//     20 -> 18 us); larger matrices come from HBM, 1.11 where the estimates would choose it (128 x 7168 x 18432 49.8 against 40.3 us);
-//   - a ragged K, for which only the register-staged kernels remain: always.  Up to 16 rows 0.80 / 1.01 at up to 80 MB and 0.68 /
-//     0.71 above, 17 .. 64 rows 0.70 from HBM, more rows 0.67 (300 x 1000 x 1040 11.2 -> 4.6 us, 4096 x 24576 x 1040 372 -> 237 us).
+//     take them several rounds, whose waves idle while K is short.  From 24576 columns on 0.95 / 1.04 at up to 7 K blocks, 0.91 /
+//     1.04 at 8 .. 11, 0.93 / 1.09 at 12 .. 16, 1.02 / 1.15 and 1.14 / 1.15 above (16 x 36864 x 7168 50.3 against 46.9 us): up to 11;
+//   - 17 .. 64 rows: always.  17 .. 32 rows 0.87 / 1.06 at up to 80 MB (K < 2048 0.92 / 1.01, < 4096 0.85 / 1.10, longer 0.77 / 1.13:
+//     32 x 2112 x 7168 11.5 against 9.6 us), 1.01 / 1.04 above; 33 .. 64 rows 0.76 / 0.92 and 0.97 / 1.02;
+//   - more rows: at up to 80 MB where the estimates say so (0.70 / 0.80 there; 100 x 2112 x 7168 14.5 -> 13.4 us, 300 x 4096 x 4096
+//     20 -> 18 us); larger matrices 1.22 / 1.25, and the estimates do not see it (128 x 7168 x 18432 49.8 against 40.3 us): never;
+//   - a ragged K, for which only the register-staged kernels remain: always.  Up to 16 rows 0.78 / 1.00 at up to 80 MB and 0.70 /
+//     0.74 above, 17 .. 64 rows 0.61 / 0.78, more 0.59 / 0.65 (300 x 1000 x 1040 10.9 -> 4.9 us, 4096 x 24576 x 1040 372 -> 240 us).
 int pick_wavek(int64_t M, int64_t N, int64_t K, int cus, size_t ws_bytes) {
   const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
   const int knob = g_knob[kKnobWaveK];
@@ -783,6 +783,9 @@ constexpr int kStreamActSpan = 192;  // the longest experts the weight-streaming
 // expert (twice the caller's hint covers nearly all of them).  A tile's step lasts what is longer of the trip its loads
 // take with the chip to themselves, 0.25 us + 1.9 ns per row of the two operands (a lone CU fetches 40 - 50 GB/s), and its
 // share of the HBM stream (6.9 TB/s over the busy CUs); tiles of 64 or 128 weight rows win while those of 256 leave CUs idle.
+// (bench.py --planner-sweep stream: 1.20 x / 1.18 x the ring kernels, plain / quantising, 3 % behind the best shape, geometric
+// means.  A few experts whose 128 x 128 ring tiles just fill one round are the exception: 8 experts x 0 .. 128 rows x 4096 x 7168
+// 75 against 54 us; at 65 .. 128 rows such problems are even on average.)
 int pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, int cus, int* chunk_len, bool* ahead) {
   const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
   const int knob = g_knob[kKnobStream];
@@ -803,8 +806,7 @@ int pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool 
     const double mtiles = span <= d.bm ? 1.0 : 0.5 * (span / d.bm + 1.0);
     const double tiles = static_cast<double>(G) * mtiles * static_cast<double>(act ? N / 256 : ceil_div(N, d.bn));
     const double rows = std::min(0.5 * span, static_cast<double>(d.bm));
-    // the row tiles of long experts run in step and share the weights in the L2 (30 problems of 8 .. 32 experts, 200 .. 448
-    // rows: this choice against the ring kernels 1.19 x, geometric mean; 0.96 the worst)
+    // the row tiles of long experts run in step and share the weights in the L2
     const double sharing = span > 192 ? mtiles : 1.0;
     auto step = [&](double busy) { return std::max(0.25 + 0.0019 * (d.bn + rows), d.bn * 128.0 * busy / sharing / 6.9e6); };
     const double full = std::floor(tiles / cus), rest = tiles - full * cus;

@@ -13,8 +13,9 @@
 //
 // Measured (MI355X, 32 experts, against the 128 x 256 ring kernel it replaces there): gate/up + activation 4096 x 7168,
 // ~16 / ~32 rows per expert 186 -> 143 / 161 -> 148 us, down 7168 x 2048 97 -> 83 / 101 -> 91 us; 940 MB of weights at 4 rows
-// 138 us = 6.8 TB/s, i.e. 12 us + bytes at 7.5 TB/s.  Over 90 problems of 8 .. 32 experts, 512 .. 7168 weight rows and K, up
-// to 192 rows per expert: 1.26 x (geometric mean; the largest gains where 256-column tiles left CUs idle).  With AHEAD (below)
+// 138 us = 6.8 TB/s, i.e. 12 us + bytes at 7.5 TB/s.  Where the library chooses it 1.20 x for the plain product, 1.18 x with the
+// quantising epilogue (bench.py --planner-sweep stream, 70 of 96 problems of 8 .. 32 experts, up to 512 rows per expert, geometric
+// means; the largest gains where 256-column tiles left CUs idle).  With AHEAD (below)
 // 0 .. 256 rows: 7168 x 2048 141 -> 128 us with cold operands, 8 experts x 4096 x 7168 88 -> 68, 16 x 1024 x 2048 (0 .. 448
 // rows) 37 -> 25.  Its 128 x 256 step without any load takes 0.85 us, half of that the 128 KB of fragment reads.  The longest
 // experts stay with the ring kernels, whose 256-row tiles read less LDS per product.

@@ -9,10 +9,12 @@
 // others' matrix instructions.  A wave issues the DMA of its next block as soon as the fragments of the current one are in
 // registers.  The partial tiles meet in LDS at the end, added in wave order.
 //
-// Measured (MI355X, kernel time, against the ring or register-staged kernel it replaces): 300 x 1000 x 1040 11.4 -> 4.7 us
-// (there in two launches), 100 x 2112 x 7168 13.4 -> 10.2 us (two launches), 64 x 2112 x 7168 12.7 -> 7.9 us, 256 x 7168 x 2048
-// 12.8 -> 10.4 us, 500 x 4096 x 7168 33 -> 26 us; 110 random problems of 1 .. 1500 rows 1.23 x (geometric mean, the library's
-// choice).  The bound is the DMA path of a CU (64 x 64 tiles: 16 KB per K block at 86 - 110 GB/s), and from about 10^10
+// Measured (MI355X, us per launch with weights from HBM, against the ring or register-staged kernel it replaces; bench.py
+// --planner-sweep wave_k): 300 x 1000 x 1040 10.9 -> 4.9 us (there in two launches), 100 x 2112 x 7168 14.5 -> 13.4 us (two
+// launches), 64 x 2112 x 7168 12.9 -> 11.1 us, 300 x 4096 x 4096 20.2 -> 18.2 us, 500 x 4096 x 7168 32 -> 30 us (25.7 us with
+// three sets of operands in turn, which the Infinity cache holds), 4096 x 24576 x 1040 372 -> 240 us; where the library chooses
+// it, 1.10 x at 33 .. 64 rows, 1.16 x above, 1.5 x for a ragged K (geometric means; 17 .. 32 rows 0.99 x, from the caches 1.2 x).
+// The bound is the DMA path of a CU (64 x 64 tiles: 16 KB per K block at 86 - 110 GB/s), and from about 10^10
 // multiply-adds on the L2s (a 64 x 64 tile asks for 4 bytes per 128 of them), where the larger tiles of the ring kernels win.
 // Small workgroups, so that two or more share a CU: 500 x 4096 x 7168 as 64 x 64 tiles takes 31 us with 8 waves, 26.6 with 4.
 //

@@ -235,7 +235,8 @@ int dlb_fp8_gemm_grouped_contiguous_gather_silu_quant(const void* a, const void*
  *                                             to [0, M_max].
  *   expected_m                                scheduling hint only (typical masked_m); <= 0 = unknown.
  *                                             It picks kernel and tile shape (the weight-streaming kernel while
- *                                             twice the hint, or M_max, is at most 192 rows; 256-row tiles from
+ *                                             twice the hint, or M_max, is at most 256 rows, 448 for K <= 3072, 192
+ *                                             for the form with the quantising epilogue; 256-row tiles from
  *                                             several hundred rows per expert on) and never changes a result bit.
  *
  * The tile schedule is built on the device from masked_m: no host synchronisation and no tiles
@@ -421,7 +422,8 @@ int dlb_fp8_gemm_force_variant(int variant);
  *                           whenever a workspace allows it, 2 = uniform 128-row tiles (default: lists from more than two
  *                           rounds of 128 x 256 tiles on)
  *   DLB_KNOB_STREAM         masked layout: 1 = never the weight-streaming kernel, 2 .. 6 = its tile shape 0 .. 4 (32 x 256,
- *                           64 x 256, 64 x 128, 128 x 256, 64 x 64) wherever it applies (default: by size)
+ *                           64 x 256, 64 x 128, 128 x 256, 64 x 64) wherever it applies, 7 .. 11 = the same with fragments
+ *                           read one step ahead where that form exists (plain product, not 32 x 256) (default: by size)
  *   DLB_KNOB_WAVE_K         dense: 1 = never the kernel whose waves split K, 2 .. 8 = its tile shape 0 .. 6 (32 x 32 with 8 / 4
  *                           waves, 64 x 32 with 8, 32 x 64 with 4, 64 x 32 with 4, 64 x 64 with 4 / 2) wherever it applies
  *   DLB_KNOB_LDS_OVERSIZE   test hook: 1 = every kernel asks for more LDS than the GPU has, so the call is refused
