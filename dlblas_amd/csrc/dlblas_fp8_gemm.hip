@@ -95,7 +95,7 @@ enum Knob : int {
   kKnobSkinnyNFrags,
   kKnobGroupM,
   kKnobSkinnyDma,  // 0 / 1: DMA-staged decode kernel where possible, 2: register-load decode kernel
-  kKnobEpilogue,   // 0 / 1: bf16 output of the pipelined kernels goes through LDS where it can, 2: straight from registers
+  kKnobEpilogue,   // 0 / 1: output of the pipelined kernels goes through LDS, 2: straight from registers
   kKnobSkinnyBn,   // columns per workgroup of the DMA-staged decode kernels (0 = heuristic)
   kKnobSplitKMode, // 1: K slices of the ring kernels are added inside the launch where that applies; 0 / 2: by a second launch (faster on MI355X)
   kKnobSpinLimit,  // one-launch split-K: value - 1 polls for the other slices of a tile (0 = default; 1 = none: the last arrival adds every share)
@@ -1040,8 +1040,6 @@ int run_ragged(const RaggedProblem& pr) {
   ar.act_eps = pr.eps;
   ar.act_cols = static_cast<int>(pr.N / 2);
   ar.act_q_stride = pr.N / 2;
-  ar.vec_store = (pr.N % 4 == 0) && !misaligned(pr.c, 4 * (ar.out_f32 ? 4 : 2));
-  ar.c_vec16 = !ar.out_f32 && pr.N % 8 == 0 && !misaligned(pr.c, 16);
   const int64_t worst = static_cast<int64_t>(ar.tiles_n) * (pr.G + pr.M_sum / kStreamDims[shape].bm);
   const int grid = static_cast<int>(ceil_div(worst < cus ? worst : cus, 32) * 32);
   hipError_t e;
@@ -1172,8 +1170,7 @@ int run(const Problem& pr) {
   ar.act_eps = pr.act_eps;
   ar.act_cols = static_cast<int>(pr.N / 2);
   ar.act_q_stride = pr.N / 2;
-  ar.vec_store = (pr.N % 4 == 0) && !misaligned(pr.c, 4 * (ar.out_f32 ? 4 : 2));
-  ar.c_vec16 = !ar.out_f32 && pr.N % 8 == 0 && !misaligned(pr.c, 16) && g_knob[kKnobEpilogue] != 2;
+  ar.c_lds = g_knob[kKnobEpilogue] != 2;
   if (pr.ws && pr.ws_bytes >= DLB_WS_COUNTER_BYTES) {
     ar.ctr = static_cast<uint32_t*>(pr.ws);
     ar.ws = reinterpret_cast<float*>(static_cast<char*>(pr.ws) + DLB_WS_COUNTER_BYTES);
@@ -1185,7 +1182,6 @@ int run(const Problem& pr) {
   ar.sct_pitch = rs.sct_pitch;
   ar.chunk_len = rs.chunk_len;
   const bool tile_list = rs.tile_list;
-  const size_t esz = ar.out_f32 ? 4 : 2;
 
   // The main kernel of the call.  With g_prepare_only set it only raises the kernel's dynamic-LDS limit (the one
   // step of a launch that can still fail), so that run() can do that before it enqueues the first pre-pass.
@@ -1333,9 +1329,8 @@ int run(const Problem& pr) {
   if (e != hipSuccess) return fail(DLB_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
   if (ar.splitk > 1 && !rs.fused && pr.mode == kDense && pl.variant != kVarExact && !is_skinny(pl.variant)) {
     const int64_t total = pr.rows * pr.N;
-    const int vec_ok = total % 4 == 0 && !misaligned(pr.c, 4 * esz);
     hipLaunchKernelGGL(fp8_splitk_reduce_kernel, dim3(static_cast<unsigned>(ceil_div(ceil_div(total, 4), 256))), dim3(256), 0,
-                       pr.stream, ar.ws, pr.c, total, ar.splitk, ar.out_f32, vec_ok);
+                       pr.stream, ar.ws, pr.c, total, ar.splitk, ar.out_f32);
     e = hipGetLastError();
     if (e != hipSuccess) return fail(DLB_ERR_LAUNCH, "split-K reduction launch failed: %s", hipGetErrorString(e));
   }

@@ -58,8 +58,7 @@ struct Args {
   int sct_pitch;        // kernels with a scale table in LDS: floats per table row (odd, >= K blocks per workgroup)
   int group_m;          // m-tiles per L2 swizzle group
   int out_f32;
-  int vec_store;        // rows of c are aligned for 4-element vector stores
-  int c_vec16;          // bf16 c whose rows are 16-byte aligned (N % 8 == 0): the LDS-transposed epilogue applies
+  int c_lds;            // ring kernels: results leave through LDS, whole rows per store instruction (else straight from the registers)
   int n_split;          // mixed-width launch: first column of the narrow-tile region
   int tiles_a;          //   tiles in the wide region (tiles_m x tiles_n_a)
   int tiles_n_a;
@@ -124,30 +123,46 @@ __device__ __forceinline__ float e4m3_to_f32(uint8_t v) {
   return __uint_as_float(sign | ((e + 120u) << 23) | (m << 20));
 }
 
+// Vector stores of output elements at their own alignment: rows of a C with an odd N start anywhere, and global memory takes
+// a 4-, 8- or 16-byte store at any element boundary.
+typedef v4f v4f_el __attribute__((aligned(4)));
+typedef v4bf v4bf_el __attribute__((aligned(2)));
+typedef v4i v4i_el __attribute__((aligned(2)));
+
 // Store up to four consecutive output elements c[0..3] of one row; `n_left` = elements left in the row.
 template <bool F32>
-__device__ __forceinline__ void store_row4(void* c_row, int64_t col, v4f v, int n_left, bool vec_ok) {
+__device__ __forceinline__ void store_row4(void* c_row, int64_t col, v4f v, int n_left) {
   if (n_left <= 0) return;
   if (F32) {
     float* dst = static_cast<float*>(c_row) + col;
-    if (vec_ok && n_left >= 4) {
-      *reinterpret_cast<v4f*>(dst) = v;
+    if (n_left >= 4) {
+      *reinterpret_cast<v4f_el*>(dst) = v;
     } else {
       dst[0] = v.x;
       if (n_left > 1) dst[1] = v.y;
       if (n_left > 2) dst[2] = v.z;
-      if (n_left > 3) dst[3] = v.w;
     }
   } else {
     __bf16* dst = static_cast<__bf16*>(c_row) + col;
     const v4bf h = __builtin_convertvector(v, v4bf);  // round-to-nearest-even
-    if (vec_ok && n_left >= 4) {
-      *reinterpret_cast<v4bf*>(dst) = h;
+    if (n_left >= 4) {
+      *reinterpret_cast<v4bf_el*>(dst) = h;
     } else {
       dst[0] = h.x;
       if (n_left > 1) dst[1] = h.y;
       if (n_left > 2) dst[2] = h.z;
-      if (n_left > 3) dst[3] = h.w;
+    }
+  }
+}
+
+// Eight consecutive bf16 elements of one row, in four registers; `n_left` (at least 1) = elements left in the row.
+__device__ __forceinline__ void store_row8_bf16(__bf16* dst, v4i v, int n_left) {
+  if (n_left >= 8) {
+    *reinterpret_cast<v4i_el*>(dst) = v;
+  } else {
+    for (int i = 0; i < n_left; ++i) {
+      const uint32_t pair = static_cast<uint32_t>(i < 4 ? (i < 2 ? v.x : v.y) : (i < 6 ? v.z : v.w));
+      dst[i] = __builtin_bit_cast(__bf16, static_cast<uint16_t>(i & 1 ? pair >> 16 : pair & 0xffffu));
     }
   }
 }

@@ -723,6 +723,11 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
     }
 
     // epilogue: lane holds c[m0 + wm0 + 32 mi + (lane & 31)][n0 + wn0 + 32 ni + 8 u + 4 (lane >> 5) + 0..3], u = 0..3
+    // (the lane index passes through an empty asm: what is computed from it then stays behind the K loop instead of
+    // taking registers across it: the 256-row kernels spilled 19 to 49 of them)
+    int el = lane;
+    asm volatile("" : "+v"(el));
+    const int el32 = el & 31, eh = el >> 5;
     if constexpr (kAct) {
       // The tile goes to LDS as the bf16 matrix the unfused GEMM would have written ([BM][gate 128 | up 128], 8-byte
       // chunks XOR-ed with an even function of the row so that the 32 rows of a store instruction spread over the
@@ -733,19 +738,20 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
       __syncthreads();  // every wave is done reading the ring
 #pragma unroll
       for (int mi = 0; mi < MF; ++mi) {
-        const int row = wm0 + mi * 32 + l32;
+        const int row = wm0 + mi * 32 + el32;
         const int x = (row & 31) << 1;
 #pragma unroll
         for (int ni = 0; ni < NF; ++ni)
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const v4f v = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
-            const int chunk = (wn0 + ni * 32 + u * 8 + h * 4) >> 2;
+            const int chunk = (wn0 + ni * 32 + u * 8 + eh * 4) >> 2;
             *reinterpret_cast<v4bf*>(smem + row * kRowB + ((chunk ^ x) << 3)) = __builtin_convertvector(v, v4bf);
           }
       }
       __syncthreads();
-      const int sub = tid & 15;
+      const int et = wave * 64 + el;
+      const int sub = et & 15;
       uint8_t* q_out = static_cast<uint8_t*>(p.c);
       float* s_out = p.act_s;
       if (kMaskedLike) {
@@ -754,7 +760,7 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
       }
 #pragma unroll 2
       for (int r0 = 0; r0 < BM; r0 += Cfg::NT / 16) {
-        const int row = r0 + (tid >> 4);
+        const int row = r0 + (et >> 4);
         const int x = (row & 31) << 1;
         const v4i graw = *reinterpret_cast<const v4i*>(smem + row * kRowB + (((2 * sub) ^ x) << 3));
         const v4i uraw = *reinterpret_cast<const v4i*>(smem + row * kRowB + (((BN / 4 / 2 + 2 * sub) ^ x) << 3));
@@ -859,9 +865,9 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
         if (m >= m_end) return;
         char* c_row = c_base + static_cast<int64_t>(m) * p.N * esz_c;
         if (p.out_f32)
-          store_row4<true>(c_row, n, sum, p.N - n, p.vec_store);
+          store_row4<true>(c_row, n, sum, p.N - n);
         else
-          store_row4<false>(c_row, n, sum, p.N - n, p.vec_store);
+          store_row4<false>(c_row, n, sum, p.N - n);
       };
       for (int round = 0; round < (last ? 2 : 1); ++round) {
         if (round == 1) {
@@ -910,78 +916,98 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
       }
       continue;
     }
-    if (sliced) {
-      // first pass of split-K: the slice's sums go to the workspace as an fp32 [M][N] matrix of their own;
-      // fp8_splitk_reduce_kernel, launched behind this kernel on the same stream, adds the slices in index order
-      float* mine = p.ws + static_cast<int64_t>(split) * p.M * p.N;
-      const bool vec_ok = (p.N % 4) == 0;
+    // Results leave through LDS: stored straight from the accumulator layout every instruction would touch 32 rows with
+    // 16 or 32 bytes each, partial sectors that the L2 has to merge.  Each wave parks rows of its tile in its own slice
+    // of the (now idle) ring, rotated by their index to spread the banks, and reads them back row-wise: a store
+    // instruction then writes whole rows, 16 bytes per lane, at whatever alignment N leaves the rows.
+    // (us per call: 3779 x 6111 x 1024 bf16, rows at odd addresses that used to leave 2 bytes a store, 95 -> 42; 2000 x 5001 x
+    // 4096 fp32 79 -> 53; 3875 x 11520 x 640 fp32, aligned rows, 75 -> 71.)
+    auto store_rows_f32 = [&](float* c_tile) __attribute__((always_inline)) {
+      // 32 rows of the wave's tile at a time
+      constexpr int kRowBytes = NF * 32 * 4;
+      constexpr int kCpr = kRowBytes / 16;   // 16-byte chunks per row
+      constexpr int kRpi = 64 / kCpr;        // rows per store instruction
+      static_assert(32 * kRowBytes * WAVES <= Cfg::LDS_BYTES, "the staging slices fit in the ring");
+      uint8_t* st = smem + wave * (32 * kRowBytes);
+      const int r_in = el / kCpr, ch = el % kCpr;
+      const int n_left = p.N - (n0 + wn0 + ch * 4);
 #pragma unroll
       for (int mi = 0; mi < MF; ++mi) {
-        const int m = m0 + wm0 + mi * 32 + l32;
-        if (m >= m_end) continue;
-        float* w_row = mine + static_cast<int64_t>(m) * p.N;
 #pragma unroll
         for (int ni = 0; ni < NF; ++ni)
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            const int n = n0 + wn0 + ni * 32 + u * 8 + h * 4;
             const v4f v = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
-            store_row4<true>(w_row, n, v, p.N - n, vec_ok);
+            *reinterpret_cast<v4f*>(st + el32 * kRowBytes + (ni * 8 + 2 * u + eh + el32) % kCpr * 16) = v;
           }
+        // a wave reads only what it wrote: no barrier, the LDS counter orders the two
+#pragma unroll 4
+        for (int r0 = 0; r0 < 32; r0 += kRpi) {
+          const int row = r0 + r_in;
+          if (el >= kRpi * kCpr || row >= 32) continue;
+          const v4f v = *reinterpret_cast<const v4f*>(st + row * kRowBytes + (ch + row) % kCpr * 16);
+          if (m0 + wm0 + mi * 32 + row < m_end) store_row4<true>(c_tile + static_cast<int64_t>(mi * 32 + row) * p.N, ch * 4, v, n_left);
+        }
       }
+    };
+    if (sliced) {
+      // first pass of split-K: the slice's sums go to the workspace as an fp32 [M][N] matrix of their own;
+      // fp8_splitk_reduce_kernel, launched behind this kernel on the same stream, adds the slices in index order
+      __syncthreads();  // every wave is done reading the ring
+      store_rows_f32(p.ws + static_cast<int64_t>(split) * p.M * p.N + static_cast<int64_t>(m0 + wm0) * p.N + n0 + wn0);
       continue;
     }
-    if (p.c_vec16) {
-      // bf16 through LDS: stored straight from the accumulator layout every instruction would touch 32 rows with
-      // 16 bytes each, partial sectors that the L2 has to merge.  Each wave parks its 64-row tile in its own slice of
-      // the (now idle) ring, rows rotated by their index to spread the banks, and reads it back row-wise: a store
-      // instruction then writes whole rows, 16 bytes per lane.
+    if (p.c_lds && p.out_f32) {
+      __syncthreads();
+      store_rows_f32(reinterpret_cast<float*>(c_base) + static_cast<int64_t>(m0 + wm0) * p.N + n0 + wn0);
+      continue;
+    }
+    if (p.c_lds) {
       constexpr int kRowBytes = NF * 32 * 2;
       constexpr int kCpr = kRowBytes / 16;   // 16-byte chunks per row
       constexpr int kRpi = 64 / kCpr;        // rows per store instruction
       static_assert(MF * 32 * kRowBytes * WAVES <= Cfg::LDS_BYTES, "the staging slices fit in the ring");
-      __syncthreads();  // every wave is done reading the ring
+      __syncthreads();
       uint8_t* st = smem + wave * (MF * 32 * kRowBytes);
 #pragma unroll
       for (int mi = 0; mi < MF; ++mi) {
-        const int row = mi * 32 + l32;
+        const int row = mi * 32 + el32;
 #pragma unroll
         for (int ni = 0; ni < NF; ++ni)
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const v4f v = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
             const int chunk = (ni * 4 + u + row) % kCpr;
-            *reinterpret_cast<v4bf*>(st + row * kRowBytes + chunk * 16 + h * 8) = __builtin_convertvector(v, v4bf);
+            *reinterpret_cast<v4bf*>(st + row * kRowBytes + chunk * 16 + eh * 8) = __builtin_convertvector(v, v4bf);
           }
       }
-      // a wave reads only what it wrote: no barrier, the LDS counter orders the two
-      const int r_in = lane / kCpr, ch = lane % kCpr;
+      const int r_in = el / kCpr, ch = el % kCpr;
+      const int n_left = p.N - (n0 + wn0 + ch * 8);
       __bf16* c_tile = reinterpret_cast<__bf16*>(c_base) + static_cast<int64_t>(m0 + wm0) * p.N + n0 + wn0;
 #pragma unroll 4
       for (int r0 = 0; r0 < MF * 32; r0 += kRpi) {
         const int row = r0 + r_in;
-        if (lane >= kRpi * kCpr || row >= MF * 32) continue;
+        if (el >= kRpi * kCpr || row >= MF * 32) continue;
         const v4i v = *reinterpret_cast<const v4i*>(st + row * kRowBytes + ((ch + row) % kCpr) * 16);
-        if (m0 + wm0 + row < m_end && n0 + wn0 + ch * 8 < p.N)
-          *reinterpret_cast<v4i*>(c_tile + static_cast<int64_t>(row) * p.N + ch * 8) = v;
+        if (m0 + wm0 + row < m_end && n_left > 0) store_row8_bf16(c_tile + static_cast<int64_t>(row) * p.N + ch * 8, v, n_left);
       }
       continue;
     }
 #pragma unroll
     for (int mi = 0; mi < MF; ++mi) {
-      const int m = m0 + wm0 + mi * 32 + l32;
+      const int m = m0 + wm0 + mi * 32 + el32;
       if (m >= m_end) continue;
       char* c_row = c_base + static_cast<int64_t>(m) * p.N * esz;
 #pragma unroll
       for (int ni = 0; ni < NF; ++ni) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const int n = n0 + wn0 + ni * 32 + u * 8 + h * 4;
+          const int n = n0 + wn0 + ni * 32 + u * 8 + eh * 4;
           const v4f v = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
           if (p.out_f32)
-            store_row4<true>(c_row, n, v, p.N - n, p.vec_store);
+            store_row4<true>(c_row, n, v, p.N - n);
           else
-            store_row4<false>(c_row, n, v, p.N - n, p.vec_store);
+            store_row4<false>(c_row, n, v, p.N - n);
         }
       }
     }

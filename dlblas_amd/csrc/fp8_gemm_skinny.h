@@ -141,9 +141,9 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_skinny_kernel(const Args p) 
     if (m >= p.M) continue;
     char* c_row = static_cast<char*>(p.c) + static_cast<int64_t>(m) * p.N * esz;
     if (p.out_f32)
-      store_row4<true>(c_row, n, sum, p.N - n, p.vec_store);
+      store_row4<true>(c_row, n, sum, p.N - n);
     else
-      store_row4<false>(c_row, n, sum, p.N - n, p.vec_store);
+      store_row4<false>(c_row, n, sum, p.N - n);
   }
 }
 
@@ -324,9 +324,9 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_skinny_dma_kernel(const Args
     if (m >= p.M || n >= n0 + cols) continue;
     char* c_row = static_cast<char*>(p.c) + static_cast<int64_t>(m) * p.N * esz;
     if (p.out_f32)
-      store_row4<true>(c_row, n, sum, n0 + cols - n, p.vec_store);
+      store_row4<true>(c_row, n, sum, n0 + cols - n);
     else
-      store_row4<false>(c_row, n, sum, n0 + cols - n, p.vec_store);
+      store_row4<false>(c_row, n, sum, n0 + cols - n);
   }
 }
 

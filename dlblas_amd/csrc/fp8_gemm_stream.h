@@ -554,8 +554,8 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
 #pragma unroll
         for (int ni = 0; ni < NF; ++ni) {
           const int nf = ct.n0 + wn0 + ni * 32;
-          if (p.c_vec16) {
-            // bf16 rows that are 16-byte aligned: lanes l and l + 32 swap halves so that each stores 8 consecutive columns
+          if (!p.out_f32) {
+            // lanes l and l + 32 swap halves so that each stores 8 consecutive columns
 #pragma unroll
             for (int u = 0; u < 4; u += 2) {
               v2i lo, hi;
@@ -569,18 +569,15 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
               const auto s1 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.y), static_cast<unsigned>(hi.y), false, false);
               const int n = nf + 8 * u + 8 * h;
               if (live && n < p.N)
-                *reinterpret_cast<v4i*>(c_row + static_cast<int64_t>(n) * 2) =
-                    v4i{static_cast<int>(s0[0]), static_cast<int>(s1[0]), static_cast<int>(s0[1]), static_cast<int>(s1[1])};
+                store_row8_bf16(reinterpret_cast<__bf16*>(c_row) + n,
+                                v4i{static_cast<int>(s0[0]), static_cast<int>(s1[0]), static_cast<int>(s0[1]), static_cast<int>(s1[1])}, p.N - n);
             }
           } else if (live) {
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
               const int n = nf + u * 8 + h * 4;
               const v4f v = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
-              if (p.out_f32)
-                store_row4<true>(c_row, n, v, p.N - n, p.vec_store);
-              else
-                store_row4<false>(c_row, n, v, p.N - n, p.vec_store);
+              store_row4<true>(c_row, n, v, p.N - n);
             }
           }
         }

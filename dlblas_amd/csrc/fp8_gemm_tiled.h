@@ -217,7 +217,6 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_tiled_kernel(const Args p) {
       // own; fp8_splitk_reduce_kernel, launched behind this kernel on the same stream, adds the slices in index
       // order (deterministic) and casts.  No fence, no counter: stream order makes the partial sums visible.
       float* mine = p.ws + static_cast<int64_t>(split) * p.M * p.N;
-      const bool vec_ok = (p.N % 4) == 0;
 #pragma unroll
       for (int mi = 0; mi < MF; ++mi) {
         const int m = m0 + wm0 + mi * 16 + l16;
@@ -226,7 +225,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_tiled_kernel(const Args p) {
 #pragma unroll
         for (int ni = 0; ni < NF; ++ni) {
           const int n = n0 + wn0 + ni * 16 + q * 4;
-          store_row4<true>(w_row, n, acc[mi][ni], p.N - n, vec_ok);
+          store_row4<true>(w_row, n, acc[mi][ni], p.N - n);
         }
       }
       continue;
@@ -242,9 +241,9 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_tiled_kernel(const Args p) {
       for (int ni = 0; ni < NF; ++ni) {
         const int n = n0 + wn0 + ni * 16 + q * 4;
         if (p.out_f32)
-          store_row4<true>(c_row, n, acc[mi][ni], p.N - n, p.vec_store);
+          store_row4<true>(c_row, n, acc[mi][ni], p.N - n);
         else
-          store_row4<false>(c_row, n, acc[mi][ni], p.N - n, p.vec_store);
+          store_row4<false>(c_row, n, acc[mi][ni], p.N - n);
       }
     }
   }
@@ -252,27 +251,26 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_tiled_kernel(const Args p) {
 
 // Split-K, second pass: c[i] = sum over s (in index order) of ws[s][i], i over the M x N outputs, four per thread.
 __global__ void __launch_bounds__(256) fp8_splitk_reduce_kernel(const float* ws, void* c, int64_t total, int splits,
-                                                                int out_f32, int vec_ok) {
+                                                                int out_f32) {
   const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
   if (i >= total) return;
   const int left = static_cast<int>(total - i < 4 ? total - i : 4);
   v4f sum = {0.f, 0.f, 0.f, 0.f};
-  if (vec_ok) {  // total % 4 == 0 and 16-byte aligned slices
+  if (left == 4) {
     for (int s = 0; s < splits; ++s)
-      sum += __builtin_nontemporal_load(reinterpret_cast<const v4f*>(ws + static_cast<int64_t>(s) * total + i));
+      sum += __builtin_nontemporal_load(reinterpret_cast<const v4f_el*>(ws + static_cast<int64_t>(s) * total + i));
   } else {
     for (int s = 0; s < splits; ++s) {
       const float* src = ws + static_cast<int64_t>(s) * total + i;
       sum.x += src[0];
       if (left > 1) sum.y += src[1];
       if (left > 2) sum.z += src[2];
-      if (left > 3) sum.w += src[3];
     }
   }
   if (out_f32)
-    store_row4<true>(c, i, sum, left, vec_ok != 0);
+    store_row4<true>(c, i, sum, left);
   else
-    store_row4<false>(c, i, sum, left, vec_ok != 0);
+    store_row4<false>(c, i, sum, left);
 }
 
 }  // namespace dlb

@@ -187,22 +187,19 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_wavek_kernel(const Args p) {
       const int m = f / NF * 32 + l32;
       const int n = n0 + f % NF * 32 + u * 8;
       char* c_row = static_cast<char*>(p.c) + static_cast<int64_t>(m0 + m) * p.N * (p.out_f32 ? 4 : 2);
-      if (p.c_vec16) {
+      if (!p.out_f32) {
         // lanes l and l + 32 swap halves so that each stores 8 consecutive columns
         const v2i lo = __builtin_bit_cast(v2i, __builtin_convertvector(s[0], v4bf)), hi = __builtin_bit_cast(v2i, __builtin_convertvector(s[1], v4bf));
         const auto s0 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.x), static_cast<unsigned>(hi.x), false, false);
         const auto s1 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.y), static_cast<unsigned>(hi.y), false, false);
         if (m < rows && n + 8 * h < p.N)
-          *reinterpret_cast<v4i*>(c_row + static_cast<int64_t>(n + 8 * h) * 2) =
-              v4i{static_cast<int>(s0[0]), static_cast<int>(s1[0]), static_cast<int>(s0[1]), static_cast<int>(s1[1])};
+          store_row8_bf16(reinterpret_cast<__bf16*>(c_row) + n + 8 * h,
+                          v4i{static_cast<int>(s0[0]), static_cast<int>(s1[0]), static_cast<int>(s0[1]), static_cast<int>(s1[1])}, p.N - n - 8 * h);
       } else if (m < rows) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const int col = n + 8 * i + 4 * h;
-          if (p.out_f32)
-            store_row4<true>(c_row, col, s[i], p.N - col, p.vec_store);
-          else
-            store_row4<false>(c_row, col, s[i], p.N - col, p.vec_store);
+          store_row4<true>(c_row, col, s[i], p.N - col);
         }
       }
     }

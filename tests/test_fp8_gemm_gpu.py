@@ -189,6 +189,54 @@ def test_epilogue_through_lds_equals_direct_stores(dev, variant, M, N, K):
     helpers.tolerance_check(staged, orc.dequant_ref(a_q, a_s, b_q, b_s), f'epilogue {variant}')
 
 
+@pytest.mark.parametrize('variant', ['pipe256x256', 'pipe128x256w8', 'pipe256mix', 'pipe128x128', 'pipe128x64', None])
+@pytest.mark.parametrize('M,N,K', [(257, 389, 256), (130, 1, 128), (33, 1023, 384), (5, 387, 512), (300, 514, 1040)])
+@pytest.mark.parametrize('out_dtype', [torch.bfloat16, torch.float32])
+def test_rows_at_any_alignment(dev, variant, M, N, K, out_dtype):
+    """Results whose rows start at odd elements, and fp32 results, through LDS and whole-row stores: the same bits as stored
+    element groups straight from the registers, in every kernel family."""
+    from dlblas_amd import _lib
+    if variant is not None and K % 128 != 0:
+        pytest.skip('the ring kernels take whole K blocks')
+    print(f'case rows variant={variant} M={M} N={N} K={K} {out_dtype}', flush=True)
+    a_q, a_s, b_q, b_s = helpers.make_dense(M, N, K, seed=29)
+    try:
+        _lib.tune('epilogue', 2)
+        direct = _run_dense(dev, a_q, a_s, b_q, b_s, dtype=out_dtype, variant=variant)
+    finally:
+        _lib.tune('epilogue', 0)
+    staged = _run_dense(dev, a_q, a_s, b_q, b_s, dtype=out_dtype, variant=variant)
+    assert torch.equal(direct, staged)
+    helpers.tolerance_check(staged, orc.dequant_ref(a_q, a_s, b_q, b_s), f'rows {variant}')
+
+
+@pytest.mark.parametrize('N', [389, 131, 514])
+@pytest.mark.parametrize('variant', ['pipe256x256', 'pipe128x256w8', 'pipe128x128', 'tile128x128', None])
+@pytest.mark.parametrize('out_dtype', [torch.bfloat16, torch.float32])
+def test_stores_end_with_the_row(dev, N, variant, out_dtype):
+    """The last valid row of an expert is followed by a row nobody may write: a store past the end of an odd row would show."""
+    from dlblas_amd import _lib
+    from dlblas_amd.kernels.fp8_gemm_grouped import m_grouped_fp8_gemm_nt_masked
+    G, cap, K = 3, 70, 256
+    a_q, a_s, b_q, b_s = helpers.make_dense(G * cap, G * 640, K, seed=31)
+    b_q = b_q.view(G, 640, K)[:, :N].contiguous()
+    b_s = b_s.view(G, 5, -1)[:, :-(-N // 128)].contiguous()
+    masked = torch.tensor([1, 33, 70], dtype=torch.int32)
+    out = torch.full((G, cap, N), 7.0, dtype=out_dtype, device=dev)
+    print(f'case row ends N={N} variant={variant} {out_dtype}', flush=True)
+    try:
+        _lib.force_variant(variant)
+        m_grouped_fp8_gemm_nt_masked((a_q.view(G, cap, K).to(dev), a_s.view(G, cap, -1).to(dev)), (b_q.to(dev), b_s.to(dev)), out, masked.to(dev), 35)
+        torch.cuda.synchronize()
+    finally:
+        _lib.force_variant(None)
+    for g in range(G):
+        v = int(masked[g])
+        rows = slice(g * cap, g * cap + v)
+        helpers.tolerance_check(out[g, :v].cpu(), orc.dequant_ref(a_q[rows], a_s[rows], b_q[g], b_s[g]), f'expert {g}')
+        assert bool((out[g, v:] == 7.0).all())
+
+
 @pytest.mark.parametrize('out_dtype', [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize('bn', [0, 4, 12, 20, 28, 32])
 @pytest.mark.parametrize('M,N,K', [(16, 1000, 1024), (5, 130, 256), (40, 2112, 1024), (100, 392, 512)])
