@@ -160,6 +160,7 @@ __device__ __forceinline__ void store_row8_bf16(__bf16* dst, v4i v, int n_left) 
   if (n_left >= 8) {
     *reinterpret_cast<v4i_el*>(dst) = v;
   } else {
+#pragma unroll 1
     for (int i = 0; i < n_left; ++i) {
       const uint32_t pair = static_cast<uint32_t>(i < 4 ? (i < 2 ? v.x : v.y) : (i < 6 ? v.z : v.w));
       dst[i] = __builtin_bit_cast(__bf16, static_cast<uint16_t>(i & 1 ? pair >> 16 : pair & 0xffffu));

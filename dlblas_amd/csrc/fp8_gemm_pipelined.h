@@ -724,9 +724,9 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
 
     // epilogue: lane holds c[m0 + wm0 + 32 mi + (lane & 31)][n0 + wn0 + 32 ni + 8 u + 4 (lane >> 5) + 0..3], u = 0..3
     // (the lane index passes through an empty asm: what is computed from it then stays behind the K loop instead of
-    // taking registers across it: the 256-row kernels spilled 19 to 49 of them)
+    // taking registers across it: the 256-row kernels spilled 19 to 49 of them.  One wave per SIMD has them to spare.)
     int el = lane;
-    asm volatile("" : "+v"(el));
+    if (!Cfg::PREFETCH) asm volatile("" : "+v"(el));
     const int el32 = el & 31, eh = el >> 5;
     if constexpr (kAct) {
       // The tile goes to LDS as the bf16 matrix the unfused GEMM would have written ([BM][gate 128 | up 128], 8-byte
@@ -922,6 +922,7 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
     // instruction then writes whole rows, 16 bytes per lane, at whatever alignment N leaves the rows.
     // (us per call: 3779 x 6111 x 1024 bf16, rows at odd addresses that used to leave 2 bytes a store, 95 -> 42; 2000 x 5001 x
     // 4096 fp32 79 -> 53; 3875 x 11520 x 640 fp32, aligned rows, 75 -> 71.)
+    const bool cols_inside = n0 + wn0 + NF * 32 <= p.N;  // no column of the wave's tile lies past N: stores without a tail
     auto store_rows_f32 = [&](float* c_tile) __attribute__((always_inline)) {
       // 32 rows of the wave's tile at a time
       constexpr int kRowBytes = NF * 32 * 4;
@@ -941,13 +942,19 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
             *reinterpret_cast<v4f*>(st + el32 * kRowBytes + (ni * 8 + 2 * u + eh + el32) % kCpr * 16) = v;
           }
         // a wave reads only what it wrote: no barrier, the LDS counter orders the two
+        auto store_rows = [&](auto inside) __attribute__((always_inline)) {
 #pragma unroll 4
-        for (int r0 = 0; r0 < 32; r0 += kRpi) {
-          const int row = r0 + r_in;
-          if (el >= kRpi * kCpr || row >= 32) continue;
-          const v4f v = *reinterpret_cast<const v4f*>(st + row * kRowBytes + (ch + row) % kCpr * 16);
-          if (m0 + wm0 + mi * 32 + row < m_end) store_row4<true>(c_tile + static_cast<int64_t>(mi * 32 + row) * p.N, ch * 4, v, n_left);
-        }
+          for (int r0 = 0; r0 < 32; r0 += kRpi) {
+            const int row = r0 + r_in;
+            if (el >= kRpi * kCpr || row >= 32) continue;
+            const v4f v = *reinterpret_cast<const v4f*>(st + row * kRowBytes + (ch + row) % kCpr * 16);
+            if (m0 + wm0 + mi * 32 + row < m_end) store_row4<true>(c_tile + static_cast<int64_t>(mi * 32 + row) * p.N, ch * 4, v, inside ? 4 : n_left);
+          }
+        };
+        if (cols_inside)
+          store_rows(std::true_type{});
+        else
+          store_rows(std::false_type{});
       }
     };
     if (sliced) {
@@ -984,13 +991,19 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
       const int r_in = el / kCpr, ch = el % kCpr;
       const int n_left = p.N - (n0 + wn0 + ch * 8);
       __bf16* c_tile = reinterpret_cast<__bf16*>(c_base) + static_cast<int64_t>(m0 + wm0) * p.N + n0 + wn0;
+      auto store_rows = [&](auto inside) __attribute__((always_inline)) {
 #pragma unroll 4
-      for (int r0 = 0; r0 < MF * 32; r0 += kRpi) {
-        const int row = r0 + r_in;
-        if (el >= kRpi * kCpr || row >= MF * 32) continue;
-        const v4i v = *reinterpret_cast<const v4i*>(st + row * kRowBytes + ((ch + row) % kCpr) * 16);
-        if (m0 + wm0 + row < m_end && n_left > 0) store_row8_bf16(c_tile + static_cast<int64_t>(row) * p.N + ch * 8, v, n_left);
-      }
+        for (int r0 = 0; r0 < MF * 32; r0 += kRpi) {
+          const int row = r0 + r_in;
+          if (el >= kRpi * kCpr || row >= MF * 32) continue;
+          const v4i v = *reinterpret_cast<const v4i*>(st + row * kRowBytes + ((ch + row) % kCpr) * 16);
+          if (m0 + wm0 + row < m_end && (inside || n_left > 0)) store_row8_bf16(c_tile + static_cast<int64_t>(row) * p.N + ch * 8, v, inside ? 8 : n_left);
+        }
+      };
+      if (cols_inside)
+        store_rows(std::true_type{});
+      else
+        store_rows(std::false_type{});
       continue;
     }
 #pragma unroll

@@ -192,14 +192,19 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_wavek_kernel(const Args p) {
         const v2i lo = __builtin_bit_cast(v2i, __builtin_convertvector(s[0], v4bf)), hi = __builtin_bit_cast(v2i, __builtin_convertvector(s[1], v4bf));
         const auto s0 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.x), static_cast<unsigned>(hi.x), false, false);
         const auto s1 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.y), static_cast<unsigned>(hi.y), false, false);
-        if (m < rows && n + 8 * h < p.N)
-          store_row8_bf16(reinterpret_cast<__bf16*>(c_row) + n + 8 * h,
-                          v4i{static_cast<int>(s0[0]), static_cast<int>(s1[0]), static_cast<int>(s0[1]), static_cast<int>(s1[1])}, p.N - n - 8 * h);
+        const v4i v = {static_cast<int>(s0[0]), static_cast<int>(s1[0]), static_cast<int>(s0[1]), static_cast<int>(s1[1])};
+        if (m < rows && n + 8 * h < p.N) {
+          __bf16* dst = reinterpret_cast<__bf16*>(c_row) + n + 8 * h;
+          if (cols == BN)  // no store crosses the row's end
+            store_row8_bf16(dst, v, 8);
+          else
+            store_row8_bf16(dst, v, p.N - n - 8 * h);
+        }
       } else if (m < rows) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const int col = n + 8 * i + 4 * h;
-          store_row4<true>(c_row, col, s[i], p.N - col);
+          store_row4<true>(c_row, col, s[i], cols == BN ? 4 : p.N - col);
         }
       }
     }
