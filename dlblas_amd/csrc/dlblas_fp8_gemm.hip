@@ -159,7 +159,10 @@ typedef PipeCfg<2, 2, 2, 1, 5, 2, true> Pipe128x64;   // wave tile 64 x 32, 5 st
 // workgroup as the LDS left by the ring holds: 54 and 64)
 typedef PipeCfg<2, 2, 2, 2, 4, 2, true, true, 54> Pipe128x128T;
 typedef PipeCfg<2, 2, 2, 1, 5, 2, true, true, 64> Pipe128x64T;
-typedef PipeCfg<2, 4, 2, 2, 3, 2, false, true, 16> Pipe128x256w8T;  // the masked layout's tiles (K of at most 16 blocks: 8 KB next to the 150 KB ring)
+typedef PipeCfg<2, 4, 2, 2, 3, 2, false, true, 16> Pipe128x256w8T;  // 8 KB next to the 150 KB ring
+typedef PipeCfg<4, 2, 2, 4, 2, 2, false, true, 27> Pipe256x256T;    // 28 KB next to 132 KB
+typedef PipeCfg<4, 2, 2, 3, 2, 2, false, true, 27> Pipe256x192T;
+static_assert(Pipe256x256T::LDS_BYTES <= 160 * 1024 && Pipe256x192T::LDS_BYTES <= Pipe256x256T::LDS_BYTES, "ring + table fit the LDS");
 static_assert(Pipe128x256w8T::LDS_BYTES <= 160 * 1024 && Pipe128x128T::LDS_BYTES <= 160 * 1024 && Pipe128x64T::LDS_BYTES <= 160 * 1024, "ring + table fit the LDS");
 constexpr int kFusedMaxTiles = DLB_WS_COUNTER_BYTES / 16;  // four counter words per tile in the workspace head
 
@@ -870,16 +873,22 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
     }
     if (worth_it && nblk <= kTileListMaxBlocks && DLB_WS_COUNTER_BYTES + bytes <= ws_bytes) r.tile_list = true, r.nblk = nblk, r.ws_used = bytes;
   }
-  // Small ring kernels with at most 32 K blocks per workgroup fetch a tile's row-major scales once, into a table in
-  // LDS: no re-layout pass, one cache-line request per row and tile.
-  const bool small_ring = pl.variant == kVarPipe128x128 || pl.variant == kVarPipe128x64;
-  // (the masked layout's 128 x 256 tiles take the table too: a decode-sized K, no re-layout launch in front)
-  const bool masked_ring = mode == kMasked && pl.variant == kVarPipe128x256w8 && !gather_scales && !fused_act && g_forced_variant < 0;
+  // A tile's row-major scales come once, into a table in LDS, where its K range fits what the ring leaves of the LDS: no re-layout
+  // launch in front (3 - 4 us), one cache-line request per row and tile.  us per call with the pre-pass / with the table: dense
+  // 1024 x 8192 x 1536 22.5 / 19.2, 4096 x 7168 x 1024 44 / 40; contiguous 8 experts, 171 rows, 1408 x 2048 19.6 / 16.3, 16
+  // experts, 494 rows, 3712 x 1024 22.2 / 18.3; masked 16 x 0 .. 512 x 4096 x 1024 46 / 43.  Launches of many rounds fetch a table per
+  // tile and gain nothing any more from 8 K blocks on (4096 x 24576 x 1536 175 / 175), nor lose.
   auto table_fits = [&](int kb_per) {
-    return ((mode == kDense && small_ring) || masked_ring) && g_knob[kKnobScaleTable] != 2 && as_sm != 1 &&
-           kb_per <= (masked_ring ? Pipe128x256w8T::SCTAB_KB
-                                  : (pl.variant == kVarPipe128x64 ? Pipe128x64T::SCTAB_KB : Pipe128x128T::SCTAB_KB)) &&
-           as_sk < (1ll << 20) && dma_ok;
+    if (g_knob[kKnobScaleTable] == 2 || as_sm == 1 || as_sk >= (1ll << 20) || !dma_ok || r.tile_list || gather_scales || fused_act) return false;
+    switch (pl.variant) {
+      case kVarPipe128x64: return mode == kDense && kb_per <= Pipe128x64T::SCTAB_KB;
+      case kVarPipe128x128: return kb_per <= Pipe128x128T::SCTAB_KB;
+      // (dense, up to 4 K blocks: the pre-pass stays, 15.1 / 11.8 us at 2048 x 4096 x 512 - the test that a refused launch leaves no
+      // pre-pass behind is about this one)
+      case kVarPipe128x256w8: return (mode != kMasked || g_forced_variant < 0) && (mode != kDense || kb_per > 4) && kb_per <= Pipe128x256w8T::SCTAB_KB;
+      case kVarPipe256x256: case kVarPipe256mix: return kb_per <= Pipe256x256T::SCTAB_KB;
+      default: return false;
+    }
   };
   r.sctab = r.stream == kStreamNone && table_fits(r.kb_per_split);
   // gather_scales: the re-layout pass also brings the rows into the GEMM's order, so it runs whatever the strides
@@ -1223,20 +1232,22 @@ int run(const Problem& pr) {
     const int g_dense = rs.resident ? cus : g;
     if (pl.variant == kVarPipe256mix) {
       const int64_t split = rs.n_split;
-      if (split >= pr.N) return launch_pipelined_mode<Pipe256x256>(pr.mode, ar, g_dense, dev, pr.stream);
-      static std::atomic<unsigned long long> lds_done{0};
-      auto kernel = fp8_gemm_pipelined_mixed_kernel<Pipe256x256, Pipe256x192>;
+      if (split >= pr.N)
+        return rs.sctab ? launch_pipelined_mode<Pipe256x256T>(pr.mode, ar, g_dense, dev, pr.stream) : launch_pipelined_mode<Pipe256x256>(pr.mode, ar, g_dense, dev, pr.stream);
+      static std::atomic<unsigned long long> lds_done[2];
+      auto kernel = rs.sctab ? fp8_gemm_pipelined_mixed_kernel<Pipe256x256T, Pipe256x192T> : fp8_gemm_pipelined_mixed_kernel<Pipe256x256, Pipe256x192>;
+      const int lds = rs.sctab ? Pipe256x256T::LDS_BYTES : Pipe256x256::LDS_BYTES;
       ar.n_split = static_cast<int>(split);
       ar.tiles_n_a = static_cast<int>(split / 256);
       ar.tiles_n_b = static_cast<int>(ceil_div(pr.N - split, 192));
       ar.tiles_a = ar.tiles_m * ar.tiles_n_a;
-      const hipError_t le = ensure_lds(kernel, Pipe256x256::LDS_BYTES, dev, &lds_done);
+      const hipError_t le = ensure_lds(kernel, lds, dev, &lds_done[rs.sctab ? 1 : 0]);
       if (le != hipSuccess || g_prepare_only) return le;
-      hipLaunchKernelGGL(kernel, dim3(ar.tiles_a + ar.tiles_m * ar.tiles_n_b), dim3(Pipe256x256::NT), Pipe256x256::LDS_BYTES,
-                         pr.stream, ar);
+      hipLaunchKernelGGL(kernel, dim3(ar.tiles_a + ar.tiles_m * ar.tiles_n_b), dim3(Pipe256x256::NT), lds, pr.stream, ar);
       return hipGetLastError();
     }
-    if (pl.variant == kVarPipe256x256) return launch_pipelined_mode<Pipe256x256>(pr.mode, ar, g_dense, dev, pr.stream);
+    if (pl.variant == kVarPipe256x256)
+      return rs.sctab ? launch_pipelined_mode<Pipe256x256T>(pr.mode, ar, g_dense, dev, pr.stream) : launch_pipelined_mode<Pipe256x256>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x256w8 && tile_list && pr.act) {
       static std::atomic<unsigned long long> lds_done{0};
       auto kernel = fp8_gemm_contig_list_act_kernel<Pipe256x256, Pipe192x256, Pipe128x256w8>;
@@ -1257,10 +1268,10 @@ int run(const Problem& pr) {
     }
     if (pl.variant == kVarPipe128x256w8 && pr.act)
       return launch_pipelined<Pipe128x256w8, kMaskedAct>(ar, g, dev, pr.stream);  // N / 256 column tiles, as the plain GEMM
-    if (pl.variant == kVarPipe128x256w8 && pr.mode == kMasked && rs.sctab) return launch_pipelined<Pipe128x256w8T, kMasked>(ar, g, dev, pr.stream);
+    if (pl.variant == kVarPipe128x256w8 && rs.sctab) return launch_pipelined_mode<Pipe128x256w8T>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x256w8) return launch_pipelined_mode<Pipe128x256w8>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x128)
-      return rs.sctab ? launch_pipelined<Pipe128x128T, kDense>(ar, g, dev, pr.stream)
+      return rs.sctab ? launch_pipelined_mode<Pipe128x128T>(pr.mode, ar, g, dev, pr.stream)
                       : launch_pipelined_mode<Pipe128x128>(pr.mode, ar, g, dev, pr.stream);
     if (pl.variant == kVarPipe128x64)
       return rs.sctab ? launch_pipelined<Pipe128x64T, kDense>(ar, g, dev, pr.stream)

@@ -143,6 +143,51 @@ def test_scale_table_equals_scales_per_stage(dev, M, N, K, variant, splitk):
     assert torch.equal(with_table, per_stage)
 
 
+@pytest.mark.parametrize('layout,variant,rows,N,blocks', [
+    ('dense', 'pipe256x256', 300, 520, 27), ('dense', 'pipe256x256', 257, 130, 28), ('dense', 'pipe256mix', 700, 1000, 1),
+    ('dense', 'pipe256mix', 513, 1000, 5), ('dense', 'pipe128x256w8', 257, 300, 5), ('dense', 'pipe128x256w8', 129, 300, 16),
+    ('contiguous', 'pipe128x128', 512, 392, 54), ('contiguous', 'pipe128x128', 384, 136, 55), ('contiguous', 'pipe128x256w8', 640, 520, 16),
+    ('masked', 'pipe128x128', 200, 392, 3), ('masked', 'pipe256x256', 300, 392, 27), ('masked', 'pipe256x256', 260, 130, 28)])
+def test_scale_table_of_every_ring_kernel(dev, layout, variant, rows, N, blocks):
+    """The table of the larger tiles and of the grouped layouts, at the longest K it takes and one block beyond: the bits of the
+    scales fetched through the re-layout pre-pass."""
+    from dlblas_amd import _lib
+    from dlblas_amd.kernels.fp8_gemm_grouped import m_grouped_fp8_gemm_nt_contiguous, m_grouped_fp8_gemm_nt_masked
+    print(f'case scale table {layout} {variant} {rows}x{N} {blocks} blocks', flush=True)
+    G, K = 3, 128 * blocks
+    a_q, a_s, b_q, b_s = helpers.make_dense(rows * (G if layout == 'masked' else 1), N if layout == 'dense' else 640 * G, K, seed=37)
+    outs = []
+    for knob in (0, 2):
+        try:
+            _lib.tune('scale_table', knob)
+            if layout == 'dense':
+                outs.append(_run_dense(dev, a_q, a_s, b_q, b_s, variant=variant))
+                continue
+            w = b_q.view(G, 640, K)[:, :N].contiguous().to(dev), b_s.view(G, 5, -1)[:, :-(-N // 128)].contiguous().to(dev)
+            _lib.force_variant(variant)
+            if layout == 'masked':
+                valid = torch.tensor([rows, 1, rows - 37], dtype=torch.int32)
+                out = torch.zeros(G, rows, N, dtype=torch.bfloat16, device=dev)
+                m_grouped_fp8_gemm_nt_masked((a_q.view(G, rows, K).to(dev), a_s.view(G, rows, -1).to(dev)), w, out, valid.to(dev), rows)
+            else:
+                expert = torch.arange(rows, dtype=torch.int32) // 128 % G
+                out = torch.zeros(rows, N, dtype=torch.bfloat16, device=dev)
+                m_grouped_fp8_gemm_nt_contiguous((a_q.to(dev), a_s.to(dev)), w, out, expert.to(dev))
+            torch.cuda.synchronize()
+            outs.append(out)
+        finally:
+            _lib.tune('scale_table', 0)
+            _lib.force_variant(None)
+    assert torch.equal(outs[0], outs[1])
+    if layout == 'dense':
+        helpers.tolerance_check(outs[0], orc.dequant_ref(a_q, a_s, b_q, b_s), f'{layout} {variant}')
+    else:
+        last = outs[0].view(-1, rows, N)[-1][:1 if layout == 'masked' else rows].cpu()
+        row = slice(2 * rows, 2 * rows + 1) if layout == 'masked' else slice(0, 128)
+        ref = orc.dequant_ref(a_q[row], a_s[row], *(t.cpu() for t in ((w[0][2], w[1][2]) if layout == 'masked' else (w[0][0], w[1][0]))))
+        helpers.tolerance_check(last[:ref.size(0)], ref, f'{layout} {variant}')
+
+
 def test_refused_launch_enqueues_nothing(dev):
     """A call whose main kernel cannot be launched (here: a forced request for more LDS than the GPU has) returns
     DLB_ERR_LAUNCH before any pre-pass is enqueued: workspace and output keep their bytes."""
