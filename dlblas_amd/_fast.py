@@ -12,8 +12,7 @@ from ._build import HOST_PATH
 # the library's entry points in the order of the Abi struct in csrc/host_calls.cpp
 _ABI = ('dlb_last_error', 'dlb_workspace_lock', 'dlb_workspace_unlock', 'dlb_fp8_gemm', 'dlb_fp8_gemm_grouped_contiguous', 'dlb_fp8_gemm_grouped_contiguous_same_rows',
         'dlb_fp8_gemm_grouped_contiguous_gather_silu_quant', 'dlb_fp8_gemm_grouped_masked',
-        'dlb_fp8_gemm_grouped_masked_silu_quant', 'dlb_fp8_gemm_grouped_ragged', 'dlb_fp8_gemm_grouped_ragged_silu_quant',
-        'dlb_fp8_gemm_plan_grouped', 'dlb_fp8_gemm_plan_stream', 'dlb_fp8_gemm_variant_name', 'dlb_fp8_quant_group',
+        'dlb_expert_gate_up_masked', 'dlb_fp8_gemm_grouped_ragged', 'dlb_expert_gate_up_ragged', 'dlb_expert_plan', 'dlb_fp8_quant_group',
         'dlb_silu_mul_quant_masked', 'dlb_ep_scatter_workspace_bytes', 'dlb_ep_scatter_rows_host', 'dlb_ep_gather')
 
 

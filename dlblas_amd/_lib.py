@@ -12,7 +12,7 @@ import torch
 
 from ._build import LIB_PATH
 
-ABI_VERSION = 9
+ABI_VERSION = 10
 OUT_BF16, OUT_F32 = 0, 1
 WS_COUNTER_BYTES = 65536
 WORKSPACE_BYTES = WS_COUNTER_BYTES + (32 << 20)
@@ -48,6 +48,11 @@ SYMBOLS = {
     (ctypes.c_int, [_c_vp] * 7 + [_c_i32] + [_c_i64] * 3 + [_c_i32] + [_c_i64] * 2 + [ctypes.c_int, _c_vp]),
     'dlb_fp8_gemm_grouped_ragged_silu_quant':
     (ctypes.c_int, [_c_vp] * 9 + [_c_i64, _c_i32] + [_c_i64] * 3 + [_c_i32] + [_c_i64] * 4 + [ctypes.c_float, _c_vp]),
+    'dlb_expert_gate_up_masked':
+    (ctypes.c_int, [_c_vp] * 7 + [_c_i32] + [_c_i64] * 3 + [_c_i32] + [_c_i64] * 6 + [ctypes.c_float, _c_vp, _c_sz, _c_vp]),
+    'dlb_expert_gate_up_ragged':
+    (ctypes.c_int, [_c_vp] * 9 + [_c_i64, _c_i32] + [_c_i64] * 3 + [_c_i32] + [_c_i64] * 4 + [ctypes.c_float, _c_vp, _c_sz, _c_vp]),
+    'dlb_expert_plan': (ctypes.c_int, [ctypes.c_int] + [_c_i64] * 3 + [_c_i32] * 2 + [ctypes.c_int, _c_sz, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]),
     'dlb_fp8_quant_1x128': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp, _c_vp] + [_c_i64] * 5 + [ctypes.c_float, _c_vp]),
     'dlb_fp8_quant_group': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp, _c_vp] + [_c_i64] * 6 + [ctypes.c_float, _c_vp]),
     'dlb_fp8_quant_128x128': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp, _c_vp] + [_c_i64] * 4 + [ctypes.c_float, _c_vp]),
@@ -232,6 +237,17 @@ def plan_stream(M_max: int, N: int, K: int, G: int, expected_m: int = -1, quanti
     return (out[0].value, out[1].value, bool(out[2].value)) if out[0].value else None
 
 
+STEPS_APART, ON_ROW_RANGES, ON_WHOLE_BLOCKS = 0, 1, 2  # forms of expert_plan()
+
+
+def expert_plan(mode: int, rows: int, N: int, K: int, G: int, expected_m: int, quantising: bool, compute_units: int = 256) -> int:
+    """Which kernels run a projection of an expert MLP fastest (quantising: gate/up, N = 2 I).  mode 1: expert-contiguous rows,
+    2: masked layout (nonzero: dlb_expert_gate_up_masked takes the gate/up projection)."""
+    form = ctypes.c_int()
+    check(load().dlb_expert_plan(mode, rows, N, K, G, expected_m, int(quantising), WORKSPACE_BYTES, compute_units, ctypes.byref(form)))
+    return form.value
+
+
 def force_variant(name_or_id) -> None:
     """Pin the kernel variant used by later calls from this thread (None or -1: back to the heuristic)."""
     lib = load()
@@ -243,7 +259,7 @@ def force_variant(name_or_id) -> None:
 
 
 KNOBS = {'splitk': 0, 'skinny_waves': 1, 'skinny_unroll': 2, 'skinny_nfrags': 3, 'group_m': 4, 'skinny_dma': 5, 'epilogue': 6, 'skinny_bn': 7,
-         'splitk_mode': 8, 'spin_limit': 9, 'scale_table': 10, 'lds_oversize': 11, 'masked_grid': 12, 'tile_list': 13, 'stream': 14, 'wave_k': 15}
+         'splitk_mode': 8, 'spin_limit': 9, 'scale_table': 10, 'lds_oversize': 11, 'masked_grid': 12, 'tile_list': 13, 'stream': 14, 'wave_k': 15, 'stream_slices': 16}
 
 
 def tune(knob: str, value) -> None:
@@ -343,17 +359,17 @@ def gemm_masked(a, b, a_s, b_s, c, masked_m, expected_m, M_max, N, K, G, as_sg, 
                                             out_code(c.dtype), _ptr(ws), ws.numel(), ctypes.c_void_p(stream)))
 
 
-def gemm_masked_silu_quant(a, b, a_s, b_s, out_q, out_s, masked_m, expected_m, M_max, N, K, G, as_sg, as_sm, as_sk, eps) -> bool:
+def gemm_masked_silu_quant(a, b, a_s, b_s, out_q, out_s, masked_m, expected_m, M_max, N, K, G, as_sg, as_sm, as_sk, eps, mlp=False) -> bool:
     """The fused masked gate/up GEMM + up * silu(gate) + 1 x 128 quantiser.  False when the library has no fused kernel
-    for the shape (ERR_BAD_SHAPE): nothing was enqueued and the caller runs the steps apart."""
+    for the shape (ERR_BAD_SHAPE): nothing was enqueued and the caller runs the steps apart.  mlp: as a step of an expert MLP
+    (dlb_expert_gate_up_masked)."""
     _require_gpu(a, b, a_s, b_s, out_q, out_s, masked_m)
     lib = load()
     with torch.cuda.device(a.device):
         stream, ws = _stream_and_ws(a)
-        rc = lib.dlb_fp8_gemm_grouped_masked_silu_quant(_ptr(a), _ptr(b), _ptr(a_s), _ptr(b_s), _ptr(out_q), _ptr(out_s),
-                                                        _ptr(masked_m), int(expected_m), M_max, N, K, G, as_sg, as_sm, as_sk,
-                                                        out_s.stride(0), out_s.stride(1), out_s.stride(2), float(eps),
-                                                        _ptr(ws), ws.numel(), ctypes.c_void_p(stream))
+        call = lib.dlb_expert_gate_up_masked if mlp else lib.dlb_fp8_gemm_grouped_masked_silu_quant
+        rc = call(_ptr(a), _ptr(b), _ptr(a_s), _ptr(b_s), _ptr(out_q), _ptr(out_s), _ptr(masked_m), int(expected_m), M_max, N, K, G, as_sg, as_sm,
+                  as_sk, out_s.stride(0), out_s.stride(1), out_s.stride(2), float(eps), _ptr(ws), ws.numel(), ctypes.c_void_p(stream))
         if rc == ERR_BAD_SHAPE:
             return False
         check(rc)
@@ -471,6 +487,23 @@ def ep_scatter_rows_host(recv_topk, counts, row_start, row_end, expert_start_loc
                                           _ptr(row_start), _ptr(row_end), _ptr(expert_start_loc), _ptr(m_indices), _ptr(src_row),
                                           m_indices.numel(), _ptr(output_index), _idx_code(output_index), output_index.stride(0),
                                           output_index.stride(1), T, topk, E, _ptr(ws), ws.numel(), ctypes.c_void_p(stream))
+    if rc == ERR_BAD_SHAPE:
+        return False
+    check(rc)
+    return True
+
+
+def expert_gate_up_ragged(a, b, a_s, b_s, out_q, out_s, row_start, row_end, a_row_index, expected_m, eps) -> bool:
+    """dlb_expert_gate_up_ragged (a_row_index: None or the source row of every GEMM row); False when declined."""
+    _require_gpu(a, b, a_s, b_s, out_q, out_s, row_start, row_end)
+    lib = load()
+    G, N, K = b.shape
+    stream = torch.cuda.current_stream(a.device).cuda_stream
+    ws = workspace(a.device, stream)
+    with torch.cuda.device(a.device):
+        rc = lib.dlb_expert_gate_up_ragged(_ptr(a), _ptr(b), _ptr(a_s), _ptr(b_s), _ptr(out_q), _ptr(out_s), _ptr(row_start), _ptr(row_end),
+                                           _ptr(a_row_index), a.size(0), expected_m, out_q.size(0), N, K, G, a_s.stride(0), a_s.stride(1),
+                                           out_s.stride(0), out_s.stride(1), float(eps), _ptr(ws), ws.numel(), ctypes.c_void_p(stream))
     if rc == ERR_BAD_SHAPE:
         return False
     check(rc)

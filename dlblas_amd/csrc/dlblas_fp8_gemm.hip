@@ -105,6 +105,7 @@ enum Knob : int {
   kKnobTileList,     // expert-contiguous rows: 1 = device-built tile lists whenever possible, 2 = never (0 = by batch size)
   kKnobStream,       // masked layout: 1 = never the weight-streaming kernel, 2 + i = its tile shape i wherever it applies (0 = by size), 7 + i = the same, fragments read ahead
   kKnobWaveK,        // dense: 1 = never the kernel whose waves split K, 2 + i = its tile shape i wherever it applies (0 = by size)
+  kKnobStreamSlices, // K slices of the weight-streaming kernel (0 = by estimate, or one where its shape is forced)
   kKnobCount
 };
 thread_local int g_knob[kKnobCount] = {};
@@ -175,6 +176,14 @@ typedef StreamCfg<2, 2, 1, 1, 9, 16> Stream64x64;
 enum StreamShape : int { kStreamNone = -1, kStream32x256 = 0, kStream64x256, kStream64x128, kStream128x256, kStream64x64, kStreamCount };
 struct StreamDims { int bm, bn, stages, ch; };
 constexpr StreamDims kStreamDims[kStreamCount] = {{32, 256, 4, 16}, {64, 256, 3, 16}, {64, 128, 6, 16}, {128, 256, 3, 11}, {64, 64, 9, 16}};
+
+struct StreamPlan {
+  int shape = kStreamNone;  // tile shape (kStreamNone: a ring kernel runs)
+  int chunk_len = 0;        // K blocks per chunk of the scale table
+  bool ahead = false;       // fragments read one step ahead
+  int slices = 0;           // K slices whose fp32 sums a second launch adds (it also carries the quantising epilogue then); 0: one launch
+  double us = 0.0;
+};
 
 // Tile shapes of the dense kernel whose waves split K
 struct WaveKDims { int mf, nf, waves; };
@@ -272,7 +281,7 @@ hipError_t launch_stream(const Args& args, int grid, int dev, hipStream_t stream
 // ahead: fragments read one step ahead of their use (plain product, tiles of 64 rows or more)
 template <int EPI, bool GATHER>
 hipError_t launch_stream_shape(int shape, bool ahead, const Args& args, int grid, int dev, hipStream_t stream) {
-  if constexpr (EPI == kStoreProduct) {
+  if constexpr (EPI == kStoreProduct || EPI == kStoreSlice) {
     if (ahead) switch (shape) {
       case kStream64x256: return launch_stream<Stream64x256, EPI, GATHER, true>(args, grid, dev, stream);
       case kStream64x128: return launch_stream<Stream64x128, EPI, GATHER, true>(args, grid, dev, stream);
@@ -292,6 +301,47 @@ hipError_t launch_stream_shape(int shape, bool ahead, const Args& args, int grid
     case kStream128x256: return launch_stream<Stream128x256, EPI, GATHER, false>(args, grid, dev, stream);
     default: return hipErrorInvalidValue;
   }
+}
+
+// One call of the weight-streaming kernel and, with K slices, of the kernel that adds them.  worst_mtiles: row tiles at most, over all
+// experts; span: rows that cover nearly every expert; all_rows: of the output.
+hipError_t launch_stream_plan(const StreamPlan& sp, int epi, Args ar, int64_t worst_mtiles, int64_t span, int64_t all_rows, int cus, int dev, hipStream_t stream) {
+  const bool sliced = sp.slices > 0;
+  const bool fused = epi != kStoreProduct && !sliced;
+  ar.chunk_len = sp.chunk_len;
+  ar.splitk = sliced ? sp.slices : 1;
+  ar.kb_per_split = ar.kblocks / ar.splitk;
+  ar.tiles_n = static_cast<int>(fused ? ar.N / 256 : ceil_div(ar.N, kStreamDims[sp.shape].bn));
+  const int64_t worst = static_cast<int64_t>(ar.tiles_n) * worst_mtiles * ar.splitk;
+  const int grid = static_cast<int>(ceil_div(worst < cus ? worst : cus, 32) * 32);  // tiles are dealt to the XCDs four at a time
+  const Args out = ar;
+  if (sliced) {
+    ar.c = ar.ws;
+    ar.c_gs = all_rows * ar.N;
+  }
+  hipError_t e;
+  if (fused && epi == kSiluQuantMasked)
+    e = launch_stream_shape<kSiluQuantMasked, false>(sp.shape, false, ar, grid, dev, stream);
+  else if (fused)
+    e = ar.a_rows ? launch_stream_shape<kSiluQuant, true>(sp.shape, false, ar, grid, dev, stream) : launch_stream_shape<kSiluQuant, false>(sp.shape, false, ar, grid, dev, stream);
+  else if (sliced)
+    e = ar.a_rows ? launch_stream_shape<kStoreSlice, true>(sp.shape, sp.ahead, ar, grid, dev, stream) : launch_stream_shape<kStoreSlice, false>(sp.shape, sp.ahead, ar, grid, dev, stream);
+  else
+    e = launch_stream_shape<kStoreProduct, false>(sp.shape, sp.ahead, ar, grid, dev, stream);
+  if (e != hipSuccess || g_prepare_only || !sliced) return e;
+  Args red = out;
+  red.c_gs = ar.c_gs;
+  // blocks for the rows nearly every expert has; a longer expert's blocks go round again
+  const int64_t per_row = epi == kStoreProduct ? ceil_div(ar.N, 4) : ar.act_cols / 8;
+  const int64_t blocks = std::min<int64_t>(ceil_div(span * per_row, 256), ceil_div(4096, ar.G));
+  const dim3 rgrid(static_cast<unsigned>(blocks < 1 ? 1 : blocks), static_cast<unsigned>(ar.G));
+  if (epi == kStoreProduct)
+    hipLaunchKernelGGL(fp8_stream_reduce_kernel, rgrid, dim3(256), 0, stream, red);
+  else if (epi == kSiluQuantMasked)
+    hipLaunchKernelGGL(fp8_stream_reduce_act_kernel<kSiluQuantMasked>, rgrid, dim3(256), 0, stream, red);
+  else
+    hipLaunchKernelGGL(fp8_stream_reduce_act_kernel<kSiluQuant>, rgrid, dim3(256), 0, stream, red);
+  return hipGetLastError();
 }
 
 template <class Cfg>
@@ -699,9 +749,7 @@ struct Resolved {
   bool sctab;                // small ring kernels: row-major activation scales through the per-tile table in LDS
   int sct_pitch;             //   floats per table row (odd)
   bool fused;                // K slices added inside the launch (counters in the workspace head), no second pass
-  int stream;                // masked layout: tile shape of the weight-streaming kernel (kStreamNone: a ring kernel)
-  int chunk_len;             //   K blocks per chunk of its scale table
-  bool ahead;                //   and whether it reads its fragments one step ahead
+  StreamPlan stream;         // masked layout: the weight-streaming kernel's share of the plan
   int wavek;                 // dense: tile shape of the kernel whose waves split K (kWaveKNone: another kernel)
 };
 
@@ -769,60 +817,162 @@ int pick_wavek(int64_t M, int64_t N, int64_t K, int cus, size_t ws_bytes) {
 }
 
 // K blocks per chunk of the streaming kernel's scale table: equal chunks of at most `ch` blocks, none shorter than the
-// stages - 1 steps the issue side runs ahead (the table has two buffers).  0: no such cut.
-int stream_chunk_len(int kblocks, int ch, int stages) {
-  for (int len = static_cast<int>(ceil_div(kblocks, ceil_div(kblocks, ch))); len >= stages - 1 && len > 0; --len) {
-    const int last = kblocks % len == 0 ? len : kblocks % len;
-    if (last >= stages - 1) return len;
-  }
+// stages - 1 steps the issue side runs ahead (the table has two buffers), for tiles of kb_min and of kb_max blocks.  0: no such cut.
+int stream_chunk_len(int kb_min, int kb_max, int ch, int stages) {
+  auto last = [](int kb, int len) { return kb % len == 0 ? len : kb % len; };
+  for (int len = static_cast<int>(ceil_div(kb_max, ceil_div(kb_max, ch))); len >= stages - 1 && len > 0; --len)
+    if (last(kb_min, len) >= stages - 1 && last(kb_max, len) >= stages - 1) return len;
   return 0;
 }
 
 // Rows that cover nearly all experts: twice the caller's hint, at most the buffers' height.
 int64_t stream_span(int64_t M, int64_t hint_rows) { return hint_rows > 0 && 2 * hint_rows < M ? 2 * hint_rows : M; }
-constexpr int kStreamActSpan = 192;  // the longest experts the weight-streaming kernel takes with the quantising epilogue
-
-// Which tile shape of the weight-streaming kernel runs a masked launch (kStreamNone: none), from the typical rows of an
-// expert (twice the caller's hint covers nearly all of them).  A tile's step lasts what is longer of the trip its loads
-// take with the chip to themselves, 0.25 us + 1.9 ns per row of the two operands (a lone CU fetches 40 - 50 GB/s), and its
-// share of the HBM stream (6.9 TB/s over the busy CUs); tiles of 64 or 128 weight rows win while those of 256 leave CUs idle.
-// (bench.py --planner-sweep stream: 1.20 x / 1.18 x the ring kernels, plain / quantising, 3 % behind the best shape, geometric
-// means.  A few experts whose 128 x 128 ring tiles just fill one round are the exception: 8 experts x 0 .. 128 rows x 4096 x 7168
-// 75 against 54 us; at 65 .. 128 rows such problems are even on average.)
-int pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, int cus, int* chunk_len, bool* ahead) {
-  const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
-  const int knob = g_knob[kKnobStream];
-  if (knob == 1 || g_forced_variant >= 0) return kStreamNone;
-  const double span = static_cast<double>(stream_span(M, hint_rows));
-  // Longer experts go to the ring kernels.  Plain product, us here / there, 0 .. cap rows: 32 x 7168 x 2048 cap 256 116 / 141,
-  // cap 384 161 / 166, cap 512 210 / 205; 32 x 7168 x 1024 cap 448 116 / 123; 32 x 4096 x 7168 cap 256 217 / 226, cap 384 305 /
-  // 298; 32 x 2048 x 7168 cap 448 208 / 202.  The quantising epilogue (its row tiles drift apart and fetch weights twice): kStreamActSpan.
-  if (knob == 0 && span > (act ? kStreamActSpan : kblocks <= 24 ? 448 : 256)) return kStreamNone;
-  int best = kStreamNone;
-  double best_us = 0.0;
-  for (int i = 0; i < kStreamCount; ++i) {
-    const StreamDims& d = kStreamDims[i];
-    if (knob >= 2 && i != (knob - 2) % kStreamCount) continue;
-    if ((act && d.bn != 256) || kblocks < d.stages) continue;
-    const int len = stream_chunk_len(kblocks, d.ch, d.stages);
-    if (len <= 0) continue;
-    const double mtiles = span <= d.bm ? 1.0 : 0.5 * (span / d.bm + 1.0);
-    const double tiles = static_cast<double>(G) * mtiles * static_cast<double>(act ? N / 256 : ceil_div(N, d.bn));
-    const double rows = std::min(0.5 * span, static_cast<double>(d.bm));
-    // the row tiles of long experts run in step and share the weights in the L2
-    const double sharing = span > 192 ? mtiles : 1.0;
-    auto step = [&](double busy) { return std::max(0.25 + 0.0019 * (d.bn + rows), d.bn * 128.0 * busy / sharing / 6.9e6); };
-    const double full = std::floor(tiles / cus), rest = tiles - full * cus;
-    const double us = full * (1.0 + kblocks * step(cus)) + (rest > 0.5 ? 1.0 + kblocks * step(rest) : 0.0);
-    if (best == kStreamNone || us < best_us) best = i, best_us = us, *chunk_len = len, *ahead = !act && (knob >= 2 ? knob >= 2 + kStreamCount : span > d.bm);
+// Time of a grouped launch (microseconds, fitted on MI355X to 828 problems of 8 .. 32 experts x 1 .. 960 rows, N = 512 .. 7168, K =
+// 384 .. 7168; rms 8 - 12 %): `start` + rounds of tiles x (`tile` + K blocks x a step of `step` + `row` per activation row of the
+// tile, but no shorter than its share of the stream of weights that the busy CUs draw, bytes per microsecond in `rate`).  Taken
+// over 0.92, 1 and 1.08 times the tile count, which is an estimate itself - except that experts of one row tile have no more
+// than that (32 experts x 0 .. 16 rows x 1024 x 6144 in 64 x 128 tiles are one round of 256, never two).
+struct TileCost {
+  double start, tile, step, row;
+};
+double grouped_us(const TileCost& c, double tiles, bool at_most, int kblocks, int bn, double rows, double sharing, double rate, int cus) {
+  auto step = [&](double busy) { return std::max(c.step + c.row * rows, bn * 128.0 * busy / sharing / rate); };
+  double us = 0.0;
+  for (double spread : {0.92, 1.0, at_most ? 1.0 : 1.08}) {
+    const double full = std::floor(tiles * spread / cus), rest = tiles * spread - full * cus;
+    us += full * (c.tile + kblocks * step(cus)) + (rest > 0.5 ? c.tile + kblocks * step(rest) : 0.0);
   }
+  return c.start + us / 3.0;
+}
+
+// Typical experts of a grouped launch, from the buffers' height M and the caller's hint.
+struct ExpertRows {
+  double span;  // rows that cover nearly all experts
+  double live;  // share of the experts that have a row
+  ExpertRows(int64_t M, int64_t hint_rows) : span(static_cast<double>(stream_span(M, hint_rows))), live(span < static_cast<double>(M) ? 1.0 - std::exp(-0.5 * span) : 1.0) {}
+  double row_tiles(int bm) const { return span <= bm ? 1.0 : 0.5 * (span / bm + 1.0); }
+  double rows(int bm) const { return std::min(0.5 * span, static_cast<double>(bm)); }
+  // the row tiles of long experts run in step and share the weights in the L2
+  double sharing(int bm) const { return span > 192.0 ? row_tiles(bm) : 1.0; }
+};
+
+// The masked layout's ring kernel that make_plan chose (act: the 128 x 256 tiles with the quantising epilogue).
+double masked_ring_us(int variant, int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, int cus) {
+  const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
+  int bm, bn;
+  tile_dims(variant, &bm, &bn);
+  TileCost c = {2.4, 5.0, 0.80, 0.0028};  // 128 x 256
+  if (act) c = {8.8, 0.8, 0.88, 0.0024};
+  else if (variant == kVarPipe128x128) c = {2.3, 3.6, 0.65, 0.0014};
+  else if (variant == kVarPipe256x256) c = {1.5, 7.1, 1.51, 0.0015};
+  const ExpertRows e(M, hint_rows);
+  const bool table = !act && kblocks <= (variant == kVarPipe128x128 ? Pipe128x128T::SCTAB_KB : variant == kVarPipe256x256 ? Pipe256x256T::SCTAB_KB : Pipe128x256w8T::SCTAB_KB);
+  const double tiles = G * e.live * e.row_tiles(bm) * static_cast<double>(act ? N / 256 : ceil_div(N, bn));
+  return (M > kRelayoutMinRows && !table ? 3.5 : 0.0) + grouped_us(c, tiles, e.span <= bm, kblocks, bn, e.rows(bm), e.sharing(bm), 6.2e6, cus);
+}
+
+// Tile shapes of the weight-streaming kernel: fragments read when needed / one step ahead / with the quantising epilogue
+constexpr TileCost kStreamCost[kStreamCount] = {{2.9, 0.5, 0.74, 0.0048}, {2.5, 1.9, 0.69, 0.0066}, {4.1, 0.6, 0.42, 0.0048}, {2.8, 1.7, 0.69, 0.0074}, {4.2, 0.9, 0.38, 0.0016}};
+constexpr TileCost kStreamCostAhead[kStreamCount] = {{}, {3.0, 2.2, 0.71, 0.0041}, {4.9, 1.0, 0.44, 0.0025}, {3.4, 2.2, 0.71, 0.0058}, {5.6, 0.8, 0.30, 0.0012}};
+constexpr TileCost kStreamCostAct[kStreamCount] = {{3.7, 0.6, 0.73, 0.0025}, {3.6, 2.0, 0.72, 0.0044}, {}, {5.2, 2.0, 0.70, 0.0049}, {}};
+
+// How the weight-streaming kernel runs a grouped launch (shape kStreamNone: it does not), from the typical rows of an expert, and
+// whether it is to run at all: other_us is the estimate of the kernel that would run instead (0: none).  The choice is 2.9 % behind
+// the best kernel and shape for the plain product, 2.7 % with the quantising epilogue (geometric means over the problems above; the
+// rule before it, the longest experts by a limit on their rows, 6.6 and 10.9 %).
+// With the quantising epilogue a launch may also run in two: the plain product of every (tile, K slice) first, in any tile shape, then
+// the slices' sum with the activation and the quantiser.  That pays where 256-column tiles leave most CUs idle (it costs 3.8 us +
+// the partial sums' way there and back): 8 experts x ~15 rows x 1792 x 3584 24.9 -> 17.0 us, 32 x ~9 x 512 x 5632 36.9 -> 22.4 us.
+// The plain product gains nothing from slices that smaller tiles do not give it (1.001 x over 195 problems).
+// max_slices: 1 where the bits have to be those of the steps apart (one slice changes nothing about the sums), up to kMaxStreamSlices
+// inside an expert MLP.  all_rows: rows of the partial sums' matrices; slice_floats: room for them.
+StreamPlan pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, int cus, int max_slices, int64_t all_rows, size_t slice_floats,
+                       double other_us) {
+  StreamPlan best;
+  const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
+  const int knob = g_knob[kKnobStream], slice_knob = g_knob[kKnobStreamSlices];
+  if (knob == 1 || g_forced_variant >= 0) return best;
+  const ExpertRows e(M, hint_rows);
+  const double part_bytes = static_cast<double>(G) * std::min(0.5 * e.span, static_cast<double>(M)) * static_cast<double>(N) * 4.0;
+  auto offer = [&](int shape, bool ahead, bool fused_act, int slices) {
+    const StreamDims& d = kStreamDims[shape];
+    const int parts = slices > 0 ? slices : 1;
+    const int kb_min = kblocks / parts, kb_max = static_cast<int>(ceil_div(kblocks, parts));
+    if (kb_min < d.stages) return;
+    if (slices > 0 && static_cast<double>(slices) * static_cast<double>(all_rows) * static_cast<double>(N) > static_cast<double>(slice_floats)) return;
+    const int len = stream_chunk_len(kb_min, kb_max, d.ch, d.stages);
+    if (len <= 0) return;
+    const TileCost& c = fused_act ? kStreamCostAct[shape] : ahead ? kStreamCostAhead[shape] : kStreamCost[shape];
+    const double tiles = G * e.live * e.row_tiles(d.bm) * static_cast<double>(fused_act ? N / 256 : ceil_div(N, d.bn)) * parts;
+    double us = grouped_us(c, tiles, e.span <= d.bm, kb_max, d.bn, e.rows(d.bm), e.sharing(d.bm), 6.9e6, cus);
+    if (slices > 0) us += 3.8 + slices * part_bytes / 2.0e6;
+    if (best.shape == kStreamNone || us < 0.98 * best.us) best.shape = shape, best.us = us, best.chunk_len = len, best.slices = slices, best.ahead = ahead;
+  };
+  for (int i = 0; i < kStreamCount; ++i) {
+    if (knob >= 2 && i != (knob - 2) % kStreamCount) continue;
+    const bool may_ahead = kStreamDims[i].bm > 32 && (knob < 2 || knob >= 2 + kStreamCount);
+    const bool must_ahead = may_ahead && knob >= 2;
+    if (act && kStreamDims[i].bn == 256 && slice_knob == 0) offer(i, false, true, 0);
+    if (act && (knob == 0 || slice_knob > 0))
+      for (int slices = std::max(slice_knob, 1); slices <= (slice_knob > 0 ? slice_knob : max_slices); ++slices) {
+        if (!must_ahead) offer(i, false, false, slices);
+        if (may_ahead) offer(i, true, false, slices);
+      }
+    if (!act && !must_ahead) offer(i, false, false, 0);
+    if (!act && may_ahead) offer(i, true, false, 0);
+  }
+  // Longer experts go to the ring kernels unless the estimates say otherwise (a few of them, or narrow ones).  Plain product, us
+  // here / there, 0 .. cap rows: 32 x 7168 x 2048 cap 256 116 / 141, cap 384 161 / 166, cap 512 210 / 205; 32 x 7168 x 1024 cap 448
+  // 116 / 123; 32 x 4096 x 7168 cap 256 217 / 226, cap 384 305 / 298; 8 x 1152 x 768, ~640 rows 15.6 / 22.8; 8 x 512 x 1920, ~244
+  // rows 14.4 / 20.1.  Quantising: 8 x 512 x 2176, ~137 rows 17.6 / 26.1; 32 x 2048 x 1920, ~181 rows 50 / 61.
+  const bool longer = e.span > (act ? 192 : kblocks <= 24 ? 448 : 256);
+  if (longer && knob == 0 && slice_knob == 0 && other_us > 0.0 && best.us > 0.95 * other_us) best.shape = kStreamNone;
   return best;
+}
+
+// Expert-contiguous rows.  Taller tiles save weight traffic, not time per tile.  Estimates (microseconds, constants as in
+// prefers_128_row_tiles): uniform 128-row tiles take rounds x (5.5 + 1.2 K blocks: most of their weights come from HBM) or, when
+// that is longer, the time to stream every block's weight matrix (6.4 TB/s: neighbouring tiles of an expert share some of it in
+// the L2); the lists take 5 us for their pre-pass + rounds x (11.5 + 1.62 K blocks) or the weights of their tiles at 4.85 TB/s, with
+// as many tiles as pairs of blocks, but at least one per expert.  8 experts, 1408 rows, 4096 x 7168: 107 us with lists, 69 us
+// without; 2432 rows: 106 us with, 128 us without; 32 experts x 128 rows: 183 / 174.
+double contiguous_plain_us(int64_t rows, int64_t N, int64_t K, int cus) {
+  const int64_t nblk = ceil_div(rows, kScaleBlock), kblocks = ceil_div(K, kScaleBlock);
+  const double mat_mb = static_cast<double>(N) * static_cast<double>(K) * 1e-6;
+  return std::max(static_cast<double>(ceil_div(nblk * ceil_div(N, 256), cus)) * (5.5 + 1.2 * static_cast<double>(kblocks)),
+                  static_cast<double>(nblk) * mat_mb / 6.4);
+}
+double contiguous_lists_us(int64_t rows, int64_t N, int64_t K, int G, int cus) {
+  const int64_t nblk = ceil_div(rows, kScaleBlock), kblocks = ceil_div(K, kScaleBlock);
+  const double mat_mb = static_cast<double>(N) * static_cast<double>(K) * 1e-6;
+  const int64_t tall = std::max(ceil_div(nblk, 2), std::min<int64_t>(nblk, G));
+  return 5.0 + std::max(static_cast<double>(ceil_div(tall * ceil_div(N, 256), cus)) * (11.5 + 1.62 * static_cast<double>(kblocks)),
+                        static_cast<double>(tall) * mat_mb / 4.85);
+}
+
+// (act: the quantising epilogue exists for the lists only)
+double contiguous_us(int64_t rows, int64_t N, int64_t K, int G, bool act, int cus) {
+  const double lists_us = contiguous_lists_us(rows, N, K, G, cus);
+  return act ? lists_us : std::min(lists_us, contiguous_plain_us(rows, N, K, cus));
+}
+
+// A step of an expert MLP on expert-contiguous rows (act: the gate/up projection, N = 2 I): 1 = the weight-streaming kernel on the
+// experts' row ranges, 2 = the expert-contiguous kernels on whole blocks (act: from tile lists), 0 = neither.
+int expert_form(int64_t rows, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, size_t ws_bytes, int cus) {
+  const size_t room = ws_bytes > DLB_WS_COUNTER_BYTES ? ws_bytes - DLB_WS_COUNTER_BYTES : 0;
+  const int64_t nblk = ceil_div(rows, kScaleBlock);
+  const bool shape_ok = K > 0 && K % kScaleBlock == 0 && K < (1ll << 24) && rows < (1ll << 31) && (!act || (N % (2 * kScaleBlock) == 0 && N * K < (1ll << 32)));
+  if (!shape_ok || g_forced_variant >= 0) return 0;
+  const bool lists = g_knob[kKnobTileList] != 2 && nblk <= kTileListMaxBlocks && tile_list_bytes(nblk) <= room;
+  const double other_us = contiguous_us(rows, N, K, G, act, cus);
+  if (pick_stream(rows, N, K, G, hint_rows, act, cus, kMaxStreamSlices, rows, room / sizeof(float), other_us).shape != kStreamNone) return 1;
+  return act && !lists ? 0 : 2;
 }
 
 // overlay: the kernel whose waves split K may take the launch over from the planned variant.
 // fused_act: the launch is one of the gate/up GEMMs with the activation in its epilogue (their kernels take no scale table)
 Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as_sm, int64_t as_sk, bool have_ws,
-                 size_t ws_bytes, int cus, bool gather_scales = false, bool fused_act = false, int64_t hint_rows = -1, bool overlay = true) {
+                 size_t ws_bytes, int cus, bool gather_scales = false, bool fused_act = false, int64_t hint_rows = -1, bool overlay = true, int max_slices = 1) {
   Resolved r{};
   const int64_t kblocks = ceil_div(K, kScaleBlock);
   const int64_t groups = mode == kMasked ? G : 1;  // a_s is per expert only in the masked layout; contiguous rows are one matrix
@@ -830,7 +980,6 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
   const bool usable_ws = have_ws && ws_bytes > DLB_WS_COUNTER_BYTES;
   r.pl = make_plan(mode, rows, N, K, cus, usable_ws ? ws_bytes : 0, dma_ok, G, hint_rows, fused_act || gather_scales);
   const Plan& pl = r.pl;
-  r.stream = kStreamNone;
   r.wavek = kWaveKNone;
   // (its scale table is fetched through 32-bit byte offsets from the tile's first row; tiles have up to 64 rows)
   const bool table_near = dma_ok && as_sk < (1ll << 20) && 63 * as_sm + (kblocks - 1) * as_sk < (1ll << 30);
@@ -845,7 +994,8 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
     return r;
   }
   if (mode == kMasked && dma_ok && K % kScaleBlock == 0 && K > 0 && static_cast<int64_t>(G) * rows < (1ll << 31))
-    r.stream = pick_stream(rows, N, K, G, hint_rows, fused_act, cus, &r.chunk_len, &r.ahead);
+    r.stream = pick_stream(rows, N, K, G, hint_rows, fused_act, cus, max_slices, rows * G, usable_ws ? (ws_bytes - DLB_WS_COUNTER_BYTES) / sizeof(float) : 0,
+                           masked_ring_us(pl.variant, rows, N, K, G, hint_rows, fused_act, cus));
   const int want = usable_ws ? pl.splitk : 1;
   r.kb_per_split = static_cast<int>(ceil_div(kblocks > 0 ? kblocks : 1, want));
   r.splitk = static_cast<int>(ceil_div(kblocks > 0 ? kblocks : 1, r.kb_per_split));  // no empty slice
@@ -853,24 +1003,9 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
   if (mode == kContiguous && pl.variant == kVarPipe128x256w8 && g_forced_variant < 0 && usable_ws && kblocks > 0) {
     const int64_t nblk = ceil_div(rows, kScaleBlock);
     const size_t bytes = tile_list_bytes(nblk);
-    // Taller tiles save weight traffic, not time per tile.  Estimates (microseconds, constants as in
-    // prefers_128_row_tiles): uniform 128-row tiles take rounds x (5.5 + 1.2 K blocks: most of their weights come from HBM) or, when that is longer, the time
-    // to stream every block's weight matrix (6.4 TB/s: neighbouring tiles of an expert share some of it in the L2);
-    // the lists take 5 us for their pre-pass + rounds x (11.5 + 1.62 K blocks) or the weights of their tiles at
-    // 4.85 TB/s, with as many tiles as pairs of blocks, but at least one per expert.  8 experts, 1408 rows, 4096 x
-    // 7168: 107 us with lists, 69 us without; 2432 rows: 106 us with, 128 us without; 32 experts x 128 rows: 183 / 174.
-    // The fused epilogues exist for the list kernel only.
+    // (the fused epilogues exist for the list kernel only)
     bool worth_it = fused_act || gather_scales || g_knob[kKnobTileList] == 1;
-    if (!worth_it && g_knob[kKnobTileList] != 2 && nblk > G) {
-      const int64_t tn = ceil_div(N, 256);
-      const double mat_mb = static_cast<double>(N) * static_cast<double>(K) * 1e-6;
-      const double plain_us = std::max(static_cast<double>(ceil_div(nblk * tn, cus)) * (5.5 + 1.2 * static_cast<double>(kblocks)),
-                                       static_cast<double>(nblk) * mat_mb / 6.4);
-      const int64_t tall = std::max(ceil_div(nblk, 2), std::min<int64_t>(nblk, G));
-      const double list_us = 5.0 + std::max(static_cast<double>(ceil_div(tall * tn, cus)) * (11.5 + 1.62 * static_cast<double>(kblocks)),
-                                            static_cast<double>(tall) * mat_mb / 4.85);
-      worth_it = list_us < plain_us;
-    }
+    if (!worth_it && g_knob[kKnobTileList] != 2 && nblk > G) worth_it = contiguous_lists_us(rows, N, K, G, cus) < contiguous_plain_us(rows, N, K, cus);
     if (worth_it && nblk <= kTileListMaxBlocks && DLB_WS_COUNTER_BYTES + bytes <= ws_bytes) r.tile_list = true, r.nblk = nblk, r.ws_used = bytes;
   }
   // A tile's row-major scales come once, into a table in LDS, where its K range fits what the ring leaves of the LDS: no re-layout
@@ -890,9 +1025,9 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
       default: return false;
     }
   };
-  r.sctab = r.stream == kStreamNone && table_fits(r.kb_per_split);
+  r.sctab = r.stream.shape == kStreamNone && table_fits(r.kb_per_split);
   // gather_scales: the re-layout pass also brings the rows into the GEMM's order, so it runs whatever the strides
-  if (is_pipelined(pl.variant) && usable_ws && !r.sctab && r.stream == kStreamNone &&
+  if (is_pipelined(pl.variant) && usable_ws && !r.sctab && r.stream.shape == kStreamNone &&
       (gather_scales ? kblocks > 0 : as_sk == 1 && as_sm > 1 && kblocks > 1 && rows > kRelayoutMinRows)) {
     // row-major activation scales: re-lay them rows-contiguous in the workspace first (a few microseconds) so the
     // GEMM fetches 8 cache lines of scales per K step and tile instead of 256.  Up to 128 rows the extra launch costs
@@ -969,6 +1104,7 @@ struct Problem {
   float act_eps = 0.f;
   bool act = false;
   int64_t hint_rows = -1;  // masked layout: the caller's expected_m
+  bool mlp = false;        // a step of an expert MLP: K may be sliced, and where the steps apart are faster the call is declined
   bool list_there = false;  // contiguous: the workspace still holds the tile lists of these rows
 };
 
@@ -990,6 +1126,9 @@ struct RaggedProblem {
   int64_t act_s_sm, act_s_sk;
   float eps;
   hipStream_t stream;
+  void* ws = nullptr;  // or NULL: nothing in two launches
+  size_t ws_bytes = 0;
+  bool mlp = false;
 };
 
 int run_ragged(const RaggedProblem& pr) {
@@ -1009,14 +1148,16 @@ int run_ragged(const RaggedProblem& pr) {
   const int cus = device_cu_count(&dev);
   if (cus < 0) return fail(DLB_ERR_LAUNCH, "hipGetDevice failed");
   const int64_t kblocks = ceil_div(pr.K, kScaleBlock);
-  int chunk_len = 0;
-  bool ahead = false;
-  int shape = kStreamNone;
+  if (pr.ws && misaligned(pr.ws, 16)) return fail(DLB_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
+  const bool usable_ws = pr.ws && pr.ws_bytes > DLB_WS_COUNTER_BYTES;
+  StreamPlan sp;
   const bool fits = pr.K > 0 && pr.K % kScaleBlock == 0 && pr.K < (1ll << 24) && pr.as_sm < (1ll << 21) && pr.M_sum < (1ll << 31) &&
                     pr.N < (1ll << 31) && (!pr.act || (pr.N % (2 * kScaleBlock) == 0 && pr.N * pr.K < (1ll << 32))) &&
                     (!pr.a_rows || (pr.act && pr.a_src_rows > 0 && pr.a_src_rows * pr.K < (1ll << 31)));
-  if (fits) shape = pick_stream(pr.M_sum, pr.N, pr.K, pr.G, pr.hint_rows, pr.act, cus, &chunk_len, &ahead);
-  if (shape == kStreamNone)
+  if (fits)
+    sp = pick_stream(pr.M_sum, pr.N, pr.K, pr.G, pr.hint_rows, pr.act, cus, pr.mlp ? kMaxStreamSlices : 1, pr.M_sum, usable_ws ? (pr.ws_bytes - DLB_WS_COUNTER_BYTES) / sizeof(float) : 0,
+                     contiguous_us(pr.M_sum, pr.N, pr.K, pr.G, pr.act, cus));
+  if (sp.shape == kStreamNone)
     return fail(DLB_ERR_BAD_SHAPE, "the weight-streaming kernel does not take this problem (N=%lld K=%lld, about %lld rows per expert)",
                 (long long)pr.N, (long long)pr.K, (long long)pr.hint_rows);
   Args ar;
@@ -1040,8 +1181,6 @@ int run_ragged(const RaggedProblem& pr) {
   ar.as_sk = pr.as_sk;
   ar.b_gs = pr.N * pr.K;
   ar.bs_gs = static_cast<int64_t>(ar.nblocks) * kblocks;
-  ar.chunk_len = chunk_len;
-  ar.tiles_n = static_cast<int>(pr.act ? pr.N / 256 : ceil_div(pr.N, kStreamDims[shape].bn));
   ar.out_f32 = pr.out_dtype == DLB_OUT_F32;
   ar.act_s = pr.act_s;
   ar.act_s_sm = pr.act_s_sm;
@@ -1049,15 +1188,18 @@ int run_ragged(const RaggedProblem& pr) {
   ar.act_eps = pr.eps;
   ar.act_cols = static_cast<int>(pr.N / 2);
   ar.act_q_stride = pr.N / 2;
-  const int64_t worst = static_cast<int64_t>(ar.tiles_n) * (pr.G + pr.M_sum / kStreamDims[shape].bm);
-  const int grid = static_cast<int>(ceil_div(worst < cus ? worst : cus, 32) * 32);
-  hipError_t e;
-  if (pr.act)
-    e = pr.a_rows ? launch_stream_shape<kSiluQuant, true>(shape, false, ar, grid, dev, pr.stream) : launch_stream_shape<kSiluQuant, false>(shape, false, ar, grid, dev, pr.stream);
-  else
-    e = launch_stream_shape<kStoreProduct, false>(shape, ahead, ar, grid, dev, pr.stream);
+  if (usable_ws) ar.ws = reinterpret_cast<float*>(static_cast<char*>(pr.ws) + DLB_WS_COUNTER_BYTES);
+  const WorkspaceLock lock(pr.ws);
+  const hipError_t e = launch_stream_plan(sp, pr.act ? kSiluQuant : kStoreProduct, ar, pr.G + pr.M_sum / kStreamDims[sp.shape].bm,
+                                          stream_span(pr.M_sum, pr.hint_rows), pr.M_sum, cus, dev, pr.stream);
   if (e != hipSuccess) return fail(DLB_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
   return DLB_OK;
+}
+
+// Masked gate/up projection with the epilogue fused (rs) or the plain product and the activation apart?  Several hundred rows per
+// expert: the plain product's taller tiles (32 experts x ~520 rows: 619 against 678 us).
+bool steps_apart(const Resolved& rs, int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, size_t ws_bytes, int cus) {
+  return rs.stream.shape == kStreamNone && make_plan(kMasked, M, N, K, cus, ws_bytes, true, G, hint_rows).variant != kVarPipe128x256w8;
 }
 
 // Argument checks that need no device.  Returns DLB_OK with *empty set when there is nothing to compute.
@@ -1116,8 +1258,10 @@ int run(const Problem& pr) {
 
   if (pr.ws && misaligned(pr.ws, 16)) return fail(DLB_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
   const Resolved rs = resolve(pr.mode, pr.rows, pr.N, pr.K, pr.G, pr.as_sm, pr.as_sk, pr.ws != nullptr, pr.ws_bytes, cus,
-                              pr.a_rows != nullptr, pr.act, pr.hint_rows);
+                              pr.a_rows != nullptr, pr.act, pr.hint_rows, true, pr.mlp ? kMaxStreamSlices : 1);
   const Plan& pl = rs.pl;
+  if (pr.mlp && pr.mode == kMasked && steps_apart(rs, pr.rows, pr.N, pr.K, pr.G, pr.hint_rows, pr.ws ? pr.ws_bytes : 0, cus))
+    return fail(DLB_ERR_BAD_SHAPE, "GEMM, activation and quantiser apart are the faster way");
   // everything that can refuse the launch is checked before the first pre-pass kernel is enqueued
   if (rs.grid > (1ll << 30)) return fail(DLB_ERR_BAD_SHAPE, "too many tiles (%lld)", (long long)rs.grid);
   if (pl.variant == kVarExact && pr.mode != kDense) return fail(DLB_ERR_BAD_SHAPE, "exact path is dense only");
@@ -1125,7 +1269,7 @@ int run(const Problem& pr) {
     // the fused epilogue exists for the tile-list kernel (contiguous) and the 128 x 256 ring kernel (masked) only:
     // whole 128-blocks of K and of the output, a workspace for the list, no forced variant; anything else is the
     // caller's cue to run the GEMM and the activation apart
-    const bool kernel_ok = pr.mode == kContiguous ? rs.tile_list : pr.mode == kMasked && (rs.stream != kStreamNone || pl.variant == kVarPipe128x256w8);
+    const bool kernel_ok = pr.mode == kContiguous ? rs.tile_list : pr.mode == kMasked && (rs.stream.shape != kStreamNone || pl.variant == kVarPipe128x256w8);
     if (!kernel_ok || pr.K % kScaleBlock != 0 || pr.N % (2 * kScaleBlock) != 0 || pr.N * pr.K >= (1ll << 32))
       return fail(DLB_ERR_BAD_SHAPE,
                   "fused activation needs K %% 128 == 0, N %% 256 == 0, N K < 2^32%s (N=%lld K=%lld)",
@@ -1189,7 +1333,6 @@ int run(const Problem& pr) {
   ar.fused_reduce = rs.fused ? 1 : 0;
   ar.spin_limit = g_knob[kKnobSpinLimit] > 0 ? g_knob[kKnobSpinLimit] - 1 : kDefaultSpinLimit;
   ar.sct_pitch = rs.sct_pitch;
-  ar.chunk_len = rs.chunk_len;
   const bool tile_list = rs.tile_list;
 
   // The main kernel of the call.  With g_prepare_only set it only raises the kernel's dynamic-LDS limit (the one
@@ -1221,12 +1364,10 @@ int run(const Problem& pr) {
       return pr.K % kScaleBlock != 0 ? launch_wavek<true>(rs.wavek, ar, static_cast<int>(rs.grid), dev, pr.stream)
                                      : launch_wavek<false>(rs.wavek, ar, static_cast<int>(rs.grid), dev, pr.stream);
     }
-    if (rs.stream != kStreamNone) {
-      ar.tiles_n = static_cast<int>(pr.act ? pr.N / 256 : ceil_div(pr.N, kStreamDims[rs.stream].bn));
-      const int64_t worst = static_cast<int64_t>(ar.tiles_n) * pr.G * ceil_div(pr.rows, kStreamDims[rs.stream].bm);
-      const int grid = static_cast<int>(ceil_div(worst < cus ? worst : cus, 32) * 32);  // tiles are dealt to the XCDs four at a time
-      return pr.act ? launch_stream_shape<kSiluQuantMasked, false>(rs.stream, false, ar, grid, dev, pr.stream)
-                    : launch_stream_shape<kStoreProduct, false>(rs.stream, rs.ahead, ar, grid, dev, pr.stream);
+    if (rs.stream.shape != kStreamNone) {
+      const int64_t worst_rows = pr.G * ceil_div(pr.rows, kStreamDims[rs.stream.shape].bm);
+      return launch_stream_plan(rs.stream, pr.act ? kSiluQuantMasked : kStoreProduct, ar, worst_rows, stream_span(pr.rows, pr.hint_rows), pr.G * pr.rows,
+                                cus, dev, pr.stream);
     }
     const int g = static_cast<int>(rs.grid);
     const int g_dense = rs.resident ? cus : g;
@@ -1568,6 +1709,52 @@ int dlb_fp8_gemm_grouped_ragged_silu_quant(const void* a, const void* b, const f
   return dlb::run_ragged(pr);
 }
 
+int dlb_expert_gate_up_ragged(const void* a, const void* b, const float* a_s, const float* b_s, void* out_q, float* out_s, const int32_t* row_start,
+                              const int32_t* row_end, const int32_t* a_row_index, int64_t a_rows, int32_t expected_m, int64_t M_sum, int64_t N,
+                              int64_t K, int32_t G, int64_t as_stride_m, int64_t as_stride_k, int64_t os_stride_m, int64_t os_stride_k, float eps,
+                              void* workspace, size_t workspace_bytes, void* stream) {
+  dlb::RaggedProblem pr{a, b, a_s, b_s, out_q, row_start, row_end, a_row_index, a_rows, M_sum, N, K, G, expected_m, as_stride_m, as_stride_k,
+                        DLB_OUT_BF16, true, out_s, os_stride_m, os_stride_k, eps, static_cast<hipStream_t>(stream), workspace, workspace_bytes, true};
+  return dlb::run_ragged(pr);
+}
+
+int dlb_expert_gate_up_masked(const void* a, const void* b, const float* a_s, const float* b_s, void* out_q, float* out_s, const int32_t* masked_m,
+                              int32_t expected_m, int64_t M_max, int64_t N, int64_t K, int32_t G, int64_t as_stride_g, int64_t as_stride_m,
+                              int64_t as_stride_k, int64_t os_stride_g, int64_t os_stride_m, int64_t os_stride_k, float eps, void* workspace,
+                              size_t workspace_bytes, void* stream) {
+  dlb::Problem pr{dlb::kMasked, a, b, a_s, b_s, out_q, masked_m, M_max, N, K, G, as_stride_g, as_stride_m, as_stride_k,
+                  DLB_OUT_BF16, workspace, workspace_bytes, static_cast<hipStream_t>(stream)};
+  pr.act = true;
+  pr.mlp = true;
+  pr.act_s = out_s;
+  pr.act_s_sg = os_stride_g;
+  pr.act_s_sm = os_stride_m;
+  pr.act_s_sk = os_stride_k;
+  pr.act_eps = eps;
+  pr.hint_rows = expected_m;
+  if (M_max > 0 && N > 0 && G > 0 && !out_s) return dlb::fail(DLB_ERR_NULL_POINTER, "out_s is NULL");
+  return dlb::run(pr);
+}
+
+int dlb_expert_plan(int mode, int64_t rows, int64_t N, int64_t K, int32_t G, int32_t expected_m, int quantising, size_t workspace_bytes, int compute_units,
+                    int* form) {
+  dlb::clear_error();
+  const int64_t lim = (1ll << 31) - 1024;
+  if (rows < 0 || N < 0 || K < 0 || G < 0 || rows > lim || N > lim || K > lim || compute_units <= 0)
+    return dlb::fail(DLB_ERR_BAD_SHAPE, "bad dimension (rows=%lld, N=%lld, K=%lld, G=%d)", (long long)rows, (long long)N, (long long)K, G);
+  if (mode != dlb::kContiguous && mode != dlb::kMasked) return dlb::fail(DLB_ERR_BAD_SHAPE, "mode %d is not 1 (contiguous) or 2 (masked)", mode);
+  if (!form) return DLB_OK;
+  if (mode == dlb::kContiguous) {
+    *form = dlb::expert_form(rows, N, K, G, expected_m, quantising != 0, workspace_bytes, compute_units);
+  } else {
+    const dlb::Resolved rs = dlb::resolve(dlb::kMasked, rows, N, K, G, dlb::ceil_div(K, dlb::kScaleBlock), 1, workspace_bytes > 0, workspace_bytes,
+                                          compute_units, false, quantising != 0, expected_m, true, dlb::kMaxStreamSlices);
+    const bool shape_ok = K > 0 && K % dlb::kScaleBlock == 0 && N % (2 * dlb::kScaleBlock) == 0 && N * K < (1ll << 32);
+    *form = shape_ok && dlb::g_forced_variant < 0 && !dlb::steps_apart(rs, rows, N, K, G, expected_m, workspace_bytes, compute_units) ? 1 : 0;
+  }
+  return DLB_OK;
+}
+
 int dlb_fp8_quant_group(const void* x, int x_dtype, void* q, float* s, int64_t rows, int64_t K, int64_t group_size,
                         int64_t x_row_stride, int64_t s_stride_m, int64_t s_stride_k, float eps, void* stream) {
   using namespace dlb;
@@ -1703,10 +1890,10 @@ int dlb_fp8_gemm_plan_stream(int64_t rows, int64_t N, int64_t K, int32_t G, int3
     return dlb::fail(DLB_ERR_BAD_SHAPE, "bad dimension (rows=%lld, N=%lld, K=%lld, G=%d)", (long long)rows, (long long)N, (long long)K, G);
   const bool act = quantising != 0;
   const dlb::Resolved rs = dlb::resolve(dlb::kMasked, rows, N, K, G, dlb::ceil_div(K, dlb::kScaleBlock), 1, false, 0, compute_units, false, act, expected_m);
-  const bool on = rs.stream != dlb::kStreamNone && (!act || (N % (2 * dlb::kScaleBlock) == 0 && N * K < (1ll << 32)));
-  if (tile_rows) *tile_rows = on ? dlb::kStreamDims[rs.stream].bm : 0;
-  if (tile_columns) *tile_columns = on ? dlb::kStreamDims[rs.stream].bn : 0;
-  if (ahead) *ahead = on && rs.ahead ? 1 : 0;
+  const bool on = rs.stream.shape != dlb::kStreamNone && (!act || (N % (2 * dlb::kScaleBlock) == 0 && N * K < (1ll << 32)));
+  if (tile_rows) *tile_rows = on ? dlb::kStreamDims[rs.stream.shape].bm : 0;
+  if (tile_columns) *tile_columns = on ? dlb::kStreamDims[rs.stream.shape].bn : 0;
+  if (ahead) *ahead = on && rs.stream.ahead ? 1 : 0;
   return DLB_OK;
 }
 

@@ -30,8 +30,9 @@
 namespace dlb {
 
 // What the epilogue does: store the product; silu(gate) * up + quantise with one rounding (expert-contiguous rows) or
-// with the masked activation's two (dlblas/kernels/moe.py:256-257).
-enum StreamEpilogue : int { kStoreProduct = 0, kSiluQuant = 1, kSiluQuantMasked = 2 };
+// with the masked activation's two (dlblas/kernels/moe.py:256-257); or leave the fp32 sums of one K slice of the product, for the
+// reduction kernels at the end of this file.
+enum StreamEpilogue : int { kStoreProduct = 0, kSiluQuant = 1, kSiluQuantMasked = 2, kStoreSlice = 3 };
 
 template <int WGM_, int WGN_, int MF_, int NF_, int STAGES_, int CH_>
 struct StreamCfg {
@@ -99,7 +100,8 @@ struct ExpertWalk {
 template <class Cfg, int EPI, bool GATHER, bool AHEAD>
 __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, MF = Cfg::MF, NF = Cfg::NF, WAVES = Cfg::WAVES, WGM = Cfg::WGM, STAGES = Cfg::STAGES;
-  constexpr bool kAct = EPI != kStoreProduct;
+  constexpr bool kAct = EPI == kSiluQuant || EPI == kSiluQuantMasked;
+  constexpr bool kSliced = EPI == kStoreSlice;
   static_assert(!kAct || BN == 256, "a quantisation group is the 128 output columns of 256 weight rows");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int lane = threadIdx.x & 63;
@@ -107,7 +109,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
   const int l32 = lane & 31, h = lane >> 5;
   const int wrow = wave / Cfg::WGN;  // the wave's fragment mi is the tile's fragment mi WGM + wrow: wave rows share short tiles evenly
   const LaneChunks lc = make_lane_chunks(l32, h);
-  const int nk = p.kblocks;
+  const int slices = kSliced ? p.splitk : 1;
   const int grid = static_cast<int>(gridDim.x);
   const int bid = static_cast<int>(blockIdx.x);
   // the row tiles of an expert are adjacent in the order; of every 32 consecutive tiles an XCD takes 4 consecutive ones
@@ -131,7 +133,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     ew.row0 = row0;
     ew.rows = rows;
     ew.mtiles = (rows + BM - 1) / BM;
-    int incl = ew.mtiles * p.tiles_n;
+    int incl = ew.mtiles * p.tiles_n * slices;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const int up = __shfl_up(incl, off);
@@ -144,8 +146,11 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
   // one tile: wave-uniform
   struct Tile {
     int g, row, rows, n0;  // expert, first row (of a / of the output), valid rows, first weight row / output column
+    int slice, kb0, kb1;   // K slice: blocks [kb0, kb1)
     bool ok;
   };
+  auto first_kb = [&](const Tile& t) __attribute__((always_inline)) { return kSliced ? t.kb0 : 0; };
+  auto end_kb = [&](const Tile& t) __attribute__((always_inline)) { return kSliced ? t.kb1 : p.kblocks; };
   auto locate = [&](int id) {
     Tile t{};
     while (id >= ew.base + ew.total) {
@@ -155,7 +160,16 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     const int rel = id - ew.base;
     const int i = __builtin_ctzll(__ballot(ew.incl > rel));
     const int mtiles = __builtin_amdgcn_readlane(ew.mtiles, i);
-    const int local = rel - (__builtin_amdgcn_readlane(ew.incl, i) - mtiles * p.tiles_n);
+    const int per_slice = mtiles * p.tiles_n;
+    int local = rel - (__builtin_amdgcn_readlane(ew.incl, i) - per_slice * slices);
+    if (kSliced) {
+      // K slices of equal length, the first few one block longer
+      const int longer = p.kblocks - slices * p.kb_per_split;
+      t.slice = local / per_slice;
+      local -= t.slice * per_slice;
+      t.kb0 = t.slice * p.kb_per_split + min(t.slice, longer);
+      t.kb1 = t.kb0 + p.kb_per_split + (t.slice < longer ? 1 : 0);
+    }
     const int nt = local / mtiles, mt = local - nt * mtiles;
     t.g = ew.first + i;
     // the row tiles of an expert are equally high (in fragments): they run side by side and share its weights in the L2
@@ -188,7 +202,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
   const int tab_rs = tab_by_row ? Cfg::PITCH : 1, tab_js = tab_by_row ? 1 : BM;
 
   Tile it;                      // the tile the issue side works on
-  int it_seq = 0, it_kb = 0;    // its number in this workgroup's sequence; its next K block
+  int it_seq = 0, it_kb = 0;    // its number in this workgroup's sequence; its next K block (counted from the first of all slices)
   int it_stage = 0, it_tab = 0, it_chunk_kb = 0;
   __amdgpu_buffer_rsrc_t a_src, b_src;
   const float* as_src = nullptr;
@@ -196,8 +210,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
   auto enter_tile = [&]() {
     it = locate(it_seq * grid + slot0);
     ++it_seq;
-    it_kb = 0;
-    it_chunk_kb = 0;
+    it_kb = it_chunk_kb = first_kb(it);
     if (!it.ok) return;
     const uint8_t* bg = p.b + static_cast<int64_t>(it.g) * p.b_gs + static_cast<int64_t>(it.n0) * p.K;
     b_src = make_rsrc(bg, static_cast<uint32_t>(kAct ? p.N - it.n0 : min(BN, p.N - it.n0)) * uK);
@@ -229,12 +242,10 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     ++it_kb;
     it_stage = it_stage + 1 == STAGES ? 0 : it_stage + 1;
   };
-  auto issue_step = [&]() {
-    if (it.ok && it_kb == nk) enter_tile();
-    if (!it.ok) return;
+  auto open_chunk = [&]() {
     if (it_kb == it_chunk_kb) {
       // this step opens a chunk of the scale table
-      const int len = min(p.chunk_len, nk - it_kb);
+      const int len = min(p.chunk_len, end_kb(it) - it_kb);
       uint8_t* tab = smem + Cfg::TAB_OFF + it_tab * Cfg::TAB_BYTES;
 #pragma unroll
       for (int i = 0; i < Cfg::TAB_INST; ++i) {
@@ -250,6 +261,11 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
       it_tab ^= 1;
       it_chunk_kb += p.chunk_len;
     }
+  };
+  auto issue_step = [&]() {
+    if (it.ok && it_kb == end_kb(it)) enter_tile();
+    if (!it.ok) return;
+    open_chunk();
     issue_loads();
   };
 
@@ -257,8 +273,14 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
   enter_tile();
   if (!it.ok) return;
   Tile ct = it;  // the tile the compute side works on
+  // a tile has at least STAGES K blocks and a chunk at least STAGES - 1
+  open_chunk();
 #pragma unroll
-  for (int s = 0; s < (AHEAD ? STAGES : STAGES - 1); ++s) issue_step();
+  for (int s = 0; s < STAGES - 1; ++s) issue_loads();
+  if (AHEAD) {
+    open_chunk();
+    issue_loads();
+  }
 
   // ---- compute side ------------------------------------------------------------------------------------------------
   // AHEAD: the fragments of a K block are in registers when its step begins; each is replaced by the next block's as soon as
@@ -292,9 +314,9 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     w[ni][1] = lds_read_frag32(smem, base + frag_off[ni], lc, 1);
   };
   auto next_stage = [&]() __attribute__((always_inline)) { base = base + Cfg::STAGE_BYTES == STAGES * Cfg::STAGE_BYTES ? 0 : base + Cfg::STAGE_BYTES; };
-  auto enter_block = [&](int kb) {  // block kb of a tile is the one whose fragments are read next
+  auto enter_block = [&](int kb, bool first) {  // block kb is the one whose fragments are read next; first: of its tile
     ++tab_kb;
-    if (kb == 0) chunk_end = 0;
+    if (first) chunk_end = kb;
     if (kb == chunk_end) {
       tab_ptr = reinterpret_cast<const float*>(smem + Cfg::TAB_OFF + tab * Cfg::TAB_BYTES);
       tab ^= 1;
@@ -307,8 +329,8 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
   auto enter_scales = [&](const Tile& t) {
     const float* bs_g = p.b_s + static_cast<int64_t>(t.g) * p.bs_gs;
     const int nb0 = kAct ? t.n0 / kScaleBlock : min((t.n0 + wn0) / kScaleBlock, p.nblocks - 1);
-    bs0 = (const_float_ptr_t)(bs_g + static_cast<int64_t>(nb0) * nk);
-    bs1 = (const_float_ptr_t)(bs_g + static_cast<int64_t>(kAct ? nb0 + p.act_cols / kScaleBlock : nb0) * nk);
+    bs0 = (const_float_ptr_t)(bs_g + static_cast<int64_t>(nb0) * p.kblocks);
+    bs1 = (const_float_ptr_t)(bs_g + static_cast<int64_t>(kAct ? nb0 + p.act_cols / kScaleBlock : nb0) * p.kblocks);
   };
   auto multiply = [&](int ni, int mi) __attribute__((always_inline)) {
     v16f z;
@@ -326,10 +348,10 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
 
   if constexpr (AHEAD) {
     enter_scales(ct);
-    sb0 = bs0[0], sb1 = bs1[0];
+    sb0 = bs0[first_kb(ct)], sb1 = bs1[first_kb(ct)];
     wait_vmcnt<(STAGES - 1) * Cfg::L>();
     lds_barrier();
-    enter_block(0);
+    enter_block(first_kb(ct), true);
 #pragma unroll
     for (int mi = 0; mi < MF; ++mi)
       if (frag_row(mi) < ct.rows) read_x(mi);
@@ -391,7 +413,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
   while (true) {
     if (!AHEAD) {
       enter_scales(ct);
-      sb0 = bs0[0], sb1 = bs1[0];
+      sb0 = bs0[first_kb(ct)], sb1 = bs1[first_kb(ct)];
     }
 #pragma unroll
     for (int mi = 0; mi < MF; ++mi)
@@ -401,9 +423,9 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
         for (int t = 0; t < 16; ++t) acc[mi][ni][t] = 0.f;
     const bool full = AHEAD && frag_row(MF - 1) < ct.rows;
 
-    for (int kb = 0; AHEAD && kb < nk; ++kb) {
+    for (int kb = first_kb(ct); AHEAD && kb < end_kb(ct); ++kb) {
       if (full && it.ok) {
-        const int n = min(min(nk, it_chunk_kb) - it_kb, min(nk, chunk_end) - 1 - kb);
+        const int n = min(min(end_kb(it), it_chunk_kb) - it_kb, min(end_kb(ct), chunk_end) - 1 - kb);
         if (n > 0) {
           run_fast(kb, n);
           kb += n;
@@ -424,19 +446,21 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
         }
         if (mi == 0) {
           // younger than the next block's loads: those of STAGES - 2 steps, fewer at the end of the last tile
-          wait_groups<Cfg::L, STAGES - 2>(it.ok ? STAGES - 2 : nk - 2 - kb);
+          wait_groups<Cfg::L, STAGES - 2>(it.ok ? STAGES - 2 : end_kb(ct) - 2 - kb);
           lds_barrier();
           issue_step();
           next_stage();
-          if (kb + 1 < nk) {
+          const bool next_tile = kb + 1 == end_kb(ct);
+          if (!next_tile) {
             kb_n = kb + 1;
             rows_n = ct.rows;
-          } else {
-            // the issue side is in the next tile: nk >= STAGES
-            rows_n = it.ok ? it.rows : 0;
-            if (it.ok) enter_scales(it);
+          } else if (it.ok) {
+            // the issue side is in the next tile: every tile has at least STAGES K blocks
+            kb_n = first_kb(it);
+            rows_n = it.rows;
+            enter_scales(it);
           }
-          enter_block(kb_n);
+          enter_block(kb_n, next_tile);
           sb0 = bs0[kb_n];
           sb1 = bs1[kb_n];
         }
@@ -449,12 +473,12 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     }
 
     if constexpr (!AHEAD) {
-      for (int kb = 0; kb < nk; ++kb) {
+      for (int kb = first_kb(ct); kb < end_kb(ct); ++kb) {
         // the loads of this step have landed: behind them at most the groups of the next STAGES - 2 steps are out
-        wait_groups<Cfg::L, STAGES - 2>(it.ok ? STAGES - 2 : nk - 1 - kb);
+        wait_groups<Cfg::L, STAGES - 2>(it.ok ? STAGES - 2 : end_kb(ct) - 1 - kb);
         lds_barrier();  // ... those of every wave, and nobody reads the stage before this one any more
         issue_step();
-        enter_block(kb);
+        enter_block(kb, kb == first_kb(ct));
         if (WGM == 1 || frag_row(0) < ct.rows) {
           v8i wf[NF][2];
 #pragma unroll
@@ -480,7 +504,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
             }
           }
         }
-        const int kn = min(kb + 1, nk - 1);
+        const int kn = min(kb + 1, end_kb(ct) - 1);
         sb0 = bs0[kn];
         sb1 = bs1[kn];
         next_stage();
@@ -546,45 +570,179 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
         }
       }
     } else {
+      // F32: the output type; INSIDE: no column of the wave's tile lies past N, so no store has a tail
+      auto store_tile = [&](auto f32, auto inside) __attribute__((always_inline)) {
+        constexpr bool F32 = decltype(f32)::value, INSIDE = decltype(inside)::value;
 #pragma unroll
-      for (int mi = 0; mi < MF; ++mi) {
-        const int row = frag_row(mi) + l32;
-        const bool live = row < ct.rows;
-        char* c_row = static_cast<char*>(p.c) + static_cast<int64_t>(ct.row + row) * p.N * (p.out_f32 ? 4 : 2);
+        for (int mi = 0; mi < MF; ++mi) {
+          const int row = frag_row(mi) + l32;
+          const bool live = row < ct.rows;
+          // (a K slice's sums: an [all rows][N] matrix of its own)
+          const int64_t at = (kSliced ? static_cast<int64_t>(ct.slice) * p.c_gs : 0) + static_cast<int64_t>(ct.row + row) * p.N;
+          char* c_row = static_cast<char*>(p.c) + at * (F32 ? 4 : 2);
 #pragma unroll
-        for (int ni = 0; ni < NF; ++ni) {
-          const int nf = ct.n0 + wn0 + ni * 32;
-          if (!p.out_f32) {
-            // lanes l and l + 32 swap halves so that each stores 8 consecutive columns
+          for (int ni = 0; ni < NF; ++ni) {
+            const int nf = ct.n0 + wn0 + ni * 32;
+            if constexpr (F32) {
+              if (live) {
 #pragma unroll
-            for (int u = 0; u < 4; u += 2) {
-              v2i lo, hi;
-              {
-                const v4f a4 = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
-                const v4f b4 = {acc[mi][ni][4 * u + 4], acc[mi][ni][4 * u + 5], acc[mi][ni][4 * u + 6], acc[mi][ni][4 * u + 7]};
-                lo = __builtin_bit_cast(v2i, __builtin_convertvector(a4, v4bf));
-                hi = __builtin_bit_cast(v2i, __builtin_convertvector(b4, v4bf));
+                for (int u = 0; u < 4; ++u) {
+                  const int n = nf + u * 8 + h * 4;
+                  store_row4<true>(c_row, n, v4f{acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]}, INSIDE ? 4 : p.N - n);
+                }
               }
-              const auto s0 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.x), static_cast<unsigned>(hi.x), false, false);
-              const auto s1 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.y), static_cast<unsigned>(hi.y), false, false);
-              const int n = nf + 8 * u + 8 * h;
-              if (live && n < p.N)
-                store_row8_bf16(reinterpret_cast<__bf16*>(c_row) + n,
-                                v4i{static_cast<int>(s0[0]), static_cast<int>(s1[0]), static_cast<int>(s0[1]), static_cast<int>(s1[1])}, p.N - n);
-            }
-          } else if (live) {
+            } else {
+              // lanes l and l + 32 swap halves so that each stores 8 consecutive columns
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int n = nf + u * 8 + h * 4;
-              const v4f v = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
-              store_row4<true>(c_row, n, v, p.N - n);
+              for (int u = 0; u < 4; u += 2) {
+                v2i lo, hi;
+                {
+                  const v4f a4 = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
+                  const v4f b4 = {acc[mi][ni][4 * u + 4], acc[mi][ni][4 * u + 5], acc[mi][ni][4 * u + 6], acc[mi][ni][4 * u + 7]};
+                  lo = __builtin_bit_cast(v2i, __builtin_convertvector(a4, v4bf));
+                  hi = __builtin_bit_cast(v2i, __builtin_convertvector(b4, v4bf));
+                }
+                const auto s0 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.x), static_cast<unsigned>(hi.x), false, false);
+                const auto s1 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.y), static_cast<unsigned>(hi.y), false, false);
+                const int n = nf + 8 * u + 8 * h;
+                if (live && (INSIDE || n < p.N))
+                  store_row8_bf16(reinterpret_cast<__bf16*>(c_row) + n,
+                                  v4i{static_cast<int>(s0[0]), static_cast<int>(s1[0]), static_cast<int>(s0[1]), static_cast<int>(s1[1])}, INSIDE ? 8 : p.N - n);
+              }
             }
           }
         }
+      };
+      const bool inside = ct.n0 + wn0 + NF * 32 <= p.N;
+      if (kSliced || p.out_f32) {
+        if (inside)
+          store_tile(std::true_type{}, std::true_type{});
+        else
+          store_tile(std::true_type{}, std::false_type{});
+      } else if constexpr (!kSliced) {
+        if (inside)
+          store_tile(std::false_type{}, std::true_type{});
+        else
+          store_tile(std::false_type{}, std::false_type{});
       }
     }
     if (!it.ok) break;  // the issue side is one tile ahead: it has found no further one
     ct = it;
+  }
+}
+
+// K slices (p.splitk of them): few experts, or narrow ones, have fewer tiles than the chip has CUs, and a CU fetches 40 - 50 GB/s
+// whatever it is asked for.  The streaming kernel then runs the plain product of every (tile, K slice), fp32 sums in an
+// [all rows][N] matrix per slice (p.ws, p.c_gs floats apart), and one of the two kernels below adds the slices in index order, behind
+// it on the stream: 8 experts x ~15 rows x 1792 x 3584 24.9 -> 17.0 us, 32 x ~9 rows x 512 x 5632 36.9 -> 22.4 us.  Bound: the partial sums' way through the caches, 3 us with the
+// launch at decode sizes; loads of up to kReduceBatch slices are in flight per lane.
+constexpr int kReduceBatch = 4;
+constexpr int kMaxStreamSlices = 8;
+
+// rows [row0, row0 + rows) of expert g, as the streaming kernel sees them
+__device__ __forceinline__ void stream_expert_rows(const Args& p, int g, int* row0, int* rows) {
+  if (p.row_start != nullptr) {
+    *row0 = p.row_start[g];
+    *rows = max(p.gidx[g] - *row0, 0);
+  } else {
+    *row0 = g * p.M;
+    *rows = min(max(p.gidx[g], 0), p.M);
+  }
+}
+
+__device__ __forceinline__ v4f stream_add_slices(const float* at, int64_t stride, int slices) {
+  v4f sum = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < slices; s0 += kReduceBatch) {
+    v4f part[kReduceBatch];
+#pragma unroll
+    for (int i = 0; i < kReduceBatch; ++i)
+      if (s0 + i < slices) part[i] = *reinterpret_cast<const v4f_el*>(at + (s0 + i) * stride);
+#pragma unroll
+    for (int i = 0; i < kReduceBatch; ++i)
+      if (s0 + i < slices) sum += part[i];
+  }
+  return sum;
+}
+
+// grid (blocks, experts): c[row][n .. n + 3] = the slices' sum, four columns per lane
+__global__ void __launch_bounds__(256) fp8_stream_reduce_kernel(const Args p) {
+  int row0, rows;
+  stream_expert_rows(p, blockIdx.y, &row0, &rows);
+  const int cpr = (p.N + 3) / 4;
+  const int64_t total = static_cast<int64_t>(rows) * cpr;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < total; i += static_cast<int64_t>(gridDim.x) * 256) {
+    const int row = static_cast<int>(i / cpr), n = static_cast<int>(i - static_cast<int64_t>(row) * cpr) * 4;
+    const int64_t at = static_cast<int64_t>(row0 + row) * p.N;
+    v4f sum;
+    if (n + 4 <= p.N) {
+      sum = stream_add_slices(p.ws + at + n, p.c_gs, p.splitk);
+    } else {
+      for (int j = 0; j < 4; ++j) {
+        sum[j] = 0.f;
+        if (n + j < p.N)
+          for (int s = 0; s < p.splitk; ++s) sum[j] += p.ws[s * p.c_gs + at + n + j];
+      }
+    }
+    if (p.out_f32)
+      store_row4<true>(static_cast<float*>(p.c) + at, n, sum, p.N - n);
+    else
+      store_row4<false>(static_cast<__bf16*>(p.c) + at, n, sum, p.N - n);
+  }
+}
+
+// grid (blocks, experts): silu(gate) * up of the summed row and its 1 x 128 quantiser, 16 lanes per output group.  The sums pass
+// through bf16 as the plain GEMM would have stored them, so codes and scales have the bits of the separate steps.
+template <int EPI>
+__global__ void __launch_bounds__(256) fp8_stream_reduce_act_kernel(const Args p) {
+  int row0, rows;
+  stream_expert_rows(p, blockIdx.y, &row0, &rows);
+  const int lane = threadIdx.x & 63, sub = lane & 15;
+  const int gpr = p.act_cols / kScaleBlock;
+  const int total = rows * gpr;  // host: partial sums of rows x N floats fit the workspace
+  for (int base = (static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x >> 6)) * 4; base < total; base += static_cast<int>(gridDim.x) * 16) {
+    const int item = min(base + (lane >> 4), total - 1);
+    const int row = item / gpr, kg = item - row * gpr;
+    const float* at = p.ws + static_cast<int64_t>(row0 + row) * p.N + kg * kScaleBlock + sub * 8;
+    float v[8];
+    float amax = 0.f;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const v4f gate4 = stream_add_slices(at + 4 * half, p.c_gs, p.splitk);
+      const v4f up4 = stream_add_slices(at + p.act_cols + 4 * half, p.c_gs, p.splitk);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float gate = static_cast<float>(static_cast<__bf16>(gate4[j]));
+        const float up = static_cast<float>(static_cast<__bf16>(up4[j]));
+        float r;
+        if (EPI == kSiluQuantMasked)
+          r = static_cast<float>(static_cast<__bf16>(up * static_cast<float>(static_cast<__bf16>(act_silu_f32(gate)))));
+        else
+          r = static_cast<float>(static_cast<__bf16>(act_silu_f32(gate) * up));
+        v[4 * half + j] = r;
+        amax = fmaxf(amax, fabsf(r));
+      }
+    }
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 16));
+    const float scale = fmaxf(amax, p.act_eps) / 448.0f;
+    const float inv_scale = 1.0f / scale;
+    int packed[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float c4[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) c4[j] = fminf(fmaxf(act_div_by_scale(v[4 * i + j], scale, inv_scale), -448.0f), 448.0f);
+      int wd = __builtin_amdgcn_cvt_pk_fp8_f32(c4[0], c4[1], 0, false);
+      packed[i] = __builtin_amdgcn_cvt_pk_fp8_f32(c4[2], c4[3], wd, true);
+    }
+    if (base + (lane >> 4) < total) {
+      *reinterpret_cast<v2i*>(static_cast<uint8_t*>(p.c) + static_cast<int64_t>(row0 + row) * p.act_q_stride + kg * kScaleBlock + sub * 8) = v2i{packed[0], packed[1]};
+      if (sub == 0) {
+        const int64_t s_at = p.row_start != nullptr ? static_cast<int64_t>(row0 + row) * p.act_s_sm
+                                                    : static_cast<int64_t>(blockIdx.y) * p.act_s_gs + static_cast<int64_t>(row) * p.act_s_sm;
+        p.act_s[s_at + static_cast<int64_t>(kg) * p.act_s_sk] = scale;
+      }
+    }
   }
 }
 

@@ -46,12 +46,10 @@ struct Abi {
   decltype(&dlb_fp8_gemm_grouped_contiguous_same_rows) contiguous_same_rows;
   decltype(&dlb_fp8_gemm_grouped_contiguous_gather_silu_quant) contiguous_gather_act;
   decltype(&dlb_fp8_gemm_grouped_masked) masked;
-  decltype(&dlb_fp8_gemm_grouped_masked_silu_quant) masked_act;
+  decltype(&dlb_expert_gate_up_masked) masked_act;
   decltype(&dlb_fp8_gemm_grouped_ragged) ragged;
-  decltype(&dlb_fp8_gemm_grouped_ragged_silu_quant) ragged_act;
-  decltype(&dlb_fp8_gemm_plan_grouped) plan_grouped;
-  decltype(&dlb_fp8_gemm_plan_stream) plan_stream;
-  decltype(&dlb_fp8_gemm_variant_name) variant_name;
+  decltype(&dlb_expert_gate_up_ragged) ragged_act;
+  decltype(&dlb_expert_plan) plan;
   decltype(&dlb_fp8_quant_group) quant_group;
   decltype(&dlb_silu_mul_quant_masked) silu_masked;
   decltype(&dlb_ep_scatter_workspace_bytes) scatter_ws;
@@ -374,11 +372,13 @@ PyObject* grouped_masked(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // ---- expert MLPs ------------------------------------------------------------------------------------------------------
 
-// whether the weight-streaming kernel runs experts of about `hint` rows
-bool streams(int64_t rows, int64_t N, int64_t K, int64_t G, int64_t hint, bool quantising) {
-  int tile_rows = 0;
-  return abi.plan_stream(rows, N, K, static_cast<int32_t>(G), static_cast<int32_t>(hint), quantising, 256, &tile_rows, nullptr, nullptr) == DLB_OK &&
-         tile_rows > 0;
+// forms of dlb_expert_plan
+enum Form : int { kStepsApart = 0, kOnRowRanges = 1, kOnWholeBlocks = 2 };
+
+Form expert_form(int mode, int64_t rows, int64_t N, int64_t K, int64_t G, int64_t hint, bool quantising, const Workspace& ws) {
+  int form = kOnWholeBlocks;
+  if (abi.plan(mode, rows, N, K, static_cast<int32_t>(G), static_cast<int32_t>(hint), quantising, ws.bytes, 256, &form) != DLB_OK) return kStepsApart;
+  return static_cast<Form>(form);
 }
 
 // low_latency_experts(a, a_s, w13, w13_s, w2, w2_s, masked_m, expected_m) -> down_output (bf16)
@@ -403,14 +403,6 @@ PyObject* low_latency_experts(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const hipStream_t stream = stream_of(a);
   Workspace ws;
   if (!workspace_of(scope.dev, stream, a, &ws)) return nullptr;
-  int variant = 0;
-  if (abi.plan_grouped(2, M, N, K, static_cast<int32_t>(G), static_cast<int32_t>(hint), ws.bytes, 256, &variant, nullptr) != DLB_OK) NOT_PLAIN;
-  static const int kRing128 = [] {
-    for (int i = 0;; ++i) {
-      const char* name = abi.variant_name(i);
-      if (!name || std::string(name) == "pipe128x256w8") return i;
-    }
-  }();
   const int32_t g = static_cast<int32_t>(G), m_hint = static_cast<int32_t>(hint);
   at::Tensor q, s, gate_up, out;
   int rc = DLB_OK;
@@ -419,7 +411,7 @@ PyObject* low_latency_experts(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const NoGil nogil;
     q = empty({G, M, inter}, at::kFloat8_e4m3fn, a);
     bool fused = false;
-    if (variant == kRing128 || streams(M, N, K, G, hint, true)) {
+    if (expert_form(2, M, N, K, G, hint, true, ws) != kStepsApart) {
       // rows of a K block contiguous: what the second GEMM reads without a re-layout pass
       s = empty_strided({G, M, inter / kBlock}, {inter / kBlock * M, 1, M}, at::kFloat, a);
       fused = abi.masked_act(ptr(a), ptr(w13), fptr(a_s), fptr(w13_s), ptr(q), fptr(s), iptr(mm), m_hint, M, N, K, g, a_s.stride(0), a_s.stride(1),
@@ -521,10 +513,13 @@ PyObject* fused_moe_v3(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (abi.scatter_ws(T, topk, E) > ws.bytes) NOT_PLAIN;
   // typical rows of an expert: half a block of its span is padding on average
   const int64_t rows_each = std::max<int64_t>(1, std::min(rows / used - 64, ceil_div(T * topk, used)));
-  int lists = 0;
-  const bool short_experts = streams(rows, N, H, E, rows_each, true) && streams(rows, H, inter, E, rows_each, false);
-  if (!short_experts && (abi.plan_grouped(1, rows, N, H, static_cast<int32_t>(E), -1, ws.bytes, 256, nullptr, &lists) != DLB_OK || !lists))
-    NOT_PLAIN;  // three steps on uniform tiles
+  Form up_form, down_form;
+  {
+    const NoGil nogil;
+    up_form = expert_form(1, rows, N, H, E, rows_each, true, ws);
+    down_form = expert_form(1, rows, H, inter, E, rows_each, false, ws);
+  }
+  if (up_form == kStepsApart) NOT_PLAIN;
   const OpRecord record("dlblas::fused_moe_v3", t);
 
   at::Tensor out;
@@ -545,23 +540,27 @@ PyObject* fused_moe_v3(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const Together together(ws);  // the down GEMM reads what the gate/up GEMM leaves in the workspace
     rc = abi.scatter_rows(ptr(ids), idx_code(ids.scalar_type()), ids.stride(0), ids.stride(1), counts, row_start, row_end, first_free, row_expert, row_token,
                           rows, ptr(slot_row), idx_code(slot_row.scalar_type()), topk, 1, T, topk, E, ws.ptr, ws.bytes, stream);
-    int64_t s_m = inter / kBlock, s_k = 1;
-    bool lists_now = rc == DLB_OK;
-    if (rc == DLB_OK && short_experts) {
+    // the order the down GEMM reads in place: rows whole, or the rows of a K block together
+    const int64_t s_m = down_form == kOnRowRanges ? inter / kBlock : 1, s_k = down_form == kOnRowRanges ? 1 : rows;
+    if (rc == DLB_OK && up_form == kOnRowRanges) {
       rc = abi.ragged_act(ptr(x), ptr(w13), fptr(x_s), fptr(w13_s), ptr(q), fptr(s), row_start, row_end, row_token, T, hint, rows, N, H, g, x_s.stride(0),
-                          x_s.stride(1), s_m, s_k, 1e-10f, stream);
-      if (rc == DLB_OK) rc = abi.ragged(ptr(q), ptr(w2), fptr(s), fptr(w2_s), ptr(down), row_start, row_end, hint, rows, H, inter, g, s_m, s_k, DLB_OUT_BF16, stream);
-      lists_now = rc == DLB_ERR_BAD_SHAPE;
-      begun = !lists_now;
+                          x_s.stride(1), s_m, s_k, 1e-10f, ws.ptr, ws.bytes, stream);
+      if (rc == DLB_ERR_BAD_SHAPE) up_form = kOnWholeBlocks, rc = DLB_OK;
+      begun = up_form == kOnRowRanges;
     }
-    if (lists_now) {
-      s_m = 1, s_k = rows;  // rows of a K block contiguous: what the down GEMM reads in place
+    if (rc == DLB_OK && up_form == kOnWholeBlocks) {
       rc = abi.contiguous_gather_act(ptr(x), ptr(w13), fptr(x_s), fptr(w13_s), ptr(q), fptr(s), row_expert, row_token, T, rows, N, H, g, x_s.stride(0),
                                      x_s.stride(1), s_m, s_k, 1e-10f, ws.ptr, ws.bytes, stream);
       begun = rc != DLB_ERR_BAD_SHAPE;  // declined: the Python path starts over with the three steps
-      if (rc == DLB_OK)
-        rc = abi.contiguous_same_rows(ptr(q), ptr(w2), fptr(s), fptr(w2_s), ptr(down), row_expert, rows, H, inter, g, s_m, s_k, DLB_OUT_BF16, ws.ptr,
-                                      ws.bytes, stream);
+    }
+    if (rc == DLB_OK) {
+      rc = DLB_ERR_BAD_SHAPE;
+      if (down_form == kOnRowRanges)
+        rc = abi.ragged(ptr(q), ptr(w2), fptr(s), fptr(w2_s), ptr(down), row_start, row_end, hint, rows, H, inter, g, s_m, s_k, DLB_OUT_BF16, stream);
+      if (rc == DLB_ERR_BAD_SHAPE) {
+        const auto gemm = up_form == kOnWholeBlocks ? abi.contiguous_same_rows : abi.contiguous;  // the lists the gate/up GEMM left
+        rc = gemm(ptr(q), ptr(w2), fptr(s), fptr(w2_s), ptr(down), row_expert, rows, H, inter, g, s_m, s_k, DLB_OUT_BF16, ws.ptr, ws.bytes, stream);
+      }
     }
     if (rc == DLB_OK) rc = gather(down, ids, weights, slot_row, out, stream);
   }

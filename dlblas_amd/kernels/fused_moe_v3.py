@@ -106,6 +106,13 @@ def ep_gather(
     return
 
 
+def _scales(rows, blocks, form, device):
+    """[rows, blocks] fp32 in the order the down GEMM of this form reads in place: rows whole, or the rows of a K block together."""
+    if form == _lib.ON_ROW_RANGES:
+        return torch.empty((rows, blocks), device=device)
+    return torch.empty((blocks, rows), device=device).t()
+
+
 def _down(act, w2_weight_fp8, row_expert, out):
     m_grouped_fp8_gemm_nt_contiguous(act, w2_weight_fp8, out, row_expert)
     return out
@@ -152,44 +159,43 @@ def fused_moe_v3(
     # the expert-sorted copy of the activations nor the bf16 [rows, 2 I] intermediate reaches memory.  Same bits as the
     # steps of the reference (:288-334).
     if tokens_q.is_contiguous() and hidden % 128 == 0 and inter2 % 256 == 0 and n_tokens * hidden < (1 << 32):
-        # A short batch - a block or so of rows per expert, most of them padding - is a matter of reading the experts'
-        # weights once: the weight-streaming kernels, on the rows that hold a token (500 tokens, 32 experts of 7168 x 2048:
-        # 333 -> 245 us; their token offsets are 31 bits).  A long one pairs the blocks of an expert into taller tiles.  In
-        # between, where the library's planner prefers uniform 128-row tiles, which have no fused epilogue, the three steps
-        # below are the faster way.
-        streams = False
-        if n_experts <= 256 and n_tokens * hidden < (1 << 31):
-            used = sum(1 for c in num_recv_tokens_per_expert if c > 0)
-            rows_each = max(1, min(rows_total // used - 64, -(-n_tokens * topk_idx.size(1) // used)))  # half a block of padding on average
-            streams = (_lib.plan_stream(rows_total, inter2, hidden, n_experts, rows_each, quantising=True) is not None
-                       and _lib.plan_stream(rows_total, hidden, inter2 // 2, n_experts, rows_each) is not None)
-        lists = _lib.plan_grouped(1, rows_total, inter2, hidden, n_experts)[1]
-        if streams or lists:
+        # Short experts, few of them or narrow ones are a matter of reading the weights once with every CU: the weight-streaming
+        # kernels, on the rows that hold a token (500 tokens, 32 experts of 7168 x 2048: 333 -> 245 us; their token offsets are 31
+        # bits).  Longer ones pair the blocks of an expert into taller tiles.
+        used = sum(1 for c in num_recv_tokens_per_expert if c > 0)
+        rows_each = max(1, min(rows_total // used - 64, -(-n_tokens * topk_idx.size(1) // used)))  # half a block of padding on average
+        up_form = _lib.expert_plan(1, rows_total, inter2, hidden, n_experts, rows_each, quantising=True)
+        down_form = _lib.expert_plan(1, rows_total, hidden, inter2 // 2, n_experts, rows_each, quantising=False)
+        if up_form != _lib.STEPS_APART:
             row_token = buf((rows_total, ), torch.int32)
             ranges = buf((3, n_experts), torch.int32)
-            have_tables = _lib.ep_scatter_rows_host(topk_idx, num_recv_tokens_per_expert, ranges[0], ranges[1], ranges[2], row_expert,
-                                                    row_token, slot_row)
+            have_tables = (n_experts <= 256 and
+                           _lib.ep_scatter_rows_host(topk_idx, num_recv_tokens_per_expert, ranges[0], ranges[1], ranges[2], row_expert,
+                                                     row_token, slot_row))
             if not have_tables:
-                streams = False  # the row ranges come with the tables of the host form only
-                if lists:
-                    # more experts, or more tokens times experts, than travel in the launch: the same tables from counts
-                    # in device memory
-                    ep_scatter_rows(topk_idx, upload_counts(), ranges[2], row_expert, row_token, slot_row)
-                    have_tables = True
-            if have_tables:
-                down = buf((rows_total, hidden), torch.bfloat16)
-                if streams:
-                    act_q = buf((rows_total, inter2 // 2), torch.float8_e4m3fn)
-                    act_scale = buf((rows_total, inter2 // 256), torch.float32)
-                    streams = (_lib.gemm_ragged_silu_quant(tokens_q, w13_weight_fp8[0], tokens_scale, w13_weight_fp8[1], act_q,
-                                                           act_scale, ranges[0], ranges[1], row_token, rows_each, 1e-10)
-                               and _lib.gemm_ragged(act_q, w2_weight_fp8[0], act_scale, w2_weight_fp8[1], down, ranges[0], ranges[1],
-                                                    rows_each))
-                if not streams:
-                    fused = fp8_gemm_grouped_contiguous_silu_quant(tokens_q, tokens_scale, w13_weight_fp8[0], w13_weight_fp8[1],
-                                                                   row_expert, column_major_scales=True,  # what the down GEMM reads in place
-                                                                   a_row_index=row_token)
-                    down = _down(fused, w2_weight_fp8, row_expert, down) if fused is not None else None
+                # more experts, or more tokens times experts, than travel in the launch: the same tables from counts in device
+                # memory.  The row ranges come with the host form only
+                up_form = down_form = _lib.ON_WHOLE_BLOCKS
+                ep_scatter_rows(topk_idx, upload_counts(), ranges[2], row_expert, row_token, slot_row)
+            if n_tokens * hidden >= (1 << 31):
+                up_form = _lib.ON_WHOLE_BLOCKS
+            down = buf((rows_total, hidden), torch.bfloat16)
+            fused = None
+            if up_form == _lib.ON_ROW_RANGES:
+                act_q = buf((rows_total, inter2 // 2), torch.float8_e4m3fn)
+                act_scale = _scales(rows_total, inter2 // 256, down_form, dev)
+                if _lib.expert_gate_up_ragged(tokens_q, w13_weight_fp8[0], tokens_scale, w13_weight_fp8[1], act_q, act_scale, ranges[0], ranges[1],
+                                              row_token, rows_each, 1e-10):
+                    fused = act_q, act_scale
+            if fused is None:
+                fused = fp8_gemm_grouped_contiguous_silu_quant(tokens_q, tokens_scale, w13_weight_fp8[0], w13_weight_fp8[1],
+                                                               row_expert, column_major_scales=down_form != _lib.ON_ROW_RANGES,
+                                                               a_row_index=row_token)
+            if fused is None:
+                down = None
+            elif not (down_form == _lib.ON_ROW_RANGES and
+                      _lib.gemm_ragged(fused[0], w2_weight_fp8[0], fused[1], w2_weight_fp8[1], down, ranges[0], ranges[1], rows_each)):
+                down = _down(fused, w2_weight_fp8, row_expert, down)
     if down is None:
         # Expert-sorted activations.  The spans are padded to 128 rows per expert; the padding rows keep whatever the
         # allocator hands out, as in the reference driver (:269-278).  The GEMMs and the quantiser treat every row on its

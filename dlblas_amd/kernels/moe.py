@@ -77,17 +77,15 @@ def low_latency_experts(
     expected_m = min(expected_m, m)
     down_input = torch.empty((num_groups, m, n // 2), device=a.device, dtype=gate_down_weight.dtype)
     fused = False
-    # The fused epilogue exists for the weight-streaming kernel (short experts) and for the 128 x 256 tiles; where the
-    # library picks other tiles for the plain GEMM (several hundred rows per expert) the steps apart are faster (32
-    # experts x ~520 rows: 619 against 678 us).
-    want_fused = (_lib.plan_grouped(2, m, n, k, num_groups, expected_m)[0] == 'pipe128x256w8'
-                  or _lib.plan_stream(m, n, k, num_groups, expected_m, quantising=True) is not None)
+    # where the library picks other tiles for the plain GEMM (several hundred rows per expert) the steps apart are faster (32
+    # experts x ~520 rows: 619 against 678 us)
+    want_fused = _lib.expert_plan(2, m, n, k, num_groups, expected_m, quantising=True) != _lib.STEPS_APART
     if want_fused and out_dtype == torch.bfloat16 and block_size == 128 and n % 256 == 0 and masked_m.dtype == torch.int32:
-        # one kernel for GEMM + activation + quantiser, same bits; its scales go out with the rows of a K block
+        # one call for GEMM + activation + quantiser; its scales go out with the rows of a K block
         # contiguous, the layout the second GEMM reads without a re-layout pass
         down_input_scale = torch.empty((num_groups, n // 2 // block_size, m), device=a.device, dtype=torch.float32).transpose(1, 2)
         fused = fp8_gemm_grouped_masked_silu_quant(a, a_s, gate_up_weight, gate_up_scale, down_input, down_input_scale,
-                                                   masked_m, expected_m)
+                                                   masked_m, expected_m, mlp=True)
     if not fused:
         gateup_output = torch.empty((num_groups, m, n), device=a.device, dtype=out_dtype)
         m_grouped_fp8_gemm_nt_masked((a, a_s), (gate_up_weight, gate_up_scale), gateup_output, masked_m, expected_m)

@@ -47,7 +47,7 @@
 extern "C" {
 #endif
 
-#define DLB_ABI_VERSION 9
+#define DLB_ABI_VERSION 10
 
 /* output element type of C */
 #define DLB_OUT_BF16 0
@@ -299,6 +299,34 @@ int dlb_fp8_gemm_grouped_ragged_silu_quant(const void* a, const void* b, const f
                                            int64_t as_stride_m, int64_t as_stride_k, int64_t os_stride_m, int64_t os_stride_k,
                                            float eps, void* stream);
 
+/*
+ * The gate/up projection as a step of an expert MLP, in whichever form is fastest: dlb_fp8_gemm_grouped_masked_silu_quant /
+ * dlb_fp8_gemm_grouped_ragged_silu_quant in one launch, or the plain product of every tile and K slice followed by a launch that
+ * adds the slices, activates and quantises (few experts, or narrow ones, whose 256-column tiles would leave most CUs idle; the
+ * partial sums live in the workspace).  Sums of K slices are added in another order than in one launch, so a value next to a
+ * rounding boundary may differ from those calls' in its last place.  DLB_ERR_BAD_SHAPE, nothing enqueued: another way is the
+ * faster one - the masked GEMM and the activation apart, the expert-contiguous kernels - or the call declines as those do.
+ */
+int dlb_expert_gate_up_masked(const void* a, const void* b, const float* a_s, const float* b_s, void* out_q, float* out_s,
+                              const int32_t* masked_m, int32_t expected_m, int64_t M_max, int64_t N, int64_t K, int32_t G,
+                              int64_t as_stride_g, int64_t as_stride_m, int64_t as_stride_k, int64_t os_stride_g,
+                              int64_t os_stride_m, int64_t os_stride_k, float eps, void* workspace, size_t workspace_bytes,
+                              void* stream);
+int dlb_expert_gate_up_ragged(const void* a, const void* b, const float* a_s, const float* b_s, void* out_q, float* out_s,
+                              const int32_t* row_start, const int32_t* row_end, const int32_t* a_row_index, int64_t a_rows,
+                              int32_t expected_m, int64_t M_sum, int64_t N, int64_t K, int32_t G, int64_t as_stride_m,
+                              int64_t as_stride_k, int64_t os_stride_m, int64_t os_stride_k, float eps, void* workspace,
+                              size_t workspace_bytes, void* stream);
+
+/*
+ * Which kernels run a projection of an expert MLP fastest (quantising != 0: gate/up, N = 2 I).  Masked layout (mode 2, rows =
+ * M_max): *form 1 = dlb_expert_gate_up_masked takes it, 0 = it declines.  Expert-contiguous rows (mode 1): 1 = the ragged entry points (dlb_expert_gate_up_ragged, dlb_fp8_gemm_grouped_ragged), 2 = the expert-contiguous ones (gate/up: with
+ * the quantising epilogue), 0 = neither applies.  rows: padded rows of all experts; expected_m: typical rows of an expert that hold
+ * a token.  From sizes alone, nothing is launched.
+ */
+int dlb_expert_plan(int mode, int64_t rows, int64_t N, int64_t K, int32_t G, int32_t expected_m, int quantising, size_t workspace_bytes,
+                    int compute_units, int* form);
+
 /* element type of the quantiser input */
 #define DLB_IN_BF16 0
 #define DLB_IN_F16 1
@@ -424,6 +452,7 @@ int dlb_fp8_gemm_force_variant(int variant);
  *   DLB_KNOB_STREAM         masked layout: 1 = never the weight-streaming kernel, 2 .. 6 = its tile shape 0 .. 4 (32 x 256,
  *                           64 x 256, 64 x 128, 128 x 256, 64 x 64) wherever it applies, 7 .. 11 = the same with fragments
  *                           read one step ahead where that form exists (plain product, not 32 x 256) (default: by size)
+ *   DLB_KNOB_STREAM_SLICES  n = the weight-streaming kernel's quantising launches in two, with n K slices (default: by size)
  *   DLB_KNOB_WAVE_K         dense: 1 = never the kernel whose waves split K, 2 .. 8 = its tile shape 0 .. 6 (32 x 32 with 8 / 4
  *                           waves, 64 x 32 with 8, 32 x 64 with 4, 64 x 32 with 4, 64 x 64 with 4 / 2) wherever it applies
  *   DLB_KNOB_LDS_OVERSIZE   test hook: 1 = every kernel asks for more LDS than the GPU has, so the call is refused
@@ -445,6 +474,7 @@ int dlb_fp8_gemm_force_variant(int variant);
 #define DLB_KNOB_TILE_LIST 13
 #define DLB_KNOB_STREAM 14
 #define DLB_KNOB_WAVE_K 15
+#define DLB_KNOB_STREAM_SLICES 16
 int dlb_fp8_gemm_tune(int knob, int value);
 
 /* Name of kernel variant `variant`, or NULL beyond the last one. */

@@ -268,3 +268,92 @@ def test_row_tables_where_more_slots_are_routed_than_reserved(dev, T, topk, E):
         assert torch.equal(got, held) and torch.equal(src.cpu().long(), src_ref)
     else:
         assert E > 256
+
+
+def _close_codes(q, s, ref_q, ref_s, rows):
+    """Sums of K slices are added in another order, 1e-7 of them: a bf16 value next to a rounding boundary moves by its last place,
+    and with it at most a code by one step (an eighth of the value, or the smallest code's worth), here and there."""
+    got, ref = (x.float() * y.repeat_interleave(128, dim=-1) for x, y in ((q, s), (ref_q, ref_s)))
+    got, ref = got[rows], ref[rows]
+    step = ref.abs() / 8 + ref_s.repeat_interleave(128, dim=-1)[rows] * 2.0**-9
+    assert bool(((got - ref).abs() <= 1.01 * step).all())
+    assert float((q.view(torch.uint8)[rows] != ref_q.view(torch.uint8)[rows]).float().mean()) < 1e-2
+
+
+@pytest.mark.parametrize('masked,M_max,N,K,slices', [
+    ([1, 31, 32, 33, 0, 64], 64, 512, 1280, [1, 2, 3]),         # 10 blocks: slices of unequal length, as short as the rings
+    ([65, 128, 3], 136, 256, 6784, [1, 5, 8]),                  # 53 blocks: several chunks of the scale table in a slice
+    ([i % 4 for i in range(70)], 8, 256, 2304, [2]),            # a second window of 64 experts
+])
+def test_gate_up_in_two_launches(dev, masked, M_max, N, K, slices):
+    """The gate/up projection as partial products of every tile and K slice + one launch that adds, activates and quantises: with
+    one slice the bits of the fused kernel, with more what another order of the fp32 sums gives; masked rows keep their content."""
+    from dlblas_amd import _lib
+    from dlblas_amd.kernels.fp8_gemm_grouped import fp8_gemm_grouped_masked_silu_quant
+    a_q, a_s, w_q, w_s, mm = _inputs(masked, M_max, N, K, 70 + N + K, dev)
+    G = len(masked)
+    rows = torch.arange(M_max, device=dev)[None] < mm[:, None]
+
+    def run(mlp):
+        q = torch.full((G, M_max, N // 2), 0x5a, dtype=torch.uint8, device=dev).view(torch.float8_e4m3fn)
+        s = torch.full((G, N // 256, M_max), -7.0, device=dev).transpose(1, 2)
+        assert fp8_gemm_grouped_masked_silu_quant(a_q, a_s, w_q, w_s, q, s, mm, 0, mlp=mlp)
+        torch.cuda.synchronize()
+        assert (q.view(torch.uint8)[~rows] == 0x5a).all() and (s[~rows] == -7.0).all()
+        return q, s
+
+    _lib.tune('stream', 1)
+    ref_q, ref_s = run(False)
+    for knob, shape in zip([2, 3, 4, 5, 6, 8, 9, 10, 11], SHAPES + AHEAD):
+        for n in slices:
+            print(f'case gate/up in two launches masked={masked[:6]} N={N} K={K} {shape} slices={n}', flush=True)
+            _lib.tune('stream', knob), _lib.tune('stream_slices', n)
+            q, s = run(True)
+            _lib.tune('stream', 0), _lib.tune('stream_slices', 0)
+            if n == 1:
+                assert torch.equal(q.view(torch.uint8)[rows], ref_q.view(torch.uint8)[rows]) and torch.equal(s[rows], ref_s[rows])
+            else:
+                _close_codes(q, s, ref_q, ref_s, rows)
+
+
+@pytest.mark.parametrize('tokens,E,H,inter', [(30, 8, 2560, 768), (300, 8, 1024, 256), (900, 16, 512, 384), (2500, 4, 768, 128)])
+def test_expert_mlps_in_every_form(dev, tokens, E, H, inter):
+    """fused_moe_v3 and low_latency_experts from short to long experts, in whichever form their planner picks: native and Python path
+    agree, and the result stays within what the quantiser between the GEMMs makes of a last place (the bar of the end-to-end tests)
+    of the ring kernels'."""
+    from dlblas_amd import _fast, _lib
+    from dlblas_amd.kernels.fp8 import per_block_quant_fp8, per_token_group_quant_fp8
+    from dlblas_amd.kernels.fused_moe_v3 import fused_moe_v3
+    from dlblas_amd.kernels.moe import low_latency_experts
+    print(f'case expert MLP forms tokens={tokens} E={E} H={H} I={inter}', flush=True)
+    g = helpers.gen(15)
+
+    def weights(n, k):
+        q, s = zip(*(per_block_quant_fp8((torch.randn(n, k, generator=g) * 0.05).to(torch.bfloat16).to(dev)) for _ in range(E)))
+        return torch.stack(q), torch.stack(s)
+
+    w13, w2 = weights(2 * inter, H), weights(H, inter)
+    x = per_token_group_quant_fp8(torch.randn(tokens, H, generator=g).to(torch.bfloat16).to(dev), 128)
+    ids = torch.rand(tokens, 4 * E, generator=g).topk(4, dim=1).indices
+    ids = torch.where(ids < E, ids, torch.full_like(ids, -1))
+    counts = ((torch.bincount(ids[ids >= 0], minlength=E) + 127) // 128 * 128).tolist()
+    args = ids.to(dev), torch.rand(tokens, 4, generator=g).to(dev), w13, w2, counts
+    valid = torch.bincount(ids[ids >= 0], minlength=E).to(torch.int32)
+    cap = int(valid.max()) + 5
+    a_q, a_s = per_token_group_quant_fp8(torch.randn(E * cap, H, generator=g).to(torch.bfloat16).to(dev), 128)
+    low = (a_q.view(E, cap, H), a_s.view(E, cap, -1)), *w13, *w2, valid.to(dev), max(1, int(valid.float().mean()))
+    rows = torch.arange(cap, device=dev)[None] < low[5][:, None]
+    outs = []
+    for knob in (0, 1):
+        _lib.tune('stream', knob)
+        out, down = fused_moe_v3(x, *args), low_latency_experts(*low)
+        assert _fast.fused_moe_v3(*x, *args[:2], *w13, *w2, counts) is not None
+        with torch.overrides.BaseTorchFunctionMode():
+            out2, down2 = fused_moe_v3(x, *args), low_latency_experts(*low)
+        torch.cuda.synchronize()
+        assert torch.equal(out, out2) and torch.equal(down[rows], down2[rows])
+        outs.append((out.float(), down[rows].float()))
+    _lib.tune('stream', 0)
+    for got, ref in zip(*outs):
+        assert orc.similarity_gap(got.cpu(), ref.cpu()) <= 1e-4
+        assert float((got - ref).abs().max()) <= 0.05 * float(ref.pow(2).mean().sqrt())
