@@ -1313,7 +1313,11 @@ int run(const Problem& pr) {
   ar.sk_bn = pl.sk_bn;
   ar.splitk = rs.splitk;
   ar.kb_per_split = rs.kb_per_split;
-  ar.group_m = g_knob[kKnobGroupM] > 0 ? g_knob[kKnobGroupM] : 8;
+  // Row tiles per L2 patch: 8, but 7 in launches of many rounds, whose workgroups step through the patches together: us per call with 8
+  // / 7 row tiles 4096 x 24576 x 1536 179 / 163, 4096 x 32768 x 512 156 / 128, 4000 x 28160 x 768 128 / 120, 4096 x 24576 x 4608
+  // 419 / 416 (14 such problems 1.03 x, none more than 1.5 % slower; 3 and 5 gain as much, 4, 6 and 16 do not); with one to
+  // four rounds the difference is noise.
+  ar.group_m = g_knob[kKnobGroupM] > 0 ? g_knob[kKnobGroupM] : (rs.resident ? 7 : 8);
   ar.out_f32 = pr.out_dtype == DLB_OUT_F32;
   ar.a_rows = pr.a_rows;
   ar.act_s = pr.act_s;
