@@ -277,8 +277,9 @@ __global__ void __launch_bounds__(kCopyThreads) ep_scatter_copy_kernel(const Sca
 
 // The tables of the scatter without its copy.  A block ranks its 256 entries by matching the expert ids inside a wave (one
 // ballot per id bit) on top of the counts of the waves before it.  What it has to know of the other blocks' entries:
-//   kRowsAlone: it reads the ids of every entry itself and counts them in LDS (up to kRowsOneLaunch entries: 4096 entries take
-//     6.2 us where the count launch and the summing launch took 4.2 + 18.6);
+//   kRowsAlone: it reads the ids of every entry itself and counts them in LDS (up to kRowsOneLaunch entries; a contiguous table
+//     through 16-byte loads that are all in flight at once and one atomic per routed entry: 16384 entries 8.1 -> 5.5 us, 8000
+//     5.6 -> 4.6 us against element loads with a division each.  At 24000 entries the two launches of kRowsSum are ahead, 6.1 / 6.4 us);
 //   kRowsSum: ep_scatter_count_kernel has left the blocks' histograms, and the rows of the blocks before (for the padding
 //     also behind) are added up 8 loads at a time (65536 entries: 15.3 -> 5.3 us against one dependent load after the other);
 //   kRowsScanned: many blocks; ep_scatter_scan_kernel has turned the histograms into first rows.
@@ -312,23 +313,39 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
   if (MODE == kRowsAlone) {
     const int n = static_cast<int>(p.T) * p.topk_n;
     const int mine = b * p.tokens_per_block * p.topk_n;
-    for (int i0 = tid; i0 < n; i0 += 4 * kRowsThreads) {
-      int id[4];
+    // one atomic per routed entry: all entries in the low half of routed[e], those of earlier blocks in the high half
+    auto count = [&](int id, int i) { atomicAdd(&routed[id], i < mine ? 0x10001 : 1); };
+    const bool rows_whole = p.topk_s1 == 1 && p.topk_s0 == p.topk_n && reinterpret_cast<uintptr_t>(p.topk) % 16 == 0;
+    const int first_alone = rows_whole ? n / 4 * 4 : 0;
+    if (rows_whole) {
+      // the table is one array of ids: 16-byte loads, all of a thread's in flight, no division
+      constexpr int kBatch = 8;
+      const int per = p.topk_is64 ? 2 : 4;
+      const int chunks = first_alone / per;
+      const v4i* ids = static_cast<const v4i*>(p.topk);
+      for (int c0 = tid; c0 < chunks; c0 += kBatch * kRowsThreads) {
+        v4i raw[kBatch];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int i = i0 + u * kRowsThreads;
-        id[u] = -1;
-        if (i < n) {
-          const int64_t v = load_index(p.topk, p.topk_is64, static_cast<int64_t>(i / p.topk_n) * p.topk_s0 + (i % p.topk_n) * p.topk_s1);
-          if (v >= 0 && v < E) id[u] = static_cast<int>(v);
+        for (int u = 0; u < kBatch; ++u)
+          if (c0 + u * kRowsThreads < chunks) raw[u] = ids[c0 + u * kRowsThreads];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+          const int c = c0 + u * kRowsThreads;
+          if (c >= chunks) continue;
+          if (p.topk_is64) {  // low and high words of two ids
+            if (raw[u].y == 0 && static_cast<uint32_t>(raw[u].x) < static_cast<uint32_t>(E)) count(raw[u].x, 2 * c);
+            if (raw[u].w == 0 && static_cast<uint32_t>(raw[u].z) < static_cast<uint32_t>(E)) count(raw[u].z, 2 * c + 1);
+          } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              if (static_cast<uint32_t>(raw[u][k]) < static_cast<uint32_t>(E)) count(raw[u][k], 4 * c + k);
+          }
         }
       }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (id[u] >= 0) {
-          atomicAdd(&routed[id[u]], 1);
-          if (i0 + u * kRowsThreads < mine) atomicAdd(&before[id[u]], 1);
-        }
+    }
+    for (int i = first_alone + tid; i < n; i += kRowsThreads) {
+      const int64_t v = load_index(p.topk, p.topk_is64, static_cast<int64_t>(i / p.topk_n) * p.topk_s0 + (i % p.topk_n) * p.topk_s1);
+      if (v >= 0 && v < E) count(static_cast<int>(v), i);
     }
   } else if (MODE == kRowsScanned) {
     for (int e = tid; e < E; e += kRowsThreads) {
@@ -359,6 +376,8 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
       atomicAdd(&before[e], sum_before);
     }
   }
+  auto routed_to = [&](int e) { return MODE == kRowsAlone ? routed[e] & 0xffff : routed[e]; };
+  auto routed_before = [&](int e) { return MODE == kRowsAlone ? routed[e] >> 16 : before[e]; };
   if (wave == 4) {  // a wave with no entries of its own scans the reserved rows
     int carry = 0;
     for (int e0 = 0; e0 < E; e0 += 64) {
@@ -390,7 +409,7 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
   __syncthreads();
   if (id >= 0) {
     for (int w = 0; w < wave; ++w) rank += wave_cnt[w * E + id];
-    const int d = excl[id] + before[id] + rank;
+    const int d = excl[id] + routed_before(id) + rank;
     const int64_t t = static_cast<int64_t>(b) * p.tokens_per_block + tid / p.topk_n;
     store_index(p.out_index, p.oi_is64, t * p.oi_s0 + (tid % p.topk_n) * p.oi_s1, d);
     if (d < p.m_len) p.src_row[d] = static_cast<int32_t>(t);
@@ -399,12 +418,12 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
   // rows, they run on into the spans behind its own, as in ep_scatter, and those rows are not empty.  Every wave looks for
   // such an expert itself: with a vote of the block and 64-bit row numbers in the main loop the kernel took 0.4 .. 1.0 us longer.
   int over = 0;
-  for (int e = lane; e < E; e += 64) over |= routed[e] > excl[e + 1] - excl[e];
+  for (int e = lane; e < E; e += 64) over |= routed_to(e) > excl[e + 1] - excl[e];
   over = __any(over);
   auto end_of = [&](int e) {
-    int end = excl[e] + routed[e];
+    int end = excl[e] + routed_to(e);
     if (over)
-      for (int i = 0; i < e; ++i) end = max(end, excl[i] + routed[i]);
+      for (int i = 0; i < e; ++i) end = max(end, excl[i] + routed_to(i));
     return end;
   };
   // rows [0, excl[E]) in slices over the blocks: their expert, and token 0 for the rows that no slot is given
@@ -431,7 +450,7 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
   }
   if (b == 0)
     for (int e = tid; e < E; e += kRowsThreads) {
-      if (MODE != kRowsScanned) store_index(p.start_loc, p.start_is64, e, static_cast<int64_t>(excl[e]) + routed[e]);
+      if (MODE != kRowsScanned) store_index(p.start_loc, p.start_is64, e, static_cast<int64_t>(excl[e]) + routed_to(e));
       if (p.row_start != nullptr) p.row_start[e] = excl[e];
       if (p.row_end != nullptr) p.row_end[e] = min(end_of(e), excl[e + 1]);
     }

@@ -210,6 +210,38 @@ def test_row_tables_longer_than_the_spans(dev, T, topk, E):
     assert torch.equal(m_indices[:rows].cpu().long(), torch.repeat_interleave(torch.arange(E), counts)) and (m_indices[rows:] == -1).all()
 
 
+@pytest.mark.parametrize('T,topk,E,dtype,form', [(1, 1, 1, torch.int64, 'whole'), (333, 3, 9, torch.int32, 'whole'), (333, 3, 9, torch.int64, 'whole'),
+                                                 (2048, 8, 1, torch.int64, 'whole'), (2047, 8, 77, torch.int32, 'shifted'),
+                                                 (1001, 5, 12, torch.int64, 'columns')])
+def test_row_tables_from_any_layout_of_ids(dev, T, topk, E, dtype, form):
+    """The ids as one array of 16-byte chunks with a remainder, as one that starts off such a boundary, and as columns of a
+    wider table; one expert that takes every entry of the largest table ranked in one launch; ids at and past the number of experts."""
+    from dlblas_amd.kernels.fused_moe_v3 import ep_scatter_rows
+    print(f'case row tables T={T} topk={topk} E={E} {dtype} {form}', flush=True)
+    g = helpers.gen(T + E)
+    lo, hi = (0, 1) if E == 1 else (-2, E + 2)
+    ids = torch.randint(lo, hi, (T, topk), generator=g).to(dtype)
+    if form == 'whole':
+        on_dev = ids.to(dev)
+    elif form == 'shifted':
+        on_dev = torch.empty(T * topk + 1, dtype=dtype, device=dev)[1:].view(T, topk).copy_(ids)
+    else:
+        on_dev = torch.empty(T, topk + 3, dtype=dtype, device=dev)[:, 1:topk + 1].copy_(ids)
+    kept = torch.where(ids < E, ids, -1).clamp(min=-1).long()
+    counts = (torch.bincount(kept[kept >= 0], minlength=E) + 127) // 128 * 128
+    rows = int(counts.sum())
+    i32 = lambda n: torch.full((n, ), -9, dtype=torch.int32, device=dev)
+    first, m_indices, src, slot = i32(E), i32(rows), i32(rows), torch.full((T, topk), -9, dtype=torch.int64, device=dev)
+    ep_scatter_rows(on_dev, counts.to(torch.int32).to(dev), first, m_indices, src, slot)
+    torch.cuda.synchronize()
+    excl, routed, dest = _row_tables_ref(kept, counts)
+    src_ref = torch.zeros(rows, dtype=torch.long)
+    src_ref[dest[dest >= 0]] = (torch.arange(T * topk) // topk)[dest >= 0]
+    assert torch.equal(src.cpu().long(), src_ref)
+    assert torch.equal(slot.cpu().flatten(), dest) and torch.equal(first.cpu().long(), excl + routed)
+    assert torch.equal(m_indices.cpu().long(), torch.repeat_interleave(torch.arange(E), counts))
+
+
 def test_gathering_gemm_on_a_table_longer_than_the_spans(dev):
     from dlblas_amd.kernels.fp8_gemm_grouped import fp8_gemm_grouped_contiguous_silu_quant
     from dlblas_amd.kernels.fused_moe_v3 import ep_scatter_rows
