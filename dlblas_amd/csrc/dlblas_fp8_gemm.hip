@@ -234,10 +234,10 @@ hipError_t launch_tiled_mode(int mode, const Args& args, int grid, int dev, hipS
   }
 }
 
-template <class Cfg, int MODE>
+template <class Cfg, int MODE, bool AHEAD = false>
 hipError_t launch_pipelined(const Args& args, int grid, int dev, hipStream_t stream) {
   static std::atomic<unsigned long long> lds_done{0};
-  auto kernel = fp8_gemm_pipelined_kernel<Cfg, MODE>;
+  auto kernel = fp8_gemm_pipelined_kernel<Cfg, MODE, AHEAD>;
   hipError_t e = ensure_lds(kernel, Cfg::LDS_BYTES, dev, &lds_done);
   if (e != hipSuccess || g_prepare_only) return e;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, args);
@@ -348,6 +348,9 @@ template <class Cfg>
 hipError_t launch_pipelined_mode(int mode, const Args& args, int grid, int dev, hipStream_t stream) {
   switch (mode) {
     case kDense:
+      // resident workgroups of more than one tile: the ring that runs on (a single tile is 1 us faster without its code)
+      if constexpr (!Cfg::PREFETCH)
+        if (static_cast<int64_t>(args.tiles_m) * args.tiles_n * args.splitk > grid) return launch_pipelined<Cfg, kDense, true>(args, grid, dev, stream);
       return launch_pipelined<Cfg, kDense>(args, grid, dev, stream);
     case kContiguous:
       return launch_pipelined<Cfg, kContiguous>(args, grid, dev, stream);
@@ -457,28 +460,49 @@ int64_t pick_mixed_split(int64_t M, int64_t N, int cus, double* makespan = nullp
     const int64_t split = ca * 256;
     if (split >= N) continue;
     const double t = mixed_makespan(tm * ca, tm * ceil_div(N - split, 192), narrow_cost, cus);
-    if (t < best - 1e-6 && t < 0.96 * uniform) best = t, best_split = split;  // a uniform launch of many rounds runs resident, worth 4 %
+    if (t < best - 1e-6 && t < 0.96 * uniform) best = t, best_split = split;  // not for less than 4 %
   }
   if (makespan) *makespan = best;
   return best_split;
 }
 
-// Prefill-sized dense problems: 256-row tiles (256 and 192 columns wide, mixed so that the rounds come out even) or
-// 128 x 256 tiles?  Both run from the L2 at the pace of the matrix pipe there - 1.62 us per K step of a 256 x 256 tile,
-// 1.0 us for 128 x 256 - and a tile costs a fixed 11.5 / 5.5 us on top (its first loads, its output; 4.3 us in a launch
-// of four rounds or more, which runs as resident workgroups; measured on MI355X, 192 ... 4096 rows, K = 512 ... 18432).
-// The larger tile wins unless its rows are mostly padding (384 rows are two 256-row tiles but three of 128), its tiles
-// leave much of a round empty (2048 x 4096: 128 tiles of 256 x 256 on 256 CUs, but 256 tiles of 128 x 256), or K is so
-// short that the fixed part decides: 384 x 18432 x 7168 82 -> 67 us, 2048 x 4096 x 7168 79 -> 67 us,
-// 4096 x 32768 x 512 166 -> 155 us.
-bool prefers_128_row_tiles(int64_t M, int64_t N, int kblocks, int cus, double* us = nullptr) {
+// Tiles of 256 rows: widths mixed so that the rounds come out even, or all equal?  us on MI355X, 256 ... 4096 rows, K = 384 ... 7168:
+//   - a workgroup per tile (one round, or a mixed launch): 11.5 + 1.62 K blocks per round, the first loads and the output of
+//     every tile included; a mixed launch of several rounds comes out 6 % above the sum of its tiles.
+//   - equal tiles, more than one round: resident workgroups whose ring runs on from tile to tile: 5.4 + 1.82 K blocks per round
+//     and 3 for the launch.
+// A last round that is not full costs 0.6 of a round plus its share of the rest (the chip is faster with fewer tiles).  33
+// launches of 1.1 to 8.8 rounds of equal tiles lie within 7 % of that, mixed ones within 10 %.
+// Mixed tiles win where K is long and the last round short (4096 x 5248 x 4096: 104 / 113 us, 2048 x 17408 x 7168: 265 / 292),
+// equal ones where the fixed part of a tile counts (3500 x 33024 x 1280: 203 / 183, 2048 x 18176 x 512: 45 / 38).
+int pick_wide_variant(int64_t M, int64_t N, int kblocks, int cus, double* us = nullptr) {
   double span = 0.0;
-  pick_mixed_split(M, N, cus, &span);
-  const double wide_us = span * (11.5 + 1.62 * kblocks);
+  const int64_t split = pick_mixed_split(M, N, cus, &span);
+  const bool mixed = split < N;
+  const int64_t tiles = ceil_div(M, 256) * ceil_div(N, 256);
+  const double lone_us = 11.5 + 1.62 * kblocks, rounds = static_cast<double>(tiles) / cus;
+  const double equal_us = tiles <= cus ? lone_us : 3.0 + (0.4 * rounds + 0.6 * static_cast<double>(ceil_div(tiles, cus))) * (5.4 + 1.82 * kblocks);
+  const double load = static_cast<double>(ceil_div(M, 256)) * (split / 256 + 0.78 * static_cast<double>(ceil_div(N - split, 192))) / cus;
+  const double mixed_us = 1.06 * (0.6 * span + 0.4 * load) * lone_us;
+  const bool equal = !mixed || equal_us <= mixed_us;
+  if (us) *us = equal ? equal_us : mixed_us;
+  return mixed && equal ? kVarPipe256x256 : kVarPipe256mix;  // without a narrow region both are the launch of equal tiles
+}
+
+// Prefill-sized dense problems: 256-row tiles (above) or 128 x 256 tiles?  Both run from the L2 at the pace of the matrix
+// pipe there; a round of 128 x 256 tiles takes 2.9 + 1.05 K blocks, its ring runs on from tile to tile as well.
+// The larger tile wins unless its rows are mostly padding (384 rows are two 256-row tiles but three of 128) or its tiles
+// leave much of a round empty (2048 x 4096: 128 tiles of 256 x 256 on 256 CUs, but 256 tiles of 128 x 256):
+// 384 x 18432 x 7168 82 -> 67 us, 2048 x 4096 x 7168 79 -> 67 us.  Up to four K blocks the output decides: fp32, which is not
+// known here, is faster in the smaller tile (2330 x 20000 x 384 54 -> 47 us), bf16 in the larger one (4096 x 32768 x 512
+// 105 against 118), so the smaller one is taken up to 12 % above the estimates, which are of bf16.
+bool prefers_128_row_tiles(int64_t M, int64_t N, int kblocks, int cus, double* us = nullptr) {
+  double wide_us = 0.0;
+  pick_wide_variant(M, N, kblocks, cus, &wide_us);
   const int64_t rounds = ceil_div(ceil_div(M, 128) * ceil_div(N, 256), cus);
-  const double half_us = static_cast<double>(rounds) * ((rounds >= 4 ? 4.3 : 5.5) + 1.0 * kblocks);
+  const double half_us = 3.0 + static_cast<double>(rounds) * (2.9 + 1.05 * kblocks);
   if (us) *us = std::min(wide_us, half_us);
-  return half_us < 0.95 * wide_us;
+  return half_us < (kblocks <= 4 ? 1.12 : 0.95) * wide_us;
 }
 
 struct Plan {
@@ -645,7 +669,7 @@ Plan make_plan(int mode, int64_t M, int64_t N, int64_t K, int cus, size_t ws_byt
     } else if (whole_blocks && mode == kDense) {
       const int64_t t256 = ceil_div(M, 256) * ceil_div(N, 256);
       if (t256 * 2 >= cus) {
-        v = prefers_128_row_tiles(M, N, kblocks, cus) ? kVarPipe128x256w8 : kVarPipe256mix;
+        v = prefers_128_row_tiles(M, N, kblocks, cus) ? kVarPipe128x256w8 : pick_wide_variant(M, N, kblocks, cus);
       } else {
         const MidChoice mid = pick_mid_plan(M, N, kblocks, cus, ws_avail);
         v = mid.variant, mid_splitk = mid.splitk;
@@ -1020,7 +1044,7 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
       case kVarPipe128x128: return kb_per <= Pipe128x128T::SCTAB_KB;
       // (dense, up to 4 K blocks: the pre-pass stays, 15.1 / 11.8 us at 2048 x 4096 x 512 - the test that a refused launch leaves no
       // pre-pass behind is about this one)
-      case kVarPipe128x256w8: return (mode != kMasked || g_forced_variant < 0) && (mode != kDense || kb_per > 4) && kb_per <= Pipe128x256w8T::SCTAB_KB;
+      case kVarPipe128x256w8: return (mode != kMasked || g_forced_variant < 0) && (mode != kDense || kb_per > 4 || ceil_div(rows, pl.bm) * ceil_div(N, pl.bn) >= 4ll * cus) && kb_per <= Pipe128x256w8T::SCTAB_KB;
       case kVarPipe256x256: case kVarPipe256mix: return kb_per <= Pipe256x256T::SCTAB_KB;
       default: return false;
     }
@@ -1073,8 +1097,11 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
     grid = (grid + 31) / 32 * 32;  // the ring kernels deal tiles to the XCDs four at a time
   }
   // Dense launches of many rounds of equal tiles run one resident workgroup per CU that walks its tiles itself (the
-  // ring kernels loop over tiles anyway): saves the hardware's per-workgroup start, 4 % at six rounds.
-  r.resident = mode == kDense && grid >= 4ll * cus;
+  // ring kernels loop over tiles anyway): saves the hardware's per-workgroup start, 4 % at six rounds.  The 256-row kernel's
+  // ring runs on from tile to tile, which pays from the second tile on (1 to 2 rounds 3 to 5 %, 2 to 4 rounds 7 %).
+  const bool runs_on = pl.variant == kVarPipe256x256 || pl.variant == kVarPipe256mix || pl.variant == kVarPipe128x256w8;
+  const bool mixed = pl.variant == kVarPipe256mix && r.n_split < N;  // a workgroup per tile
+  r.resident = mode == kDense && !mixed && grid >= (runs_on ? cus + 1ll : 4ll * cus);
   r.grid = grid;
   return r;
 }

@@ -99,6 +99,12 @@ __device__ __forceinline__ v4f coherent_load16(const float* src) {
   return v4f{lo.x, lo.y, hi.x, hi.y};
 }
 
+// f(0), f(1), ... with compile-time indices
+template <class F, int... I>
+__device__ __forceinline__ void each_index(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
 // PARTS_: 2 = the scale FMAs of a fragment run under the MFMAs of the NEXT fragment of the same wave (two partial
 // accumulators); 1 = they follow their own MFMAs and overlap with the other wave of the SIMD instead (16 fewer VGPRs).
 // PREFETCH_: true (one wave per SIMD, 512 registers) = every fragment of the NEXT K step is read into a second
@@ -172,7 +178,7 @@ constexpr int kTileListHeader = 3;  // tile counts in front of the three tile li
 
 // Work of one workgroup: tiles vb_first, vb_first + gridDim.x, ... of a region that is tiles_m x tiles_n tiles of
 // BM x BN and starts at column n_base of the output.
-template <class Cfg, int MODE>
+template <class Cfg, int MODE, bool AHEAD = false>
 __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int vb_first, int tiles_m, int tiles_n,
                                                int n_base) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, MF = Cfg::MF, NF = Cfg::NF, WAVES = Cfg::WAVES, STAGES = Cfg::STAGES;
@@ -202,7 +208,31 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
   const int tiles = tiles_m * tiles_n;
   int walk_g = 0;
   int walk_base = 0;
-
+  // Unit id of a dense launch: the tile, in patches of group_m row tiles, and the slice of K.  The K range is cut into
+  // p.splitk slices of p.kb_per_split blocks; slices of one tile are far apart in the order.
+  const int units = MODE == kDense ? tiles * p.splitk : tiles;
+  auto locate = [&](int v, int& tile, int& slice, int& tm, int& tn) __attribute__((always_inline)) {
+    const int id = xcd_remap(v, units);
+    slice = MODE == kDense ? id / tiles : 0;
+    tile = id - slice * tiles;
+    const int width = p.group_m * tiles_n;
+    const int grp = tile / width;
+    const int first_m = grp * p.group_m;
+    const int gsz = min(tiles_m - first_m, p.group_m);
+    const int in_grp = tile - grp * width;
+    tm = first_m + in_grp % gsz;
+    tn = in_grp / gsz;
+  };
+  // AHEAD (dense): the ring runs on from tile to tile.  The steps of a tile whose fetches lie past the end of K
+  // fetch the first K blocks of the workgroup's NEXT tile: its first block is on its way under the last steps and is waited
+  // for by the last one like any other, so that it lands before this tile's
+  // stores are issued (the memory counter is one for loads and stores: a load behind them is only known to have landed
+  // when they have).  A tile of 256 x 256 then takes 5.4 us on top of its K steps in place of 7.8: the stores (3 to 4 us of
+  // 128 KB per CU) and the staging of the results remain.  4096 x 24576 x 1536 177 -> 165 us, 4000 x 28160 x 768 124 -> 113,
+  // 4096 x 20480 x 1024 fp32 137 -> 127.
+  static_assert(!AHEAD || (MODE == kDense && !Cfg::PREFETCH), "the tile kernels this is written for");
+  int stage = 0;
+  bool staged = false;  // AHEAD: the ring holds the tile's first STAGES - 1 K blocks from `stage` on, and the next block's activations
   for (int vb = vb_first;; vb += gridDim.x) {
     int g = 0, mt = 0, nt, m_end, m_first = -1, split = 0, tile_lin = 0;
     if (kMaskedLike) {
@@ -251,21 +281,8 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
       g = p.gidx[m_first];
       m_end = min(p.M, m_first + BM);
     } else {
-      // dense split-K: the K range is cut into p.splitk slices of p.kb_per_split blocks, every (tile, slice) pair is a
-      // unit of work, slices of one tile far apart in the order
-      const int units = MODE == kDense ? tiles * p.splitk : tiles;
       if (vb >= units) break;
-      const int id = xcd_remap(vb, units);
-      split = MODE == kDense ? id / tiles : 0;
-      const int t = id - split * tiles;
-      tile_lin = t;
-      const int width = p.group_m * tiles_n;
-      const int grp = t / width;
-      const int first_m = grp * p.group_m;
-      const int gsz = min(tiles_m - first_m, p.group_m);
-      const int in_grp = t - grp * width;
-      mt = first_m + in_grp % gsz;
-      nt = in_grp / gsz;
+      locate(vb, tile_lin, split, mt, nt);
       m_end = p.M;
       if (MODE == kContiguous) {
         g = p.gidx[mt * BM];
@@ -285,6 +302,7 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
     // activation rows named by a table (the fused gate/up kernel reading the tokens where they lie, instead of a copy
     // sorted by expert): per-lane offsets then count from the first row of the matrix
     const bool a_indirect = MODE == kContigListAct && p.a_rows != nullptr;
+    const bool ahead = AHEAD && !sliced && p.c_lds && nk >= STAGES && vb + static_cast<int>(gridDim.x) < units;
     const uint8_t* a_tile = p.a + static_cast<int64_t>(a_indirect ? 0 : m0) * p.K + static_cast<int64_t>(kb_first) * kScaleBlock;
     const float* as_tile = p.a_s + static_cast<int64_t>(m0) * p.as_sm + static_cast<int64_t>(kb_first) * p.as_sk;
     char* c_base = static_cast<char*>(p.c);
@@ -298,7 +316,7 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
     // weight scales: lane i of the wave fetches the scale of the wave's fragment (i & 3) (fragment 0 beyond NF)
     const float* bs_g = p.b_s + static_cast<int64_t>(g) * p.bs_gs + kb_first;
     const int bs_frag = (lane & 3) < NF ? (lane & 3) : 0;
-    const uint32_t bs_off =
+    uint32_t bs_off =
         static_cast<uint32_t>(min((kAct ? w_row(wn0 + 32 * bs_frag) : n0 + wn0 + 32 * bs_frag) / kScaleBlock, p.nblocks - 1)) *
         static_cast<uint32_t>(p.kblocks) * 4u;
 
@@ -308,7 +326,7 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
     // recomputed per instruction (two VALU ops) instead of being kept in registers.  Rows past the valid range
     // re-read the last valid row.
     static_assert(WAVES % 2 == 0, "chunk swizzle must not depend on the DMA instruction index");
-    const int a_last = m_end - 1 - m0;
+    int a_last = m_end - 1 - m0;
     const int b_last = p.N - 1 - n0;
     const int dma_row = 8 * wave + (lane >> 3);
     const uint32_t dma_chunk = static_cast<uint32_t>(((lane & 7) ^ chunk_swizzle(dma_row)) * 16);
@@ -329,6 +347,36 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
 #pragma unroll
     for (int j = 0; j < Cfg::S_INST; ++j)
       s_off[j] = static_cast<uint32_t>(min((j * WAVES + wave) * 64 + lane, a_last)) * static_cast<uint32_t>(p.as_sm) * 4u;
+
+    // AHEAD: from here on the DMA addresses (of the activations / of all else) are those of the workgroup's next tile, or of
+    // this tile again without one.  Computed from the lane index alone, so that nothing is kept for it across the K loop.
+    auto point_ahead = [&](auto which) __attribute__((always_inline)) {
+      constexpr bool kActs = decltype(which)::value;
+      int tile, slice, tm, tn;
+      locate(ahead ? vb + static_cast<int>(gridDim.x) : vb, tile, slice, tm, tn);
+      const int m1 = __builtin_amdgcn_readfirstlane(tm * BM), n1 = __builtin_amdgcn_readfirstlane(n_base + tn * BN);
+      int nl = lane;
+      asm volatile("" : "+v"(nl));
+      const int row = 8 * wave + (nl >> 3);
+      const uint32_t chunk = static_cast<uint32_t>(((nl & 7) ^ chunk_swizzle(row)) * 16);
+      const int m_last = p.M - 1 - m1, n_last = p.N - 1 - n1;
+      if constexpr (kActs) {
+        a_tile = p.a + static_cast<int64_t>(m1) * p.K;
+#pragma unroll
+        for (int j = 0; j < Cfg::A_INST; ++j) a_off[j] = static_cast<uint32_t>(min(row + 8 * j * WAVES, m_last)) * uK + chunk;
+      } else {
+        as_tile = p.a_s + static_cast<int64_t>(m1) * p.as_sm;
+        b_tile = p.b + static_cast<int64_t>(n1) * p.K;
+        const int frag = (nl & 3) < NF ? (nl & 3) : 0;
+        bs_off = static_cast<uint32_t>(min((n1 + wn0 + 32 * frag) / kScaleBlock, p.nblocks - 1)) * static_cast<uint32_t>(p.kblocks) * 4u;
+        a_last = m_last;
+#pragma unroll
+        for (int j = 0; j < Cfg::B_INST; ++j) b_off[j] = static_cast<uint32_t>(min(row + 8 * j * WAVES, n_last)) * uK + chunk;
+#pragma unroll
+        for (int j = 0; j < Cfg::S_INST; ++j)
+          s_off[j] = static_cast<uint32_t>(min((j * WAVES + wave) * 64 + nl, m_last)) * static_cast<uint32_t>(p.as_sm) * 4u;
+      }
+    };
 
     auto issue_stage = [&](int kb, int stage) {
       uint8_t* sbase = smem + stage * Cfg::STAGE_BYTES;
@@ -415,13 +463,12 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
     constexpr int kScaleOff = Cfg::A_BYTES + Cfg::B_BYTES;
     constexpr int kWScaleOff = kScaleOff + Cfg::S_BYTES;
 
-    __syncthreads();  // the previous tile's readers and DMA groups are done with the ring
-    if constexpr (Cfg::SCTAB) {
-      // scale table [BM][p.sct_pitch]: entry (r, j) = a_s of tile row r at the workgroup's j-th K block.  One DMA
-      // instruction moves 64 consecutive entries, i.e. whole runs of a row's scales; issued ahead of the first stages,
-      // so the wait for stage 0 covers them.  The pitch is odd: the 32 rows a wave reads at one K block then lie in 32
-      // different banks (with a power-of-two pitch of 32 floats they shared two banks, and every such read held the
-      // LDS for 16 turns while the other waves' fragment reads waited: 256 x 7168 x 4096 27.2 -> 24 us).
+    // scale table [BM][p.sct_pitch]: entry (r, j) = a_s of tile row r at the workgroup's j-th K block.  One DMA
+    // instruction moves 64 consecutive entries, i.e. whole runs of a row's scales; issued ahead of the first stages,
+    // so the wait for stage 0 covers them.  The pitch is odd: the 32 rows a wave reads at one K block then lie in 32
+    // different banks (with a power-of-two pitch of 32 floats they shared two banks, and every such read held the
+    // LDS for 16 turns while the other waves' fragment reads waited: 256 x 7168 x 4096 27.2 -> 24 us).
+    auto issue_table = [&]() __attribute__((always_inline)) {
       const int pitch = p.sct_pitch;
       const float inv_pitch = 1.0f / static_cast<float>(pitch);
       const int n_inst = (BM * pitch + 63) >> 6;
@@ -433,21 +480,50 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
         dma_4(reinterpret_cast<const uint8_t*>(as_tile),
               (r * static_cast<uint32_t>(p.as_sm) + j * static_cast<uint32_t>(p.as_sk)) * 4u, smem + Cfg::SCTAB_OFF + i * 256);
       }
-    }
+    };
     // kExactK: only K blocks that exist are fetched - a tile shorter than the ring, and the last STAGES steps of every
     // tile, issue nothing (wave-uniform branches), so no load is in flight when the tile ends and the next tile starts
     // without waiting for loads nobody reads.  The kernels whose wave tile fills the register file (64 x 128) cannot
     // afford those branches' scalar registers inside the K loop (wave tiles above 64 x 64): they keep every step the same code, fetch the last
     // block again past the end of K into a stage nobody reads, and drain at the end of the tile.
     constexpr bool kExactK = MF * NF <= 4;
+    // DMA slots of a K step: the group that refills the step's stage starts at the barrier slot kP and is spread over kSlots
+    // tile slots, wrapping into the next step (whose slots t < kP therefore finish the PREVIOUS step's group)
+    constexpr int kP = (S - 1) * H;
+    constexpr int kSlots = T >= 8 ? 5 : (T >= 4 ? 3 : 1);  // measured: 3 to 5 of 8 slots are equally good, 6 and 7 leave the loads too little time
+    constexpr int L = Cfg::LOADS_PER_STAGE;
+    // The first H slots' part of a group is issued by its own step, the rest by the next one.  AHEAD: that part is the
+    // activations, all of them and nothing else, and all that the prologue issues of its last group.
+    constexpr auto part_begin = [](int q) {
+      return AHEAD ? (q <= H ? q * Cfg::A_INST / H : Cfg::A_INST + (q - H) * (L - Cfg::A_INST) / (kSlots - H)) : q * L / kSlots;
+    };
+    constexpr int kFirstPart = !AHEAD ? L : part_begin(H < kSlots ? H : kSlots);
+    auto issue_first_part = [&](int kb, int stg) __attribute__((always_inline)) {
+      each_index([&](auto i) __attribute__((always_inline)) { issue_one(i, kb, stg); }, std::make_integer_sequence<int, kFirstPart>{});
+    };
+    if (!AHEAD) stage = 0;
+    if (AHEAD && staged) {
+      lds_barrier();  // the previous tile's results have been read from the ring, the scale table has landed
+    } else {
+      __syncthreads();  // the previous tile's readers and DMA groups are done with the ring
+      if constexpr (Cfg::SCTAB) issue_table();
 #pragma unroll
-    for (int s = 0; s < STAGES; ++s)
-      if (!kExactK || s < nk) issue_stage(min(s, nk - 1), s);
-    if (!kExactK || nk >= STAGES)
-      wait_vmcnt<(STAGES - 1) * Cfg::LOADS_PER_STAGE>();  // all but the first stage's group may still be on their way
-    else
-      wait_vmcnt<0>();
-    lds_barrier();
+      for (int s = 0; s < STAGES; ++s) {
+        if (kExactK && s >= nk) continue;
+        const int stg = AHEAD ? (stage + s) % STAGES : s;
+        if (s < STAGES - 1)
+          issue_stage(min(s, nk - 1), stg);
+        else
+          issue_first_part(min(s, nk - 1), stg);
+      }
+      if (!kExactK || nk >= STAGES)
+        wait_vmcnt<(STAGES - 2) * L + kFirstPart>();  // all but the first stage's group may still be on their way
+      else
+        wait_vmcnt<0>();
+      lds_barrier();
+    }
+    staged = ahead;
+    const int base0 = AHEAD ? stage * Cfg::STAGE_BYTES : 0;
 
     // first table entry of this lane's rows (scale-table kernels)
     int tab_row[MF];
@@ -537,7 +613,6 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
       };
       typedef std::integral_constant<int, 0> B0;
       typedef std::integral_constant<int, 1> B1;
-      int stage = 0;
       int kb = 0;
       for (; kb + 1 < nk; kb += 2) {
         k_step(B0{}, kb, stage);
@@ -570,14 +645,14 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
         for (int j = 0; j < NS; ++j) dst[mi][j] = sa * sb[j];
       }
     };
-    load_scales(0, 0, sc);
+    load_scales(base0, 0, sc);
 #pragma unroll
     for (int hi = 0; hi < H; ++hi) {
-      hf[hi][0] = lds_read_frag32(smem, held0 + hi * kFragBytes, lc, 0);
-      hf[hi][1] = lds_read_frag32(smem, held0 + hi * kFragBytes, lc, 1);
+      hf[hi][0] = lds_read_frag32(smem, base0 + held0 + hi * kFragBytes, lc, 0);
+      hf[hi][1] = lds_read_frag32(smem, base0 + held0 + hi * kFragBytes, lc, 1);
     }
-    sf[0] = lds_read_frag32(smem, strm0, lc, 0);
-    sf[1] = lds_read_frag32(smem, strm0, lc, 1);
+    sf[0] = lds_read_frag32(smem, base0 + strm0, lc, 0);
+    sf[1] = lds_read_frag32(smem, base0 + strm0, lc, 1);
 
     // One K step; every step is the same code (see the note in the register-double-buffered path above).
     auto k_step = [&](int kb, int stage) __attribute__((always_inline)) {
@@ -585,22 +660,21 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
       const int cur_base = stage * Cfg::STAGE_BYTES;
       const int nxt_base = next_stage * Cfg::STAGE_BYTES;
       float sc_next[MF][NS];
-      // DMA slots: the group that refills this step's stage starts at the barrier slot kP and is spread over kSlots
-      // tile slots, wrapping into the next step (whose slots t < kP therefore finish the PREVIOUS step's group)
-      constexpr int kP = (S - 1) * H;
-      constexpr int kSlots = T >= 8 ? 5 : (T >= 4 ? 3 : 1);  // measured: 3 to 5 of 8 slots are equally good, 6 and 7 leave the loads too little time
-      constexpr int L = Cfg::LOADS_PER_STAGE;
       const int prev_stage = stage == 0 ? STAGES - 1 : stage - 1;
-      const int kb_new = kExactK ? kb + STAGES : min(kb + STAGES, nk - 1), kb_prev = kExactK ? kb + STAGES - 1 : min(kb + STAGES - 1, nk - 1);
-      const bool do_new = !kExactK || kb_new < nk, do_prev = !kExactK || kb_prev < nk;  // kExactK: K blocks past the end are not fetched
+      // past the end of K: the next tile's first blocks (AHEAD), nothing (kExactK), or the last block again
+      auto block = [&](int k) { return AHEAD ? (k < nk ? k : min(k - nk, nk - 1)) : kExactK ? k : min(k, nk - 1); };
+      const int kb_new = block(kb + STAGES), kb_prev = block(kb + STAGES - 1);
+      const bool do_new = !kExactK || ahead || kb + STAGES < nk, do_prev = !kExactK || ahead || kb + STAGES - 1 < nk;
       auto issue_slot = [&](auto qtag, int kbx, int stg) __attribute__((always_inline)) {
         constexpr int q = decltype(qtag)::value;
-        constexpr int i0 = q * L / kSlots, i1 = (q + 1) * L / kSlots;
+        constexpr int i0 = part_begin(q), i1 = part_begin(q + 1);
         if constexpr (i0 + 0 < i1) issue_one(std::integral_constant<int, i0 + 0>{}, kbx, stg);
         if constexpr (i0 + 1 < i1) issue_one(std::integral_constant<int, i0 + 1>{}, kbx, stg);
         if constexpr (i0 + 2 < i1) issue_one(std::integral_constant<int, i0 + 2>{}, kbx, stg);
         if constexpr (i0 + 3 < i1) issue_one(std::integral_constant<int, i0 + 3>{}, kbx, stg);
-        static_assert(i1 - i0 <= 4, "at most four DMA instructions per slot");
+        if constexpr (i0 + 4 < i1) issue_one(std::integral_constant<int, i0 + 4>{}, kbx, stg);
+        if constexpr (i0 + 5 < i1) issue_one(std::integral_constant<int, i0 + 5>{}, kbx, stg);
+        static_assert(i1 - i0 <= 6, "at most six DMA instructions per slot");
       };
 #pragma unroll
       for (int t = 0; t < T; ++t) {
@@ -611,7 +685,7 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
           // purpose; what a launch gains by it is what that part costs.  Never defined in the library build.)
 #ifndef DLB_ABLATE_VMCNT
           // the group of step kb + 1 has landed: behind it at most STAGES - 2 younger groups are out, fewer at the tile's end
-          if (kExactK && kb + STAGES > nk)
+          if (kExactK && !ahead && kb + STAGES > nk)
             wait_vmcnt<0>();
           else
             wait_vmcnt<(STAGES - 2) * Cfg::LOADS_PER_STAGE>();
@@ -713,13 +787,17 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
 #pragma unroll
         for (int j = 0; j < NS; ++j) sc[m2][j] = sc_next[m2][j];
     };
-    int stage = 0;
     for (int kb = 0; kb < nk; ++kb) {
+      if (AHEAD && (ahead || !kExactK)) {
+        if (kb == max(nk - STAGES, 0)) point_ahead(std::true_type{});
+        if (kb == max(nk - STAGES + 1, 0)) point_ahead(std::false_type{});
+      }
       k_step(kb, stage);
       stage = stage + 1 == STAGES ? 0 : stage + 1;
     }
     if (Cfg::PARTS == 2) acc[MF - 1][NF - 1] += part[(T - 1) & 1] * sc_last;
-    if (!kExactK) wait_vmcnt<0>();  // the trailing re-read groups must not land in the next tile's ring
+    if (AHEAD && Cfg::SCTAB && ahead) issue_table();  // every wave has read the scales of the last K block
+    if (!kExactK && !ahead) wait_vmcnt<0>();  // the trailing re-read groups must not land in the next tile's ring
     }
 
     // epilogue: lane holds c[m0 + wm0 + 32 mi + (lane & 31)][n0 + wn0 + 32 ni + 8 u + 4 (lane >> 5) + 0..3], u = 0..3
@@ -957,6 +1035,65 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
           store_rows(std::false_type{});
       }
     };
+    if (AHEAD && p.c_lds && !sliced) {
+      // The same through the weight part of the last step's stage, 32 rows x 128 bytes of a wave at a time: the rest of the
+      // ring belongs to the next tile already.
+      static_assert(!AHEAD || 32 * 128 * WAVES <= Cfg::B_BYTES, "the staging slices fit in the weights of a stage");
+      uint8_t* idle = smem + (stage == 0 ? STAGES - 1 : stage - 1) * Cfg::STAGE_BYTES + Cfg::A_BYTES;
+      auto store_wave_tile = [&](auto f32, auto inside) __attribute__((always_inline)) {
+        constexpr bool F32 = decltype(f32)::value;
+        constexpr int NP = F32 ? 1 : 2;        // column fragments of a pass
+        constexpr int kEl = F32 ? 4 : 2;
+        constexpr int kRowBytes = NP * 32 * kEl;
+        constexpr int kCpr = kRowBytes / 16;   // 16-byte chunks per row
+        constexpr int kRpi = 64 / kCpr;        // rows per store instruction
+        uint8_t* st = idle + wave * (32 * kRowBytes);
+        const int r_in = el / kCpr, ch = el % kCpr;
+#pragma unroll
+        for (int mi = 0; mi < MF; ++mi)
+#pragma unroll
+          for (int nb = 0; nb < NF; nb += NP) {
+#pragma unroll
+            for (int ni = nb; ni < nb + NP; ++ni)
+#pragma unroll
+              for (int u = 0; u < 4; ++u) {
+                const v4f v = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
+                if constexpr (F32)
+                  *reinterpret_cast<v4f*>(st + el32 * kRowBytes + (2 * u + eh + el32) % kCpr * 16) = v;
+                else
+                  *reinterpret_cast<v4bf*>(st + el32 * kRowBytes + ((ni - nb) * 4 + u + el32) % kCpr * 16 + eh * 8) = __builtin_convertvector(v, v4bf);
+              }
+            if (Cfg::SCTAB && mi == 0 && nb == 0) wait_vmcnt<0>();  // the table, ahead of the stores
+            const int col = n0 + wn0 + nb * 32 + ch * (16 / kEl);
+            const int n_left = p.N - col;
+            char* c_col = c_base + static_cast<int64_t>(col) * kEl;
+#pragma unroll
+            for (int r0 = 0; r0 < 32; r0 += kRpi) {
+              const int row = r0 + r_in;
+              const v4i v = *reinterpret_cast<const v4i*>(st + row * kRowBytes + (ch + row) % kCpr * 16);
+              const int m = m0 + wm0 + mi * 32 + row;
+              if (m >= m_end || !(inside || n_left > 0)) continue;
+              char* dst = c_col + static_cast<int64_t>(m) * p.N * kEl;
+              if constexpr (F32)
+                store_row4<true>(dst, 0, __builtin_bit_cast(v4f, v), inside ? 4 : n_left);
+              else
+                store_row8_bf16(reinterpret_cast<__bf16*>(dst), v, inside ? 8 : n_left);
+            }
+          }
+      };
+      if (p.out_f32) {
+        if (cols_inside)
+          store_wave_tile(std::true_type{}, std::true_type{});
+        else
+          store_wave_tile(std::true_type{}, std::false_type{});
+      } else {
+        if (cols_inside)
+          store_wave_tile(std::false_type{}, std::true_type{});
+        else
+          store_wave_tile(std::false_type{}, std::false_type{});
+      }
+      continue;
+    }
     if (sliced) {
       // first pass of split-K: the slice's sums go to the workspace as an fp32 [M][N] matrix of their own;
       // fp8_splitk_reduce_kernel, launched behind this kernel on the same stream, adds the slices in index order
@@ -1027,10 +1164,10 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
   }
 }
 
-template <class Cfg, int MODE>
+template <class Cfg, int MODE, bool AHEAD>
 __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_pipelined_kernel(const Args p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  pipelined_body<Cfg, MODE>(p, smem, blockIdx.x, p.tiles_m, p.tiles_n, 0);
+  pipelined_body<Cfg, MODE, AHEAD>(p, smem, blockIdx.x, p.tiles_m, p.tiles_n, 0);
 }
 
 // Dense GEMM whose columns are cut at p.n_split into a region of CfgA tiles and a region of narrower CfgB tiles,

@@ -188,6 +188,21 @@ def test_scale_table_of_every_ring_kernel(dev, layout, variant, rows, N, blocks)
         helpers.tolerance_check(last[:ref.size(0)], ref, f'{layout} {variant}')
 
 
+@pytest.mark.parametrize('variant,M', [('pipe256x256', 260), ('pipe128x256w8', 132)])
+@pytest.mark.parametrize('kb,dtype', [(1, torch.bfloat16), (2, torch.float32), (3, torch.bfloat16), (4, torch.float32), (17, torch.bfloat16),
+                                      (27, torch.bfloat16), (28, torch.float32)])
+def test_tiles_of_a_resident_workgroup(dev, variant, M, kb, dtype):
+    """258 tiles of 256 columns on 256 resident workgroups or fewer: the ring runs on into the next tile from as many K blocks
+    on as it has stages; a last row tile of 4 rows and a last column tile of 233 columns, so that a workgroup goes from a
+    whole tile to a ragged one; K on both sides of the longest whose scales come from the table."""
+    N, K = 33001, kb * 128
+    print(f'case resident tiles {variant} K={K} {dtype}', flush=True)
+    a_q, a_s, b_q, b_s = helpers.make_dense(M, N, K, seed=kb)
+    outs = [_run_dense(dev, a_q, a_s, b_q, b_s, dtype=dtype, variant=variant) for _ in range(2)]
+    assert torch.equal(outs[0], outs[1])
+    helpers.tolerance_check(outs[0], orc.dequant_ref(a_q, a_s, b_q, b_s), f'resident tiles {variant} K={K}')
+
+
 def test_refused_launch_enqueues_nothing(dev):
     """A call whose main kernel cannot be launched (here: a forced request for more LDS than the GPU has) returns
     DLB_ERR_LAUNCH before any pre-pass is enqueued: workspace and output keep their bytes."""
