@@ -412,8 +412,8 @@ int dlb_fp8_gemm_plan_grouped(int mode, int64_t rows, int64_t N, int64_t K, int3
  * Whether the weight-streaming kernel takes a masked launch over from the variant dlb_fp8_gemm_plan_grouped names, and with
  * which tile: rows, weight rows and whether it reads its fragments one step ahead, all 0 when it does not.  `quantising` != 0
  * asks for dlb_fp8_gemm_grouped_masked_silu_quant (N = its weight rows), 0 for dlb_fp8_gemm_grouped_masked.  The ragged entry
- * points run the same choice with rows = M_sum and have no other kernel: they decline where this says 0.  No counterpart in
- * the reference.
+ * points choose the same tiles with rows = M_sum and weigh them against the expert-contiguous kernels, whose padded rows they
+ * replace: dlb_expert_plan (mode 1) says whether they take a call.  No counterpart in the reference.
  */
 int dlb_fp8_gemm_plan_stream(int64_t rows, int64_t N, int64_t K, int32_t G, int32_t expected_m, int quantising, int compute_units,
                              int* tile_rows, int* tile_columns, int* ahead);
