@@ -109,8 +109,8 @@ def ep_gather(
 def _scales(rows, blocks, form, device):
     """[rows, blocks] fp32 in the order the down GEMM of this form reads in place: rows whole, or the rows of a K block together."""
     if form == _lib.ON_ROW_RANGES:
-        return torch.empty((rows, blocks), device=device)
-    return torch.empty((blocks, rows), device=device).t()
+        return torch.empty((rows, blocks), device=device, dtype=torch.float32)
+    return torch.empty((blocks, rows), device=device, dtype=torch.float32).t()
 
 
 def _down(act, w2_weight_fp8, row_expert, out):

@@ -227,6 +227,32 @@ def _small_experts(dev, E=2, H=512, inter=512):
     return (codes(E, 2 * inter, H), torch.ones(E, 2 * inter // 128, H // 128, device=dev)), (codes(E, H, inter), torch.ones(E, H // 128, inter // 128, device=dev)), codes
 
 
+@pytest.mark.parametrize('inter,down_form', [(256, 'ON_WHOLE_BLOCKS'), (512, 'ON_ROW_RANGES')])
+def test_fused_moe_v3_on_its_python_path_under_a_16_bit_default_dtype(dev, inter, down_form):
+    """The default dtype is the type fp8_gemm returns; it changes no scale and no bit of an expert MLP, in either order of the scales
+    between its GEMMs."""
+    from dlblas_amd import _fast, _lib
+    from dlblas_amd.kernels.fused_moe_v3 import fused_moe_v3
+    H, T = 512, 40
+    w13, w2, codes = _small_experts(dev, 2, H, inter)
+    x = codes(T, H), torch.full((T, H // 128), 2e-3, device=dev)
+    ids = (torch.arange(2 * T, device=dev) % 2).view(T, 2)
+    wts, counts = torch.ones(T, 2, device=dev), [128, 128]
+    plan = lambda n, k, quantising: _lib.expert_plan(1, 256, n, k, 2, 40, quantising)
+    assert (plan(2 * inter, H, True), plan(H, inter, False)) == (_lib.ON_ROW_RANGES, getattr(_lib, down_form))
+    print(f'case 16-bit default dtype {down_form}', flush=True)
+    ref = _fast.fused_moe_v3(*x, ids, wts, *w13, *w2, counts)
+    prev = torch.get_default_dtype()
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        with torch.overrides.BaseTorchFunctionMode():
+            out = fused_moe_v3(x, ids, wts, w13, w2, counts)
+    finally:
+        torch.set_default_dtype(prev)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref) and bool(out.isfinite().all()) and float(out.abs().max()) > 0
+
+
 def test_native_calls_are_ops_to_the_profiler(dev):
     """Every native call leaves an op event, with its inputs' shapes where they are asked for."""
     from dlblas_amd.kernels.fp8 import per_token_group_quant_fp8

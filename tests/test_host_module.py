@@ -48,3 +48,20 @@ def test_the_module_is_used_when_it_is_there(fresh):
         warnings.simplefilter('error')
         assert _fast.fp8_gemm is not _fast._declined
         assert _fast.fp8_gemm(1, 2, 3, 4) is None  # not tensors: left to the Python path
+
+
+@pytest.mark.parametrize('form', [_lib.ON_ROW_RANGES, _lib.ON_WHOLE_BLOCKS])
+def test_scales_between_the_expert_gemms_are_float32(form):
+    """The kernels write 32 bits per scale, whatever the default dtype (it chooses the type fp8_gemm returns)."""
+    import importlib
+
+    import torch
+    moe = importlib.import_module('dlblas_amd.kernels.fused_moe_v3')
+    prev = torch.get_default_dtype()
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        s = moe._scales(256, 16, form, 'cpu')
+    finally:
+        torch.set_default_dtype(prev)
+    assert s.dtype == torch.float32 and tuple(s.shape) == (256, 16) and s.untyped_storage().nbytes() == 256 * 16 * 4
+    assert s.stride() == ((16, 1) if form == _lib.ON_ROW_RANGES else (1, 256))
