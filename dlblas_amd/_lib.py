@@ -493,9 +493,33 @@ def ep_scatter_rows_host(recv_topk, counts, row_start, row_end, expert_start_loc
     return True
 
 
+def _check_ragged(a, b, a_s, b_s, out, row_start, row_end, out_s=None, a_row_index=None):
+    """What the library cannot see behind a pointer: types, shapes and layouts of a problem on row ranges (out_s: of the quantising
+    forms, whose result is half as wide)."""
+    f8, f32, i32 = torch.float8_e4m3fn, torch.float32, torch.int32
+    typed = [('a', a, f8), ('b', b, f8), ('a_s', a_s, f32), ('b_s', b_s, f32), ('row_start', row_start, i32), ('row_end', row_end, i32)]
+    typed += [] if out_s is None else [('out_q', out, f8), ('out_s', out_s, f32)]
+    typed += [] if a_row_index is None else [('a_row_index', a_row_index, i32)]
+    for name, t, dt in typed:
+        if t.dtype != dt:
+            raise TypeError(f'{name} must be {dt}, got {t.dtype}')
+    for t in (a, b, b_s, out, row_start, row_end) + (() if a_row_index is None else (a_row_index, )):
+        assert t.is_contiguous(), 'Input tensors must be contiguous'
+    G, N, K = b.shape
+    rows, blocks = out.size(0), lambda n: -(-n // 128)
+    shapes = [('a', a, (rows if a_row_index is None else a.size(0), K)), ('a_s', a_s, (a.size(0), blocks(K))), ('b_s', b_s, (G, blocks(N), blocks(K))),
+              ('out', out, (rows, N if out_s is None else N // 2)), ('row_start', row_start, (G, )), ('row_end', row_end, (G, ))]
+    shapes += [] if out_s is None else [('out_s', out_s, (rows, N // 256))]
+    shapes += [] if a_row_index is None else [('a_row_index', a_row_index, (rows, ))]
+    for name, t, shape in shapes:
+        if tuple(t.shape) != shape:
+            raise ValueError(f'{name} must be {list(shape)}, got {list(t.shape)}')
+
+
 def expert_gate_up_ragged(a, b, a_s, b_s, out_q, out_s, row_start, row_end, a_row_index, expected_m, eps) -> bool:
     """dlb_expert_gate_up_ragged (a_row_index: None or the source row of every GEMM row); False when declined."""
-    _require_gpu(a, b, a_s, b_s, out_q, out_s, row_start, row_end)
+    _check_ragged(a, b, a_s, b_s, out_q, row_start, row_end, out_s, a_row_index)
+    _require_gpu(a, b, a_s, b_s, out_q, out_s, row_start, row_end, *(() if a_row_index is None else (a_row_index, )))
     lib = load()
     G, N, K = b.shape
     stream = torch.cuda.current_stream(a.device).cuda_stream
@@ -512,6 +536,7 @@ def expert_gate_up_ragged(a, b, a_s, b_s, out_q, out_s, row_start, row_end, a_ro
 
 def gemm_ragged(a, b, a_s, b_s, c, row_start, row_end, expected_m) -> bool:
     """dlb_fp8_gemm_grouped_ragged; False when the library declines the shape (nothing enqueued)."""
+    _check_ragged(a, b, a_s, b_s, c, row_start, row_end)
     _require_gpu(a, b, a_s, b_s, c, row_start, row_end)
     lib = load()
     G, N, K = b.shape
@@ -526,7 +551,8 @@ def gemm_ragged(a, b, a_s, b_s, c, row_start, row_end, expected_m) -> bool:
 
 def gemm_ragged_silu_quant(a, b, a_s, b_s, out_q, out_s, row_start, row_end, a_row_index, expected_m, eps) -> bool:
     """dlb_fp8_gemm_grouped_ragged_silu_quant (a_row_index: None or the source row of every GEMM row); False when declined."""
-    _require_gpu(a, b, a_s, b_s, out_q, out_s, row_start, row_end)
+    _check_ragged(a, b, a_s, b_s, out_q, row_start, row_end, out_s, a_row_index)
+    _require_gpu(a, b, a_s, b_s, out_q, out_s, row_start, row_end, *(() if a_row_index is None else (a_row_index, )))
     lib = load()
     G, N, K = b.shape
     with torch.cuda.device(a.device):

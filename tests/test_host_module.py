@@ -65,3 +65,28 @@ def test_scales_between_the_expert_gemms_are_float32(form):
         torch.set_default_dtype(prev)
     assert s.dtype == torch.float32 and tuple(s.shape) == (256, 16) and s.untyped_storage().nbytes() == 256 * 16 * 4
     assert s.stride() == ((16, 1) if form == _lib.ON_ROW_RANGES else (1, 256))
+
+
+@pytest.mark.parametrize('wrong,error', [
+    ({}, RuntimeError),  # nothing but the device
+    ({'out_s': lambda t: t.bfloat16()}, TypeError),
+    ({'b_s': lambda t: t.double()}, TypeError),
+    ({'row_start': lambda t: t.long()}, TypeError),
+    ({'b': lambda t: t.transpose(1, 2).contiguous().transpose(1, 2)}, AssertionError),
+    ({'b_s': lambda t: t[:, :1]}, AssertionError),
+    ({'a_s': lambda t: t[:, :1]}, ValueError),
+    ({'out_s': lambda t: t[:-1]}, ValueError),
+    ({'out': lambda t: t[:-1]}, ValueError),
+    ({'a_row_index': lambda t: t[:-1]}, ValueError),
+])
+def test_row_range_gemms_check_what_goes_behind_a_pointer(wrong, error):
+    import torch
+    f8 = lambda *s: torch.zeros(*s, dtype=torch.uint8).view(torch.float8_e4m3fn)
+    args = dict(a=f8(5, 256), b=f8(2, 512, 256), a_s=torch.ones(5, 2), b_s=torch.ones(2, 4, 2), out=f8(256, 256), out_s=torch.ones(2, 256).t(),
+                row_start=torch.zeros(2, dtype=torch.int32), row_end=torch.zeros(2, dtype=torch.int32),
+                a_row_index=torch.zeros(256, dtype=torch.int32))
+    for name, change in wrong.items():
+        args[name] = change(args[name])
+    for call in (_lib.expert_gate_up_ragged, _lib.gemm_ragged_silu_quant):
+        with pytest.raises(error):
+            call(*(args[n] for n in ('a', 'b', 'a_s', 'b_s', 'out', 'out_s', 'row_start', 'row_end', 'a_row_index')), 64, 1e-10)
