@@ -1215,6 +1215,7 @@ int run_ragged(const RaggedProblem& pr) {
   ar.act_eps = pr.eps;
   ar.act_cols = static_cast<int>(pr.N / 2);
   ar.act_q_stride = pr.N / 2;
+  ar.c_whole = !ar.out_f32 && pr.N % 8 == 0;
   if (usable_ws) ar.ws = reinterpret_cast<float*>(static_cast<char*>(pr.ws) + DLB_WS_COUNTER_BYTES);
   const WorkspaceLock lock(pr.ws);
   const hipError_t e = launch_stream_plan(sp, pr.act ? kSiluQuant : kStoreProduct, ar, pr.G + pr.M_sum / kStreamDims[sp.shape].bm,
@@ -1354,6 +1355,7 @@ int run(const Problem& pr) {
   ar.act_eps = pr.act_eps;
   ar.act_cols = static_cast<int>(pr.N / 2);
   ar.act_q_stride = pr.N / 2;
+  ar.c_whole = !ar.out_f32 && pr.N % 8 == 0;
   ar.c_lds = g_knob[kKnobEpilogue] != 2;
   if (pr.ws && pr.ws_bytes >= DLB_WS_COUNTER_BYTES) {
     ar.ctr = static_cast<uint32_t*>(pr.ws);
