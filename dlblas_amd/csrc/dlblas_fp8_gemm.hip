@@ -1042,9 +1042,7 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
     switch (pl.variant) {
       case kVarPipe128x64: return mode == kDense && kb_per <= Pipe128x64T::SCTAB_KB;
       case kVarPipe128x128: return kb_per <= Pipe128x128T::SCTAB_KB;
-      // (dense, up to 4 K blocks: the pre-pass stays, 15.1 / 11.8 us at 2048 x 4096 x 512 - the test that a refused launch leaves no
-      // pre-pass behind is about this one)
-      case kVarPipe128x256w8: return (mode != kMasked || g_forced_variant < 0) && (mode != kDense || kb_per > 4 || ceil_div(rows, pl.bm) * ceil_div(N, pl.bn) >= 4ll * cus) && kb_per <= Pipe128x256w8T::SCTAB_KB;
+      case kVarPipe128x256w8: return (mode != kMasked || g_forced_variant < 0) && kb_per <= Pipe128x256w8T::SCTAB_KB;
       case kVarPipe256x256: case kVarPipe256mix: return kb_per <= Pipe256x256T::SCTAB_KB;
       default: return false;
     }

@@ -209,7 +209,7 @@ def test_refused_launch_enqueues_nothing(dev):
     import ctypes
     from dlblas_amd import _lib
     lib = _lib.load()
-    M, N, K = 2048, 4096, 512  # row-major scales, 256-row tiles: the call starts with a scale re-layout pass
+    M, N, K = 2048, 4096, 512  # row-major scales that are not to come through the table in LDS: the call starts with a re-layout pass
     a_q, a_s, b_q, b_s = (t.to(dev) for t in helpers.make_dense(M, N, K, seed=5))
     out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=dev)
     ws = torch.full((_lib.WORKSPACE_BYTES, ), 0x5a, dtype=torch.uint8, device=dev)
@@ -218,17 +218,49 @@ def test_refused_launch_enqueues_nothing(dev):
     args = (vp(a_q.data_ptr()), vp(b_q.data_ptr()), vp(a_s.data_ptr()), vp(b_s.data_ptr()), vp(out.data_ptr()), M, N, K, a_s.stride(0),
             a_s.stride(1), _lib.OUT_BF16, vp(ws.data_ptr()), ws.numel(), vp(torch.cuda.current_stream().cuda_stream))
     try:
+        _lib.tune('scale_table', 2)
         _lib.tune('lds_oversize', 1)
         rc = lib.dlb_fp8_gemm(*args)
+        _lib.tune('lds_oversize', 0)
+        torch.cuda.synchronize()
+        assert rc == _lib.ERR_LAUNCH and 'nothing enqueued' in _lib.last_error()
+        assert bool((ws[_lib.WS_COUNTER_BYTES:] == 0x5a).all()) and bool((out == 7.0).all())
+        assert lib.dlb_fp8_gemm(*args) == 0  # the same call goes through once the hook is off ...
     finally:
         _lib.tune('lds_oversize', 0)
-    torch.cuda.synchronize()
-    assert rc == _lib.ERR_LAUNCH and 'nothing enqueued' in _lib.last_error()
-    assert bool((ws[_lib.WS_COUNTER_BYTES:] == 0x5a).all()) and bool((out == 7.0).all())
-    assert lib.dlb_fp8_gemm(*args) == 0  # the same call goes through once the hook is off ...
+        _lib.tune('scale_table', 0)
     torch.cuda.synchronize()
     assert not bool((ws[_lib.WS_COUNTER_BYTES:] == 0x5a).all())  # ... and it does use the workspace
     helpers.tolerance_check(out, orc.dequant_ref(a_q.cpu(), a_s.cpu(), b_q.cpu(), b_s.cpu()), 'after a refused launch')
+
+
+@pytest.mark.parametrize('M,N,K', [(2048, 4096, 512), (1000, 8192, 384), (2048, 8192, 256), (2048, 4096, 128), (200, 30000, 512)])
+def test_short_k_takes_its_scales_from_the_table(dev, M, N, K):
+    """One to four K blocks in the 128 x 256 tiles the planner picks there: no launch in front of the GEMM, so the workspace keeps
+    its bytes; the bits of scales fetched through the re-layout pass."""
+    import ctypes
+
+    from dlblas_amd import _lib
+    print(f'case short K {M}x{N}x{K}', flush=True)
+    assert _lib.plan(0, M, N, K)[:2] == ('pipe128x256w8', 1) and _lib.plan_wave_k(M, N, K) is None
+    a_q, a_s, b_q, b_s = (t.to(dev) for t in helpers.make_dense(M, N, K, seed=43))
+    vp, stream, outs = ctypes.c_void_p, torch.cuda.current_stream().cuda_stream, []
+    for knob in (0, 2):
+        out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+        ws = torch.full((_lib.WORKSPACE_BYTES, ), 0x5a, dtype=torch.uint8, device=dev)
+        ws[:_lib.WS_COUNTER_BYTES] = 0
+        try:
+            _lib.tune('scale_table', knob)
+            rc = _lib.load().dlb_fp8_gemm(vp(a_q.data_ptr()), vp(b_q.data_ptr()), vp(a_s.data_ptr()), vp(b_s.data_ptr()), vp(out.data_ptr()), M, N, K,
+                                          a_s.stride(0), a_s.stride(1), _lib.OUT_BF16, vp(ws.data_ptr()), ws.numel(), vp(stream))
+        finally:
+            _lib.tune('scale_table', 0)
+        torch.cuda.synchronize()
+        assert rc == 0
+        assert bool((ws[_lib.WS_COUNTER_BYTES:] == 0x5a).all()) == (knob == 0 or K == 128)  # scales of one K block are never laid out again
+        outs.append(out)
+    assert torch.equal(*outs)
+    helpers.tolerance_check(outs[0], orc.dequant_ref(*(t.cpu() for t in (a_q, a_s, b_q, b_s))), f'short K {M}x{N}x{K}')
 
 
 @pytest.mark.parametrize('variant', ['pipe256x256', 'pipe128x256w8', 'pipe256mix', 'pipe128x128', 'pipe128x64'])
