@@ -279,7 +279,8 @@ __global__ void __launch_bounds__(kCopyThreads) ep_scatter_copy_kernel(const Sca
 // ballot per id bit) on top of the counts of the waves before it.  What it has to know of the other blocks' entries:
 //   kRowsAlone: it reads the ids of every entry itself and counts them in LDS (up to kRowsOneLaunch entries; a contiguous table
 //     through 16-byte loads that are all in flight at once and one atomic per routed entry: 16384 entries 8.1 -> 5.5 us, 8000
-//     5.6 -> 4.6 us against element loads with a division each.  At 24000 entries the two launches of kRowsSum are ahead, 6.1 / 6.4 us);
+//     5.6 -> 4.5 us against element loads with a division each; other layouts 8.1 -> 6.9 and 5.6 -> 5.1 us, four loads in flight and
+//     no division.  At 24000 entries the two launches of kRowsSum are ahead, 6.1 / 6.4 us);
 //   kRowsSum: ep_scatter_count_kernel has left the blocks' histograms, and the rows of the blocks before (for the padding
 //     also behind) are added up 8 loads at a time (65536 entries: 15.3 -> 5.3 us against one dependent load after the other);
 //   kRowsScanned: many blocks; ep_scatter_scan_kernel has turned the histograms into first rows.
@@ -315,14 +316,15 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
     const int mine = b * p.tokens_per_block * p.topk_n;
     // one atomic per routed entry: all entries in the low half of routed[e], those of earlier blocks in the high half
     auto count = [&](int id, int i) { atomicAdd(&routed[id], i < mine ? 0x10001 : 1); };
-    const bool rows_whole = p.topk_s1 == 1 && p.topk_s0 == p.topk_n && reinterpret_cast<uintptr_t>(p.topk) % 16 == 0;
+    const bool rows_whole = p.topk_s1 == 1 && p.topk_s0 == p.topk_n;
     const int first_alone = rows_whole ? n / 4 * 4 : 0;
     if (rows_whole) {
-      // the table is one array of ids: 16-byte loads, all of a thread's in flight, no division
+      // the table is one array of ids: 16-byte loads at the ids' own alignment, all of a thread's in flight, no division
       constexpr int kBatch = 8;
       const int per = p.topk_is64 ? 2 : 4;
       const int chunks = first_alone / per;
-      const v4i* ids = static_cast<const v4i*>(p.topk);
+      typedef v4i v4i_ids __attribute__((aligned(4)));
+      const v4i_ids* ids = static_cast<const v4i_ids*>(p.topk);
       for (int c0 = tid; c0 < chunks; c0 += kBatch * kRowsThreads) {
         v4i raw[kBatch];
 #pragma unroll
@@ -343,9 +345,28 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
         }
       }
     }
-    for (int i = first_alone + tid; i < n; i += kRowsThreads) {
-      const int64_t v = load_index(p.topk, p.topk_is64, static_cast<int64_t>(i / p.topk_n) * p.topk_s0 + (i % p.topk_n) * p.topk_s1);
-      if (v >= 0 && v < E) count(static_cast<int>(v), i);
+    // ids in any other order, and the array's last few: element loads, four of a thread's in flight, rows by a multiplication (exact:
+    // entry numbers and row lengths are below 2^15)
+    auto count_elements = [&](const auto* ids) __attribute__((always_inline)) {
+      const uint32_t per_row = p.topk_n > 1 ? 0xffffffffu / static_cast<uint32_t>(p.topk_n) + 1 : 0;
+      for (int i0 = first_alone + tid; i0 < n; i0 += 4 * kRowsThreads) {
+        std::remove_cv_t<std::remove_reference_t<decltype(*ids)>> id[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int i = i0 + u * kRowsThreads;
+          const int row = p.topk_n > 1 ? static_cast<int>(__umulhi(static_cast<uint32_t>(i), per_row)) : i;
+          id[u] = i < n ? ids[row * p.topk_s0 + (i - row * p.topk_n) * p.topk_s1] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (id[u] >= 0 && id[u] < E) count(static_cast<int>(id[u]), i0 + u * kRowsThreads);
+      }
+    };
+    if (first_alone < n) {
+      if (p.topk_is64)
+        count_elements(static_cast<const int64_t*>(p.topk));
+      else
+        count_elements(static_cast<const int32_t*>(p.topk));
     }
   } else if (MODE == kRowsScanned) {
     for (int e = tid; e < E; e += kRowsThreads) {

@@ -212,10 +212,11 @@ def test_row_tables_longer_than_the_spans(dev, T, topk, E):
 
 @pytest.mark.parametrize('T,topk,E,dtype,form', [(1, 1, 1, torch.int64, 'whole'), (333, 3, 9, torch.int32, 'whole'), (333, 3, 9, torch.int64, 'whole'),
                                                  (2048, 8, 1, torch.int64, 'whole'), (2047, 8, 77, torch.int32, 'shifted'),
-                                                 (1001, 5, 12, torch.int64, 'columns')])
+                                                 (1001, 5, 12, torch.int64, 'columns'), (1999, 7, 40, torch.int32, 'transposed'),
+                                                 (5000, 1, 6, torch.int64, 'transposed')])
 def test_row_tables_from_any_layout_of_ids(dev, T, topk, E, dtype, form):
-    """The ids as one array of 16-byte chunks with a remainder, as one that starts off such a boundary, and as columns of a
-    wider table; one expert that takes every entry of the largest table ranked in one launch; ids at and past the number of experts."""
+    """The ids as one array of 16-byte chunks with a remainder, as one that starts off such a boundary, as columns of a
+    wider table and column by column; one expert that takes every entry of the largest table ranked in one launch; ids at and past the number of experts."""
     from dlblas_amd.kernels.fused_moe_v3 import ep_scatter_rows
     print(f'case row tables T={T} topk={topk} E={E} {dtype} {form}', flush=True)
     g = helpers.gen(T + E)
@@ -225,6 +226,8 @@ def test_row_tables_from_any_layout_of_ids(dev, T, topk, E, dtype, form):
         on_dev = ids.to(dev)
     elif form == 'shifted':
         on_dev = torch.empty(T * topk + 1, dtype=dtype, device=dev)[1:].view(T, topk).copy_(ids)
+    elif form == 'transposed':
+        on_dev = torch.empty(topk, T + 1, dtype=dtype, device=dev)[:, :T].t().copy_(ids)
     else:
         on_dev = torch.empty(T, topk + 3, dtype=dtype, device=dev)[:, 1:topk + 1].copy_(ids)
     kept = torch.where(ids < E, ids, -1).clamp(min=-1).long()
