@@ -181,7 +181,7 @@ struct StreamPlan {
   int shape = kStreamNone;  // tile shape (kStreamNone: a ring kernel runs)
   int chunk_len = 0;        // K blocks per chunk of the scale table
   bool ahead = false;       // fragments read one step ahead
-  int slices = 0;           // K slices whose fp32 sums a second launch adds (it also carries the quantising epilogue then); 0: one launch
+  int slices = 0;           // K slices of a gate/up projection, whose fp32 sums a second launch adds, activates and quantises; 0: one launch
   double us = 0.0;
 };
 
@@ -303,7 +303,7 @@ hipError_t launch_stream_shape(int shape, bool ahead, const Args& args, int grid
   }
 }
 
-// One call of the weight-streaming kernel and, with K slices, of the kernel that adds them.  worst_mtiles: row tiles at most, over all
+// One call of the weight-streaming kernel and, with K slices (of a gate/up projection), of the kernel that adds them.  worst_mtiles: row tiles at most, over all
 // experts; span: rows that cover nearly every expert; all_rows: of the output.
 hipError_t launch_stream_plan(const StreamPlan& sp, int epi, Args ar, int64_t worst_mtiles, int64_t span, int64_t all_rows, int cus, int dev, hipStream_t stream) {
   const bool sliced = sp.slices > 0;
@@ -332,12 +332,9 @@ hipError_t launch_stream_plan(const StreamPlan& sp, int epi, Args ar, int64_t wo
   Args red = out;
   red.c_gs = ar.c_gs;
   // blocks for the rows nearly every expert has; a longer expert's blocks go round again
-  const int64_t per_row = epi == kStoreProduct ? ceil_div(ar.N, 4) : ar.act_cols / 8;
-  const int64_t blocks = std::min<int64_t>(ceil_div(span * per_row, 256), ceil_div(4096, ar.G));
+  const int64_t blocks = std::min<int64_t>(ceil_div(span * (ar.act_cols / 8), 256), ceil_div(4096, ar.G));
   const dim3 rgrid(static_cast<unsigned>(blocks < 1 ? 1 : blocks), static_cast<unsigned>(ar.G));
-  if (epi == kStoreProduct)
-    hipLaunchKernelGGL(fp8_stream_reduce_kernel, rgrid, dim3(256), 0, stream, red);
-  else if (epi == kSiluQuantMasked)
+  if (epi == kSiluQuantMasked)
     hipLaunchKernelGGL(fp8_stream_reduce_act_kernel<kSiluQuantMasked>, rgrid, dim3(256), 0, stream, red);
   else
     hipLaunchKernelGGL(fp8_stream_reduce_act_kernel<kSiluQuant>, rgrid, dim3(256), 0, stream, red);

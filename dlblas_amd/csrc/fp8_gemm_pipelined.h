@@ -495,7 +495,7 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
     // The first H slots' part of a group is issued by its own step, the rest by the next one.  AHEAD: that part is the
     // activations, all of them and nothing else, and all that the prologue issues of its last group.
     constexpr auto part_begin = [](int q) {
-      return AHEAD ? (q <= H ? q * Cfg::A_INST / H : Cfg::A_INST + (q - H) * (L - Cfg::A_INST) / (kSlots - H)) : q * L / kSlots;
+      return AHEAD ? (q <= H ? q * Cfg::A_INST / H : Cfg::A_INST + (q - H) * (L - Cfg::A_INST) / (kSlots > H ? kSlots - H : 1)) : q * L / kSlots;
     };
     constexpr int kFirstPart = !AHEAD ? L : part_begin(H < kSlots ? H : kSlots);
     auto issue_first_part = [&](int kb, int stg) __attribute__((always_inline)) {

@@ -31,7 +31,7 @@ namespace dlb {
 
 // What the epilogue does: store the product; silu(gate) * up + quantise with one rounding (expert-contiguous rows) or
 // with the masked activation's two (dlblas/kernels/moe.py:256-257); or leave the fp32 sums of one K slice of the product, for the
-// reduction kernels at the end of this file.
+// reduction kernel at the end of this file.
 enum StreamEpilogue : int { kStoreProduct = 0, kSiluQuant = 1, kSiluQuantMasked = 2, kStoreSlice = 3 };
 
 template <int WGM_, int WGN_, int MF_, int NF_, int STAGES_, int CH_>
@@ -619,11 +619,12 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
   }
 }
 
-// K slices (p.splitk of them): few experts, or narrow ones, have fewer tiles than the chip has CUs, and a CU fetches 40 - 50 GB/s
-// whatever it is asked for.  The streaming kernel then runs the plain product of every (tile, K slice), fp32 sums in an
-// [all rows][N] matrix per slice (p.ws, p.c_gs floats apart), and one of the two kernels below adds the slices in index order, behind
-// it on the stream: 8 experts x ~15 rows x 1792 x 3584 24.9 -> 17.0 us, 32 x ~9 rows x 512 x 5632 36.9 -> 22.4 us.  Bound: the partial sums' way through the caches, 3 us with the
-// launch at decode sizes; loads of up to kReduceBatch slices are in flight per lane.
+// K slices (p.splitk of them) of a gate/up projection: few experts, or narrow ones, have fewer tiles than the chip has CUs, and a CU
+// fetches 40 - 50 GB/s whatever it is asked for.  The streaming kernel then runs the plain product of every (tile, K slice), fp32 sums
+// in an [all rows][N] matrix per slice (p.ws, p.c_gs floats apart), and the kernel below, behind it on the stream, adds the slices in
+// index order, activates and quantises: 8 experts x ~15 rows x 1792 x 3584 24.9 -> 17.0 us, 32 x ~9 rows x 512 x 5632 36.9 -> 22.4 us.
+// Bound: the partial sums' way through the caches, 3 us with the launch at decode sizes; loads of up to kReduceBatch slices are in
+// flight per lane.  (The plain product gains nothing from slices that smaller tiles do not give it: 1.001 x over 195 problems.)
 constexpr int kReduceBatch = 4;
 constexpr int kMaxStreamSlices = 8;
 
@@ -650,32 +651,6 @@ __device__ __forceinline__ v4f stream_add_slices(const float* at, int64_t stride
       if (s0 + i < slices) sum += part[i];
   }
   return sum;
-}
-
-// grid (blocks, experts): c[row][n .. n + 3] = the slices' sum, four columns per lane
-__global__ void __launch_bounds__(256) fp8_stream_reduce_kernel(const Args p) {
-  int row0, rows;
-  stream_expert_rows(p, blockIdx.y, &row0, &rows);
-  const int cpr = (p.N + 3) / 4;
-  const int64_t total = static_cast<int64_t>(rows) * cpr;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < total; i += static_cast<int64_t>(gridDim.x) * 256) {
-    const int row = static_cast<int>(i / cpr), n = static_cast<int>(i - static_cast<int64_t>(row) * cpr) * 4;
-    const int64_t at = static_cast<int64_t>(row0 + row) * p.N;
-    v4f sum;
-    if (n + 4 <= p.N) {
-      sum = stream_add_slices(p.ws + at + n, p.c_gs, p.splitk);
-    } else {
-      for (int j = 0; j < 4; ++j) {
-        sum[j] = 0.f;
-        if (n + j < p.N)
-          for (int s = 0; s < p.splitk; ++s) sum[j] += p.ws[s * p.c_gs + at + n + j];
-      }
-    }
-    if (p.out_f32)
-      store_row4<true>(static_cast<float*>(p.c) + at, n, sum, p.N - n);
-    else
-      store_row4<false>(static_cast<__bf16*>(p.c) + at, n, sum, p.N - n);
-  }
 }
 
 // grid (blocks, experts): silu(gate) * up of the summed row and its 1 x 128 quantiser, 16 lanes per output group.  The sums pass
