@@ -12,7 +12,7 @@ import torch
 
 from ._build import LIB_PATH
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 OUT_BF16, OUT_F32 = 0, 1
 WS_COUNTER_BYTES = 65536
 WORKSPACE_BYTES = WS_COUNTER_BYTES + (32 << 20)
@@ -66,6 +66,7 @@ SYMBOLS = {
                                                 ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]),
     'dlb_workspace_lock': (ctypes.c_int, [_c_vp]),
     'dlb_workspace_unlock': (ctypes.c_int, [_c_vp]),
+    'dlb_fp8_gemm_plan_stream_launch': (ctypes.c_int, [ctypes.c_int] + [_c_i64] * 3 + [_c_i32] * 2 + [ctypes.c_int] * 2 + [_c_sz, ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 4),
     'dlb_fp8_gemm_plan_stream': (ctypes.c_int, [_c_i64] * 3 + [_c_i32] * 2 + [ctypes.c_int] * 2 + [ctypes.POINTER(ctypes.c_int)] * 3),
     'dlb_silu_mul': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp] + [_c_i64] * 4 + [_c_vp]),
     'dlb_silu_mul_quant': (ctypes.c_int, [_c_vp, ctypes.c_int, _c_vp, _c_vp] + [_c_i64] * 5 + [ctypes.c_float, _c_vp]),
@@ -231,10 +232,20 @@ def plan_grouped(mode: int, rows: int, N: int, K: int, G: int, expected_m: int =
 def plan_stream(M_max: int, N: int, K: int, G: int, expected_m: int = -1, quantising: bool = False, compute_units: int = 256):
     """(tile rows, weight rows per tile, fragments read ahead) when the weight-streaming kernel takes a masked launch over from
     the variant that plan_grouped() names, None otherwise; quantising: the gate/up GEMM with the activation in its epilogue,
-    N = its weight rows.  Touches no GPU."""
-    out = [ctypes.c_int() for _ in range(3)]
-    check(load().dlb_fp8_gemm_plan_stream(M_max, N, K, G, expected_m, int(quantising), compute_units, *(ctypes.byref(v) for v in out)))
-    return (out[0].value, out[1].value, bool(out[2].value)) if out[0].value else None
+    N = its weight rows.  For a call with this package's workspace.  Touches no GPU."""
+    found = plan_stream_launch(2, M_max, N, K, G, expected_m, quantising, compute_units=compute_units)
+    return found and found[:3]
+
+
+def plan_stream_launch(mode: int, rows: int, N: int, K: int, G: int, expected_m: int = -1, quantising: bool = False, mlp: bool = False,
+                       workspace_bytes: int = None, compute_units: int = 256):
+    """plan_stream() of either layout (mode 1: the ragged calls, 2: masked) with a fourth value: K slices whose sums a second launch
+    adds, activates and quantises (0: one launch).  mlp: a step of an expert MLP, which may slice K."""
+    out = [ctypes.c_int() for _ in range(4)]
+    ws = WORKSPACE_BYTES if workspace_bytes is None else workspace_bytes
+    check(load().dlb_fp8_gemm_plan_stream_launch(mode, rows, N, K, G, expected_m, int(quantising), int(mlp), ws, compute_units,
+                                                 *(ctypes.byref(v) for v in out)))
+    return (out[0].value, out[1].value, bool(out[2].value), out[3].value) if out[0].value else None
 
 
 STEPS_APART, ON_ROW_RANGES, ON_WHOLE_BLOCKS = 0, 1, 2  # forms of expert_plan()

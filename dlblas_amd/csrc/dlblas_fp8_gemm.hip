@@ -977,6 +977,14 @@ double contiguous_us(int64_t rows, int64_t N, int64_t K, int G, bool act, int cu
   return act ? lists_us : std::min(lists_us, contiguous_plain_us(rows, N, K, cus));
 }
 
+// How the weight-streaming kernel runs a launch on row ranges (mlp: a step of an expert MLP, whose K may be sliced).
+StreamPlan ragged_stream(int64_t rows, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, bool mlp, size_t ws_bytes, int cus) {
+  const bool shape_ok = K > 0 && K % kScaleBlock == 0 && K < (1ll << 24) && rows < (1ll << 31) && (!act || (N % (2 * kScaleBlock) == 0 && N * K < (1ll << 32)));
+  const size_t room = ws_bytes > DLB_WS_COUNTER_BYTES ? ws_bytes - DLB_WS_COUNTER_BYTES : 0;
+  if (!shape_ok) return StreamPlan{};
+  return pick_stream(rows, N, K, G, hint_rows, act, cus, mlp ? kMaxStreamSlices : 1, rows, room / sizeof(float), contiguous_us(rows, N, K, G, act, cus));
+}
+
 // A step of an expert MLP on expert-contiguous rows (act: the gate/up projection, N = 2 I): 1 = the weight-streaming kernel on the
 // experts' row ranges, 2 = the expert-contiguous kernels on whole blocks (act: from tile lists), 0 = neither.
 int expert_form(int64_t rows, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, size_t ws_bytes, int cus) {
@@ -985,8 +993,7 @@ int expert_form(int64_t rows, int64_t N, int64_t K, int G, int64_t hint_rows, bo
   const bool shape_ok = K > 0 && K % kScaleBlock == 0 && K < (1ll << 24) && rows < (1ll << 31) && (!act || (N % (2 * kScaleBlock) == 0 && N * K < (1ll << 32)));
   if (!shape_ok || g_forced_variant >= 0) return 0;
   const bool lists = g_knob[kKnobTileList] != 2 && nblk <= kTileListMaxBlocks && tile_list_bytes(nblk) <= room;
-  const double other_us = contiguous_us(rows, N, K, G, act, cus);
-  if (pick_stream(rows, N, K, G, hint_rows, act, cus, kMaxStreamSlices, rows, room / sizeof(float), other_us).shape != kStreamNone) return 1;
+  if (ragged_stream(rows, N, K, G, hint_rows, act, true, ws_bytes, cus).shape != kStreamNone) return 1;
   return act && !lists ? 0 : 2;
 }
 
@@ -1173,12 +1180,8 @@ int run_ragged(const RaggedProblem& pr) {
   if (pr.ws && misaligned(pr.ws, 16)) return fail(DLB_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
   const bool usable_ws = pr.ws && pr.ws_bytes > DLB_WS_COUNTER_BYTES;
   StreamPlan sp;
-  const bool fits = pr.K > 0 && pr.K % kScaleBlock == 0 && pr.K < (1ll << 24) && pr.as_sm < (1ll << 21) && pr.M_sum < (1ll << 31) &&
-                    pr.N < (1ll << 31) && (!pr.act || (pr.N % (2 * kScaleBlock) == 0 && pr.N * pr.K < (1ll << 32))) &&
-                    (!pr.a_rows || (pr.act && pr.a_src_rows > 0 && pr.a_src_rows * pr.K < (1ll << 31)));
-  if (fits)
-    sp = pick_stream(pr.M_sum, pr.N, pr.K, pr.G, pr.hint_rows, pr.act, cus, pr.mlp ? kMaxStreamSlices : 1, pr.M_sum, usable_ws ? (pr.ws_bytes - DLB_WS_COUNTER_BYTES) / sizeof(float) : 0,
-                     contiguous_us(pr.M_sum, pr.N, pr.K, pr.G, pr.act, cus));
+  const bool fits = pr.as_sm < (1ll << 21) && pr.N < (1ll << 31) && (!pr.a_rows || (pr.act && pr.a_src_rows > 0 && pr.a_src_rows * pr.K < (1ll << 31)));
+  if (fits) sp = ragged_stream(pr.M_sum, pr.N, pr.K, pr.G, pr.hint_rows, pr.act, pr.mlp, pr.ws ? pr.ws_bytes : 0, cus);
   if (sp.shape == kStreamNone)
     return fail(DLB_ERR_BAD_SHAPE, "the weight-streaming kernel does not take this problem (N=%lld K=%lld, about %lld rows per expert)",
                 (long long)pr.N, (long long)pr.K, (long long)pr.hint_rows);
@@ -1910,19 +1913,33 @@ int dlb_fp8_gemm_plan_grouped(int mode, int64_t rows, int64_t N, int64_t K, int3
   return DLB_OK;
 }
 
-int dlb_fp8_gemm_plan_stream(int64_t rows, int64_t N, int64_t K, int32_t G, int32_t expected_m, int quantising, int compute_units,
-                             int* tile_rows, int* tile_columns, int* ahead) {
+int dlb_fp8_gemm_plan_stream_launch(int mode, int64_t rows, int64_t N, int64_t K, int32_t G, int32_t expected_m, int quantising, int mlp,
+                                    size_t workspace_bytes, int compute_units, int* tile_rows, int* tile_columns, int* ahead, int* slices) {
   dlb::clear_error();
   const int64_t lim = (1ll << 31) - 1024;
   if (rows < 0 || N < 0 || K < 0 || G < 0 || rows > lim || N > lim || K > lim || compute_units <= 0)
     return dlb::fail(DLB_ERR_BAD_SHAPE, "bad dimension (rows=%lld, N=%lld, K=%lld, G=%d)", (long long)rows, (long long)N, (long long)K, G);
+  if (mode != dlb::kContiguous && mode != dlb::kMasked) return dlb::fail(DLB_ERR_BAD_SHAPE, "mode %d is not 1 (contiguous) or 2 (masked)", mode);
   const bool act = quantising != 0;
-  const dlb::Resolved rs = dlb::resolve(dlb::kMasked, rows, N, K, G, dlb::ceil_div(K, dlb::kScaleBlock), 1, false, 0, compute_units, false, act, expected_m);
-  const bool on = rs.stream.shape != dlb::kStreamNone && (!act || (N % (2 * dlb::kScaleBlock) == 0 && N * K < (1ll << 32)));
-  if (tile_rows) *tile_rows = on ? dlb::kStreamDims[rs.stream.shape].bm : 0;
-  if (tile_columns) *tile_columns = on ? dlb::kStreamDims[rs.stream.shape].bn : 0;
-  if (ahead) *ahead = on && rs.stream.ahead ? 1 : 0;
+  dlb::StreamPlan sp;
+  if (mode == dlb::kContiguous) {
+    sp = dlb::ragged_stream(rows, N, K, G, expected_m, act, mlp != 0, workspace_bytes, compute_units);
+  } else if (!act || (N % (2 * dlb::kScaleBlock) == 0 && N * K < (1ll << 32))) {
+    sp = dlb::resolve(dlb::kMasked, rows, N, K, G, dlb::ceil_div(K, dlb::kScaleBlock), 1, workspace_bytes > 0, workspace_bytes, compute_units, false, act,
+                      expected_m, true, mlp != 0 ? dlb::kMaxStreamSlices : 1)
+             .stream;
+  }
+  const bool on = sp.shape != dlb::kStreamNone;
+  if (tile_rows) *tile_rows = on ? dlb::kStreamDims[sp.shape].bm : 0;
+  if (tile_columns) *tile_columns = on ? dlb::kStreamDims[sp.shape].bn : 0;
+  if (ahead) *ahead = on && sp.ahead ? 1 : 0;
+  if (slices) *slices = on ? sp.slices : 0;
   return DLB_OK;
+}
+
+int dlb_fp8_gemm_plan_stream(int64_t rows, int64_t N, int64_t K, int32_t G, int32_t expected_m, int quantising, int compute_units,
+                             int* tile_rows, int* tile_columns, int* ahead) {
+  return dlb_fp8_gemm_plan_stream_launch(dlb::kMasked, rows, N, K, G, expected_m, quantising, 0, 0, compute_units, tile_rows, tile_columns, ahead, nullptr);
 }
 
 int dlb_fp8_gemm_force_variant(int variant) {

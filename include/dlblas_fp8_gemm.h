@@ -47,7 +47,7 @@
 extern "C" {
 #endif
 
-#define DLB_ABI_VERSION 10
+#define DLB_ABI_VERSION 11
 
 /* output element type of C */
 #define DLB_OUT_BF16 0
@@ -379,9 +379,9 @@ int dlb_fp8_quant_128x128(const void* w, int w_dtype, void* q, float* s, int64_t
  * is the CU count to plan for (256 on MI355X); activation scales are taken to be row-major.  Outputs (each may be
  * NULL): the kernel variant id (dlb_fp8_gemm_variant_name); the number of K slices summed in a second pass (1 = none),
  * exactly as a launch with this workspace size would use it, unless the kernel of dlb_fp8_gemm_plan_wave_k takes it over
- * (mode 2: that of dlb_fp8_gemm_plan_stream); the output columns per workgroup of the decode kernels (0 for other variants); the first column of the 192-wide tiles of the mixed-width prefill launch (N when all tiles
- * are equal).  Honours the calling thread's forced variant and knobs, as a launch does (both run the same code).
- * Costs a few microseconds at most and keeps no state.  No counterpart in the reference, whose single Triton
+ * (mode 2: that of dlb_fp8_gemm_plan_stream_launch); the output columns per workgroup of the decode kernels (0 for other variants);
+ * the first column of the 192-wide tiles of the mixed-width prefill launch (N when all tiles are equal).  Honours the calling thread's forced variant and knobs, as a launch does (both run the same code).
+ * Costs 2 to 20 microseconds (the wide launches try every cut of their columns) and keeps no state.  No counterpart in the reference, whose single Triton
  * configuration needs no plan.
  */
 int dlb_fp8_gemm_plan(int mode, int64_t rows, int64_t N, int64_t K, size_t workspace_bytes, int compute_units, int* variant,
@@ -400,7 +400,7 @@ int dlb_fp8_gemm_plan_wave_k(int64_t M, int64_t N, int64_t K, size_t workspace_b
  * the masked layout (mode 2), the caller's expected_m (<= 0: unknown).  mode 1 = contiguous (rows = M_sum), 2 = masked
  * (rows = M_max).  Outputs (each may be NULL): the kernel variant id; whether a contiguous launch of this size pairs
  * blocks into taller tiles from lists built on the device (1) or runs uniform 128-row tiles (0; always 0 for the masked
- * layout, where dlb_fp8_gemm_plan_stream may take the launch over from the named variant).  The fused gate/up entry points
+ * layout, where the kernel of dlb_fp8_gemm_plan_stream_launch may take the launch over from the named variant).  The fused gate/up entry points
  * of the contiguous layout always take the lists, so a caller that can also run GEMM and activation apart does that where
  * this says 0 (a batch of at most a round or two of tiles, where the uniform tiles are faster).  No counterpart in the
  * reference.
@@ -409,12 +409,18 @@ int dlb_fp8_gemm_plan_grouped(int mode, int64_t rows, int64_t N, int64_t K, int3
                               int compute_units, int* variant, int* tile_lists);
 
 /*
- * Whether the weight-streaming kernel takes a masked launch over from the variant dlb_fp8_gemm_plan_grouped names, and with
- * which tile: rows, weight rows and whether it reads its fragments one step ahead, all 0 when it does not.  `quantising` != 0
- * asks for dlb_fp8_gemm_grouped_masked_silu_quant (N = its weight rows), 0 for dlb_fp8_gemm_grouped_masked.  The ragged entry
- * points choose the same tiles with rows = M_sum and weigh them against the expert-contiguous kernels, whose padded rows they
- * replace: dlb_expert_plan (mode 1) says whether they take a call.  No counterpart in the reference.
+ * Whether the weight-streaming kernel runs a grouped launch, and how: rows and weight rows of its tiles, whether it reads its
+ * fragments one step ahead, and the K slices whose sums a second launch adds, activates and quantises (0: one launch); all 0 when it
+ * does not.  mode 2 = masked (rows = M_max; the launch is taken over from the variant dlb_fp8_gemm_plan_grouped names), 1 = the
+ * ragged entry points (rows = M_sum; they decline what the kernel does not take).  `quantising` != 0 asks for the gate/up forms
+ * (N = their weight rows); `mlp` != 0 for dlb_expert_gate_up_masked / _ragged, which may slice K, 0 for the entry points that
+ * keep the bits of the steps apart (one slice at most).  workspace_bytes: that of the call, 0 = none (a plain ragged call has none).
+ * No counterpart in the reference.
  */
+int dlb_fp8_gemm_plan_stream_launch(int mode, int64_t rows, int64_t N, int64_t K, int32_t G, int32_t expected_m, int quantising, int mlp,
+                                    size_t workspace_bytes, int compute_units, int* tile_rows, int* tile_columns, int* ahead, int* slices);
+
+/* The same for a masked call without a workspace, which is one launch. */
 int dlb_fp8_gemm_plan_stream(int64_t rows, int64_t N, int64_t K, int32_t G, int32_t expected_m, int quantising, int compute_units,
                              int* tile_rows, int* tile_columns, int* ahead);
 

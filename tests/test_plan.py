@@ -229,3 +229,16 @@ def test_plan_stream_answers_for_either_form():
         assert _lib.plan_grouped(MASKED, rows, 4096, 7168, 32, hint)[1] is False
     assert _lib.plan_grouped(CONTIGUOUS, 9728, 4096, 7168, 32)[1] is True
     assert _lib.load().dlb_fp8_gemm_plan_stream(-1, 1, 1, 1, 0, 0, 256, None, None, None) == _lib.ERR_BAD_SHAPE
+
+
+@pytest.mark.parametrize('mode,rows', [(CONTIGUOUS, 1024), (MASKED, 64)])
+def test_plan_stream_knows_the_gate_up_form_in_two_launches(mode, rows):
+    """Few narrow experts: with a workspace the sums of every tile, and inside an expert MLP of K slices, leave the first launch;
+    without one, or with one too small for them, the whole projection is one launch."""
+    query = lambda **how: _lib.plan_stream_launch(mode, rows, 1792, 3584, 8, 15, **how)
+    assert query(quantising=True, mlp=True)[3] > 1 and query(quantising=True)[3] == 1
+    for size in (0, _lib.WS_COUNTER_BYTES + 4096):
+        assert query(quantising=True, mlp=True, workspace_bytes=size)[3] == 0
+    assert query()[3] == query(mlp=True)[3] == 0  # the plain product
+    assert _lib.expert_plan(mode, rows, 1792, 3584, 8, 15, quantising=True) == _lib.ON_ROW_RANGES
+    assert _lib.load().dlb_fp8_gemm_plan_stream_launch(0, 1, 1, 1, 1, 0, 0, 0, 0, 256, None, None, None, None) == _lib.ERR_BAD_SHAPE
