@@ -376,7 +376,7 @@ PyObject* grouped_masked(PyObject*, PyObject* const* args, Py_ssize_t n) {
 enum Form : int { kStepsApart = 0, kOnRowRanges = 1, kOnWholeBlocks = 2 };
 
 Form expert_form(int mode, int64_t rows, int64_t N, int64_t K, int64_t G, int64_t hint, bool quantising, const Workspace& ws) {
-  int form = kOnWholeBlocks;
+  int form = kStepsApart;
   if (abi.plan(mode, rows, N, K, static_cast<int32_t>(G), static_cast<int32_t>(hint), quantising, ws.bytes, 256, &form) != DLB_OK) return kStepsApart;
   return static_cast<Form>(form);
 }

@@ -362,21 +362,26 @@ def test_native_calls_run_without_the_interpreter_lock(dev):
         'fused_moe_v3': (codes(3, 512), torch.ones(3, 4, device=dev), ids, wts, *w13, *w2, [128, 128]),
     }
     assert calls.keys() == set(_fast._FUNCTIONS)
-    for name, a in calls.items():  # with the library itself: nothing declines these
+    # an expert MLP on row ranges (above), and one whose K is too short for them in the first and the second projection
+    (v13, v2, _), form = _small_experts(dev, 2, 256, 256), lambda n, k, quantising: _lib.expert_plan(1, 256, n, k, 2, 2, quantising)
+    assert (form(1024, 512, True), form(512, 512, False)) == (_lib.ON_ROW_RANGES, _lib.ON_ROW_RANGES)
+    assert (form(512, 256, True), form(256, 256, False)) == (_lib.ON_WHOLE_BLOCKS, _lib.ON_WHOLE_BLOCKS)
+    calls = list(calls.items()) + [('fused_moe_v3', (codes(3, 256), torch.ones(3, 2, device=dev), ids, wts, *v13, *v2, [128, 128]))]
+    for name, a in calls:  # with the library itself: nothing declines these
         assert getattr(_fast, name)(*a) is not None, name
     torch.cuda.synchronize()
     init = _fast.fp8_gemm.__self__.init
     address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
     real = [address(getattr(lib, n)) for n in _fast._ABI]
-    asks = ('dlb_last_error', 'dlb_workspace_lock', 'dlb_workspace_unlock', 'dlb_fp8_gemm_plan_grouped', 'dlb_fp8_gemm_plan_stream',
-            'dlb_fp8_gemm_variant_name', 'dlb_ep_scatter_workspace_bytes')
+    asks = ('dlb_last_error', 'dlb_workspace_lock', 'dlb_workspace_unlock', 'dlb_expert_plan', 'dlb_ep_scatter_workspace_bytes')
+    assert set(asks) <= set(_fast._ABI)
     probe = address(ctypes.pythonapi.PyGILState_Check)
     try:
         init([r if n in asks else probe for n, r in zip(_fast._ABI, real)], _lib.workspace)
-        without = {name: getattr(_fast, name)(*a) is not None for name, a in calls.items()}
+        without = [(name, getattr(_fast, name)(*a) is not None) for name, a in calls]
     finally:
         init(real, _lib.workspace)
-    assert all(without.values()), without
+    assert all(went for _, went in without), without
 
 
 def test_threads_on_one_stream_keep_their_launches_together(dev):
