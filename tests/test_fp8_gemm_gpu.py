@@ -189,18 +189,39 @@ def test_scale_table_of_every_ring_kernel(dev, layout, variant, rows, N, blocks)
 
 
 @pytest.mark.parametrize('variant,M', [('pipe256x256', 260), ('pipe128x256w8', 132)])
-@pytest.mark.parametrize('kb,dtype', [(1, torch.bfloat16), (2, torch.float32), (3, torch.bfloat16), (4, torch.float32), (17, torch.bfloat16),
-                                      (27, torch.bfloat16), (28, torch.float32)])
+@pytest.mark.parametrize('kb,dtype', [(1, torch.bfloat16), (2, torch.float32), (3, torch.bfloat16), (4, torch.float32), (5, torch.float32),
+                                      (15, torch.bfloat16), (16, torch.float32), (17, torch.bfloat16), (27, torch.bfloat16), (28, torch.float32)])
 def test_tiles_of_a_resident_workgroup(dev, variant, M, kb, dtype):
     """258 tiles of 256 columns on 256 resident workgroups or fewer: the ring runs on into the next tile from as many K blocks
     on as it has stages; a last row tile of 4 rows and a last column tile of 233 columns, so that a workgroup goes from a
-    whole tile to a ragged one; K on both sides of the longest whose scales come from the table."""
+    whole tile to a ragged one; K on both sides of the longest whose scales come from the table (27 and 16 blocks)."""
     N, K = 33001, kb * 128
     print(f'case resident tiles {variant} K={K} {dtype}', flush=True)
     a_q, a_s, b_q, b_s = helpers.make_dense(M, N, K, seed=kb)
     outs = [_run_dense(dev, a_q, a_s, b_q, b_s, dtype=dtype, variant=variant) for _ in range(2)]
     assert torch.equal(outs[0], outs[1])
     helpers.tolerance_check(outs[0], orc.dequant_ref(a_q, a_s, b_q, b_s), f'resident tiles {variant} K={K}')
+
+
+@pytest.mark.parametrize('variant,M,kb', [('pipe256x256', 2052, kb) for kb in (2, 3, 5, 28)] + [('pipe128x256w8', 1028, kb) for kb in (3, 4, 5, 17)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
+def test_ring_runs_on_through_three_tiles(dev, variant, M, kb, dtype):
+    """9 x 87 tiles on 256 workgroups, the last ones 4 rows high and 84 columns wide: tiles that start from a carried ring and carry
+    it on, at as many K blocks as the ring has stages, one more, and counts that are no multiple of them, with the scale table (up
+    to 27 / 16 blocks) and without.  The bits of the same kernel without the carry, which stores through LDS alone take."""
+    from dlblas_amd import _lib
+    N, K = 22100, kb * 128
+    print(f'case three tiles {variant} K={K} {dtype}', flush=True)
+    a_q, a_s, b_q, b_s = helpers.make_dense(M, N, K, seed=kb)
+    carried = _run_dense(dev, a_q, a_s, b_q, b_s, dtype=dtype, variant=variant)
+    try:
+        _lib.tune('epilogue', 2)
+        apart = _run_dense(dev, a_q, a_s, b_q, b_s, dtype=dtype, variant=variant)
+    finally:
+        _lib.tune('epilogue', 0)
+    assert torch.equal(carried, apart)
+    rows = torch.tensor([0, 127, 128, 255, 256, 770, 1023, 1024, M - 1])
+    helpers.tolerance_check(carried[rows.to(carried.device)], orc.dequant_ref(a_q[rows], a_s[rows], b_q, b_s), f'three tiles {variant} K={K}')
 
 
 def test_refused_launch_enqueues_nothing(dev):
