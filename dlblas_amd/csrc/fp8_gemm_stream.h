@@ -273,10 +273,16 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
   enter_tile();
   if (!it.ok) return;
   Tile ct = it;  // the tile the compute side works on
-  // a tile has at least STAGES K blocks and a chunk at least STAGES - 1
-  open_chunk();
+  // a tile has at least STAGES K blocks and a chunk at least STAGES - 1.  (Gathered rows in whole steps: the compiler then spills 37 to
+  // 51 scalar registers there in place of 60 to 71, 16 experts x ~48 gathered rows x 3328 x 1792 21.4 -> 21.0 us.)
+  if constexpr (GATHER) {
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s) issue_loads();
+    for (int s = 0; s < STAGES - 1; ++s) issue_step();
+  } else {
+    open_chunk();
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s) issue_loads();
+  }
   if (AHEAD) {
     open_chunk();
     issue_loads();
