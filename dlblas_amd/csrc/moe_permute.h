@@ -316,7 +316,7 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
     const int mine = b * p.tokens_per_block * p.topk_n;
     // one atomic per routed entry: all entries in the low half of routed[e], those of earlier blocks in the high half
     auto count = [&](int id, int i) { atomicAdd(&routed[id], i < mine ? 0x10001 : 1); };
-    const bool rows_whole = p.topk_s1 == 1 && p.topk_s0 == p.topk_n;
+    const bool rows_whole = p.topk_s1 == 1 && p.topk_s0 == p.topk_n && n > kRowsThreads;  // fewer: one id a thread
     const int first_alone = rows_whole ? n / 4 * 4 : 0;
     if (rows_whole) {
       // the table is one array of ids: 16-byte loads at the ids' own alignment, all of a thread's in flight, no division
@@ -346,11 +346,18 @@ __global__ void __launch_bounds__(kRowsThreads) ep_rows_kernel(const RowsArgs a)
       }
     }
     // ids in any other order, and the array's last few: element loads, four of a thread's in flight, rows by a multiplication (exact:
-    // entry numbers and row lengths are below 2^15)
+    // entry numbers and row lengths are below 2^15); where each thread has at most one id, as one load and one division
     auto count_elements = [&](const auto* ids) __attribute__((always_inline)) {
+      typedef std::remove_cv_t<std::remove_reference_t<decltype(*ids)>> Id;
+      if (n <= kRowsThreads) {
+        if (tid >= n) return;
+        const Id id = ids[tid / p.topk_n * p.topk_s0 + tid % p.topk_n * p.topk_s1];
+        if (id >= 0 && id < E) count(static_cast<int>(id), tid);
+        return;
+      }
       const uint32_t per_row = p.topk_n > 1 ? 0xffffffffu / static_cast<uint32_t>(p.topk_n) + 1 : 0;
       for (int i0 = first_alone + tid; i0 < n; i0 += 4 * kRowsThreads) {
-        std::remove_cv_t<std::remove_reference_t<decltype(*ids)>> id[4];
+        Id id[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int i = i0 + u * kRowsThreads;
