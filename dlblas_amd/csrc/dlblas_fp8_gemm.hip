@@ -441,7 +441,7 @@ double mixed_makespan(int64_t ta, int64_t tb, double cb, int workers) {
 }
 
 // Columns [0, n_split) in 256-wide tiles, the rest in 192-wide tiles; returns n_split (== N: no narrow region).
-// Cost: (N / 256 + 1) candidate cuts x a few steps per round, a few microseconds at most, no state.
+// Cost: (N / 256 + 1) candidate cuts x a few steps per round, 1 to 8 us, no state.
 // *makespan (optional): the launch's length in units of one 256-wide tile.
 int64_t pick_mixed_split(int64_t M, int64_t N, int cus, double* makespan = nullptr) {
   const int64_t tm = ceil_div(M, 256);
@@ -607,9 +607,9 @@ MidChoice pick_mid_plan(int64_t M, int64_t N, int kblocks, int cus, size_t ws_av
       const int per = static_cast<int>(ceil_div(kblocks, want));
       const int sk = static_cast<int>(ceil_div(kblocks, per));
       const int64_t units = ceil_div(M, c.bm) * ceil_div(N, c.bn) * sk;
-      // the small tiles fetch a tile's scales once, into a table in LDS, when the slice is short enough: no re-layout
-      // launch and no scattered scale lines per K step
-      const bool table = (c.variant == kVarPipe128x64 && per <= Pipe128x64T::SCTAB_KB) || (c.variant == kVarPipe128x128 && per <= Pipe128x128T::SCTAB_KB);
+      // a tile's scales come once, into a table in LDS, when the slice is short enough: no re-layout launch and no scattered scale
+      // lines per K step
+      const bool table = per <= (c.variant == kVarPipe128x64 ? Pipe128x64T::SCTAB_KB : c.variant == kVarPipe128x128 ? Pipe128x128T::SCTAB_KB : Pipe128x256w8T::SCTAB_KB);
       double us = launch + (table ? 0.0 : relayout) +
                   static_cast<double>(ceil_div(units, cus)) * (tile_fixed + per * c.step_us * short_rows * (table ? 1.0 : scattered));
       if (sk > 1) us += second_pass + (2.0 * sk + 0.5) * out_bytes / ws_rate;  // partial sums written, read back, result written
@@ -1038,7 +1038,7 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
   }
   // A tile's row-major scales come once, into a table in LDS, where its K range fits what the ring leaves of the LDS: no re-layout
   // launch in front (3 - 4 us), one cache-line request per row and tile.  us per call with the pre-pass / with the table: dense
-  // 1024 x 8192 x 1536 22.5 / 19.2, 4096 x 7168 x 1024 44 / 40; contiguous 8 experts, 171 rows, 1408 x 2048 19.6 / 16.3, 16
+  // 1024 x 8192 x 1536 22.5 / 19.2, 4096 x 7168 x 1024 44 / 40, 2048 x 4096 x 512 15.0 / 11.6; contiguous 8 experts, 171 rows, 1408 x 2048 19.6 / 16.3, 16
   // experts, 494 rows, 3712 x 1024 22.2 / 18.3; masked 16 x 0 .. 512 x 4096 x 1024 46 / 43.  Launches of many rounds fetch a table per
   // tile and gain nothing any more from 8 K blocks on (4096 x 24576 x 1536 175 / 175), nor lose.
   auto table_fits = [&](int kb_per) {
