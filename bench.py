@@ -802,6 +802,21 @@ def wave_k_random(dev, count=1500, seconds=240):
         print(f'{name}: {len(hbm)}, {gm(cache):.2f}, {gm(hbm):.2f}', flush=True)
 
 
+def _log_pick(rng, lo, hi, step=1):
+    import math
+    return max(lo, min(hi, int(round(math.exp(rng.uniform(math.log(lo), math.log(hi))) / step)) * step))
+
+
+def wide_problems(count):
+    import random
+    rng, found = random.Random(22), []
+    while len(found) < count:
+        M, N, K = _log_pick(rng, 256, 4096), _log_pick(rng, 2048, 36864, rng.choice([1, 8, 64, 128])), _log_pick(rng, 384, 7168, 128)
+        if 256 < -(-M // 256) * -(-N // 256) <= 9 * 256:
+            found.append((M, N, K))
+    return found
+
+
 def planner_sweep(dev, which):
     """The planner's launch against every alternative forced in turn; prints one line per problem and returns the rows.
     'dense': kernel variants (no K split forced) over 13 weight shapes x 15 row counts; 'mid': the three small ring
@@ -809,7 +824,12 @@ def planner_sweep(dev, which):
     flight of the streaming kernels at 1, 16 and 32 rows; 'grouped': ring variants for both grouped layouts, 8 and 32
     experts; 'wave_k': the launch without the kernel whose waves split K and with each of its tile shapes, at the row counts
     and the ragged K it is meant for and around them; 'stream': the same for the weight-streaming kernel of the masked layout,
-    plain and with the quantising epilogue.  A row's 'regret' is default / best - 1."""
+    plain and with the quantising epilogue; 'wide_random': random prefill problems of one to nine rounds of 256 x 256 tiles, mixed
+    and equal tiles of 256 rows and tiles of 128 rows; 'stream_random': random masked problems, plain and gate/up inside an expert
+    MLP, on the ring kernel, every streaming tile and (gate/up) 1, 2, 4 and 8 K slices.  A row's 'regret' is default / best - 1."""
+    import math
+    import random
+
     import torch
 
     from dlblas_amd import _lib
@@ -872,6 +892,17 @@ def planner_sweep(dev, which):
                         _lib.force_variant(None)
                         t0 = min(t0, timed(launch, reps))
                     report(f'{M}x{N}x{K}', wave_k_or(plan[:2], M, N, K), t0, min(best[0], t0), best[1])
+        elif which == 'wide_random':
+            for M, N, K in wide_problems(80):
+                launch, reps = dense_problem(M, N, K)
+                times = {'default': timed(launch, reps)}
+                for v in ('pipe256mix', 'pipe256x256', 'pipe128x256w8'):
+                    _lib.force_variant(v)
+                    times[v] = timed(launch, reps)
+                _lib.force_variant(None)
+                times['default'] = min(times['default'], timed(launch, reps))
+                best = min(times, key=lambda n: times[n])
+                report(f'{M}x{N}x{K}', _lib.plan(0, M, N, K)[0], times['default'], times[best], best, {n: t for n, t in times.items() if n != 'default'})
         elif which == 'mid':
             for (N, K) in PLANNER_SWEEP_WEIGHTS + [(4096, 4096), (1024, 16384), (7168, 4096)]:
                 for M in (48, 64, 96, 128, 192, 256, 384, 512, 1024):
@@ -1013,6 +1044,62 @@ def planner_sweep(dev, which):
                                {n: t for n, t in times.items() if n != 'default'})
                     del a_q, a_s, out, q, sc
                 del w_q, w_s
+        elif which == 'stream_random':
+            shapes = ('32x256', '64x256', '64x128', '128x256', '64x64', None, '64x256 ahead', '64x128 ahead', '128x256 ahead', '64x64 ahead')
+            rng = random.Random(23)
+            codes = torch.randint(0, 0x60, (32 * 7168 * 7168, ), dtype=torch.uint8, device=dev).view(torch.float8_e4m3fn)  # finite
+            unit = torch.rand(1 << 20, device=dev)
+            side = torch.cuda.Stream()
+
+            def replayed(call):
+                """us a call from a graph of 10: the fused calls cost more host time than most of them run."""
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.stream(side):
+                    call()
+                    side.synchronize()
+                    with torch.cuda.graph(graph, stream=side):
+                        for _ in range(10):
+                            call()
+                torch.cuda.synchronize()
+                return min(time_call(graph.replay, 3, 1) for _ in range(3)) * 100
+
+            for _ in range(80):
+                G, N, K, mean = rng.choice([8, 16, 32]), _log_pick(rng, 512, 7168, 256), _log_pick(rng, 384, 7168, 128), _log_pick(rng, 1, 960)
+                cap, act = 2 * mean, rng.random() < 0.5
+                mm = torch.randint(0, cap + 1, (G, ), generator=torch.Generator().manual_seed(mean), dtype=torch.int32).to(dev)
+                w, w_s = codes[:G * N * K].view(G, N, K), unit[:G * (N // 128) * (K // 128)].view(G, N // 128, K // 128)
+                a, a_s = codes[:G * cap * K].clone().view(G, cap, K), torch.rand(G, cap, K // 128, device=dev)
+                out = torch.empty(G, cap, N, dtype=torch.bfloat16, device=dev)
+                q, sc = torch.empty(G, cap, N // 2, dtype=torch.float8_e4m3fn, device=dev), torch.empty(G, N // 256, cap, device=dev).transpose(1, 2)
+
+                def call():
+                    if not act:
+                        fp8_gemm_grouped_masked(a, a_s, w, w_s, out, mm, mean)
+                    elif not fp8_gemm_grouped_masked_silu_quant(a, a_s, w, w_s, q, sc, mm, mean, mlp=True):
+                        raise RuntimeError('declined')
+
+                try:
+                    times = {'default': replayed(call), 'ring kernels': None}
+                except RuntimeError:  # gate/up that is left to GEMM and activation apart
+                    continue
+                for knob, name in enumerate(('ring kernels', ) + shapes, 1):
+                    if name is None:
+                        continue
+                    for slices in (0, 1, 2, 4, 8) if act and knob > 1 else (0, ):
+                        _lib.tune('stream', knob), _lib.tune('stream_slices', slices)
+                        how = 2, cap, N, K, G, mean
+                        if knob > 1 and _lib.plan_stream_launch(*how, quantising=act, mlp=act) is not None:
+                            times[f'{name}, {slices} slices' if slices else name] = replayed(call)
+                        elif knob == 1 and not (act and _lib.expert_plan(2, *how[1:], quantising=True) == _lib.STEPS_APART):
+                            times[name] = replayed(call)
+                _lib.tune('stream', 0), _lib.tune('stream_slices', 0)
+                times['default'] = min(times['default'], replayed(call))
+                best = min((n for n in times if times[n] is not None), key=lambda n: times[n])
+                plan = _lib.plan_stream_launch(2, cap, N, K, G, mean, quantising=act, mlp=act)
+                report(f"masked {'gate/up' if act else 'plain'}, {G} experts x {cap} slots, {int(mm.sum())} valid rows, {N}x{K}",
+                       'stream {}x{}{}{}'.format(plan[0], plan[1], ' ahead' if plan[2] else '', f', {plan[3]} slices' if plan[3] else '') if plan else 'ring kernels',
+                       times['default'], times[best], best)
+                del a, a_s, out, q, sc
         else:
             raise ValueError(which)
     finally:
@@ -1021,6 +1108,7 @@ def planner_sweep(dev, which):
             _lib.tune(knob, 0)
     worst = sorted(rows, key=lambda r: -r['regret'])[:5]
     print(f"{len(rows)} problems; over 5 %: {sum(r['regret'] > 0.05 for r in rows)}, over 10 %: {sum(r['regret'] > 0.10 for r in rows)}; "
+          f"geometric mean {100 * math.expm1(sum(math.log1p(r['regret']) for r in rows) / len(rows)):.1f} %; "
           'largest: ' + '; '.join(f"{r['problem']} {100 * r['regret']:.0f} %" for r in worst), flush=True)
     return rows
 
@@ -1050,7 +1138,7 @@ def main():
     ap.add_argument('--grouped-only', action='store_true',
                     help='run only the two grouped MoE workloads and print their rows (the command the rocprofv3 summaries of '
                     'the grouped kernels are made with)')
-    ap.add_argument('--planner-sweep', choices=['dense', 'mid', 'decode', 'grouped', 'wave_k', 'stream', 'wave_k_random'], default=None,
+    ap.add_argument('--planner-sweep', choices=['dense', 'mid', 'decode', 'grouped', 'wave_k', 'stream', 'wave_k_random', 'wide_random', 'stream_random'], default=None,
                     help="time the planner's launch against every alternative forced in turn over a grid of problems and "
                     'print where it is not the fastest (a minute or two)')
     args = ap.parse_args()

@@ -469,7 +469,8 @@ int64_t pick_mixed_split(int64_t M, int64_t N, int cus, double* makespan = nullp
 //   - equal tiles, more than one round: resident workgroups whose ring runs on from tile to tile: 5.4 + 1.82 K blocks per round
 //     and 3 for the launch.
 // A last round that is not full costs 0.6 of a round plus its share of the rest (the chip is faster with fewer tiles).  33
-// launches of 1.1 to 8.8 rounds of equal tiles lie within 7 % of that, mixed ones within 10 %.
+// launches of 1.1 to 8.8 rounds of equal tiles lie within 7 % of that, mixed ones within 10 %.  The choice, 128-row tiles included, is
+// 0.8 % behind the best of the three (geometric mean of 80 random problems, bench.py --planner-sweep wide_random; 10 % at worst).
 // Mixed tiles win where K is long and the last round short (4096 x 5248 x 4096: 104 / 113 us, 2048 x 17408 x 7168: 265 / 292),
 // equal ones where the fixed part of a tile counts (3500 x 33024 x 1280: 203 / 183, 2048 x 18176 x 512: 45 / 38).
 int pick_wide_variant(int64_t M, int64_t N, int kblocks, int cus, double* us = nullptr) {
@@ -898,9 +899,10 @@ constexpr TileCost kStreamCostAhead[kStreamCount] = {{}, {3.0, 2.2, 0.71, 0.0041
 constexpr TileCost kStreamCostAct[kStreamCount] = {{3.7, 0.6, 0.73, 0.0025}, {3.6, 2.0, 0.72, 0.0044}, {}, {5.2, 2.0, 0.70, 0.0049}, {}};
 
 // How the weight-streaming kernel runs a grouped launch (shape kStreamNone: it does not), from the typical rows of an expert, and
-// whether it is to run at all: other_us is the estimate of the kernel that would run instead (0: none).  The choice is 2.9 % behind
-// the best kernel and shape for the plain product, 2.7 % with the quantising epilogue (geometric means over the problems above; the
-// rule before it, the longest experts by a limit on their rows, 6.6 and 10.9 %).
+// whether it is to run at all: other_us is the estimate of the kernel that would run instead (0: none).  The choice is 2.3 % behind
+// the best kernel, shape and number of slices (geometric mean of 75 random problems, bench.py --planner-sweep stream_random; 35 %
+// at worst, 8 experts x ~418 rows x 1280 x 1920); a limit on the experts' rows in its place was 6.6 % behind for the plain product and
+// 10.9 % with the quantising epilogue.
 // With the quantising epilogue a launch may also run in two: the plain product of every (tile, K slice) first, in any tile shape, then
 // the slices' sum with the activation and the quantiser.  That pays where 256-column tiles leave most CUs idle (it costs 3.8 us +
 // the partial sums' way there and back): 8 experts x ~15 rows x 1792 x 3584 24.9 -> 17.0 us, 32 x ~9 x 512 x 5632 36.9 -> 22.4 us.
@@ -1340,9 +1342,9 @@ int run(const Problem& pr) {
   ar.splitk = rs.splitk;
   ar.kb_per_split = rs.kb_per_split;
   // Row tiles per L2 patch: 8, but 7 in launches of many rounds, whose workgroups step through the patches together: us per call with 8
-  // / 7 row tiles 4096 x 24576 x 1536 179 / 163, 4096 x 32768 x 512 156 / 128, 4000 x 28160 x 768 128 / 120, 4096 x 24576 x 4608
-  // 419 / 416 (14 such problems 1.03 x, none more than 1.5 % slower; 3 and 5 gain as much, 4, 6 and 16 do not); with one to
-  // four rounds the difference is noise.
+  // / 7 row tiles 4096 x 24576 x 1536 174 / 168, 4096 x 32768 x 512 130 / 124, 4000 x 28160 x 768 123 / 120, 3500 x 33024 x 1280
+  // 191 / 186, 4096 x 24576 x 4608 447 / 446, 2048 x 36864 x 1024 99 / 100 (5 and 6 within 2 % of 7, 4 and 16 up to 11 % behind it);
+  // with one to four rounds the difference is noise.
   ar.group_m = g_knob[kKnobGroupM] > 0 ? g_knob[kKnobGroupM] : (rs.resident ? 7 : 8);
   ar.out_f32 = pr.out_dtype == DLB_OUT_F32;
   ar.a_rows = pr.a_rows;

@@ -2,9 +2,10 @@
 package: ``ep_scatter`` (:95-158), ``ep_gather`` (:199-233) and the driver ``fused_moe_v3`` (:246-343) with the same
 positional signatures.  Differences a caller can observe: destination rows are handed out in token-major order instead
 of atomic order (both satisfy the contract that ``output_index`` names the row each slot was copied to), and the
-driver runs the gate/up GEMM, silu_and_mul and the quantiser as one kernel (same bits as the three steps) that reads the
-tokens through the row table of ``ep_scatter_rows`` instead of an expert-sorted copy, and skips the scale re-layout the
-reference needs for its GEMM.
+driver runs the gate/up GEMM, silu_and_mul and the quantiser as one kernel (same bits as the three steps), or for few or
+narrow short experts as two that add slices of K (another order of the fp32 sums, so a value next to a rounding boundary may
+move by its last place), which read the tokens through the row table of ``ep_scatter_rows`` instead of an expert-sorted copy,
+and skips the scale re-layout the reference needs for its GEMM.
 """
 from typing import List, Optional, Tuple
 
@@ -154,10 +155,10 @@ def fused_moe_v3(
     n_experts = len(num_recv_tokens_per_expert)
     down = None
 
-    # gate/up projection, silu(gate) * up and the 1 x 128 quantiser as one kernel that reads the tokens where they lie:
-    # the row tables say which expert and which token each sorted row stands for, the kernel follows them, and neither
+    # gate/up projection, silu(gate) * up and the 1 x 128 quantiser in one call that reads the tokens where they lie:
+    # the row tables say which expert and which token each sorted row stands for, the kernels follow them, and neither
     # the expert-sorted copy of the activations nor the bf16 [rows, 2 I] intermediate reaches memory.  Same bits as the
-    # steps of the reference (:288-334).
+    # steps of the reference (:288-334) unless the planner cuts K into slices, whose sums are added in another order.
     if tokens_q.is_contiguous() and hidden % 128 == 0 and inter2 % 256 == 0 and n_tokens * hidden < (1 << 32):
         # Short experts, few of them or narrow ones are a matter of reading the weights once with every CU: the weight-streaming
         # kernels, on the rows that hold a token (500 tokens, 32 experts of 7168 x 2048: 333 -> 245 us; their token offsets are 31
