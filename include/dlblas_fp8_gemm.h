@@ -401,8 +401,7 @@ int dlb_fp8_gemm_plan_wave_k(int64_t M, int64_t N, int64_t K, size_t workspace_b
  * (rows = M_max).  Outputs (each may be NULL): the kernel variant id; whether a contiguous launch of this size pairs
  * blocks into taller tiles from lists built on the device (1) or runs uniform 128-row tiles (0; always 0 for the masked
  * layout, where the kernel of dlb_fp8_gemm_plan_stream_launch may take the launch over from the named variant).  The fused gate/up entry points
- * of the contiguous layout always take the lists, so a caller that can also run GEMM and activation apart does that where
- * this says 0 (a batch of at most a round or two of tiles, where the uniform tiles are faster).  No counterpart in the
+ * of the contiguous layout always take the lists; dlb_expert_plan weighs them against the ragged ones.  No counterpart in the
  * reference.
  */
 int dlb_fp8_gemm_plan_grouped(int mode, int64_t rows, int64_t N, int64_t K, int32_t G, int32_t expected_m, size_t workspace_bytes,
