@@ -13,6 +13,7 @@
 #include "fp8_gemm_common.h"
 #include "host_common.h"
 #include "fp8_gemm_pipelined.h"
+#include "fp8_gemm_ring.h"
 #include "fp8_gemm_skinny.h"
 #include "fp8_gemm_stream.h"
 #include "fp8_gemm_tiled.h"
@@ -138,7 +139,13 @@ typedef TileCfg<128, 128, 2, 2> Tile128x128;
 typedef TileCfg<64, 128, 2, 2> Tile64x128;
 typedef TileCfg<128, 64, 2, 2> Tile128x64;
 typedef PipeCfg<4, 2, 2, 4, 2, 2> Pipe256x256;  // 8 waves, wave tile 64 x 128
-typedef PipeCfg<4, 2, 2, 3, 2, 2> Pipe256x192;  // narrow tiles of the mixed-width launch
+typedef RingCfg<4, 2, 4, 8, 2> Ring256x256;      // 8 waves, wave tile 64 x 128
+typedef RingCfg<4, 2, 4, 6, 2> Ring256x192;      // narrow tiles of the mixed-width launch
+typedef RingCfg<2, 4, 4, 4, 3> Ring128x256;      // wave tile 64 x 64
+// the same with a tile's activation scales in a table behind the ring (row-major a_s)
+typedef RingCfg<4, 2, 4, 8, 2, true, 27> Ring256x256T;
+typedef RingCfg<4, 2, 4, 6, 2, true, 27> Ring256x192T;
+typedef RingCfg<2, 4, 4, 4, 3, true, 16> Ring128x256T;
 typedef PipeCfg<2, 4, 3, 2, 2, 2> Pipe192x256;  // the two tiles of an expert's run of three 128-row blocks
 
 // bytes of the three tile lists of an expert-contiguous launch over nblk 128-row blocks
@@ -160,11 +167,8 @@ typedef PipeCfg<2, 2, 2, 1, 5, 2, true> Pipe128x64;   // wave tile 64 x 32, 5 st
 // workgroup as the LDS left by the ring holds: 54 and 64)
 typedef PipeCfg<2, 2, 2, 2, 4, 2, true, true, 54> Pipe128x128T;
 typedef PipeCfg<2, 2, 2, 1, 5, 2, true, true, 64> Pipe128x64T;
-typedef PipeCfg<2, 4, 2, 2, 3, 2, false, true, 16> Pipe128x256w8T;  // 8 KB next to the 150 KB ring
-typedef PipeCfg<4, 2, 2, 4, 2, 2, false, true, 27> Pipe256x256T;    // 28 KB next to 132 KB
-typedef PipeCfg<4, 2, 2, 3, 2, 2, false, true, 27> Pipe256x192T;
-static_assert(Pipe256x256T::LDS_BYTES <= 160 * 1024 && Pipe256x192T::LDS_BYTES <= Pipe256x256T::LDS_BYTES, "ring + table fit the LDS");
-static_assert(Pipe128x256w8T::LDS_BYTES <= 160 * 1024 && Pipe128x128T::LDS_BYTES <= 160 * 1024 && Pipe128x64T::LDS_BYTES <= 160 * 1024, "ring + table fit the LDS");
+static_assert(Ring256x192T::LDS_BYTES <= Ring256x256T::LDS_BYTES && Ring256x192::LDS_BYTES <= Ring256x256::LDS_BYTES, "a mixed launch asks for the wide tiles' LDS");
+static_assert(Pipe128x128T::LDS_BYTES <= 160 * 1024 && Pipe128x64T::LDS_BYTES <= 160 * 1024, "ring + table fit the LDS");
 constexpr int kFusedMaxTiles = DLB_WS_COUNTER_BYTES / 16;  // four counter words per tile in the workspace head
 
 // Tile shapes of the weight-streaming grouped kernel: rows x weight rows per tile, and the ring each leaves room for.
@@ -190,6 +194,14 @@ struct WaveKDims { int mf, nf, waves; };
 constexpr WaveKDims kWaveKDims[] = {{1, 1, 8}, {1, 1, 4}, {2, 1, 8}, {1, 2, 4}, {2, 1, 4}, {2, 2, 4}, {2, 2, 2}};
 constexpr int kWaveKCount = sizeof(kWaveKDims) / sizeof(kWaveKDims[0]);
 constexpr int kWaveKNone = -1;
+
+// Resident workgroups for a dense launch of `tiles` equal tiles: as many rounds as with one per CU, but even ones.  448 tiles are
+// two rounds of 224 workgroups, whose clock is higher than that of 256 of which the last 64 have one tile.  A multiple of 8,
+// so that a workgroup's tiles stay on one XCD.
+int64_t resident_grid(int64_t tiles, int cus) {
+  const int64_t even = ceil_div(ceil_div(tiles, ceil_div(tiles, cus)), 8) * 8;
+  return even < cus ? even : cus;
+}
 
 // Raise a kernel's dynamic LDS limit once per (kernel, device).
 template <class Kernel>
@@ -242,6 +254,31 @@ hipError_t launch_pipelined(const Args& args, int grid, int dev, hipStream_t str
   if (e != hipSuccess || g_prepare_only) return e;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, args);
   return hipGetLastError();
+}
+
+template <class Cfg, int MODE, bool AHEAD = false>
+hipError_t launch_ring(const Args& args, int grid, int dev, hipStream_t stream) {
+  static std::atomic<unsigned long long> lds_done{0};
+  auto kernel = fp8_gemm_ring_kernel<Cfg, MODE, AHEAD>;
+  hipError_t e = ensure_lds(kernel, Cfg::LDS_BYTES, dev, &lds_done);
+  if (e != hipSuccess || g_prepare_only) return e;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, args);
+  return hipGetLastError();
+}
+
+template <class Cfg>
+hipError_t launch_ring_mode(int mode, const Args& args, int grid, int dev, hipStream_t stream) {
+  switch (mode) {
+    case kDense:
+      // resident workgroups of more than one tile: the ring that runs on (a single tile is 1 us faster without its code)
+      if (args.splitk == 1 && static_cast<int64_t>(args.tiles_m) * args.tiles_n > grid) return launch_ring<Cfg, kDense, true>(args, grid, dev, stream);
+      return launch_ring<Cfg, kDense>(args, grid, dev, stream);
+    case kContiguous:
+      if constexpr (Cfg::BM == kScaleBlock) return launch_ring<Cfg, kContiguous>(args, grid, dev, stream);  // taller tiles come from the lists
+      return hipErrorInvalidValue;
+    default:
+      return launch_ring<Cfg, kMasked>(args, grid, dev, stream);
+  }
 }
 
 template <class Cfg, bool KTAIL>
@@ -345,9 +382,6 @@ template <class Cfg>
 hipError_t launch_pipelined_mode(int mode, const Args& args, int grid, int dev, hipStream_t stream) {
   switch (mode) {
     case kDense:
-      // resident workgroups of more than one tile: the ring that runs on (a single tile is 1 us faster without its code)
-      if constexpr (!Cfg::PREFETCH)
-        if (static_cast<int64_t>(args.tiles_m) * args.tiles_n * args.splitk > grid) return launch_pipelined<Cfg, kDense, true>(args, grid, dev, stream);
       return launch_pipelined<Cfg, kDense>(args, grid, dev, stream);
     case kContiguous:
       return launch_pipelined<Cfg, kContiguous>(args, grid, dev, stream);
@@ -610,7 +644,7 @@ MidChoice pick_mid_plan(int64_t M, int64_t N, int kblocks, int cus, size_t ws_av
       const int64_t units = ceil_div(M, c.bm) * ceil_div(N, c.bn) * sk;
       // a tile's scales come once, into a table in LDS, when the slice is short enough: no re-layout launch and no scattered scale
       // lines per K step
-      const bool table = per <= (c.variant == kVarPipe128x64 ? Pipe128x64T::SCTAB_KB : c.variant == kVarPipe128x128 ? Pipe128x128T::SCTAB_KB : Pipe128x256w8T::SCTAB_KB);
+      const bool table = per <= (c.variant == kVarPipe128x64 ? Pipe128x64T::SCTAB_KB : c.variant == kVarPipe128x128 ? Pipe128x128T::SCTAB_KB : Ring128x256T::SCTAB_KB);
       double us = launch + (table ? 0.0 : relayout) +
                   static_cast<double>(ceil_div(units, cus)) * (tile_fixed + per * c.step_us * short_rows * (table ? 1.0 : scattered));
       if (sk > 1) us += second_pass + (2.0 * sk + 0.5) * out_bytes / ws_rate;  // partial sums written, read back, result written
@@ -888,7 +922,7 @@ double masked_ring_us(int variant, int64_t M, int64_t N, int64_t K, int G, int64
   else if (variant == kVarPipe128x128) c = {2.3, 3.6, 0.65, 0.0014};
   else if (variant == kVarPipe256x256) c = {1.5, 7.1, 1.51, 0.0015};
   const ExpertRows e(M, hint_rows);
-  const bool table = !act && kblocks <= (variant == kVarPipe128x128 ? Pipe128x128T::SCTAB_KB : variant == kVarPipe256x256 ? Pipe256x256T::SCTAB_KB : Pipe128x256w8T::SCTAB_KB);
+  const bool table = !act && kblocks <= (variant == kVarPipe128x128 ? Pipe128x128T::SCTAB_KB : variant == kVarPipe256x256 ? Ring256x256T::SCTAB_KB : Ring128x256T::SCTAB_KB);
   const double tiles = G * e.live * e.row_tiles(bm) * static_cast<double>(act ? N / 256 : ceil_div(N, bn));
   return (M > kRelayoutMinRows && !table ? 3.5 : 0.0) + grouped_us(c, tiles, e.span <= bm, kblocks, bn, e.rows(bm), e.sharing(bm), 6.2e6, cus);
 }
@@ -1048,8 +1082,8 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
     switch (pl.variant) {
       case kVarPipe128x64: return mode == kDense && kb_per <= Pipe128x64T::SCTAB_KB;
       case kVarPipe128x128: return kb_per <= Pipe128x128T::SCTAB_KB;
-      case kVarPipe128x256w8: return (mode != kMasked || g_forced_variant < 0) && kb_per <= Pipe128x256w8T::SCTAB_KB;
-      case kVarPipe256x256: case kVarPipe256mix: return kb_per <= Pipe256x256T::SCTAB_KB;
+      case kVarPipe128x256w8: return (mode != kMasked || g_forced_variant < 0) && kb_per <= Ring128x256T::SCTAB_KB;
+      case kVarPipe256x256: case kVarPipe256mix: return kb_per <= Ring256x256T::SCTAB_KB;
       default: return false;
     }
   };
@@ -1348,6 +1382,7 @@ int run(const Problem& pr) {
   ar.group_m = g_knob[kKnobGroupM] > 0 ? g_knob[kKnobGroupM] : (rs.resident ? 7 : 8);
   ar.out_f32 = pr.out_dtype == DLB_OUT_F32;
   ar.a_rows = pr.a_rows;
+  ar.a_src_rows = pr.a_src_rows;
   ar.act_s = pr.act_s;
   ar.act_s_gs = pr.act_s_sg;
   ar.act_s_sm = pr.act_s_sm;
@@ -1403,25 +1438,25 @@ int run(const Problem& pr) {
                                 cus, dev, pr.stream);
     }
     const int g = static_cast<int>(rs.grid);
-    const int g_dense = rs.resident ? cus : g;
+    const int g_dense = static_cast<int>(rs.resident ? resident_grid(rs.grid, cus) : rs.grid);
     if (pl.variant == kVarPipe256mix) {
       const int64_t split = rs.n_split;
       if (split >= pr.N)
-        return rs.sctab ? launch_pipelined_mode<Pipe256x256T>(pr.mode, ar, g_dense, dev, pr.stream) : launch_pipelined_mode<Pipe256x256>(pr.mode, ar, g_dense, dev, pr.stream);
+        return rs.sctab ? launch_ring_mode<Ring256x256T>(pr.mode, ar, g_dense, dev, pr.stream) : launch_ring_mode<Ring256x256>(pr.mode, ar, g_dense, dev, pr.stream);
       static std::atomic<unsigned long long> lds_done[2];
-      auto kernel = rs.sctab ? fp8_gemm_pipelined_mixed_kernel<Pipe256x256T, Pipe256x192T> : fp8_gemm_pipelined_mixed_kernel<Pipe256x256, Pipe256x192>;
-      const int lds = rs.sctab ? Pipe256x256T::LDS_BYTES : Pipe256x256::LDS_BYTES;
+      auto kernel = rs.sctab ? fp8_gemm_ring_mixed_kernel<Ring256x256T, Ring256x192T> : fp8_gemm_ring_mixed_kernel<Ring256x256, Ring256x192>;
+      const int lds = rs.sctab ? Ring256x256T::LDS_BYTES : Ring256x256::LDS_BYTES;
       ar.n_split = static_cast<int>(split);
       ar.tiles_n_a = static_cast<int>(split / 256);
       ar.tiles_n_b = static_cast<int>(ceil_div(pr.N - split, 192));
       ar.tiles_a = ar.tiles_m * ar.tiles_n_a;
       const hipError_t le = ensure_lds(kernel, lds, dev, &lds_done[rs.sctab ? 1 : 0]);
       if (le != hipSuccess || g_prepare_only) return le;
-      hipLaunchKernelGGL(kernel, dim3(ar.tiles_a + ar.tiles_m * ar.tiles_n_b), dim3(Pipe256x256::NT), lds, pr.stream, ar);
+      hipLaunchKernelGGL(kernel, dim3(ar.tiles_a + ar.tiles_m * ar.tiles_n_b), dim3(Ring256x256::NT), lds, pr.stream, ar);
       return hipGetLastError();
     }
     if (pl.variant == kVarPipe256x256)
-      return rs.sctab ? launch_pipelined_mode<Pipe256x256T>(pr.mode, ar, g_dense, dev, pr.stream) : launch_pipelined_mode<Pipe256x256>(pr.mode, ar, g_dense, dev, pr.stream);
+      return rs.sctab ? launch_ring_mode<Ring256x256T>(pr.mode, ar, g_dense, dev, pr.stream) : launch_ring_mode<Ring256x256>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x256w8 && tile_list && pr.act) {
       static std::atomic<unsigned long long> lds_done{0};
       auto kernel = fp8_gemm_contig_list_act_kernel<Pipe256x256, Pipe192x256, Pipe128x256w8>;
@@ -1442,8 +1477,8 @@ int run(const Problem& pr) {
     }
     if (pl.variant == kVarPipe128x256w8 && pr.act)
       return launch_pipelined<Pipe128x256w8, kMaskedAct>(ar, g, dev, pr.stream);  // N / 256 column tiles, as the plain GEMM
-    if (pl.variant == kVarPipe128x256w8 && rs.sctab) return launch_pipelined_mode<Pipe128x256w8T>(pr.mode, ar, g_dense, dev, pr.stream);
-    if (pl.variant == kVarPipe128x256w8) return launch_pipelined_mode<Pipe128x256w8>(pr.mode, ar, g_dense, dev, pr.stream);
+    if (pl.variant == kVarPipe128x256w8 && rs.sctab) return launch_ring_mode<Ring128x256T>(pr.mode, ar, g_dense, dev, pr.stream);
+    if (pl.variant == kVarPipe128x256w8) return launch_ring_mode<Ring128x256>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x128)
       return rs.sctab ? launch_pipelined_mode<Pipe128x128T>(pr.mode, ar, g, dev, pr.stream)
                       : launch_pipelined_mode<Pipe128x128>(pr.mode, ar, g, dev, pr.stream);

@@ -72,6 +72,15 @@ __device__ __forceinline__ void dma_4(const uint8_t* base, uint32_t voff, uint8_
   __builtin_amdgcn_global_load_lds((global_ptr_t)(base + voff), (lds_ptr_t)lds_dst, 4, 0, 0);
 }
 
+template <int POLICY>
+__device__ __forceinline__ void buf_dma_16(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff, uint8_t* lds_dst) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)lds_dst, 16, voff, soff, 0, POLICY);
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const uint8_t* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, bytes, 0x00020000);
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   // s_waitcnt with only vmcnt constrained: vmcnt = simm16[3:0] | simm16[15:14] << 4, expcnt [6:4], lgkmcnt [11:8]

@@ -63,15 +63,6 @@ struct StreamCfg {
 
 typedef const __attribute__((address_space(4))) float* const_float_ptr_t;
 
-template <int POLICY>
-__device__ __forceinline__ void buf_dma_16(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff, uint8_t* lds_dst) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)lds_dst, 16, voff, soff, 0, POLICY);
-}
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const uint8_t* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, bytes, 0x00020000);
-}
-
 // Wait until at most `younger` (0 .. MAX) groups of L vector-memory instructions are on their way.
 template <int L, int MAX>
 __device__ __forceinline__ void wait_groups(int younger) {
