@@ -138,35 +138,29 @@ const char* const kVariantNames[kVarCount] = {
 typedef TileCfg<128, 128, 2, 2> Tile128x128;
 typedef TileCfg<64, 128, 2, 2> Tile64x128;
 typedef TileCfg<128, 64, 2, 2> Tile128x64;
-typedef PipeCfg<4, 2, 2, 4, 2, 2> Pipe256x256;  // 8 waves, wave tile 64 x 128
 typedef RingCfg<4, 2, 4, 8, 2> Ring256x256;      // 8 waves, wave tile 64 x 128
 typedef RingCfg<4, 2, 4, 6, 2> Ring256x192;      // narrow tiles of the mixed-width launch
+typedef RingCfg<2, 4, 6, 4, 2> Ring192x256;      // wave tile 96 x 64: the two tiles of an expert's run of three 128-row blocks
 typedef RingCfg<2, 4, 4, 4, 3> Ring128x256;      // wave tile 64 x 64
 // the same with a tile's activation scales in a table behind the ring (row-major a_s)
 typedef RingCfg<4, 2, 4, 8, 2, true, 27> Ring256x256T;
 typedef RingCfg<4, 2, 4, 6, 2, true, 27> Ring256x192T;
 typedef RingCfg<2, 4, 4, 4, 3, true, 16> Ring128x256T;
-typedef PipeCfg<2, 4, 3, 2, 2, 2> Pipe192x256;  // the two tiles of an expert's run of three 128-row blocks
 
 // bytes of the three tile lists of an expert-contiguous launch over nblk 128-row blocks
 constexpr size_t tile_list_bytes(int64_t nblk) {
   return (static_cast<size_t>(kTileListHeader + 3 * nblk) * sizeof(int32_t) + 255) / 256 * 256;
 }
-typedef PipeCfg<2, 4, 2, 2, 3> Pipe128x256w8;  // 8 waves, wave tile 64 x 64
-constexpr int kListLds = Pipe256x256::LDS_BYTES > Pipe128x256w8::LDS_BYTES
-                             ? (Pipe256x256::LDS_BYTES > Pipe192x256::LDS_BYTES ? Pipe256x256::LDS_BYTES : Pipe192x256::LDS_BYTES)
-                             : (Pipe128x256w8::LDS_BYTES > Pipe192x256::LDS_BYTES ? Pipe128x256w8::LDS_BYTES : Pipe192x256::LDS_BYTES);
+constexpr int kListLds = Ring256x256::ACT_LDS_BYTES > Ring128x256::ACT_LDS_BYTES
+                             ? (Ring256x256::ACT_LDS_BYTES > Ring192x256::ACT_LDS_BYTES ? Ring256x256::ACT_LDS_BYTES : Ring192x256::ACT_LDS_BYTES)
+                             : (Ring128x256::ACT_LDS_BYTES > Ring192x256::ACT_LDS_BYTES ? Ring128x256::ACT_LDS_BYTES : Ring192x256::ACT_LDS_BYTES);
 // small tiles for problems with few of the large ones (M of a few hundred, or a narrow N): 4 waves, deep rings
-#ifdef DLB_EXP_P128
-typedef PipeCfg<2, 2, 2, 2, DLB_EXP_P128, 2, false> Pipe128x128;  // experiment: 4 waves, in-place K loop, DLB_EXP_P128 stages
-#else
-typedef PipeCfg<2, 2, 2, 2, 4, 2, true> Pipe128x128;  // wave tile 64 x 64, 4 stages of 34 KB
-#endif
-typedef PipeCfg<2, 2, 2, 1, 5, 2, true> Pipe128x64;   // wave tile 64 x 32, 5 stages of 26 KB
+typedef PipeCfg<2, 2, 2, 2, 4> Pipe128x128;  // wave tile 64 x 64, 4 stages of 34 KB
+typedef PipeCfg<2, 2, 2, 1, 5> Pipe128x64;   // wave tile 64 x 32, 5 stages of 26 KB
 // the same with the activation scales of a tile in a table behind the ring (row-major a_s; as many K blocks per
 // workgroup as the LDS left by the ring holds: 54 and 64)
-typedef PipeCfg<2, 2, 2, 2, 4, 2, true, true, 54> Pipe128x128T;
-typedef PipeCfg<2, 2, 2, 1, 5, 2, true, true, 64> Pipe128x64T;
+typedef PipeCfg<2, 2, 2, 2, 4, true, 54> Pipe128x128T;
+typedef PipeCfg<2, 2, 2, 1, 5, true, 64> Pipe128x64T;
 static_assert(Ring256x192T::LDS_BYTES <= Ring256x256T::LDS_BYTES && Ring256x192::LDS_BYTES <= Ring256x256::LDS_BYTES, "a mixed launch asks for the wide tiles' LDS");
 static_assert(Pipe128x128T::LDS_BYTES <= 160 * 1024 && Pipe128x64T::LDS_BYTES <= 160 * 1024, "ring + table fit the LDS");
 constexpr int kFusedMaxTiles = DLB_WS_COUNTER_BYTES / 16;  // four counter words per tile in the workspace head
@@ -246,10 +240,10 @@ hipError_t launch_tiled_mode(int mode, const Args& args, int grid, int dev, hipS
   }
 }
 
-template <class Cfg, int MODE, bool AHEAD = false>
+template <class Cfg, int MODE>
 hipError_t launch_pipelined(const Args& args, int grid, int dev, hipStream_t stream) {
   static std::atomic<unsigned long long> lds_done{0};
-  auto kernel = fp8_gemm_pipelined_kernel<Cfg, MODE, AHEAD>;
+  auto kernel = fp8_gemm_pipelined_kernel<Cfg, MODE>;
   hipError_t e = ensure_lds(kernel, Cfg::LDS_BYTES, dev, &lds_done);
   if (e != hipSuccess || g_prepare_only) return e;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, args);
@@ -259,10 +253,11 @@ hipError_t launch_pipelined(const Args& args, int grid, int dev, hipStream_t str
 template <class Cfg, int MODE, bool AHEAD = false>
 hipError_t launch_ring(const Args& args, int grid, int dev, hipStream_t stream) {
   static std::atomic<unsigned long long> lds_done{0};
+  constexpr int lds = MODE == kMaskedAct ? Cfg::ACT_LDS_BYTES : Cfg::LDS_BYTES;
   auto kernel = fp8_gemm_ring_kernel<Cfg, MODE, AHEAD>;
-  hipError_t e = ensure_lds(kernel, Cfg::LDS_BYTES, dev, &lds_done);
+  hipError_t e = ensure_lds(kernel, lds, dev, &lds_done);
   if (e != hipSuccess || g_prepare_only) return e;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, args);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NT), lds, stream, args);
   return hipGetLastError();
 }
 
@@ -270,8 +265,9 @@ template <class Cfg>
 hipError_t launch_ring_mode(int mode, const Args& args, int grid, int dev, hipStream_t stream) {
   switch (mode) {
     case kDense:
-      // resident workgroups of more than one tile: the ring that runs on (a single tile is 1 us faster without its code)
-      if (args.splitk == 1 && static_cast<int64_t>(args.tiles_m) * args.tiles_n > grid) return launch_ring<Cfg, kDense, true>(args, grid, dev, stream);
+      // resident workgroups of more than one tile: the ring that runs on (a single tile is 1 us faster without its code; the knob for
+      // stores apart from the ring asks for tiles that start afresh)
+      if (args.splitk == 1 && args.c_lds && static_cast<int64_t>(args.tiles_m) * args.tiles_n > grid) return launch_ring<Cfg, kDense, true>(args, grid, dev, stream);
       return launch_ring<Cfg, kDense>(args, grid, dev, stream);
     case kContiguous:
       if constexpr (Cfg::BM == kScaleBlock) return launch_ring<Cfg, kContiguous>(args, grid, dev, stream);  // taller tiles come from the lists
@@ -1459,24 +1455,24 @@ int run(const Problem& pr) {
       return rs.sctab ? launch_ring_mode<Ring256x256T>(pr.mode, ar, g_dense, dev, pr.stream) : launch_ring_mode<Ring256x256>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x256w8 && tile_list && pr.act) {
       static std::atomic<unsigned long long> lds_done{0};
-      auto kernel = fp8_gemm_contig_list_act_kernel<Pipe256x256, Pipe192x256, Pipe128x256w8>;
+      auto kernel = fp8_gemm_ring_list_kernel<Ring256x256, Ring192x256, Ring128x256, kContigListAct>;
       const hipError_t le = ensure_lds(kernel, kListLds, dev, &lds_done);
       if (le != hipSuccess || g_prepare_only) return le;
       ar.tiles_n = static_cast<int>(pr.N / 256);  // 128 output columns = 128 gate + 128 up weight rows per tile
-      hipLaunchKernelGGL(kernel, dim3(cus), dim3(Pipe256x256::NT), kListLds, pr.stream, ar);
+      hipLaunchKernelGGL(kernel, dim3(cus), dim3(Ring256x256::NT), kListLds, pr.stream, ar);
       return hipGetLastError();
     }
     if (pl.variant == kVarPipe128x256w8 && tile_list) {
       static std::atomic<unsigned long long> lds_done{0};
-      auto kernel = fp8_gemm_contig_list_kernel<Pipe256x256, Pipe192x256, Pipe128x256w8>;
+      auto kernel = fp8_gemm_ring_list_kernel<Ring256x256, Ring192x256, Ring128x256, kContigList>;
       const hipError_t le = ensure_lds(kernel, kListLds, dev, &lds_done);
       if (le != hipSuccess || g_prepare_only) return le;
       ar.tiles_n = static_cast<int>(ceil_div(pr.N, 256));
-      hipLaunchKernelGGL(kernel, dim3(cus), dim3(Pipe256x256::NT), kListLds, pr.stream, ar);  // one resident workgroup per CU
+      hipLaunchKernelGGL(kernel, dim3(cus), dim3(Ring256x256::NT), kListLds, pr.stream, ar);  // one resident workgroup per CU
       return hipGetLastError();
     }
     if (pl.variant == kVarPipe128x256w8 && pr.act)
-      return launch_pipelined<Pipe128x256w8, kMaskedAct>(ar, g, dev, pr.stream);  // N / 256 column tiles, as the plain GEMM
+      return launch_ring<Ring128x256, kMaskedAct>(ar, g, dev, pr.stream);  // N / 256 column tiles, as the plain GEMM
     if (pl.variant == kVarPipe128x256w8 && rs.sctab) return launch_ring_mode<Ring128x256T>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x256w8) return launch_ring_mode<Ring128x256>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x128)

@@ -21,7 +21,7 @@ typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
 constexpr int kScaleBlock = 128;  // K (and N) extent covered by one scale; also bytes per LDS tile row
 
 // kContigList: contiguous, tiles from a device-built list.  kContigListAct: the same for the gate/up projection of an
-// expert MLP with silu(gate) * up and the 1 x 128 quantiser applied in the epilogue (see fp8_gemm_contig_list_act_kernel).
+// expert MLP with silu(gate) * up and the 1 x 128 quantiser applied in the epilogue (see fp8_gemm_ring_list_kernel).
 // kMaskedAct: that epilogue on the masked layout, with the masked activation's two roundings (dlblas/kernels/moe.py:256-257).
 enum Mode : int { kDense = 0, kContiguous = 1, kMasked = 2, kContigList = 3, kContigListAct = 4, kMaskedAct = 5 };
 
@@ -64,7 +64,7 @@ struct Args {
   int tiles_a;          //   tiles in the wide region (tiles_m x tiles_n_a)
   int tiles_n_a;
   int tiles_n_b;
-  const int32_t* tlist;  // kContigList: [0] = 256-row tiles, [1] = 128-row tiles, then the two lists of 128-row block indices
+  const int32_t* tlist;  // kContigList: counts of 256-, 192- and 128-row tiles, then the three lists of first rows (see contiguous_tile_list_block)
   int tlist_cap;         //   entries per list
   // kContigListAct / kMaskedAct: c is the e4m3 output [G][M][act_cols] with row stride act_q_stride (bytes);
   // N = 2 act_cols weight rows

@@ -1,6 +1,7 @@
-// Compute-bound FP8 block-scaled GEMM for gfx950: 32x32x64 e4m3 MFMA, tiles streamed HBM -> LDS by the DMA
-// path of the memory pipeline (global_load_lds_dwordx4, no VGPR staging), multi-stage LDS ring, one barrier
-// per 128-wide K step, block scales applied with one FMA per accumulator element and K step.
+// FP8 block-scaled GEMM for gfx950 in tiles of 128 x 128 and 128 x 64, for problems with too few of the larger tiles for the chip
+// (fp8_gemm_ring.h): 32x32x64 e4m3 MFMA, tiles streamed HBM -> LDS by the DMA path of the memory pipeline
+// (global_load_lds_dwordx4, no VGPR staging), multi-stage LDS ring, one barrier per 128-wide K step, block scales applied with
+// one FMA per accumulator element and K step.  Also what both files share: DMA and wait primitives, the pre-passes.
 //
 // Workgroup = WGM x WGN waves, one wave per SIMD; a wave owns MF x NF fragments of 32 x 32 outputs.
 // MFMA operand roles: "A" = 32 rows of the weight tile (n), "B" = 32 rows of the activation tile (m), so a lane's
@@ -114,19 +115,15 @@ __device__ __forceinline__ void each_index(F&& f, std::integer_sequence<int, I..
   (f(std::integral_constant<int, I>{}), ...);
 }
 
-// PARTS_: 2 = the scale FMAs of a fragment run under the MFMAs of the NEXT fragment of the same wave (two partial
-// accumulators); 1 = they follow their own MFMAs and overlap with the other wave of the SIMD instead (16 fewer VGPRs).
-// PREFETCH_: true (one wave per SIMD, 512 registers) = every fragment of the NEXT K step is read into a second
-// register set while the current step computes, so no MFMA of a step waits for LDS.
+// One wave per SIMD, 512 registers: every fragment of the NEXT K step is read into a second register set while the current step
+// computes, so no MFMA of a step waits for LDS.
 // SCTAB_: true = the activation scales of a tile's rows for ALL K blocks of the workgroup's K range (at most
 // SCTAB_KB) are fetched once per tile into a table behind the ring, lanes along K: a row-major a_s then costs one
 // cache-line request per row and tile instead of one per row and K step, and needs no re-layout pass in front.
-template <int WGM_, int WGN_, int MF_, int NF_, int STAGES_, int PARTS_ = 2, bool PREFETCH_ = false, bool SCTAB_ = false, int SCTAB_KB_ = 32>
+template <int WGM_, int WGN_, int MF_, int NF_, int STAGES_, bool SCTAB_ = false, int SCTAB_KB_ = 32>
 struct PipeCfg {
-  static constexpr int WGM = WGM_, WGN = WGN_, MF = MF_, NF = NF_, STAGES = STAGES_, PARTS = PARTS_;
-  static constexpr bool PREFETCH = PREFETCH_;
+  static constexpr int WGM = WGM_, WGN = WGN_, MF = MF_, NF = NF_, STAGES = STAGES_;
   static constexpr bool SCTAB = SCTAB_;
-  static constexpr bool UNIFORM_W = (128 % (NF_ * 32)) == 0;
   static constexpr int WAVES = WGM * WGN;
   static constexpr int NT = WAVES * 64;
   static constexpr int BM = WGM * MF * 32;
@@ -145,7 +142,8 @@ struct PipeCfg {
   static constexpr int LDS_BYTES = STAGES * STAGE_BYTES + SCTAB_BYTES;
   static constexpr int LOADS_PER_STAGE = A_INST + B_INST + S_INST + 1;  // vmcnt units per wave and stage
   static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "tile rows must divide over the DMA instructions");
-  static_assert(NF <= 4, "weight scales are fetched for at most four fragments per wave");
+  static_assert(128 % (NF * 32) == 0, "a wave's columns share one weight scale");
+  static_assert(MF * NF <= 4, "both fragment sets fit the registers");
   static_assert(LOADS_PER_STAGE * (STAGES - 1) < 64, "vmcnt is a 6-bit counter");
 };
 
@@ -185,25 +183,13 @@ __global__ void __launch_bounds__(256) fp8_scale_transpose_kernel(const float* s
 
 constexpr int kTileListHeader = 3;  // tile counts in front of the three tile lists of an expert-contiguous launch
 
-// Work of one workgroup: tiles vb_first, vb_first + gridDim.x, ... of a region that is tiles_m x tiles_n tiles of
-// BM x BN and starts at column n_base of the output.
-template <class Cfg, int MODE, bool AHEAD = false>
-__device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int vb_first, int tiles_m, int tiles_n,
-                                               int n_base) {
+// Work of one workgroup: tiles vb_first, vb_first + gridDim.x, ... of tiles_m x tiles_n tiles of BM x BN.
+template <class Cfg, int MODE>
+__device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int vb_first, int tiles_m, int tiles_n) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, MF = Cfg::MF, NF = Cfg::NF, WAVES = Cfg::WAVES, STAGES = Cfg::STAGES;
-  // One weight scale per wave and K step when the wave's n span cannot straddle a 128-column scale block,
-  // otherwise one per 32-column fragment.
-  constexpr bool kUniformW = Cfg::UNIFORM_W;
-  constexpr int NS = kUniformW ? 1 : NF;
-  constexpr bool kList = MODE == kContigList || MODE == kContigListAct;
-  // Fused activation: a tile's 256 weight rows are 128 gate rows and the 128 up rows of the same output columns, so
-  // that the epilogue has silu(gate) * up of 128 columns - one quantisation group - for every row of the tile.
-  constexpr bool kAct = MODE == kContigListAct || MODE == kMaskedAct;
-  constexpr bool kMaskedLike = MODE == kMasked || MODE == kMaskedAct;
   // Grouped modes: an expert's weight tile is read by the one to three row tiles of that expert, not by a column of
   // the grid: streamed (2 - 7 % faster from 128 to 768 rows per expert at 32 x 4096 x 7168).
   constexpr int kWeightPolicy = MODE == kDense ? kDmaKeep : kDmaStream;
-  static_assert(!kAct || (BN == 256 && kUniformW), "the fused activation pairs 128 gate columns with 128 up columns");
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -232,19 +218,9 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
     tm = first_m + in_grp % gsz;
     tn = in_grp / gsz;
   };
-  // AHEAD (dense): the ring runs on from tile to tile.  The steps of a tile whose fetches lie past the end of K
-  // fetch the first K blocks of the workgroup's NEXT tile: its first block is on its way under the last steps and is waited
-  // for by the last one like any other, so that it lands before this tile's
-  // stores are issued (the memory counter is one for loads and stores: a load behind them is only known to have landed
-  // when they have).  A tile of 256 x 256 then takes 5.4 us on top of its K steps in place of 7.8: the stores (3 to 4 us of
-  // 128 KB per CU) and the staging of the results remain.  4096 x 24576 x 1536 177 -> 165 us, 4000 x 28160 x 768 124 -> 113,
-  // 4096 x 20480 x 1024 fp32 137 -> 127.
-  static_assert(!AHEAD || (MODE == kDense && !Cfg::PREFETCH), "the tile kernels this is written for");
-  int stage = 0;
-  bool staged = false;  // AHEAD: the ring holds the tile's first STAGES - 1 K blocks from `stage` on, and the next block's activations
   for (int vb = vb_first;; vb += gridDim.x) {
-    int g = 0, mt = 0, nt, m_end, m_first = -1, split = 0, tile_lin = 0;
-    if (kMaskedLike) {
+    int g = 0, mt = 0, nt, m_end, split = 0, tile_lin = 0;
+    if (MODE == kMasked) {
       // The tile count is only known on the device, so the grid is persistent; the hardware deals consecutive
       // workgroups to the 8 XCDs in turn.  Of every 32 consecutive tiles each XCD takes 4 consecutive ones: the row
       // tiles of an expert, which are adjacent in the order and read the same weight tile, meet in one L2, and the
@@ -267,28 +243,6 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
       mt = local % mtiles;
       nt = local / mtiles;
       m_end = min(max(p.gidx[g], 0), p.M);
-    } else if (kList) {
-      // tiles of this height come from the list the pre-pass built: entry = first 128-row block of the tile.  The
-      // column tiles of one row block are adjacent in the order, so they share the activation tile in L2.
-      static_assert(BM == 256 || BM == 192 || BM == 128, "tile heights of the three lists");
-      constexpr int kWhich = BM == 256 ? 0 : (BM == 192 ? 1 : 2);
-      const int cnt = p.tlist[kWhich];
-      const int total = cnt * tiles_n;
-      if (vb >= total) break;
-      const int t = xcd_remap(vb, total);
-      int li;
-      if (BM == 192) {
-        // the two tiles of a pair side by side for every column tile: neighbours in the order run on one XCD at the same time
-        const int pair = t / (2 * tiles_n), r = t - pair * 2 * tiles_n;
-        nt = r >> 1;
-        li = 2 * pair + (r & 1);
-      } else {
-        li = t / tiles_n;
-        nt = t - li * tiles_n;
-      }
-      m_first = p.tlist[kTileListHeader + kWhich * p.tlist_cap + li] * 64;
-      g = p.gidx[m_first];
-      m_end = min(p.M, m_first + BM);
     } else {
       if (vb >= units) break;
       locate(vb, tile_lin, split, mt, nt);
@@ -299,35 +253,26 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
       }
     }
     g = __builtin_amdgcn_readfirstlane(g);
-    const int m0 = __builtin_amdgcn_readfirstlane(kList ? m_first : mt * BM);
-    // fused activation: n0 is the first OUTPUT column of the tile; weight row of tile column c: see w_row below
-    const int n0 = __builtin_amdgcn_readfirstlane(kAct ? nt * (BN / 2) : n_base + nt * BN);
-    auto w_row = [&](int c) { return c < BN / 2 ? n0 + c : p.act_cols + n0 + c - BN / 2; };
+    const int m0 = __builtin_amdgcn_readfirstlane(mt * BM);
+    const int n0 = __builtin_amdgcn_readfirstlane(nt * BN);
 
     const int64_t esz = p.out_f32 ? 4 : 2;
     const bool sliced = MODE == kDense && p.splitk > 1;
     const int kb_first = sliced ? split * p.kb_per_split : 0;  // the host leaves no slice empty
     const int nk = sliced ? min(p.kblocks, kb_first + p.kb_per_split) - kb_first : p.kblocks;  // K blocks of this unit
-    // activation rows named by a table (the fused gate/up kernel reading the tokens where they lie, instead of a copy
-    // sorted by expert): per-lane offsets then count from the first row of the matrix
-    const bool a_indirect = MODE == kContigListAct && p.a_rows != nullptr;
-    const bool ahead = AHEAD && !sliced && p.c_lds && nk >= STAGES && vb + static_cast<int>(gridDim.x) < units;
-    const uint8_t* a_tile = p.a + static_cast<int64_t>(a_indirect ? 0 : m0) * p.K + static_cast<int64_t>(kb_first) * kScaleBlock;
+    const uint8_t* a_tile = p.a + static_cast<int64_t>(m0) * p.K + static_cast<int64_t>(kb_first) * kScaleBlock;
     const float* as_tile = p.a_s + static_cast<int64_t>(m0) * p.as_sm + static_cast<int64_t>(kb_first) * p.as_sk;
     char* c_base = static_cast<char*>(p.c);
-    if (kMaskedLike) {
+    if (MODE == kMasked) {
       a_tile += static_cast<int64_t>(g) * p.a_gs;
       as_tile += static_cast<int64_t>(g) * p.as_gs;
       c_base += static_cast<int64_t>(g) * p.c_gs * esz;
     }
-    const uint8_t* b_tile = p.b + static_cast<int64_t>(g) * p.b_gs + static_cast<int64_t>(kAct ? 0 : n0) * p.K +
+    const uint8_t* b_tile = p.b + static_cast<int64_t>(g) * p.b_gs + static_cast<int64_t>(n0) * p.K +
                             static_cast<int64_t>(kb_first) * kScaleBlock;
-    // weight scales: lane i of the wave fetches the scale of the wave's fragment (i & 3) (fragment 0 beyond NF)
+    // the wave's weight scale, fetched by every lane
     const float* bs_g = p.b_s + static_cast<int64_t>(g) * p.bs_gs + kb_first;
-    const int bs_frag = (lane & 3) < NF ? (lane & 3) : 0;
-    uint32_t bs_off =
-        static_cast<uint32_t>(min((kAct ? w_row(wn0 + 32 * bs_frag) : n0 + wn0 + 32 * bs_frag) / kScaleBlock, p.nblocks - 1)) *
-        static_cast<uint32_t>(p.kblocks) * 4u;
+    const uint32_t bs_off = static_cast<uint32_t>(min((n0 + wn0) / kScaleBlock, p.nblocks - 1)) * static_cast<uint32_t>(p.kblocks) * 4u;
 
     // DMA addressing.  Instruction j of this wave fills LDS rows 8 (j WAVES + wave) .. + 7; lane i fills physical
     // chunk (i & 7) of row (i >> 3), which holds logical chunk (i & 7) ^ swizzle(row).  WAVES is even, so the
@@ -335,7 +280,7 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
     // recomputed per instruction (two VALU ops) instead of being kept in registers.  Rows past the valid range
     // re-read the last valid row.
     static_assert(WAVES % 2 == 0, "chunk swizzle must not depend on the DMA instruction index");
-    int a_last = m_end - 1 - m0;
+    const int a_last = m_end - 1 - m0;
     const int b_last = p.N - 1 - n0;
     const int dma_row = 8 * wave + (lane >> 3);
     const uint32_t dma_chunk = static_cast<uint32_t>(((lane & 7) ^ chunk_swizzle(dma_row)) * 16);
@@ -348,44 +293,14 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
 #pragma unroll
     for (int j = 0; j < Cfg::A_INST; ++j) {
       const int r = min(dma_row + 8 * j * WAVES, a_last);
-      a_off[j] = static_cast<uint32_t>(a_indirect ? max(p.a_rows[m0 + r], 0) : r) * uK + dma_chunk;
+      a_off[j] = static_cast<uint32_t>(r) * uK + dma_chunk;
     }
 #pragma unroll
     for (int j = 0; j < Cfg::B_INST; ++j)
-      b_off[j] = static_cast<uint32_t>(kAct ? w_row(dma_row + 8 * j * WAVES) : min(dma_row + 8 * j * WAVES, b_last)) * uK + dma_chunk;
+      b_off[j] = static_cast<uint32_t>(min(dma_row + 8 * j * WAVES, b_last)) * uK + dma_chunk;
 #pragma unroll
     for (int j = 0; j < Cfg::S_INST; ++j)
       s_off[j] = static_cast<uint32_t>(min((j * WAVES + wave) * 64 + lane, a_last)) * static_cast<uint32_t>(p.as_sm) * 4u;
-
-    // AHEAD: from here on the DMA addresses (of the activations / of all else) are those of the workgroup's next tile, or of
-    // this tile again without one.  Computed from the lane index alone, so that nothing is kept for it across the K loop.
-    auto point_ahead = [&](auto which) __attribute__((always_inline)) {
-      constexpr bool kActs = decltype(which)::value;
-      int tile, slice, tm, tn;
-      locate(ahead ? vb + static_cast<int>(gridDim.x) : vb, tile, slice, tm, tn);
-      const int m1 = __builtin_amdgcn_readfirstlane(tm * BM), n1 = __builtin_amdgcn_readfirstlane(n_base + tn * BN);
-      int nl = lane;
-      asm volatile("" : "+v"(nl));
-      const int row = 8 * wave + (nl >> 3);
-      const uint32_t chunk = static_cast<uint32_t>(((nl & 7) ^ chunk_swizzle(row)) * 16);
-      const int m_last = p.M - 1 - m1, n_last = p.N - 1 - n1;
-      if constexpr (kActs) {
-        a_tile = p.a + static_cast<int64_t>(m1) * p.K;
-#pragma unroll
-        for (int j = 0; j < Cfg::A_INST; ++j) a_off[j] = static_cast<uint32_t>(min(row + 8 * j * WAVES, m_last)) * uK + chunk;
-      } else {
-        as_tile = p.a_s + static_cast<int64_t>(m1) * p.as_sm;
-        b_tile = p.b + static_cast<int64_t>(n1) * p.K;
-        const int frag = (nl & 3) < NF ? (nl & 3) : 0;
-        bs_off = static_cast<uint32_t>(min((n1 + wn0 + 32 * frag) / kScaleBlock, p.nblocks - 1)) * static_cast<uint32_t>(p.kblocks) * 4u;
-        a_last = m_last;
-#pragma unroll
-        for (int j = 0; j < Cfg::B_INST; ++j) b_off[j] = static_cast<uint32_t>(min(row + 8 * j * WAVES, n_last)) * uK + chunk;
-#pragma unroll
-        for (int j = 0; j < Cfg::S_INST; ++j)
-          s_off[j] = static_cast<uint32_t>(min((j * WAVES + wave) * 64 + nl, m_last)) * static_cast<uint32_t>(p.as_sm) * 4u;
-      }
-    };
 
     auto issue_stage = [&](int kb, int stage) {
       uint8_t* sbase = smem + stage * Cfg::STAGE_BYTES;
@@ -412,38 +327,9 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
         asm volatile("" : "+v"(o));
         dma_4(sg, o, sbase + Cfg::A_BYTES + Cfg::B_BYTES + (j * WAVES + wave) * 256);
       }
-      // weight scales of the wave's fragments at this K block, one per lane slot
+      // weight scale of the wave's columns at this K block
       dma_4(reinterpret_cast<const uint8_t*>(bs_g + kb), bs_off,
             sbase + Cfg::A_BYTES + Cfg::B_BYTES + Cfg::S_BYTES + wave * 256);
-    };
-    // The same group, one instruction at a time (i = 0 .. LOADS_PER_STAGE - 1, compile-time): the in-place K loop
-    // spreads a stage's DMA over several tile slots instead of issuing it in one burst behind the barrier, where
-    // the eight waves' 80 instructions queue up in front of the texture path and keep the waves from their MFMAs.
-    auto issue_one = [&](auto idx, int kb, int stage) __attribute__((always_inline)) {
-      constexpr int i = decltype(idx)::value;
-      uint8_t* sbase = smem + stage * Cfg::STAGE_BYTES;
-      if constexpr (i < Cfg::A_INST) {
-#ifdef DLB_ABLATE_A
-        return;
-#endif
-        uint32_t o = a_off[i];
-        asm volatile("" : "+v"(o));
-        dma_16(a_tile + static_cast<int64_t>(kb) * kScaleBlock, o, sbase + (i * WAVES + wave) * 1024);
-      } else if constexpr (i < Cfg::A_INST + Cfg::B_INST) {
-        constexpr int j = i - Cfg::A_INST;
-        uint32_t o = b_off[j];
-        asm volatile("" : "+v"(o));
-        dma_16<kWeightPolicy>(b_tile + static_cast<int64_t>(kb) * kScaleBlock, o, sbase + Cfg::A_BYTES + (j * WAVES + wave) * 1024);
-      } else if constexpr (i < Cfg::A_INST + Cfg::B_INST + Cfg::S_INST) {
-        constexpr int j = i - Cfg::A_INST - Cfg::B_INST;
-        uint32_t o = s_off[j];
-        asm volatile("" : "+v"(o));
-        dma_4(reinterpret_cast<const uint8_t*>(as_tile + static_cast<int64_t>(kb) * p.as_sk), o,
-              sbase + Cfg::A_BYTES + Cfg::B_BYTES + (j * WAVES + wave) * 256);
-      } else {
-        dma_4(reinterpret_cast<const uint8_t*>(bs_g + kb), bs_off,
-              sbase + Cfg::A_BYTES + Cfg::B_BYTES + Cfg::S_BYTES + wave * 256);
-      }
     };
 
     v16f acc[MF][NF];
@@ -455,20 +341,8 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
         for (int t = 0; t < 16; ++t) acc[mi][ni][t] = 0.f;
 
     // ---- K loop ---------------------------------------------------------------------------------------------
-    // One operand's fragments are held in registers for the whole K step ("held": the one with fewer fragments),
-    // the other's are streamed past them one fragment at a time.  Tiles are visited streamed-major.  Registers
-    // are reloaded in place as soon as the last MFMA that reads them has been issued, and the single barrier of a
-    // K step sits before the tiles of the LAST streamed fragment: by then every LDS read of the current stage
-    // has returned, so the stage can be handed to the DMA, and the first fragments of the next stage are fetched
-    // while those last tiles run on the matrix pipe.  The step body is branch-free (the last steps are peeled
-    // through template flags) so that the scheduling fences inside it hold.
-    constexpr bool kHoldX = MF <= NF;          // hold activations (x), stream weights (w); else the reverse
-    constexpr int H = kHoldX ? MF : NF;        // held fragments
-    constexpr int S = kHoldX ? NF : MF;        // streamed fragments
-    constexpr int T = H * S;
+    constexpr int T = MF * NF;
     constexpr int kFragBytes = 32 * kScaleBlock;
-    const int held0 = (kHoldX ? wm0 : Cfg::BM + wn0) * kScaleBlock;      // byte offset of held fragment 0 in a stage
-    const int strm0 = (kHoldX ? Cfg::BM + wn0 : wm0) * kScaleBlock;
     constexpr int kScaleOff = Cfg::A_BYTES + Cfg::B_BYTES;
     constexpr int kWScaleOff = kScaleOff + Cfg::S_BYTES;
 
@@ -490,406 +364,116 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
               (r * static_cast<uint32_t>(p.as_sm) + j * static_cast<uint32_t>(p.as_sk)) * 4u, smem + Cfg::SCTAB_OFF + i * 256);
       }
     };
-    // kExactK: only K blocks that exist are fetched - a tile shorter than the ring, and the last STAGES steps of every
-    // tile, issue nothing (wave-uniform branches), so no load is in flight when the tile ends and the next tile starts
-    // without waiting for loads nobody reads.  The kernels whose wave tile fills the register file (64 x 128) cannot
-    // afford those branches' scalar registers inside the K loop (wave tiles above 64 x 64): they keep every step the same code, fetch the last
-    // block again past the end of K into a stage nobody reads, and drain at the end of the tile.
-    constexpr bool kExactK = MF * NF <= 4;
-    // DMA slots of a K step: the group that refills the step's stage starts at the barrier slot kP and is spread over kSlots
-    // tile slots, wrapping into the next step (whose slots t < kP therefore finish the PREVIOUS step's group)
-    constexpr int kP = (S - 1) * H;
-    constexpr int kSlots = T >= 8 ? 5 : (T >= 4 ? 3 : 1);  // measured: 3 to 5 of 8 slots are equally good, 6 and 7 leave the loads too little time
-    constexpr int L = Cfg::LOADS_PER_STAGE;
-    // The first H slots' part of a group is issued by its own step, the rest by the next one.  AHEAD: that part is the
-    // activations, all of them and nothing else, and all that the prologue issues of its last group.
-    constexpr auto part_begin = [](int q) {
-      return AHEAD ? (q <= H ? q * Cfg::A_INST / H : Cfg::A_INST + (q - H) * (L - Cfg::A_INST) / (kSlots > H ? kSlots - H : 1)) : q * L / kSlots;
-    };
-    constexpr int kFirstPart = !AHEAD ? L : part_begin(H < kSlots ? H : kSlots);
-    auto issue_first_part = [&](int kb, int stg) __attribute__((always_inline)) {
-      each_index([&](auto i) __attribute__((always_inline)) { issue_one(i, kb, stg); }, std::make_integer_sequence<int, kFirstPart>{});
-    };
-    if (!AHEAD) stage = 0;
-    if (AHEAD && staged) {
-      lds_barrier();  // the previous tile's results have been read from the ring, the scale table has landed
-    } else {
-      __syncthreads();  // the previous tile's readers and DMA groups are done with the ring
-      if constexpr (Cfg::SCTAB) issue_table();
+    int stage = 0;
+    __syncthreads();  // the previous tile's readers are done with the ring
+    if constexpr (Cfg::SCTAB) issue_table();
 #pragma unroll
-      for (int s = 0; s < STAGES; ++s) {
-        if (kExactK && s >= nk) continue;
-        const int stg = AHEAD ? (stage + s) % STAGES : s;
-        if (s < STAGES - 1)
-          issue_stage(min(s, nk - 1), stg);
-        else
-          issue_first_part(min(s, nk - 1), stg);
-      }
-      if (!kExactK || nk >= STAGES)
-        wait_vmcnt<(STAGES - 2) * L + kFirstPart>();  // all but the first stage's group may still be on their way
-      else
-        wait_vmcnt<0>();
-      lds_barrier();
-    }
-    staged = ahead;
-    const int base0 = AHEAD ? stage * Cfg::STAGE_BYTES : 0;
+    for (int s = 0; s < STAGES; ++s)
+      if (s < nk) issue_stage(s, s);
+    // all but the first stage's group may still be on their way
+    if (nk >= STAGES)
+      wait_vmcnt<(STAGES - 1) * Cfg::LOADS_PER_STAGE>();
+    else
+      wait_vmcnt<0>();
+    lds_barrier();
 
     // first table entry of this lane's rows (scale-table kernels)
     int tab_row[MF];
 #pragma unroll
     for (int mi = 0; mi < MF; ++mi) tab_row[mi] = Cfg::SCTAB ? (wm0 + mi * 32 + l32) * p.sct_pitch : 0;
 
-    if constexpr (Cfg::PREFETCH) {
-      static_assert(kUniformW, "the register-double-buffered path assumes one weight scale per wave");
-      // ---- full register double buffering (one wave per SIMD) ------------------------------------------------
-      v8i xr[2][MF][2];
-      v8i wr[2][NF][2];
-      float scb[2][MF];
-      float sc_last = 0.f;
-      v16f part[2];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) part[0][u] = part[1][u] = 0.f;
-      const int x0 = wm0 * kScaleBlock;
-      const int w0 = (Cfg::BM + wn0) * kScaleBlock;
-      auto load_scales = [&](int base, int kbl, float (&dst)[MF]) {
-        const float sb = *reinterpret_cast<const float*>(smem + base + kWScaleOff + wave * 256);
-        if constexpr (Cfg::SCTAB) {
-          const float* tab = reinterpret_cast<const float*>(smem + Cfg::SCTAB_OFF);
-#pragma unroll
-          for (int mi = 0; mi < MF; ++mi) dst[mi] = tab[tab_row[mi] + kbl] * sb;
-        } else {
-          const float* sS = reinterpret_cast<const float*>(smem + base + kScaleOff);
-#pragma unroll
-          for (int mi = 0; mi < MF; ++mi) dst[mi] = sS[wm0 + mi * 32 + l32] * sb;
-        }
-      };
-      // half-fragment q of a stage: q < 2 MF -> activation fragment q / 2, K half q % 2; else weight fragment
-      constexpr int kHalves = 2 * (MF + NF);
-      constexpr int kPerTile = (kHalves + (MF * NF) - 2) / (MF * NF - 1);  // spread over the first T - 1 tiles
-      load_scales(0, 0, scb[0]);
-#pragma unroll
-      for (int mi = 0; mi < MF; ++mi) {
-        xr[0][mi][0] = lds_read_frag32(smem, x0 + mi * kFragBytes, lc, 0);
-        xr[0][mi][1] = lds_read_frag32(smem, x0 + mi * kFragBytes, lc, 1);
-      }
-#pragma unroll
-      for (int ni = 0; ni < NF; ++ni) {
-        wr[0][ni][0] = lds_read_frag32(smem, w0 + ni * kFragBytes, lc, 0);
-        wr[0][ni][1] = lds_read_frag32(smem, w0 + ni * kFragBytes, lc, 1);
-      }
-
-      // Every step is the same code: a step always prefetches "the next stage" into registers (garbage after the
-      // last one, never used); whether it hands its stage to the DMA and how many groups it leaves in flight at its
-      // barrier are wave-uniform branches on the step's distance from the end of K.
-      auto k_step = [&](auto buf_tag, int kb, int stage) __attribute__((always_inline)) {
-        constexpr int B = decltype(buf_tag)::value;
-        const int next_stage = stage + 1 == STAGES ? 0 : stage + 1;
-        const int nxt_base = next_stage * Cfg::STAGE_BYTES;
-        // every wave holds this stage's fragments in registers and has its share of the next stage in LDS
-        // the group of step kb + 1 has landed: behind it at most STAGES - 2 younger groups are out, fewer at the tile's end
-        if (kExactK && kb + STAGES > nk)
-          wait_vmcnt<0>();
-        else
-          wait_vmcnt<(STAGES - 2) * Cfg::LOADS_PER_STAGE>();
-        lds_barrier();
-        if (!kExactK || kb + STAGES < nk) issue_stage(min(kb + STAGES, nk - 1), stage);
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-          const int mi = t / NF, ni = t % NF;
-          __builtin_amdgcn_sched_barrier(0);
-          v16f z;
-#pragma unroll
-          for (int u = 0; u < 16; ++u) z[u] = 0.f;
-          z = mfma_32x32x64_e4m3(wr[B][ni][0], xr[B][mi][0], z);
-          part[t & 1] = mfma_32x32x64_e4m3(wr[B][ni][1], xr[B][mi][1], z);
-          __builtin_amdgcn_sched_barrier(0);
-          if (t == 0) load_scales(nxt_base, min(kb + 1, nk - 1), scb[B ^ 1]);
-#pragma unroll
-          for (int q = t * kPerTile; q < (t + 1) * kPerTile && q < kHalves; ++q) {
-            if (q < 2 * MF)
-              xr[B ^ 1][q / 2][q % 2] = lds_read_frag32(smem, nxt_base + x0 + (q / 2) * kFragBytes, lc, q % 2);
-            else
-              wr[B ^ 1][(q - 2 * MF) / 2][q % 2] =
-                  lds_read_frag32(smem, nxt_base + w0 + ((q - 2 * MF) / 2) * kFragBytes, lc, q % 2);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-          if (t == 0)
-            acc[MF - 1][NF - 1] += part[(T - 1) & 1] * sc_last;  // last tile of the previous K step
-          else
-            acc[(t - 1) / NF][(t - 1) % NF] += part[(t - 1) & 1] * scb[B][(t - 1) / NF];
-        }
-        sc_last = scb[B][MF - 1];
-      };
-      typedef std::integral_constant<int, 0> B0;
-      typedef std::integral_constant<int, 1> B1;
-      int kb = 0;
-      for (; kb + 1 < nk; kb += 2) {
-        k_step(B0{}, kb, stage);
-        stage = stage + 1 == STAGES ? 0 : stage + 1;
-        k_step(B1{}, kb + 1, stage);
-        stage = stage + 1 == STAGES ? 0 : stage + 1;
-      }
-      if (kb < nk) k_step(B0{}, kb, stage);
-      acc[MF - 1][NF - 1] += part[(T - 1) & 1] * sc_last;
-      if (!kExactK) wait_vmcnt<0>();  // the trailing re-read groups must not land in the next tile's ring
-    } else {
-    v8i hf[H][2];
-    v8i sf[2];
-    float sc[MF][NS];
+    v8i xr[2][MF][2];
+    v8i wr[2][NF][2];
+    float scb[2][MF];
     float sc_last = 0.f;
     v16f part[2];
 #pragma unroll
     for (int u = 0; u < 16; ++u) part[0][u] = part[1][u] = 0.f;
-
-    auto load_scales = [&](int base, int kbl, float (&dst)[MF][NS]) {
-      float sb[NS];
+    const int x0 = wm0 * kScaleBlock;
+    const int w0 = (Cfg::BM + wn0) * kScaleBlock;
+    auto load_scales = [&](int base, int kbl, float (&dst)[MF]) {
+      const float sb = *reinterpret_cast<const float*>(smem + base + kWScaleOff + wave * 256);
+      if constexpr (Cfg::SCTAB) {
+        const float* tab = reinterpret_cast<const float*>(smem + Cfg::SCTAB_OFF);
 #pragma unroll
-      for (int j = 0; j < NS; ++j) sb[j] = *reinterpret_cast<const float*>(smem + base + kWScaleOff + wave * 256 + j * 4);
-      const float* sS = reinterpret_cast<const float*>(smem + base + kScaleOff);
-      const float* tab = reinterpret_cast<const float*>(smem + Cfg::SCTAB_OFF);
+        for (int mi = 0; mi < MF; ++mi) dst[mi] = tab[tab_row[mi] + kbl] * sb;
+      } else {
+        const float* sS = reinterpret_cast<const float*>(smem + base + kScaleOff);
 #pragma unroll
-      for (int mi = 0; mi < MF; ++mi) {
-        const float sa = Cfg::SCTAB ? tab[tab_row[mi] + kbl] : sS[wm0 + mi * 32 + l32];
-#pragma unroll
-        for (int j = 0; j < NS; ++j) dst[mi][j] = sa * sb[j];
+        for (int mi = 0; mi < MF; ++mi) dst[mi] = sS[wm0 + mi * 32 + l32] * sb;
       }
     };
-    load_scales(base0, 0, sc);
+    // half-fragment q of a stage: q < 2 MF -> activation fragment q / 2, K half q % 2; else weight fragment
+    constexpr int kHalves = 2 * (MF + NF);
+    constexpr int kPerTile = (kHalves + (MF * NF) - 2) / (MF * NF - 1);  // spread over the first T - 1 tiles
+    load_scales(0, 0, scb[0]);
 #pragma unroll
-    for (int hi = 0; hi < H; ++hi) {
-      hf[hi][0] = lds_read_frag32(smem, base0 + held0 + hi * kFragBytes, lc, 0);
-      hf[hi][1] = lds_read_frag32(smem, base0 + held0 + hi * kFragBytes, lc, 1);
+    for (int mi = 0; mi < MF; ++mi) {
+      xr[0][mi][0] = lds_read_frag32(smem, x0 + mi * kFragBytes, lc, 0);
+      xr[0][mi][1] = lds_read_frag32(smem, x0 + mi * kFragBytes, lc, 1);
     }
-    sf[0] = lds_read_frag32(smem, base0 + strm0, lc, 0);
-    sf[1] = lds_read_frag32(smem, base0 + strm0, lc, 1);
+#pragma unroll
+    for (int ni = 0; ni < NF; ++ni) {
+      wr[0][ni][0] = lds_read_frag32(smem, w0 + ni * kFragBytes, lc, 0);
+      wr[0][ni][1] = lds_read_frag32(smem, w0 + ni * kFragBytes, lc, 1);
+    }
 
-    // One K step; every step is the same code (see the note in the register-double-buffered path above).
-    auto k_step = [&](int kb, int stage) __attribute__((always_inline)) {
+    // Every step is the same code: a step always prefetches "the next stage" into registers (garbage after the
+    // last one, never used); whether it hands its stage to the DMA and how many groups it leaves in flight at its
+    // barrier are wave-uniform branches on the step's distance from the end of K.
+    auto k_step = [&](auto buf_tag, int kb, int stage) __attribute__((always_inline)) {
+      constexpr int B = decltype(buf_tag)::value;
       const int next_stage = stage + 1 == STAGES ? 0 : stage + 1;
-      const int cur_base = stage * Cfg::STAGE_BYTES;
       const int nxt_base = next_stage * Cfg::STAGE_BYTES;
-      float sc_next[MF][NS];
-      const int prev_stage = stage == 0 ? STAGES - 1 : stage - 1;
-      // past the end of K: the next tile's first blocks (AHEAD), nothing (kExactK), or the last block again
-      auto block = [&](int k) { return AHEAD ? (k < nk ? k : min(k - nk, nk - 1)) : kExactK ? k : min(k, nk - 1); };
-      const int kb_new = block(kb + STAGES), kb_prev = block(kb + STAGES - 1);
-      const bool do_new = !kExactK || ahead || kb + STAGES < nk, do_prev = !kExactK || ahead || kb + STAGES - 1 < nk;
-      auto issue_slot = [&](auto qtag, int kbx, int stg) __attribute__((always_inline)) {
-        constexpr int q = decltype(qtag)::value;
-        constexpr int i0 = part_begin(q), i1 = part_begin(q + 1);
-        if constexpr (i0 + 0 < i1) issue_one(std::integral_constant<int, i0 + 0>{}, kbx, stg);
-        if constexpr (i0 + 1 < i1) issue_one(std::integral_constant<int, i0 + 1>{}, kbx, stg);
-        if constexpr (i0 + 2 < i1) issue_one(std::integral_constant<int, i0 + 2>{}, kbx, stg);
-        if constexpr (i0 + 3 < i1) issue_one(std::integral_constant<int, i0 + 3>{}, kbx, stg);
-        if constexpr (i0 + 4 < i1) issue_one(std::integral_constant<int, i0 + 4>{}, kbx, stg);
-        if constexpr (i0 + 5 < i1) issue_one(std::integral_constant<int, i0 + 5>{}, kbx, stg);
-        static_assert(i1 - i0 <= 6, "at most six DMA instructions per slot");
-      };
+      // every wave holds this stage's fragments in registers and has its share of the next stage in LDS
+      // the group of step kb + 1 has landed: behind it at most STAGES - 2 younger groups are out, fewer at the tile's end
+      if (kb + STAGES > nk)
+        wait_vmcnt<0>();
+      else
+        wait_vmcnt<(STAGES - 2) * Cfg::LOADS_PER_STAGE>();
+      lds_barrier();
+      if (kb + STAGES < nk) issue_stage(kb + STAGES, stage);
 #pragma unroll
       for (int t = 0; t < T; ++t) {
-        const int si = t / H, hi = t % H;
-        if (si == S - 1 && hi == 0) {
-          // every LDS read of this stage has been issued and the barrier waits for their return: hand it over
-          // (DLB_ABLATE_*: measurement builds with one part of the K step compiled out - their results are wrong on
-          // purpose; what a launch gains by it is what that part costs.  Never defined in the library build.)
-#ifndef DLB_ABLATE_VMCNT
-          // the group of step kb + 1 has landed: behind it at most STAGES - 2 younger groups are out, fewer at the tile's end
-          if (kExactK && !ahead && kb + STAGES > nk)
-            wait_vmcnt<0>();
-          else
-            wait_vmcnt<(STAGES - 2) * Cfg::LOADS_PER_STAGE>();
-#endif
-#ifndef DLB_ABLATE_BARRIER
-          lds_barrier();
-#else
-          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#endif
-        }
-#ifndef DLB_ABLATE_DMA
-        if (t >= kP) {
-          if (t - kP < kSlots && do_new) {
-            if (t - kP == 0) issue_slot(std::integral_constant<int, 0>{}, kb_new, stage);
-            if (t - kP == 1) issue_slot(std::integral_constant<int, 1>{}, kb_new, stage);
-            if (t - kP == 2) issue_slot(std::integral_constant<int, 2>{}, kb_new, stage);
-            if (t - kP == 3) issue_slot(std::integral_constant<int, 3>{}, kb_new, stage);
-            if (t - kP == 4) issue_slot(std::integral_constant<int, 4>{}, kb_new, stage);
-          }
-        } else if (t + T - kP < kSlots && do_prev) {
-          if (t + T - kP == 1) issue_slot(std::integral_constant<int, 1>{}, kb_prev, prev_stage);
-          if (t + T - kP == 2) issue_slot(std::integral_constant<int, 2>{}, kb_prev, prev_stage);
-          if (t + T - kP == 3) issue_slot(std::integral_constant<int, 3>{}, kb_prev, prev_stage);
-          if (t + T - kP == 4) issue_slot(std::integral_constant<int, 4>{}, kb_prev, prev_stage);
-        }
-#endif
-        // The scheduling fences pin the order MFMA pair -> reloads -> scale FMAs; without them the compiler
-        // hoists the reloads above the MFMAs into fresh registers and the kernel spills.
+        const int mi = t / NF, ni = t % NF;
         __builtin_amdgcn_sched_barrier(0);
         v16f z;
 #pragma unroll
         for (int u = 0; u < 16; ++u) z[u] = 0.f;
-        constexpr int kSlot = Cfg::PARTS == 2 ? 1 : 0;
-#ifdef DLB_ABLATE_MFMADEP
-        if (kHoldX) {  // the two MFMAs of a tile independent of each other (the first one's product is dropped)
-          v16f z2;
+        z = mfma_32x32x64_e4m3(wr[B][ni][0], xr[B][mi][0], z);
+        part[t & 1] = mfma_32x32x64_e4m3(wr[B][ni][1], xr[B][mi][1], z);
+        __builtin_amdgcn_sched_barrier(0);
+        if (t == 0) load_scales(nxt_base, min(kb + 1, nk - 1), scb[B ^ 1]);
 #pragma unroll
-          for (int u = 0; u < 16; ++u) z2[u] = 0.f;
-          z = mfma_32x32x64_e4m3(sf[0], hf[hi][0], z);
-          part[t & kSlot] = mfma_32x32x64_e4m3(sf[1], hf[hi][1], z2);
-          asm volatile("" ::"v"(z));
-        } else
-#endif
-        if (kHoldX) {
-          z = mfma_32x32x64_e4m3(sf[0], hf[hi][0], z);
-          part[t & kSlot] = mfma_32x32x64_e4m3(sf[1], hf[hi][1], z);
-        } else {
-          z = mfma_32x32x64_e4m3(hf[hi][0], sf[0], z);
-          part[t & kSlot] = mfma_32x32x64_e4m3(hf[hi][1], sf[1], z);
+        for (int q = t * kPerTile; q < (t + 1) * kPerTile && q < kHalves; ++q) {
+          if (q < 2 * MF)
+            xr[B ^ 1][q / 2][q % 2] = lds_read_frag32(smem, nxt_base + x0 + (q / 2) * kFragBytes, lc, q % 2);
+          else
+            wr[B ^ 1][(q - 2 * MF) / 2][q % 2] =
+                lds_read_frag32(smem, nxt_base + w0 + ((q - 2 * MF) / 2) * kFragBytes, lc, q % 2);
         }
         __builtin_amdgcn_sched_barrier(0);
-        // in-place reloads: the MFMAs above were the last readers of these registers
-#ifndef DLB_ABLATE_LDSREAD
-        if (hi == H - 1 && si + 1 < S) {
-          sf[0] = lds_read_frag32(smem, cur_base + strm0 + (si + 1) * kFragBytes, lc, 0);
-          sf[1] = lds_read_frag32(smem, cur_base + strm0 + (si + 1) * kFragBytes, lc, 1);
-        }
-        if (si == S - 1) {
-#ifndef DLB_ABLATE_A
-          hf[hi][0] = lds_read_frag32(smem, nxt_base + held0 + hi * kFragBytes, lc, 0);
-          hf[hi][1] = lds_read_frag32(smem, nxt_base + held0 + hi * kFragBytes, lc, 1);
-#else
-          asm volatile("" : "+v"(hf[hi][0]), "+v"(hf[hi][1]));
-#endif
-          if (hi == 0) load_scales(nxt_base, min(kb + 1, nk - 1), sc_next);
-          if (hi == H - 1) {
-            sf[0] = lds_read_frag32(smem, nxt_base + strm0, lc, 0);
-            sf[1] = lds_read_frag32(smem, nxt_base + strm0, lc, 1);
-          }
-        }
-#else
-        if (si == S - 1 && hi == 0) load_scales(nxt_base, min(kb + 1, nk - 1), sc_next);
-        asm volatile("" : "+v"(sf[0]), "+v"(sf[1]), "+v"(hf[hi][0]), "+v"(hf[hi][1]));  // the operands change for all the compiler knows
-#endif
-        __builtin_amdgcn_sched_barrier(0);
-#ifdef DLB_ABLATE_SCALE
-        {  // one of the 16 scale FMAs of a tile, so that its MFMAs stay
-          const int mi = kHoldX ? hi : si, ni = kHoldX ? si : hi;
-          acc[mi][ni][0] += part[t & kSlot][0] * sc[mi][kUniformW ? 0 : ni];
-        }
-#else
-        if (Cfg::PARTS == 1) {
-          // scale-and-accumulate this tile; the other wave of the SIMD owns the matrix pipe meanwhile
-          const int mi = kHoldX ? hi : si, ni = kHoldX ? si : hi;
-          acc[mi][ni] += part[0] * sc[mi][kUniformW ? 0 : ni];
-        } else if (t == 0) {
-          // scale-and-accumulate the previous tile while this tile's MFMAs run
-          acc[MF - 1][NF - 1] += part[(T - 1) & 1] * sc_last;  // last tile of the previous K step (zero at kb = 0)
-        } else {
-          const int pt = t - 1;
-          const int pmi = kHoldX ? pt % H : pt / H, pni = kHoldX ? pt / H : pt % H;
-          acc[pmi][pni] += part[pt & 1] * sc[pmi][kUniformW ? 0 : pni];
-        }
-#endif
+        if (t == 0)
+          acc[MF - 1][NF - 1] += part[(T - 1) & 1] * sc_last;  // last tile of the previous K step
+        else
+          acc[(t - 1) / NF][(t - 1) % NF] += part[(t - 1) & 1] * scb[B][(t - 1) / NF];
       }
-      sc_last = sc[MF - 1][NS - 1];
-#pragma unroll
-      for (int m2 = 0; m2 < MF; ++m2)
-#pragma unroll
-        for (int j = 0; j < NS; ++j) sc[m2][j] = sc_next[m2][j];
+      sc_last = scb[B][MF - 1];
     };
-    for (int kb = 0; kb < nk; ++kb) {
-      if (AHEAD && (ahead || !kExactK)) {
-        if (kb == max(nk - STAGES, 0)) point_ahead(std::true_type{});
-        if (kb == max(nk - STAGES + 1, 0)) point_ahead(std::false_type{});
-      }
-      k_step(kb, stage);
+    typedef std::integral_constant<int, 0> B0;
+    typedef std::integral_constant<int, 1> B1;
+    int kb = 0;
+    for (; kb + 1 < nk; kb += 2) {
+      k_step(B0{}, kb, stage);
+      stage = stage + 1 == STAGES ? 0 : stage + 1;
+      k_step(B1{}, kb + 1, stage);
       stage = stage + 1 == STAGES ? 0 : stage + 1;
     }
-    if (Cfg::PARTS == 2) acc[MF - 1][NF - 1] += part[(T - 1) & 1] * sc_last;
-    if (AHEAD && Cfg::SCTAB && ahead) issue_table();  // every wave has read the scales of the last K block
-    if (!kExactK && !ahead) wait_vmcnt<0>();  // the trailing re-read groups must not land in the next tile's ring
-    }
+    if (kb < nk) k_step(B0{}, kb, stage);
+    acc[MF - 1][NF - 1] += part[(T - 1) & 1] * sc_last;
 
     // epilogue: lane holds c[m0 + wm0 + 32 mi + (lane & 31)][n0 + wn0 + 32 ni + 8 u + 4 (lane >> 5) + 0..3], u = 0..3
-    // (the lane index passes through an empty asm: what is computed from it then stays behind the K loop instead of
-    // taking registers across it: the 256-row kernels spilled 19 to 49 of them.  One wave per SIMD has them to spare.)
-    int el = lane;
-    if (!Cfg::PREFETCH) asm volatile("" : "+v"(el));
-    const int el32 = el & 31, eh = el >> 5;
-    if constexpr (kAct) {
-      // The tile goes to LDS as the bf16 matrix the unfused GEMM would have written ([BM][gate 128 | up 128], 8-byte
-      // chunks XOR-ed with an even function of the row so that the 32 rows of a store instruction spread over the
-      // banks and 16-byte reads stay whole), then 16 lanes per row compute silu(gate) * up rounded to bf16 and quantise
-      // the 128 values exactly as silu_and_mul + per_token_group_quant_fp8 do (moe_activation.h, fp8_quant.h).
-      constexpr int kRowB = BN * 2;
-      static_assert(BM * kRowB <= Cfg::LDS_BYTES, "the staged tile fits in the ring");
-      __syncthreads();  // every wave is done reading the ring
-#pragma unroll
-      for (int mi = 0; mi < MF; ++mi) {
-        const int row = wm0 + mi * 32 + el32;
-        const int x = (row & 31) << 1;
-#pragma unroll
-        for (int ni = 0; ni < NF; ++ni)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const v4f v = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
-            const int chunk = (wn0 + ni * 32 + u * 8 + eh * 4) >> 2;
-            *reinterpret_cast<v4bf*>(smem + row * kRowB + ((chunk ^ x) << 3)) = __builtin_convertvector(v, v4bf);
-          }
-      }
-      __syncthreads();
-      const int et = wave * 64 + el;
-      const int sub = et & 15;
-      uint8_t* q_out = static_cast<uint8_t*>(p.c);
-      float* s_out = p.act_s;
-      if (kMaskedLike) {
-        q_out += static_cast<int64_t>(g) * p.M * p.act_q_stride;
-        s_out += static_cast<int64_t>(g) * p.act_s_gs;
-      }
-#pragma unroll 2
-      for (int r0 = 0; r0 < BM; r0 += Cfg::NT / 16) {
-        const int row = r0 + (et >> 4);
-        const int x = (row & 31) << 1;
-        const v4i graw = *reinterpret_cast<const v4i*>(smem + row * kRowB + (((2 * sub) ^ x) << 3));
-        const v4i uraw = *reinterpret_cast<const v4i*>(smem + row * kRowB + (((BN / 4 / 2 + 2 * sub) ^ x) << 3));
-        float v[8];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t gw = static_cast<uint32_t>(graw[i]), uw = static_cast<uint32_t>(uraw[i]);
-          const float g0 = __builtin_bit_cast(float, gw << 16), g1 = __builtin_bit_cast(float, gw & 0xffff0000u);
-          const float u0 = __builtin_bit_cast(float, uw << 16), u1 = __builtin_bit_cast(float, uw & 0xffff0000u);
-          if (kMaskedLike) {  // the masked activation rounds silu(gate) before the product (moe.py:256-257)
-            v[2 * i] = static_cast<float>(static_cast<__bf16>(u0 * static_cast<float>(static_cast<__bf16>(act_silu_f32(g0)))));
-            v[2 * i + 1] = static_cast<float>(static_cast<__bf16>(u1 * static_cast<float>(static_cast<__bf16>(act_silu_f32(g1)))));
-          } else {
-            v[2 * i] = static_cast<float>(static_cast<__bf16>(act_silu_f32(g0) * u0));
-            v[2 * i + 1] = static_cast<float>(static_cast<__bf16>(act_silu_f32(g1) * u1));
-          }
-        }
-        float amax = 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
-#pragma unroll
-        for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 16));
-        const float scale = fmaxf(amax, p.act_eps) / 448.0f;
-        const float inv_scale = 1.0f / scale;
-        int packed[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          float c4[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) c4[j] = fminf(fmaxf(act_div_by_scale(v[4 * i + j], scale, inv_scale), -448.0f), 448.0f);
-          int wd = __builtin_amdgcn_cvt_pk_fp8_f32(c4[0], c4[1], 0, false);
-          wd = __builtin_amdgcn_cvt_pk_fp8_f32(c4[2], c4[3], wd, true);
-          packed[i] = wd;
-        }
-        const int m = m0 + row;
-        if (row < BM && m < m_end) {
-          *reinterpret_cast<v2i*>(q_out + static_cast<int64_t>(m) * p.act_q_stride + n0 + sub * 8) = v2i{packed[0], packed[1]};
-          if (sub == 0) s_out[static_cast<int64_t>(m) * p.act_s_sm + static_cast<int64_t>(n0 / kScaleBlock) * p.act_s_sk] = scale;
-        }
-      }
-      continue;
-    }
+    const int el = lane, el32 = lane & 31, eh = lane >> 5;
     if (sliced && p.fused_reduce) {
       // Split-K in one launch.  The workgroups of a tile (one per K slice) park their fp32 sums in the workspace,
       // count themselves in on the tile's arrival counter, wait - for a bounded time - until all slices are in, and
@@ -1044,65 +628,6 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
           store_rows(std::false_type{});
       }
     };
-    if (AHEAD && p.c_lds && !sliced) {
-      // The same through the weight part of the last step's stage, 32 rows x 128 bytes of a wave at a time: the rest of the
-      // ring belongs to the next tile already.
-      static_assert(!AHEAD || 32 * 128 * WAVES <= Cfg::B_BYTES, "the staging slices fit in the weights of a stage");
-      uint8_t* idle = smem + (stage == 0 ? STAGES - 1 : stage - 1) * Cfg::STAGE_BYTES + Cfg::A_BYTES;
-      auto store_wave_tile = [&](auto f32, auto inside) __attribute__((always_inline)) {
-        constexpr bool F32 = decltype(f32)::value;
-        constexpr int NP = F32 ? 1 : 2;        // column fragments of a pass
-        constexpr int kEl = F32 ? 4 : 2;
-        constexpr int kRowBytes = NP * 32 * kEl;
-        constexpr int kCpr = kRowBytes / 16;   // 16-byte chunks per row
-        constexpr int kRpi = 64 / kCpr;        // rows per store instruction
-        uint8_t* st = idle + wave * (32 * kRowBytes);
-        const int r_in = el / kCpr, ch = el % kCpr;
-#pragma unroll
-        for (int mi = 0; mi < MF; ++mi)
-#pragma unroll
-          for (int nb = 0; nb < NF; nb += NP) {
-#pragma unroll
-            for (int ni = nb; ni < nb + NP; ++ni)
-#pragma unroll
-              for (int u = 0; u < 4; ++u) {
-                const v4f v = {acc[mi][ni][4 * u], acc[mi][ni][4 * u + 1], acc[mi][ni][4 * u + 2], acc[mi][ni][4 * u + 3]};
-                if constexpr (F32)
-                  *reinterpret_cast<v4f*>(st + el32 * kRowBytes + (2 * u + eh + el32) % kCpr * 16) = v;
-                else
-                  *reinterpret_cast<v4bf*>(st + el32 * kRowBytes + ((ni - nb) * 4 + u + el32) % kCpr * 16 + eh * 8) = __builtin_convertvector(v, v4bf);
-              }
-            if (Cfg::SCTAB && mi == 0 && nb == 0) wait_vmcnt<0>();  // the table, ahead of the stores
-            const int col = n0 + wn0 + nb * 32 + ch * (16 / kEl);
-            const int n_left = p.N - col;
-            char* c_col = c_base + static_cast<int64_t>(col) * kEl;
-#pragma unroll
-            for (int r0 = 0; r0 < 32; r0 += kRpi) {
-              const int row = r0 + r_in;
-              const v4i v = *reinterpret_cast<const v4i*>(st + row * kRowBytes + (ch + row) % kCpr * 16);
-              const int m = m0 + wm0 + mi * 32 + row;
-              if (m >= m_end || !(inside || n_left > 0)) continue;
-              char* dst = c_col + static_cast<int64_t>(m) * p.N * kEl;
-              if constexpr (F32)
-                store_row4<true>(dst, 0, __builtin_bit_cast(v4f, v), inside ? 4 : n_left);
-              else
-                store_row8_bf16(reinterpret_cast<__bf16*>(dst), v, inside ? 8 : n_left);
-            }
-          }
-      };
-      if (p.out_f32) {
-        if (cols_inside)
-          store_wave_tile(std::true_type{}, std::true_type{});
-        else
-          store_wave_tile(std::true_type{}, std::false_type{});
-      } else {
-        if (cols_inside)
-          store_wave_tile(std::false_type{}, std::true_type{});
-        else
-          store_wave_tile(std::false_type{}, std::false_type{});
-      }
-      continue;
-    }
     if (sliced) {
       // first pass of split-K: the slice's sums go to the workspace as an fp32 [M][N] matrix of their own;
       // fp8_splitk_reduce_kernel, launched behind this kernel on the same stream, adds the slices in index order
@@ -1173,16 +698,12 @@ __device__ __forceinline__ void pipelined_body(const Args& p, uint8_t* smem, int
   }
 }
 
-template <class Cfg, int MODE, bool AHEAD>
+template <class Cfg, int MODE>
 __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_pipelined_kernel(const Args p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  pipelined_body<Cfg, MODE, AHEAD>(p, smem, blockIdx.x, p.tiles_m, p.tiles_n, 0);
+  pipelined_body<Cfg, MODE>(p, smem, blockIdx.x, p.tiles_m, p.tiles_n);
 }
 
-// Dense GEMM whose columns are cut at p.n_split into a region of CfgA tiles and a region of narrower CfgB tiles,
-// one workgroup per tile, region A first.  The host picks the cut so that the last round of workgroups fills the
-// chip: e.g. 448 tiles of 256 x 256 on 256 CUs leave a quarter of the chip idle in the second round, while 256
-// tiles of 256 x 256 followed by 256 tiles of 256 x 192 cover the same output and keep every CU busy.
 // Expert-contiguous rows: a one-block pre-pass turns m_indices into three tile lists.  A run of R adjacent 128-row
 // blocks of one expert becomes R / 2 tiles of 256 rows when R is even, one tile of 128 rows when R = 1, and
 // (R - 3) / 2 tiles of 256 rows followed by two tiles of 192 rows when R is odd: most weight tiles are then fetched
@@ -1282,45 +803,6 @@ __global__ void __launch_bounds__(256) contiguous_prepass_kernel(const int32_t* 
 __device__ __forceinline__ int continue_round_robin(int before) {
   const int grid = static_cast<int>(gridDim.x);
   return (static_cast<int>(blockIdx.x) + grid - before % grid) % grid;
-}
-
-template <class CfgA, class CfgC, class CfgB>
-__global__ void __launch_bounds__(CfgA::NT) fp8_gemm_contig_list_kernel(const Args p) {
-  static_assert(CfgA::NT == CfgB::NT && CfgA::NT == CfgC::NT && CfgA::BN == CfgB::BN && CfgA::BN == CfgC::BN,
-                "the tile heights use the same workgroup shape and width");
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  // persistent workgroups: the 192-row pairs first - every workgroup starts at the same moment, so the two tiles of a
-  // pair run in step from their first K block (2 - 4 % over starting them behind the 256-row tiles) - then the 256-row
-  // tiles, then the 128-row ones
-  const int total_a = p.tlist[0] * p.tiles_n, total_c = p.tlist[1] * p.tiles_n;
-  pipelined_body<CfgC, kContigList>(p, smem, blockIdx.x, 0, p.tiles_n, 0);
-  pipelined_body<CfgA, kContigList>(p, smem, continue_round_robin(total_c), 0, p.tiles_n, 0);
-  pipelined_body<CfgB, kContigList>(p, smem, continue_round_robin(total_a + total_c), 0, p.tiles_n, 0);
-}
-
-// The gate/up projection of an expert MLP with the activation and the quantiser of its output fused into the epilogue
-// (dlblas/kernels/fused_moe_v3.py:307-334 as one kernel): weights [G][2 I][K] with the gate rows first, output
-// e4m3 [M][I] + scales [M][I / 128].  Same tile lists and schedule as fp8_gemm_contig_list_kernel; tiles_n = I / 128.
-template <class CfgA, class CfgC, class CfgB>
-__global__ void __launch_bounds__(CfgA::NT) fp8_gemm_contig_list_act_kernel(const Args p) {
-  static_assert(CfgA::NT == CfgB::NT && CfgA::NT == CfgC::NT && CfgA::BN == CfgB::BN && CfgA::BN == CfgC::BN,
-                "the tile heights use the same workgroup shape and width");
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  const int total_a = p.tlist[0] * p.tiles_n, total_c = p.tlist[1] * p.tiles_n;
-  pipelined_body<CfgC, kContigListAct>(p, smem, blockIdx.x, 0, p.tiles_n, 0);
-  pipelined_body<CfgA, kContigListAct>(p, smem, continue_round_robin(total_c), 0, p.tiles_n, 0);
-  pipelined_body<CfgB, kContigListAct>(p, smem, continue_round_robin(total_a + total_c), 0, p.tiles_n, 0);
-}
-
-template <class CfgA, class CfgB>
-__global__ void __launch_bounds__(CfgA::NT) fp8_gemm_pipelined_mixed_kernel(const Args p) {
-  static_assert(CfgA::NT == CfgB::NT && CfgA::BM == CfgB::BM, "both regions use the same workgroup shape and tile height");
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  const int bid = blockIdx.x;
-  if (bid < p.tiles_a)
-    pipelined_body<CfgA, kDense>(p, smem, bid, p.tiles_m, p.tiles_n_a, 0);
-  else
-    pipelined_body<CfgB, kDense>(p, smem, bid - p.tiles_a, p.tiles_m, p.tiles_n_b, p.n_split);
 }
 
 }  // namespace dlb

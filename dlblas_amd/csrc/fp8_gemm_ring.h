@@ -13,9 +13,13 @@
 //     they cost 3 %.
 //   - fragments take every other group of four rows, so that a lane's two results of a pair of fragments are 8 consecutive
 //     columns: results go from the registers to memory in 16-byte pieces, 64 or 128 bytes of a row per instruction.  No LDS
-//     is involved, so the ring runs on from tile to tile (AHEAD) in every layout.
+//     is involved, so the ring runs on from tile to tile (AHEAD) in every layout.  A tile with the quantising epilogue shares
+//     nothing but its rows' largest magnitudes through LDS, where the whole tile used to pass in bf16.
 // 4096 x 8192 x 18432 in 256 x 256 tiles: 505 us with 32 x 32 MFMAs and one hand-over per step, 471 us in this form
 // (2.62 PFLOP/s); its K steps take 2740 cycles of which 2048 are MFMA.  Without the scale FMAs it would be 421 us.
+// Expert-contiguous lists, 32 experts, 8192 rows, 4096 x 7168: 330 us per call with the former kernels (32 x 32 MFMAs, results
+// through LDS, a ring that drained between tiles), 306 us with these; the whole expert MLP on 8192 tokens 589 -> 532 us, of
+// which the ring that runs on is 5.
 //
 // Arithmetic: fp8_gemm_kernel of the reference (dlblas/kernels/fp8_gemm.py:49-60).  Requires K % 128 == 0.
 #pragma once
@@ -30,7 +34,7 @@ namespace dlb {
 template <int WGM_, int WGN_, int MF_, int NF_, int STAGES_, bool SCTAB_ = false, int SCTAB_KB_ = 0>
 struct RingCfg {
   static constexpr int WGM = WGM_, WGN = WGN_, MF = MF_, NF = NF_, STAGES = STAGES_;
-  static constexpr bool SCTAB = SCTAB_, PREFETCH = false;
+  static constexpr bool SCTAB = SCTAB_;
   static constexpr int WAVES = WGM * WGN, NT = WAVES * 64;
   static constexpr int BM = WGM * MF * 16, BN = WGN * NF * 16;
   static constexpr bool UNIFORM_W = 128 % (NF * 16) == 0;  // a wave's columns share one weight scale
@@ -718,6 +722,23 @@ __global__ void __launch_bounds__(CfgA::NT) fp8_gemm_ring_mixed_kernel(const Arg
     ring_body<CfgA, kDense, false>(p, smem, bid, p.tiles_m, p.tiles_n_a, 0);
   else
     ring_body<CfgB, kDense, false>(p, smem, bid - p.tiles_a, p.tiles_m, p.tiles_n_b, p.n_split);
+}
+
+// Expert-contiguous rows from the three tile lists (see contiguous_tile_list_block): persistent workgroups.  The 192-row pairs first:
+// every workgroup starts at the same moment, so the two tiles of a pair run in step from their first K block (2 - 4 % over
+// starting them behind the 256-row tiles); then the 256-row tiles, then the 128-row ones.
+// kContigListAct: the gate/up projection of an expert MLP with the activation and the quantiser of its output in the epilogue
+// (dlblas/kernels/fused_moe_v3.py:307-334 as one kernel): weights [G][2 I][K] with the gate rows first, output
+// e4m3 [M][I] + scales [M][I / 128]; tiles_n = I / 128.
+template <class CfgA, class CfgC, class CfgB, int MODE>
+__global__ void __launch_bounds__(CfgA::NT) fp8_gemm_ring_list_kernel(const Args p) {
+  static_assert(CfgA::NT == CfgB::NT && CfgA::NT == CfgC::NT && CfgA::BN == CfgB::BN && CfgA::BN == CfgC::BN,
+                "the tile heights use the same workgroup shape and width");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int total_a = p.tlist[0] * p.tiles_n, total_c = p.tlist[1] * p.tiles_n;
+  ring_body<CfgC, MODE, true>(p, smem, blockIdx.x, 0, p.tiles_n, 0);
+  ring_body<CfgA, MODE, true>(p, smem, continue_round_robin(total_c), 0, p.tiles_n, 0);
+  ring_body<CfgB, MODE, true>(p, smem, continue_round_robin(total_a + total_c), 0, p.tiles_n, 0);
 }
 
 }  // namespace dlb

@@ -597,6 +597,37 @@ def test_grouped_contiguous_run_lengths(dev, variant):
     helpers.tolerance_check(out, ref, f'contiguous run lengths {variant}')
 
 
+@pytest.mark.parametrize('kb,dtype', [(1, torch.bfloat16), (2, torch.float32), (3, torch.bfloat16), (4, torch.bfloat16), (5, torch.float32), (8, torch.bfloat16)])
+def test_list_tiles_carry_the_ring(dev, kb, dtype):
+    """Four tiles of every height (128, 192 and 256 rows) by 130 column tiles, the last of them 233 columns wide: each resident
+    workgroup goes through two or three tiles of a list, at fewer K blocks than the ring has stages, as many, and more.  Every
+    result has the bits of the uniform 128-row tiles."""
+    from dlblas_amd import _lib
+    from dlblas_amd.kernels.fp8_gemm_grouped import m_grouped_fp8_gemm_nt_contiguous
+    blocks, N, K = [1, 2, 3, 2, 1, 1, 3, 2, 2, 1], 129 * 256 + 233, kb * 128
+    print(f'case list ring K={K} {dtype}', flush=True)
+    G, M_sum = len(blocks), 128 * sum(blocks)
+    g = torch.Generator(device=dev).manual_seed(40 + kb)
+    a_q, a_s = helpers.quantise_act_device(torch.randn(M_sum, K, device=dev, generator=g).to(torch.bfloat16))
+    w_q, w_s = helpers.expert_weights_device(G, N, K, dev, 41)
+    m_indices = torch.repeat_interleave(torch.arange(G, dtype=torch.int32), torch.tensor(blocks) * 128).to(dev)
+    outs = []
+    try:
+        for variant in (None, 'pipe128x256w8'):
+            out = torch.full((M_sum, N), 7.0, dtype=dtype, device=dev)
+            _lib.tune('tile_list', 1 if variant is None else 0)
+            _lib.force_variant(variant)
+            m_grouped_fp8_gemm_nt_contiguous((a_q, a_s), (w_q, w_s), out, m_indices)
+            outs.append(out)
+    finally:
+        _lib.force_variant(None)
+        _lib.tune('tile_list', 0)
+    assert torch.equal(outs[0], outs[1])
+    rows = torch.tensor([0, 383, 384, 767, 768])  # experts 0 to 2
+    ref = torch.cat([orc.dequant_ref(a_q[r:r + 1].cpu(), a_s[r:r + 1].cpu(), w_q[e].cpu(), w_s[e].cpu()) for r, e in zip(rows.tolist(), (0, 1, 2, 2, 3))])
+    helpers.tolerance_check(outs[0][rows.to(dev)], ref, f'list ring K={K}')
+
+
 def test_grouped_contiguous_many_blocks(dev):
     """700 blocks of 128 rows: the device-side tile list then works in chunks of several blocks per thread, and runs of
     1 to 7 blocks (256-row tiles, pairs of 192-row tiles for the odd ones, single 128-row tiles) cross the chunk

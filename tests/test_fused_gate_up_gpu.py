@@ -180,6 +180,31 @@ def test_masked_fused_full_size_and_low_latency_experts(dev):
     assert torch.equal(out[valid], ref[valid])
 
 
+@pytest.mark.parametrize('kb', [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize('gathered', [False, True])
+def test_fused_list_tiles_carry_the_ring(dev, kb, gathered):
+    """Four tiles of every height by 130 column tiles (two or three tiles of a list per resident workgroup), at fewer K blocks
+    than a carried ring of gathered rows needs, as many, and more; rows that go up to the end of the token table.  The bytes and
+    scales of the three steps on the same rows."""
+    from dlblas_amd.kernels.fp8_gemm_grouped import fp8_gemm_grouped_contiguous_silu_quant
+    print(f'case fused list ring K={128 * kb} gathered={gathered}', flush=True)
+    blocks, inter, K, T = [1, 2, 3, 2, 1, 1, 3, 2, 2, 1], 130 * 128, kb * 128, 333
+    G, M_sum = len(blocks), 128 * sum(blocks)
+    g = torch.Generator(device=dev).manual_seed(60 + kb)
+    x_q, x_s = helpers.quantise_act_device((torch.randn(T, K, device=dev, generator=g) * 1.5).to(torch.bfloat16))
+    row_token = torch.randint(0, T, (M_sum, ), device=dev, generator=g, dtype=torch.int32)
+    row_token[-1] = T - 1
+    w_q, w_s = helpers.expert_weights_device(G, 2 * inter, K, dev, 61)
+    m_indices = torch.repeat_interleave(torch.arange(G, dtype=torch.int32), torch.tensor(blocks) * 128).to(dev)
+    a_q, a_s = x_q.view(torch.uint8)[row_token.long()].view(torch.float8_e4m3fn), x_s[row_token.long()]
+    fused, (ref_q, ref_s) = _both(dev, a_q, a_s, w_q, w_s, m_indices)
+    if gathered:
+        fused = fp8_gemm_grouped_contiguous_silu_quant(x_q, x_s, w_q, w_s, m_indices, a_row_index=row_token, column_major_scales=True)
+    assert fused is not None
+    assert torch.equal(fused[0].view(torch.uint8), ref_q.view(torch.uint8)), 'quantised codes differ'
+    assert torch.equal(fused[1], ref_s), 'scales differ'
+
+
 # --- the fused kernel reading the tokens through the row table of ep_scatter_rows (no expert-sorted copy) ------------
 
 
