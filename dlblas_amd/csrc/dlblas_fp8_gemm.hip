@@ -141,6 +141,7 @@ typedef TileCfg<128, 64, 2, 2> Tile128x64;
 typedef RingCfg<4, 2, 4, 8, 2> Ring256x256;      // 8 waves, wave tile 64 x 128
 typedef RingCfg<4, 2, 4, 6, 2> Ring256x192;      // narrow tiles of the mixed-width launch
 typedef RingCfg<2, 4, 6, 4, 2> Ring192x256;      // wave tile 96 x 64: the two tiles of an expert's run of three 128-row blocks
+typedef RingCfg<2, 4, 2, 4, 3> Ring64x256;       // wave tile 32 x 64: pieces of the tiles of a last round that is nearly empty
 typedef RingCfg<2, 4, 4, 4, 3> Ring128x256;      // wave tile 64 x 64
 // the same with a tile's activation scales in a table behind the ring (row-major a_s)
 typedef RingCfg<4, 2, 4, 8, 2, true, 27> Ring256x256T;
@@ -1455,7 +1456,7 @@ int run(const Problem& pr) {
       return rs.sctab ? launch_ring_mode<Ring256x256T>(pr.mode, ar, g_dense, dev, pr.stream) : launch_ring_mode<Ring256x256>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x256w8 && tile_list && pr.act) {
       static std::atomic<unsigned long long> lds_done{0};
-      auto kernel = fp8_gemm_ring_list_kernel<Ring256x256, Ring192x256, Ring128x256, kContigListAct>;
+      auto kernel = fp8_gemm_ring_list_kernel<Ring256x256, Ring192x256, Ring128x256, Ring64x256, kContigListAct>;
       const hipError_t le = ensure_lds(kernel, kListLds, dev, &lds_done);
       if (le != hipSuccess || g_prepare_only) return le;
       ar.tiles_n = static_cast<int>(pr.N / 256);  // 128 output columns = 128 gate + 128 up weight rows per tile
@@ -1464,7 +1465,7 @@ int run(const Problem& pr) {
     }
     if (pl.variant == kVarPipe128x256w8 && tile_list) {
       static std::atomic<unsigned long long> lds_done{0};
-      auto kernel = fp8_gemm_ring_list_kernel<Ring256x256, Ring192x256, Ring128x256, kContigList>;
+      auto kernel = fp8_gemm_ring_list_kernel<Ring256x256, Ring192x256, Ring128x256, Ring64x256, kContigList>;
       const hipError_t le = ensure_lds(kernel, kListLds, dev, &lds_done);
       if (le != hipSuccess || g_prepare_only) return le;
       ar.tiles_n = static_cast<int>(ceil_div(pr.N, 256));

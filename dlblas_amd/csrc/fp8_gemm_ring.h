@@ -63,7 +63,7 @@ struct RingCfg {
   static constexpr int T = H * S;                                  // MFMA slots of a K step
   static constexpr int B1 = H - 1, B2 = H * (S - 1 - PD) + H - 1;  // slots in front of which the parts' LDS is handed over
   static constexpr bool ONE_POINT = B1 == B2;
-  static_assert(WAVES == 8 && MF % 2 == 0 && NF % 2 == 0 && H == 4 && (S == 4 || S == 6 || S == 8), "the shapes this is written for");
+  static_assert(WAVES == 8 && MF % 2 == 0 && NF % 2 == 0 && (H == 4 || (H == 2 && S == 4)) && (S == 4 || S == 6 || S == 8), "the shapes this is written for");
   static_assert(S % NB == 0 && STRIPS * LOW % 4 == 0 && (ONE_POINT ? P2 == 0 : PD <= LOW), "fragments of a part are there when they are read");
   static_assert(LDS_BYTES <= 160 * 1024, "ring and table fit the LDS");
 };
@@ -103,8 +103,14 @@ struct RingTile {
 // starts at column n_base of the output.
 // AHEAD: the ring runs on from tile to tile; the steps of a tile whose fetches lie past the end of K fetch the first K blocks of
 // the workgroup's next tile.
+// Tile lists: the region is entries [lists.first, lists.first + lists.count) of a list's tiles (an entry per row tile and column tile), or, with 64-row tiles,
+// the entries' 64-row pieces, lists.pieces each.
+struct ListRegion {
+  int which, first, count, pieces;
+};
+
 template <class Cfg, int MODE, bool AHEAD>
-__device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_first, int tiles_m, int tiles_n, int n_base) {
+__device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_first, int tiles_m, int tiles_n, int n_base, ListRegion lists = {}) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, MF = Cfg::MF, NF = Cfg::NF, STAGES = Cfg::STAGES, H = Cfg::H, S = Cfg::S, L = Cfg::L;
   constexpr bool kList = MODE == kContigList || MODE == kContigListAct;
   constexpr bool kAct = MODE == kContigListAct || MODE == kMaskedAct;
@@ -160,13 +166,21 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
     } else if (kList) {
       // tiles of this height come from the list the pre-pass built: entry = first 128-row block of the tile.  The
       // column tiles of one row block are adjacent in the order, so they share the activation tile in L2.
-      static_assert(!kList || BM == 256 || BM == 192 || BM == 128, "tile heights of the three lists");
-      constexpr int kWhich = BM == 256 ? 0 : (BM == 192 ? 1 : 2);
-      const int total = entry(p.tlist, kWhich) * tiles_n;
+      static_assert(!kList || BM == 256 || BM == 192 || BM == 128 || BM == 64, "tile heights of the three lists and their pieces");
+      constexpr bool kPieces = BM == 64;
+      const int which = kPieces ? lists.which : BM == 256 ? 0 : (BM == 192 ? 1 : 2);
+      const int total = kPieces ? lists.count * lists.pieces : lists.count;
       if (vb >= total) return false;
-      const int v = xcd_remap(vb, total);
+      int v = xcd_remap(vb, total);
+      int piece = 0;
+      if (kPieces) {
+        const int w = v / lists.pieces;  // a tile's pieces side by side: they share its weights in one L2
+        piece = v - w * lists.pieces;
+        v = w;
+      }
+      v += lists.first;
       int li;
-      if (BM == 192) {
+      if (which == 1) {
         // the two tiles of a pair side by side for every column tile: neighbours in the order run on one XCD at the same time
         const int pair = v / (2 * tiles_n), r = v - pair * 2 * tiles_n;
         nt = r >> 1;
@@ -175,8 +189,9 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
         li = v / tiles_n;
         nt = v - li * tiles_n;
       }
-      m_first = entry(p.tlist, kTileListHeader + kWhich * p.tlist_cap + li) * 64;
+      m_first = entry(p.tlist, kTileListHeader + which * p.tlist_cap + li) * 64;
       g = entry(p.gidx, m_first);
+      m_first = min(m_first + piece * 64, p.M - 1);  // a piece past the end of a short last block: its last row once more
       t.m_end = min(p.M, m_first + BM);
     } else {
       if (vb >= units) return false;
@@ -730,15 +745,25 @@ __global__ void __launch_bounds__(CfgA::NT) fp8_gemm_ring_mixed_kernel(const Arg
 // kContigListAct: the gate/up projection of an expert MLP with the activation and the quantiser of its output in the epilogue
 // (dlblas/kernels/fused_moe_v3.py:307-334 as one kernel): weights [G][2 I][K] with the gate rows first, output
 // e4m3 [M][I] + scales [M][I / 128]; tiles_n = I / 128.
-template <class CfgA, class CfgC, class CfgB, int MODE>
+template <class CfgA, class CfgC, class CfgB, class CfgP, int MODE>
 __global__ void __launch_bounds__(CfgA::NT) fp8_gemm_ring_list_kernel(const Args p) {
-  static_assert(CfgA::NT == CfgB::NT && CfgA::NT == CfgC::NT && CfgA::BN == CfgB::BN && CfgA::BN == CfgC::BN,
+  static_assert(CfgA::NT == CfgB::NT && CfgA::NT == CfgC::NT && CfgA::NT == CfgP::NT && CfgA::BN == CfgB::BN && CfgA::BN == CfgC::BN && CfgA::BN == CfgP::BN,
                 "the tile heights use the same workgroup shape and width");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  const int total_a = p.tlist[0] * p.tiles_n, total_c = p.tlist[1] * p.tiles_n;
-  ring_body<CfgC, MODE, true>(p, smem, blockIdx.x, 0, p.tiles_n, 0);
-  ring_body<CfgA, MODE, true>(p, smem, continue_round_robin(total_c), 0, p.tiles_n, 0);
-  ring_body<CfgB, MODE, true>(p, smem, continue_round_robin(total_a + total_c), 0, p.tiles_n, 0);
+  const int grid = static_cast<int>(gridDim.x);
+  const int total_a = p.tlist[0] * p.tiles_n, total_c = p.tlist[1] * p.tiles_n, total_b = p.tlist[2] * p.tiles_n;
+  // The tiles a last round would hold too few of: cut where that round then takes their 64-row pieces, one for a workgroup at most.
+  // A piece's K step is bound by its 40 KB of loads, a whole tile's by its latency, so a round of pieces takes 25 to 35 us where one
+  // of whole tiles takes 56 (K = 7168); two rounds of pieces are no faster than one of tiles.  us per call without / with,
+  // 4096 x 7168, experts of 256 rows: 17 experts 183 / 151, 20 185 / 167, 33 286 / 270, 36 298 / 290; of 384 rows: 17 230 / 214; 14
+  // of 256 and 18 of 384 rows 339 / 326.  No difference without a cut.
+  const int rest = (total_a + total_b + total_c) % grid;
+  const int cut_a = rest <= total_a && rest * 4 <= grid ? rest : 0, cut_c = rest > total_a && rest <= total_c && rest * 3 <= grid ? rest : 0;
+  ring_body<CfgC, MODE, true>(p, smem, blockIdx.x, 0, p.tiles_n, 0, {1, 0, total_c - cut_c, 1});
+  ring_body<CfgA, MODE, true>(p, smem, continue_round_robin(total_c - cut_c), 0, p.tiles_n, 0, {0, 0, total_a - cut_a, 1});
+  ring_body<CfgB, MODE, true>(p, smem, continue_round_robin(total_a + total_c - cut_a - cut_c), 0, p.tiles_n, 0, {2, 0, total_b, 1});
+  const ListRegion pieces = cut_a > 0 ? ListRegion{0, total_a - cut_a, cut_a, 4} : ListRegion{1, total_c - cut_c, cut_c, 3};
+  ring_body<CfgP, MODE, true>(p, smem, blockIdx.x, 0, p.tiles_n, 0, pieces);
 }
 
 }  // namespace dlb
