@@ -147,6 +147,12 @@ typedef RingCfg<2, 4, 4, 4, 3> Ring128x256;      // wave tile 64 x 64
 typedef RingCfg<4, 2, 4, 8, 2, true, 27> Ring256x256T;
 typedef RingCfg<4, 2, 4, 6, 2, true, 27> Ring256x192T;
 typedef RingCfg<2, 4, 4, 4, 3, true, 16> Ring128x256T;
+// wave tile 32 x 64, for problems with few of the larger ones.  Eight waves instead of four with every fragment of the next step in a
+// second register set (the former kernel), and a ring that runs on: us per call 1024 x 4096 x 7168 51.1 -> 44.8, 512 x 7168 x 2048 16.5
+// -> 15.4, 500 x 4096 x 7168 in two slices 32.7 -> 31.6; of more than one round 3500 x 4096 x 512 26.1 -> 20.5, 2500 x 7168 x 2048 72 -> 60.
+// A second register set here changes nothing (44.4): on zeros the launch takes 34 us, the rest is the clock under load.
+typedef RingCfg<4, 2, 2, 4, 3> Ring128x128;
+typedef RingCfg<4, 2, 2, 4, 3, true, 54> Ring128x128T;
 
 // bytes of the three tile lists of an expert-contiguous launch over nblk 128-row blocks
 constexpr size_t tile_list_bytes(int64_t nblk) {
@@ -155,15 +161,13 @@ constexpr size_t tile_list_bytes(int64_t nblk) {
 constexpr int kListLds = Ring256x256::ACT_LDS_BYTES > Ring128x256::ACT_LDS_BYTES
                              ? (Ring256x256::ACT_LDS_BYTES > Ring192x256::ACT_LDS_BYTES ? Ring256x256::ACT_LDS_BYTES : Ring192x256::ACT_LDS_BYTES)
                              : (Ring128x256::ACT_LDS_BYTES > Ring192x256::ACT_LDS_BYTES ? Ring128x256::ACT_LDS_BYTES : Ring192x256::ACT_LDS_BYTES);
-// small tiles for problems with few of the large ones (M of a few hundred, or a narrow N): 4 waves, deep rings
-typedef PipeCfg<2, 2, 2, 2, 4> Pipe128x128;  // wave tile 64 x 64, 4 stages of 34 KB
+// small tiles for problems with few of the large ones (M of a few hundred, or a narrow N): 4 waves, a deep ring
 typedef PipeCfg<2, 2, 2, 1, 5> Pipe128x64;   // wave tile 64 x 32, 5 stages of 26 KB
 // the same with the activation scales of a tile in a table behind the ring (row-major a_s; as many K blocks per
-// workgroup as the LDS left by the ring holds: 54 and 64)
-typedef PipeCfg<2, 2, 2, 2, 4, true, 54> Pipe128x128T;
+// workgroup as the LDS left by the ring holds)
 typedef PipeCfg<2, 2, 2, 1, 5, true, 64> Pipe128x64T;
 static_assert(Ring256x192T::LDS_BYTES <= Ring256x256T::LDS_BYTES && Ring256x192::LDS_BYTES <= Ring256x256::LDS_BYTES, "a mixed launch asks for the wide tiles' LDS");
-static_assert(Pipe128x128T::LDS_BYTES <= 160 * 1024 && Pipe128x64T::LDS_BYTES <= 160 * 1024, "ring + table fit the LDS");
+static_assert(Pipe128x64T::LDS_BYTES <= 160 * 1024, "ring + table fit the LDS");
 constexpr int kFusedMaxTiles = DLB_WS_COUNTER_BYTES / 16;  // four counter words per tile in the workspace head
 
 // Tile shapes of the weight-streaming grouped kernel: rows x weight rows per tile, and the ring each leaves room for.
@@ -641,7 +645,7 @@ MidChoice pick_mid_plan(int64_t M, int64_t N, int kblocks, int cus, size_t ws_av
       const int64_t units = ceil_div(M, c.bm) * ceil_div(N, c.bn) * sk;
       // a tile's scales come once, into a table in LDS, when the slice is short enough: no re-layout launch and no scattered scale
       // lines per K step
-      const bool table = per <= (c.variant == kVarPipe128x64 ? Pipe128x64T::SCTAB_KB : c.variant == kVarPipe128x128 ? Pipe128x128T::SCTAB_KB : Ring128x256T::SCTAB_KB);
+      const bool table = per <= (c.variant == kVarPipe128x64 ? Pipe128x64T::SCTAB_KB : c.variant == kVarPipe128x128 ? Ring128x128T::SCTAB_KB : Ring128x256T::SCTAB_KB);
       double us = launch + (table ? 0.0 : relayout) +
                   static_cast<double>(ceil_div(units, cus)) * (tile_fixed + per * c.step_us * short_rows * (table ? 1.0 : scattered));
       if (sk > 1) us += second_pass + (2.0 * sk + 0.5) * out_bytes / ws_rate;  // partial sums written, read back, result written
@@ -919,7 +923,7 @@ double masked_ring_us(int variant, int64_t M, int64_t N, int64_t K, int G, int64
   else if (variant == kVarPipe128x128) c = {2.3, 3.6, 0.65, 0.0014};
   else if (variant == kVarPipe256x256) c = {1.5, 7.1, 1.51, 0.0015};
   const ExpertRows e(M, hint_rows);
-  const bool table = !act && kblocks <= (variant == kVarPipe128x128 ? Pipe128x128T::SCTAB_KB : variant == kVarPipe256x256 ? Ring256x256T::SCTAB_KB : Ring128x256T::SCTAB_KB);
+  const bool table = !act && kblocks <= (variant == kVarPipe128x128 ? Ring128x128T::SCTAB_KB : variant == kVarPipe256x256 ? Ring256x256T::SCTAB_KB : Ring128x256T::SCTAB_KB);
   const double tiles = G * e.live * e.row_tiles(bm) * static_cast<double>(act ? N / 256 : ceil_div(N, bn));
   return (M > kRelayoutMinRows && !table ? 3.5 : 0.0) + grouped_us(c, tiles, e.span <= bm, kblocks, bn, e.rows(bm), e.sharing(bm), 6.2e6, cus);
 }
@@ -1078,7 +1082,7 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
     if (g_knob[kKnobScaleTable] == 2 || as_sm == 1 || as_sk >= (1ll << 20) || !dma_ok || r.tile_list || gather_scales || fused_act) return false;
     switch (pl.variant) {
       case kVarPipe128x64: return mode == kDense && kb_per <= Pipe128x64T::SCTAB_KB;
-      case kVarPipe128x128: return kb_per <= Pipe128x128T::SCTAB_KB;
+      case kVarPipe128x128: return kb_per <= Ring128x128T::SCTAB_KB;
       case kVarPipe128x256w8: return (mode != kMasked || g_forced_variant < 0) && kb_per <= Ring128x256T::SCTAB_KB;
       case kVarPipe256x256: case kVarPipe256mix: return kb_per <= Ring256x256T::SCTAB_KB;
       default: return false;
@@ -1134,7 +1138,7 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
   // Dense launches of many rounds of equal tiles run one resident workgroup per CU that walks its tiles itself (the
   // ring kernels loop over tiles anyway): saves the hardware's per-workgroup start, 4 % at six rounds.  The 256-row kernel's
   // ring runs on from tile to tile, which pays from the second tile on (1 to 2 rounds 3 to 5 %, 2 to 4 rounds 7 %).
-  const bool runs_on = pl.variant == kVarPipe256x256 || pl.variant == kVarPipe256mix || pl.variant == kVarPipe128x256w8;
+  const bool runs_on = pl.variant == kVarPipe256x256 || pl.variant == kVarPipe256mix || pl.variant == kVarPipe128x256w8 || pl.variant == kVarPipe128x128;
   const bool mixed = pl.variant == kVarPipe256mix && r.n_split < N;  // a workgroup per tile
   r.resident = mode == kDense && !mixed && grid >= (runs_on ? cus + 1ll : 4ll * cus);
   r.grid = grid;
@@ -1477,8 +1481,7 @@ int run(const Problem& pr) {
     if (pl.variant == kVarPipe128x256w8 && rs.sctab) return launch_ring_mode<Ring128x256T>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x256w8) return launch_ring_mode<Ring128x256>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x128)
-      return rs.sctab ? launch_pipelined_mode<Pipe128x128T>(pr.mode, ar, g, dev, pr.stream)
-                      : launch_pipelined_mode<Pipe128x128>(pr.mode, ar, g, dev, pr.stream);
+      return rs.sctab ? launch_ring_mode<Ring128x128T>(pr.mode, ar, g_dense, dev, pr.stream) : launch_ring_mode<Ring128x128>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x64)
       return rs.sctab ? launch_pipelined<Pipe128x64T, kDense>(ar, g, dev, pr.stream)
                       : launch_pipelined_mode<Pipe128x64>(pr.mode, ar, g, dev, pr.stream);

@@ -1,4 +1,4 @@
-// FP8 block-scaled GEMM for gfx950 in tiles of 128 x 128 and 128 x 64, for problems with too few of the larger tiles for the chip
+// FP8 block-scaled GEMM for gfx950 in tiles of 128 x 64, for problems with too few of the larger tiles for the chip
 // (fp8_gemm_ring.h): 32x32x64 e4m3 MFMA, tiles streamed HBM -> LDS by the DMA path of the memory pipeline
 // (global_load_lds_dwordx4, no VGPR staging), multi-stage LDS ring, one barrier per 128-wide K step, block scales applied with
 // one FMA per accumulator element and K step.  Also what both files share: DMA and wait primitives, the pre-passes.
@@ -55,6 +55,7 @@ __device__ __forceinline__ v8i lds_read_frag32(const uint8_t* ring, int frag_byt
 }
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
+typedef __attribute__((address_space(3))) uint8_t* lds_bytes_t;
 typedef const __attribute__((address_space(1))) void* global_ptr_t;
 
 // Cache policy operand of the DMA instruction: kDmaStream sets the non-temporal bit.  It is for bytes that few
@@ -69,12 +70,13 @@ __device__ __forceinline__ void dma_16(const uint8_t* base, uint32_t voff, uint8
   __builtin_amdgcn_global_load_lds((global_ptr_t)(base + voff), (lds_ptr_t)lds_dst, 16, 0, POLICY);
 }
 // lane i moves 4 bytes from (base + voff) to lds_dst + 4 i.
-__device__ __forceinline__ void dma_4(const uint8_t* base, uint32_t voff, uint8_t* lds_dst) {
+template <class LdsPtr>
+__device__ __forceinline__ void dma_4(const uint8_t* base, uint32_t voff, LdsPtr lds_dst) {
   __builtin_amdgcn_global_load_lds((global_ptr_t)(base + voff), (lds_ptr_t)lds_dst, 4, 0, 0);
 }
 
-template <int POLICY>
-__device__ __forceinline__ void buf_dma_16(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff, uint8_t* lds_dst) {
+template <int POLICY, class LdsPtr>
+__device__ __forceinline__ void buf_dma_16(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff, LdsPtr lds_dst) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)lds_dst, 16, voff, soff, 0, POLICY);
 }
 

@@ -125,6 +125,7 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, q = lane >> 4;
+  const lds_bytes_t lds = (lds_bytes_t)smem;  // destination of the DMA: an address in LDS from the start, not a generic one cast at each load
   const int wm0 = (wave / Cfg::WGN) * (MF * 16), wn0 = (wave % Cfg::WGN) * (NF * 16);
   const uint32_t uK = static_cast<uint32_t>(p.K);
 
@@ -280,7 +281,7 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
   // instruction i of a K step's group into stage `stage_base`: i < P1 the first part, else the second
   auto issue_one = [&](auto idx, int stage_base, uint32_t off) __attribute__((always_inline)) {
     constexpr int i = decltype(idx)::value;
-    uint8_t* sbase = smem + stage_base;
+    const lds_bytes_t sbase = lds + stage_base;
     constexpr bool kScale = i == Cfg::P1 - 1;
     constexpr bool kHeld = i < Cfg::H_INST;
     constexpr int j = kHeld ? i : i < Cfg::P1 - 1 ? i - Cfg::H_INST : i - Cfg::H_INST - 1;
@@ -320,7 +321,7 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
       const uint32_t r = static_cast<uint32_t>(min(row, last));
       const uint32_t j = static_cast<uint32_t>(min(e - row * pitch, nk - 1));
       dma_4(reinterpret_cast<const uint8_t*>(as_tile), (r * static_cast<uint32_t>(p.as_sm) + j * static_cast<uint32_t>(p.as_sk)) * 4u,
-            smem + Cfg::SCTAB_OFF + i * 256);
+            lds + Cfg::SCTAB_OFF + i * 256);
     }
   };
 
@@ -394,7 +395,7 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
     if (AHEAD && gather && ahead && wave < BM / 64) {
       // the next tile's source rows, on their way before any group that is waited for
       const int r = wave * 64 + lane;
-      dma_4(reinterpret_cast<const uint8_t*>(p.a_rows + tn.m0), static_cast<uint32_t>(min(r, min(BM, tn.m_end - tn.m0) - 1)) * 4u, smem + Cfg::ROWS_OFF + wave * 256);
+      dma_4(reinterpret_cast<const uint8_t*>(p.a_rows + tn.m0), static_cast<uint32_t>(min(r, min(BM, tn.m_end - tn.m0) - 1)) * 4u, lds + Cfg::ROWS_OFF + wave * 256);
     }
     // K steps of this tile whose blocks landed before the last tile's results were stored: nothing to wait for
     const int landed = AHEAD && staged ? STAGES : 0;

@@ -440,7 +440,7 @@ int dlb_fp8_gemm_force_variant(int variant);
  *   DLB_KNOB_SKINNY_NFRAGS  16-row weight fragments per decode workgroup (1 or 2)
  *   DLB_KNOB_GROUP_M        m-tiles per L2 swizzle group of the tiled kernels
  *   DLB_KNOB_SKINNY_DMA     2 = decode kernels load operands through registers instead of the LDS DMA path
- *   DLB_KNOB_EPILOGUE       2 = the 128 x 128 and 128 x 64 kernels store their results straight from registers (no LDS transpose),
+ *   DLB_KNOB_EPILOGUE       2 = the 128 x 64 kernel stores its results straight from registers (no LDS transpose),
  *                           dense tiles of resident workgroups start with an empty ring
  *   DLB_KNOB_SKINNY_BN      output columns per workgroup of the DMA-staged decode kernels (multiple of 4, at most 32)
  *   DLB_KNOB_SPLITK_MODE    1 = the K slices of the DMA-ring kernels are added inside the launch (one launch per call: the
