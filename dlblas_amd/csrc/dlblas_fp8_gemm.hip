@@ -278,7 +278,7 @@ hipError_t launch_ring_mode(int mode, const Args& args, int grid, int dev, hipSt
       if constexpr (Cfg::BM == kScaleBlock) return launch_ring<Cfg, kContiguous>(args, grid, dev, stream);  // taller tiles come from the lists
       return hipErrorInvalidValue;
     default:
-      return launch_ring<Cfg, kMasked>(args, grid, dev, stream);
+      return launch_ring<Cfg, kMasked, true>(args, grid, dev, stream);
   }
 }
 
@@ -669,12 +669,17 @@ double decode_us(int64_t M, int64_t N, int64_t K, int kblocks, int cus) {
   return 2.6 + (l2_us > chain_us ? l2_us : chain_us);
 }
 
+double masked_ring_us(int variant, int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, int cus);
+double contiguous_small_us(int64_t rows, int64_t N, int64_t K, int G, int cus);
+double contiguous_plain_us(int64_t rows, int64_t N, int64_t K, int G, int cus);
+double contiguous_lists_us(int64_t rows, int64_t N, int64_t K, int G, int cus, bool there = false);
+
 // dma_ok: the DMA kernels address their sources with 32-bit byte offsets from the tile's first row (up to 256 rows x K
 // bytes, 512 scale rows x stride); false sends such problems to the kernels with 64-bit addressing.
 // G, hint_rows (grouped layouts): experts, and the masked layout's typical rows per expert (<= 0: unknown).
 // fixed_grouped: the caller needs the 128 x 256 kernel (the fused activation epilogues exist for it only).
 Plan make_plan(int mode, int64_t M, int64_t N, int64_t K, int cus, size_t ws_bytes, bool dma_ok, int G = 1,
-               int64_t hint_rows = -1, bool fixed_grouped = false) {
+               int64_t hint_rows = -1, bool fixed_grouped = false, bool lists_there = false) {
   Plan pl{kVarTile128x128, 128, 128, 1, 4, 4, 1, 16, dma_ok};
   const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
   const size_t ws_avail = ws_bytes > DLB_WS_COUNTER_BYTES ? ws_bytes - DLB_WS_COUNTER_BYTES : 0;
@@ -712,19 +717,22 @@ Plan make_plan(int mode, int64_t M, int64_t N, int64_t K, int cus, size_t ws_byt
       const int64_t tn = ceil_div(N, 256);
       if (fixed_grouped || (mode == kContiguous && g_knob[kKnobTileList] == 1)) {
       } else if (mode == kContiguous) {
-        // a small batch: 128 x 128 tiles while 128 x 256 ones would leave half the CUs idle
-        // (8 experts x 128 rows x 4096 x 7168: 67 -> 54 us)
-        if (ceil_div(M, 128) * tn * 2 <= cus) v = kVarPipe128x128;
+        // (the lists belong to the 128 x 256 variant)
+        const double small_us = contiguous_small_us(M, N, K, G, cus);
+        if (small_us < contiguous_plain_us(M, N, K, G, cus) && (ceil_div(M, kScaleBlock) <= G || small_us < contiguous_lists_us(M, N, K, G, cus, lists_there))) v = kVarPipe128x128;
       } else if (hint_rows > 0) {
-        // masked, with the caller's hint: few rows per expert and few experts - smaller tiles, as above (8 experts,
-        // 4096 x 7168, up to 128 rows each: 54 - 75 -> 44 - 55 us); several hundred rows per expert - 256-row tiles,
-        // which fetch an expert's weights once per 256 rows (32 experts x ~520 rows x 4096 x 7168: 665 -> 573 us,
-        // 7168 x 2048: 363 -> 335 us)
-        // (or two 128-row tiles per expert that fill one round at most: 8 experts x ~240 rows: 121 -> 110 us)
-        const int64_t em = hint_rows < M ? hint_rows : M;
-        const int64_t units = static_cast<int64_t>(G) * ceil_div(em, 128) * tn;
-        if (units * 2 <= cus) v = kVarPipe128x128;
-        else if (em >= 384 || (em >= 192 && units <= cus)) v = kVarPipe256x256;
+        // masked, with the caller's hint: from 384 rows per expert on 256-row tiles, which fetch an expert's weights once per 256 rows (32
+        // experts x ~520 rows x 4096 x 7168: 665 -> 573 us when they were introduced); fewer: the shape of the smallest estimate (the
+        // same choice from 384 rows on is 0.03 % worse over 350 problems)
+        if (hint_rows < M ? hint_rows >= 384 : M >= 384) {
+          v = kVarPipe256x256;
+        } else {
+          double best_us = masked_ring_us(v, M, N, K, G, hint_rows, false, cus);
+          for (int other : {kVarPipe128x128, kVarPipe256x256}) {
+            const double us = masked_ring_us(other, M, N, K, G, hint_rows, false, cus);
+            if (us < best_us) v = other, best_us = us;
+          }
+        }
       }
     } else {
       v = (M <= 64 && mode != kContiguous) ? kVarTile64x128 : kVarTile128x128;
@@ -884,16 +892,17 @@ int stream_chunk_len(int kb_min, int kb_max, int ch, int stages) {
 
 // Rows that cover nearly all experts: twice the caller's hint, at most the buffers' height.
 int64_t stream_span(int64_t M, int64_t hint_rows) { return hint_rows > 0 && 2 * hint_rows < M ? 2 * hint_rows : M; }
-// Time of a grouped launch (microseconds, fitted on MI355X to 828 problems of 8 .. 32 experts x 1 .. 960 rows, N = 512 .. 7168, K =
-// 384 .. 7168; rms 8 - 12 %): `start` + rounds of tiles x (`tile` + K blocks x a step of `step` + `row` per activation row of the
-// tile, but no shorter than its share of the stream of weights that the busy CUs draw, bytes per microsecond in `rate`).  Taken
-// over 0.92, 1 and 1.08 times the tile count, which is an estimate itself - except that experts of one row tile have no more
-// than that (32 experts x 0 .. 16 rows x 1024 x 6144 in 64 x 128 tiles are one round of 256, never two).
+// Time of a grouped launch (microseconds, fitted on MI355X: the weight-streaming kernel to 828 problems of 8 .. 32 experts x 1 .. 960 rows,
+// N = 512 .. 7168, K = 384 .. 7168, the ring kernels to 233 of 16 .. 1024 slots; rms 8 - 12 %): `start` + rounds of tiles x (`tile` +
+// K blocks x a step of `step` + `row` per activation row of the tile, but no shorter than its share of the stream of weights that
+// the busy CUs draw, `rate` TB/s).  Taken over 0.92, 1 and 1.08 times the tile count, which is an estimate itself - except
+// that experts of one row tile have no more than that (32 experts x 0 .. 16 rows x 1024 x 6144 in 64 x 128 tiles are one round of
+// 256, never two).
 struct TileCost {
-  double start, tile, step, row;
+  double start, tile, step, row, rate;
 };
-double grouped_us(const TileCost& c, double tiles, bool at_most, int kblocks, int bn, double rows, double sharing, double rate, int cus) {
-  auto step = [&](double busy) { return std::max(c.step + c.row * rows, bn * 128.0 * busy / sharing / rate); };
+double grouped_us(const TileCost& c, double tiles, bool at_most, int kblocks, int bn, double rows, double sharing, int cus) {
+  auto step = [&](double busy) { return std::max(c.step + c.row * rows, bn * 128.0 * busy / sharing / (c.rate * 1e6)); };
   double us = 0.0;
   for (double spread : {0.92, 1.0, at_most ? 1.0 : 1.08}) {
     const double full = std::floor(tiles * spread / cus), rest = tiles * spread - full * cus;
@@ -918,20 +927,20 @@ double masked_ring_us(int variant, int64_t M, int64_t N, int64_t K, int G, int64
   const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
   int bm, bn;
   tile_dims(variant, &bm, &bn);
-  TileCost c = {2.4, 5.0, 0.80, 0.0028};  // 128 x 256
-  if (act) c = {8.8, 0.8, 0.88, 0.0024};
-  else if (variant == kVarPipe128x128) c = {2.3, 3.6, 0.65, 0.0014};
-  else if (variant == kVarPipe256x256) c = {1.5, 7.1, 1.51, 0.0015};
+  TileCost c = {2.7248, 4.6095, 0.8149, 0.0024, 6.3341};  // 128 x 256
+  if (act) c = {8.8, 0.8, 0.88, 0.0024, 6.2};
+  else if (variant == kVarPipe128x128) c = {4.1558, 2.2571, 0.453, 0.0023, 5.7111};
+  else if (variant == kVarPipe256x256) c = {3.1421, 6.5096, 1.0252, 0.0027, 5.7668};
   const ExpertRows e(M, hint_rows);
   const bool table = !act && kblocks <= (variant == kVarPipe128x128 ? Ring128x128T::SCTAB_KB : variant == kVarPipe256x256 ? Ring256x256T::SCTAB_KB : Ring128x256T::SCTAB_KB);
   const double tiles = G * e.live * e.row_tiles(bm) * static_cast<double>(act ? N / 256 : ceil_div(N, bn));
-  return (M > kRelayoutMinRows && !table ? 3.5 : 0.0) + grouped_us(c, tiles, e.span <= bm, kblocks, bn, e.rows(bm), e.sharing(bm), 6.2e6, cus);
+  return (M > kRelayoutMinRows && !table ? 3.5 : 0.0) + grouped_us(c, tiles, e.span <= bm, kblocks, bn, e.rows(bm), e.sharing(bm), cus);
 }
 
 // Tile shapes of the weight-streaming kernel: fragments read when needed / one step ahead / with the quantising epilogue
-constexpr TileCost kStreamCost[kStreamCount] = {{2.9, 0.5, 0.74, 0.0048}, {2.5, 1.9, 0.69, 0.0066}, {4.1, 0.6, 0.42, 0.0048}, {2.8, 1.7, 0.69, 0.0074}, {4.2, 0.9, 0.38, 0.0016}};
-constexpr TileCost kStreamCostAhead[kStreamCount] = {{}, {3.0, 2.2, 0.71, 0.0041}, {4.9, 1.0, 0.44, 0.0025}, {3.4, 2.2, 0.71, 0.0058}, {5.6, 0.8, 0.30, 0.0012}};
-constexpr TileCost kStreamCostAct[kStreamCount] = {{3.7, 0.6, 0.73, 0.0025}, {3.6, 2.0, 0.72, 0.0044}, {}, {5.2, 2.0, 0.70, 0.0049}, {}};
+constexpr TileCost kStreamCost[kStreamCount] = {{2.9, 0.5, 0.74, 0.0048, 6.9}, {2.5, 1.9, 0.69, 0.0066, 6.9}, {4.1, 0.6, 0.42, 0.0048, 6.9}, {2.8, 1.7, 0.69, 0.0074, 6.9}, {4.2, 0.9, 0.38, 0.0016, 6.9}};
+constexpr TileCost kStreamCostAhead[kStreamCount] = {{}, {3.0, 2.2, 0.71, 0.0041, 6.9}, {4.9, 1.0, 0.44, 0.0025, 6.9}, {3.4, 2.2, 0.71, 0.0058, 6.9}, {5.6, 0.8, 0.30, 0.0012, 6.9}};
+constexpr TileCost kStreamCostAct[kStreamCount] = {{3.7, 0.6, 0.73, 0.0025, 6.9}, {3.6, 2.0, 0.72, 0.0044, 6.9}, {}, {5.2, 2.0, 0.70, 0.0049, 6.9}, {}};
 
 // How the weight-streaming kernel runs a grouped launch (shape kStreamNone: it does not), from the typical rows of an expert, and
 // whether it is to run at all: other_us is the estimate of the kernel that would run instead (0: none).  The choice is 2.3 % behind
@@ -945,7 +954,7 @@ constexpr TileCost kStreamCostAct[kStreamCount] = {{3.7, 0.6, 0.73, 0.0025}, {3.
 // max_slices: 1 where the bits have to be those of the steps apart (one slice changes nothing about the sums), up to kMaxStreamSlices
 // inside an expert MLP.  all_rows: rows of the partial sums' matrices; slice_floats: room for them.
 StreamPlan pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, int cus, int max_slices, int64_t all_rows, size_t slice_floats,
-                       double other_us) {
+                       double other_us, bool by_estimates = false) {
   StreamPlan best;
   const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
   const int knob = g_knob[kKnobStream], slice_knob = g_knob[kKnobStreamSlices];
@@ -962,7 +971,7 @@ StreamPlan pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows
     if (len <= 0) return;
     const TileCost& c = fused_act ? kStreamCostAct[shape] : ahead ? kStreamCostAhead[shape] : kStreamCost[shape];
     const double tiles = G * e.live * e.row_tiles(d.bm) * static_cast<double>(fused_act ? N / 256 : ceil_div(N, d.bn)) * parts;
-    double us = grouped_us(c, tiles, e.span <= d.bm, kb_max, d.bn, e.rows(d.bm), e.sharing(d.bm), 6.9e6, cus);
+    double us = grouped_us(c, tiles, e.span <= d.bm, kb_max, d.bn, e.rows(d.bm), e.sharing(d.bm), cus);
     if (slices > 0) us += 3.8 + slices * part_bytes / 2.0e6;
     if (best.shape == kStreamNone || us < 0.98 * best.us) best.shape = shape, best.us = us, best.chunk_len = len, best.slices = slices, best.ahead = ahead;
   };
@@ -984,34 +993,56 @@ StreamPlan pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows
   // 116 / 123; 32 x 4096 x 7168 cap 256 217 / 226, cap 384 305 / 298; 8 x 1152 x 768, ~640 rows 15.6 / 22.8; 8 x 512 x 1920, ~244
   // rows 14.4 / 20.1.  Quantising: 8 x 512 x 2176, ~137 rows 17.6 / 26.1; 32 x 2048 x 1920, ~181 rows 50 / 61.
   const bool longer = e.span > (act ? 192 : kblocks <= 24 ? 448 : 256);
-  if (longer && knob == 0 && slice_knob == 0 && other_us > 0.0 && best.us > 0.95 * other_us) best.shape = kStreamNone;
+  // by_estimates: the masked layout's plain product with a hint, where the estimates of both kernels decide from 64 rows on.  Over 350
+  // problems 2.8 % behind the best kernel and shape, 5.1 % with the limits (from 256 slots on they cost 6.9 %).  This kernel runs
+  // faster than its estimate there, most of all in launches of more than two rounds of 256 x 256 tiles: 32 x 256 x 7168 x 2048 118 us
+  // for 148, the ring 126 for 121; 32 x 256 x 4096 x 7168 223 for 282, the ring 209 for 181.
+  const bool many_rounds = static_cast<double>(G) * e.live * e.row_tiles(256) * static_cast<double>(ceil_div(N, 256)) > 2.0 * cus;
+  by_estimates = by_estimates && e.span > 64.0;
+  const double ahead = by_estimates ? (many_rounds ? 1.23 : 1.12) : 0.95;
+  if ((longer || by_estimates) && knob == 0 && slice_knob == 0 && other_us > 0.0 && best.us > ahead * other_us) best.shape = kStreamNone;
   return best;
 }
 
-// Expert-contiguous rows.  Taller tiles save weight traffic, not time per tile.  Estimates (microseconds, constants as in
-// prefers_128_row_tiles): uniform 128-row tiles take rounds x (5.5 + 1.2 K blocks: most of their weights come from HBM) or, when
-// that is longer, the time to stream every block's weight matrix (6.4 TB/s: neighbouring tiles of an expert share some of it in
-// the L2); the lists take 5 us for their pre-pass + rounds x (11.5 + 1.62 K blocks) or the weights of their tiles at 4.85 TB/s, with
-// as many tiles as pairs of blocks, but at least one per expert.  8 experts, 1408 rows, 4096 x 7168: 107 us with lists, 69 us
-// without; 2432 rows: 106 us with, 128 us without; 32 experts x 128 rows: 183 / 174.
-double contiguous_plain_us(int64_t rows, int64_t N, int64_t K, int cus) {
-  const int64_t nblk = ceil_div(rows, kScaleBlock), kblocks = ceil_div(K, kScaleBlock);
-  const double mat_mb = static_cast<double>(N) * static_cast<double>(K) * 1e-6;
-  return std::max(static_cast<double>(ceil_div(nblk * ceil_div(N, 256), cus)) * (5.5 + 1.2 * static_cast<double>(kblocks)),
-                  static_cast<double>(nblk) * mat_mb / 6.4);
+// Expert-contiguous rows: estimates (microseconds, fitted on MI355X to 200 problems of 8 .. 32 experts x 500 .. 12000 tokens, N and K = 512 ..
+// 7168; rms 8, 8 and 17 %; their choice is 0.7 % behind the best of the three there and 0.9 % on 90 others) of 128 x 128 tiles, 128 x
+// 256 tiles and the lists.  Rounds of tiles x (fixed part + K blocks x the longer of a step and its share of the weights' stream, which
+// neighbouring row tiles of an expert share); the lists' step grows with the rows of a tile, two blocks where an expert has them.
+// us with 128 x 256 tiles / lists: 32 experts, 5888 rows, 7168 x 2048 154 / 127, 8 experts, 9344 rows, 4096 x 1280 83 / 75; 8
+// experts, 1920 rows, 3840 x 6144 68 / 78.
+double contiguous_rounds_us(double tiles, double tile, double step, int kblocks, double stream_us, int cus) {
+  const double full = std::floor(tiles / cus), rest = tiles - full * cus;
+  auto round = [&](double busy) { return tile + kblocks * std::max(step, stream_us * busy); };
+  return full * round(cus) + (rest > 0.5 ? round(rest) : 0.0);
 }
-double contiguous_lists_us(int64_t rows, int64_t N, int64_t K, int G, int cus) {
-  const int64_t nblk = ceil_div(rows, kScaleBlock), kblocks = ceil_div(K, kScaleBlock);
-  const double mat_mb = static_cast<double>(N) * static_cast<double>(K) * 1e-6;
-  const int64_t tall = std::max(ceil_div(nblk, 2), std::min<int64_t>(nblk, G));
-  return 5.0 + std::max(static_cast<double>(ceil_div(tall * ceil_div(N, 256), cus)) * (11.5 + 1.62 * static_cast<double>(kblocks)),
-                        static_cast<double>(tall) * mat_mb / 4.85);
+// blocks of a typical expert
+double contiguous_run(int64_t nblk, int G) { return std::max(1.0, static_cast<double>(nblk) / static_cast<double>(std::max<int64_t>(1, std::min<int64_t>(nblk, G)))); }
+double contiguous_small_us(int64_t rows, int64_t N, int64_t K, int G, int cus) {
+  const int64_t nblk = ceil_div(rows, kScaleBlock);
+  const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
+  return 1.5 + contiguous_rounds_us(static_cast<double>(nblk * ceil_div(N, 128)), 4.06, 0.649, kblocks, 128 * 128.0 / (std::min(contiguous_run(nblk, G), 2.0) * 4.74e6), cus);
+}
+double contiguous_plain_us(int64_t rows, int64_t N, int64_t K, int G, int cus) {
+  const int64_t nblk = ceil_div(rows, kScaleBlock);
+  const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
+  return (kblocks > Ring128x256T::SCTAB_KB ? 5.5 : 2.0) +
+         contiguous_rounds_us(static_cast<double>(nblk * ceil_div(N, 256)), 5.77, 0.907, kblocks, 256 * 128.0 / (std::min(contiguous_run(nblk, G), 1.44) * 5.4e6), cus);
+}
+double contiguous_lists_us(int64_t rows, int64_t N, int64_t K, int G, int cus, bool there) {
+  const int64_t nblk = ceil_div(rows, kScaleBlock);
+  const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
+  const double tall = std::max(0.5 * static_cast<double>(nblk), static_cast<double>(std::min<int64_t>(nblk, G)));
+  const double step = 0.351 + 1.196 * 0.5 * static_cast<double>(nblk) / tall;
+  double us = 0.0;
+  for (double spread : {0.95, 1.0, 1.05})
+    us += contiguous_rounds_us(spread * tall * static_cast<double>(ceil_div(N, 256)), 9.47, step, kblocks, 256 * 128.0 / (1.294 * 5.24e6), cus) / 3.0;
+  return (there ? 0.0 : 3.6) + us;  // there: the workspace holds the lists, no launch in front builds them
 }
 
 // (act: the quantising epilogue exists for the lists only)
 double contiguous_us(int64_t rows, int64_t N, int64_t K, int G, bool act, int cus) {
   const double lists_us = contiguous_lists_us(rows, N, K, G, cus);
-  return act ? lists_us : std::min(lists_us, contiguous_plain_us(rows, N, K, cus));
+  return act ? lists_us : std::min(lists_us, std::min(contiguous_small_us(rows, N, K, G, cus), contiguous_plain_us(rows, N, K, G, cus)));
 }
 
 // How the weight-streaming kernel runs a launch on row ranges (mlp: a step of an expert MLP, whose K may be sliced).
@@ -1037,13 +1068,13 @@ int expert_form(int64_t rows, int64_t N, int64_t K, int G, int64_t hint_rows, bo
 // overlay: the kernel whose waves split K may take the launch over from the planned variant.
 // fused_act: the launch is one of the gate/up GEMMs with the activation in its epilogue (their kernels take no scale table)
 Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as_sm, int64_t as_sk, bool have_ws,
-                 size_t ws_bytes, int cus, bool gather_scales = false, bool fused_act = false, int64_t hint_rows = -1, bool overlay = true, int max_slices = 1) {
+                 size_t ws_bytes, int cus, bool gather_scales = false, bool fused_act = false, int64_t hint_rows = -1, bool overlay = true, int max_slices = 1, bool lists_there = false) {
   Resolved r{};
   const int64_t kblocks = ceil_div(K, kScaleBlock);
   const int64_t groups = mode == kMasked ? G : 1;  // a_s is per expert only in the masked layout; contiguous rows are one matrix
   const bool dma_ok = K < (1ll << 24) && as_sm < (1ll << 21);
   const bool usable_ws = have_ws && ws_bytes > DLB_WS_COUNTER_BYTES;
-  r.pl = make_plan(mode, rows, N, K, cus, usable_ws ? ws_bytes : 0, dma_ok, G, hint_rows, fused_act || gather_scales);
+  r.pl = make_plan(mode, rows, N, K, cus, usable_ws ? ws_bytes : 0, dma_ok, G, hint_rows, fused_act || gather_scales, lists_there);
   const Plan& pl = r.pl;
   r.wavek = kWaveKNone;
   // (its scale table is fetched through 32-bit byte offsets from the tile's first row; tiles have up to 64 rows)
@@ -1060,7 +1091,7 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
   }
   if (mode == kMasked && dma_ok && K % kScaleBlock == 0 && K > 0 && static_cast<int64_t>(G) * rows < (1ll << 31))
     r.stream = pick_stream(rows, N, K, G, hint_rows, fused_act, cus, max_slices, rows * G, usable_ws ? (ws_bytes - DLB_WS_COUNTER_BYTES) / sizeof(float) : 0,
-                           masked_ring_us(pl.variant, rows, N, K, G, hint_rows, fused_act, cus));
+                           masked_ring_us(pl.variant, rows, N, K, G, hint_rows, fused_act, cus), !fused_act && hint_rows > 0);
   const int want = usable_ws ? pl.splitk : 1;
   r.kb_per_split = static_cast<int>(ceil_div(kblocks > 0 ? kblocks : 1, want));
   r.splitk = static_cast<int>(ceil_div(kblocks > 0 ? kblocks : 1, r.kb_per_split));  // no empty slice
@@ -1070,7 +1101,7 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
     const size_t bytes = tile_list_bytes(nblk);
     // (the fused epilogues exist for the list kernel only)
     bool worth_it = fused_act || gather_scales || g_knob[kKnobTileList] == 1;
-    if (!worth_it && g_knob[kKnobTileList] != 2 && nblk > G) worth_it = contiguous_lists_us(rows, N, K, G, cus) < contiguous_plain_us(rows, N, K, cus);
+    if (!worth_it && g_knob[kKnobTileList] != 2 && nblk > G) worth_it = contiguous_lists_us(rows, N, K, G, cus, lists_there) < contiguous_plain_us(rows, N, K, G, cus);
     if (worth_it && nblk <= kTileListMaxBlocks && DLB_WS_COUNTER_BYTES + bytes <= ws_bytes) r.tile_list = true, r.nblk = nblk, r.ws_used = bytes;
   }
   // A tile's row-major scales come once, into a table in LDS, where its K range fits what the ring leaves of the LDS: no re-layout
@@ -1261,8 +1292,10 @@ int run_ragged(const RaggedProblem& pr) {
 
 // Masked gate/up projection with the epilogue fused (rs) or the plain product and the activation apart?  Several hundred rows per
 // expert: the plain product's taller tiles (32 experts x ~520 rows: 619 against 678 us).
-bool steps_apart(const Resolved& rs, int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, size_t ws_bytes, int cus) {
-  return rs.stream.shape == kStreamNone && make_plan(kMasked, M, N, K, cus, ws_bytes, true, G, hint_rows).variant != kVarPipe128x256w8;
+bool steps_apart(const Resolved& rs, int64_t M, int64_t N, int G, int64_t hint_rows, int cus) {
+  if (rs.stream.shape != kStreamNone || hint_rows <= 0) return false;
+  const int64_t em = std::min(hint_rows, M), units = static_cast<int64_t>(G) * ceil_div(em, 128) * ceil_div(N, 256);
+  return units * 2 <= cus || em >= 384 || (em >= 192 && units <= cus);
 }
 
 // Argument checks that need no device.  Returns DLB_OK with *empty set when there is nothing to compute.
@@ -1321,9 +1354,9 @@ int run(const Problem& pr) {
 
   if (pr.ws && misaligned(pr.ws, 16)) return fail(DLB_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
   const Resolved rs = resolve(pr.mode, pr.rows, pr.N, pr.K, pr.G, pr.as_sm, pr.as_sk, pr.ws != nullptr, pr.ws_bytes, cus,
-                              pr.a_rows != nullptr, pr.act, pr.hint_rows, true, pr.mlp ? kMaxStreamSlices : 1);
+                              pr.a_rows != nullptr, pr.act, pr.hint_rows, true, pr.mlp ? kMaxStreamSlices : 1, pr.list_there);
   const Plan& pl = rs.pl;
-  if (pr.mlp && pr.mode == kMasked && steps_apart(rs, pr.rows, pr.N, pr.K, pr.G, pr.hint_rows, pr.ws ? pr.ws_bytes : 0, cus))
+  if (pr.mlp && pr.mode == kMasked && steps_apart(rs, pr.rows, pr.N, pr.G, pr.hint_rows, cus))
     return fail(DLB_ERR_BAD_SHAPE, "GEMM, activation and quantiser apart are the faster way");
   // everything that can refuse the launch is checked before the first pre-pass kernel is enqueued
   if (rs.grid > (1ll << 30)) return fail(DLB_ERR_BAD_SHAPE, "too many tiles (%lld)", (long long)rs.grid);
@@ -1477,7 +1510,7 @@ int run(const Problem& pr) {
       return hipGetLastError();
     }
     if (pl.variant == kVarPipe128x256w8 && pr.act)
-      return launch_ring<Ring128x256, kMaskedAct>(ar, g, dev, pr.stream);  // N / 256 column tiles, as the plain GEMM
+      return launch_ring<Ring128x256, kMaskedAct, true>(ar, g, dev, pr.stream);  // N / 256 column tiles, as the plain GEMM
     if (pl.variant == kVarPipe128x256w8 && rs.sctab) return launch_ring_mode<Ring128x256T>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x256w8) return launch_ring_mode<Ring128x256>(pr.mode, ar, g_dense, dev, pr.stream);
     if (pl.variant == kVarPipe128x128)
@@ -1818,7 +1851,7 @@ int dlb_expert_plan(int mode, int64_t rows, int64_t N, int64_t K, int32_t G, int
     const dlb::Resolved rs = dlb::resolve(dlb::kMasked, rows, N, K, G, dlb::ceil_div(K, dlb::kScaleBlock), 1, workspace_bytes > 0, workspace_bytes,
                                           compute_units, false, quantising != 0, expected_m, true, dlb::kMaxStreamSlices);
     const bool shape_ok = K > 0 && K % dlb::kScaleBlock == 0 && N % (2 * dlb::kScaleBlock) == 0 && N * K < (1ll << 32);
-    *form = shape_ok && dlb::g_forced_variant < 0 && !dlb::steps_apart(rs, rows, N, K, G, expected_m, workspace_bytes, compute_units) ? 1 : 0;
+    *form = shape_ok && dlb::g_forced_variant < 0 && !dlb::steps_apart(rs, rows, N, G, expected_m, compute_units) ? 1 : 0;
   }
   return DLB_OK;
 }

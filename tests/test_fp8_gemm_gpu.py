@@ -712,6 +712,39 @@ def test_grouped_masked_hint_picks_the_tile_shape(dev):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
+@pytest.mark.parametrize('kb,dtype', [(1, torch.bfloat16), (2, torch.float32), (3, torch.bfloat16), (4, torch.float32), (5, torch.bfloat16), (17, torch.bfloat16)])
+def test_masked_tiles_carry_the_ring(dev, kb, dtype):
+    """Six experts of 0 to 300 rows by 25673 columns: every resident workgroup of the masked layout's ring kernels goes through several
+    tiles, whole and ragged ones, of one expert and of the next, at fewer K blocks than the ring has stages, as many, and more
+    (17: more than the scale table of the 128 x 256 tiles holds).  The three tile shapes and the weight-streaming kernel agree
+    bit for bit, rows at or beyond masked_m stay as they were."""
+    from dlblas_amd import _lib
+    from dlblas_amd.kernels.fp8_gemm_grouped import m_grouped_fp8_gemm_nt_masked
+    G, M_max, N, K = 6, 300, 100 * 256 + 73, kb * 128
+    print(f'case masked ring K={K} {dtype}', flush=True)
+    g = torch.Generator(device=dev).manual_seed(50 + kb)
+    masked_m = torch.tensor([300, 0, 1, 256, 129, 64], dtype=torch.int32)
+    a_q, a_s = helpers.quantise_act_device(torch.randn(G * M_max, K, device=dev, generator=g).to(torch.bfloat16))
+    a_q, a_s = a_q.view(G, M_max, K), a_s.view(G, M_max, kb)
+    w_q, w_s = helpers.expert_weights_device(G, N, K, dev, 51)
+    beyond = torch.arange(M_max)[None, :] >= masked_m[:, None]
+    outs = []
+    try:
+        for variant in ('pipe256x256', 'pipe128x256w8', 'pipe128x128', None):
+            out = torch.full((G, M_max, N), 7.0, dtype=dtype, device=dev)
+            _lib.force_variant(variant)
+            m_grouped_fp8_gemm_nt_masked((a_q, a_s), (w_q, w_s), out, masked_m.to(dev), 150)
+            assert torch.all(out[beyond.to(dev)] == 7.0), f'{variant}: rows beyond masked_m were written'
+            outs.append(out)
+    finally:
+        _lib.force_variant(None)
+    for out in outs[1:]:
+        assert torch.equal(outs[0], out)
+    for e, row in ((0, 299), (3, 255), (5, 0)):
+        ref = orc.dequant_ref(a_q[e, row:row + 1].cpu(), a_s[e, row:row + 1].cpu(), w_q[e].cpu(), w_s[e].cpu())
+        helpers.tolerance_check(outs[0][e, row:row + 1], ref, f'masked ring K={K} expert {e}')
+
+
 @pytest.mark.parametrize('K', [384, 2048, 2176])
 def test_grouped_masked_scale_table(dev, K):
     """The masked layout fetches a tile's row-major activation scales once, into a table in LDS, when K has at most 16

@@ -205,6 +205,27 @@ def test_fused_list_tiles_carry_the_ring(dev, kb, gathered):
     assert torch.equal(fused[1], ref_s), 'scales differ'
 
 
+@pytest.mark.parametrize('kb', [1, 2, 3, 4, 8])
+def test_masked_fused_tiles_carry_the_ring(dev, kb):
+    """Experts of 0 to 300 rows by 130 column tiles on the masked layout's ring kernel (the weight-streaming kernel kept out): several
+    tiles per resident workgroup, at fewer K blocks than the ring has stages, as many, and more."""
+    from dlblas_amd import _lib
+    print(f'case fused masked ring K={128 * kb}', flush=True)
+    G, M_max, inter, K = 6, 300, 130 * 128, kb * 128
+    g = torch.Generator(device=dev).manual_seed(70 + kb)
+    a_q, a_s = helpers.quantise_act_device((torch.randn(G * M_max, K, device=dev, generator=g) * 1.5).to(torch.bfloat16))
+    w_q, w_s = helpers.expert_weights_device(G, 2 * inter, K, dev, 71)
+    masked_m = torch.tensor([300, 0, 1, 256, 129, 64], dtype=torch.int32, device=dev)
+    try:
+        _lib.tune('stream', 1)
+        ok, (q, s), (ref_q, ref_s) = _masked_both(dev, a_q.view(G, M_max, K), a_s.view(G, M_max, kb), w_q, w_s, masked_m)
+    finally:
+        _lib.tune('stream', 0)
+    assert ok
+    assert torch.equal(q.view(torch.uint8), ref_q.view(torch.uint8)), 'quantised codes differ'
+    assert torch.equal(s, ref_s), 'scales differ'
+
+
 # --- the fused kernel reading the tokens through the row table of ep_scatter_rows (no expert-sorted copy) ------------
 
 
