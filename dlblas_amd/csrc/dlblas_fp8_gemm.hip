@@ -173,9 +173,12 @@ constexpr int kFusedMaxTiles = DLB_WS_COUNTER_BYTES / 16;  // four counter words
 // Tile shapes of the weight-streaming grouped kernel: rows x weight rows per tile, and the ring each leaves room for.
 typedef StreamCfg<1, 4, 1, 2, 4, 16> Stream32x256;
 typedef StreamCfg<1, 4, 2, 2, 3, 16> Stream64x256;
-typedef StreamCfg<1, 4, 2, 1, 6, 16> Stream64x128;
+typedef StreamCfg<1, 4, 2, 1, 6, 16, true> Stream64x128;
 typedef StreamCfg<2, 4, 2, 2, 3, 11> Stream128x256;
-typedef StreamCfg<2, 2, 1, 1, 9, 16> Stream64x64;
+typedef StreamCfg<2, 2, 1, 1, 9, 16, true> Stream64x64;
+// 256-column tiles with waves apart for the loads: with the quantising epilogue
+typedef StreamCfg<1, 4, 1, 2, 4, 16, true> Stream32x256Apart;
+typedef StreamCfg<1, 4, 2, 2, 3, 16, true> Stream64x256Apart;
 enum StreamShape : int { kStreamNone = -1, kStream32x256 = 0, kStream64x256, kStream64x128, kStream128x256, kStream64x64, kStreamCount };
 struct StreamDims { int bm, bn, stages, ch; };
 constexpr StreamDims kStreamDims[kStreamCount] = {{32, 256, 4, 16}, {64, 256, 3, 16}, {64, 128, 6, 16}, {128, 256, 3, 11}, {64, 64, 9, 16}};
@@ -333,9 +336,12 @@ hipError_t launch_stream_shape(int shape, bool ahead, const Args& args, int grid
       default: break;
     }
   }
+  constexpr bool act = EPI == kSiluQuant || EPI == kSiluQuantMasked;
+  typedef std::conditional_t<act, Stream32x256Apart, Stream32x256> Low;
+  typedef std::conditional_t<act, Stream64x256Apart, Stream64x256> High;
   switch (shape) {
-    case kStream32x256: return launch_stream<Stream32x256, EPI, GATHER, false>(args, grid, dev, stream);
-    case kStream64x256: return launch_stream<Stream64x256, EPI, GATHER, false>(args, grid, dev, stream);
+    case kStream32x256: return launch_stream<Low, EPI, GATHER, false>(args, grid, dev, stream);
+    case kStream64x256: return launch_stream<High, EPI, GATHER, false>(args, grid, dev, stream);
     case kStream128x256: return launch_stream<Stream128x256, EPI, GATHER, false>(args, grid, dev, stream);
     default: return hipErrorInvalidValue;
   }

@@ -34,11 +34,19 @@ namespace dlb {
 // reduction kernel at the end of this file.
 enum StreamEpilogue : int { kStoreProduct = 0, kSiluQuant = 1, kSiluQuantMasked = 2, kStoreSlice = 3 };
 
-template <int WGM_, int WGN_, int MF_, int NF_, int STAGES_, int CH_>
+// SPLIT: as many waves again issue every load, the others only compute and store.  The loads of a step then don't wait for the stores
+// of a tile, which share a wave's memory counter, and the computing waves, whose short steps are mostly issue, carry no address
+// arithmetic.  Their bf16 stores write through the L2: the end of the launch has fewer lines to flush.  us per call without / with:
+// 64 x 64 tiles 8 experts x 0 .. 64 rows x 1792 x 6656 29.7 / 24.3, 16 x 1024 x 2048 12.8 / 10.6, 8 x 0 .. 32 x 1024 x 4096 17.4 / 13.3;
+// 64 x 128 tiles 32 x 0 .. 64 x 7168 x 2048 88.3 / 82.0, 2048 x 7168 85.5 / 79.4, 16 x 1024 x 2048 15.2 / 12.9.  The plain product in
+// 256-column tiles, whose steps are long, loses where K is short (16 x 768 x 1024 10.9 / 11.8) and keeps one kind of wave; with
+// the quantising epilogue it gains 1 %.  Of eight computing waves the registers leave no room for others.
+template <int WGM_, int WGN_, int MF_, int NF_, int STAGES_, int CH_, bool SPLIT_ = false>
 struct StreamCfg {
   static constexpr int WGM = WGM_, WGN = WGN_, MF = MF_, NF = NF_, STAGES = STAGES_;
   static constexpr int WAVES = WGM * WGN;
-  static constexpr int NT = WAVES * 64;
+  static constexpr bool SPLIT = SPLIT_;
+  static constexpr int NT = (SPLIT ? 2 : 1) * WAVES * 64;
   static constexpr int BM = WGM * MF * 32;
   static constexpr int BN = WGN * NF * 32;
   static constexpr int A_INST = BM / 8 / WAVES;
@@ -56,12 +64,14 @@ struct StreamCfg {
   static constexpr int MAX_OFF = ROW_OFF + BM * 4;         // row maxima of the waves (quantising epilogue)
   static constexpr int LDS_BYTES = MAX_OFF + WGN * BM * 4;
   static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "tile rows must divide over the DMA instructions");
+  static_assert(!SPLIT || WAVES == 4, "eight waves share the registers");
   static_assert(WAVES % 2 == 0, "chunk swizzle must not depend on the DMA instruction index");
   static_assert(L * (STAGES - 1) < 64, "vmcnt is a 6-bit counter");
   static_assert(LDS_BYTES <= 160 * 1024, "ring, table and row maxima fit the LDS");
 };
 
 typedef const __attribute__((address_space(4))) float* const_float_ptr_t;
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 // Wait until at most `younger` (0 .. MAX) groups of L vector-memory instructions are on their way.
 template <int L, int MAX>
@@ -96,7 +106,10 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
   static_assert(!kAct || BN == 256, "a quantisation group is the 128 output columns of 256 weight rows");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  constexpr bool kSplit = Cfg::SPLIT;
+  const int wave_id = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const bool loads = kSplit && wave_id >= WAVES;  // this wave issues loads and nothing else
+  const int wave = loads ? wave_id - WAVES : wave_id;
   const int l32 = lane & 31, h = lane >> 5;
   const int wrow = wave / Cfg::WGN;  // the wave's fragment mi is the tile's fragment mi WGM + wrow: wave rows share short tiles evenly
   const LaneChunks lc = make_lane_chunks(l32, h);
@@ -259,24 +272,54 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     open_chunk();
     issue_loads();
   };
+  // kSplit, waves that compute: `it` is the tile after ct
+  auto advance = [&]() { it = locate(it_seq++ * grid + slot0); };
 
   load_window(0, 0);
-  enter_tile();
+  if (kSplit && !loads)
+    advance();
+  else
+    enter_tile();
   if (!it.ok) return;
   Tile ct = it;  // the tile the compute side works on
-  // a tile has at least STAGES K blocks and a chunk at least STAGES - 1.  (Gathered rows in whole steps: the compiler then spills 37 to
-  // 51 scalar registers there in place of 60 to 71, 16 experts x ~48 gathered rows x 3328 x 1792 21.4 -> 21.0 us.)
-  if constexpr (GATHER) {
+  if (!kSplit || loads) {
+    // a tile has at least STAGES K blocks and a chunk at least STAGES - 1.  (Gathered rows in whole steps: the compiler then spills 37 to
+    // 51 scalar registers there in place of 60 to 71, 16 experts x ~48 gathered rows x 3328 x 1792 21.4 -> 21.0 us.)
+    if constexpr (GATHER) {
 #pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s) issue_step();
-  } else {
-    open_chunk();
+      for (int s = 0; s < STAGES - 1; ++s) issue_step();
+    } else {
+      open_chunk();
 #pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s) issue_loads();
+      for (int s = 0; s < STAGES - 1; ++s) issue_loads();
+    }
+    if (AHEAD) {
+      open_chunk();
+      issue_loads();
+    }
   }
-  if (AHEAD) {
-    open_chunk();
-    issue_loads();
+  if constexpr (kSplit) {
+    if (loads) {
+      // in step with the waves that compute, barrier for barrier: of step `done`, and of a tile's quantising epilogue
+      if (AHEAD) {
+        wait_vmcnt<(STAGES - 1) * Cfg::L>();
+        lds_barrier();
+      }
+      int left = p.kblocks;
+      for (int done = 0, issued = STAGES - 1 + (AHEAD ? 1 : 0); done < issued; ++done) {
+        // (AHEAD: the next block's loads have landed; else this one's)
+        wait_groups<Cfg::L, STAGES - 2>(issued - done - (AHEAD ? 2 : 1));
+        lds_barrier();
+        issue_step();
+        if (it.ok) ++issued;
+        if (kAct && --left == 0) {
+          left = p.kblocks;
+          lds_barrier();
+        }
+      }
+      return;
+    }
+    advance();
   }
 
   // ---- compute side ------------------------------------------------------------------------------------------------
@@ -346,7 +389,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
   if constexpr (AHEAD) {
     enter_scales(ct);
     sb0 = bs0[first_kb(ct)], sb1 = bs1[first_kb(ct)];
-    wait_vmcnt<(STAGES - 1) * Cfg::L>();
+    if (!kSplit) wait_vmcnt<(STAGES - 1) * Cfg::L>();
     lds_barrier();
     enter_block(first_kb(ct), true);
 #pragma unroll
@@ -367,7 +410,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
       for (int ni = 0; ni < NF; ++ni) z[ni] = multiply(ni, 0);
       __builtin_amdgcn_sched_barrier(0);
       // the next block's loads have landed, and every wave holds this block in registers: its stage can be refilled
-      wait_vmcnt<(STAGES - 2) * Cfg::L>();
+      if (!kSplit) wait_vmcnt<(STAGES - 2) * Cfg::L>();
       lds_barrier();
       float s0[MF], s1[MF];
 #pragma unroll
@@ -375,7 +418,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
       sb0 = *q0;
       if (kAct) sb1 = *q1;
       else sb1 = sb0;
-      issue_loads();
+      if (!kSplit) issue_loads();
       next_stage();
       ++tab_kb;
       if (MF == 1) {
@@ -421,8 +464,9 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     const bool full = AHEAD && frag_row(MF - 1) < ct.rows;
 
     for (int kb = first_kb(ct); AHEAD && kb < end_kb(ct); ++kb) {
-      if (full && it.ok) {
-        const int n = min(min(end_kb(it), it_chunk_kb) - it_kb, min(end_kb(ct), chunk_end) - 1 - kb);
+      if (full && (kSplit || it.ok)) {
+        int n = min(end_kb(ct), chunk_end) - 1 - kb;
+        if (!kSplit) n = min(n, min(end_kb(it), it_chunk_kb) - it_kb);
         if (n > 0) {
           run_fast(kb, n);
           kb += n;
@@ -443,9 +487,9 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
         }
         if (mi == 0) {
           // younger than the next block's loads: those of STAGES - 2 steps, fewer at the end of the last tile
-          wait_groups<Cfg::L, STAGES - 2>(it.ok ? STAGES - 2 : end_kb(ct) - 2 - kb);
+          if (!kSplit) wait_groups<Cfg::L, STAGES - 2>(it.ok ? STAGES - 2 : end_kb(ct) - 2 - kb);
           lds_barrier();
-          issue_step();
+          if (!kSplit) issue_step();
           next_stage();
           const bool next_tile = kb + 1 == end_kb(ct);
           if (!next_tile) {
@@ -472,9 +516,9 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     if constexpr (!AHEAD) {
       for (int kb = first_kb(ct); kb < end_kb(ct); ++kb) {
         // the loads of this step have landed: behind them at most the groups of the next STAGES - 2 steps are out
-        wait_groups<Cfg::L, STAGES - 2>(it.ok ? STAGES - 2 : end_kb(ct) - 1 - kb);
+        if (!kSplit) wait_groups<Cfg::L, STAGES - 2>(it.ok ? STAGES - 2 : end_kb(ct) - 1 - kb);
         lds_barrier();  // ... those of every wave, and nobody reads the stage before this one any more
-        issue_step();
+        if (!kSplit) issue_step();
         enter_block(kb, kb == first_kb(ct));
         if (WGM == 1 || frag_row(0) < ct.rows) {
           v8i wf[NF][2];
@@ -593,9 +637,16 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
               const auto s0 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.x), static_cast<unsigned>(hi.x), false, false);
               const auto s1 = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(lo.y), static_cast<unsigned>(hi.y), false, false);
               const int n = nf + 8 * u + 8 * h;
-              if (live && n < p.N)
-                *reinterpret_cast<v4i_el*>(c_row + static_cast<int64_t>(n) * 2) =
-                    v4i{static_cast<int>(s0[0]), static_cast<int>(s1[0]), static_cast<int>(s0[1]), static_cast<int>(s1[1])};
+              const v4i c8 = {static_cast<int>(s0[0]), static_cast<int>(s1[0]), static_cast<int>(s0[1]), static_cast<int>(s1[1])};
+              if (live && n < p.N) {
+                if (kSplit && p.N < (1 << 24)) {
+                  // write-through: bit 4 of the policy is sc1
+                  const __amdgpu_buffer_rsrc_t c_rsrc = make_rsrc(static_cast<const uint8_t*>(p.c) + static_cast<int64_t>(ct.row) * p.N * 2, static_cast<uint32_t>(ct.rows * p.N) * 2u);
+                  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, c8), c_rsrc, static_cast<uint32_t>(row * p.N + n) * 2u, 0, 16);
+                } else {
+                  *reinterpret_cast<v4i_el*>(c_row + static_cast<int64_t>(n) * 2) = c8;
+                }
+              }
             }
           } else if (live) {
 #pragma unroll
@@ -613,6 +664,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
     }
     if (!it.ok) break;  // the issue side is one tile ahead: it has found no further one
     ct = it;
+    if (kSplit) advance();
   }
 }
 
