@@ -170,6 +170,12 @@ static_assert(Ring256x192T::LDS_BYTES <= Ring256x256T::LDS_BYTES && Ring256x192:
 static_assert(Pipe128x64T::LDS_BYTES <= 160 * 1024, "ring + table fit the LDS");
 constexpr int kFusedMaxTiles = DLB_WS_COUNTER_BYTES / 16;  // four counter words per tile in the workspace head
 
+// Args::c_whole.  Buffer stores need dwords; plain ones take the elements' own alignment, and c may lie on any element.
+inline int whole_rows(const void* c, int64_t N, bool out_f32) {
+  if (out_f32 || N % 8 != 0) return 0;
+  return !misaligned(c, 4) && N < (1 << 24) ? 2 : 1;
+}
+
 // Tile shapes of the weight-streaming grouped kernel: rows x weight rows per tile, and the ring each leaves room for.
 typedef StreamCfg<1, 4, 1, 2, 4, 16> Stream32x256;
 typedef StreamCfg<1, 4, 2, 2, 3, 16> Stream64x256;
@@ -1287,7 +1293,7 @@ int run_ragged(const RaggedProblem& pr) {
   ar.act_eps = pr.eps;
   ar.act_cols = static_cast<int>(pr.N / 2);
   ar.act_q_stride = pr.N / 2;
-  ar.c_whole = !ar.out_f32 && pr.N % 8 == 0;
+  ar.c_whole = whole_rows(pr.c, pr.N, ar.out_f32);
   if (usable_ws) ar.ws = reinterpret_cast<float*>(static_cast<char*>(pr.ws) + DLB_WS_COUNTER_BYTES);
   const WorkspaceLock lock(pr.ws);
   const hipError_t e = launch_stream_plan(sp, pr.act ? kSiluQuant : kStoreProduct, ar, pr.G + pr.M_sum / kStreamDims[sp.shape].bm,
@@ -1430,7 +1436,7 @@ int run(const Problem& pr) {
   ar.act_eps = pr.act_eps;
   ar.act_cols = static_cast<int>(pr.N / 2);
   ar.act_q_stride = pr.N / 2;
-  ar.c_whole = !ar.out_f32 && pr.N % 8 == 0;
+  ar.c_whole = whole_rows(pr.c, pr.N, ar.out_f32);
   ar.c_lds = g_knob[kKnobEpilogue] != 2;
   if (pr.ws && pr.ws_bytes >= DLB_WS_COUNTER_BYTES) {
     ar.ctr = static_cast<uint32_t*>(pr.ws);

@@ -58,7 +58,8 @@ struct Args {
   int sct_pitch;        // kernels with a scale table in LDS: floats per table row (odd, >= K blocks per workgroup)
   int group_m;          // m-tiles per L2 swizzle group
   int out_f32;
-  int c_whole;          // bf16 c with N % 8 == 0: a group of 8 columns lies inside the row or past it, its store has no tail
+  int c_whole;          // bf16 c with N % 8 == 0: a group of 8 columns lies inside the row or past it, its store has no tail.
+                        // 2: and c lies on dwords, N below 2^24, as a buffer store of such a group needs
   int c_lds;            // ring kernels: results leave through LDS, whole rows per store instruction (else straight from the registers)
   int n_split;          // mixed-width launch: first column of the narrow-tile region
   int tiles_a;          //   tiles in the wide region (tiles_m x tiles_n_a)

@@ -639,7 +639,7 @@ __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_stream_kernel(const Args p) 
               const int n = nf + 8 * u + 8 * h;
               const v4i c8 = {static_cast<int>(s0[0]), static_cast<int>(s1[0]), static_cast<int>(s0[1]), static_cast<int>(s1[1])};
               if (live && n < p.N) {
-                if (kSplit && p.N < (1 << 24)) {
+                if (kSplit && p.c_whole == 2) {
                   // write-through: bit 4 of the policy is sc1
                   const __amdgpu_buffer_rsrc_t c_rsrc = make_rsrc(static_cast<const uint8_t*>(p.c) + static_cast<int64_t>(ct.row) * p.N * 2, static_cast<uint32_t>(ct.rows * p.N) * 2u);
                   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, c8), c_rsrc, static_cast<uint32_t>(row * p.N + n) * 2u, 0, 16);

@@ -70,6 +70,29 @@ def test_masked_equals_the_ring_kernels(dev, masked, M_max, N, K, out_dtype, col
         helpers.tolerance_check(outs[1].cpu()[valid], ref[valid], f'stream {N}x{K}')
 
 
+@pytest.mark.parametrize('masked,M_max,N,K', [([1, 63, 64, 0, 7], 64, 264, 1280), ([70, 128, 33] * 4, 128, 1024, 1152)])
+def test_masked_results_at_an_odd_element(dev, masked, M_max, N, K):
+    """The same bits where the results start on an element that is no dword: kernels that store through buffer descriptors leave
+    such calls to plain stores."""
+    from dlblas_amd import _lib
+    from dlblas_amd.kernels.fp8_gemm_grouped import m_grouped_fp8_gemm_nt_masked
+    a_q, a_s, w_q, w_s, mm = _inputs(masked, M_max, N, K, 80 + N + K, dev)
+    count = len(masked) * M_max * N
+    for knob, shape in zip([2, 3, 4, 5, 6, 8, 9, 10, 11], SHAPES + AHEAD):
+        outs = []
+        for first in (0, 1):
+            print(f'case stream masked={masked[:6]} M_max={M_max} N={N} K={K} shape={shape} first element {first}', flush=True)
+            whole = torch.full((count + 8, ), -555.0, dtype=torch.bfloat16, device=dev)
+            out = whole[first:first + count].view(len(masked), M_max, N)
+            _lib.tune('stream', knob)
+            m_grouped_fp8_gemm_nt_masked((a_q, a_s), (w_q, w_s), out, mm, 0)
+            torch.cuda.synchronize()
+            _lib.tune('stream', 0)
+            assert (whole[:first] == -555.0).all() and (whole[first + count:] == -555.0).all()
+            outs.append(out)
+        assert torch.equal(outs[0], outs[1]), shape
+
+
 @pytest.mark.parametrize('masked,M_max,inter,K', [
     ([1, 32, 33, 0, 128, 64], 128, 256, 512),
     ([130, 5], 160, 128, 2304),
