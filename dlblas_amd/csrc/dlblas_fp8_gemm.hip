@@ -510,14 +510,15 @@ int64_t pick_mixed_split(int64_t M, int64_t N, int cus, double* makespan = nullp
   return best_split;
 }
 
-// Tiles of 256 rows: widths mixed so that the rounds come out even, or all equal?  us on MI355X, 256 ... 4096 rows, K = 384 ... 7168:
-//   - a workgroup per tile (one round, or a mixed launch): 11.5 + 1.62 K blocks per round, the first loads and the output of
-//     every tile included; a mixed launch of several rounds comes out 6 % above the sum of its tiles.
-//   - equal tiles, more than one round: resident workgroups whose ring runs on from tile to tile: 5.4 + 1.82 K blocks per round
-//     and 3 for the launch.
-// A last round that is not full costs 0.6 of a round plus its share of the rest (the chip is faster with fewer tiles).  33
-// launches of 1.1 to 8.8 rounds of equal tiles lie within 7 % of that, mixed ones within 10 %.  The choice, 128-row tiles included, is
-// 0.8 % behind the best of the three (geometric mean of 80 random problems, bench.py --planner-sweep wide_random; 10 % at worst).
+// Tiles of 256 rows: widths mixed so that the rounds come out even, or all equal?  us on MI355X, 256 ... 4096 rows, K = 512 ... 18432:
+//   - a workgroup per tile, one round: 9.6 + 1.26 K blocks, the first loads and the output of the tile included; a mixed launch of
+//     several rounds: 2.1 + 9.3 + 1.52 K blocks per round;
+//   - equal tiles, more than one round: resident workgroups whose ring runs on from tile to tile: 5.4 + 1.53 K blocks per round
+//     and 5.8 for the launch.
+// A last round that is not full costs half of a round (0.7 in a mixed launch, 0.44 in 128 x 256 tiles) plus its share of the rest: the chip is
+// faster with fewer tiles.  43 launches lie within 5 % rms of that.  The choice, 128-row tiles included, is 0.5 % behind
+// the best of the three over 90 random problems it was not fitted to, 6 % at worst (bench.py --planner-sweep wide_random draws such); with the
+// constants of the kernels before these 1.3 % and 14 %.
 // Mixed tiles win where K is long and the last round short (4096 x 5248 x 4096: 104 / 113 us, 2048 x 17408 x 7168: 265 / 292),
 // equal ones where the fixed part of a tile counts (3500 x 33024 x 1280: 203 / 183, 2048 x 18176 x 512: 45 / 38).
 int pick_wide_variant(int64_t M, int64_t N, int kblocks, int cus, double* us = nullptr) {
@@ -525,29 +526,30 @@ int pick_wide_variant(int64_t M, int64_t N, int kblocks, int cus, double* us = n
   const int64_t split = pick_mixed_split(M, N, cus, &span);
   const bool mixed = split < N;
   const int64_t tiles = ceil_div(M, 256) * ceil_div(N, 256);
-  const double lone_us = 11.5 + 1.62 * kblocks, rounds = static_cast<double>(tiles) / cus;
-  const double equal_us = tiles <= cus ? lone_us : 3.0 + (0.4 * rounds + 0.6 * static_cast<double>(ceil_div(tiles, cus))) * (5.4 + 1.82 * kblocks);
+  const double rounds = static_cast<double>(tiles) / cus;
+  const double equal_us = tiles <= cus ? 9.6 + 1.26 * kblocks : 5.8 + (0.49 * rounds + 0.51 * static_cast<double>(ceil_div(tiles, cus))) * (5.4 + 1.53 * kblocks);
   const double load = static_cast<double>(ceil_div(M, 256)) * (split / 256 + 0.78 * static_cast<double>(ceil_div(N - split, 192))) / cus;
-  const double mixed_us = 1.06 * (0.6 * span + 0.4 * load) * lone_us;
+  const double mixed_us = 2.1 + (0.7 * span + 0.3 * load) * (9.3 + 1.52 * kblocks);
   const bool equal = !mixed || equal_us <= mixed_us;
   if (us) *us = equal ? equal_us : mixed_us;
   return mixed && equal ? kVarPipe256x256 : kVarPipe256mix;  // without a narrow region both are the launch of equal tiles
 }
 
 // Prefill-sized dense problems: 256-row tiles (above) or 128 x 256 tiles?  Both run from the L2 at the pace of the matrix
-// pipe there; a round of 128 x 256 tiles takes 2.9 + 1.05 K blocks, its ring runs on from tile to tile as well.
+// pipe there; a round of 128 x 256 tiles takes 2.4 + 0.94 K blocks, its ring runs on from tile to tile as well.
 // The larger tile wins unless its rows are mostly padding (384 rows are two 256-row tiles but three of 128) or its tiles
 // leave much of a round empty (2048 x 4096: 128 tiles of 256 x 256 on 256 CUs, but 256 tiles of 128 x 256):
-// 384 x 18432 x 7168 82 -> 67 us, 2048 x 4096 x 7168 79 -> 67 us.  Up to four K blocks the output decides: fp32, which is not
-// known here, is faster in the smaller tile (2330 x 20000 x 384 54 -> 47 us), bf16 in the larger one (4096 x 32768 x 512
-// 105 against 118), so the smaller one is taken up to 12 % above the estimates, which are of bf16.
+// 384 x 18432 x 7168 82 -> 67 us, 2048 x 4096 x 7168 79 -> 67 us.  bf16 and fp32 results agree about it since both leave from the registers
+// (30 shapes of 2 to 5 K blocks; the smaller tile over the larger one 0.69 .. 1.33 and 0.66 .. 1.20).  The smaller tile is kept up to 7 %
+// above the estimates at three and four K blocks, where they are no closer than that, and up to 20 % below three, which were not fitted.
 bool prefers_128_row_tiles(int64_t M, int64_t N, int kblocks, int cus, double* us = nullptr) {
   double wide_us = 0.0;
   pick_wide_variant(M, N, kblocks, cus, &wide_us);
-  const int64_t rounds = ceil_div(ceil_div(M, 128) * ceil_div(N, 256), cus);
-  const double half_us = 3.0 + static_cast<double>(rounds) * (2.9 + 1.05 * kblocks);
+  const int64_t tiles = ceil_div(M, 128) * ceil_div(N, 256);
+  const double rounds = 0.56 * static_cast<double>(tiles) / cus + 0.44 * static_cast<double>(ceil_div(tiles, cus));
+  const double half_us = 5.5 + rounds * (2.4 + 0.94 * kblocks);
   if (us) *us = std::min(wide_us, half_us);
-  return half_us < (kblocks <= 4 ? 1.12 : 0.95) * wide_us;
+  return half_us < (kblocks <= 2 ? 1.2 : kblocks <= 4 ? 1.07 : 1.0) * wide_us;
 }
 
 struct Plan {
@@ -885,12 +887,15 @@ int pick_wavek(int64_t M, int64_t N, int64_t K, int cus, size_t ws_bytes) {
   if (best == kWaveKNone || knob >= 2 || M <= 64 || ragged) return best;
   const size_t ws_avail = ws_bytes > DLB_WS_COUNTER_BYTES ? ws_bytes - DLB_WS_COUNTER_BYTES : 0;
   double other;
-  if (M > 128 && ceil_div(M, 256) * ceil_div(N, 256) * 2 >= cus)
+  const bool wide = M > 128 && ceil_div(M, 256) * ceil_div(N, 256) * 2 >= cus;
+  if (wide)
     prefers_128_row_tiles(M, N, kblocks, cus, &other);
   else
     other = pick_mid_plan(M, N, kblocks, cus, ws_avail).us;
   if (M <= 128) other = std::min(other, 1.3 * decode_us(M, N, K, kblocks, cus));  // (the 128-row decode kernel runs above its estimate at short K)
-  return best_us < 0.95 * other ? best : kWaveKNone;
+  // (where tiles of 256 columns fill half of the chip or more, this kernel's estimate is the lower one at short K and its time is not: 1326 x
+  // 5696 x 512 12.7 us for 11.0, 1883 x 9088 x 512 24.0 for 21.4, 259 x 27200 x 1920 30.5 for 28.5; over 55 problems it won none by 1 %)
+  return best_us < (wide ? 0.85 : 0.95) * other ? best : kWaveKNone;
 }
 
 // K blocks per chunk of the streaming kernel's scale table: equal chunks of at most `ch` blocks, none shorter than the
