@@ -60,7 +60,7 @@ struct Args {
   int out_f32;
   int c_whole;          // bf16 c with N % 8 == 0: a group of 8 columns lies inside the row or past it, its store has no tail.
                         // 2: and c lies on dwords, N below 2^24, as a buffer store of such a group needs
-  int c_lds;            // ring kernels: results leave through LDS, whole rows per store instruction (else straight from the registers)
+  int c_lds;            // 128 x 64 kernel: results leave through LDS, whole rows per store instruction (else straight from the registers); ring kernels: a dense ring may run on
   int n_split;          // mixed-width launch: first column of the narrow-tile region
   int tiles_a;          //   tiles in the wide region (tiles_m x tiles_n_a)
   int tiles_n_a;

@@ -16,7 +16,8 @@
 //     is involved, so the ring runs on from tile to tile (AHEAD) in every layout.  A tile with the quantising epilogue shares
 //     nothing but its rows' largest magnitudes through LDS, where the whole tile used to pass in bf16.
 // 4096 x 8192 x 18432 in 256 x 256 tiles: 505 us with 32 x 32 MFMAs and one hand-over per step, 471 us in this form
-// (2.62 PFLOP/s); its K steps take 2740 cycles of which 2048 are MFMA.  Without the scale FMAs it would be 421 us.
+// (2.62 PFLOP/s); its K steps take 2740 cycles of which 2048 are MFMA.  Without the scale FMAs it would be 421 us.  (All before
+// ring_swizzle had its present form, which is worth 2 % more.)
 // Expert-contiguous lists, 32 experts, 8192 rows, 4096 x 7168: 330 us per call with the former kernels (32 x 32 MFMAs, results
 // through LDS, a ring that drained between tiles), 306 us with these; the whole expert MLP on 8192 tokens 589 -> 532 us, of
 // which the ring that runs on is 5.
