@@ -12,7 +12,8 @@
 //     more, where a single hand-over leaves the last of a group 0.4.  Loads are issued one in two MFMA slots; in one burst
 //     they cost 3 %.
 //   - fragments take every other group of four rows, so that a lane's two results of a pair of fragments are 8 consecutive
-//     columns: results go from the registers to memory in 16-byte pieces, 64 or 128 bytes of a row per instruction.  No LDS
+//     columns: results go from the registers to memory in 16-byte pieces, 128 or 256 bytes of a row per instruction (lanes exchange chunks
+//     through DPP first).  No LDS
 //     is involved, so the ring runs on from tile to tile (AHEAD) in every layout.  A tile with the quantising epilogue shares
 //     nothing but its rows' largest magnitudes through LDS, where the whole tile used to pass in bf16.
 // 4096 x 8192 x 18432 in 256 x 256 tiles: 505 us with 32 x 32 MFMAs and one hand-over per step, 471 us in this form
@@ -697,77 +698,63 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
       // fp32 also for the first pass of split-K: the slice's sums as an [M][N] matrix of their own in the workspace, which
       // fp8_splitk_reduce_kernel, launched behind this kernel on the same stream, adds in index order
       const bool cols_inside = t.n0 + wn0 + NF * 16 <= p.N;  // no column of the wave's tile lies past N: stores without a tail
-      // fp32 rows and bf16 rows at any address: the four lanes of consecutive rows exchange chunks first, so that an instruction writes
-      // 256 bytes (128 in narrower wave tiles) of a row instead of 64 in pieces.  us per call, both on one GPU: bf16 914 x 28119 x 512 38.8 -> 32.4,
-      // 3779 x 6111 x 1024 45.4 -> 36.3, 2000 x 5001 x 4096 52.0 -> 47.6; fp32 914 x 28120 x 512 39.3 -> 32.1, 271 x 18112 x 640 13.9 -> 12.0.
-      auto store_tile = [&](auto f32, auto whole, auto inside, void* out) __attribute__((always_inline)) {
-        constexpr bool F32 = decltype(f32)::value, WHOLE = decltype(whole)::value;
+      // The four lanes of consecutive rows exchange chunks first, so that an instruction writes 256 bytes (128 in narrower wave tiles) of a
+      // row instead of 64, or of 16-byte pieces of fp32.  us per call, both on one GPU: bf16 rows at odd addresses 914 x 28119 x 512 38.8 ->
+      // 32.4, 3779 x 6111 x 1024 45.4 -> 36.3, 2000 x 5001 x 4096 52.0 -> 47.6; fp32 914 x 28120 x 512 39.3 -> 32.1, 271 x 18112 x 640 13.9 ->
+      // 12.0; bf16 rows on 16 bytes 271 x 18112 x 640 11.1 -> 10.1, 3500 x 4096 x 512 15.1 -> 14.2, 4096 x 24576 x 1536 141 -> 138.
+      auto store_tile = [&](auto f32, auto inside, void* out) __attribute__((always_inline)) {
+        constexpr bool F32 = decltype(f32)::value;
         const int col = t.n0 + wn0 + eq * 8;
 #pragma unroll
         for (int mi = 0; mi < MF; ++mi) {
-          if constexpr (F32 || !WHOLE) {
-            // chunk `at` columns into the lane's first, of row r of the lane's four
-            auto put = [&](int r, int at, v4i v) __attribute__((always_inline)) {
-              const int m = t.m0 + e_row - (el & 3) + r + ring_row(mi, 0);
-              if (m >= t.m_end) return;
-              char* dst = static_cast<char*>(out) + (static_cast<int64_t>(m) * p.N + col) * (F32 ? 4 : 2);
-              const int n_left = p.N - col - at;
-              if constexpr (F32)
-                store_row4<true>(dst, at, __builtin_bit_cast(v4f, v), inside ? 4 : n_left);
-              else if (inside || n_left > 0)
-                store_row8_bf16(reinterpret_cast<__bf16*>(dst) + at, v, inside ? 8 : n_left);
-            };
-            constexpr int CHUNKS = F32 ? NF : NF / 2, kFour = CHUNKS / 4 * 4;
-            auto chunk = [&](int c) __attribute__((always_inline)) {
-              if constexpr (F32) {
-                return __builtin_bit_cast(v4i, acc[mi][c]);
-              } else {
-                const v4bf lo = __builtin_convertvector(acc[mi][2 * c], v4bf), hi = __builtin_convertvector(acc[mi][2 * c + 1], v4bf);
-                const v2i a = __builtin_bit_cast(v2i, lo), b = __builtin_bit_cast(v2i, hi);
-                return v4i{a.x, a.y, b.x, b.y};
-              }
-            };
-            auto chunk_col = [](int c) __attribute__((always_inline)) { return F32 ? (c >> 1) * 32 + (c & 1) * 4 : c * 32; };
-            const int j = el & 3;
-#pragma unroll
-            for (int c = 0; c < kFour; c += 4) {
-              v4i x[4] = {chunk(c), chunk(c + 1), chunk(c + 2), chunk(c + 3)};
-              swap_chunks<1>(x[0], x[1], el), swap_chunks<1>(x[2], x[3], el);
-              swap_chunks<2>(x[0], x[2], el), swap_chunks<2>(x[1], x[3], el);
-#pragma unroll
-              for (int r = 0; r < 4; ++r) put(r, chunk_col(c) + chunk_col(j), x[r]);
-            }
-#pragma unroll
-            for (int c = kFour; c + 1 < CHUNKS; c += 2) {
-              v4i x[2] = {chunk(c), chunk(c + 1)};
-              swap_chunks<1>(x[0], x[1], el);
-#pragma unroll
-              for (int r = 0; r < 2; ++r) put((j & 2) + r, chunk_col(c) + chunk_col(j & 1), x[r]);
-            }
-            if constexpr (CHUNKS % 2 != 0) put(j, chunk_col(CHUNKS - 1), chunk(CHUNKS - 1));
-          } else {
-            const int m = t.m0 + e_row + ring_row(mi, 0);
-            if (m >= t.m_end) continue;
-            char* dst = static_cast<char*>(out) + (static_cast<int64_t>(m) * p.N + col) * 2;
-#pragma unroll
-            for (int np = 0; np < NF / 2; ++np) {
-              const int n_left = p.N - col - np * 32;
-              const v4bf lo = __builtin_convertvector(acc[mi][2 * np], v4bf), hi = __builtin_convertvector(acc[mi][2 * np + 1], v4bf);
+          // chunk `at` columns into the lane's first, of row r of the lane's four
+          auto put = [&](int r, int at, v4i v) __attribute__((always_inline)) {
+            const int m = t.m0 + e_row - (el & 3) + r + ring_row(mi, 0);
+            if (m >= t.m_end) return;
+            char* dst = static_cast<char*>(out) + (static_cast<int64_t>(m) * p.N + col) * (F32 ? 4 : 2);
+            const int n_left = p.N - col - at;
+            if constexpr (F32)
+              store_row4<true>(dst, at, __builtin_bit_cast(v4f, v), inside ? 4 : n_left);
+            else if (inside || n_left > 0)
+              store_row8_bf16(reinterpret_cast<__bf16*>(dst) + at, v, inside ? 8 : n_left);
+          };
+          constexpr int CHUNKS = F32 ? NF : NF / 2, kFour = CHUNKS / 4 * 4;
+          auto chunk = [&](int c) __attribute__((always_inline)) {
+            if constexpr (F32) {
+              return __builtin_bit_cast(v4i, acc[mi][c]);
+            } else {
+              const v4bf lo = __builtin_convertvector(acc[mi][2 * c], v4bf), hi = __builtin_convertvector(acc[mi][2 * c + 1], v4bf);
               const v2i a = __builtin_bit_cast(v2i, lo), b = __builtin_bit_cast(v2i, hi);
-              if (inside || n_left > 0) store_row8_bf16(reinterpret_cast<__bf16*>(dst) + np * 32, v4i{a.x, a.y, b.x, b.y}, inside ? 8 : n_left);
+              return v4i{a.x, a.y, b.x, b.y};
             }
+          };
+          auto chunk_col = [](int c) __attribute__((always_inline)) { return F32 ? (c >> 1) * 32 + (c & 1) * 4 : c * 32; };
+          const int j = el & 3;
+#pragma unroll
+          for (int c = 0; c < kFour; c += 4) {
+            v4i x[4] = {chunk(c), chunk(c + 1), chunk(c + 2), chunk(c + 3)};
+            swap_chunks<1>(x[0], x[1], el), swap_chunks<1>(x[2], x[3], el);
+            swap_chunks<2>(x[0], x[2], el), swap_chunks<2>(x[1], x[3], el);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) put(r, chunk_col(c) + chunk_col(j), x[r]);
           }
+#pragma unroll
+          for (int c = kFour; c + 1 < CHUNKS; c += 2) {
+            v4i x[2] = {chunk(c), chunk(c + 1)};
+            swap_chunks<1>(x[0], x[1], el);
+#pragma unroll
+            for (int r = 0; r < 2; ++r) put((j & 2) + r, chunk_col(c) + chunk_col(j & 1), x[r]);
+          }
+          if constexpr (CHUNKS % 2 != 0) put(j, chunk_col(CHUNKS - 1), chunk(CHUNKS - 1));
         }
       };
       void* out = sliced ? static_cast<void*>(p.ws + static_cast<int64_t>(t.split) * p.M * p.N) : static_cast<void*>(c_base);
       constexpr std::true_type yes{};
       constexpr std::false_type no{};
       if (sliced || p.out_f32)
-        cols_inside ? store_tile(yes, no, yes, out) : store_tile(yes, no, no, out);
-      else if (p.c_whole)
-        cols_inside ? store_tile(no, yes, yes, out) : store_tile(no, yes, no, out);
+        cols_inside ? store_tile(yes, yes, out) : store_tile(yes, no, out);
       else
-        cols_inside ? store_tile(no, no, yes, out) : store_tile(no, no, no, out);
+        cols_inside ? store_tile(no, yes, out) : store_tile(no, no, out);
     }
     if (!AHEAD || !ahead) wait_vmcnt<0>();  // the empty groups behind the end of K must not land in the next tile's ring
     t = tn, have = more;
