@@ -361,19 +361,19 @@ def ceilings(dev):
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
     g = torch.Generator().manual_seed(20)
-    codes = torch.randint(0, 256, (12288, ), generator=g, dtype=torch.uint8)
+    codes = torch.randint(0, 256, (16384, ), generator=g, dtype=torch.uint8)
     codes[(codes & 0x7f) == 0x7f] = 0x30                       # no NaN codes
-    operands = {'constant 1.0': torch.full((12288, ), 0x38, dtype=torch.uint8).to(dev), 'random e4m3 codes': codes.to(dev)}
+    operands = {'constant 1.0': torch.full((16384, ), 0x38, dtype=torch.uint8).to(dev), 'random e4m3 codes': codes.to(dev)}
     sink = torch.empty(cus * 512, dtype=torch.float32, device=dev)
     iters = 400                                                 # ~1 ms per launch
-    flop = cus * 8.0 * iters * 16 * 131072
+    flop = cus * 8.0 * iters * 2097152
     res = {'mfma_loop_TFLOPs': {}, 'panel_stream_GBps': {}}
     for name, buf in operands.items():
-        for reads in (0, 3):
-            def run(buf=buf, reads=reads):
-                lib.floor_mfma(ctypes.c_void_p(buf.data_ptr()), ctypes.c_void_p(sink.data_ptr()), cus, iters, reads, stream)
+        for form, what in enumerate(('pairs of 32x32x64', '16x16x128', '16x16x128, fragments read from LDS')):
+            def run(buf=buf, form=form):
+                lib.floor_mfma(ctypes.c_void_p(buf.data_ptr()), ctypes.c_void_p(sink.data_ptr()), cus, iters, form, stream)
             ms = time_call(run, 40, 100)
-            res['mfma_loop_TFLOPs'][f'{name}, {reads} ds_read_b128 per MFMA pair'] = flop / ms / 1e9
+            res['mfma_loop_TFLOPs'][f'{name}, {what}'] = flop / ms / 1e9
     # 256-row panels of a [65536, 7168]-byte matrix (470 MB: past the 256 MB cache), the rows of one expert's weight tile
     panels, row_bytes = 256, 7168
     mat = torch.randint(0, 255, (panels * 256 * row_bytes, ), dtype=torch.uint8, device=dev)
@@ -412,8 +412,8 @@ def ceilings(dev):
             res['l2_stream'][f'{name}, {depth} K steps in flight'] = {'GBps_per_cu': steps_per_launch * 65536 / ms / 1e6,
                                                                        'ns_per_64KB_step': ms * 1e6 / steps_per_launch}
     res['note'] = ('l2_stream: one workgroup per CU, every request an L2 hit after the first touch (the prefill kernel moves 64 KB '
-                   'per K step of about 1600 ns). mfma_loop: pairs of v_mfma_f32_32x32x64_f8f6f4 + 16 scale FMAs from registers, 8 waves per CU, no memory '
-                   'traffic except the optional LDS reads (the prefill kernel issues 3 per pair); peak 5000 TFLOP/s. '
+                   'per K step of about 1400 ns). mfma_loop: the products and scale FMAs of a 64 x 128 wave tile, 8 waves per CU, operands in '
+                   'registers or (the 24 ds_read_b128 of a K step, as in the prefill kernels) from LDS, nothing else; peak 5000 TFLOP/s. '
                    'panel_stream: one workgroup per CU pulls 256 x 7168-byte panels from HBM through the LDS DMA path, '
                    '128 bytes per row and K step, and computes nothing')
     return res

@@ -4,10 +4,11 @@
 //                queue (dependent launches on one stream)
 //   floor_read   every byte of the weight matrix read once with 16-byte loads, nothing else: launch cost + the time the
 //                memory system needs to deliver the bytes to 256 workgroups
-//   floor_mfma   the prefill kernel's arithmetic from registers only: pairs of v_mfma_f32_32x32x64_f8f6f4 (first of a
-//                pair on a zero accumulator) + 16 scale FMAs per pair, two waves per SIMD, optionally with the kernel's
-//                rate of LDS fragment reads (3 ds_read_b128 per pair) whose data nobody waits for.  The operands come
-//                from the caller, so the same loop runs on constant and on random e4m3 codes
+//   floor_mfma   the prefill kernels' arithmetic and nothing else, two waves per SIMD: MFMAs on a zero accumulator, scale FMAs two MFMAs
+//                behind.  Form 1: the kernels' 16 x 16 x 128, 32 of them and 128 FMAs per K step of a 64 x 128 wave tile, from registers;
+//                form 2: the same with every fragment read from LDS, at the kernels' distance ahead of its use; form 0: the same
+//                products as pairs of 32 x 32 x 64 from registers.  The operands come from the caller, so that the same loop runs on
+//                constant and on random e4m3 codes
 //   floor_panel_stream  one workgroup per CU streams 256-row panels of a row-major byte matrix through the LDS DMA path
 //                (global_load_lds_dwordx4, 8 rows x 128 bytes per wave instruction, K step by K step, S steps in
 //                flight) and does nothing with them: the rate at which a CU can pull a weight tile's rows from HBM
@@ -20,6 +21,7 @@
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef const __attribute__((address_space(1))) void* global_ptr_t;
@@ -69,45 +71,75 @@ __global__ void __launch_bounds__(512) floor_read_store_kernel(const v4i* src, i
   for (int64_t t = threadIdx.x; t < per_wg; t += 512) out[static_cast<int64_t>(blockIdx.x) * per_wg + t] = mixed;
 }
 
-// R = ds_read_b128 per MFMA pair (0 or 3).  in: 6 x 64 x 32 bytes of e4m3 codes (4 "A" + 2 "B" operand registers per lane).
-template <int R>
-__global__ void __launch_bounds__(512) floor_mfma_kernel(const v8i* in, float* out, int iters, float scale) {
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  for (int i = threadIdx.x; i < 65536 / 4; i += 512) reinterpret_cast<int*>(lds)[i] = 0x38383838;
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = lane & 31, half = lane >> 5, swz = (row & 7) ^ ((row >> 3) & 1);
-  int addr[3];
-  for (int i = 0; i < 3; ++i) addr[i] = wave * 8192 + row * 128 + ((((i >> 1) * 4 + 2 * half + (i & 1)) ^ swz) << 4);
+// in: 8 x 64 x 32 bytes of e4m3 codes
+__global__ void __launch_bounds__(512) floor_mfma_pairs_kernel(const v8i* in, float* out, int iters, float scale) {
+  const int lane = threadIdx.x & 63;
   v8i a[4], b[2];
   for (int i = 0; i < 4; ++i) a[i] = in[lane + 64 * i];
   for (int i = 0; i < 2; ++i) b[i] = in[lane + 64 * (4 + i)];
   v16f acc[4], part[2];
   for (int j = 0; j < 16; ++j) acc[0][j] = acc[1][j] = acc[2][j] = acc[3][j] = part[0][j] = part[1][j] = 0.0f;
-  v4i d[3] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
   for (int it = 0; it < iters; ++it) {
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-      if (t == 4) asm volatile("" : "+v"(a[0][0]), "+v"(a[1][0]), "+v"(a[2][0]), "+v"(a[3][0]));  // pairs 4..7 are not copies of 0..3
+      if (t % 4 == 0) asm volatile("" : "+v"(a[0][0]), "+v"(a[1][0]), "+v"(a[2][0]), "+v"(a[3][0]));  // no four pairs are copies of others
       __builtin_amdgcn_sched_barrier(0);
       v16f z;
       for (int j = 0; j < 16; ++j) z[j] = 0.0f;
       z = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[t & 3], b[0], z, 0, 0, 0, 0, 0, 0);
       part[t & 1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[(t + 1) & 3], b[1], z, 0, 0, 0, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int r = 0; r < R; ++r) asm volatile("ds_read_b128 %0, %1" : "=v"(d[r]) : "v"(addr[r] + (t & 1) * 4096));
-      __builtin_amdgcn_sched_barrier(0);
       acc[(t + 3) & 3] += part[(t + 1) & 1] * scale;  // the scale FMAs of the previous pair
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    // fold the (constant) LDS data in and move the operands a little, so that no iteration is a copy of another
-    a[0][0] ^= it ^ (d[0].x ^ d[1].y ^ d[2].z ^ 0x38383838 ^ (R == 0 ? 0x38383838 : 0));
-    b[0][1] += 0x01010101;
   }
   float r = 0.0f;
   for (int i = 0; i < 4; ++i)
     for (int j = 0; j < 16; ++j) r += acc[i][j];
+  out[blockIdx.x * 512 + threadIdx.x] = r;
+}
+
+// in: as above.  LDS: a 64 KB copy of it, read row by row as 128-byte rows of K; the reads are ordinary loads, whose waits the compiler places.
+template <bool LDS>
+__global__ void __launch_bounds__(512) floor_mfma_kernel(const v8i* in, float* out, int iters, float scale) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (LDS) {
+    for (int i = threadIdx.x; i < 65536 / 16; i += 512) reinterpret_cast<v4i*>(lds)[i] = reinterpret_cast<const v4i*>(in)[i % 1024];
+    __syncthreads();
+  }
+  // fragment f of a stage: rows f / 2 * 32 + f % 2 * 4 + ..., chunk pattern without bank conflicts, as in the ring kernels
+  const int row = ((lane & 15) >> 2) * 8 + (lane & 3), q = lane >> 4;
+  const int at = row * 128 + (((((q & 1) * 2 + (q >> 1)) ^ ((row & 2) | ((row >> 3) & 1) | ((row >> 2) & 4))) & 7) << 4);
+  auto read = [&](int stage, int f) {  // stage: 0 or 1, 32 KB each; held fragments are 0 .. 3, streamed ones 4 .. 11
+    const int base = stage * 32768 + (wave & 3) * 1024 + f / 2 * 4096 + f % 2 * 512 + at;  // ends at 60416 at most
+    const v4i lo = *reinterpret_cast<const v4i*>(lds + base), hi = *reinterpret_cast<const v4i*>(lds + (base ^ 64));
+    return v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+  };
+  v8i held[4], strm[4];
+  for (int i = 0; i < 4; ++i) held[i] = in[lane + 64 * i], strm[i] = in[lane + 64 * (4 + i)];
+  v4f acc[4][8], part[4];
+  for (int i = 0; i < 4; ++i) {
+    part[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < 8; ++j) acc[i][j] = part[i];
+  }
+  for (int it = 0; it < iters; ++it) {
+#pragma unroll
+    for (int s = 0; s < 32; ++s) {
+      const int n = s / 4, m = s % 4, behind = (s + 30) % 32;
+      if (!LDS && s % 16 == 0) asm volatile("" : "+v"(held[0][0]), "+v"(held[1][0]), "+v"(held[2][0]), "+v"(held[3][0]));  // no 16 products are copies of others
+      __builtin_amdgcn_sched_barrier(0);
+      part[s % 4] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(strm[n % 4], held[m], v4f{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (LDS && m == 0) strm[(n + 3) % 4] = read((it + (n + 3) / 8) & 1, 4 + (n + 3) % 8);
+      if (LDS && n == 7) held[m] = read((it + 1) & 1, m);
+      __builtin_amdgcn_sched_barrier(0);
+      acc[behind % 4][behind / 4] += part[behind % 4] * scale;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  float r = 0.0f;
+  for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < 8; ++j) r += acc[i][j].x + acc[i][j].y + acc[i][j].z + acc[i][j].w;
   out[blockIdx.x * 512 + threadIdx.x] = r;
 }
 
@@ -239,17 +271,19 @@ int floor_read_store(const void* src, int64_t bytes, int workgroups, int loads_i
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// operands: 12288 bytes of e4m3 codes on the device; out: workgroups * 512 floats.  FLOP per launch =
-// workgroups * 8 waves * iters * 16 MFMAs * 131072.
-int floor_mfma(const void* operands, float* out, int workgroups, int iters, int lds_reads, void* stream) {
+// operands: 16384 bytes of e4m3 codes on the device; out: workgroups * 512 floats; form 0, 1 or 2 (above).  FLOP per launch =
+// workgroups * 8 waves * iters * 2097152 in every form.
+int floor_mfma(const void* operands, float* out, int workgroups, int iters, int form, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   const v8i* in = static_cast<const v8i*>(operands);
-  hipFuncSetAttribute(reinterpret_cast<const void*>(floor_mfma_kernel<3>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536);
-  hipFuncSetAttribute(reinterpret_cast<const void*>(floor_mfma_kernel<0>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536);
-  if (lds_reads > 0)
-    hipLaunchKernelGGL(floor_mfma_kernel<3>, dim3(workgroups), dim3(512), 65536, st, in, out, iters, 1.5f);
-  else
-    hipLaunchKernelGGL(floor_mfma_kernel<0>, dim3(workgroups), dim3(512), 65536, st, in, out, iters, 1.5f);
+  if (form == 0) {
+    hipLaunchKernelGGL(floor_mfma_pairs_kernel, dim3(workgroups), dim3(512), 0, st, in, out, iters, 1.5f);
+  } else if (form == 1) {
+    hipLaunchKernelGGL(floor_mfma_kernel<false>, dim3(workgroups), dim3(512), 0, st, in, out, iters, 1.5f);
+  } else {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(floor_mfma_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, 65536) != hipSuccess) return -1;
+    hipLaunchKernelGGL(floor_mfma_kernel<true>, dim3(workgroups), dim3(512), 65536, st, in, out, iters, 1.5f);
+  }
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
