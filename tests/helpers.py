@@ -120,3 +120,15 @@ def expert_weights_device(G, N, K, dev, seed):
         qs.append(q)
         ss.append(s)
     return torch.stack(qs), torch.stack(ss)
+
+
+def list_cut(blocks, tiles_n, grid):
+    """(256-row, 192-row) tiles that the tile-list kernel runs as 64-row pieces on `grid` workgroups, experts with runs of `blocks` blocks:
+    those of a last round that would hold too few whole tiles.  Runs of 1 block are 128-row tiles, even ones 256-row tiles, odd
+    ones end in two 192-row tiles."""
+    tall = tiles_n * sum(r // 2 if r % 2 == 0 else (r - 3) // 2 for r in blocks if r > 1)
+    middle = tiles_n * sum(2 for r in blocks if r % 2 and r > 1)
+    rest = (tall + middle + tiles_n * blocks.count(1)) % grid
+    if rest <= tall:
+        return (rest if 4 * rest <= grid else 0), 0
+    return 0, (rest if rest <= middle and 3 * rest <= grid else 0)

@@ -31,6 +31,29 @@ def _run_dense(dev, a_q, a_s, b_q, b_s, dtype=torch.bfloat16, variant=None):
     return out
 
 
+def _run_dense_guarded(dev, a_q, a_s, b_q, b_s, dtype=torch.bfloat16, variant=None, first=0):
+    """The result written from element `first` of a buffer on; the elements before and behind it have to stay as they were."""
+    import ctypes
+
+    from dlblas_amd import _lib
+    (M, K), N, vp = a_q.shape, b_q.size(0), ctypes.c_void_p
+    a, b, sa, sb = (t.to(dev) for t in (a_q, b_q, a_s, b_s))
+    whole = torch.full((first + M * N + 64, ), -777.0, dtype=dtype, device=dev)
+    stream = torch.cuda.current_stream().cuda_stream
+    ws = _lib.workspace(dev, stream)
+    try:
+        _lib.force_variant(variant)
+        rc = _lib.load().dlb_fp8_gemm(vp(a.data_ptr()), vp(b.data_ptr()), vp(sa.data_ptr()), vp(sb.data_ptr()),
+                                      vp(whole.data_ptr() + first * whole.element_size()), M, N, K, sa.stride(0), sa.stride(1),
+                                      _lib.OUT_F32 if dtype == torch.float32 else _lib.OUT_BF16, vp(ws.data_ptr()), ws.numel(), vp(stream))
+        torch.cuda.synchronize()
+    finally:
+        _lib.force_variant(None)
+    assert rc == 0, _lib.last_error()
+    assert bool((whole[:first] == -777.0).all()) and bool((whole[first + M * N:] == -777.0).all()), f'{variant}: written beside the result'
+    return whole[first:first + M * N].view(M, N)
+
+
 DENSE_SHAPES = [
     (64, 512, 1024),      # the reference's CPU-runnable configuration
     (512, 512, 512),      # the shape of tests/kernels/test_fp8_gemm.py
@@ -203,14 +226,16 @@ def test_tiles_of_a_resident_workgroup(dev, variant, M, kb, dtype):
     helpers.tolerance_check(outs[0], orc.dequant_ref(a_q, a_s, b_q, b_s), f'resident tiles {variant} K={K}')
 
 
-@pytest.mark.parametrize('variant,M,kb', [('pipe256x256', 2052, kb) for kb in (2, 3, 5, 28)] + [('pipe128x256w8', 1028, kb) for kb in (3, 4, 5, 17)])
+@pytest.mark.parametrize('variant,M,kb', [('pipe256x256', 2052, kb) for kb in (2, 3, 5, 28)] + [('pipe128x256w8', 1028, kb) for kb in (3, 4, 5, 17)] +
+                         [('pipe128x128', 1028, kb) for kb in (3, 4, 5, 54, 55)])
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
 def test_ring_runs_on_through_three_tiles(dev, variant, M, kb, dtype):
-    """9 x 87 tiles on 256 workgroups, the last ones 4 rows high and 84 columns wide: tiles that start from a carried ring and carry
-    it on, at as many K blocks as the ring has stages, one more, and counts that are no multiple of them, with the scale table (up
-    to 27 / 16 blocks) and without.  The bits of the same kernel without the carry, which stores through LDS alone take."""
+    """9 x 87 tiles of 256 columns or 9 x 73 of 128 on 256 workgroups, the last ones 4 rows high and 84 columns wide: tiles that start
+    from a carried ring and carry it on, at as many K blocks as the ring has stages, one more, and counts that are no multiple of them,
+    with the scale table (up to 27 / 16 / 54 blocks) and without.  The bits of the same kernel whose tiles start with an empty ring, which
+    the knob asks for."""
     from dlblas_amd import _lib
-    N, K = 22100, kb * 128
+    N, K = 9300 if variant == 'pipe128x128' else 22100, kb * 128
     print(f'case three tiles {variant} K={K} {dtype}', flush=True)
     a_q, a_s, b_q, b_s = helpers.make_dense(M, N, K, seed=kb)
     carried = _run_dense(dev, a_q, a_s, b_q, b_s, dtype=dtype, variant=variant)
@@ -287,8 +312,9 @@ def test_short_k_takes_its_scales_from_the_table(dev, M, N, K):
 @pytest.mark.parametrize('variant', ['pipe256x256', 'pipe128x256w8', 'pipe256mix', 'pipe128x128', 'pipe128x64'])
 @pytest.mark.parametrize('M,N,K', [(200, 392, 2048), (513, 1032, 256)])
 def test_epilogue_through_lds_equals_direct_stores(dev, variant, M, N, K):
-    """bf16 results of the pipelined kernels leave through an LDS transpose (whole rows per store instruction) or, by
-    knob, straight from the accumulator registers: the same fp32 values, the same rounding, the same bits."""
+    """bf16 results of the 128 x 64 kernel leave through an LDS transpose (whole rows per store instruction) or, by knob, straight from
+    the accumulator registers; those of the ring kernels from the registers, after lanes have exchanged pieces: the same fp32
+    values, the same rounding, the same bits."""
     from dlblas_amd import _lib
     print(f'case epilogue variant={variant} M={M} N={N} K={K}', flush=True)
     a_q, a_s, b_q, b_s = helpers.make_dense(M, N, K, seed=23)
@@ -297,30 +323,34 @@ def test_epilogue_through_lds_equals_direct_stores(dev, variant, M, N, K):
         direct = _run_dense(dev, a_q, a_s, b_q, b_s, variant=variant)
     finally:
         _lib.tune('epilogue', 0)
-    staged = _run_dense(dev, a_q, a_s, b_q, b_s, variant=variant)
+    staged = _run_dense(dev, a_q, a_s, b_q, b_s, variant='pipe128x64')
     assert torch.equal(direct, staged)
-    helpers.tolerance_check(staged, orc.dequant_ref(a_q, a_s, b_q, b_s), f'epilogue {variant}')
+    helpers.tolerance_check(direct, orc.dequant_ref(a_q, a_s, b_q, b_s), f'epilogue {variant}')
 
 
 @pytest.mark.parametrize('variant', ['pipe256x256', 'pipe128x256w8', 'pipe256mix', 'pipe128x128', 'pipe128x64', None])
 @pytest.mark.parametrize('M,N,K', [(257, 389, 256), (130, 1, 128), (33, 1023, 384), (5, 387, 512), (300, 514, 1040)])
 @pytest.mark.parametrize('out_dtype', [torch.bfloat16, torch.float32])
 def test_rows_at_any_alignment(dev, variant, M, N, K, out_dtype):
-    """Results whose rows start at odd elements, and fp32 results, through LDS and whole-row stores: the same bits as stored
-    element groups straight from the registers, in every kernel family."""
+    """Results that start at an odd element and rows that do, bf16 and fp32, in every kernel family: nothing is written beside them, and
+    the bits are those of the 128 x 64 kernel, whose rows pass through LDS (that kernel itself: of its stores straight from the
+    registers; the planner's choice, which may add K in another order: of its own result at an even element)."""
     from dlblas_amd import _lib
     if variant is not None and K % 128 != 0:
         pytest.skip('the ring kernels take whole K blocks')
     print(f'case rows variant={variant} M={M} N={N} K={K} {out_dtype}', flush=True)
-    a_q, a_s, b_q, b_s = helpers.make_dense(M, N, K, seed=29)
-    try:
-        _lib.tune('epilogue', 2)
-        direct = _run_dense(dev, a_q, a_s, b_q, b_s, dtype=out_dtype, variant=variant)
-    finally:
-        _lib.tune('epilogue', 0)
-    staged = _run_dense(dev, a_q, a_s, b_q, b_s, dtype=out_dtype, variant=variant)
-    assert torch.equal(direct, staged)
-    helpers.tolerance_check(staged, orc.dequant_ref(a_q, a_s, b_q, b_s), f'rows {variant}')
+    ops = helpers.make_dense(M, N, K, seed=29)
+    even = _run_dense_guarded(dev, *ops, dtype=out_dtype, variant=variant)
+    odd = _run_dense_guarded(dev, *ops, dtype=out_dtype, variant=variant, first=1)
+    assert torch.equal(even, odd)
+    if variant is not None:
+        try:
+            _lib.tune('epilogue', 2 if variant == 'pipe128x64' else 0)
+            other = _run_dense_guarded(dev, *ops, dtype=out_dtype, variant='pipe128x64', first=1)
+        finally:
+            _lib.tune('epilogue', 0)
+        assert torch.equal(even, other)
+    helpers.tolerance_check(odd, orc.dequant_ref(*ops), f'rows {variant}')
 
 
 @pytest.mark.parametrize('N', [389, 131, 514])
@@ -628,11 +658,51 @@ def test_list_tiles_carry_the_ring(dev, kb, dtype):
     helpers.tolerance_check(outs[0][rows.to(dev)], ref, f'list ring K={K}')
 
 
+# blocks per expert, column tiles, rows in the last block, whole tiles (256 / 192 rows) that the last round runs as 64-row pieces
+LIST_CUTS = [([3, 3, 1, 3], 39, 128, (0, 17)), ([1, 3], 91, 1, (0, 17)), ([1, 3], 91, 64, (0, 17)), ([1, 3], 91, 65, (0, 17)), ([2], 270, 1, (14, 0)),
+             ([2], 270, 64, (14, 0)), ([2], 270, 65, (14, 0))]
+
+
+@pytest.mark.parametrize('blocks,tiles_n,last,cut', LIST_CUTS)
+@pytest.mark.parametrize('kb,dtype', [(1, torch.bfloat16), (3, torch.float32), (5, torch.bfloat16)])
+def test_list_tiles_in_pieces(dev, blocks, tiles_n, last, cut, kb, dtype):
+    """A last round of few tiles runs as 64-row pieces: of 192-row tiles (an odd number, so that a pair is divided) and of the one 256-row
+    tile; a last block so short that its last piece would start behind the last row, and one row more.  The bits of the
+    uniform 128-row tiles, and the rows behind the last one stay as they were."""
+    from dlblas_amd import _lib
+    from dlblas_amd.kernels.fp8_gemm_grouped import m_grouped_fp8_gemm_nt_contiguous
+    assert helpers.list_cut(blocks, tiles_n, torch.cuda.get_device_properties(dev).multi_processor_count) == cut
+    G, M_sum, N, K = len(blocks), 128 * (sum(blocks) - 1) + last, 256 * tiles_n - 23, kb * 128
+    print(f'case list pieces blocks={blocks} last={last} N={N} K={K} {dtype}', flush=True)
+    g = torch.Generator(device=dev).manual_seed(80 + kb)
+    a_q, a_s = helpers.quantise_act_device(torch.randn(M_sum, K, device=dev, generator=g).to(torch.bfloat16))
+    w_q, w_s = helpers.expert_weights_device(G, N, K, dev, 81)
+    m_indices = torch.repeat_interleave(torch.arange(G, dtype=torch.int32), torch.tensor(blocks) * 128)[:M_sum].contiguous().to(dev)
+    outs = []
+    try:
+        for variant in (None, 'pipe128x256w8'):
+            whole = torch.full((M_sum + 64, N), 7.0, dtype=dtype, device=dev)
+            _lib.tune('tile_list', 1 if variant is None else 0)
+            _lib.force_variant(variant)
+            assert _lib.plan_grouped(1, M_sum, N, K, G) == ('pipe128x256w8', variant is None)
+            m_grouped_fp8_gemm_nt_contiguous((a_q, a_s), (w_q, w_s), whole[:M_sum], m_indices)
+            torch.cuda.synchronize()
+            assert bool((whole[M_sum:] == 7.0).all()), 'a row behind the last one was written'
+            outs.append(whole[:M_sum])
+    finally:
+        _lib.force_variant(None)
+        _lib.tune('tile_list', 0)
+    assert torch.equal(outs[0], outs[1])
+    rows = torch.tensor([M_sum - 1])
+    helpers.tolerance_check(outs[0][rows.to(dev)], orc.dequant_ref(a_q[rows.to(dev)].cpu(), a_s[rows.to(dev)].cpu(), w_q[G - 1].cpu(), w_s[G - 1].cpu()), f'list pieces K={K}')
+
+
 def test_grouped_contiguous_many_blocks(dev):
     """700 blocks of 128 rows: the device-side tile list then works in chunks of several blocks per thread, and runs of
     1 to 7 blocks (256-row tiles, pairs of 192-row tiles for the odd ones, single 128-row tiles) cross the chunk
     boundaries in every way.  Skipped blocks in between; the last block is short."""
     print('case contiguous many blocks', flush=True)
+    from dlblas_amd import _lib
     from dlblas_amd.kernels.fp8_gemm_grouped import m_grouped_fp8_gemm_nt_contiguous
     G, N, K = 12, 256, 128
     g = helpers.gen(31)
@@ -648,8 +718,13 @@ def test_grouped_contiguous_many_blocks(dev):
     sentinel = 99.0
     ref = orc.grouped_contiguous_ref(a_q, a_s, w_q, w_s, torch.full((M_sum, N), sentinel), m_indices)
     out = torch.full((M_sum, N), sentinel, dtype=torch.bfloat16, device=dev)
-    m_grouped_fp8_gemm_nt_contiguous((a_q.to(dev), a_s.to(dev)), (w_q.to(dev), w_s.to(dev)), out, m_indices.to(dev))
-    torch.cuda.synchronize()
+    try:
+        _lib.tune('tile_list', 1)  # at so short a K the planner keeps to the uniform tiles
+        assert _lib.plan_grouped(1, M_sum, N, K, G) == ('pipe128x256w8', True)
+        m_grouped_fp8_gemm_nt_contiguous((a_q.to(dev), a_s.to(dev)), (w_q.to(dev), w_s.to(dev)), out, m_indices.to(dev))
+        torch.cuda.synchronize()
+    finally:
+        _lib.tune('tile_list', 0)
     assert torch.all(out.cpu()[m_indices < 0] == sentinel), 'a skipped block was written'
     helpers.tolerance_check(out, ref, 'contiguous many blocks')
 
@@ -716,8 +791,8 @@ def test_grouped_masked_hint_picks_the_tile_shape(dev):
 def test_masked_tiles_carry_the_ring(dev, kb, dtype):
     """Six experts of 0 to 300 rows by 25673 columns: every resident workgroup of the masked layout's ring kernels goes through several
     tiles, whole and ragged ones, of one expert and of the next, at fewer K blocks than the ring has stages, as many, and more
-    (17: more than the scale table of the 128 x 256 tiles holds).  The three tile shapes and the weight-streaming kernel agree
-    bit for bit, rows at or beyond masked_m stay as they were."""
+    (17: more than the scale table of the 128 x 256 tiles holds).  The three tile shapes and, from the three K blocks on that it needs,
+    the weight-streaming kernel agree bit for bit, rows at or beyond masked_m stay as they were."""
     from dlblas_amd import _lib
     from dlblas_amd.kernels.fp8_gemm_grouped import m_grouped_fp8_gemm_nt_masked
     G, M_max, N, K = 6, 300, 100 * 256 + 73, kb * 128
@@ -730,14 +805,20 @@ def test_masked_tiles_carry_the_ring(dev, kb, dtype):
     beyond = torch.arange(M_max)[None, :] >= masked_m[:, None]
     outs = []
     try:
-        for variant in ('pipe256x256', 'pipe128x256w8', 'pipe128x128', None):
+        for variant in ('pipe256x256', 'pipe128x256w8', 'pipe128x128', 'stream128x256')[:3 if kb < 3 else 4]:
             out = torch.full((G, M_max, N), 7.0, dtype=dtype, device=dev)
-            _lib.force_variant(variant)
+            if variant == 'stream128x256':
+                _lib.force_variant(None)
+                _lib.tune('stream', 5)
+                assert _lib.plan_stream(M_max, N, K, G, 150) == (128, 256, False)
+            else:
+                _lib.force_variant(variant)
             m_grouped_fp8_gemm_nt_masked((a_q, a_s), (w_q, w_s), out, masked_m.to(dev), 150)
             assert torch.all(out[beyond.to(dev)] == 7.0), f'{variant}: rows beyond masked_m were written'
             outs.append(out)
     finally:
         _lib.force_variant(None)
+        _lib.tune('stream', 0)
     for out in outs[1:]:
         assert torch.equal(outs[0], out)
     for e, row in ((0, 299), (3, 255), (5, 0)):

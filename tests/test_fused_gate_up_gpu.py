@@ -205,6 +205,42 @@ def test_fused_list_tiles_carry_the_ring(dev, kb, gathered):
     assert torch.equal(fused[1], ref_s), 'scales differ'
 
 
+@pytest.mark.parametrize('blocks,tiles_n,last,cut', [([1, 3], 91, 1, (0, 17)), ([1, 3], 91, 65, (0, 17)), ([2], 270, 64, (14, 0)), ([2], 270, 128, (14, 0))])
+@pytest.mark.parametrize('kb,gathered', [(1, True), (3, False), (5, True)])
+def test_fused_list_tiles_in_pieces(dev, blocks, tiles_n, last, cut, kb, gathered):
+    """A last round of few tiles runs as 64-row pieces, of 192-row tiles (an odd number, so that a pair is divided) and of the one 256-row
+    tile, with a last block so short that its last piece would start behind the last row, and with longer ones.  The bytes and
+    scales of the activation and the quantiser on the product of the uniform 128-row tiles."""
+    from dlblas_amd import _lib
+    from dlblas_amd.kernels.activation import silu_and_mul_post_quant
+    from dlblas_amd.kernels.fp8_gemm_grouped import fp8_gemm_grouped_contiguous_silu_quant, m_grouped_fp8_gemm_nt_contiguous
+    assert helpers.list_cut(blocks, tiles_n, torch.cuda.get_device_properties(dev).multi_processor_count) == cut
+    G, M_sum, inter, K, T = len(blocks), 128 * (sum(blocks) - 1) + last, 128 * tiles_n, 128 * kb, 333
+    print(f'case fused list pieces blocks={blocks} last={last} I={inter} K={K} gathered={gathered}', flush=True)
+    g = torch.Generator(device=dev).manual_seed(90 + kb)
+    x_q, x_s = helpers.quantise_act_device((torch.randn(T, K, device=dev, generator=g) * 1.5).to(torch.bfloat16))
+    row_token = torch.randint(0, T, (M_sum, ), device=dev, generator=g, dtype=torch.int32)
+    row_token[-1] = T - 1
+    w_q, w_s = helpers.expert_weights_device(G, 2 * inter, K, dev, 91)
+    m_indices = torch.repeat_interleave(torch.arange(G, dtype=torch.int32), torch.tensor(blocks) * 128)[:M_sum].contiguous().to(dev)
+    a_q, a_s = x_q.view(torch.uint8)[row_token.long()].view(torch.float8_e4m3fn), x_s[row_token.long()]
+    if gathered:
+        fused = fp8_gemm_grouped_contiguous_silu_quant(x_q, x_s, w_q, w_s, m_indices, a_row_index=row_token)
+    else:
+        fused = fp8_gemm_grouped_contiguous_silu_quant(a_q, a_s, w_q, w_s, m_indices)
+    assert fused is not None
+    gate_up = torch.zeros(M_sum, 2 * inter, dtype=torch.bfloat16, device=dev)
+    try:
+        _lib.force_variant('pipe128x256w8')
+        m_grouped_fp8_gemm_nt_contiguous((a_q, a_s), (w_q, w_s), gate_up, m_indices)
+    finally:
+        _lib.force_variant(None)
+    ref_q, ref_s = silu_and_mul_post_quant(gate_up, 128)
+    torch.cuda.synchronize()
+    assert torch.equal(fused[0].view(torch.uint8), ref_q.view(torch.uint8)), 'quantised codes differ'
+    assert torch.equal(fused[1], ref_s), 'scales differ'
+
+
 @pytest.mark.parametrize('kb', [1, 2, 3, 4, 8])
 def test_masked_fused_tiles_carry_the_ring(dev, kb):
     """Experts of 0 to 300 rows by 130 column tiles on the masked layout's ring kernel (the weight-streaming kernel kept out): several
