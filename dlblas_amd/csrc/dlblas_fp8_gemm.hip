@@ -264,25 +264,34 @@ hipError_t launch_pipelined(const Args& args, int grid, int dev, hipStream_t str
   return hipGetLastError();
 }
 
-template <class Cfg, int MODE, bool AHEAD = false>
+template <class Cfg, int MODE, bool AHEAD = false, bool ODD = false>
 hipError_t launch_ring(const Args& args, int grid, int dev, hipStream_t stream) {
   static std::atomic<unsigned long long> lds_done{0};
   constexpr int lds = MODE == kMaskedAct ? Cfg::ACT_LDS_BYTES : Cfg::LDS_BYTES;
-  auto kernel = fp8_gemm_ring_kernel<Cfg, MODE, AHEAD>;
+  auto kernel = fp8_gemm_ring_kernel<Cfg, MODE, AHEAD, ODD>;
   hipError_t e = ensure_lds(kernel, lds, dev, &lds_done);
   if (e != hipSuccess || g_prepare_only) return e;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NT), lds, stream, args);
   return hipGetLastError();
 }
 
+// Whether a dense launch has bf16 rows off dwords, for which the 256-column tiles have kernels of their own.  us per call without / with:
+// 374 x 30809 x 640 18.0 / 17.1, 1504 x 5457 x 2560 30.5 / 29.3, 2200 x 12001 x 1024 40.5 / 36.5, in 128 x 256 tiles 2683 x 10447 x 512
+// 32.5 / 30.0.  Rows on dwords lose by them (374 x 30810 x 640 17.8 / 18.3) and so do 128 x 256 tiles, whose waves write 128 bytes of
+// a row, at one and two K blocks (1640 x 16773 x 256 25.6 / 27.7).
+inline bool odd_rows(const Args& args) { return !args.out_f32 && (args.N % 2 != 0 || misaligned(args.c, 4)) && args.splitk == 1; }
+
 template <class Cfg>
 hipError_t launch_ring_mode(int mode, const Args& args, int grid, int dev, hipStream_t stream) {
   switch (mode) {
-    case kDense:
+    case kDense: {
       // resident workgroups of more than one tile: the ring that runs on (a single tile is 1 us faster without its code; the knob for
       // stores apart from the ring asks for tiles that start afresh)
-      if (args.splitk == 1 && args.c_lds && static_cast<int64_t>(args.tiles_m) * args.tiles_n > grid) return launch_ring<Cfg, kDense, true>(args, grid, dev, stream);
-      return launch_ring<Cfg, kDense>(args, grid, dev, stream);
+      const bool ahead = args.splitk == 1 && args.c_lds && static_cast<int64_t>(args.tiles_m) * args.tiles_n > grid;
+      if constexpr (Cfg::BN == 256)
+        if (odd_rows(args) && (Cfg::BM == 256 || args.kblocks > 2)) return ahead ? launch_ring<Cfg, kDense, true, true>(args, grid, dev, stream) : launch_ring<Cfg, kDense, false, true>(args, grid, dev, stream);
+      return ahead ? launch_ring<Cfg, kDense, true>(args, grid, dev, stream) : launch_ring<Cfg, kDense>(args, grid, dev, stream);
+    }
     case kContiguous:
       if constexpr (Cfg::BM == kScaleBlock) return launch_ring<Cfg, kContiguous>(args, grid, dev, stream);  // taller tiles come from the lists
       return hipErrorInvalidValue;
@@ -1494,14 +1503,16 @@ int run(const Problem& pr) {
       const int64_t split = rs.n_split;
       if (split >= pr.N)
         return rs.sctab ? launch_ring_mode<Ring256x256T>(pr.mode, ar, g_dense, dev, pr.stream) : launch_ring_mode<Ring256x256>(pr.mode, ar, g_dense, dev, pr.stream);
-      static std::atomic<unsigned long long> lds_done[2];
-      auto kernel = rs.sctab ? fp8_gemm_ring_mixed_kernel<Ring256x256T, Ring256x192T> : fp8_gemm_ring_mixed_kernel<Ring256x256, Ring256x192>;
+      static std::atomic<unsigned long long> lds_done[4];
+      const bool odd = odd_rows(ar);
+      auto kernel = odd ? (rs.sctab ? fp8_gemm_ring_mixed_kernel<Ring256x256T, Ring256x192T, true> : fp8_gemm_ring_mixed_kernel<Ring256x256, Ring256x192, true>)
+                        : (rs.sctab ? fp8_gemm_ring_mixed_kernel<Ring256x256T, Ring256x192T, false> : fp8_gemm_ring_mixed_kernel<Ring256x256, Ring256x192, false>);
       const int lds = rs.sctab ? Ring256x256T::LDS_BYTES : Ring256x256::LDS_BYTES;
       ar.n_split = static_cast<int>(split);
       ar.tiles_n_a = static_cast<int>(split / 256);
       ar.tiles_n_b = static_cast<int>(ceil_div(pr.N - split, 192));
       ar.tiles_a = ar.tiles_m * ar.tiles_n_a;
-      const hipError_t le = ensure_lds(kernel, lds, dev, &lds_done[rs.sctab ? 1 : 0]);
+      const hipError_t le = ensure_lds(kernel, lds, dev, &lds_done[(rs.sctab ? 1 : 0) + (odd ? 2 : 0)]);
       if (le != hipSuccess || g_prepare_only) return le;
       hipLaunchKernelGGL(kernel, dim3(ar.tiles_a + ar.tiles_m * ar.tiles_n_b), dim3(Ring256x256::NT), lds, pr.stream, ar);
       return hipGetLastError();

@@ -93,6 +93,22 @@ __device__ __forceinline__ void swap_chunks(v4i& a, v4i& b, int lane) {
   }
 }
 
+// The same for bit BIT (16 or 32) of the lane number.
+template <int BIT>
+__device__ __forceinline__ void swap_far_chunks(v4i& a, v4i& b) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const unsigned ua = static_cast<unsigned>(a[i]), ub = static_cast<unsigned>(b[i]);
+    if constexpr (BIT == 16) {
+      const auto s = __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
+      a[i] = static_cast<int>(s[0]), b[i] = static_cast<int>(s[1]);
+    } else {
+      const auto s = __builtin_amdgcn_permlane32_swap(ua, ub, false, false);
+      a[i] = static_cast<int>(s[0]), b[i] = static_cast<int>(s[1]);
+    }
+  }
+}
+
 // Workgroup barrier that orders LDS traffic only (see lds_barrier), as builtins: the compiler then knows that no LDS read is out
 // and counts the reads behind it instead of waiting for all of them.
 __device__ __forceinline__ void ring_barrier() {
@@ -128,7 +144,8 @@ struct ListRegion {
   int which, first, count, pieces;
 };
 
-template <class Cfg, int MODE, bool AHEAD>
+// ODD: bf16 results whose rows lie off dwords (dense, K in one piece).
+template <class Cfg, int MODE, bool AHEAD, bool ODD = false>
 __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_first, int tiles_m, int tiles_n, int n_base, ListRegion lists = {}) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, MF = Cfg::MF, NF = Cfg::NF, STAGES = Cfg::STAGES, H = Cfg::H, S = Cfg::S, L = Cfg::L;
   constexpr bool kList = MODE == kContigList || MODE == kContigListAct;
@@ -151,7 +168,7 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
   // ---- tiles ------------------------------------------------------------------------------------------------
   const int tiles = tiles_m * tiles_n;
   // Unit id of a dense launch: the tile, in patches of group_m row tiles, and the slice of K; slices of one tile are far apart.
-  const int units = MODE == kDense && !AHEAD ? tiles * p.splitk : tiles;
+  const int units = MODE == kDense && !AHEAD && !ODD ? tiles * p.splitk : tiles;
   int walk_g = 0, walk_base = 0;
   // tables of a launch's tiles, written by the launch before: scalar loads
   typedef const __attribute__((address_space(4))) int32_t* table_ptr;
@@ -216,7 +233,7 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
     } else {
       if (vb >= units) return false;
       const int id = xcd_remap(vb, units);
-      t.split = MODE == kDense && !AHEAD ? id / tiles : 0;
+      t.split = MODE == kDense && !AHEAD && !ODD ? id / tiles : 0;
       t.lin = id - t.split * tiles;
       const int width = p.group_m * tiles_n;
       const int grp = t.lin / width;
@@ -383,7 +400,7 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
       t = tn, have = more;
       continue;
     }
-    const bool sliced = MODE == kDense && !AHEAD && p.splitk > 1;  // (launches of K slices use the kernels without AHEAD)
+    const bool sliced = MODE == kDense && !AHEAD && !ODD && p.splitk > 1;  // (launches of K slices use the kernels without AHEAD)
     const int kb_first = sliced ? t.split * p.kb_per_split : 0;  // the host leaves no slice empty
     const int nk = sliced ? min(p.kblocks, kb_first + p.kb_per_split) - kb_first : p.kblocks;  // K blocks of this unit
     // (the table of gathered rows is waited for together with the first group of the tile)
@@ -589,7 +606,7 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
         }
         if (live && eq == 0 && wave % Cfg::WGN == 0) s_out[static_cast<int64_t>(m) * p.act_s_sm + static_cast<int64_t>(t.n0 / kScaleBlock) * p.act_s_sk] = scale;
       }
-    } else if (sliced && p.fused_reduce) {
+    } else if (!ODD && sliced && p.fused_reduce) {
       // Split-K in one launch.  The workgroups of a tile (one per K slice) park their fp32 sums in the workspace,
       // count themselves in on the tile's arrival counter, wait - for a bounded time - until all slices are in, and
       // then each adds up its share of the tile: the slices in index order (the same order, and so the same bits, as
@@ -702,12 +719,15 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
       // row instead of 64, or of 16-byte pieces of fp32.  us per call, both on one GPU: bf16 rows at odd addresses 914 x 28119 x 512 38.8 ->
       // 32.4, 3779 x 6111 x 1024 45.4 -> 36.3, 2000 x 5001 x 4096 52.0 -> 47.6; fp32 914 x 28120 x 512 39.3 -> 32.1, 271 x 18112 x 640 13.9 ->
       // 12.0; bf16 rows on 16 bytes 271 x 18112 x 640 11.1 -> 10.1, 3500 x 4096 x 512 15.1 -> 14.2, 4096 x 24576 x 1536 141 -> 138.
+      // Neighbouring lanes then hold chunks 64 bytes apart, which is as good as any order where rows lie on dwords.  ODD: elsewhere the lanes
+      // of a row's chunks exchange first, so that neighbours write 64 bytes (32 in narrower wave tiles) on end.  In kernels of its own,
+      // because beside this form other calls lose up to 1 %.
       auto store_tile = [&](auto f32, auto inside, void* out) __attribute__((always_inline)) {
-        constexpr bool F32 = decltype(f32)::value;
-        const int col = t.n0 + wn0 + eq * 8;
+        constexpr bool F32 = decltype(f32)::value, FAR = ODD && !F32;
+        const int col = t.n0 + wn0 + (FAR ? 0 : eq * 8);
 #pragma unroll
         for (int mi = 0; mi < MF; ++mi) {
-          // chunk `at` columns into the lane's first, of row r of the lane's four
+          // chunk `at` columns behind col, of row r of the lane's four
           auto put = [&](int r, int at, v4i v) __attribute__((always_inline)) {
             const int m = t.m0 + e_row - (el & 3) + r + ring_row(mi, 0);
             if (m >= t.m_end) return;
@@ -733,25 +753,30 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
 #pragma unroll
           for (int c = 0; c < kFour; c += 4) {
             v4i x[4] = {chunk(c), chunk(c + 1), chunk(c + 2), chunk(c + 3)};
+            if constexpr (FAR) {
+              swap_far_chunks<16>(x[0], x[1]), swap_far_chunks<16>(x[2], x[3]);
+              swap_far_chunks<32>(x[0], x[2]), swap_far_chunks<32>(x[1], x[3]);
+            }
             swap_chunks<1>(x[0], x[1], el), swap_chunks<1>(x[2], x[3], el);
             swap_chunks<2>(x[0], x[2], el), swap_chunks<2>(x[1], x[3], el);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) put(r, chunk_col(c) + chunk_col(j), x[r]);
+            for (int r = 0; r < 4; ++r) put(r, FAR ? chunk_col(c + eq) + 8 * j : chunk_col(c) + chunk_col(j), x[r]);
           }
 #pragma unroll
           for (int c = kFour; c + 1 < CHUNKS; c += 2) {
             v4i x[2] = {chunk(c), chunk(c + 1)};
+            if constexpr (FAR) swap_far_chunks<16>(x[0], x[1]);
             swap_chunks<1>(x[0], x[1], el);
 #pragma unroll
-            for (int r = 0; r < 2; ++r) put((j & 2) + r, chunk_col(c) + chunk_col(j & 1), x[r]);
+            for (int r = 0; r < 2; ++r) put((j & 2) + r, FAR ? chunk_col(c + (eq & 1)) + (eq & 2) * 8 + 8 * (j & 1) : chunk_col(c) + chunk_col(j & 1), x[r]);
           }
-          if constexpr (CHUNKS % 2 != 0) put(j, chunk_col(CHUNKS - 1), chunk(CHUNKS - 1));
+          if constexpr (CHUNKS % 2 != 0) put(j, chunk_col(CHUNKS - 1) + (FAR ? eq * 8 : 0), chunk(CHUNKS - 1));
         }
       };
       void* out = sliced ? static_cast<void*>(p.ws + static_cast<int64_t>(t.split) * p.M * p.N) : static_cast<void*>(c_base);
       constexpr std::true_type yes{};
       constexpr std::false_type no{};
-      if (sliced || p.out_f32)
+      if (!ODD && (sliced || p.out_f32))
         cols_inside ? store_tile(yes, yes, out) : store_tile(yes, no, out);
       else
         cols_inside ? store_tile(no, yes, out) : store_tile(no, no, out);
@@ -761,25 +786,25 @@ __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_f
   }
 }
 
-template <class Cfg, int MODE, bool AHEAD>
+template <class Cfg, int MODE, bool AHEAD, bool ODD>
 __global__ void __launch_bounds__(Cfg::NT) fp8_gemm_ring_kernel(const Args p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  ring_body<Cfg, MODE, AHEAD>(p, smem, blockIdx.x, p.tiles_m, p.tiles_n, 0);
+  ring_body<Cfg, MODE, AHEAD, ODD>(p, smem, blockIdx.x, p.tiles_m, p.tiles_n, 0);
 }
 
 // Dense GEMM whose columns are cut at p.n_split into a region of CfgA tiles and a region of narrower CfgB tiles,
 // one workgroup per tile, region A first.  The host picks the cut so that the last round of workgroups fills the
 // chip: e.g. 448 tiles of 256 x 256 on 256 CUs leave a quarter of the chip idle in the second round, while 256
 // tiles of 256 x 256 followed by 256 tiles of 256 x 192 cover the same output and keep every CU busy.
-template <class CfgA, class CfgB>
+template <class CfgA, class CfgB, bool ODD>
 __global__ void __launch_bounds__(CfgA::NT) fp8_gemm_ring_mixed_kernel(const Args p) {
   static_assert(CfgA::NT == CfgB::NT && CfgA::BM == CfgB::BM, "both regions use the same workgroup shape and tile height");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int bid = blockIdx.x;
   if (bid < p.tiles_a)
-    ring_body<CfgA, kDense, false>(p, smem, bid, p.tiles_m, p.tiles_n_a, 0);
+    ring_body<CfgA, kDense, false, ODD>(p, smem, bid, p.tiles_m, p.tiles_n_a, 0);
   else
-    ring_body<CfgB, kDense, false>(p, smem, bid - p.tiles_a, p.tiles_m, p.tiles_n_b, p.n_split);
+    ring_body<CfgB, kDense, false, ODD>(p, smem, bid - p.tiles_a, p.tiles_m, p.tiles_n_b, p.n_split);
 }
 
 // Expert-contiguous rows from the three tile lists (see contiguous_tile_list_block): persistent workgroups.  The 192-row pairs first:

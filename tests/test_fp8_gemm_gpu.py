@@ -329,7 +329,7 @@ def test_epilogue_through_lds_equals_direct_stores(dev, variant, M, N, K):
 
 
 @pytest.mark.parametrize('variant', ['pipe256x256', 'pipe128x256w8', 'pipe256mix', 'pipe128x128', 'pipe128x64', None])
-@pytest.mark.parametrize('M,N,K', [(257, 389, 256), (130, 1, 128), (33, 1023, 384), (5, 387, 512), (300, 514, 1040)])
+@pytest.mark.parametrize('M,N,K', [(257, 389, 256), (130, 1, 128), (33, 1023, 384), (130, 264, 384), (5, 387, 512), (300, 514, 1040)])
 @pytest.mark.parametrize('out_dtype', [torch.bfloat16, torch.float32])
 def test_rows_at_any_alignment(dev, variant, M, N, K, out_dtype):
     """Results that start at an odd element and rows that do, bf16 and fp32, in every kernel family: nothing is written beside them, and
