@@ -525,9 +525,9 @@ int64_t pick_mixed_split(int64_t M, int64_t N, int cus, double* makespan = nullp
 //   - equal tiles, more than one round: resident workgroups whose ring runs on from tile to tile: 5.4 + 1.53 K blocks per round
 //     and 5.8 for the launch.
 // A last round that is not full costs half of a round (0.7 in a mixed launch, 0.44 in 128 x 256 tiles) plus its share of the rest: the chip is
-// faster with fewer tiles.  43 launches lie within 5 % rms of that.  The choice, 128-row tiles included, is 0.5 % behind
-// the best of the three over 90 random problems it was not fitted to, 6 % at worst (bench.py --planner-sweep wide_random draws such); with the
-// constants of the kernels before these 1.3 % and 14 %.
+// faster with fewer tiles.  43 launches lie within 5 % rms of that.  Results stored as they are now, which the fit was made before, the choice,
+// 128-row tiles included, is 0.8 % behind the best of the three over 529 random problems of five K blocks and more (15 % at worst, 573 x 18582 x
+// 768) and 1.1 % over the 80 of bench.py --planner-sweep wide_random (18 %, 2394 x 16192 x 640).
 // Mixed tiles win where K is long and the last round short (4096 x 5248 x 4096: 104 / 113 us, 2048 x 17408 x 7168: 265 / 292),
 // equal ones where the fixed part of a tile counts (3500 x 33024 x 1280: 203 / 183, 2048 x 18176 x 512: 45 / 38).
 int pick_wide_variant(int64_t M, int64_t N, int kblocks, int cus, double* us = nullptr) {
@@ -548,17 +548,24 @@ int pick_wide_variant(int64_t M, int64_t N, int kblocks, int cus, double* us = n
 // pipe there; a round of 128 x 256 tiles takes 2.4 + 0.94 K blocks, its ring runs on from tile to tile as well.
 // The larger tile wins unless its rows are mostly padding (384 rows are two 256-row tiles but three of 128) or its tiles
 // leave much of a round empty (2048 x 4096: 128 tiles of 256 x 256 on 256 CUs, but 256 tiles of 128 x 256):
-// 384 x 18432 x 7168 82 -> 67 us, 2048 x 4096 x 7168 79 -> 67 us.  bf16 and fp32 results agree about it since both leave from the registers
-// (30 shapes of 2 to 5 K blocks; the smaller tile over the larger one 0.69 .. 1.33 and 0.66 .. 1.20).  The smaller tile is kept up to 7 %
-// above the estimates at three and four K blocks, where they are no closer than that, and up to 20 % below three, which were not fitted.
+// 384 x 18432 x 7168 82 -> 67 us, 2048 x 4096 x 7168 79 -> 67 us.  bf16 and fp32 results agree about it since both leave from the
+// registers.  Limits of the smaller tile's estimate, in units of the larger one's:
+//   - one and two K blocks, which the estimates were not fitted to: 0.9.  us per call, 128-row tiles / 256-row ones: 2504 x 29504 x 256 50.8
+//     / 37.2, 3897 x 19856 x 256 52.7 / 38.4, 691 x 12248 x 256 13.1 / 11.4; behind the best over 285 random problems 2.4 % (10.7 %
+//     with 1.2).  But 1.2 where its tiles are one round (1121 x 7040 x 256 9.4 / 10.7) and where they fill a good part of a second
+//     beside one round of the larger ones, which are up to 8 % ahead there (2048 x 8192 x 256 15.5 / 14.5);
+//   - three and four K blocks: 0.95, in launches of more than four rounds of the larger ones 1.07 (4096 x 32768 x 512 105 / 98): 0.9 % behind
+//     the best over 286 problems, 1.6 % with 1.07 everywhere (928 x 26768 x 512 29.2 / 23.6, 1606 x 35392 x 384 fp32 71 / 52).
 bool prefers_128_row_tiles(int64_t M, int64_t N, int kblocks, int cus, double* us = nullptr) {
   double wide_us = 0.0;
   pick_wide_variant(M, N, kblocks, cus, &wide_us);
-  const int64_t tiles = ceil_div(M, 128) * ceil_div(N, 256);
+  const int64_t tiles = ceil_div(M, 128) * ceil_div(N, 256), tall = ceil_div(M, 256) * ceil_div(N, 256);
   const double rounds = 0.56 * static_cast<double>(tiles) / cus + 0.44 * static_cast<double>(ceil_div(tiles, cus));
   const double half_us = 5.5 + rounds * (2.4 + 0.94 * kblocks);
   if (us) *us = std::min(wide_us, half_us);
-  return half_us < (kblocks <= 2 ? 1.2 : kblocks <= 4 ? 1.07 : 1.0) * wide_us;
+  const bool few = tiles <= cus || (tall <= cus && 2 * tiles > 3 * cus);
+  const double limit = kblocks <= 2 ? (few ? 1.2 : 0.9) : kblocks > 4 ? 1.0 : tall > 4 * cus ? 1.07 : 0.95;
+  return half_us < limit * wide_us;
 }
 
 struct Plan {
@@ -897,13 +904,15 @@ int pick_wavek(int64_t M, int64_t N, int64_t K, int cus, size_t ws_bytes) {
   const size_t ws_avail = ws_bytes > DLB_WS_COUNTER_BYTES ? ws_bytes - DLB_WS_COUNTER_BYTES : 0;
   double other;
   const bool wide = M > 128 && ceil_div(M, 256) * ceil_div(N, 256) * 2 >= cus;
+  if (wide && kblocks <= 4) return kWaveKNone;
   if (wide)
     prefers_128_row_tiles(M, N, kblocks, cus, &other);
   else
     other = pick_mid_plan(M, N, kblocks, cus, ws_avail).us;
   if (M <= 128) other = std::min(other, 1.3 * decode_us(M, N, K, kblocks, cus));  // (the 128-row decode kernel runs above its estimate at short K)
-  // (where tiles of 256 columns fill half of the chip or more, this kernel's estimate is the lower one at short K and its time is not: 1326 x
-  // 5696 x 512 12.7 us for 11.0, 1883 x 9088 x 512 24.0 for 21.4, 259 x 27200 x 1920 30.5 for 28.5; over 55 problems it won none by 1 %)
+  // (where tiles of 256 columns fill half of the chip or more, this kernel's estimate is the lower one at short K and its time is not: 6 to 11
+  // % behind them over 49 problems of one to four K blocks, 1121 x 7040 x 256 11.0 us for 9.4; 259 x 27200 x 1920 30.5 for 28.5; over 56 longer
+  // ones it won none by 1 %)
   return best_us < (wide ? 0.85 : 0.95) * other ? best : kWaveKNone;
 }
 

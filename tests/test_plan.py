@@ -48,6 +48,17 @@ def test_documented_choices():
     assert _lib.plan(MASKED, 256, 7168, 2048) == ('pipe128x256w8', 1, 0)
 
 
+def test_short_k_keeps_the_taller_tiles():
+    """One to four K blocks: 256-row tiles where 128-row ones take several rounds, 128-row ones where they are one round; the wave-split
+    kernel stays out."""
+    for M, N, K in ((2504, 29504, 256), (3897, 19856, 256), (1606, 16128, 256), (691, 12248, 256), (928, 26768, 512), (1606, 35392, 384)):
+        assert _lib.plan(DENSE, M, N, K)[0] in ('pipe256x256', 'pipe256mix'), (M, N, K)
+    for M, N, K in ((1121, 7040, 256), (2414, 3112, 256), (320, 18176, 128), (310, 18297, 256)):
+        assert _lib.plan(DENSE, M, N, K)[0] == 'pipe128x256w8', (M, N, K)
+    for M, N, K in ((1121, 7040, 256), (335, 18179, 256), (517, 16714, 256), (272, 18072, 512), (149, 36800, 384)):
+        assert _lib.plan_wave_k(M, N, K) is None, (M, N, K)
+
+
 def test_invariants_over_a_sweep():
     Ms = (1, 15, 16, 17, 33, 64, 65, 100, 128, 129, 200, 256, 300, 512, 1000, 2048, 4096, 10000)
     Ns = (8, 100, 128, 392, 1000, 1536, 2112, 4096, 7168, 24576)
