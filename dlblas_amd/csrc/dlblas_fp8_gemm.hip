@@ -1039,6 +1039,79 @@ StreamPlan pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows
   return best;
 }
 
+// Masked plain product with a hint, from three K blocks on: a second look at the choice.  The estimates above know neither the output's
+// bytes nor how the experts' rows vary, and those of the streaming kernel are older than its waves apart: beside the kernels of before 26 of
+// 1200 random calls had become more than 5 % slower (16 x 1152 x 5760, 144 rows each 48 -> 65 us, 16 x 3712 x 3840, ~477 rows 132 -> 160).
+// These (us, fitted on MI355X to 2700 problems of 8 .. 32 experts x 4 .. 640 rows, rms 7 - 9 %): `start` + rounds of tiles x (`tile` + K
+// blocks x (`step` + `row` per activation row of a tile)) + the weights and the output at `weights` and `out` TB/s.  Rounds are whole
+// ones, averaged over what the tile count may come to: rows of 0 to twice the hint in buffers of about that height, rows about
+// the hint, as balanced routing leaves them, in taller ones.
+// Another kernel is taken where it is estimated 12 % ahead of the chosen one.  Over 1200 problems the fit had not seen the choice is then 2.6 %
+// behind the best kernel and shape (3.6 before), 14 calls are more than 5 % behind the kernels of before and 4 behind the choice without
+// it; the estimates alone would be at 1.7 %, but leave 21 and 24.
+struct MaskedCost {
+  double start, tile, step, row, weights, out;
+};
+constexpr MaskedCost kMaskedStream[kStreamCount] = {{3.2, 1.07, 0.542, 0.0068, 17.5, 11.4}, {3.49, 1.17, 0.562, 0.00622, 18.1, 5.6}, {4.15, 0.611, 0.268, 0.00407, 16.5, 2.92}, {3.99, 0.897, 0.572, 0.0059, 18.7, 4.34}, {4.89, 0.59, 0.213, 0.00181, 29.4, 3.23}};
+constexpr MaskedCost kMaskedStreamAhead[kStreamCount] = {{}, {4.14, 1.33, 0.644, 0.0031, 20.5, 4.66}, {4.24, 1.1, 0.295, 0.00343, 19.2, 3.79}, {4.61, 1.16, 0.622, 0.00406, 19.5, 4.02}, {4.71, 0.64, 0.167, 0.00264, 21.9, 4.9}};
+constexpr MaskedCost kMasked128x256 = {4.52, 2.27, 0.625, 0.00241, 15.4, 5.67}, kMasked128x128 = {4.6, 1.84, 0.388, 0.00204, 18.1, 8.51}, kMasked256x256 = {4.91, 3.58, 1, 0.00117, 22.8, 5.42};
+
+double masked_us(const MaskedCost& c, int bm, int bn, int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, int cus) {
+  const double h = static_cast<double>(std::min(hint_rows, M)), weights = static_cast<double>(N) * static_cast<double>(K);
+  double rows = h, live, row_tiles, spread;  // of an expert: rows, share that has any, row tiles; relative spread of all tiles
+  if (static_cast<double>(M) > 3.0 * h) {
+    const double sd = std::sqrt(h);
+    live = row_tiles = 1.0 - std::exp(-h);
+    for (double above = bm; above < h + 4.0 * sd; above += bm) row_tiles += 0.5 * std::erfc((above - h) / (sd * std::sqrt(2.0)));
+    spread = 0.03;
+  } else {
+    const double most = std::min(static_cast<double>(M), 2.0 * h), q = most / bm;
+    rows = 0.5 * most;
+    live = most / (most + 1.0);
+    row_tiles = q <= 1.0 ? live : 0.5 * (q + 1.0);
+    spread = std::max(0.02, std::sqrt(std::max(0.0, q * q - 1.0) / 12.0 / G) / row_tiles);
+  }
+  const double tiles = G * row_tiles * static_cast<double>(ceil_div(N, bn));
+  double rounds = 0.4 * std::max(1.0, std::ceil(tiles / cus));
+  for (double z : {-1.2, 1.2}) rounds += 0.3 * std::max(1.0, std::ceil(tiles * (1.0 + z * spread) / cus));
+  return c.start + rounds * (c.tile + static_cast<double>(ceil_div(K, kScaleBlock)) * (c.step + c.row * rows / row_tiles)) + live * G * weights / (c.weights * 1e6) +
+         G * rows * static_cast<double>(N) * 2.0 / (c.out * 1e6);
+}
+
+void masked_second_look(Plan& pl, StreamPlan& stream, int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, int cus) {
+  const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
+  auto ring_us = [&](int variant) {
+    int bm, bn;
+    tile_dims(variant, &bm, &bn);
+    const bool small = variant == kVarPipe128x128, tall = variant == kVarPipe256x256;
+    const bool table = kblocks <= (small ? Ring128x128T::SCTAB_KB : tall ? Ring256x256T::SCTAB_KB : Ring128x256T::SCTAB_KB);
+    return (M > kRelayoutMinRows && !table ? 3.5 : 0.0) + masked_us(small ? kMasked128x128 : tall ? kMasked256x256 : kMasked128x256, bm, bn, M, N, K, G, hint_rows, cus);
+  };
+  auto stream_us = [&](int shape, bool ahead) {
+    return masked_us((ahead ? kMaskedStreamAhead : kMaskedStream)[shape], kStreamDims[shape].bm, kStreamDims[shape].bn, M, N, K, G, hint_rows, cus);
+  };
+  const bool streams = stream.shape != kStreamNone;
+  double best_us = 0.88 * (streams ? stream_us(stream.shape, stream.ahead) : ring_us(pl.variant));
+  for (int variant : {kVarPipe128x256w8, kVarPipe128x128, kVarPipe256x256}) {
+    const double us = ring_us(variant);
+    if (us >= best_us) continue;
+    best_us = us;
+    stream = StreamPlan{};
+    pl.variant = variant;
+    tile_dims(variant, &pl.bm, &pl.bn);
+  }
+  for (int shape = 0; shape < kStreamCount; ++shape)
+    for (bool ahead : {false, true}) {
+      const StreamDims& d = kStreamDims[shape];
+      const int len = kblocks < d.stages || (ahead && d.bm <= 32) ? 0 : stream_chunk_len(kblocks, kblocks, d.ch, d.stages);
+      if (len <= 0) continue;
+      const double us = stream_us(shape, ahead);
+      if (us >= best_us) continue;
+      best_us = us;
+      stream.shape = shape, stream.us = us, stream.chunk_len = len, stream.slices = 0, stream.ahead = ahead;
+    }
+}
+
 // Expert-contiguous rows: estimates (microseconds, fitted on MI355X to 200 problems of 8 .. 32 experts x 500 .. 12000 tokens, N and K = 512 ..
 // 7168; rms 8, 8 and 17 %; their choice is 0.7 % behind the best of the three there and 0.9 % on 90 others) of 128 x 128 tiles, 128 x
 // 256 tiles and the lists.  Rounds of tiles x (fixed part + K blocks x the longer of a step and its share of the weights' stream, which
@@ -1127,6 +1200,9 @@ Resolved resolve(int mode, int64_t rows, int64_t N, int64_t K, int G, int64_t as
   if (mode == kMasked && dma_ok && K % kScaleBlock == 0 && K > 0 && static_cast<int64_t>(G) * rows < (1ll << 31))
     r.stream = pick_stream(rows, N, K, G, hint_rows, fused_act, cus, max_slices, rows * G, usable_ws ? (ws_bytes - DLB_WS_COUNTER_BYTES) / sizeof(float) : 0,
                            masked_ring_us(pl.variant, rows, N, K, G, hint_rows, fused_act, cus), !fused_act && hint_rows > 0);
+  if (mode == kMasked && hint_rows > 32 && rows > 64 && kblocks > 2 && !fused_act && is_pipelined(pl.variant) && static_cast<int64_t>(G) * rows < (1ll << 31) && g_forced_variant < 0 &&
+      g_knob[kKnobStream] == 0 && g_knob[kKnobStreamSlices] == 0)
+    masked_second_look(r.pl, r.stream, rows, N, K, G, hint_rows, cus);
   const int want = usable_ws ? pl.splitk : 1;
   r.kb_per_split = static_cast<int>(ceil_div(kblocks > 0 ? kblocks : 1, want));
   r.splitk = static_cast<int>(ceil_div(kblocks > 0 ? kblocks : 1, r.kb_per_split));  // no empty slice

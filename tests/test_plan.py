@@ -242,6 +242,15 @@ def test_plan_stream_answers_for_either_form():
     assert _lib.load().dlb_fp8_gemm_plan_stream(-1, 1, 1, 1, 0, 0, 256, None, None, None) == _lib.ERR_BAD_SHAPE
 
 
+def test_masked_hint_second_look():
+    """Masked products with a hint where the first estimates name a kernel that is 17 to 35 % behind: few rows in tall buffers stream, long
+    experts go to 256-row tiles.  Two K blocks, which the second estimates were not fitted to, keep the first choice."""
+    assert _lib.plan_stream(576, 1152, 5760, 16, 144) == (64, 256, True)
+    for M_max, N, K, G, hint in ((1024, 3712, 3840, 16, 477), (1024, 5120, 768, 8, 566), (1064, 5504, 1920, 32, 489), (776, 4864, 5248, 16, 455)):
+        assert _lib.plan_stream(M_max, N, K, G, hint) is None and _lib.plan_grouped(MASKED, M_max, N, K, G, hint)[0] == 'pipe256x256'
+    assert _lib.plan_grouped(MASKED, 512, 1536, 256, 6, 500)[0] == 'pipe256x256' and _lib.plan_stream(512, 1536, 256, 6, 500) is None
+
+
 @pytest.mark.parametrize('mode,rows', [(CONTIGUOUS, 1024), (MASKED, 64)])
 def test_plan_stream_knows_the_gate_up_form_in_two_launches(mode, rows):
     """Few narrow experts: with a workspace the sums of every tile, and inside an expert MLP of K slices, leave the first launch;
