@@ -527,7 +527,7 @@ int64_t pick_mixed_split(int64_t M, int64_t N, int cus, double* makespan = nullp
 // A last round that is not full costs half of a round (0.7 in a mixed launch, 0.44 in 128 x 256 tiles) plus its share of the rest: the chip is
 // faster with fewer tiles.  43 launches lie within 5 % rms of that.  Results stored as they are now, which the fit was made before, the choice,
 // 128-row tiles included, is 0.8 % behind the best of the three over 529 random problems of five K blocks and more (15 % at worst, 573 x 18582 x
-// 768) and 1.1 % over the 80 of bench.py --planner-sweep wide_random (18 %, 2394 x 16192 x 640).
+// 768) and 1.1 to 1.5 % over the 80 of bench.py --planner-sweep wide_random (18 %, 2394 x 16192 x 640).
 // Mixed tiles win where K is long and the last round short (4096 x 5248 x 4096: 104 / 113 us, 2048 x 17408 x 7168: 265 / 292),
 // equal ones where the fixed part of a tile counts (3500 x 33024 x 1280: 203 / 183, 2048 x 18176 x 512: 45 / 38).
 int pick_wide_variant(int64_t M, int64_t N, int kblocks, int cus, double* us = nullptr) {
@@ -646,7 +646,8 @@ int pick_skinny_bn(int64_t N, int act_rows, int cus) {
 // few 256 x 256 tiles to fill the chip, and weight rows that come from HBM because only one or two row tiles use
 // them.  There a K step of a DMA-ring kernel lasts about (latency of HBM under load) / (stages in flight), whatever
 // the tile size, so the estimate below is: launches + rounds of workgroups x (fixed part of a tile + K steps x time
-// per step) + the second pass when K is split.  Constants measured on MI355X (microseconds; bytes per microsecond).
+// per step) + the second pass when K is split.  Constants measured on MI355X (microseconds; bytes per microsecond) with four-wave
+// 128 x 128 tiles and 32 x 32 x 64 MFMA in all of them.
 struct MidChoice {
   int variant, splitk;
   double us;
@@ -928,7 +929,9 @@ int stream_chunk_len(int kb_min, int kb_max, int ch, int stages) {
 // Rows that cover nearly all experts: twice the caller's hint, at most the buffers' height.
 int64_t stream_span(int64_t M, int64_t hint_rows) { return hint_rows > 0 && 2 * hint_rows < M ? 2 * hint_rows : M; }
 // Time of a grouped launch (microseconds, fitted on MI355X: the weight-streaming kernel to 828 problems of 8 .. 32 experts x 1 .. 960 rows,
-// N = 512 .. 7168, K = 384 .. 7168, the ring kernels to 233 of 16 .. 1024 slots; rms 8 - 12 %): `start` + rounds of tiles x (`tile` +
+// N = 512 .. 7168, K = 384 .. 7168, the ring kernels to 233 of 16 .. 1024 slots; rms 8 - 12 % then.  The 64 x 64, 64 x 128 and quantising
+// 256-column tiles of the former got waves of their own for the loads afterwards and take down to 0.75 of their estimates, the quantising
+// ring the kernels of now; masked_second_look has estimates of the present kernels): `start` + rounds of tiles x (`tile` +
 // K blocks x a step of `step` + `row` per activation row of the tile, but no shorter than its share of the stream of weights that
 // the busy CUs draw, `rate` TB/s).  Taken over 0.92, 1 and 1.08 times the tile count, which is an estimate itself - except
 // that experts of one row tile have no more than that (32 experts x 0 .. 16 rows x 1024 x 6144 in 64 x 128 tiles are one round of
@@ -957,7 +960,8 @@ struct ExpertRows {
   double sharing(int bm) const { return span > 192.0 ? row_tiles(bm) : 1.0; }
 };
 
-// The masked layout's ring kernel that make_plan chose (act: the 128 x 256 tiles with the quantising epilogue).
+// The masked layout's ring kernel that make_plan chose (act: the 128 x 256 tiles with the quantising epilogue, whose constants are of the
+// kernel before the present one).
 double masked_ring_us(int variant, int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, int cus) {
   const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
   int bm, bn;
@@ -978,10 +982,10 @@ constexpr TileCost kStreamCostAhead[kStreamCount] = {{}, {3.0, 2.2, 0.71, 0.0041
 constexpr TileCost kStreamCostAct[kStreamCount] = {{3.7, 0.6, 0.73, 0.0025, 6.9}, {3.6, 2.0, 0.72, 0.0044, 6.9}, {}, {5.2, 2.0, 0.70, 0.0049, 6.9}, {}};
 
 // How the weight-streaming kernel runs a grouped launch (shape kStreamNone: it does not), from the typical rows of an expert, and
-// whether it is to run at all: other_us is the estimate of the kernel that would run instead (0: none).  The choice is 2.3 % behind
-// the best kernel, shape and number of slices (geometric mean of 75 random problems, bench.py --planner-sweep stream_random; 35 %
-// at worst, 8 experts x ~418 rows x 1280 x 1920); a limit on the experts' rows in its place was 6.6 % behind for the plain product and
-// 10.9 % with the quantising epilogue.
+// whether it is to run at all: other_us is the estimate of the kernel that would run instead (0: none).  The choice is 2.8 % behind
+// the best kernel, shape and number of slices (geometric mean of 75 random problems, bench.py --planner-sweep stream_random; 30 %
+// at worst, gate/up of 8 experts x ~57 rows x 2560 x 2944).  With the kernels that these estimates were fitted to it was 2.3 %; a limit on
+// the experts' rows in its place was 6.6 % behind for the plain product and 10.9 % with the quantising epilogue.
 // With the quantising epilogue a launch may also run in two: the plain product of every (tile, K slice) first, in any tile shape, then
 // the slices' sum with the activation and the quantiser.  That pays where 256-column tiles leave most CUs idle (it costs 3.8 us +
 // the partial sums' way there and back): 8 experts x ~15 rows x 1792 x 3584 24.9 -> 17.0 us, 32 x ~9 x 512 x 5632 36.9 -> 22.4 us.
@@ -989,7 +993,7 @@ constexpr TileCost kStreamCostAct[kStreamCount] = {{3.7, 0.6, 0.73, 0.0025, 6.9}
 // max_slices: 1 where the bits have to be those of the steps apart (one slice changes nothing about the sums), up to kMaxStreamSlices
 // inside an expert MLP.  all_rows: rows of the partial sums' matrices; slice_floats: room for them.
 StreamPlan pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, int cus, int max_slices, int64_t all_rows, size_t slice_floats,
-                       double other_us, bool by_estimates = false) {
+                       double other_us, bool second_look = false) {
   StreamPlan best;
   const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
   const int knob = g_knob[kKnobStream], slice_knob = g_knob[kKnobStreamSlices];
@@ -1028,54 +1032,65 @@ StreamPlan pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows
   // 116 / 123; 32 x 4096 x 7168 cap 256 217 / 226, cap 384 305 / 298; 8 x 1152 x 768, ~640 rows 15.6 / 22.8; 8 x 512 x 1920, ~244
   // rows 14.4 / 20.1.  Quantising: 8 x 512 x 2176, ~137 rows 17.6 / 26.1; 32 x 2048 x 1920, ~181 rows 50 / 61.
   const bool longer = e.span > (act ? 192 : kblocks <= 24 ? 448 : 256);
-  // by_estimates: the masked layout's plain product with a hint, where the estimates of both kernels decide from 64 rows on.  Over 350
-  // problems 2.8 % behind the best kernel and shape, 5.1 % with the limits (from 256 slots on they cost 6.9 %).  This kernel runs
-  // faster than its estimate there, most of all in launches of more than two rounds of 256 x 256 tiles: 32 x 256 x 7168 x 2048 118 us
-  // for 148, the ring 126 for 121; 32 x 256 x 4096 x 7168 223 for 282, the ring 209 for 181.
-  const bool many_rounds = static_cast<double>(G) * e.live * e.row_tiles(256) * static_cast<double>(ceil_div(N, 256)) > 2.0 * cus;
-  by_estimates = by_estimates && e.span > 64.0;
-  const double ahead = by_estimates ? (many_rounds ? 1.23 : 1.12) : 0.95;
-  if ((longer || by_estimates) && knob == 0 && slice_knob == 0 && other_us > 0.0 && best.us > ahead * other_us) best.shape = kStreamNone;
+  // second_look: masked_second_look compares the kernels afterwards; what this kernel's estimates are too high by counts for it here.
+  const double ahead = second_look ? 1.15 : 0.95;
+  if (longer && knob == 0 && slice_knob == 0 && other_us > 0.0 && best.us > ahead * other_us) best.shape = kStreamNone;
   return best;
 }
 
-// Masked plain product with a hint, from three K blocks on: a second look at the choice.  The estimates above know neither the output's
-// bytes nor how the experts' rows vary, and those of the streaming kernel are older than its waves apart: beside the kernels of before 26 of
-// 1200 random calls had become more than 5 % slower (16 x 1152 x 5760, 144 rows each 48 -> 65 us, 16 x 3712 x 3840, ~477 rows 132 -> 160).
-// These (us, fitted on MI355X to 2700 problems of 8 .. 32 experts x 4 .. 640 rows, rms 7 - 9 %): `start` + rounds of tiles x (`tile` + K
-// blocks x (`step` + `row` per activation row of a tile)) + the weights and the output at `weights` and `out` TB/s.  Rounds are whole
-// ones, averaged over what the tile count may come to: rows of 0 to twice the hint in buffers of about that height, rows about
-// the hint, as balanced routing leaves them, in taller ones.
-// Another kernel is taken where it is estimated 12 % ahead of the chosen one.  Over 1200 problems the fit had not seen the choice is then 2.6 %
-// behind the best kernel and shape (3.6 before), 14 calls are more than 5 % behind the kernels of before and 4 behind the choice without
-// it; the estimates alone would be at 1.7 %, but leave 21 and 24.
+// Masked plain product with a hint above 32, from three K blocks on: a second look at the choice.  The estimates above know neither the
+// output's bytes nor how the experts' rows vary, take half of the buffers for an expert's rows where twice the hint is more, and those of
+// the streaming kernel are older than its waves apart.  These (us, fitted on MI355X to 2400 problems of 4 .. 64 experts x hints of 33 .. 640,
+// rms 7 - 10 %): `start` + `expert` per expert + rounds of tiles x (`tile` + K blocks x (`step` + `row` per activation row of a tile)) + the
+// weights and the output at `weights` and `out` TB/s.  Rounds are whole ones, averaged over what the tile count may come to: rows
+// about the hint, as balanced routing leaves them, in buffers of more than three times it, rows evenly spread about it, as far as both ends
+// of the buffer allow, in lower ones.
+// Another kernel is taken where it is estimated 12 % ahead of the chosen one (at 6 % the choice is closer to the best, 3.3 instead of 4.2 %
+// behind it over 1200 problems outside the fit, but 19 instead of 11 calls are more than 10 % behind the kernels of before).
+// us per call, estimates that took half of the buffers for an expert's rows / these: 8 x 1664 x 7040, 603 rows of 896 126 / 82, 8 x 1408 x 6016
+// fp32, 165 of 216 53 / 33, 4 x 1408 x 1792, 414 of 520 20.6 / 12.9, 64 x 896 x 1664, 71 of 320 30 / 20; but 8 x 7168 x 2560, 153 of 336 38 / 55.
+// 1500 calls outside the fit, beside the kernels of before: 1.057 x without a second look, 82 more than 5 % and 45 more than 10 % slower;
+// with it 1.078 x, 29 and 9.
 struct MaskedCost {
-  double start, tile, step, row, weights, out;
+  double start, expert, tile, step, row, weights, out;
 };
-constexpr MaskedCost kMaskedStream[kStreamCount] = {{3.2, 1.07, 0.542, 0.0068, 17.5, 11.4}, {3.49, 1.17, 0.562, 0.00622, 18.1, 5.6}, {4.15, 0.611, 0.268, 0.00407, 16.5, 2.92}, {3.99, 0.897, 0.572, 0.0059, 18.7, 4.34}, {4.89, 0.59, 0.213, 0.00181, 29.4, 3.23}};
-constexpr MaskedCost kMaskedStreamAhead[kStreamCount] = {{}, {4.14, 1.33, 0.644, 0.0031, 20.5, 4.66}, {4.24, 1.1, 0.295, 0.00343, 19.2, 3.79}, {4.61, 1.16, 0.622, 0.00406, 19.5, 4.02}, {4.71, 0.64, 0.167, 0.00264, 21.9, 4.9}};
-constexpr MaskedCost kMasked128x256 = {4.52, 2.27, 0.625, 0.00241, 15.4, 5.67}, kMasked128x128 = {4.6, 1.84, 0.388, 0.00204, 18.1, 8.51}, kMasked256x256 = {4.91, 3.58, 1, 0.00117, 22.8, 5.42};
+constexpr MaskedCost kMaskedStream[kStreamCount] = {
+    {2.56, 0, 0.257, 0.334, 0.0129, 14.3, 4.05}, {3.01, 0, 0.663, 0.786, 0.00198, 25.4, 4.52}, {2.94, 0.0134, 1.31, 0.303, 0.00334, 21.7, 8.72}, {3.68, 0, 0.635, 0.584, 0.00563, 22.1, 4.84}, {3.78, 0.028, 0.665, 0.28, 0.000621, 69.7, 5.23}};
+constexpr MaskedCost kMaskedStreamAhead[kStreamCount] = {
+    {}, {3.5, 0, 0.908, 0.674, 0.00199, 22.3, 4.19}, {2.72, 0.0167, 1.55, 0.266, 0.00376, 20, 10}, {3.79, 0, 0.977, 0.775, 0.00232, 26.4, 4.11}, {3.25, 0.0475, 0.526, 0.254, 0.0011, 43.9, 4.55}};
+constexpr MaskedCost kMasked128x256 = {2.82, 0.0957, 1.34, 0.637, 0.00193, 16.4, 5.41}, kMasked128x128 = {2.59, 0.104, 1.03, 0.405, 0.00181, 19.6, 5.41}, kMasked256x256 = {3.48, 0.0875, 2.59, 0.99, 0.000923, 21.9, 5.94};
 
 double masked_us(const MaskedCost& c, int bm, int bn, int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, int cus) {
   const double h = static_cast<double>(std::min(hint_rows, M)), weights = static_cast<double>(N) * static_cast<double>(K);
-  double rows = h, live, row_tiles, spread;  // of an expert: rows, share that has any, row tiles; relative spread of all tiles
+  double live = 1.0, row_tiles, spread;  // of an expert: share that has rows, row tiles; relative spread of all tiles
   if (static_cast<double>(M) > 3.0 * h) {
     const double sd = std::sqrt(h);
-    live = row_tiles = 1.0 - std::exp(-h);
-    for (double above = bm; above < h + 4.0 * sd; above += bm) row_tiles += 0.5 * std::erfc((above - h) / (sd * std::sqrt(2.0)));
+    live = 1.0 - std::exp(-h);
+    const double sure = std::max(0.0, std::floor((h - 4.0 * sd) / bm));  // tiles of nearly every expert
+    row_tiles = live + sure;
+    for (double above = (sure + 1.0) * bm; above < h + 4.0 * sd; above += bm) row_tiles += 0.5 * std::erfc((above - h) / (sd * std::sqrt(2.0)));
     spread = 0.03;
   } else {
-    const double most = std::min(static_cast<double>(M), 2.0 * h), q = most / bm;
-    rows = 0.5 * most;
-    live = most / (most + 1.0);
-    row_tiles = q <= 1.0 ? live : 0.5 * (q + 1.0);
-    spread = std::max(0.02, std::sqrt(std::max(0.0, q * q - 1.0) / 12.0 / G) / row_tiles);
+    const double lo = std::max(0.0, 2.0 * h - static_cast<double>(M)), hi = std::min(static_cast<double>(M), 2.0 * h);
+    double mean = std::ceil(h / bm), square = mean * mean;
+    if (hi > 64.0 * bm) {  // long experts: without the ends of the range
+      mean = h / bm + 0.5, square = mean * mean + (hi - lo) * (hi - lo) / (12.0 * bm * bm);
+    } else if (hi - lo >= 1.0) {
+      mean = square = 0.0;
+      for (double t = std::floor(lo / bm); t * bm < hi; t += 1.0) {
+        const double share = (std::min(hi, (t + 1.0) * bm) - std::max(lo, t * bm)) / (hi - lo);
+        mean += share * (t + 1.0), square += share * (t + 1.0) * (t + 1.0);
+      }
+    }
+    if (lo == 0.0) live = hi / (hi + 1.0);
+    row_tiles = mean * live;
+    spread = std::max(0.02, std::sqrt(std::max(0.0, square - mean * mean) / G) / row_tiles);
   }
   const double tiles = G * row_tiles * static_cast<double>(ceil_div(N, bn));
   double rounds = 0.4 * std::max(1.0, std::ceil(tiles / cus));
   for (double z : {-1.2, 1.2}) rounds += 0.3 * std::max(1.0, std::ceil(tiles * (1.0 + z * spread) / cus));
-  return c.start + rounds * (c.tile + static_cast<double>(ceil_div(K, kScaleBlock)) * (c.step + c.row * rows / row_tiles)) + live * G * weights / (c.weights * 1e6) +
-         G * rows * static_cast<double>(N) * 2.0 / (c.out * 1e6);
+  return c.start + c.expert * G + rounds * (c.tile + static_cast<double>(ceil_div(K, kScaleBlock)) * (c.step + c.row * h / row_tiles)) + live * G * weights / (c.weights * 1e6) +
+         G * h * static_cast<double>(N) * 2.0 / (c.out * 1e6);
 }
 
 void masked_second_look(Plan& pl, StreamPlan& stream, int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, int cus) {

@@ -249,6 +249,12 @@ def test_masked_hint_second_look():
     for M_max, N, K, G, hint in ((1024, 3712, 3840, 16, 477), (1024, 5120, 768, 8, 566), (1064, 5504, 1920, 32, 489), (776, 4864, 5248, 16, 455)):
         assert _lib.plan_stream(M_max, N, K, G, hint) is None and _lib.plan_grouped(MASKED, M_max, N, K, G, hint)[0] == 'pipe256x256'
     assert _lib.plan_grouped(MASKED, 512, 1536, 256, 6, 500)[0] == 'pipe256x256' and _lib.plan_stream(512, 1536, 256, 6, 500) is None
+    # buffers lower than twice the hint: an expert's rows are the hint, not half of the buffer
+    for M_max, N, K, G, hint, variant in ((896, 1664, 7040, 8, 603, 'pipe256x256'), (216, 1408, 6016, 8, 165, 'pipe128x128'), (520, 1408, 1792, 4, 414, 'pipe128x128')):
+        assert _lib.plan_stream(M_max, N, K, G, hint) is None and _lib.plan_grouped(MASKED, M_max, N, K, G, hint)[0] == variant
+    # the estimates count an expert's tiles: long experts, short and tall buffers
+    for M_max, hint in ((1 << 30, 1 << 29), (1 << 30, 1 << 20), (1 << 30, 1 << 30), (20000, 9000), (9000, 9000)):
+        assert _lib.plan_grouped(MASKED, M_max, 7168, 2048, 1, hint)[0] == 'pipe256x256'
 
 
 @pytest.mark.parametrize('mode,rows', [(CONTIGUOUS, 1024), (MASKED, 64)])
