@@ -993,7 +993,7 @@ constexpr TileCost kStreamCostAct[kStreamCount] = {{3.7, 0.6, 0.73, 0.0025, 6.9}
 // max_slices: 1 where the bits have to be those of the steps apart (one slice changes nothing about the sums), up to kMaxStreamSlices
 // inside an expert MLP.  all_rows: rows of the partial sums' matrices; slice_floats: room for them.
 StreamPlan pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows, bool act, int cus, int max_slices, int64_t all_rows, size_t slice_floats,
-                       double other_us, bool second_look = false) {
+                       double other_us, bool by_estimates = false) {
   StreamPlan best;
   const int kblocks = static_cast<int>(ceil_div(K, kScaleBlock));
   const int knob = g_knob[kKnobStream], slice_knob = g_knob[kKnobStreamSlices];
@@ -1032,25 +1032,29 @@ StreamPlan pick_stream(int64_t M, int64_t N, int64_t K, int G, int64_t hint_rows
   // 116 / 123; 32 x 4096 x 7168 cap 256 217 / 226, cap 384 305 / 298; 8 x 1152 x 768, ~640 rows 15.6 / 22.8; 8 x 512 x 1920, ~244
   // rows 14.4 / 20.1.  Quantising: 8 x 512 x 2176, ~137 rows 17.6 / 26.1; 32 x 2048 x 1920, ~181 rows 50 / 61.
   const bool longer = e.span > (act ? 192 : kblocks <= 24 ? 448 : 256);
-  // second_look: masked_second_look compares the kernels afterwards; what this kernel's estimates are too high by counts for it here.
-  const double ahead = second_look ? 1.15 : 0.95;
-  if (longer && knob == 0 && slice_knob == 0 && other_us > 0.0 && best.us > ahead * other_us) best.shape = kStreamNone;
+  // by_estimates: the masked layout's plain product with a hint, where the estimates of both kernels decide from 64 rows on.  Over 350
+  // problems 2.8 % behind the best kernel and shape, 5.1 % with the limits (from 256 slots on they cost 6.9 %).  This kernel runs
+  // faster than its estimate there, most of all in launches of more than two rounds of 256 x 256 tiles: 32 x 256 x 7168 x 2048 118 us
+  // for 148, the ring 126 for 121; 32 x 256 x 4096 x 7168 223 for 282, the ring 209 for 181.
+  const bool many_rounds = static_cast<double>(G) * e.live * e.row_tiles(256) * static_cast<double>(ceil_div(N, 256)) > 2.0 * cus;
+  by_estimates = by_estimates && e.span > 64.0;
+  const double ahead = by_estimates ? (many_rounds ? 1.23 : 1.12) : 0.95;
+  if ((longer || by_estimates) && knob == 0 && slice_knob == 0 && other_us > 0.0 && best.us > ahead * other_us) best.shape = kStreamNone;
   return best;
 }
 
 // Masked plain product with a hint above 32, from three K blocks on: a second look at the choice.  The estimates above know neither the
-// output's bytes nor how the experts' rows vary, take half of the buffers for an expert's rows where twice the hint is more, and those of
+// output's bytes (of bf16 here) nor how the experts' rows vary, take half of the buffers for an expert's rows where twice the hint is more, and those of
 // the streaming kernel are older than its waves apart.  These (us, fitted on MI355X to 2400 problems of 4 .. 64 experts x hints of 33 .. 640,
 // rms 7 - 10 %): `start` + `expert` per expert + rounds of tiles x (`tile` + K blocks x (`step` + `row` per activation row of a tile)) + the
 // weights and the output at `weights` and `out` TB/s.  Rounds are whole ones, averaged over what the tile count may come to: rows
 // about the hint, as balanced routing leaves them, in buffers of more than three times it, rows evenly spread about it, as far as both ends
 // of the buffer allow, in lower ones.
-// Another kernel is taken where it is estimated 12 % ahead of the chosen one (at 6 % the choice is closer to the best, 3.3 instead of 4.2 %
-// behind it over 1200 problems outside the fit, but 19 instead of 11 calls are more than 10 % behind the kernels of before).
+// Another kernel is taken where it is estimated 12 % ahead of the chosen one.  1200 problems outside the fit, beside the first choice alone:
+// 1.024 x, 8 calls more than 5 % slower, 3.2 % behind the best kernel and shape instead of 5.6; at 6 % 1.031 x, 26 and 2.5 %.
 // us per call, estimates that took half of the buffers for an expert's rows / these: 8 x 1664 x 7040, 603 rows of 896 126 / 82, 8 x 1408 x 6016
-// fp32, 165 of 216 53 / 33, 4 x 1408 x 1792, 414 of 520 20.6 / 12.9, 64 x 896 x 1664, 71 of 320 30 / 20; but 8 x 7168 x 2560, 153 of 336 38 / 55.
-// 1500 calls outside the fit, beside the kernels of before: 1.057 x without a second look, 82 more than 5 % and 45 more than 10 % slower;
-// with it 1.078 x, 29 and 9.
+// fp32, 165 of 216 53 / 33, 4 x 1408 x 1792, 414 of 520 20.6 / 12.9, 16 x 640 x 512 fp32, 311 of 528 16.6 / 10.9; but 8 x 2688 x 768,
+// 129 of 336 10.9 / 14.3.  Of 1500 further calls 185 take another kernel than the first choice: 1.20 x, 156 more than 5 % faster, 8 slower.
 struct MaskedCost {
   double start, expert, tile, step, row, weights, out;
 };
