@@ -53,7 +53,7 @@ struct Args {
   int sk_bn;            // decode kernels with DMA staging: output columns per workgroup (multiple of 4, <= 16 NFS)
   int splitk;
   int kb_per_split;
-  int fused_reduce;     // split-K in one launch: the workgroups of a tile add its K slices themselves (see splitk_fused_epilogue)
+  int fused_reduce;     // split-K in one launch: the workgroups of a tile add its K slices themselves (see the results of ring_body and pipelined_body)
   int spin_limit;       //   polls (about half a microsecond apart) a workgroup waits for the other slices of its tile before it leaves its share to the last one
   int sct_pitch;        // kernels with a scale table in LDS: floats per table row (odd, >= K blocks per workgroup)
   int group_m;          // m-tiles per L2 swizzle group

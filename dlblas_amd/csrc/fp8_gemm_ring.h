@@ -4,8 +4,8 @@
 // What bounds it: the power limit.  Over a long K the chip settles at 1.7 to 1.9 of its 2.4 GHz, so a K step costs its energy
 // as well as its stalls, and every choice below is about one of the two:
 //   - 16 x 16 x 128 instead of two chained 32 x 32 x 64: the same bits (see chunk0), but
-//     10 % less time at the power limit (a loop of nothing but MFMAs on random codes: 282 against 311 us for 1.24e12 operations),
-//     and a partial sum is 4 registers that are complete two instructions later, instead of 16.  The registers saved hold a
+//     8 % less time at the power limit (a loop of nothing but MFMAs and scale FMAs on random codes: 3593 against 3322 TFLOP/s,
+//     bench.py --ceilings), and a partial sum is 4 registers that are complete two instructions later, instead of 16.  The registers saved hold a
 //     ring of streamed fragments, read from LDS three fragments ahead of their use.
 //   - two points of a K step at which LDS is handed over instead of one: behind the first, the held operand's rows and the first
 //     half of the streamed operand's may be refilled, behind the second the rest.  A byte is on its way for 1.1 K steps or
@@ -14,7 +14,7 @@
 //   - fragments take every other group of four rows, so that a lane's two results of a pair of fragments are 8 consecutive
 //     columns: results go from the registers to memory in 16-byte pieces, 128 or 256 bytes of a row per instruction (lanes exchange chunks
 //     through DPP first).  No LDS
-//     is involved, so the ring runs on from tile to tile (AHEAD) in every layout.  A tile with the quantising epilogue shares
+//     is involved, so the ring runs on from tile to tile (AHEAD) in every layout but plain contiguous rows.  A tile with the quantising epilogue shares
 //     nothing but its rows' largest magnitudes through LDS, where the whole tile used to pass in bf16.
 // 4096 x 8192 x 18432 in 256 x 256 tiles: 505 us with 32 x 32 MFMAs and one hand-over per step, 471 us in this form
 // (2.62 PFLOP/s); its K steps take 2740 cycles of which 2048 are MFMA.  Without the scale FMAs it would be 421 us.  (All before
@@ -109,8 +109,10 @@ __device__ __forceinline__ void swap_far_chunks(v4i& a, v4i& b) {
   }
 }
 
-// Workgroup barrier that orders LDS traffic only (see lds_barrier), as builtins: the compiler then knows that no LDS read is out
-// and counts the reads behind it instead of waiting for all of them.
+// Workgroup barrier that orders LDS traffic only (see lds_barrier), as builtins: the compiler then knows that no LDS read is out.
+// The waits that it places in a K step are for all reads nevertheless (lgkmcnt(0) ahead of slots 0, 16 and 29 of the 256 x 256 loop, beside
+// those of the two barriers): the scale load of a group (dma_4) is the form of load that its model counts on the LDS counter as well,
+// and reads behind one are no longer in order for it.  At slot 0 that waits for held fragments of which the last is needed at slot 3.
 __device__ __forceinline__ void ring_barrier() {
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
@@ -134,16 +136,16 @@ struct RingTile {
   int g, m0, n0, m_end, split, lin;
 };
 
-// Work of one workgroup: tiles vb_first, vb_first + gridDim.x, ... of a region that is tiles_m x tiles_n tiles of BM x BN and
-// starts at column n_base of the output.
-// AHEAD: the ring runs on from tile to tile; the steps of a tile whose fetches lie past the end of K fetch the first K blocks of
-// the workgroup's next tile.
 // Tile lists: the region is entries [lists.first, lists.first + lists.count) of a list's tiles (an entry per row tile and column tile), or, with 64-row tiles,
 // the entries' 64-row pieces, lists.pieces each.
 struct ListRegion {
   int which, first, count, pieces;
 };
 
+// Work of one workgroup: tiles vb_first, vb_first + gridDim.x, ... of a region that is tiles_m x tiles_n tiles of BM x BN and
+// starts at column n_base of the output (tile lists: of `lists`).
+// AHEAD: the ring runs on from tile to tile; the steps of a tile whose fetches lie past the end of K fetch the first K blocks of
+// the workgroup's next tile.
 // ODD: bf16 results whose rows lie off dwords (dense, K in one piece).
 template <class Cfg, int MODE, bool AHEAD, bool ODD = false>
 __device__ __forceinline__ void ring_body(const Args& p, uint8_t* smem, int vb_first, int tiles_m, int tiles_n, int n_base, ListRegion lists = {}) {

@@ -21,7 +21,7 @@
 // experts stay with the ring kernels, whose 256-row tiles read less LDS per product.
 //
 // Arithmetic: fp8_gemm_kernel of the reference (dlblas/kernels/fp8_gemm.py:49-60), same order of additions as the ring
-// kernels of fp8_gemm_pipelined.h, so results have the same bits.  Requires K % 128 == 0 and K / 128 >= STAGES.
+// kernels (fp8_gemm_ring.h), so results have the same bits.  Requires K % 128 == 0 and K / 128 >= STAGES.
 #pragma once
 
 #include "fp8_gemm_common.h"

@@ -234,10 +234,9 @@ int dlb_fp8_gemm_grouped_contiguous_gather_silu_quant(const void* a, const void*
  *                                             into a valid result nor written.  Values are clamped
  *                                             to [0, M_max].
  *   expected_m                                scheduling hint only (typical masked_m); <= 0 = unknown.
- *                                             It picks kernel and tile shape (the weight-streaming kernel while
- *                                             twice the hint, or M_max, is at most 256 rows, 448 for K <= 3072, 192
- *                                             for the form with the quantising epilogue; 256-row tiles from
- *                                             several hundred rows per expert on) and never changes a result bit.
+ *                                             It picks kernel and tile shape by estimates of their times (short
+ *                                             experts the weight-streaming kernel, several hundred rows per expert
+ *                                             256-row tiles) and never changes a result bit.
  *
  * The tile schedule is built on the device from masked_m: no host synchronisation and no tiles
  * for empty row ranges.  K % 16 == 0 is required.
@@ -453,8 +452,8 @@ int dlb_fp8_gemm_force_variant(int variant);
  *                           once per tile into a table in LDS
  *   DLB_KNOB_MASKED_GRID    workgroups per CU of the persistent grid of the masked layout (default 1)
  *   DLB_KNOB_TILE_LIST      expert-contiguous rows: 1 = 256- / 192- / 128-row tiles from lists built on the device
- *                           whenever a workspace allows it, 2 = uniform 128-row tiles (default: lists from more than two
- *                           rounds of 128 x 256 tiles on)
+ *                           whenever a workspace allows it, 2 = uniform 128-row tiles (default: whichever is estimated
+ *                           to be faster)
  *   DLB_KNOB_STREAM         masked layout: 1 = never the weight-streaming kernel, 2 .. 6 = its tile shape 0 .. 4 (32 x 256,
  *                           64 x 256, 64 x 128, 128 x 256, 64 x 64) wherever it applies, 7 .. 11 = the same with fragments
  *                           read one step ahead where that form exists (plain product, not 32 x 256) (default: by size)
